@@ -535,11 +535,68 @@ static hipError_t fetch_results(const PfHipWork *w, const HostBlock &b, size_t t
     return e;
 }
 
+// Longer batches pass through a ring of PF_RING_SLOTS page-locked pieces that follows the block: the CPU fills or empties
+// one piece while the others are on their way.  A hipMemcpy2D on the caller's pageable rows moves them row by row, each
+// with a wait of its own (777 rows of 8 KB each way and 31 KB of routes: 24.9 of a call's 25.4 ms; through the ring with
+// whole-piece copies 1.3 ms).  A piece is large enough that its transfer hides the enqueueing, small enough that the
+// first transfer starts early.
+#define PF_RING_SLOTS 4
+#define PF_RING_BYTES ((size_t)512 * 1024)
 static void rows_in(void *dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
     for (size_t r = 0; r < rows; r++) memcpy((uint8_t *)dst + r * row_bytes, (const uint8_t *)src + r * src_pitch, row_bytes);
 }
 static void rows_out(void *dst, size_t dst_pitch, const void *src, size_t row_bytes, size_t rows) {
     for (size_t r = 0; r < rows; r++) memcpy((uint8_t *)dst + r * dst_pitch, (const uint8_t *)src + r * row_bytes, row_bytes);
+}
+
+// Pitched host rows to dense device rows, enqueued on the default stream; the caller's rows have been read when this
+// returns.  row_bytes fits a piece (the caller checks).
+static hipError_t ring_in(PfHipWork *w, void *d_dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
+    const size_t step = PF_RING_BYTES / row_bytes;
+    hipError_t e = hipSuccess;
+    int slot = 0;
+    for (size_t r = 0; r < rows && e == hipSuccess; r += step, slot = (slot + 1) % PF_RING_SLOTS) {
+        const size_t n = rows - r < step ? rows - r : step;
+        uint8_t *piece = w->ring + slot * PF_RING_BYTES;
+        e = hipEventSynchronize(w->ring_event[slot]);   // the piece's last transfer (none yet: returns at once)
+        if (e != hipSuccess) break;
+        rows_in(piece, (const uint8_t *)src + r * src_pitch, src_pitch, row_bytes, n);
+        e = hipMemcpyAsync((uint8_t *)d_dst + r * row_bytes, piece, n * row_bytes, hipMemcpyHostToDevice, nullptr);
+        if (e == hipSuccess) e = hipEventRecord(w->ring_event[slot], nullptr);
+    }
+    return e;
+}
+// Dense device rows to pitched host rows; all of them have arrived when this returns.
+static hipError_t ring_out(PfHipWork *w, void *dst, size_t dst_pitch, const void *d_src, size_t row_bytes, size_t rows) {
+    const size_t step = PF_RING_BYTES / row_bytes, pieces = (rows + step - 1) / step;
+    hipError_t e = hipSuccess;
+    for (size_t j = 0; j < pieces + PF_RING_SLOTS - 1 && e == hipSuccess; j++) {   // piece j is sent, piece j - (slots - 1) is emptied
+        if (j < pieces) {
+            const size_t r = j * step, n = rows - r < step ? rows - r : step;
+            const int slot = (int)(j % PF_RING_SLOTS);
+            e = hipMemcpyAsync(w->ring + slot * PF_RING_BYTES, (const uint8_t *)d_src + r * row_bytes, n * row_bytes, hipMemcpyDeviceToHost, nullptr);
+            if (e == hipSuccess) e = hipEventRecord(w->ring_event[slot], nullptr);
+            if (e != hipSuccess) break;
+        }
+        if (j + 1 < PF_RING_SLOTS) continue;
+        const size_t k = j - (PF_RING_SLOTS - 1), r = k * step;
+        if (k >= pieces) break;
+        const size_t n = rows - r < step ? rows - r : step;
+        const int slot = (int)(k % PF_RING_SLOTS);
+        e = hipEventSynchronize(w->ring_event[slot]);
+        if (e == hipSuccess) rows_out((uint8_t *)dst + r * dst_pitch, dst_pitch, w->ring + slot * PF_RING_BYTES, row_bytes, n);
+    }
+    return e;
+}
+// Either through the ring where the workspace has one, else (no page-locked memory to be had, or a row longer than a
+// piece) as one blocking copy.
+static hipError_t rows_to_device(PfHipWork *w, void *d_dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
+    if (w->ring && row_bytes <= PF_RING_BYTES) return ring_in(w, d_dst, src, src_pitch, row_bytes, rows);
+    return hipMemcpy2D(d_dst, row_bytes, src, src_pitch, row_bytes, rows, hipMemcpyHostToDevice);
+}
+static hipError_t rows_to_host(PfHipWork *w, void *dst, size_t dst_pitch, const void *d_src, size_t row_bytes, size_t rows) {
+    if (w->ring && row_bytes <= PF_RING_BYTES) return ring_out(w, dst, dst_pitch, d_src, row_bytes, rows);
+    return hipMemcpy2D(dst, dst_pitch, d_src, row_bytes, row_bytes, rows, hipMemcpyDeviceToHost);
 }
 
 extern "C" int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWork **out) {
@@ -565,13 +622,24 @@ extern "C" int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWo
     for (int j = 0; j < W_COUNT; j++) w->guard_at[j] = c.offset[j] + c.size[j];
     // short batches through host pointers stage their rows in pinned memory: the copies are then enqueued and the call
     // waits once, for the last of them (without the block the forwards fall back to one blocking copy per buffer)
-    if (hipHostMalloc((void **)&w->host, host_block_bytes(&moe->desc), hipHostMallocDefault) != hipSuccess) {
+    const size_t block = host_block_bytes(&moe->desc);
+    const bool long_batches = token_cap > PF_HOST_BLOCK_TOKENS;
+    if (hipHostMalloc((void **)&w->host, block + (long_batches ? PF_RING_SLOTS * PF_RING_BYTES : 0), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         w->host = nullptr;
     } else if (hipHostGetDevicePointer((void **)&w->host_device, w->host, 0) != hipSuccess) {
         (void)hipGetLastError();
         (void)hipHostFree(w->host);
         w->host = nullptr;
+    }
+    if (w->host && long_batches) {
+        w->ring = w->host + block;
+        for (int j = 0; j < PF_RING_SLOTS; j++)
+            if (hipEventCreateWithFlags(&w->ring_event[j], hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                w->ring_event[j] = nullptr;
+                w->ring = nullptr;
+            }
     }
     *out = w;
     return PF_HIP_OK;
@@ -619,6 +687,7 @@ static void carve_work(PfHipWork *w, const Carve &c, uint8_t *base) {
 extern "C" void pf_hip_work_destroy(PfHipWork *w) {
     if (!w) return;
     if (w->logits) (void)hipFree(w->logits);   // base of the single allocation
+    for (hipEvent_t event : w->ring_event) if (event) (void)hipEventDestroy(event);
     if (w->host) (void)hipHostFree(w->host);
     free(w);
 }
@@ -887,6 +956,21 @@ extern "C" int pf_hip_moe_forward_hc_device(const PfHipMoe *moe, PfHipWork *work
     return PF_HIP_OK;
 }
 
+// After a long batch's kernels: the error word, then (where it is zero) output rows, ids and route weights to the host.
+static int long_results(PfHipWork *work, float *y, size_t y_pitch_bytes, uint32_t *ids, size_t ids_pitch_bytes, float *weights,
+                        size_t weights_pitch_bytes, size_t tokens, uint32_t *error_word) {
+    const size_t H = work->moe->desc.hidden, K = work->moe->desc.top_k;
+    HIP_TRY(hipMemcpy(error_word, work->error_word, 4, hipMemcpyDeviceToHost));
+    if (*error_word) {
+        HIP_TRY(hipMemset(work->error_word, 0, 4));   // the word is sticky on the device; reading it clears it
+        return PF_HIP_OK;
+    }
+    HIP_TRY(rows_to_host(work, y, y_pitch_bytes, work->y, H * 4, tokens));
+    if (ids) HIP_TRY(rows_to_host(work, ids, ids_pitch_bytes, work->ids, K * 4, tokens));
+    if (weights) HIP_TRY(rows_to_host(work, weights, weights_pitch_bytes, work->route_weights, K * 4, tokens));
+    return PF_HIP_OK;
+}
+
 extern "C" int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes,
                                        float *y, size_t y_pitch_bytes, uint32_t *ids, size_t ids_pitch_bytes,
                                        float *weights, size_t weights_pitch_bytes, size_t tokens,
@@ -920,21 +1004,10 @@ extern "C" int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, con
         if (weights) rows_out(weights, weights_pitch_bytes, r.weights, K * 4, tokens);
         return PF_HIP_OK;
     }
-    HIP_TRY(hipMemcpy2D(work->x, H * 4, x, x_pitch_bytes, H * 4, tokens, hipMemcpyHostToDevice));
-    // prefill-sized batches go through whole; 2..4 tokens use the decode path in one launch
+    HIP_TRY(rows_to_device(work, work->x, x, x_pitch_bytes, H * 4, tokens));
     int rc = pf_hip_moe_forward_device(moe, work, work->x, H, work->y, H, tokens, nullptr);
     if (rc != PF_HIP_OK) return rc;
-    HIP_TRY(hipMemcpy(error_word, work->error_word, 4, hipMemcpyDeviceToHost));
-    if (*error_word) {
-        HIP_TRY(hipMemset(work->error_word, 0, 4));   // the word is sticky on the device; reading it clears it
-        return PF_HIP_OK;
-    }
-    HIP_TRY(hipMemcpy2D(y, y_pitch_bytes, work->y, H * 4, H * 4, tokens, hipMemcpyDeviceToHost));
-    if (ids) HIP_TRY(hipMemcpy2D(ids, ids_pitch_bytes, work->ids, K * 4, K * 4, tokens, hipMemcpyDeviceToHost));
-    if (weights)
-        HIP_TRY(hipMemcpy2D(weights, weights_pitch_bytes, work->route_weights, K * 4, K * 4, tokens,
-                            hipMemcpyDeviceToHost));
-    return PF_HIP_OK;
+    return long_results(work, y, y_pitch_bytes, ids, ids_pitch_bytes, weights, weights_pitch_bytes, tokens, error_word);
 }
 
 // ---- a layer whose routed experts are streamed (src/qwen4_moe_internal.h:49-54, the remap hook) -----------------
@@ -988,7 +1061,7 @@ extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *wo
         rows_in(b.x, x, x_pitch_bytes, H * 4, tokens);
         HIP_TRY(hipMemcpyAsync(work->x, b.x, tokens * H * 4, hipMemcpyHostToDevice, nullptr));
     } else {
-        HIP_TRY(hipMemcpy2D(work->x, H * 4, x, x_pitch_bytes, H * 4, tokens, hipMemcpyHostToDevice));
+        HIP_TRY(rows_to_device(work, work->x, x, x_pitch_bytes, H * 4, tokens));
     }
     PfKernelArgs a = make_args(moe, work, work->x, H, work->y, H);
     const size_t lds_route = (H + 3 * (size_t)moe->desc.experts) * 4;
@@ -1086,17 +1159,7 @@ extern "C" int pf_hip_moe_experts_streamed_host(const PfHipMoe *moe, PfHipWork *
         if (weights) rows_out(weights, weights_pitch_bytes, r.weights, K * 4, tokens);
         return PF_HIP_OK;
     }
-    HIP_TRY(hipMemcpy(error_word, work->error_word, 4, hipMemcpyDeviceToHost));
-    if (*error_word) {
-        HIP_TRY(hipMemset(work->error_word, 0, 4));
-        return PF_HIP_OK;
-    }
-    HIP_TRY(hipMemcpy2D(y, y_pitch_bytes, work->y, H * 4, H * 4, tokens, hipMemcpyDeviceToHost));
-    if (ids) HIP_TRY(hipMemcpy2D(ids, ids_pitch_bytes, work->ids, K * 4, K * 4, tokens, hipMemcpyDeviceToHost));
-    if (weights)
-        HIP_TRY(hipMemcpy2D(weights, weights_pitch_bytes, work->route_weights, K * 4, K * 4, tokens,
-                            hipMemcpyDeviceToHost));
-    return PF_HIP_OK;
+    return long_results(work, y, y_pitch_bytes, ids, ids_pitch_bytes, weights, weights_pitch_bytes, tokens, error_word);
 }
 
 struct DeviceBlock {   // one allocation, freed on scope exit

@@ -139,6 +139,8 @@ struct PfHipWork {
     uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles;
     uint8_t *host;                  // pinned host block for the host-pointer forwards of short batches (null: not available)
     uint8_t *host_device;           // the same block as the kernels address it (they write the output rows straight into it)
+    uint8_t *ring;                  // page-locked pieces behind the block, for host-pointer forwards of longer batches (null: none)
+    hipEvent_t ring_event[4];      // a piece's last transfer
     int stage_limit;                // profiling: launch only the first so many kernels of a forward; 0 = all
     int force_general;               // tests: run the general kernels even where the decode path applies
     size_t guard, guard_at[40];      // diagnostics (PF_WORK_GUARD=1): bytes of pattern behind each buffer, and where
