@@ -399,7 +399,7 @@ extern "C" size_t pf_hip_moe_bytes(const PfHipMoe *m) { return m ? m->total_byte
 // (the error word, the ids and the route weights follow each other: a short batch's are fetched by one copy)
 enum { W_LOGITS, W_SSQ, W_ERR, W_IDS, W_RW, W_ACT, W_SACT, W_SSCALE, W_X, W_Y, W_SLOTS, W_UNIQ, W_EXACT, W_FLAGS, W_XIMG, W_AIMG,
        W_FLINES, W_FGEN, W_X16, W_ACT16, W_SACT16, W_XSCALE, W_ACTSCALE, W_SACTSCALE, W_XMAX2, W_DOWN, W_COUNTS, W_OFFSETS,
-       W_P2R, W_R2P, W_GROUPBAD, W_TILES, W_COUNT };
+       W_P2R, W_R2P, W_GROUPBAD, W_TILES, W_ITEMS, W_COUNT };
 #define PF_GUARD_BYTES 4096
 struct Carve { size_t offset[W_COUNT], size[W_COUNT], total; bool fused; size_t guard; };
 // fused: plan the activation lines of the decode path's one-launch expert stage (a workspace of the library's own;
@@ -413,7 +413,10 @@ static Carve plan_work(const PfHipMoeDesc *d, size_t cap, bool fused = false, si
     // (one format throughout, or a checkpoint profile: Q8_0 shared expert)
     bool one_format = (d->type[1] == PF_Q4_K || d->type[1] == PF_IQ2_XXS) && d->type[2] == d->type[1];
     for (int t = 4; t <= 6; t++) one_format &= d->type[t] == d->type[1] || d->type[t] == PF_Q8_0;
-    const size_t Tt = !one_format ? Td : T < PF_TILE_DECODE_MAX_TOKENS ? T : PF_TILE_DECODE_MAX_TOKENS;
+    // ... and per batch of the kernels for a few rows per expert, which share the images
+    const bool prefill = T > PF_DECODE_MAX_TOKENS && pf_prefill_supported(*d);
+    const size_t Tmost = prefill ? PF_BATCH_MAX_TOKENS : PF_TILE_DECODE_MAX_TOKENS;
+    const size_t Tt = !one_format ? Td : T < Tmost ? T : Tmost;
     size_t want[W_COUNT];
     want[W_LOGITS] = T * E * 4;
     want[W_SSQ] = T * E * 4;
@@ -443,7 +446,6 @@ static Carve plan_work(const PfHipMoeDesc *d, size_t cap, bool fused = false, si
         want[W_AIMG] = rows * pf_image2_words(widest) * 4;
     }
     // prefill path: fp16 copies, per-row scales, down products in expert order, grouping tables
-    const bool prefill = T > PF_DECODE_MAX_TOKENS && pf_prefill_supported(*d);
     const size_t Tp = prefill ? T : 0, Is = d->shared_inter;
     // one more row each, never written after the workspace's initial memset: the all-zero row
     want[W_X16] = prefill ? (Tp + 1) * pf_prefill_half_row((int)H) * 2 : 0;
@@ -460,6 +462,7 @@ static Carve plan_work(const PfHipMoeDesc *d, size_t cap, bool fused = false, si
     want[W_R2P] = Tp * K * 4;
     want[W_GROUPBAD] = prefill ? 4 : 0;
     want[W_TILES] = prefill ? (1 + (size_t)pf_prefill_max_tiles((int)T, (int)E, (int)K)) * 4 : 0;
+    want[W_ITEMS] = prefill ? (size_t)pf_prefill_max_tiles((int)T, (int)E, (int)K) * 16 : 0;
     c.guard = guard;
     for (int j = 0; j < W_COUNT; j++) {
         c.offset[j] = c.total;
@@ -681,6 +684,7 @@ static void carve_work(PfHipWork *w, const Carve &c, uint8_t *base) {
         w->row_to_pair = (uint32_t *)(base + c.offset[W_R2P]);
         w->group_bad = (uint32_t *)(base + c.offset[W_GROUPBAD]);
         w->tiles = (uint32_t *)(base + c.offset[W_TILES]);
+        w->items = (uint32_t *)(base + c.offset[W_ITEMS]);
     }
 }
 
@@ -782,7 +786,7 @@ static PfKernelArgs make_args(const PfHipMoe *m, PfHipWork *w, const float *d_x,
     a.x_scale = w->x_scale; a.act_scale = w->act_scale; a.sact_scale = w->sact_scale; a.x_max2 = w->x_max2;
     a.w_norm2 = m->w_norm2; a.down = w->down;
     a.counts = w->counts; a.offsets = w->offsets; a.pair_to_row = w->pair_to_row; a.row_to_pair = w->row_to_pair;
-    a.group_bad = w->group_bad; a.tiles = w->tiles;
+    a.group_bad = w->group_bad; a.tiles = w->tiles; a.items = w->items;
     a.token_cap = (uint32_t)w->cap;
     a.router_t = m->router_t;
     for (int j = 0; j < 8; j++) { a.wt[j] = m->w_tiled[j]; a.wi[j] = m->w_itile[j]; a.wq[j] = m->w_qtile[j]; }
@@ -796,9 +800,25 @@ struct HcTarget {   // residual streams to inject into instead of writing y
     int streams;
 };
 
-// Most tokens the decode kernels take in one forward of this layer.
-static size_t decode_limit(const PfHipMoe *moe) {
-    return pf_decode_tile_layer(moe->desc, moe->w_tiled, moe->w_itile, moe->w_qtile) ? PF_TILE_DECODE_MAX_TOKENS : PF_DECODE_MAX_TOKENS;
+// Which kernels a resident layer's batch runs, by tokens (each boundary where the two sides measured the same):
+//   up to pair_to    the decode kernels, which read an expert once per (token, expert) pair: 126 us against 147 at 32 tokens
+//                    of a layer of one format throughout; the checkpoint profiles' down kernel is slower per pair (q2: 118
+//                    against 112 at 12 tokens)
+//   up to batch_to   the kernels for a few rows per expert: 202 us against 250 at 101 tokens of a Q4_K layer, 298 / 295 at
+//                    256; 325 against 563 at 101 tokens of the q2 profile, 564 / 635 at 360
+//   beyond           the grouped product of 32-row tiles
+struct BatchRange { size_t pair_to, batch_to; };
+static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
+    const int combination = pf_decode_tile_layer(moe->desc, moe->w_tiled, moe->w_itile, moe->w_qtile);
+    const size_t short_to = combination ? PF_TILE_DECODE_MAX_TOKENS : PF_DECODE_MAX_TOKENS;
+    if (!work->down || !moe->prefill_ready) return {short_to, 0};   // the workspace was planned without the grouping's tables
+    if (!combination) return {short_to, moe->desc.type[1] == PF_Q4_K ? 240u : 320u};   // no tile-ordered copies: the rows as they are stored
+    switch (combination) {
+    case 1: return {32, 240};
+    case 2: return {32, 320};
+    case 3: return {10, 400};
+    default: return {PF_TILE_DECODE_MAX_TOKENS, 400};
+    }
 }
 
 static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_x, size_t x_pitch, float *d_y,
@@ -815,8 +835,11 @@ static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_
         return PF_HIP_E_UNSUPPORTED;
     }
     const bool aligned = (x_pitch % 4 == 0) && ((uintptr_t)d_x % 16 == 0);
-    if (moe->decode_ready && tokens <= decode_limit(moe) && aligned && !work->force_general) {
+    const BatchRange range = batch_range(moe, work);
+    if (moe->decode_ready && tokens <= range.pair_to && aligned && !work->force_general) {
         pf_launch_decode(a, (int)tokens, s, work->stage_limit);
+    } else if (moe->decode_ready && tokens <= range.batch_to && aligned && !work->force_general) {
+        pf_launch_batch(a, (int)tokens, s, work->stage_limit);
     } else if (moe->prefill_ready && work->down && tokens > PF_DECODE_MAX_TOKENS && aligned && !work->force_general) {
         pf_launch_prefill(a, (int)tokens, s, work->stage_limit);
     } else {
@@ -837,7 +860,8 @@ static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_
 extern "C" int pf_hip_moe_kernel_family(const PfHipMoe *moe, const PfHipWork *work, size_t tokens) {
     if (!moe || !work || work->force_general) return 0;
     if (moe->streamed) return moe->stream_decode && tokens <= PF_TILE_DECODE_MAX_TOKENS ? 1 : 0;   // given a pool with tile-ordered slots
-    if (moe->decode_ready && tokens <= decode_limit(moe)) return 1;
+    const BatchRange range = batch_range(moe, work);
+    if (moe->decode_ready && (tokens <= range.pair_to || (range.batch_to && tokens <= PF_TILE_DECODE_MAX_TOKENS))) return 1;
     if (moe->prefill_ready && work->down && tokens > PF_DECODE_MAX_TOKENS) return 2;
     return 0;
 }
@@ -1047,6 +1071,13 @@ static bool streamed_decode(const PfHipMoe *moe, const PfHipWork *work, size_t t
     return moe->stream_decode && tiled_mask == wanted && tokens <= PF_TILE_DECODE_MAX_TOKENS && !work->force_general;
 }
 
+// Longer batches of such a layer: the kernels for a few rows per expert.
+static bool streamed_batch(const PfHipMoe *moe, const PfHipWork *work, size_t tokens, uint32_t tiled_mask) {
+    const uint32_t wanted = moe->stream_decode <= 2 ? 7u : 3u;
+    return moe->stream_decode && tiled_mask == wanted && work->down && tokens > PF_TILE_DECODE_MAX_TOKENS && tokens <= PF_BATCH_MAX_TOKENS &&
+           !work->force_general;
+}
+
 extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes,
                                               size_t tokens, uint32_t tiled_mask, uint32_t *ids, uint32_t *error_word) {
     if (!moe || !work || work->moe != moe || !error_word) return PF_HIP_E_ARGUMENT;
@@ -1069,7 +1100,10 @@ extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *wo
         snprintf(g_error, sizeof g_error, "dimensions exceed the LDS staging of the general kernels");
         return PF_HIP_E_UNSUPPORTED;
     }
-    if (streamed_decode(moe, work, tokens, tiled_mask)) {
+    if (streamed_batch(moe, work, tokens, tiled_mask)) {
+        pf_launch_batch_router(a, (int)tokens, nullptr);
+        pf_launch_dec_route(a, (int)tokens, nullptr);
+    } else if (streamed_decode(moe, work, tokens, tiled_mask)) {
         HIP_TRY(hipMemsetAsync(work->route_flags, 0, 4, nullptr));   // the routing's list starts empty (the other router kernels clear it themselves)
         pf_launch_dec_router(a, (int)tokens, (int)((moe->desc.experts + 3) / 4), nullptr);
         pf_launch_route(a, (int)tokens, nullptr);
@@ -1141,6 +1175,10 @@ extern "C" int pf_hip_moe_experts_streamed_host(const PfHipMoe *moe, PfHipWork *
     if (streamed_decode(moe, work, tokens, tiled_mask)) {
         // kernel 1 ran in the first call (logits and the token rows' images are in the workspace): kernels 2 and 3 only
         pf_launch_decode_stream_experts(a, (int)tokens, nullptr);
+    } else if (streamed_batch(moe, work, tokens, tiled_mask)) {
+        pf_launch_group(a, a.ids, (int)tokens, nullptr);
+        pf_launch_batch_experts(a, (int)tokens, nullptr, 4);
+        pf_launch_combine(a, (int)tokens, nullptr);
     } else {
         pf_launch_general(a, (int)tokens, nullptr, 0, 3);
     }

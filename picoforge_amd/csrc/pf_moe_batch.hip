@@ -1,0 +1,609 @@
+// Batches between decode and prefill: the expert products of a few rows per expert.
+//
+// A batch of some tens of tokens meets most of a layer's experts with one to a few rows each.  The grouped product of
+// pf_moe_prefill.hip pays for 32 rows whatever a tile holds, and the decode kernels read and unpack an expert's weights once
+// per (token, expert) pair.  Here a work item is an expert's row tile (up to 32 rows) against one slab of weight rows: the
+// weights come from memory once, and once in registers serve eight rows at a time.
+//
+//   pf_k_batch_gate_up   gate and up products of 32 units, SwiGLU, the activation rows' digit images (expert order)
+//   pf_k_batch_down      down products of 128 output rows, FP32, in expert order (pf_k_pf_combine adds them up)
+//
+// Arithmetic: the decode kernels'.  Activations are digit images (24-bit integers per 32-group as three balanced base-256
+// digits), weight codes signed bytes, the group's dot product exact in integers, the group's scale and minimum applied in
+// FP32.  The integer products run on v_mfma_i32_32x32x32_i8, one instruction per 32-group:
+//
+//   A (rows)     lane (m = lane % 32, h = lane / 32): digit plane m % 4 of the chunk's token m / 4, bytes 16 h .. 16 h + 15
+//                of the group (plane 3 repeats plane 2; its results are not looked at)
+//   B (columns)  lane (n = lane % 32, h): weight row n's codes 16 h .. 16 h + 15 of the group
+//   D            lane (n, h), register 4 q + p: weight row n, token 2 q + h, plane p
+//
+// so the three planes of a (row, token) sum meet in one lane, the lane's weight row is the one whose scales it holds, and a
+// chunk of up to 2 q tokens only recombines q of the four register quads.  Per 32 x 32 weights: 6 (Q4_K) to 28 (MXFP4)
+// vector instructions for the codes, about 5 for the scales, 7 per quad -- against 36 per token for the dot-product
+// instructions of the decode kernels and about 75, whatever the rows, for the FP16 product of the prefill kernels.
+#include "pf_moe_internal.h"
+#include "pf_image.h"
+#include "pf_route_device.h"
+
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef int int16v __attribute__((ext_vector_type(16)));
+typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+
+#define BATCH_ROWS 8           // rows of a chunk
+
+// ---- the weights of one 32-row tile and one piece of K ----------------------------------------------
+// GROUPS 32-groups in registers: lane (row = lane % 32, h = lane / 32).  operand(g): the row's codes 16 h .. 16 h + 15 of
+// group g as signed bytes; scale(g), minimum(g): the factors of the products' and of the activations' sums.
+// ROWS: stored row by row; else in the tile order where the format has one.
+template <int FMT, bool ROWS> struct BatchRows;
+
+template <bool ROWS> struct BatchRows<PF_Q4_K, ROWS> {   // in tile order a 64-weight run of the tile is one 1 KB load; else GGUF rows
+    static constexpr int GROUPS = 8;
+    static constexpr bool MINIMA = true, MIN_OPERAND = false;
+    uint4 hdr, q[4];
+    uint32_t sc[2], mn[2];
+    float d, dmin;
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane) {
+        if constexpr (!ROWS) {
+            const uint8_t *chunk = a.wt[t] + pf_q4t_chunk_at(a.expert_bytes[t], e, tile, a.blocks_per_row[t], piece);
+            hdr = *reinterpret_cast<const uint4 *>(chunk + pf_q4t_header_at(lane & 31));
+#pragma unroll
+            for (int run = 0; run < 4; run++) q[run] = *reinterpret_cast<const uint4 *>(chunk + pf_q4t_piece_at(run, 0, 0) + 16 * lane);
+        } else {
+            const uint8_t *block = a.w[t] + (e * (size_t)a.n_out[t] + (size_t)(32 * tile)) * a.row_bytes[t] + 144 * (size_t)piece;   // uniform
+            const uint32_t at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t], code_at = at + 16 * (uint32_t)(lane >> 5);
+            hdr = *reinterpret_cast<const uint4 *>(block + at);
+#pragma unroll
+            for (int run = 0; run < 4; run++) q[run] = *reinterpret_cast<const uint4 *>((block + 16 + 32 * run) + code_at);
+        }
+    }
+    __device__ __forceinline__ void open() {   // src/qwen4_packed.c:89-90
+        d = half_bits(hdr.x & 0xffffu); dmin = half_bits(hdr.x >> 16);
+        sc[0] = hdr.y & 0x3f3f3f3fu; mn[0] = hdr.z & 0x3f3f3f3fu;
+        sc[1] = (hdr.w & 0x0f0f0f0fu) | ((hdr.y >> 2) & 0x30303030u);
+        mn[1] = ((hdr.w >> 4) & 0x0f0f0f0fu) | ((hdr.z >> 2) & 0x30303030u);
+    }
+    __device__ __forceinline__ int4v operand(int g, const uint32_t *) const {
+        const uint4 v = q[g >> 1];
+        const int s = 4 * (g & 1);
+        return int4v{(int)((v.x >> s) & 0x0f0f0f0fu), (int)((v.y >> s) & 0x0f0f0f0fu), (int)((v.z >> s) & 0x0f0f0f0fu), (int)((v.w >> s) & 0x0f0f0f0fu)};
+    }
+    __device__ __forceinline__ int4v min_operand(int) const { return int4v{0, 0, 0, 0}; }
+    __device__ __forceinline__ float scale(int g) const { return d * (float)((sc[g >> 2] >> (8 * (g & 3))) & 255u); }
+    __device__ __forceinline__ float minimum(int g) const { return dmin * (float)((mn[g >> 2] >> (8 * (g & 3))) & 255u); }
+};
+
+// four unsigned magnitudes of at least one and their signs' byte mask: negated where the mask is set (no carry leaves a byte)
+__device__ __forceinline__ int signed_bytes(uint32_t magnitudes, uint32_t mask) { return (int)((magnitudes ^ mask) + (mask & 0x01010101u)); }
+
+template <bool ROWS> struct BatchRows<PF_IQ2_XXS, ROWS> {   // in tile order, else payloads row by row; LDS: 256 x 8 magnitudes, then 128 masks of eight sign bytes
+    static constexpr int GROUPS = 8;
+    static constexpr bool MINIMA = false, MIN_OPERAND = false;
+    uint4 q[4];
+    uint32_t dbits;
+    float d;
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane) {
+        const int kblocks = a.blocks_per_row[t];
+        if constexpr (!ROWS) {
+            const uint8_t *chunk = a.wi[t] + pf_i2t_chunk_at(pf_i2t_expert_bytes(a.n_out[t], kblocks), e, tile, kblocks, piece);
+#pragma unroll
+            for (int run = 0; run < 4; run++) q[run] = *reinterpret_cast<const uint4 *>(chunk + pf_i2t_piece_at(run, lane & 31));
+            dbits = *reinterpret_cast<const uint16_t *>(chunk + pf_i2t_scale_at(lane & 31));
+        } else {
+            const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);   // uniform
+            const uint8_t *block = a.w[t] + row0 * a.row_bytes[t] + 64 * (size_t)piece;
+            const uint8_t *scales = a.w[t] + a.scale_offset[t] + 2 * (row0 * (size_t)kblocks + (size_t)piece);
+            const uint32_t at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t];
+#pragma unroll
+            for (int run = 0; run < 4; run++) q[run] = *reinterpret_cast<const uint4 *>((block + 16 * run) + at);
+            dbits = *reinterpret_cast<const uint16_t *>(scales + 2 * (uint32_t)(lane & 31) * (uint32_t)kblocks);
+        }
+    }
+    __device__ __forceinline__ void open() { d = 0.125f * half_bits(dbits); }
+    __device__ __forceinline__ int4v operand(int g, const uint32_t *tables) const {
+        const uint4 v = q[g >> 1];
+        const bool high = pf_lane() >= 32;   // the lane's half: slots 0 and 1, or 2 and 3
+        const uint32_t idx = ((g & 1) ? v.z : v.x) >> (high ? 16 : 0), signs = ((g & 1) ? v.w : v.y) >> (high ? 14 : 0);
+        const uint2 *grid = reinterpret_cast<const uint2 *>(tables), *masks = grid + 256;
+        const uint2 m0 = grid[idx & 255u], m1 = grid[(idx >> 8) & 255u], s0 = masks[signs & 127u], s1 = masks[(signs >> 7) & 127u];
+        return int4v{signed_bytes(m0.x, s0.x), signed_bytes(m0.y, s0.y), signed_bytes(m1.x, s1.x), signed_bytes(m1.y, s1.y)};
+    }
+    __device__ __forceinline__ int4v min_operand(int) const { return int4v{0, 0, 0, 0}; }
+    __device__ __forceinline__ float scale(int g) const { return d * (float)(2u * (((g & 1) ? q[g >> 1].w : q[g >> 1].y) >> 28) + 1u); }
+    __device__ __forceinline__ float minimum(int) const { return 0.0f; }
+};
+
+template <bool ROWS> struct BatchRows<PF_Q8_0, ROWS> {   // the checkpoint profiles' shared expert: gate and up in tile order, down row by row
+    static constexpr int GROUPS = 4;
+    static constexpr bool MINIMA = false, MIN_OPERAND = false;
+    uint4 q[4];
+    uint32_t d2[2];
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane) {
+        if constexpr (!ROWS) {
+            const int runs = a.blocks_per_row[t] / 2, h = lane >> 5;
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const uint8_t *chunk = a.wq[t] + pf_q8t_chunk_at(0, 0, tile, runs, 2 * piece + r);
+                q[2 * r] = *reinterpret_cast<const uint4 *>(chunk + pf_q8t_piece_at(h, lane & 31));
+                q[2 * r + 1] = *reinterpret_cast<const uint4 *>(chunk + pf_q8t_piece_at(2 + h, lane & 31));
+                d2[r] = *reinterpret_cast<const uint32_t *>(chunk + pf_q8t_scales_at(lane & 31));
+            }
+        } else {
+            const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);   // uniform; the lane's row by a 32-bit offset
+            const uint8_t *codes = a.w[t] + row0 * a.row_bytes[t], *scales = a.w[t] + a.scale_offset[t] + 2 * row0 * (size_t)a.blocks_per_row[t];
+            const uint32_t code_at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t] + 16 * (uint32_t)(lane >> 5);
+            const uint32_t scale_at = 2 * (uint32_t)(lane & 31) * (uint32_t)a.blocks_per_row[t];
+#pragma unroll
+            for (int r = 0; r < 2; r++) {   // groups come in pairs (widths are whole 64-value segments)
+                const int g = min(GROUPS * piece + 2 * r, groups - 2);
+                q[2 * r] = *reinterpret_cast<const uint4 *>((codes + 32 * g) + code_at);
+                q[2 * r + 1] = *reinterpret_cast<const uint4 *>((codes + 32 * (g + 1)) + code_at);
+                d2[r] = *reinterpret_cast<const uint32_t *>((scales + 2 * g) + scale_at);
+            }
+        }
+    }
+    __device__ __forceinline__ void open() {}
+    __device__ __forceinline__ int4v operand(int g, const uint32_t *) const { return int4v{(int)q[g].x, (int)q[g].y, (int)q[g].z, (int)q[g].w}; }
+    __device__ __forceinline__ int4v min_operand(int) const { return int4v{0, 0, 0, 0}; }
+    __device__ __forceinline__ float scale(int g) const { return half_bits((g & 1) ? d2[g >> 1] >> 16 : d2[g >> 1] & 0xffffu); }
+    __device__ __forceinline__ float minimum(int) const { return 0.0f; }
+};
+
+template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // row by row: a lane reads its row's whole block and keeps the low or the high nibbles
+    static constexpr int GROUPS = 8;
+    static constexpr bool MINIMA = false, MIN_OPERAND = false;
+    uint4 q[8];
+    uint32_t e2[4];
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane) {
+        const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
+        const uint8_t *codes = a.w[t] + row0 * a.row_bytes[t], *scales = a.w[t] + a.scale_offset[t] + row0 * (size_t)a.blocks_per_row[t];
+        const uint32_t code_at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t], scale_at = (uint32_t)(lane & 31) * (uint32_t)a.blocks_per_row[t];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int g = min(GROUPS * piece + 2 * r, groups - 2);
+            q[2 * r] = *reinterpret_cast<const uint4 *>((codes + 16 * g) + code_at);
+            q[2 * r + 1] = *reinterpret_cast<const uint4 *>((codes + 16 * (g + 1)) + code_at);
+            e2[r] = *reinterpret_cast<const uint16_t *>((scales + g) + scale_at);
+        }
+    }
+    __device__ __forceinline__ void open() {}
+    __device__ __forceinline__ int4v operand(int g, const uint32_t *) const {
+        const int s = pf_lane() >= 32 ? 4 : 0;
+        return int4v{e2m1_twice4(q[g].x >> s), e2m1_twice4(q[g].y >> s), e2m1_twice4(q[g].z >> s), e2m1_twice4(q[g].w >> s)};
+    }
+    __device__ __forceinline__ int4v min_operand(int) const { return int4v{0, 0, 0, 0}; }
+    __device__ __forceinline__ float scale(int g) const { return 0.5f * pf_e8m0_scale((e2[g >> 1] >> (8 * (g & 1))) & 255u); }   // the integers are twice the values
+    __device__ __forceinline__ float minimum(int) const { return 0.0f; }
+};
+
+// Q2_K, row by row: a lane's half of a group is one sub-group of 16, so its 4-bit scale goes into the codes (at most 45) and
+// its 4-bit minimum is an operand of its own (the sum of the activations of a sub-group is a product with it).
+template <bool ROWS> struct BatchRows<PF_Q2_K, ROWS> {
+    static constexpr int GROUPS = 8;
+    static constexpr bool MINIMA = true, MIN_OPERAND = true;
+    uint32_t q[8], sm[4], dd;
+    float d, dmin;
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane) {
+        const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
+        const uint32_t *blocks = reinterpret_cast<const uint32_t *>(a.w[t] + row0 * a.row_bytes[t] + 84 * (size_t)piece);
+        const uint32_t at = (uint32_t)(lane & 31) * (uint32_t)(a.row_bytes[t] / 4), code_at = at + 4 + 4 * (uint32_t)(lane >> 5);
+#pragma unroll
+        for (int i = 0; i < 4; i++) sm[i] = blocks[at + i];
+#pragma unroll
+        for (int i = 0; i < 8; i++) q[i] = blocks[code_at + 8 * (i >> 2) + (i & 3)];
+        dd = blocks[at + 20];
+    }
+    __device__ __forceinline__ void open() { d = half_bits(dd & 0xffffu); dmin = half_bits(dd >> 16); }
+    __device__ __forceinline__ uint32_t scale_min(int g) const {   // byte 2 g + h
+        return (sm[g >> 1] >> (16 * (g & 1) + (pf_lane() >= 32 ? 8 : 0))) & 255u;
+    }
+    __device__ __forceinline__ int4v operand(int g, const uint32_t *) const {
+        const unsigned short s = (unsigned short)(scale_min(g) & 15u);
+        int4v out;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {   // two codes of at most 3 per 16 bits: no carry between them
+            const uint32_t codes = (q[4 * (g >> 2) + i] >> (2 * (g & 3))) & 0x03030303u;
+            out[i] = __builtin_bit_cast(int, __builtin_bit_cast(ushort2v, codes) * ushort2v{s, s});
+        }
+        return out;
+    }
+    __device__ __forceinline__ int4v min_operand(int g) const {
+        const uint32_t m = scale_min(g) >> 4;
+        const int all = (int)__builtin_amdgcn_perm(m, m, 0u);
+        return int4v{all, all, all, all};
+    }
+    __device__ __forceinline__ float scale(int) const { return d; }
+    __device__ __forceinline__ float minimum(int) const { return dmin; }
+};
+
+// ---- a chunk's rows against a piece ------------------------------------------------------------------
+struct BatchFactor { float step, sum; };   // a (token, group)'s step, and step * sum of the group's integers
+
+__device__ __forceinline__ float batch_value(const int16v &d, int q) {
+    return fmaf(65536.0f, (float)d[4 * q + 2], (float)(d[4 * q] + (d[4 * q + 1] << 8)));
+}
+
+// acc[s][q] += the products of set s's piece with tokens 2 q + h of the chunk
+template <int FMT, bool ROWS, int SETS, int QUADS>
+__device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS], const int4v (&x)[BatchRows<FMT, ROWS>::GROUPS], const BatchFactor *factors,
+                                            int here, const uint32_t *tables, float (&acc)[SETS][4]) {
+    typedef BatchRows<FMT, ROWS> Rows;
+    const int16v zero = {0};
+#pragma unroll
+    for (int g = 0; g < Rows::GROUPS; g++) {
+        if (g >= here) break;   // the ragged end of a row
+        int16v d[SETS], m[SETS];
+#pragma unroll
+        for (int s = 0; s < SETS; s++) {
+            d[s] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[g], w[s].operand(g, tables), zero, 0, 0, 0);
+            if (Rows::MIN_OPERAND) m[s] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[g], w[s].min_operand(g), zero, 0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < SETS; s++) {
+            const float scale = w[s].scale(g), minimum = Rows::MINIMA ? w[s].minimum(g) : 0.0f;
+#pragma unroll
+            for (int q = 0; q < QUADS; q++) {
+                const BatchFactor f = factors[16 * q + g];
+                if (Rows::MIN_OPERAND) {
+                    acc[s][q] = fmaf(f.step, fmaf(scale, batch_value(d[s], q), -minimum * batch_value(m[s], q)), acc[s][q]);
+                } else {
+                    acc[s][q] = fmaf(f.step * batch_value(d[s], q), scale, acc[s][q]);
+                    if (Rows::MINIMA) acc[s][q] = fmaf(-f.sum, minimum, acc[s][q]);
+                }
+            }
+        }
+    }
+}
+
+// The chunk's activation operands of a piece and the piece's factors into the wave's LDS (factors[8 * token + group]).
+// at, factor_at: the dword offsets in `images` of the images of the lane's token (lane % 32) / 4, and lane / 8.  Groups
+// beyond the row's last repeat it with a factor of zero.
+template <int GROUPS>
+__device__ __forceinline__ void batch_operands(int4v (&x)[GROUPS], BatchFactor *factors, const uint32_t *images, uint32_t at, uint32_t factor_at,
+                                               int piece, int groups, int lane) {
+    const uint32_t mine = at + 8 * (uint32_t)min(lane & 3, PF_IMG_PLANES - 1) + 4 * (uint32_t)(lane >> 5);
+#pragma unroll
+    for (int g = 0; g < GROUPS; g++) {
+        const uint32_t *group = images + PF_IMG_GROUP * min(GROUPS * piece + g, groups - 1);   // uniform
+        x[g] = *reinterpret_cast<const int4v *>(group + mine);
+    }
+    const int fg = GROUPS * piece + (lane & 7), last = min(fg, groups - 1);
+    const float step = fg < groups ? __uint_as_float((images + PF_IMG_GROUP * groups)[factor_at + (uint32_t)last]) : 0.0f;
+    const int sum = (int)(images + (PF_IMG_GROUP + 1) * groups)[factor_at + (uint32_t)last];
+    pf_wave_lds_fence();   // the piece before has been read
+    factors[lane] = BatchFactor{step, step * (float)sum};
+    pf_wave_lds_fence();
+}
+
+// The lane's index, not known to be the same from one chunk to the next: the addresses that depend on it are formed where
+// they are used, as a uniform base and a 32-bit offset, instead of being kept as 64-bit pointers across the chunks (two
+// registers a pointer, which spilled).
+__device__ __forceinline__ int batch_lane() {
+    int lane = pf_lane();
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
+// image_at(r): dword offset in `images` of the image of the chunk's row r
+template <int FMT, bool ROWS, int SETS, typename ImageAt>
+__device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&tensor)[SETS], size_t e, int tile, int first_piece, int piece_step,
+                                            int groups, const uint32_t *images, ImageAt image_at, BatchFactor *factors, int rows,
+                                            const uint32_t *tables, float (&acc)[SETS][4]) {
+    typedef BatchRows<FMT, ROWS> Rows;
+    const int pieces = (groups + Rows::GROUPS - 1) / Rows::GROUPS;
+    if (first_piece >= pieces) return;
+    Rows w[SETS];
+    uint32_t at, factor_at;
+    {
+        const int lane = batch_lane();
+#pragma unroll
+        for (int s = 0; s < SETS; s++) w[s].load(a, tensor[s], e, tile, first_piece, groups, lane);   // on their way while the rows are looked up
+        at = image_at(min((lane & 31) >> 2, rows - 1));
+        factor_at = image_at(min(lane >> 3, rows - 1));
+    }
+    for (int piece = first_piece; piece < pieces; piece += piece_step) {
+        const int lane = batch_lane();
+        int4v x[Rows::GROUPS];
+        batch_operands<Rows::GROUPS>(x, factors, images, at, factor_at, piece, groups, lane);
+#pragma unroll
+        for (int s = 0; s < SETS; s++) w[s].open();
+        const BatchFactor *mine = factors + 8 * (lane >> 5);
+        const int here = groups - Rows::GROUPS * piece;
+        if (rows <= 2) batch_piece<FMT, ROWS, SETS, 1>(w, x, mine, here, tables, acc);
+        else if (rows <= 4) batch_piece<FMT, ROWS, SETS, 2>(w, x, mine, here, tables, acc);
+        else batch_piece<FMT, ROWS, SETS, 4>(w, x, mine, here, tables, acc);
+        if (piece + piece_step < pieces) {
+            const int lane = batch_lane();
+#pragma unroll
+            for (int s = 0; s < SETS; s++) w[s].load(a, tensor[s], e, tile, piece + piece_step, groups, lane);
+        }
+    }
+}
+
+// ---- work items ------------------------------------------------------------------------------------
+struct BatchItem {
+    bool shared;
+    int first, rows;      // the item's rows (expert order; the shared expert's rows follow the pairs)
+    int token0;           // shared expert: the first row's token
+    size_t e;             // where the expert's weights are: its id, or its pool slot
+};
+__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, int tokens, uint32_t tile, BatchItem &it) {
+    const uint32_t count = a.tiles[0];
+    const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[tile];   // {expert, first row, rows, first row within the expert}
+    if (tile >= count) return false;
+    const int expert = (int)entry.x;
+    it.shared = expert == a.experts;
+    it.first = (int)entry.y;
+    it.rows = (int)entry.z;
+    it.token0 = (int)entry.w;
+    it.e = it.shared ? 0 : (size_t)expert;
+    if (a.slots && !it.shared) {   // expert streaming: the rows of an expert share its pool slot
+        uint32_t slot = a.slots[a.row_to_pair[it.first]];
+        if (slot >= a.pool_slots) {
+            if (threadIdx.x == 0) atomicOr(a.error_word, PF_HIP_ERR_BOUNDS);
+            slot = 0;
+        }
+        it.e = slot;
+    }
+    return true;
+}
+
+template <int FMT> __host__ __device__ constexpr bool batch_tables() { return FMT == PF_IQ2_XXS; }
+#define BATCH_TABLE_BYTES 3072
+__device__ __forceinline__ void batch_stage_tables(uint32_t *tables, const PfKernelArgs &a) {
+    for (int i = (int)threadIdx.x; i < 256; i += (int)blockDim.x) reinterpret_cast<uint64_t *>(tables)[i] = a.iq2_grid[i];
+    for (int i = (int)threadIdx.x; i < 128; i += (int)blockDim.x) {
+        const uint32_t bits = (uint32_t)i | (pf_parity7((uint32_t)i) << 7);   // the eighth sign: the others' parity
+        uint32_t lo = 0, hi = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            lo |= ((bits >> j) & 1u ? 255u : 0u) << (8 * j);
+            hi |= ((bits >> (4 + j)) & 1u ? 255u : 0u) << (8 * j);
+        }
+        reinterpret_cast<uint2 *>(tables)[256 + i] = make_uint2(lo, hi);
+    }
+    __syncthreads();
+}
+
+// Lanes 0..31 and 32..63, one value each: group g of two K-vectors' images (store: whether the lane's vector exists).
+__device__ __forceinline__ void batch_image_group(uint32_t *img, float v, int g, int K, int lane, bool store) {
+    float m = fabsf(v);
+#pragma unroll
+    for (int k = 0; k < 4; k++) m = fmaxf(m, __int_as_float(dpp_row_step(__float_as_int(m), k)));
+    m = fmaxf(m, __shfl_xor(m, 16));
+    float step, inv;
+    group_step2(m, step, inv);
+    const int q = __float2int_rn(v * inv);
+    int sum = q;
+#pragma unroll
+    for (int k = 0; k < 4; k++) sum += dpp_row_step(sum, k);
+    sum += __shfl_xor(sum, 16);
+    int d[PF_IMG_PLANES];
+    image_digits(q, d);
+    if (!store) return;
+    uint8_t *bytes = reinterpret_cast<uint8_t *>(img + PF_IMG_GROUP * g);
+#pragma unroll
+    for (int p = 0; p < PF_IMG_PLANES; p++) bytes[32 * p + (lane & 31)] = (uint8_t)d[p];
+    if ((lane & 31) == 0) {
+        img[PF_IMG_GROUP * (K / 32) + g] = __float_as_uint(step);
+        img[(PF_IMG_GROUP + 1) * (K / 32) + g] = (uint32_t)sum;
+    }
+}
+
+// blockIdx.x: 32 units; blockIdx.y: row tile.  The workgroup's waves share K (a 256-block each, in turn); their partial
+// sums meet in LDS and are added in wave order, a wave per pair of rows.
+// Bound by the chain a workgroup lives through (item, weights, products, the same for a second 256-block, sums): three
+// workgroups a compute unit keep 120 KB on their way, 3.9 TB/s of weights at 32 tokens (77 us for 283 MB; the 32-row FP16
+// product took 79, at 101 tokens of the q2 profile 309 against 180).  Measured and left out: eight waves with a block each,
+// two waves with four (both slower), the operands past the registers through LDS (slower: LDS becomes the bottleneck for
+// IQ2_XXS), one matrix a wave at twice the occupancy (85 us).
+#define BATCH_WAVES 4
+template <int FMT, int FMTS, bool ROWS>
+__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(3))) pf_k_batch_gate_up(PfKernelArgs a, int tokens) {
+    __shared__ float partial[BATCH_WAVES][2][4][64];
+    __shared__ BatchFactor factors[BATCH_WAVES][64];
+    __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
+    BatchItem it;
+    if (!batch_item(a, tokens, blockIdx.y, it)) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int tile = blockIdx.x, I = it.shared ? a.shared_inter : a.inter;
+    if (32 * tile >= I) return;
+    if (batch_tables<FMT>()) batch_stage_tables(tables, a);
+    const int groups = a.hidden / 32, K = a.top_k;
+    const uint32_t words = (uint32_t)pf_image2_words(a.hidden);
+    const size_t act_words = pf_image2_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
+        const int rows = min(BATCH_ROWS, it.rows - c0);
+        float acc[2][4] = {};
+        const int tensor[2] = {it.shared ? 4 : 1, it.shared ? 5 : 2};
+        auto image_at = [&](int r) {
+            const uint32_t row = (uint32_t)(c0 + r);
+            return (it.shared ? (uint32_t)it.token0 + row : a.row_to_pair[(uint32_t)it.first + row] / (uint32_t)K) * words;
+        };
+        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS, 2>(a, tensor, 0, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
+        else batch_chunk<FMT, ROWS, 2>(a, tensor, it.e, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
+        const int lane = batch_lane();
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (2 * q < rows) {
+                partial[wave][0][q][lane] = acc[0][q];
+                partial[wave][1][q][lane] = acc[1][q];
+            }
+        __syncthreads();
+        for (int q = wave; 2 * q < rows; q += BATCH_WAVES) {
+            const int lane = batch_lane();
+            float gate = 0.0f, up = 0.0f;
+            for (int w = 0; w < BATCH_WAVES; w++) {
+                gate += partial[w][0][q][lane];
+                up += partial[w][1][q][lane];
+            }
+            const float act = pf_silu(gate) * up;
+            const int r = 2 * q + (lane >> 5);
+            if (r < rows && !pf_finite(act)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
+            batch_image_group(a.aimg + (size_t)(it.first + c0 + min(r, rows - 1)) * act_words, act, tile, I, lane, r < rows);
+        }
+        if (c0 + BATCH_ROWS < it.rows) __syncthreads();   // the sums have been read
+    }
+}
+
+// blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert
+template <int FMT, int FMTS, bool ROWS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, int tokens) {
+    __shared__ BatchFactor factors[4][64];
+    __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
+    BatchItem it;
+    if (!batch_item(a, tokens, blockIdx.y, it)) return;
+    if (batch_tables<FMT>()) batch_stage_tables(tables, a);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), H = a.hidden;
+    const int tile = 4 * blockIdx.x + wave;
+    if (32 * tile >= H) return;
+    const int groups = (it.shared ? a.shared_inter : a.inter) / 32;
+    const uint32_t words = (uint32_t)pf_image2_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
+        const int rows = min(BATCH_ROWS, it.rows - c0);
+        auto image_at = [&](int r) { return (uint32_t)(it.first + c0 + r) * words; };
+        float acc[1][4] = {};
+        const int tensor[1] = {it.shared ? 6 : 3};
+        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS || FMTS == PF_Q8_0, 1>(a, tensor, 0, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
+        else batch_chunk<FMT, ROWS, 1>(a, tensor, it.e, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
+        const int lane = batch_lane();
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int r = 2 * q + (lane >> 5);
+            if (r < rows) a.down[(size_t)(it.first + c0 + r) * H + 32 * tile + (lane & 31)] = acc[0][q];
+        }
+    }
+}
+
+// ---- router ----------------------------------------------------------------------------------------
+// Logits and sums of squared products of 16 tokens against 16 experts a workgroup, on v_mfma_f32_16x16x4_f32; sixteen waves
+// share the columns.  The whole of a wave's part (at most ROUTER_LINES 128-byte lines of 16 + 16 rows) is requested at once:
+// a workgroup waits for memory once, and small tiles spread a few tokens over the chip (a 32 x 32 tile keeps a compute
+// unit's matrix cores busy for 7 us, this one for 2 + 2).  A line goes through the wave's own LDS because a product step
+// wants element k of row i from lane (i, k).  The sums of squares (the routing's tolerance) are products of the squares.
+// The last row of workgroups takes a token a wave: its digit image, and the shared router's logit and sigmoid.
+// Measured at a width of 2560: 101 tokens 37 -> 12.7 us, against the decode kernels' router in groups of four tokens (32
+// tokens of width 2048: 14.0 -> 9.6).
+typedef float float4v __attribute__((ext_vector_type(4)));
+#define ROUTER_LINES 5      // 32-column lines a wave holds: hidden <= 2560
+#define ROUTER_PITCH 36     // floats between rows of a staged line: neighbouring lanes' 16-byte reads cover all banks
+__global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int tokens) {
+    __shared__ __align__(16) float staged[16][2][16 * ROUTER_PITCH];
+    const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (blockIdx.y == gridDim.y - 1) {
+        const int t = 16 * blockIdx.x + wave;
+        if (t >= tokens) return;
+        const float4v *row = reinterpret_cast<const float4v *>(a.x + (size_t)t * a.x_pitch), *gate = reinterpret_cast<const float4v *>(a.w[7]);
+        float z = 0.0f;
+        for (int j = lane; j < H / 8; j += 64) {
+            const float4v p = row[2 * j], q = row[2 * j + 1], u = gate[2 * j], v = gate[2 * j + 1];
+            image2_chunk(a.ximg + (size_t)t * pf_image2_words(H), make_float4(p.x, p.y, p.z, p.w), make_float4(q.x, q.y, q.z, q.w), j, H);
+#pragma unroll
+            for (int c = 0; c < 4; c++) z = fmaf(p[c], u[c], fmaf(q[c], v[c], z));
+        }
+        z = pf_wave_sum(z);
+        if (lane == 0) {
+            a.shared_scale[t] = pf_sigmoid(z);
+            if (!pf_finite(z)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
+        }
+        return;
+    }
+    const int t0 = 16 * blockIdx.x, e0 = 16 * blockIdx.y, lines = H / 32, l0 = lines * wave / 16, l1 = lines * (wave + 1) / 16;
+    const int lr = lane >> 3, piece = lane & 7, i = lane & 15, kk = lane >> 4;
+    float4v xg[ROUTER_LINES][2], wg[ROUTER_LINES][2];
+#pragma unroll
+    for (int l = 0; l < ROUTER_LINES; l++) {
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            const int t = min(t0 + 8 * g + lr, tokens - 1), e = min(e0 + 8 * g + lr, E - 1);
+            if (l0 + l < l1) {
+                xg[l][g] = reinterpret_cast<const float4v *>(a.x + (size_t)t * a.x_pitch)[8 * (l0 + l) + piece];
+                wg[l][g] = reinterpret_cast<const float4v *>(a.w[0] + (size_t)e * H * 4)[8 * (l0 + l) + piece];
+            }
+        }
+    }
+    float *xs = staged[wave][0], *ws = staged[wave][1];
+    float4v acc = {0}, sq = {0};
+#pragma unroll
+    for (int l = 0; l < ROUTER_LINES; l++) {
+        if (l0 + l >= l1) break;
+        pf_wave_lds_fence();
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            *reinterpret_cast<float4v *>(xs + (8 * g + lr) * ROUTER_PITCH + 4 * piece) = xg[l][g];
+            *reinterpret_cast<float4v *>(ws + (8 * g + lr) * ROUTER_PITCH + 4 * piece) = wg[l][g];
+        }
+        pf_wave_lds_fence();
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const float4v x = *reinterpret_cast<const float4v *>(xs + i * ROUTER_PITCH + 16 * c + 4 * kk);
+            const float4v w = *reinterpret_cast<const float4v *>(ws + i * ROUTER_PITCH + 16 * c + 4 * kk);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[k], w[k], acc, 0, 0, 0);
+                sq = __builtin_amdgcn_mfma_f32_16x16x4f32(x[k] * x[k], w[k] * w[k], sq, 0, 0, 0);
+            }
+        }
+    }
+    pf_wave_lds_fence();
+#pragma unroll
+    for (int r = 0; r < 4; r++) { xs[64 * r + lane] = acc[r]; xs[64 * (4 + r) + lane] = sq[r]; }   // the wave's own part of LDS: 512 floats
+    __syncthreads();
+    if (wave >= 8) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 16; w++) sum += staged[w][0][64 * wave + lane];   // register `wave` of every wave, in wave order
+    const int t = t0 + 4 * kk + (wave & 3), e = e0 + i;
+    if (t < tokens && e < E) {
+        (wave < 4 ? a.logits : a.logit_ssq)[(size_t)t * E + e] = sum;
+        // a nonfinite activation makes every product with it nonfinite, and a sum with such a term stays so
+        if (!pf_finite(sum)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
+    }
+}
+
+void pf_launch_batch_router(const PfKernelArgs &a, int tokens, hipStream_t stream) {
+    hipLaunchKernelGGL(pf_k_batch_router, dim3((tokens + 15) / 16, (a.experts + 15) / 16 + 1), dim3(1024), 0, stream, a, tokens);
+}
+
+// ---- dispatch --------------------------------------------------------------------------------------
+template <int FG, int FD, int FS, bool ROWS>
+static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile_cap, hipStream_t stream, int last) {
+    const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
+    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a, tokens);
+    if (last < 4) return;
+    hipLaunchKernelGGL((pf_k_batch_down<FD, FS, ROWS>), dim3((a.hidden + 127) / 128, tile_cap), dim3(256), 0, stream, a, tokens);
+}
+
+template <int FG, int FD, int FS>
+static void launch_batch_experts(const PfKernelArgs &a, int tokens, unsigned tile_cap, hipStream_t stream, int last) {
+    // a layer keeps the tile-ordered copies of its gate and up tensors (and a one-format layer those of its down tensors,
+    // the profiles those of the shared gate and up) or none of them
+    const bool tiled = (FG == PF_Q4_K ? a.wt[1] && a.wt[2] : a.wi[1] && a.wi[2]) && (FS != PF_Q8_0 || (a.wq[4] && a.wq[5]));
+    if (tiled) launch_batch_format<FG, FD, FS, false>(a, tokens, tile_cap, stream, last);
+    else launch_batch_format<FG, FD, FS, true>(a, tokens, tile_cap, stream, last);
+}
+
+void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stream, int last) {
+    // row tiles there can be: an expert with rows has at least one
+    const int pairs = tokens * a.top_k;
+    unsigned cap = (unsigned)pf_prefill_max_tiles(tokens, a.experts, a.top_k), few = (unsigned)(pairs + (tokens + 31) / 32);
+    if (few < cap) cap = few;
+    switch (a.type[1] == PF_Q4_K ? (a.type[3] == PF_Q4_K ? 1 : 4) : (a.type[3] == PF_IQ2_XXS ? 2 : 3)) {
+    case 1: launch_batch_experts<PF_Q4_K, PF_Q4_K, PF_Q4_K>(a, tokens, cap, stream, last); break;
+    case 2: launch_batch_experts<PF_IQ2_XXS, PF_IQ2_XXS, PF_IQ2_XXS>(a, tokens, cap, stream, last); break;
+    case 3: launch_batch_experts<PF_IQ2_XXS, PF_Q2_K, PF_Q8_0>(a, tokens, cap, stream, last); break;
+    default: launch_batch_experts<PF_Q4_K, PF_MXFP4, PF_Q8_0>(a, tokens, cap, stream, last); break;
+    }
+}
+
+void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit) {
+    const int last = stage_limit ? stage_limit : 4;
+    pf_launch_batch_router(a, tokens, stream);
+    if (last < 2) return;
+    pf_launch_dec_route(a, tokens, stream);
+    pf_launch_group(a, a.ids, tokens, stream);
+    if (last < 3) return;
+    pf_launch_batch_experts(a, tokens, stream, last);
+    if (last < 4) return;
+    pf_launch_combine(a, tokens, stream);
+}

@@ -22,6 +22,7 @@
 // and exact; the group scales are applied in FP32 afterwards.  The activation error
 // is at most 2^-21 of the largest magnitude of its group.
 #include "pf_moe_internal.h"
+#include "pf_image.h"
 #include "pf_route_device.h"
 #include "pf_route_fast.h"
 #include "pf_route_fix.h"
@@ -73,9 +74,6 @@ __device__ __forceinline__ void xseg_load(XSeg &s, const int *img, int K, int se
     s.step[0] = steps[2 * seg]; s.step[1] = steps[2 * seg + 1];
     s.sum[0] = sums[2 * seg]; s.sum[1] = sums[2 * seg + 1];
 }
-
-__device__ __forceinline__ int dpp_quad_xor1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true); }
-__device__ __forceinline__ int dpp_quad_xor2(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true); }
 
 // power-of-two step for a group whose largest magnitude is m: |v| / step < 2^20
 __device__ __forceinline__ void group_step(float m, float &step, float &inv) {
@@ -139,104 +137,6 @@ __device__ __forceinline__ bool build_image(int *img, const float *src, int K, i
     for (int j = j0; j < K / 8; j += stride)
         bad |= image_chunk(img, reinterpret_cast<const float4 *>(src)[2 * j], reinterpret_cast<const float4 *>(src)[2 * j + 1], j, K);
     return bad;
-}
-
-// ---- digit images in global memory (kernels whose lanes are weight rows) ------------------------
-// Where every lane of a wave is a weight row, the activation digits are the same for the whole wave and
-// travel through scalar registers: the image lives in global memory (pf_image2_words), written by the
-// kernel before.  PF_IMG_PLANES balanced base-256 digits (signed bytes): the values as integers relative
-// to a step per 32-group that puts the group's largest magnitude at 127 * 256^(planes - 1); the rounding
-// error is at most 2^-24 of that magnitude with three planes.
-#define PF_IMG_TOP (PF_IMG_PLANES == 3 ? 8323072.0f : 32512.0f)   // the integer the group's largest magnitude becomes: 127 * 256^(planes - 1)
-__device__ __forceinline__ void group_step2(float m, float &step, float &inv) {
-    const bool none = !(m > 1e-30f);   // an all-zero (or vanishing) group
-    inv = none ? 0.0f : PF_IMG_TOP / m;
-    step = none ? 0.0f : m * (1.0f / PF_IMG_TOP);
-}
-// balanced base-256 digits of q, lowest first (each in -128..127)
-__device__ __forceinline__ void image_digits(int q, int (&d)[PF_IMG_PLANES]) {
-#pragma unroll
-    for (int p = 0; p + 1 < PF_IMG_PLANES; p++) {
-        d[p] = ((q + 128) & 255) - 128;
-        q = (q - d[p]) >> 8;
-    }
-    d[PF_IMG_PLANES - 1] = q;
-}
-// the integer dot product from its per-plane parts (float: three planes leave 32 bits)
-__device__ __forceinline__ float image_value(const int (&part)[PF_IMG_PLANES]) {
-    float v = (float)part[PF_IMG_PLANES - 1];
-#pragma unroll
-    for (int p = PF_IMG_PLANES - 2; p >= 0; p--) v = fmaf(256.0f, v, (float)part[p]);
-    return v;
-}
-
-// Thread j of a group of four neighbouring lanes: the eight values 8j..8j+7 of a K-vector into its image.
-__device__ __forceinline__ bool image2_chunk(uint32_t *img, const float4 a, const float4 b, int j, int K) {
-    bool bad = false;
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    float m = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 8; c++) { m = fmaxf(m, fabsf(v[c])); bad |= !pf_finite(v[c]); }
-    m = fmaxf(m, __int_as_float(dpp_quad_xor1(__float_as_int(m))));
-    m = fmaxf(m, __int_as_float(dpp_quad_xor2(__float_as_int(m))));
-    float step, inv;
-    group_step2(m, step, inv);
-    uint32_t w[PF_IMG_PLANES][2] = {};
-    int sum = 0;
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const int q = __float2int_rn(v[c] * inv);
-        sum += q;
-        int d[PF_IMG_PLANES];
-        image_digits(q, d);
-#pragma unroll
-        for (int p = 0; p < PF_IMG_PLANES; p++) w[p][c >> 2] |= (uint32_t)(d[p] & 255) << (8 * (c & 3));
-    }
-    sum += dpp_quad_xor1(sum);
-    sum += dpp_quad_xor2(sum);
-    const int g = j >> 2, at = PF_IMG_GROUP * g + 2 * (j & 3);
-#pragma unroll
-    for (int p = 0; p < PF_IMG_PLANES; p++) { img[at + 8 * p] = w[p][0]; img[at + 8 * p + 1] = w[p][1]; }
-    if ((j & 3) == 0) {
-        img[PF_IMG_GROUP * (K / 32) + g] = __float_as_uint(step);
-        img[(PF_IMG_GROUP + 1) * (K / 32) + g] = (uint32_t)sum;
-    }
-    return bad;
-}
-
-// Lanes 0..31 of a wave, one value each: group g of a K-vector's image.
-__device__ __forceinline__ int dpp_row_step(int v, const int which) {
-    switch (which) {
-    case 0: return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);    // quad_perm [1,0,3,2]
-    case 1: return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
-    case 2: return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);   // row_half_mirror
-    default: return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, true);  // row_mirror
-    }
-}
-
-__device__ __forceinline__ void image2_group(uint32_t *img, float v, int g, int K, int lane) {   // lanes 32..63 idle along
-    float m = fabsf(v);
-#pragma unroll
-    for (int k = 0; k < 4; k++) m = fmaxf(m, __int_as_float(dpp_row_step(__float_as_int(m), k)));
-    m = fmaxf(m, __shfl_xor(m, 16));
-    float step, inv;
-    group_step2(m, step, inv);
-    const int q = __float2int_rn(v * inv);
-    int sum = q;
-#pragma unroll
-    for (int k = 0; k < 4; k++) sum += dpp_row_step(sum, k);
-    sum += __shfl_xor(sum, 16);
-    int d[PF_IMG_PLANES];
-    image_digits(q, d);
-    uint8_t *bytes = reinterpret_cast<uint8_t *>(img + PF_IMG_GROUP * g);
-    if (lane < 32) {
-#pragma unroll
-        for (int p = 0; p < PF_IMG_PLANES; p++) bytes[32 * p + lane] = (uint8_t)d[p];
-    }
-    if (lane == 0) {
-        img[PF_IMG_GROUP * (K / 32) + g] = __float_as_uint(step);
-        img[(PF_IMG_GROUP + 1) * (K / 32) + g] = (uint32_t)sum;
-    }
 }
 
 // ---- one lane's 64 weights of a row --------------------------------------------------
@@ -316,10 +216,6 @@ __device__ __forceinline__ void wseg_load<PF_Q2_K>(WSeg<PF_Q2_K> &w, const PfKer
     for (int i = 0; i < 8; i++) w.q[i] = codes[i];
     w.sm = *reinterpret_cast<const uint32_t *>(a.w[t] + sp[1].at);
     w.dd = *reinterpret_cast<const uint32_t *>(a.w[t] + sp[2].at);
-}
-
-__device__ __forceinline__ float half_bits(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (unsigned short)h);
 }
 
 template <int FMT>
@@ -408,16 +304,6 @@ __device__ __forceinline__ float wseg_dot<PF_Q8_0>(const WSeg<PF_Q8_0> &w, const
         out = fmaf(x.step[g] * half_bits((w.d2 >> (16 * g)) & 0xffffu), total, out);
     }
     return out;
-}
-
-// MXFP4: four E2M1 codes of a dword as signed bytes holding twice their value (0, 1, 2, 3, 4, 6, 8, 12):
-// one byte permute per sign, merged under the sign bits' byte mask
-__device__ __forceinline__ int e2m1_twice4(uint32_t nibbles) {
-    const uint32_t sel = nibbles & 0x07070707u;
-    const uint32_t pos = __builtin_amdgcn_perm(0x0C080604u, 0x03020100u, sel);
-    const uint32_t neg = __builtin_amdgcn_perm(0xF4F8FAFCu, 0xFDFEFF00u, sel);
-    const uint32_t mask = ((nibbles >> 3) & 0x01010101u) * 0xFFu;
-    return (int)((neg & mask) | (pos & ~mask));
 }
 
 template <>
@@ -1103,8 +989,7 @@ __device__ __forceinline__ void q4t_route_fix(const float *router, const float *
 }
 
 // FMT: format of the routed gate and up tensors, FMTS: of the shared expert's (the same, or the profiles' Q8_0);
-// POOL: the routed tensors sit in pool slots (expert streaming)
-template <int NPL, int FMT, int FMTS, bool POOL>
+template <int NPL, int FMT, int FMTS>
 __device__ __forceinline__ void q4t_gate_up(PfKernelArgs &a, int routed_blocks) {
     extern __shared__ int lds[];
     __shared__ RouteLds R;
@@ -1158,19 +1043,8 @@ __device__ __forceinline__ void q4t_gate_up(PfKernelArgs &a, int routed_blocks) 
     if (!shared || FMT == PF_IQ2_XXS) __syncthreads();   // the early expert; the tables
     const uint32_t early = shared ? 0u : early_expert;
     const bool early_ok = early < (uint32_t)E;   // a nonfinite logit can leave no maximum: the error word says so below
-    // Expert streaming: the slot's expert was routed by an earlier launch and sits in pool slot slots[u]; the tile is
-    // read there, whatever the early guess says, and the routing below only has to agree with the ids it was fetched by.
-    constexpr bool pooled = POOL;
-    uint32_t pooled_at = 0u;
-    if (pooled && !shared) {
-        pooled_at = a.slots[u];
-        if (pooled_at >= a.pool_slots) {
-            if (threadIdx.x == 0) atomicOr(a.error_word, PF_HIP_ERR_BOUNDS);
-            pooled_at = 0u;
-        }
-    }
     if (shared) q4t_tile<FMTS>(a, plan, partial, tables, 0u, wave);
-    else q4t_tile<FMT>(a, plan, partial, tables, pooled ? pooled_at : early_ok ? early : 0u, wave);
+    else q4t_tile<FMT>(a, plan, partial, tables, early_ok ? early : 0u, wave);
     if (wave == 0 && !shared) {
         // the remaining slots, the candidate beyond them and one more key, while the other waves' weight bytes travel
         for (int r = u + 1; r <= rounds; r++) {
@@ -1199,7 +1073,7 @@ __device__ __forceinline__ void q4t_gate_up(PfKernelArgs &a, int routed_blocks) 
         // the slot's expert in the final order (the early guess came from truncated keys; the serial-order routing
         // can name another expert)
         e = R.ids[u];
-        if (!pooled && e != early && e < (uint32_t)E) {
+        if (e != early && e < (uint32_t)E) {
             __syncthreads();
             q4t_tile<FMT>(a, plan, partial, tables, e, wave);
             __syncthreads();
@@ -1208,7 +1082,6 @@ __device__ __forceinline__ void q4t_gate_up(PfKernelArgs &a, int routed_blocks) 
             // publish the routes for the next kernel and the caller (one token: slot = pair = unique expert)
             if (R.close[0] == 0) __syncthreads();   // R.bad above; route_finish ends with a barrier of its own
             for (int q = threadIdx.x; q < K; q += blockDim.x) {
-                if (pooled && a.ids[q] != R.ids[q]) atomicOr(a.error_word, PF_HIP_ERR_BOUNDS);   // not the experts that were fetched
                 a.ids[q] = R.ids[q];
                 a.route_weights[q] = R.weights[q];
                 if (gridDim.y == 1) {   // the table of unique experts: read by the other down kernel, which runs after this one only for one token
@@ -1249,9 +1122,9 @@ __device__ __forceinline__ void q4t_gate_up(PfKernelArgs &a, int routed_blocks) 
 
 // With several tokens there are more workgroups than compute units; two workgroups per compute unit (64 registers a
 // lane) measured slower than one after the other: the products are bound by the vector units, not by waiting.
-template <int NPL, int FMT, int FMTS, bool POOL>
+template <int NPL, int FMT, int FMTS>
 __global__ void __launch_bounds__(1024) pf_k_dec_gate_up_q4t(PfKernelArgs a, int routed_blocks) {
-    q4t_gate_up<NPL, FMT, FMTS, POOL>(a, routed_blocks);
+    q4t_gate_up<NPL, FMT, FMTS>(a, routed_blocks);
 }
 
 // ---- several tokens: routing in a launch of its own, then kernel 2 without it -----------------------------------
@@ -1297,23 +1170,24 @@ __global__ void __launch_bounds__(1024) pf_k_dec_route(PfKernelArgs a) {
     }
 }
 
-#define Q4G_WAVES 8    // all of them share the row's 64-weight runs,
+#define Q4G_WAVES 10   // at most; all of them share the row's 64-weight runs,
 #define Q4G_ITEMS 4    // this many a wave: hidden <= 64 * Q4G_ITEMS * Q4G_WAVES
+static int q4g_waves(int hidden) { return (hidden / 64 + Q4G_ITEMS - 1) / Q4G_ITEMS; }   // 8 for a hidden width of 2048, 10 for 2560
 template <int FMT>
-__device__ __forceinline__ void q4g_tile(const PfKernelArgs &a, const Q4TilePlan &p, float *partial, const uint32_t *tables, uint32_t e, int wave) {
+__device__ __forceinline__ void q4g_tile(const PfKernelArgs &a, const Q4TilePlan &p, float *partial, const uint32_t *tables, uint32_t e, int wave, int waves) {
     const int lane = pf_lane();
     const uint8_t *tile = p.base + (size_t)e * p.expert_bytes;
     const PfScalarWords image = (PfScalarWords)(uintptr_t)a.ximg;
     TileItem<FMT> w[Q4G_ITEMS];
 #pragma unroll
     for (int k = 0; k < Q4G_ITEMS; k++) {
-        const int it = wave + Q4G_WAVES * k;
+        const int it = wave + waves * k;
         if (it < p.items) q4t_load(w[k], tile + TileGeometry<FMT>::chunk_at(0, p.kblocks, it >> 2), p.row, it & 3);
     }
     float total = 0.0f;
 #pragma unroll
     for (int k = 0; k < Q4G_ITEMS; k++) {
-        const int it = wave + Q4G_WAVES * k;
+        const int it = wave + waves * k;
         if (it < p.items) {
             const int g = 2 * it;
             total += q4t_dot(w[k], image + PF_IMG_GROUP * g, image + PF_IMG_GROUP * p.groups + g, image + (PF_IMG_GROUP + 1) * p.groups + g,
@@ -1323,18 +1197,19 @@ __device__ __forceinline__ void q4g_tile(const PfKernelArgs &a, const Q4TilePlan
     partial[wave * 64 + lane] = total;
 }
 
-template <int FMT, int FMTS>
+// POOL: the routed tensors sit in pool slots (expert streaming; the routing ran before the slots were filled)
+template <int FMT, int FMTS, bool POOL>
 __global__ void __launch_bounds__(64 * Q4G_WAVES) __attribute__((amdgpu_waves_per_eu(8))) pf_k_dec_gate_up_given(PfKernelArgs a, int routed_blocks) {
     extern __shared__ int lds[];
     q4t_at_token(a, (int)blockIdx.y);
     const int K = a.top_k, lane = pf_lane();
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = (int)blockDim.x >> 6;
     uint32_t *tables = reinterpret_cast<uint32_t *>(lds);
     if (FMT == PF_IQ2_XXS) {
         const uint4 *src = reinterpret_cast<const uint4 *>(a.iq2_signed);
-        for (int i = (int)threadIdx.x; i < 2048; i += 64 * Q4G_WAVES) reinterpret_cast<uint4 *>(tables)[i] = src[i];
+        for (int i = (int)threadIdx.x; i < 2048; i += 64 * waves) reinterpret_cast<uint4 *>(tables)[i] = src[i];
     }
-    float *partial = reinterpret_cast<float *>(lds + table_words<FMT>());   // [Q4G_WAVES][64 lanes]
+    float *partial = reinterpret_cast<float *>(lds + table_words<FMT>());   // [waves][64 lanes]
     const bool shared = (int)blockIdx.x >= routed_blocks;
     const int tiles = a.inter / 32;
     const int u = shared ? K : (int)blockIdx.x / tiles;
@@ -1346,14 +1221,21 @@ __global__ void __launch_bounds__(64 * Q4G_WAVES) __attribute__((amdgpu_waves_pe
         if (threadIdx.x == 0) atomicOr(a.error_word, PF_HIP_ERR_BOUNDS | PF_HIP_ERR_NONFINITE);
         e = 0u;
     }
+    if (POOL && !shared) {
+        e = ((PfScalarWords)(uintptr_t)a.slots)[u];
+        if (e >= a.pool_slots) {
+            if (threadIdx.x == 0) atomicOr(a.error_word, PF_HIP_ERR_BOUNDS);
+            e = 0u;
+        }
+    }
     const Q4TilePlan plan = shared ? q4t_plan<FMTS>(a, true, n0) : q4t_plan<FMT>(a, false, n0);
     if (FMT == PF_IQ2_XXS) __syncthreads();   // the tables
-    if (shared) q4g_tile<FMTS>(a, plan, partial, tables, 0u, wave);
-    else q4g_tile<FMT>(a, plan, partial, tables, e, wave);
+    if (shared) q4g_tile<FMTS>(a, plan, partial, tables, 0u, wave, waves);
+    else q4g_tile<FMT>(a, plan, partial, tables, e, wave, waves);
     __syncthreads();
     if (wave == 0) {
         float sum = 0.0f;
-        for (int w = 0; w < Q4G_WAVES; w++) sum += partial[w * 64 + lane];
+        for (int w = 0; w < waves; w++) sum += partial[w * 64 + lane];
         const float up = __shfl(sum, (lane & 31) + 32);
         const float act = pf_silu(sum) * up;
         const size_t widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
@@ -1375,7 +1257,8 @@ static void launch_dec_route_lists(const PfKernelArgs &a, int tokens, size_t lds
     hipLaunchKernelGGL((pf_k_dec_route<NPL>), dim3(tokens), dim3(1024), lds, stream, a);
 }
 
-static void launch_dec_route(const PfKernelArgs &a, int tokens, hipStream_t stream) {
+#if PF_DECODE_PART == 0
+void pf_launch_dec_route(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     const size_t lds = pf_route_fix_lds_floats(a.hidden, a.experts) * 4;
     const int all = (a.experts + 63) / 64;
     if (all <= 1) launch_dec_route_lists<1>(a, tokens, lds, stream);
@@ -1384,12 +1267,14 @@ static void launch_dec_route(const PfKernelArgs &a, int tokens, hipStream_t stre
     else if (all <= 8) launch_dec_route_lists<8>(a, tokens, lds, stream);
     else launch_dec_route_lists<16>(a, tokens, lds, stream);
 }
+#endif
 
-template <int FMT, int FMTS>
+template <int FMT, int FMTS, bool POOL>
 static void launch_gate_up_given(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     const int routed_blocks = a.top_k * (a.inter / 32);
-    const size_t lds = (size_t)table_words<FMT>() * 4 + (size_t)Q4G_WAVES * 64 * 4;
-    hipLaunchKernelGGL((pf_k_dec_gate_up_given<FMT, FMTS>), dim3(routed_blocks + a.shared_inter / 32, tokens), dim3(64 * Q4G_WAVES), lds, stream, a,
+    const int waves = q4g_waves(a.hidden);
+    const size_t lds = (size_t)table_words<FMT>() * 4 + (size_t)waves * 64 * 4;
+    hipLaunchKernelGGL((pf_k_dec_gate_up_given<FMT, FMTS, POOL>), dim3(routed_blocks + a.shared_inter / 32, tokens), dim3(64 * waves), lds, stream, a,
                        routed_blocks);
 }
 
@@ -1405,29 +1290,29 @@ static bool q4t_gate_up_applies(const PfKernelArgs &a) {
            a.top_k < a.experts && a.top_k <= 15 && a.experts <= 1024;
 }
 
-template <int NPL, int FMT, int FMTS, bool POOL>
+template <int NPL, int FMT, int FMTS>
 static void launch_gate_up_q4t_lists(const PfKernelArgs &a, dim3 grid, size_t lds, hipStream_t stream, int routed_blocks) {
     static bool configured = false;   // once per instantiation: more than the default 64 KB of dynamic LDS (the re-route's chunk buffers)
     if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_dec_gate_up_q4t<NPL, FMT, FMTS, POOL>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_dec_gate_up_q4t<NPL, FMT, FMTS>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);   // the kernel has static LDS too
         configured = true;
     }
-    hipLaunchKernelGGL((pf_k_dec_gate_up_q4t<NPL, FMT, FMTS, POOL>), grid, dim3(1024), lds, stream, a, routed_blocks);
+    hipLaunchKernelGGL((pf_k_dec_gate_up_q4t<NPL, FMT, FMTS>), grid, dim3(1024), lds, stream, a, routed_blocks);
 }
 
-template <int FMT, int FMTS, bool POOL = false>
+template <int FMT, int FMTS>
 static void launch_gate_up_q4t(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     const int H = a.hidden, I = a.inter, Is = a.shared_inter, E = a.experts, K = a.top_k;
     const int routed_blocks = K * (I / 32);
     const dim3 g1(routed_blocks + Is / 32, tokens);
     const int all = (E + 63) / 64;
     const size_t lds = (size_t)table_words<FMT>() * 4 + (size_t)15 * 64 * 4 + pf_route_fix_lds_floats(H, E) * 4;
-    if (all <= 1) launch_gate_up_q4t_lists<1, FMT, FMTS, POOL>(a, g1, lds, stream, routed_blocks);
-    else if (all <= 2) launch_gate_up_q4t_lists<2, FMT, FMTS, POOL>(a, g1, lds, stream, routed_blocks);
-    else if (all <= 4) launch_gate_up_q4t_lists<4, FMT, FMTS, POOL>(a, g1, lds, stream, routed_blocks);
-    else if (all <= 8) launch_gate_up_q4t_lists<8, FMT, FMTS, POOL>(a, g1, lds, stream, routed_blocks);
-    else launch_gate_up_q4t_lists<16, FMT, FMTS, POOL>(a, g1, lds, stream, routed_blocks);
+    if (all <= 1) launch_gate_up_q4t_lists<1, FMT, FMTS>(a, g1, lds, stream, routed_blocks);
+    else if (all <= 2) launch_gate_up_q4t_lists<2, FMT, FMTS>(a, g1, lds, stream, routed_blocks);
+    else if (all <= 4) launch_gate_up_q4t_lists<4, FMT, FMTS>(a, g1, lds, stream, routed_blocks);
+    else if (all <= 8) launch_gate_up_q4t_lists<8, FMT, FMTS>(a, g1, lds, stream, routed_blocks);
+    else launch_gate_up_q4t_lists<16, FMT, FMTS>(a, g1, lds, stream, routed_blocks);
 }
 
 // ---- kernel 3: down products and the combine ---------------------------------------------------
@@ -2559,9 +2444,10 @@ static PfHipMoeDesc desc_of(const PfKernelArgs &a) {
 #ifndef PF_ROUTE_FIRST_FROM
 #define PF_ROUTE_FIRST_FROM 3
 #endif
-template <bool POOL>
+// (wider than eight waves' items: workgroups of ten waves, three a compute unit instead of four -- at 2560, from five tokens
+// on: 5 tokens 65.9 -> 62.8 us, 16 tokens 173 -> 154, but 3 correlated ones 41.8 -> 46.9)
 static bool routes_first(const PfKernelArgs &a, int tokens) {
-    return !POOL && tokens >= PF_ROUTE_FIRST_FROM && a.hidden <= 64 * Q4G_ITEMS * Q4G_WAVES && a.top_k <= 15;
+    return tokens >= (a.hidden > 64 * Q4G_ITEMS * 8 ? PF_ROUTE_FIRST_FROM + 2 : PF_ROUTE_FIRST_FROM) && a.hidden <= 64 * Q4G_ITEMS * Q4G_WAVES && a.top_k <= 15;
 }
 
 template <int FG, int FD, int FS, bool POOL = false>
@@ -2569,13 +2455,15 @@ static void launch_q4t_experts(const PfKernelArgs &a, int tokens, hipStream_t st
     const int H = a.hidden, I = a.inter, Is = a.shared_inter, K = a.top_k;
     // kernel 2: every workgroup extracts the maxima up to its own slot from all of its token's logits; with several
     // tokens the routing runs first, in a launch of its own
-    if (routes_first<POOL>(a, tokens)) {   // four launches: `last` counts them
-        launch_dec_route(a, tokens, stream);
+    if (POOL) {   // routed by an earlier call, and the slots filled since
+        launch_gate_up_given<FG, FS, true>(a, tokens, stream);
+    } else if (routes_first(a, tokens)) {   // four launches: `last` counts them
+        pf_launch_dec_route(a, tokens, stream);
         if (last < 3) return;
-        launch_gate_up_given<FG, FS>(a, tokens, stream);
+        launch_gate_up_given<FG, FS, false>(a, tokens, stream);
         if (last < 4) return;
     } else {
-        launch_gate_up_q4t<FG, FS, POOL>(a, tokens, stream);
+        launch_gate_up_q4t<FG, FS>(a, tokens, stream);
         if (last < 3) return;
     }
     if constexpr (!POOL && (FD == PF_Q4_K || FD == PF_IQ2_XXS) && (FS == PF_Q4_K || FS == PF_IQ2_XXS)) {
@@ -2706,7 +2594,7 @@ void pf_launch_decode_stream_experts(const PfKernelArgs &a, int tokens, hipStrea
 
 int pf_decode_launches(const PfKernelArgs &a, int tokens) {
     const int combination = pf_decode_tile_layer(desc_of(a), a.wt, a.wi, a.wq);
-    if (tokens != 1) return combination != 0 && routes_first<false>(a, tokens) ? 4 : 3;
+    if (tokens != 1) return combination != 0 && routes_first(a, tokens) ? 4 : 3;
     if (combination == 1) return fused_applies<PF_Q4_K>(a) ? 2 : 3;
     if (combination == 2) return fused_applies<PF_IQ2_XXS>(a) ? 2 : 3;
     return 3;

@@ -6,6 +6,8 @@
 #define PF_DECODE_MAX_TOKENS 4
 #define PF_TILE_DECODE_MAX_TOKENS 16   // Q4_K layers whose tile-ordered copies are kept: one token per grid row
 
+#define PF_BATCH_MAX_TOKENS 400        // the kernels for a few rows per expert (pf_moe_batch.hip)
+
 // Everything a kernel needs, passed by value.  Weight index order is
 // Qwen4MoeWeights': router, gate, up, down, shared gate/up/down, shared router.
 struct PfKernelArgs {
@@ -54,6 +56,7 @@ struct PfKernelArgs {
     const float *w_norm2;            // [experts] squared norm of each router row
     float *down;                     // [pairs + tokens, hidden] down products in expert order, then the shared expert's
     uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles;
+    const uint32_t *items;           // row tiles as {expert, first row, rows, first row within the expert} (pf_k_group_fused)
     // injection into hyper-connection streams in place of writing y (null: y is written)
     float *hc_residual;              // [tokens, streams, hidden], pitches in floats
     const float *hc_inject;          // [tokens, streams], dense
@@ -136,7 +139,7 @@ struct PfHipWork {
     uint32_t *ids, *uniq, *error_word, *exact_rows, *route_flags, *slots, *fuse_lines, *fuse_gen;
     uint16_t *x16, *act16, *sact16;  // prefill buffers (allocated when cap exceeds the decode path's batch)
     float *x_scale, *act_scale, *sact_scale, *x_max2, *down;
-    uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles;
+    uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles, *items;
     uint8_t *host;                  // pinned host block for the host-pointer forwards of short batches (null: not available)
     uint8_t *host_device;           // the same block as the kernels address it (they write the output rows straight into it)
     uint8_t *ring;                  // page-locked pieces behind the block, for host-pointer forwards of longer batches (null: none)
@@ -159,7 +162,7 @@ int pf_route_exact_device(const float *d_logits, int tokens, int experts, int to
 // histogram, scan, row tiles and placement (an expert's rows in no particular order) in one launch; false (nothing
 // launched) for more pairs or experts than it takes
 bool pf_launch_group_fused(const uint32_t *d_ids, int pairs, int experts, int tokens, uint32_t *d_offsets, uint32_t *d_tiles,
-                           uint32_t *d_pair_to_row, uint32_t *d_row_to_pair, hipStream_t stream);
+                           uint32_t *d_items, uint32_t *d_pair_to_row, uint32_t *d_row_to_pair, hipStream_t stream);
 void pf_launch_group_place(const uint32_t *d_ids, int pairs, int experts, const uint32_t *d_offsets,
                            uint32_t *d_pair_to_row, uint32_t *d_row_to_pair, hipStream_t stream);
 int pf_group_pairs_device(const uint32_t *d_ids, int tokens, int experts, int top_k, uint32_t *d_counts,
@@ -192,6 +195,7 @@ void pf_launch_dec_router(const PfKernelArgs &a, int tokens, int router_blocks, 
 // bytes of the activation lines a workspace needs for the one-launch expert stage of a one-token forward (0: the
 // layer's shape or formats are not taken)
 void pf_decode_fused_scratch(const PfHipMoeDesc &d, size_t *line_bytes);
+void pf_launch_dec_route(const PfKernelArgs &a, int tokens, hipStream_t stream);
 // launches per forward on the decode path: 2 for one token with the fused expert stage, 4 where the routing runs in a
 // launch of its own (three tokens or more on the tile kernels), else 3
 int pf_decode_launches(const PfKernelArgs &a, int tokens);
@@ -205,10 +209,16 @@ void pf_launch_block_split(const uint8_t *d_gguf, uint8_t *d_payload, uint8_t *d
 // pf_moe_prefill.hip
 bool pf_prefill_supported(const PfHipMoeDesc &d);
 void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
+void pf_launch_group(const PfKernelArgs &a, const uint32_t *ids, int tokens, hipStream_t stream);
+void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream);
 void pf_launch_q4k_tile(const uint8_t *d_src, uint8_t *d_dst, size_t rows, int blocks_per_row, hipStream_t stream);
 void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hipStream_t stream);
 size_t pf_prefill_half_row(int cols);   // halfs per row of the fp16 form of a matrix with `cols` columns
 int pf_prefill_max_tiles(int tokens, int experts, int top_k);
+// pf_moe_batch.hip: a few rows per expert, for the layers of the tile decode kernels
+void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
+void pf_launch_batch_router(const PfKernelArgs &a, int tokens, hipStream_t stream);
+void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stream, int last);
 // pf_moe_hc.hip
 void pf_launch_hc_read(const float *d_normed, size_t n_token_pitch, size_t n_stream_pitch, const float *d_logits,
                        size_t g_token_pitch, size_t g_stream_pitch, float *d_mixed, size_t m_pitch, int tokens,

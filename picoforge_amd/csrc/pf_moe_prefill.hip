@@ -1329,6 +1329,18 @@ static void launch_gemm_plain(const PfKernelArgs &a, int tokens, unsigned tile_c
     hipLaunchKernelGGL(pf_k_pf_gemm_plain<MODE>, dim3(tile_cap * slabs), dim3(256), PLAIN_LDS, stream, a, tokens, slabs, split);
 }
 
+// the pairs by expert: offsets, row tiles, pair <-> row
+void pf_launch_group(const PfKernelArgs &a, const uint32_t *ids, int tokens, hipStream_t stream) {
+    const int E = a.experts, P = tokens * a.top_k;
+    if (pf_launch_group_fused(ids, P, E, tokens, a.offsets, a.tiles, const_cast<uint32_t *>(a.items), a.pair_to_row, a.row_to_pair, stream)) return;
+    hipLaunchKernelGGL(pf_k_pf_count, dim3((P + 255) / 256), dim3(256), 0, stream, ids, P, E, a.counts);
+    hipLaunchKernelGGL(pf_k_pf_scan_tiles, dim3(1), dim3(256), 0, stream, a.counts, E, tokens, a.offsets, a.tiles);
+    pf_launch_group_place(ids, P, E, a.offsets, a.pair_to_row, a.row_to_pair, stream);
+}
+void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream) {
+    hipLaunchKernelGGL(pf_k_pf_combine, dim3(tokens), dim3(256), 0, stream, a, tokens);
+}
+
 void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit) {
     const int H = a.hidden, E = a.experts, K = a.top_k, I = a.inter, Is = a.shared_inter, P = tokens * K;
     const int last = stage_limit ? stage_limit : 4;
@@ -1341,11 +1353,7 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     if (last < 2) return;
     // stage 2: routes and grouping
     pf_launch_route(a, tokens, stream);
-    if (!pf_launch_group_fused(a.ids, P, E, tokens, a.offsets, a.tiles, a.pair_to_row, a.row_to_pair, stream)) {
-        hipLaunchKernelGGL(pf_k_pf_count, dim3((P + 255) / 256), dim3(256), 0, stream, a.ids, P, E, a.counts);
-        hipLaunchKernelGGL(pf_k_pf_scan_tiles, dim3(1), dim3(256), 0, stream, a.counts, E, tokens, a.offsets, a.tiles);
-        pf_launch_group_place(a.ids, P, E, a.offsets, a.pair_to_row, a.row_to_pair, stream);
-    }
+    pf_launch_group(a, a.ids, tokens, stream);
     if (last < 3) return;
     // stage 3: gate/up + SwiGLU, then fp16 parts of the activation rows
     // the ring kernel takes the items whose tensors are in the routed gate's format, the plain kernel the rest
@@ -1373,5 +1381,5 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
         else launch_gemm<PF_GEMM_DOWN, PF_Q4_K>(a, tokens, (H + 64 * NW - 1) / (64 * NW), stream);
     }
     if (a.type[3] != ring_fmt || a.type[6] != ring_fmt) launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, tile_cap, (H + 255) / 256, 0, stream);
-    hipLaunchKernelGGL(pf_k_pf_combine, dim3(tokens), dim3(256), 0, stream, a, tokens);
+    pf_launch_combine(a, tokens, stream);
 }

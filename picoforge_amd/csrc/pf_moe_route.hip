@@ -377,7 +377,7 @@ void pf_launch_group_place(const uint32_t *d_ids, int pairs, int experts, const 
 
 // ---- grouping in one launch (the prefill path) ---------------------------------------------------------
 // One workgroup of 1024 threads: counts the pairs per expert in LDS, scans the counts (offsets, and the row tiles:
-// tiles[0] = count, tiles[1 + i] = expert | tile index << 16; the shared expert = expert E with every token, as
+// tiles[0] = count, tiles[1 + i] = expert | tile index << 16, items[i] = {expert, first row, rows, first row within the expert}; the shared expert = expert E with every token, as
 // pf_k_pf_scan_tiles lists them), and hands every pair the next free row of its expert through an LDS cursor.  The rows
 // of an expert are therefore in no particular order (pf_k_group_place keeps them in pair order): every row of the
 // grouped products is computed on its own and found again through pair_to_row, so the order changes no result, and a
@@ -385,7 +385,7 @@ void pf_launch_group_place(const uint32_t *d_ids, int pairs, int experts, const 
 #define GROUP_FUSED_MAX_PAIRS 32768
 #define GROUP_FUSED_MAX_EXPERTS 2047
 __global__ void __launch_bounds__(1024) pf_k_group_fused(const uint32_t *ids, int pairs, int E, int tokens, uint32_t *offsets,
-                                                         uint32_t *tiles, uint32_t *pair_to_row, uint32_t *row_to_pair) {
+                                                         uint32_t *tiles, uint4 *items, uint32_t *pair_to_row, uint32_t *row_to_pair) {
     extern __shared__ __align__(16) uint32_t fused_lds[];
     __shared__ uint32_t wave_rows[16], wave_tiles[16];
     const int tid = threadIdx.x, quads = pairs / 4;
@@ -434,9 +434,12 @@ __global__ void __launch_bounds__(1024) pf_k_group_fused(const uint32_t *ids, in
         if (e < E) {
             cursor[e] = row;
             offsets[e] = row;
-            row += c;
         }
-        for (uint32_t i = 0; i < n; i++) tiles[1 + at + i] = (uint32_t)e | (i << 16);
+        for (uint32_t i = 0; i < n; i++) {
+            tiles[1 + at + i] = (uint32_t)e | (i << 16);
+            items[at + i] = make_uint4((uint32_t)e, (e < E ? row : (uint32_t)pairs) + 32u * i, min(32u, c - 32u * i), 32u * i);
+        }
+        if (e < E) row += c;
         at += n;
     }
     __syncthreads();
@@ -454,11 +457,11 @@ __global__ void __launch_bounds__(1024) pf_k_group_fused(const uint32_t *ids, in
 }
 
 bool pf_launch_group_fused(const uint32_t *d_ids, int pairs, int experts, int tokens, uint32_t *d_offsets, uint32_t *d_tiles,
-                           uint32_t *d_pair_to_row, uint32_t *d_row_to_pair, hipStream_t stream) {
+                           uint32_t *d_items, uint32_t *d_pair_to_row, uint32_t *d_row_to_pair, hipStream_t stream) {
     if (pairs <= 0 || pairs > GROUP_FUSED_MAX_PAIRS || experts > GROUP_FUSED_MAX_EXPERTS || (reinterpret_cast<uintptr_t>(d_ids) & 15)) return false;
     const size_t lds = 2 * ((size_t)experts + 1) * sizeof(uint32_t);
     hipLaunchKernelGGL(pf_k_group_fused, dim3(1), dim3(1024), lds, stream, d_ids, pairs, experts, tokens, d_offsets, d_tiles,
-                       d_pair_to_row, d_row_to_pair);
+                       reinterpret_cast<uint4 *>(d_items), d_pair_to_row, d_row_to_pair);
     return true;
 }
 

@@ -1,0 +1,38 @@
+"""GPU parity of the kernels for a few rows per expert (pf_moe_batch.hip) against the CPU oracle: batches that give an
+expert one row, one chunk of eight, ragged chunks and several 32-row tiles, in every format combination, at widths that
+are whole 256-blocks and at widths whose last piece is short."""
+import numpy as np
+import pytest
+
+import picoforge_amd as pf
+from picoforge_amd import abi
+
+from helpers import assert_parity, forward_with, make_layer_inputs
+
+pytestmark = pytest.mark.gpu
+
+# (h, e, k, i, s, down stored, expert type, batches): the batch sizes are on both sides of a chunk (8 rows), of a row tile
+# (32) and of a router tile (16 tokens by 16 experts)
+CASES = [
+    (512, 32, 6, 256, 256, None, abi.GGUF_Q4_K, (33, 48, 177)), (512, 32, 6, 256, 256, None, abi.GGUF_IQ2_XXS, (33, 48, 177)),
+    (2560, 40, 3, 512, 256, None, abi.GGUF_Q4_K, (35, 113)), (2048, 200, 10, 512, 512, None, abi.GGUF_IQ2_XXS, (47, 97)),
+    (512, 32, 6, 256, 256, None, "q2", (11, 16, 17, 177)), (512, 32, 6, 256, 256, None, "q4", (17, 31, 177)),
+    (1280, 24, 4, 320, 320, 512, "q2", (12, 33, 160)), (768, 24, 3, 384, 448, None, "q4", (18, 33, 160)),
+    (2560, 90, 10, 640, 640, 768, "q2", (13, 65)), (2560, 90, 10, 640, 640, None, "q4", (19, 65)),
+]
+
+
+@pytest.mark.parametrize("h,e,k,i,s,physical,fmt,batches", CASES)
+def test_batches_of_a_few_rows_per_expert(product, oracle, h, e, k, i, s, physical, fmt, batches):
+    print(f"case batch {fmt} h={h} e={e} k={k} i={i} s={s} down stored {physical or i} wide", flush=True)
+    cfg = abi.moe_config(h, e, k, i, s, down_physical=physical)
+    most = max(batches)
+    weights, x = make_layer_inputs(cfg, fmt, most, seed=h + e + i)
+    x[5:10] = x[4]                                # tokens that share every expert
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, most) as layer:
+        for tokens in batches:
+            print(f"  tokens={tokens}", flush=True)
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
+        np.testing.assert_array_equal(y, layer.forward(x[:tokens])[1], err_msg="not deterministic")
