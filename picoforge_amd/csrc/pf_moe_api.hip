@@ -396,7 +396,6 @@ extern "C" void pf_hip_moe_destroy(PfHipMoe *m) {
 extern "C" size_t pf_hip_moe_bytes(const PfHipMoe *m) { return m ? m->total_bytes : 0; }
 
 // workspace layout: buffers carved from one allocation, each 256-byte aligned
-// (the error word, the ids and the route weights follow each other: a short batch's are fetched by one copy)
 enum { W_LOGITS, W_SSQ, W_ERR, W_IDS, W_RW, W_ACT, W_SACT, W_SSCALE, W_X, W_Y, W_SLOTS, W_UNIQ, W_EXACT, W_FLAGS, W_XIMG, W_AIMG,
        W_FLINES, W_FGEN, W_X16, W_ACT16, W_SACT16, W_XSCALE, W_ACTSCALE, W_SACTSCALE, W_XMAX2, W_DOWN, W_COUNTS, W_OFFSETS,
        W_P2R, W_R2P, W_GROUPBAD, W_TILES, W_ITEMS, W_COUNT };
@@ -485,57 +484,88 @@ extern "C" size_t pf_hip_work_bytes(const PfHipMoeDesc *desc, size_t token_cap) 
 
 static void carve_work(PfHipWork *w, const Carve &c, uint8_t *base);
 
-// The pinned block of a workspace: a head that mirrors the workspace from the error word to the route weights of a short
-// batch (one copy brings all three when that span is at most PF_HOST_HEAD_BYTES; ids and weights have places of their
-// own for workspaces of more tokens), then input rows, output rows and pool slots of up to PF_HOST_BLOCK_TOKENS
-// tokens, each part 256-byte aligned.  The kernels write the output rows straight into the block.
+// The pinned block of a workspace: the error word, then input rows, output rows, ids, route weights and pool slots of up to
+// PF_HOST_BLOCK_TOKENS tokens and the number of the call whose results they are, each part 256-byte aligned.  The kernels
+// write the output rows straight into the block.
 #define PF_HOST_BLOCK_TOKENS PF_TILE_DECODE_MAX_TOKENS
-#define PF_HOST_HEAD_BYTES (32 * 1024)
+#define PF_HOST_HEAD_BYTES 256
 struct HostBlock {
     uint8_t *head;
     uint32_t *ids, *slots;
     float *x, *y, *weights;
-    size_t y_offset, bytes;
+    uint32_t *published;   // the number of the call whose results are in the block
+    size_t x_offset, y_offset, slots_offset, published_offset, ids_offset, weights_offset, bytes;
 };
 static HostBlock host_block(const PfHipMoeDesc *d, uint8_t *base) {
     const size_t T = PF_HOST_BLOCK_TOKENS, rows = (T * d->hidden * 4 + 255) & ~(size_t)255, pairs = (T * d->top_k * 4 + 255) & ~(size_t)255;
     HostBlock b;
     size_t at = 0;
     b.head = base + at; at += PF_HOST_HEAD_BYTES;
+    b.x_offset = at;
     b.x = (float *)(base + at); at += rows;
     b.y_offset = at;
     b.y = (float *)(base + at); at += rows;
+    b.ids_offset = at;
     b.ids = (uint32_t *)(base + at); at += pairs;
+    b.weights_offset = at;
     b.weights = (float *)(base + at); at += pairs;
+    b.slots_offset = at;
     b.slots = (uint32_t *)(base + at); at += pairs;
+    b.published_offset = at;
+    b.published = (uint32_t *)(base + at); at += 256;
     b.bytes = at;
     return b;
 }
 static size_t host_block_bytes(const PfHipMoeDesc *d) { return host_block(d, nullptr).bytes; }
 static bool through_host_block(const PfHipWork *w, size_t tokens) { return w->host && tokens <= PF_HOST_BLOCK_TOKENS; }
 
-// Enqueues the copies that bring a short batch's error word, ids and route weights into the block; after the stream
-// has been waited for, host_results hands them out.
-struct HostResults { const uint32_t *error_word, *ids; const float *weights; };
-static hipError_t fetch_results(const PfHipWork *w, const HostBlock &b, size_t tokens, bool want_ids, bool want_weights,
-                                HostResults *r) {
-    const size_t pairs = tokens * w->moe->desc.top_k * 4;
-    const size_t ids_at = (size_t)((const uint8_t *)w->ids - (const uint8_t *)w->error_word);
-    const size_t rw_at = (size_t)((const uint8_t *)w->route_weights - (const uint8_t *)w->error_word);
+// A short batch's rows come in and its results go out by kernels that address the block, not by copies: a copy runs on a
+// copy engine, and each change between engine and kernels waits for a signal (the two copies and the wait for the stream
+// were TODO of a one-token call).
+__global__ void pf_k_rows_in(const uint4 *src, uint4 *dst, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+struct PublishParts { const uint32_t *src[3]; uint32_t *dst[3]; int words[3]; };
+// One workgroup: the parts, then (everything before it has reached the host's memory) the call's number.
+__global__ void __launch_bounds__(256) pf_k_publish(PublishParts p, uint32_t *published, uint32_t call) {
+    for (int j = 0; j < 3; j++)
+        for (int i = threadIdx.x; i < p.words[j]; i += 256) p.dst[j][i] = p.src[j][i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(published, call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+static hipError_t host_rows_in(PfHipWork *w, const HostBlock &b, size_t tokens) {
+    const int n = (int)(tokens * w->moe->desc.hidden / 4);
+    if (w->moe->desc.hidden % 4) return hipMemcpyAsync(w->x, b.x, tokens * w->moe->desc.hidden * 4, hipMemcpyHostToDevice, nullptr);
+    hipLaunchKernelGGL(pf_k_rows_in, dim3((n + 255) / 256), dim3(256), 0, nullptr, reinterpret_cast<const uint4 *>(w->host_device + b.x_offset),
+                       reinterpret_cast<uint4 *>(w->x), n);
+    return hipGetLastError();
+}
+
+// Enqueues the kernel that publishes a short batch's error word, ids and route weights; await_results waits for it.
+struct HostResults { const uint32_t *error_word, *ids; const float *weights; uint32_t call; };
+static hipError_t publish_results(PfHipWork *w, const HostBlock &b, size_t tokens, bool want_ids, bool want_weights, HostResults *r) {
+    const int pairs = (int)(tokens * w->moe->desc.top_k);
     r->error_word = (const uint32_t *)b.head;
-    if ((const uint8_t *)w->ids > (const uint8_t *)w->error_word && w->route_weights > (const float *)w->ids &&
-        rw_at + pairs <= PF_HOST_HEAD_BYTES) {
-        const size_t span = want_weights ? rw_at + pairs : want_ids ? ids_at + pairs : 4;
-        r->ids = (const uint32_t *)(b.head + ids_at);
-        r->weights = (const float *)(b.head + rw_at);
-        return hipMemcpyAsync(b.head, w->error_word, span, hipMemcpyDeviceToHost, nullptr);
-    }
     r->ids = b.ids;
     r->weights = b.weights;
-    hipError_t e = hipMemcpyAsync(b.head, w->error_word, 4, hipMemcpyDeviceToHost, nullptr);
-    if (e == hipSuccess && want_ids) e = hipMemcpyAsync(b.ids, w->ids, pairs, hipMemcpyDeviceToHost, nullptr);
-    if (e == hipSuccess && want_weights) e = hipMemcpyAsync(b.weights, w->route_weights, pairs, hipMemcpyDeviceToHost, nullptr);
-    return e;
+    r->call = ++w->call;
+    PublishParts p;
+    p.src[0] = w->error_word; p.dst[0] = (uint32_t *)w->host_device; p.words[0] = 1;
+    p.src[1] = w->ids; p.dst[1] = (uint32_t *)(w->host_device + b.ids_offset); p.words[1] = want_ids ? pairs : 0;
+    p.src[2] = (const uint32_t *)w->route_weights; p.dst[2] = (uint32_t *)(w->host_device + b.weights_offset); p.words[2] = want_weights ? pairs : 0;
+    hipLaunchKernelGGL(pf_k_publish, dim3(1), dim3(256), 0, nullptr, p, (uint32_t *)(w->host_device + b.published_offset), r->call);
+    return hipGetLastError();
+}
+// The number is polled for as long as a short batch can take; then the stream is waited for, which also reports its errors.
+static hipError_t await_results(const HostBlock &b, const HostResults &r) {
+    for (int turn = 0; turn < 400000; turn++) {
+        if (__atomic_load_n(b.published, __ATOMIC_ACQUIRE) == r.call) return hipSuccess;
+        __builtin_ia32_pause();
+    }
+    return hipStreamSynchronize(nullptr);
 }
 
 // Longer batches pass through a ring of PF_RING_SLOTS page-locked pieces that follows the block: the CPU fills or empties
@@ -635,6 +665,7 @@ extern "C" int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWo
         (void)hipHostFree(w->host);
         w->host = nullptr;
     }
+    if (w->host) memset(w->host, 0, block);   // no call has been published
     if (w->host && long_batches) {
         w->ring = w->host + block;
         for (int j = 0; j < PF_RING_SLOTS; j++)
@@ -1011,13 +1042,13 @@ extern "C" int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, con
         // of their own)
         const HostBlock b = host_block(&moe->desc, work->host);
         rows_in(b.x, x, x_pitch_bytes, H * 4, tokens);
-        HIP_TRY(hipMemcpyAsync(work->x, b.x, tokens * H * 4, hipMemcpyHostToDevice, nullptr));
+        HIP_TRY(host_rows_in(work, b, tokens));
         // the last kernel writes the output rows into the pinned block itself
         int rc = pf_hip_moe_forward_device(moe, work, work->x, H, (float *)(work->host_device + b.y_offset), H, tokens, nullptr);
         if (rc != PF_HIP_OK) return rc;
         HostResults r;
-        HIP_TRY(fetch_results(work, b, tokens, ids != nullptr, weights != nullptr, &r));
-        HIP_TRY(hipStreamSynchronize(nullptr));
+        HIP_TRY(publish_results(work, b, tokens, ids != nullptr, weights != nullptr, &r));
+        HIP_TRY(await_results(b, r));
         *error_word = *r.error_word;
         if (*error_word) {
             HIP_TRY(hipMemset(work->error_word, 0, 4));   // the word is sticky on the device; reading it clears it
@@ -1090,7 +1121,7 @@ extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *wo
     const HostBlock b = host_block(&moe->desc, work->host);
     if (staged) {
         rows_in(b.x, x, x_pitch_bytes, H * 4, tokens);
-        HIP_TRY(hipMemcpyAsync(work->x, b.x, tokens * H * 4, hipMemcpyHostToDevice, nullptr));
+        HIP_TRY(host_rows_in(work, b, tokens));
     } else {
         HIP_TRY(rows_to_device(work, work->x, x, x_pitch_bytes, H * 4, tokens));
     }
@@ -1104,17 +1135,16 @@ extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *wo
         pf_launch_batch_router(a, (int)tokens, nullptr);
         pf_launch_dec_route(a, (int)tokens, nullptr);
     } else if (streamed_decode(moe, work, tokens, tiled_mask)) {
-        HIP_TRY(hipMemsetAsync(work->route_flags, 0, 4, nullptr));   // the routing's list starts empty (the other router kernels clear it themselves)
         pf_launch_dec_router(a, (int)tokens, (int)((moe->desc.experts + 3) / 4), nullptr);
-        pf_launch_route(a, (int)tokens, nullptr);
+        pf_launch_dec_route(a, (int)tokens, nullptr);
     } else {
         pf_launch_general(a, (int)tokens, nullptr, 2);
     }
     HIP_TRY(hipGetLastError());
-    HostResults r = {nullptr, nullptr, nullptr};
+    HostResults r = {nullptr, nullptr, nullptr, 0};
     if (staged) {
-        HIP_TRY(fetch_results(work, b, tokens, true, false, &r));
-        HIP_TRY(hipStreamSynchronize(nullptr));
+        HIP_TRY(publish_results(work, b, tokens, true, false, &r));
+        HIP_TRY(await_results(b, r));
         *error_word = *r.error_word;
     } else {
         HIP_TRY(hipMemcpy(error_word, work->error_word, 4, hipMemcpyDeviceToHost));
@@ -1154,8 +1184,7 @@ extern "C" int pf_hip_moe_experts_streamed_host(const PfHipMoe *moe, PfHipWork *
     const bool staged = through_host_block(work, tokens);
     const HostBlock b = host_block(&moe->desc, work->host);
     if (staged) {
-        memcpy(b.slots, slots, tokens * K * 4);
-        HIP_TRY(hipMemcpyAsync(work->slots, b.slots, tokens * K * 4, hipMemcpyHostToDevice, nullptr));
+        memcpy(b.slots, slots, tokens * K * 4);   // the kernels read them from the block
     } else {
         HIP_TRY(hipMemcpy(work->slots, slots, tokens * K * 4, hipMemcpyHostToDevice));
     }
@@ -1170,7 +1199,7 @@ extern "C" int pf_hip_moe_experts_streamed_host(const PfHipMoe *moe, PfHipWork *
         a.wi[t] = tiled && iq2 ? static_cast<const uint8_t *>(regions[j]) : nullptr;
         a.scale_offset[t] = scale_offsets[j];
     }
-    a.slots = work->slots;
+    a.slots = staged ? (const uint32_t *)(work->host_device + b.slots_offset) : work->slots;
     a.pool_slots = pool_slots;
     if (streamed_decode(moe, work, tokens, tiled_mask)) {
         // kernel 1 ran in the first call (logits and the token rows' images are in the workspace): kernels 2 and 3 only
@@ -1185,8 +1214,8 @@ extern "C" int pf_hip_moe_experts_streamed_host(const PfHipMoe *moe, PfHipWork *
     HIP_TRY(hipGetLastError());
     if (staged) {
         HostResults r;
-        HIP_TRY(fetch_results(work, b, tokens, ids != nullptr, weights != nullptr, &r));
-        HIP_TRY(hipStreamSynchronize(nullptr));
+        HIP_TRY(publish_results(work, b, tokens, ids != nullptr, weights != nullptr, &r));
+        HIP_TRY(await_results(b, r));
         *error_word = *r.error_word;
         if (*error_word) {
             HIP_TRY(hipMemset(work->error_word, 0, 4));
