@@ -1,11 +1,16 @@
 // C-ABI entry points of the HIP side (include/pf_moe_hip.h).
 #include "pf_moe_internal.h"
 #include "pf_moe_debug.h"
+#include "pf_host_calls.h"
 #include "../../include/pf_iq2_codes.h"
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <atomic>
+#include <condition_variable>
 #include <mutex>
+#include <new>
+#include <thread>
 
 static thread_local char g_error[256] = "";
 
@@ -487,17 +492,17 @@ static void carve_work(PfHipWork *w, const Carve &c, uint8_t *base);
 // The pinned block of a workspace: the error word, then input rows, output rows, ids, route weights and pool slots of up to
 // PF_HOST_BLOCK_TOKENS tokens and the number of the call whose results they are, each part 256-byte aligned.  The kernels
 // write the output rows straight into the block.
-#define PF_HOST_BLOCK_TOKENS PF_TILE_DECODE_MAX_TOKENS
+#define PF_HOST_BLOCK_TOKENS 64   // (beyond, a byte over the link costs a kernel more than it costs a copy engine)
 #define PF_HOST_HEAD_BYTES 256
 struct HostBlock {
     uint8_t *head;
     uint32_t *ids, *slots;
     float *x, *y, *weights;
     uint32_t *published;   // the number of the call whose results are in the block
-    size_t x_offset, y_offset, slots_offset, published_offset, ids_offset, weights_offset, bytes;
+    size_t x_offset, y_offset, slots_offset, published_offset, bytes;
 };
-static HostBlock host_block(const PfHipMoeDesc *d, uint8_t *base) {
-    const size_t T = PF_HOST_BLOCK_TOKENS, rows = (T * d->hidden * 4 + 255) & ~(size_t)255, pairs = (T * d->top_k * 4 + 255) & ~(size_t)255;
+static HostBlock host_block(const PfHipMoeDesc *d, size_t cap, uint8_t *base) {
+    const size_t T = cap < PF_HOST_BLOCK_TOKENS ? cap : PF_HOST_BLOCK_TOKENS, rows = (T * d->hidden * 4 + 255) & ~(size_t)255, pairs = (T * d->top_k * 4 + 255) & ~(size_t)255;
     HostBlock b;
     size_t at = 0;
     b.head = base + at; at += PF_HOST_HEAD_BYTES;
@@ -505,9 +510,7 @@ static HostBlock host_block(const PfHipMoeDesc *d, uint8_t *base) {
     b.x = (float *)(base + at); at += rows;
     b.y_offset = at;
     b.y = (float *)(base + at); at += rows;
-    b.ids_offset = at;
     b.ids = (uint32_t *)(base + at); at += pairs;
-    b.weights_offset = at;
     b.weights = (float *)(base + at); at += pairs;
     b.slots_offset = at;
     b.slots = (uint32_t *)(base + at); at += pairs;
@@ -516,13 +519,12 @@ static HostBlock host_block(const PfHipMoeDesc *d, uint8_t *base) {
     b.bytes = at;
     return b;
 }
-static size_t host_block_bytes(const PfHipMoeDesc *d) { return host_block(d, nullptr).bytes; }
 static bool through_host_block(const PfHipWork *w, size_t tokens) { return w->host && tokens <= PF_HOST_BLOCK_TOKENS; }
 
 // A short batch's rows come in and its results go out by kernels that address the block, not by copies: a copy runs on a
-// copy engine, and each change between engine and kernels waits for a signal (the two copies and the wait for the stream
-// were TODO of a one-token call).
-__global__ void pf_k_rows_in(const uint4 *src, uint4 *dst, int n) {
+// copy engine, and each change between engine and kernels waits for a signal (a one-token call of a 2048-wide layer with
+// both copies and a wait for the stream 34.7 us, so 30.1).
+__global__ void pf_k_copy_rows(const uint4 *src, uint4 *dst, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
 }
@@ -539,7 +541,7 @@ __global__ void __launch_bounds__(256) pf_k_publish(PublishParts p, uint32_t *pu
 static hipError_t host_rows_in(PfHipWork *w, const HostBlock &b, size_t tokens) {
     const int n = (int)(tokens * w->moe->desc.hidden / 4);
     if (w->moe->desc.hidden % 4) return hipMemcpyAsync(w->x, b.x, tokens * w->moe->desc.hidden * 4, hipMemcpyHostToDevice, nullptr);
-    hipLaunchKernelGGL(pf_k_rows_in, dim3((n + 255) / 256), dim3(256), 0, nullptr, reinterpret_cast<const uint4 *>(w->host_device + b.x_offset),
+    hipLaunchKernelGGL(pf_k_copy_rows, dim3((n + 255) / 256), dim3(256), 0, nullptr, reinterpret_cast<const uint4 *>(w->host_device + b.x_offset),
                        reinterpret_cast<uint4 *>(w->x), n);
     return hipGetLastError();
 }
@@ -548,14 +550,16 @@ static hipError_t host_rows_in(PfHipWork *w, const HostBlock &b, size_t tokens) 
 struct HostResults { const uint32_t *error_word, *ids; const float *weights; uint32_t call; };
 static hipError_t publish_results(PfHipWork *w, const HostBlock &b, size_t tokens, bool want_ids, bool want_weights, HostResults *r) {
     const int pairs = (int)(tokens * w->moe->desc.top_k);
+    const bool in_block = tokens <= PF_HOST_BLOCK_TOKENS;
+    uint8_t *const ids = in_block ? (uint8_t *)b.ids : w->routes, *const weights = in_block ? (uint8_t *)b.weights : w->routes + 4 * (size_t)pairs;
     r->error_word = (const uint32_t *)b.head;
-    r->ids = b.ids;
-    r->weights = b.weights;
+    r->ids = (const uint32_t *)ids;
+    r->weights = (const float *)weights;
     r->call = ++w->call;
     PublishParts p;
     p.src[0] = w->error_word; p.dst[0] = (uint32_t *)w->host_device; p.words[0] = 1;
-    p.src[1] = w->ids; p.dst[1] = (uint32_t *)(w->host_device + b.ids_offset); p.words[1] = want_ids ? pairs : 0;
-    p.src[2] = (const uint32_t *)w->route_weights; p.dst[2] = (uint32_t *)(w->host_device + b.weights_offset); p.words[2] = want_weights ? pairs : 0;
+    p.src[1] = w->ids; p.dst[1] = (uint32_t *)(w->host_device + (ids - w->host)); p.words[1] = want_ids ? pairs : 0;
+    p.src[2] = (const uint32_t *)w->route_weights; p.dst[2] = (uint32_t *)(w->host_device + (weights - w->host)); p.words[2] = want_weights ? pairs : 0;
     hipLaunchKernelGGL(pf_k_publish, dim3(1), dim3(256), 0, nullptr, p, (uint32_t *)(w->host_device + b.published_offset), r->call);
     return hipGetLastError();
 }
@@ -569,67 +573,186 @@ static hipError_t await_results(const HostBlock &b, const HostResults &r) {
 }
 
 // Longer batches pass through a ring of PF_RING_SLOTS page-locked pieces that follows the block: the CPU fills or empties
-// one piece while the others are on their way.  A hipMemcpy2D on the caller's pageable rows moves them row by row, each
-// with a wait of its own (777 rows of 8 KB each way and 31 KB of routes: 24.9 of a call's 25.4 ms; through the ring with
-// whole-piece copies 1.3 ms).  A piece is large enough that its transfer hides the enqueueing, small enough that the
-// first transfer starts early.
-#define PF_RING_SLOTS 4
+// some pieces while the others are on their way.  (A hipMemcpy2D on the caller's pageable rows moves them row by row, each
+// with a wait of its own: 777 rows of 8 KB each way took 24.9 ms.)  A piece is large enough that its transfer hides the
+// enqueueing.  One CPU copies at about a fifth of what the link carries, so the pieces are dealt to a few threads.
+#define PF_RING_SLOTS 8
 #define PF_RING_BYTES ((size_t)512 * 1024)
+#define PF_CREW_HELPERS 3                            // besides the calling thread
+#define PF_CREW_FROM ((size_t)1024 * 1024)           // bytes that are worth waking them for (10 to 20 us)
+
+// The helpers, one crew for the process: started with the first workspace that takes longer batches, ended with the last.
+// A call that finds the crew at work for another one copies alone.
+struct CopyCrew {
+    std::mutex busy, lock;
+    std::condition_variable wake, done;
+    std::thread thread[PF_CREW_HELPERS];
+    int helpers = 0, running = 0;
+    unsigned long round = 0;
+    bool quit = false;
+    void (*part)(void *, int, int) = nullptr;
+    void *job = nullptr;
+    void serve(int worker) {
+        unsigned long seen = 0;
+        std::unique_lock<std::mutex> hold(lock);
+        for (;;) {
+            wake.wait(hold, [&] { return quit || round != seen; });
+            if (quit) return;
+            seen = round;
+            hold.unlock();
+            part(job, worker, helpers + 1);
+            hold.lock();
+            if (--running == 0) done.notify_one();
+        }
+    }
+    CopyCrew() {
+        for (; helpers < PF_CREW_HELPERS; helpers++) {
+            try { thread[helpers] = std::thread([this, h = helpers] { serve(h + 1); }); } catch (...) { break; }
+        }
+    }
+    ~CopyCrew() {
+        { std::lock_guard<std::mutex> hold(lock); quit = true; }
+        wake.notify_all();
+        for (int h = 0; h < helpers; h++) thread[h].join();
+    }
+    // part(job, worker, workers) by every worker; the calling thread is worker 0
+    void run(void (*f)(void *, int, int), void *j) {
+        { std::lock_guard<std::mutex> hold(lock); part = f; job = j; running = helpers; round++; }
+        wake.notify_all();
+        f(j, 0, helpers + 1);
+        std::unique_lock<std::mutex> hold(lock);
+        done.wait(hold, [&] { return running == 0; });
+    }
+};
+static std::mutex g_crew_lock;
+static CopyCrew *g_crew = nullptr;
+static int g_crew_users = 0;
+static void crew_retain() {
+    std::lock_guard<std::mutex> hold(g_crew_lock);
+    if (g_crew_users++ == 0) g_crew = new (std::nothrow) CopyCrew();
+}
+static void crew_release() {
+    CopyCrew *last = nullptr;
+    {
+        std::lock_guard<std::mutex> hold(g_crew_lock);
+        if (--g_crew_users == 0) { last = g_crew; g_crew = nullptr; }
+    }
+    delete last;
+}
+
+// Rows between the caller's memory (a pitch) and dense device rows.  Piece p goes to worker p % workers, whose own slots its
+// pieces take in turn.
+struct RingJob {
+    PfHipWork *w;
+    uint8_t *device;
+    uint8_t *host;          // the caller's rows
+    size_t pitch, row_bytes, rows, step, pieces;
+    int device_id;
+    bool check;             // in: look for values that are not finite
+    std::atomic<int> error, nonfinite;
+    size_t rows_of(size_t p) const { return rows - p * step < step ? rows - p * step : step; }
+    static int slot_of(size_t p, int workers) {
+        const int per = PF_RING_SLOTS / workers;
+        return (int)(p % workers) * per + (int)(p / workers % per);
+    }
+    void fail(hipError_t e) { int none = 0; if (e != hipSuccess) error.compare_exchange_strong(none, (int)e); }
+};
 static void rows_in(void *dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
     for (size_t r = 0; r < rows; r++) memcpy((uint8_t *)dst + r * row_bytes, (const uint8_t *)src + r * src_pitch, row_bytes);
 }
 static void rows_out(void *dst, size_t dst_pitch, const void *src, size_t row_bytes, size_t rows) {
     for (size_t r = 0; r < rows; r++) memcpy((uint8_t *)dst + r * dst_pitch, (const uint8_t *)src + r * row_bytes, row_bytes);
 }
+// whether n floats are finite: an exponent of all ones carries into the sign bit
+static bool finite_floats(const void *p, size_t n) {
+    const uint8_t *bytes = static_cast<const uint8_t *>(p);
+    uint32_t carry = 0;
+    for (size_t i = 0; i < n; i++) {
+        uint32_t bits;
+        memcpy(&bits, bytes + 4 * i, 4);
+        carry |= (bits & 0x7fffffffu) + 0x00800000u;
+    }
+    return !(carry >> 31);
+}
+// A piece on its way, by a kernel that addresses the page-locked memory: 35 GB/s and no wait between engine and kernels,
+// where copies of this size brought 22 GB/s out of the device.
+static void ring_transfer(RingJob *j, int slot, void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
+    if (bytes % 16 == 0) {
+        const uint8_t *ring = j->w->ring;
+        auto on_device = [&](const void *p) {   // a piece by its device address
+            const uint8_t *b = static_cast<const uint8_t *>(p);
+            return b >= ring && b < ring + PF_RING_SLOTS * PF_RING_BYTES ? j->w->host_device + (b - j->w->host) : const_cast<uint8_t *>(b);
+        };
+        hipLaunchKernelGGL(pf_k_copy_rows, dim3((unsigned)((bytes / 16 + 255) / 256)), dim3(256), 0, nullptr, reinterpret_cast<const uint4 *>(on_device(src)),
+                           reinterpret_cast<uint4 *>(on_device(dst)), (int)(bytes / 16));
+        j->fail(hipGetLastError());
+    } else {
+        j->fail(hipMemcpyAsync(dst, src, bytes, kind, nullptr));
+    }
+    j->fail(hipEventRecord(j->w->ring_event[slot], nullptr));
+}
+static void ring_in_part(void *job, int worker, int workers) {
+    RingJob *j = static_cast<RingJob *>(job);
+    if (worker) j->fail(hipSetDevice(j->device_id));
+    for (size_t p = worker; p < j->pieces && !j->error.load() && !j->nonfinite.load(); p += workers) {
+        const int slot = RingJob::slot_of(p, workers);
+        const size_t r = p * j->step, n = j->rows_of(p);
+        uint8_t *piece = j->w->ring + slot * PF_RING_BYTES;
+        j->fail(hipEventSynchronize(j->w->ring_event[slot]));   // the piece's last transfer (none yet: returns at once)
+        rows_in(piece, j->host + r * j->pitch, j->pitch, j->row_bytes, n);
+        if (j->check && !finite_floats(piece, n * j->row_bytes / 4)) { j->nonfinite = 1; return; }
+        ring_transfer(j, slot, j->device + r * j->row_bytes, piece, n * j->row_bytes, hipMemcpyHostToDevice);
+    }
+}
+static void ring_send_out(RingJob *j, size_t p, int workers) {
+    const int slot = RingJob::slot_of(p, workers);
+    ring_transfer(j, slot, j->w->ring + slot * PF_RING_BYTES, j->device + p * j->step * j->row_bytes, j->rows_of(p) * j->row_bytes, hipMemcpyDeviceToHost);
+}
+static void ring_out_part(void *job, int worker, int workers) {   // the first PF_RING_SLOTS pieces are on their way
+    RingJob *j = static_cast<RingJob *>(job);
+    if (worker) j->fail(hipSetDevice(j->device_id));
+    const size_t ahead = (size_t)(PF_RING_SLOTS / workers) * workers;
+    for (size_t p = worker; p < j->pieces && !j->error.load(); p += workers) {
+        const int slot = RingJob::slot_of(p, workers);
+        j->fail(hipEventSynchronize(j->w->ring_event[slot]));
+        if (j->error.load()) break;
+        rows_out(j->host + p * j->step * j->pitch, j->pitch, j->w->ring + slot * PF_RING_BYTES, j->row_bytes, j->rows_of(p));
+        if (p + ahead < j->pieces) ring_send_out(j, p + ahead, workers);
+    }
+}
 
-// Pitched host rows to dense device rows, enqueued on the default stream; the caller's rows have been read when this
-// returns.  row_bytes fits a piece (the caller checks).
-static hipError_t ring_in(PfHipWork *w, void *d_dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
-    const size_t step = PF_RING_BYTES / row_bytes;
-    hipError_t e = hipSuccess;
-    int slot = 0;
-    for (size_t r = 0; r < rows && e == hipSuccess; r += step, slot = (slot + 1) % PF_RING_SLOTS) {
-        const size_t n = rows - r < step ? rows - r : step;
-        uint8_t *piece = w->ring + slot * PF_RING_BYTES;
-        e = hipEventSynchronize(w->ring_event[slot]);   // the piece's last transfer (none yet: returns at once)
-        if (e != hipSuccess) break;
-        rows_in(piece, (const uint8_t *)src + r * src_pitch, src_pitch, row_bytes, n);
-        e = hipMemcpyAsync((uint8_t *)d_dst + r * row_bytes, piece, n * row_bytes, hipMemcpyHostToDevice, nullptr);
-        if (e == hipSuccess) e = hipEventRecord(w->ring_event[slot], nullptr);
+static bool through_ring(const PfHipWork *w, size_t row_bytes) { return w->ring && row_bytes <= PF_RING_BYTES; }
+static void ring_job(RingJob *j, PfHipWork *w, void *device, const void *host, size_t pitch, size_t row_bytes, size_t rows) {
+    j->w = w; j->device = (uint8_t *)device; j->host = (uint8_t *)const_cast<void *>(host);
+    j->pitch = pitch; j->row_bytes = row_bytes; j->rows = rows;
+    j->step = PF_RING_BYTES / row_bytes;
+    j->pieces = (rows + j->step - 1) / j->step;
+    j->device_id = 0;
+    (void)hipGetDevice(&j->device_id);
+    j->check = false;
+    j->error = 0; j->nonfinite = 0;
+}
+// The crew if the rows are worth it and it is free (its `busy` is then held), else null.
+static CopyCrew *crew_for(const RingJob &j) {
+    CopyCrew *crew = j.row_bytes * j.rows >= PF_CREW_FROM ? g_crew : nullptr;   // (a workspace with a ring keeps it alive)
+    return crew && crew->helpers && PF_RING_SLOTS % (crew->helpers + 1) == 0 && crew->busy.try_lock() ? crew : nullptr;
+}
+// The caller's rows into device rows, enqueued on the default stream; they have been read when this returns.  nonfinite (may
+// be null): set where a row holds a value that is not finite; what has been sent by then is of no account.
+static hipError_t rows_to_device(PfHipWork *w, void *d_dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows, bool *nonfinite) {
+    if (!through_ring(w, row_bytes)) {   // no page-locked memory to be had, or a row longer than a piece: one blocking copy
+        for (size_t r = 0; r < rows && nonfinite && !*nonfinite; r++)
+            *nonfinite = !finite_floats((const uint8_t *)src + r * src_pitch, row_bytes / 4);
+        if (nonfinite && *nonfinite) return hipSuccess;
+        return hipMemcpy2D(d_dst, row_bytes, src, src_pitch, row_bytes, rows, hipMemcpyHostToDevice);
     }
-    return e;
-}
-// Dense device rows to pitched host rows; all of them have arrived when this returns.
-static hipError_t ring_out(PfHipWork *w, void *dst, size_t dst_pitch, const void *d_src, size_t row_bytes, size_t rows) {
-    const size_t step = PF_RING_BYTES / row_bytes, pieces = (rows + step - 1) / step;
-    hipError_t e = hipSuccess;
-    for (size_t j = 0; j < pieces + PF_RING_SLOTS - 1 && e == hipSuccess; j++) {   // piece j is sent, piece j - (slots - 1) is emptied
-        if (j < pieces) {
-            const size_t r = j * step, n = rows - r < step ? rows - r : step;
-            const int slot = (int)(j % PF_RING_SLOTS);
-            e = hipMemcpyAsync(w->ring + slot * PF_RING_BYTES, (const uint8_t *)d_src + r * row_bytes, n * row_bytes, hipMemcpyDeviceToHost, nullptr);
-            if (e == hipSuccess) e = hipEventRecord(w->ring_event[slot], nullptr);
-            if (e != hipSuccess) break;
-        }
-        if (j + 1 < PF_RING_SLOTS) continue;
-        const size_t k = j - (PF_RING_SLOTS - 1), r = k * step;
-        if (k >= pieces) break;
-        const size_t n = rows - r < step ? rows - r : step;
-        const int slot = (int)(k % PF_RING_SLOTS);
-        e = hipEventSynchronize(w->ring_event[slot]);
-        if (e == hipSuccess) rows_out((uint8_t *)dst + r * dst_pitch, dst_pitch, w->ring + slot * PF_RING_BYTES, row_bytes, n);
-    }
-    return e;
-}
-// Either through the ring where the workspace has one, else (no page-locked memory to be had, or a row longer than a
-// piece) as one blocking copy.
-static hipError_t rows_to_device(PfHipWork *w, void *d_dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
-    if (w->ring && row_bytes <= PF_RING_BYTES) return ring_in(w, d_dst, src, src_pitch, row_bytes, rows);
-    return hipMemcpy2D(d_dst, row_bytes, src, src_pitch, row_bytes, rows, hipMemcpyHostToDevice);
-}
-static hipError_t rows_to_host(PfHipWork *w, void *dst, size_t dst_pitch, const void *d_src, size_t row_bytes, size_t rows) {
-    if (w->ring && row_bytes <= PF_RING_BYTES) return ring_out(w, dst, dst_pitch, d_src, row_bytes, rows);
-    return hipMemcpy2D(dst, dst_pitch, d_src, row_bytes, row_bytes, rows, hipMemcpyDeviceToHost);
+    RingJob j;
+    ring_job(&j, w, d_dst, src, src_pitch, row_bytes, rows);
+    j.check = nonfinite != nullptr;
+    if (CopyCrew *crew = crew_for(j)) { crew->run(ring_in_part, &j); crew->busy.unlock(); }
+    else ring_in_part(&j, 0, 1);
+    if (nonfinite) *nonfinite = j.nonfinite.load() != 0;
+    return (hipError_t)j.error.load();
 }
 
 extern "C" int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWork **out) {
@@ -655,9 +778,10 @@ extern "C" int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWo
     for (int j = 0; j < W_COUNT; j++) w->guard_at[j] = c.offset[j] + c.size[j];
     // short batches through host pointers stage their rows in pinned memory: the copies are then enqueued and the call
     // waits once, for the last of them (without the block the forwards fall back to one blocking copy per buffer)
-    const size_t block = host_block_bytes(&moe->desc);
+    const size_t block = host_block(&moe->desc, token_cap, nullptr).bytes;
     const bool long_batches = token_cap > PF_HOST_BLOCK_TOKENS;
-    if (hipHostMalloc((void **)&w->host, block + (long_batches ? PF_RING_SLOTS * PF_RING_BYTES : 0), hipHostMallocDefault) != hipSuccess) {
+    const size_t routes = long_batches ? (2 * token_cap * moe->desc.top_k * 4 + 255) & ~(size_t)255 : 0;   // ids and weights of a longer batch
+    if (hipHostMalloc((void **)&w->host, block + routes + (long_batches ? PF_RING_SLOTS * PF_RING_BYTES : 0), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         w->host = nullptr;
     } else if (hipHostGetDevicePointer((void **)&w->host_device, w->host, 0) != hipSuccess) {
@@ -667,13 +791,15 @@ extern "C" int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWo
     }
     if (w->host) memset(w->host, 0, block);   // no call has been published
     if (w->host && long_batches) {
-        w->ring = w->host + block;
+        w->routes = w->host + block;
+        w->ring = w->routes + routes;
         for (int j = 0; j < PF_RING_SLOTS; j++)
             if (hipEventCreateWithFlags(&w->ring_event[j], hipEventDisableTiming) != hipSuccess) {
                 (void)hipGetLastError();
                 w->ring_event[j] = nullptr;
                 w->ring = nullptr;
             }
+        if (w->ring) crew_retain();
     }
     *out = w;
     return PF_HIP_OK;
@@ -722,6 +848,7 @@ static void carve_work(PfHipWork *w, const Carve &c, uint8_t *base) {
 extern "C" void pf_hip_work_destroy(PfHipWork *w) {
     if (!w) return;
     if (w->logits) (void)hipFree(w->logits);   // base of the single allocation
+    if (w->ring) crew_release();
     for (hipEvent_t event : w->ring_event) if (event) (void)hipEventDestroy(event);
     if (w->host) (void)hipHostFree(w->host);
     free(w);
@@ -1015,21 +1142,47 @@ extern "C" int pf_hip_moe_forward_hc_device(const PfHipMoe *moe, PfHipWork *work
 static int long_results(PfHipWork *work, float *y, size_t y_pitch_bytes, uint32_t *ids, size_t ids_pitch_bytes, float *weights,
                         size_t weights_pitch_bytes, size_t tokens, uint32_t *error_word) {
     const size_t H = work->moe->desc.hidden, K = work->moe->desc.top_k;
-    HIP_TRY(hipMemcpy(error_word, work->error_word, 4, hipMemcpyDeviceToHost));
-    if (*error_word) {
-        HIP_TRY(hipMemset(work->error_word, 0, 4));   // the word is sticky on the device; reading it clears it
+    if (!through_ring(work, H * 4)) {
+        HIP_TRY(hipMemcpy(error_word, work->error_word, 4, hipMemcpyDeviceToHost));
+        if (*error_word) {
+            HIP_TRY(hipMemset(work->error_word, 0, 4));   // the word is sticky on the device; reading it clears it
+            return PF_HIP_OK;
+        }
+        HIP_TRY(hipMemcpy2D(y, y_pitch_bytes, work->y, H * 4, H * 4, tokens, hipMemcpyDeviceToHost));
+        if (ids) HIP_TRY(hipMemcpy2D(ids, ids_pitch_bytes, work->ids, K * 4, K * 4, tokens, hipMemcpyDeviceToHost));
+        if (weights) HIP_TRY(hipMemcpy2D(weights, weights_pitch_bytes, work->route_weights, K * 4, K * 4, tokens, hipMemcpyDeviceToHost));
         return PF_HIP_OK;
     }
-    HIP_TRY(rows_to_host(work, y, y_pitch_bytes, work->y, H * 4, tokens));
-    if (ids) HIP_TRY(rows_to_host(work, ids, ids_pitch_bytes, work->ids, K * 4, tokens));
-    if (weights) HIP_TRY(rows_to_host(work, weights, weights_pitch_bytes, work->route_weights, K * 4, tokens));
+    const HostBlock b = host_block(&work->moe->desc, work->cap, work->host);
+    HostResults r;
+    HIP_TRY(publish_results(work, b, tokens, ids != nullptr, weights != nullptr, &r));
+    // the first pieces are on their way while the error word is looked at; the caller's rows are written after it
+    RingJob j;
+    ring_job(&j, work, work->y, y, y_pitch_bytes, H * 4, tokens);
+    CopyCrew *crew = crew_for(j);
+    const int workers = crew ? crew->helpers + 1 : 1;
+    for (size_t p = 0; p < j.pieces && p < PF_RING_SLOTS; p++) ring_send_out(&j, p, workers);
+    const hipError_t e = await_results(b, r);
+    const bool fine = e == hipSuccess && !j.error.load() && !*r.error_word;
+    if (fine && crew) crew->run(ring_out_part, &j);
+    else if (fine) ring_out_part(&j, 0, 1);
+    if (crew) crew->busy.unlock();
+    HIP_TRY(e);
+    HIP_TRY((hipError_t)j.error.load());
+    *error_word = *r.error_word;
+    if (*error_word) {
+        HIP_TRY(hipMemset(work->error_word, 0, 4));
+        return PF_HIP_OK;
+    }
+    if (ids) rows_out(ids, ids_pitch_bytes, r.ids, K * 4, tokens);
+    if (weights) rows_out(weights, weights_pitch_bytes, r.weights, K * 4, tokens);
     return PF_HIP_OK;
 }
 
-extern "C" int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes,
+static int forward_host(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes,
                                        float *y, size_t y_pitch_bytes, uint32_t *ids, size_t ids_pitch_bytes,
                                        float *weights, size_t weights_pitch_bytes, size_t tokens,
-                                       uint32_t *error_word) {
+                                       uint32_t *error_word, bool *nonfinite) {
     if (!moe || !work || !error_word) return PF_HIP_E_ARGUMENT;
     *error_word = 0;
     // before any row is copied: the pinned block and the workspace's rows are sized for the workspace's own layer
@@ -1040,8 +1193,9 @@ extern "C" int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, con
     if (through_host_block(work, tokens)) {
         // (the whole sequence as one replayed graph measured slower, 50 us against 43: the copies become graph nodes
         // of their own)
-        const HostBlock b = host_block(&moe->desc, work->host);
+        const HostBlock b = host_block(&moe->desc, work->cap, work->host);
         rows_in(b.x, x, x_pitch_bytes, H * 4, tokens);
+        if (nonfinite && !finite_floats(b.x, tokens * H)) { *nonfinite = true; return PF_HIP_OK; }
         HIP_TRY(host_rows_in(work, b, tokens));
         // the last kernel writes the output rows into the pinned block itself
         int rc = pf_hip_moe_forward_device(moe, work, work->x, H, (float *)(work->host_device + b.y_offset), H, tokens, nullptr);
@@ -1059,10 +1213,30 @@ extern "C" int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, con
         if (weights) rows_out(weights, weights_pitch_bytes, r.weights, K * 4, tokens);
         return PF_HIP_OK;
     }
-    HIP_TRY(rows_to_device(work, work->x, x, x_pitch_bytes, H * 4, tokens));
+    HIP_TRY(rows_to_device(work, work->x, x, x_pitch_bytes, H * 4, tokens, nonfinite));
+    if (nonfinite && *nonfinite) return PF_HIP_OK;
     int rc = pf_hip_moe_forward_device(moe, work, work->x, H, work->y, H, tokens, nullptr);
     if (rc != PF_HIP_OK) return rc;
     return long_results(work, y, y_pitch_bytes, ids, ids_pitch_bytes, weights, weights_pitch_bytes, tokens, error_word);
+}
+
+extern "C" int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes, float *y, size_t y_pitch_bytes,
+                                       uint32_t *ids, size_t ids_pitch_bytes, float *weights, size_t weights_pitch_bytes, size_t tokens,
+                                       uint32_t *error_word) {
+    return forward_host(moe, work, x, x_pitch_bytes, y, y_pitch_bytes, ids, ids_pitch_bytes, weights, weights_pitch_bytes, tokens, error_word, nullptr);
+}
+extern "C" int pf_host_forward_checked(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes, float *y, size_t y_pitch_bytes,
+                                       uint32_t *ids, size_t ids_pitch_bytes, float *weights, size_t weights_pitch_bytes, size_t tokens,
+                                       uint32_t *error_word, int *nonfinite_input) {
+    bool nonfinite = false;
+    const int rc = forward_host(moe, work, x, x_pitch_bytes, y, y_pitch_bytes, ids, ids_pitch_bytes, weights, weights_pitch_bytes, tokens, error_word, &nonfinite);
+    *nonfinite_input = nonfinite;
+    return rc;
+}
+extern "C" int pf_host_finite(const float *x, size_t pitch_bytes, size_t rows, size_t cols) {
+    for (size_t r = 0; r < rows; r++)
+        if (!finite_floats((const uint8_t *)x + r * pitch_bytes, cols)) return 0;
+    return 1;
 }
 
 // ---- a layer whose routed experts are streamed (src/qwen4_moe_internal.h:49-54, the remap hook) -----------------
@@ -1118,12 +1292,12 @@ extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *wo
     const size_t H = moe->desc.hidden, K = moe->desc.top_k;
     if (tokens * K > 0x7fffffffu / 4) return PF_HIP_E_UNSUPPORTED;
     const bool staged = through_host_block(work, tokens);
-    const HostBlock b = host_block(&moe->desc, work->host);
+    const HostBlock b = host_block(&moe->desc, work->cap, work->host);
     if (staged) {
         rows_in(b.x, x, x_pitch_bytes, H * 4, tokens);
         HIP_TRY(host_rows_in(work, b, tokens));
     } else {
-        HIP_TRY(rows_to_device(work, work->x, x, x_pitch_bytes, H * 4, tokens));
+        HIP_TRY(rows_to_device(work, work->x, x, x_pitch_bytes, H * 4, tokens, nullptr));
     }
     PfKernelArgs a = make_args(moe, work, work->x, H, work->y, H);
     const size_t lds_route = (H + 3 * (size_t)moe->desc.experts) * 4;
@@ -1182,7 +1356,7 @@ extern "C" int pf_hip_moe_experts_streamed_host(const PfHipMoe *moe, PfHipWork *
         if (expert_bytes[j] != want_bytes || scale_offsets[j] != want_scales) return PF_HIP_E_ARGUMENT;
     }
     const bool staged = through_host_block(work, tokens);
-    const HostBlock b = host_block(&moe->desc, work->host);
+    const HostBlock b = host_block(&moe->desc, work->cap, work->host);
     if (staged) {
         memcpy(b.slots, slots, tokens * K * 4);   // the kernels read them from the block
     } else {

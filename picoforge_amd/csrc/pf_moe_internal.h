@@ -143,7 +143,8 @@ struct PfHipWork {
     uint8_t *host;                  // pinned host block for the host-pointer forwards of short batches (null: not available)
     uint8_t *host_device;           // the same block as the kernels address it (they write the output rows straight into it)
     uint8_t *ring;                  // page-locked pieces behind the block, for host-pointer forwards of longer batches (null: none)
-    hipEvent_t ring_event[4];      // a piece's last transfer
+    uint8_t *routes;                // page-locked ids and route weights of a longer batch, between the block and the ring
+    hipEvent_t ring_event[8];      // a piece's last transfer
     uint32_t call;                  // number of the host-pointer call in progress (the block holds the last one published)
     int stage_limit;                // profiling: launch only the first so many kernels of a forward; 0 = all
     int force_general;               // tests: run the general kernels even where the decode path applies

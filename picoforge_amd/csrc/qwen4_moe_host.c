@@ -8,6 +8,7 @@
 #include "../../include/qwen4_expert_pool.h"
 #include "../../include/pf_moe_hip.h"
 #include "pf_hc_host.h"
+#include "pf_host_calls.h"
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -577,10 +578,9 @@ static Qwen4Status forward_checked(const Qwen4Moe *m, QW4ExpertPool *pool, uint3
             TRY(all_disjoint(two, 2, err));
         }
     }
-    const size_t xs = x.stride_bytes[0] / 4;
-    for (size_t row = 0; row < T; row++)
-        for (size_t col = 0; col < H; col++)
-            if (!isfinite(x.data[row * xs + col])) return moe_status(err, QW4_NONFINITE, "nonfinite input");
+    /* (a resident layer's rows are looked through while they are brought into page-locked memory) */
+    const bool resident = !pool && !w->observer;
+    if (!resident && !pf_host_finite(x.data, x.stride_bytes[0], T, H)) return moe_status(err, QW4_NONFINITE, "nonfinite input");
     if (!T) return moe_status(err, QW4_OK, "");
     /* the routing trace needs the ids also when the caller did not ask for them */
     Qwen4MoeRoutes traced;
@@ -597,10 +597,16 @@ static Qwen4Status forward_checked(const Qwen4Moe *m, QW4ExpertPool *pool, uint3
     else if (pool) st = streamed_forward(m, w, pool, layer, x, y, routes, err);
     else {
         uint32_t word = 0;
-        int rc = pf_hip_moe_forward_host(m->device, w->device, x.data, x.stride_bytes[0], y.data, y.stride_bytes[0],
+        int nonfinite = 0;
+        int rc = pf_host_forward_checked(m->device, w->device, x.data, x.stride_bytes[0], y.data, y.stride_bytes[0],
                                          routes ? routes->ids.data : NULL, routes ? routes->ids.row_stride_bytes : 0,
                                          routes ? routes->weights.data : NULL,
-                                         routes ? routes->weights.stride_bytes[0] : 0, T, &word);
+                                         routes ? routes->weights.stride_bytes[0] : 0, T, &word, &nonfinite);
+        if (!rc && nonfinite) {
+            w->busy = false;
+            free(trace_memory);
+            return moe_status(err, QW4_NONFINITE, "nonfinite input");
+        }
         if (rc) st = pf_device_status(rc, err, "qwen4_moe");
         else if (word & PF_HIP_ERR_NONFINITE) st = moe_status(err, QW4_NONFINITE, "nonfinite value in the MoE block");
         else if (word) st = moe_status(err, QW4_GPU_ERROR, "device error word");

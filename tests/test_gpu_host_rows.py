@@ -1,0 +1,32 @@
+"""Host-pointer forwards on both sides of each way rows travel: the page-locked block (up to 64 tokens), the ring of pieces by
+one thread, and by the crew (from 1 MB); a value that is not finite in the last row is found before anything is written."""
+import numpy as np
+import pytest
+
+import picoforge_amd as pf
+from picoforge_amd import abi
+
+from helpers import assert_parity, forward_with, make_layer_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hidden,batches", [(512, (1, 64, 65, 257, 512, 513, 700)), (2560, (64, 104, 105, 460))])
+def test_rows_through_block_ring_and_crew(product, oracle, hidden, batches):
+    cfg = abi.moe_config(hidden, 16, 3, 256, 256)
+    most = max(batches)
+    weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, most, seed=hidden)
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, most) as layer:
+        for tokens in batches:
+            print(f"case hidden={hidden} tokens={tokens}", flush=True)
+            for bad in (np.nan, -np.inf):
+                spoilt = x[:tokens].copy()
+                spoilt[-1, -1] = bad
+                st, y, ids, w = layer.forward(spoilt, check=False)
+                assert st == abi.QW4_NONFINITE and b"nonfinite input" in bytes(layer.err.detail)
+                assert (y == -99.0).all() and (w == -99.0).all() and (ids == 0xFFFFFFFF).all()
+            _, y, ids, w = layer.forward(x[:tokens])   # the workspace is as usable as before
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
+            _, y2, _, _ = layer.forward(x[:tokens], want_routes=False)
+            np.testing.assert_array_equal(y, y2)
