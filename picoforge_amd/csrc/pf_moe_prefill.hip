@@ -893,7 +893,7 @@ __global__ void __launch_bounds__(64 * (NW + NL), 3) pf_k_pf_gemm(PfKernelArgs a
             gemm_compute_iq2(ring, g.kblocks, acc0, acc1, slot_off, block_parity, g.sidx0, g.sidx1, g.bpr, (int)g.wave_rows);
         else
             gemm_compute(ring, g.kblocks, acc0, acc1, slot_off, block_parity);
-        // epilogue: the lane holds column n of its two tiles; register r is row 8 (r / 4) + 4 h + r % 4
+        // epilogue: the lane holds column n of its tiles; register r is row 8 (r / 4) + 4 h + r % 4
         const float *scales = row_scale[item_index & 3];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
@@ -975,127 +975,203 @@ __device__ __forceinline__ PlainRow plain_row(const PfKernelArgs &a, int t, size
     return r;
 }
 
-// acc0 / acc1 += staged activation columns [c0, c0 + cols) x the same columns of weight rows r0 / r1.
-// ahi / alo: this lane's activation row in LDS (high and low parts of the staged columns); sums: the
-// row's sums over every 16 staged columns (high parts, low parts sums_low further on; Q2_K only).
-// The weight bytes of several groups are requested before the first product of the batch.
-// A wave takes every `parts`-th batch (256-block for Q2_K) starting with batch `part`: with parts > 1 the
-// waves of a workgroup share one pair of rows and their partial sums are added afterwards.
-template <int FMT>
-__device__ __forceinline__ void plain_product(const PlainRow &r0, const PlainRow &r1, const half_t *ahi, const half_t *alo,
-                                              const half_t *sums, int sums_low, int c0, int cols, int h, int part, int parts,
-                                              float16v &acc0, float16v &acc1) {
-    const float16v zero = {0};
-    if (FMT == PF_Q2_K) {
-        // a row's last block may be half used (logical width 640 of 768 stored): its second half is skipped,
-        // and the sums of the groups beyond the width are zero
-        for (int b = part; b < (cols + 255) / 256; b += parts) {
-            const uint8_t *blk0 = r0.payload + 84 * (size_t)(c0 / 256 + b), *blk1 = r1.payload + 84 * (size_t)(c0 / 256 + b);
-            const uint32_t dd0 = *reinterpret_cast<const uint32_t *>(blk0 + 80), dd1 = *reinterpret_cast<const uint32_t *>(blk1 + 80);
-            float16v part0 = zero, part1 = zero;
-            const uint32_t *sw0 = reinterpret_cast<const uint32_t *>(blk0), *sw1 = reinterpret_cast<const uint32_t *>(blk1);   // 4-byte aligned
-            // Q: the 16 groups' minima (scale bytes 8h..8h+7, high nibbles) against the rows' sums over the same groups
-            const half8v sh = *reinterpret_cast<const half8v *>(sums + 16 * b + 8 * h), sl = *reinterpret_cast<const half8v *>(sums + sums_low + 16 * b + 8 * h);
-            const half8v mv0 = half8_of_bytes((sw0[2 * h] >> 4) & 0x0F0F0F0Fu, (sw0[2 * h + 1] >> 4) & 0x0F0F0F0Fu, (half_t)1024.0f);
-            const half8v mv1 = half8_of_bytes((sw1[2 * h] >> 4) & 0x0F0F0F0Fu, (sw1[2 * h + 1] >> 4) & 0x0F0F0F0Fu, (half_t)1024.0f);
-            float16v low0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(sh, mv0, zero, 0, 0, 0);
-            float16v low1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(sh, mv1, zero, 0, 0, 0);
-            low0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(sl, mv0, low0, 0, 0, 0);
-            low1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(sl, mv1, low1, 0, 0, 0);
+// One batch of a wave's two weight rows: the bytes of 128 columns (Q2_K: of a 256-block), as they were loaded.  The kernel
+// requests a batch while it multiplies the one before, across the passes too: without that a wave waited for memory once a
+// batch, about twice as long as the products of a batch take, with two waves a SIMD to cover for one another (MXFP4 down launch of a
+// 2048-token chunk at the checkpoints' widths 497 -> 412 us, Q2_K, 1024 tokens, 315 -> 293 us).
+template <int FMT, int S> struct PlainBatch;
+template <int S> struct PlainBatch<PF_Q8_0, S> {
+    static constexpr int COLS = 128;
+    uint2 q[S][4][2], scales[S];   // [row][group][half of its columns]; four half scales
+    __device__ __forceinline__ void load(const PlainRow (&r)[S], int batch, int h) {
 #pragma unroll
-            for (int half = 0; half < 2; half++) {   // eight groups of 16 weights per batch: one 32-byte half of the codes
-                if (256 * b + 128 * half >= cols) break;
-                const uint32_t *q0 = reinterpret_cast<const uint32_t *>(blk0 + 16 + 32 * half + 8 * h);
-                const uint32_t *q1 = reinterpret_cast<const uint32_t *>(blk1 + 16 + 32 * half + 8 * h);
-                // bytes 8h..8h+7 and 16 + 8h..: the groups at l % 32 = 0 and 16, each at four bit planes
-                const uint32_t c0a[2] = {q0[0], q0[1]}, c0b[2] = {q0[4], q0[5]}, c1a[2] = {q1[0], q1[1]}, c1b[2] = {q1[4], q1[5]};
-                const uint32_t scales0[4] = {sw0[0], sw0[1], sw0[2], sw0[3]}, scales1[4] = {sw1[0], sw1[1], sw1[2], sw1[3]};
+        for (int s = 0; s < S; s++) {
+            scales[s] = *reinterpret_cast<const uint2 *>(r[s].scales + 8 * (size_t)batch);
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int gi = 8 * half + j, shift = 2 * (j >> 1), k = 256 * b + 16 * gi + 8 * h;
-                    const uint32_t s0 = (scales0[gi >> 2] >> (8 * (gi & 3))) & 255u, s1 = (scales1[gi >> 2] >> (8 * (gi & 3))) & 255u;
-                    const uint32_t *w0c = (j & 1) ? c0b : c0a, *w1c = (j & 1) ? c1b : c1a;
-                    const half8v xh = *reinterpret_cast<const half8v *>(ahi + k), xl = *reinterpret_cast<const half8v *>(alo + k);
-                    // byte-wise scale * code: at most 15 * 3, no carry between bytes
-                    const half8v w0 = half8_of_bytes(((w0c[0] >> shift) & 0x03030303u) * (s0 & 15u), ((w0c[1] >> shift) & 0x03030303u) * (s0 & 15u), (half_t)1024.0f);
-                    const half8v w1 = half8_of_bytes(((w1c[0] >> shift) & 0x03030303u) * (s1 & 15u), ((w1c[1] >> shift) & 0x03030303u) * (s1 & 15u), (half_t)1024.0f);
-                    part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, w0, part0, 0, 0, 0);
-                    part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, w1, part1, 0, 0, 0);
-                    part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, w0, part0, 0, 0, 0);
-                    part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, w1, part1, 0, 0, 0);
-                }
-            }
-            const half2v h0 = __builtin_bit_cast(half2v, dd0), h1 = __builtin_bit_cast(half2v, dd1);
-            const float d0 = (float)h0.x, n0 = (float)h0.y, d1 = (float)h1.x, n1 = (float)h1.y;
+            for (int g = 0; g < 4; g++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                acc0[r] = fmaf(d0, part0[r], fmaf(-n0, low0[r], acc0[r]));
-                acc1[r] = fmaf(d1, part1[r], fmaf(-n1, low1[r], acc1[r]));
-            }
+                for (int t = 0; t < 2; t++) q[s][g][t] = *reinterpret_cast<const uint2 *>(r[s].payload + 32 * (size_t)(4 * batch + g) + 16 * t + 8 * h);
         }
-        return;
     }
-    for (int g0 = 4 * part; g0 < cols / 32; g0 += 4 * parts) {   // batches of four groups of 32 weights (cols is a multiple of 128)
-        const int first = c0 / 32 + g0;            // of the row's groups
-        uint2 q0[4][2], q1[4][2];
-        float s0[4], s1[4];
+    __device__ __forceinline__ float scale(int s, int g) const {
+        const uint32_t two = g < 2 ? scales[s].x : scales[s].y;
+        return (float)__builtin_bit_cast(half_t, (unsigned short)((g & 1) ? two >> 16 : two & 0xffffu));
+    }
+    __device__ __forceinline__ half8v operand(int s, int g, int t) const { return half8_of_signed_bytes(q[s][g][t].x, q[s][g][t].y); }
+};
+template <int S> struct PlainBatch<PF_MXFP4, S> {   // bytes 8h..8h+7 of a block: low nibbles values 8h.., high nibbles values 16 + 8h..
+    static constexpr int COLS = 128;
+    uint2 q[S][4];
+    uint32_t scales[S];
+    __device__ __forceinline__ void load(const PlainRow (&r)[S], int batch, int h) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (FMT == PF_Q8_0) {
-                s0[j] = (float)__builtin_bit_cast(half_t, reinterpret_cast<const uint16_t *>(r0.scales)[first + j]);
-                s1[j] = (float)__builtin_bit_cast(half_t, reinterpret_cast<const uint16_t *>(r1.scales)[first + j]);
+        for (int s = 0; s < S; s++) {
+            scales[s] = *reinterpret_cast<const uint32_t *>(r[s].scales + 4 * (size_t)batch);
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    q0[j][t] = *reinterpret_cast<const uint2 *>(r0.payload + 32 * (size_t)(first + j) + 16 * t + 8 * h);
-                    q1[j][t] = *reinterpret_cast<const uint2 *>(r1.payload + 32 * (size_t)(first + j) + 16 * t + 8 * h);
-                }
-            } else {   // MXFP4: bytes 8h..8h+7 of the block: low nibbles values 8h.., high nibbles values 16 + 8h..
-                s0[j] = 0.5f * pf_e8m0_scale(r0.scales[first + j]);   // the operands are twice the values
-                s1[j] = 0.5f * pf_e8m0_scale(r1.scales[first + j]);
-                q0[j][0] = *reinterpret_cast<const uint2 *>(r0.payload + 16 * (size_t)(first + j) + 8 * h);
-                q1[j][0] = *reinterpret_cast<const uint2 *>(r1.payload + 16 * (size_t)(first + j) + 8 * h);
-                q0[j][1] = uint2{q0[j][0].x >> 4, q0[j][0].y >> 4};
-                q1[j][1] = uint2{q1[j][0].x >> 4, q1[j][0].y >> 4};
+            for (int g = 0; g < 4; g++) q[s][g] = *reinterpret_cast<const uint2 *>(r[s].payload + 16 * (size_t)(4 * batch + g) + 8 * h);
+        }
+    }
+    __device__ __forceinline__ float scale(int s, int g) const { return 0.5f * pf_e8m0_scale((scales[s] >> (8 * g)) & 255u); }   // the operands are twice the values
+    __device__ __forceinline__ half8v operand(int s, int g, int t) const {
+        return half8_of_e2m1((q[s][g].x >> (4 * t)) & 0x0F0F0F0Fu, (q[s][g].y >> (4 * t)) & 0x0F0F0F0Fu);
+    }
+};
+template <int S> struct PlainBatch<PF_Q2_K, S> {
+    static constexpr int COLS = 256;
+    uint32_t codes[S][2][2][2], scales[S][4], dd[S];   // [row][half of the block][sub-group of 16][dword]
+    __device__ __forceinline__ void load(const PlainRow (&r)[S], int batch, int h) {
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            const uint32_t *block = reinterpret_cast<const uint32_t *>(r[s].payload + 84 * (size_t)batch);   // 4-byte aligned
+            dd[s] = block[20];
+#pragma unroll
+            for (int k = 0; k < 4; k++) scales[s][k] = block[k];
+#pragma unroll
+            for (int half = 0; half < 2; half++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) codes[s][half][k >> 1][k & 1] = block[4 + 8 * half + 2 * h + 4 * (k >> 1) + (k & 1)];
+        }
+    }
+};
+
+// acc[row] += the staged activation columns of the batch (local columns k0..) x the batch.  ahi / alo: this lane's activation
+// row in LDS (high and low parts); sums: the row's sums over every 16 staged columns (high parts, low parts sums_low further
+// on; Q2_K only); cols: staged columns.
+template <int FMT, int S>
+__device__ __forceinline__ void plain_product(const PlainBatch<FMT, S> &w, const half_t *ahi, const half_t *alo, const half_t *, int, int k0, int, int h,
+                                              float16v (&acc)[S]) {
+    const float16v zero = {0};
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        float16v part[S];
+#pragma unroll
+        for (int s = 0; s < S; s++) part[s] = zero;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int k = k0 + 32 * g + 16 * t + 8 * h;
+            const half8v xh = *reinterpret_cast<const half8v *>(ahi + k), xl = *reinterpret_cast<const half8v *>(alo + k);
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                const half8v v = w.operand(s, g, t);
+                part[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, v, part[s], 0, 0, 0);
+                part[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, v, part[s], 0, 0, 0);
             }
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float16v part0 = zero, part1 = zero;
+        for (int s = 0; s < S; s++) {
+            const float scale = w.scale(s, g);
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int k = 32 * (g0 + j) + 16 * t + 8 * h;
-                const half8v xh = *reinterpret_cast<const half8v *>(ahi + k), xl = *reinterpret_cast<const half8v *>(alo + k);
-                half8v w0, w1;
-                if (FMT == PF_Q8_0) {
-                    w0 = half8_of_signed_bytes(q0[j][t].x, q0[j][t].y);
-                    w1 = half8_of_signed_bytes(q1[j][t].x, q1[j][t].y);
-                } else {
-                    w0 = half8_of_e2m1(q0[j][t].x & 0x0F0F0F0Fu, q0[j][t].y & 0x0F0F0F0Fu);
-                    w1 = half8_of_e2m1(q1[j][t].x & 0x0F0F0F0Fu, q1[j][t].y & 0x0F0F0F0Fu);
-                }
-                part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, w0, part0, 0, 0, 0);
-                part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, w1, part1, 0, 0, 0);
-                part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, w0, part0, 0, 0, 0);
-                part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, w1, part1, 0, 0, 0);
-            }
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                acc0[r] = fmaf(s0[j], part0[r], acc0[r]);
-                acc1[r] = fmaf(s1[j], part1[r], acc1[r]);
-            }
+            for (int r = 0; r < 16; r++) acc[s][r] = fmaf(scale, part[s][r], acc[s][r]);
         }
     }
 }
+template <int S>
+__device__ __forceinline__ void plain_product(const PlainBatch<PF_Q2_K, S> &w, const half_t *ahi, const half_t *alo, const half_t *sums, int sums_low,
+                                                       int k0, int cols, int h, float16v (&acc)[S]) {
+    // a row's last block may be half used (logical width 640 of 768 stored): its second half is skipped, and the sums of the
+    // groups beyond the width are zero
+    const float16v zero = {0};
+    float16v part[S], low[S];
+#pragma unroll
+    for (int s = 0; s < S; s++) part[s] = zero;
+    // Q: the 16 groups' minima (scale bytes 8h..8h+7, high nibbles) against the rows' sums over the same groups
+    const half8v sh = *reinterpret_cast<const half8v *>(sums + k0 / 16 + 8 * h), sl = *reinterpret_cast<const half8v *>(sums + sums_low + k0 / 16 + 8 * h);
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        const uint32_t m0 = h ? w.scales[s][2] : w.scales[s][0], m1 = h ? w.scales[s][3] : w.scales[s][1];
+        const half8v mv = half8_of_bytes((m0 >> 4) & 0x0F0F0F0Fu, (m1 >> 4) & 0x0F0F0F0Fu, (half_t)1024.0f);
+        low[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sh, mv, zero, 0, 0, 0);
+        low[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sl, mv, low[s], 0, 0, 0);
+    }
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        if (k0 + 128 * half >= cols) break;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {   // groups of 16 weights
+            const int gi = 8 * half + j, k = k0 + 16 * gi + 8 * h;
+            const half8v xh = *reinterpret_cast<const half8v *>(ahi + k), xl = *reinterpret_cast<const half8v *>(alo + k);
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                // byte-wise scale * code: at most 15 * 3, no carry between bytes
+                const uint32_t f = (w.scales[s][gi >> 2] >> (8 * (gi & 3))) & 15u, *c = w.codes[s][half][j & 1];
+                const half8v v = half8_of_bytes(((c[0] >> (2 * (j >> 1))) & 0x03030303u) * f, ((c[1] >> (2 * (j >> 1))) & 0x03030303u) * f, (half_t)1024.0f);
+                part[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, v, part[s], 0, 0, 0);
+                part[s] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, v, part[s], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        const half2v dm = __builtin_bit_cast(half2v, w.dd[s]);
+        const float d = (float)dm.x, n = (float)dm.y;
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[s][r] = fmaf(d, part[s][r], fmaf(-n, low[s][r], acc[s][r]));
+    }
+}
 
-#define PLAIN_CHUNK 512                     // activation columns staged per pass
+#define PLAIN_CHUNK 512                     // activation columns staged per pass (256, three workgroups a compute unit: slower)
 #define PLAIN_PITCH (PLAIN_CHUNK + 8)       // halfs between staged rows: 16 bytes of padding spread the rows over the banks
 #define PLAIN_SUMS (PLAIN_CHUNK / 16 + 8)   // halfs between the rows' sums over 16 columns
 #define PLAIN_TILE_BYTES (2 * 32 * PLAIN_PITCH * 2)
 #define PLAIN_LDS (PLAIN_TILE_BYTES + 2 * 32 * PLAIN_SUMS * 2)
 
+// Stages PLAIN_CHUNK columns of the tile's 32 activation rows (high and low parts), one 1 KB row part per load instruction, and
+// multiplies them, pass after pass.  A wave takes every `parts`-th batch starting with batch `part`: with parts > 1 the waves
+// of a workgroup share one pair of rows and their partial sums are added afterwards.
+struct PlainTile { half_t *tile, *sums; const half_t *a16; const uint32_t *src_row; int a_cols; };
+template <int FMT, int S>
+__device__ __forceinline__ void plain_passes(const PlainTile &a, const PlainRow (&rows)[S], bool active, int part, int parts, float16v (&acc)[S]) {
+    typedef PlainBatch<FMT, S> Batch;
+    const int lane = pf_lane(), wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
+    const int batches = (a.a_cols + Batch::COLS - 1) / Batch::COLS;
+    const half_t *ahi = a.tile + (size_t)n * PLAIN_PITCH, *alo = ahi + 32 * PLAIN_PITCH;
+    Batch w, next;
+    if (active && part < batches) next.load(rows, part, h);   // on their way while the first columns are staged
+    for (int c0 = 0; c0 < a.a_cols; c0 += PLAIN_CHUNK) {
+        const int cols = min(PLAIN_CHUNK, a.a_cols - c0);
+        if (c0) __syncthreads();   // the previous pass has been consumed
+        // 64 row parts (32 rows, high and low) over the four waves; a lane moves 16 bytes of each
+#pragma unroll 4
+        for (int i = 0; i < 16; i++) {
+            const int row_part = 16 * wave + i, row = row_part & 31, low = row_part >> 5;
+            if (16 * lane < 2 * cols)
+                to_lds(a.a16 + (size_t)a.src_row[row] * pf_half_row(a.a_cols) + (size_t)low * a.a_cols + c0 + 8 * lane,
+                       reinterpret_cast<unsigned char *>(a.tile + ((size_t)low * 32 + row) * PLAIN_PITCH));
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (FMT == PF_Q2_K) {
+            // sums of the staged rows over every 16 columns, as two-part halfs like the values themselves:
+            // thread = (row, four neighbouring groups)
+            const int row = threadIdx.x >> 3, g0 = 4 * (threadIdx.x & 7);
+#pragma unroll
+            for (int g = g0; g < g0 + 4; g++) {
+                float total = 0.0f;
+                if (16 * g < cols) {
+                    const half_t *hi = a.tile + (size_t)row * PLAIN_PITCH + 16 * g, *lo = hi + 32 * PLAIN_PITCH;
+                    const half8v a0 = *reinterpret_cast<const half8v *>(hi), a1 = *reinterpret_cast<const half8v *>(hi + 8);
+                    const half8v b0 = *reinterpret_cast<const half8v *>(lo), b1 = *reinterpret_cast<const half8v *>(lo + 8);
+#pragma unroll
+                    for (int i = 0; i < 8; i++) total += ((float)a0[i] + (float)b0[i]) + ((float)a1[i] + (float)b1[i]);
+                }
+                const half_t top = (half_t)total;
+                a.sums[(size_t)row * PLAIN_SUMS + g] = top;
+                a.sums[(size_t)(32 + row) * PLAIN_SUMS + g] = (half_t)(total - (float)top);
+            }
+            __syncthreads();
+        }
+        if (!active) continue;
+        for (int k0 = Batch::COLS * part; k0 < cols; k0 += Batch::COLS * parts) {
+            w = next;
+            const int after = (c0 + k0) / Batch::COLS + parts;
+            if (after < batches) next.load(rows, after, h);
+            plain_product(w, ahi, alo, a.sums + (size_t)n * PLAIN_SUMS, 32 * PLAIN_SUMS, k0, cols, h, acc);
+        }
+    }
+}
+
 // grid: (row tiles the list can hold) x slabs; 4 waves.  Items whose tensors are in a format of the ring
-// kernel are skipped here, as the ring kernel skips these.  Per pass the workgroup stages 512 columns
-// of the tile's 32 activation rows (high and low parts) in LDS, one 1 KB row part per load instruction.
+// kernel are skipped here, as the ring kernel skips these.
 // split != 0 (gate/up only): the four waves share 32 units and take a quarter of the columns each; their
 // partial sums meet in LDS and wave 0 adds them in wave order.  For matrices with few row tiles (the
 // shared expert) that gives four times as many workgroups.
@@ -1120,20 +1196,11 @@ __global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int to
     const int t0 = MODE == PF_GEMM_GATE_UP ? (shared ? 4 : 1) : (shared ? 6 : 3);
     const uint32_t fmt = a.type[t0];
     if (fmt != PF_Q8_0 && fmt != PF_Q2_K && fmt != PF_MXFP4) return;
-    int row_a, row_b, t1, limit;
-    const int slab_rows = MODE != PF_GEMM_GATE_UP ? 256 : split ? 32 : 128;
-    if (MODE == PF_GEMM_GATE_UP) {
-        limit = inter;
-        row_a = row_b = slab_rows * (int)slab + (split ? 0 : 32 * wave) + n;   // the unit's gate row and up row
-        t1 = t0 + 1;
-    } else {
-        limit = a.hidden;
-        row_a = 256 * (int)slab + 64 * wave + n;
-        row_b = row_a + 32;
-        t1 = t0;
-    }
+    constexpr int S = 2;   // 32-row tiles of a wave: a gate tile and the up tile of the same units, or two down tiles (four: one wave a SIMD, slower)
+    const int slab_rows = MODE != PF_GEMM_GATE_UP ? 128 * S : split ? 32 : 128, limit = MODE == PF_GEMM_GATE_UP ? inter : a.hidden;
+    const int row0 = MODE == PF_GEMM_GATE_UP ? slab_rows * (int)slab + (split ? 0 : 32 * wave) + n : slab_rows * (int)slab + 32 * S * wave + n;
     if (slab_rows * (int)slab >= limit) return;   // the slab starts beyond the matrix: the whole workgroup
-    const bool active = row_a - n < limit;        // this wave has rows (the others stay for the barriers)
+    const bool active = row0 - n < limit;        // this wave has rows (the others stay for the barriers)
     const int part = split ? wave : 0, parts = split ? 4 : 1;
     // the tile's activation rows (the all-zero row beyond the tile's last) and their scales
     const int a_cols = MODE == PF_GEMM_GATE_UP ? a.hidden : inter;
@@ -1149,57 +1216,25 @@ __global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int to
         src_scale[m] = m < rows_here ? a_scale[src] : 0.0f;
     }
     __syncthreads();
-    const PlainRow r0 = plain_row(a, t0, ex, min(row_a, limit - 1)), r1 = plain_row(a, t1, ex, min(row_b, limit - 1));
-    const half_t *ahi = tile + (size_t)n * PLAIN_PITCH, *alo = ahi + 32 * PLAIN_PITCH;
-    float16v acc0 = {0}, acc1 = {0};
-    for (int c0 = 0; c0 < a_cols; c0 += PLAIN_CHUNK) {
-        const int cols = min(PLAIN_CHUNK, a_cols - c0);
-        if (c0) __syncthreads();   // the previous pass has been consumed
-        // 64 row parts (32 rows, high and low) over the four waves; a lane moves 16 bytes of each
-#pragma unroll 4
-        for (int i = 0; i < 16; i++) {
-            const int part = 16 * wave + i, row = part & 31, low = part >> 5;
-            if (16 * lane < 2 * cols)
-                to_lds(a16 + (size_t)src_row[row] * pf_half_row(a_cols) + (size_t)low * a_cols + c0 + 8 * lane,
-                       reinterpret_cast<unsigned char *>(tile + ((size_t)low * 32 + row) * PLAIN_PITCH));
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (fmt == PF_Q2_K) {
-            // sums of the staged rows over every 16 columns, as two-part halfs like the values themselves:
-            // thread = (row, four neighbouring groups)
-            const int row = threadIdx.x >> 3, g0 = 4 * (threadIdx.x & 7);
+    PlainRow rows[S];
 #pragma unroll
-            for (int g = g0; g < g0 + 4; g++) {
-                float total = 0.0f;
-                if (16 * g < cols) {
-                    const half_t *hi = tile + (size_t)row * PLAIN_PITCH + 16 * g, *lo = hi + 32 * PLAIN_PITCH;
-                    const half8v a0 = *reinterpret_cast<const half8v *>(hi), a1 = *reinterpret_cast<const half8v *>(hi + 8);
-                    const half8v b0 = *reinterpret_cast<const half8v *>(lo), b1 = *reinterpret_cast<const half8v *>(lo + 8);
+    for (int q = 0; q < S; q++)
+        rows[q] = MODE == PF_GEMM_GATE_UP ? plain_row(a, t0 + q, ex, min(row0, limit - 1)) : plain_row(a, t0, ex, min(row0 + 32 * q, limit - 1));
+    const PlainTile staged = {tile, sums, a16, src_row, a_cols};
+    float16v acc[S];
 #pragma unroll
-                    for (int i = 0; i < 8; i++) total += ((float)a0[i] + (float)b0[i]) + ((float)a1[i] + (float)b1[i]);
-                }
-                const half_t top = (half_t)total;
-                sums[(size_t)row * PLAIN_SUMS + g] = top;
-                sums[(size_t)(32 + row) * PLAIN_SUMS + g] = (half_t)(total - (float)top);
-            }
-            __syncthreads();
-        }
-        if (active) {
-            const half_t *mine = sums + (size_t)n * PLAIN_SUMS;
-            if (fmt == PF_Q8_0) plain_product<PF_Q8_0>(r0, r1, ahi, alo, mine, 32 * PLAIN_SUMS, c0, cols, h, part, parts, acc0, acc1);
-            else if (fmt == PF_MXFP4) plain_product<PF_MXFP4>(r0, r1, ahi, alo, mine, 32 * PLAIN_SUMS, c0, cols, h, part, parts, acc0, acc1);
-            else plain_product<PF_Q2_K>(r0, r1, ahi, alo, mine, 32 * PLAIN_SUMS, c0, cols, h, part, parts, acc0, acc1);
-        }
-    }
+    for (int q = 0; q < S; q++) acc[q] = float16v{0};
+    if (fmt == PF_Q8_0) plain_passes<PF_Q8_0, S>(staged, rows, active, part, parts, acc);
+    else if (fmt == PF_MXFP4) plain_passes<PF_MXFP4, S>(staged, rows, active, part, parts, acc);
+    else plain_passes<PF_Q2_K, S>(staged, rows, active, part, parts, acc);
     if (split) {   // every wave is active here: the partial sums of waves 1..3 go through LDS (over the staged columns)
         __syncthreads();
         float *partial = reinterpret_cast<float *>(plain_lds);
         if (wave) {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                partial[((wave - 1) * 32 + r) * 64 + lane] = acc0[r];
-                partial[((wave - 1) * 32 + 16 + r) * 64 + lane] = acc1[r];
+                partial[((wave - 1) * 32 + r) * 64 + lane] = acc[0][r];
+                partial[((wave - 1) * 32 + 16 + r) * 64 + lane] = acc[1][r];
             }
         }
         __syncthreads();
@@ -1208,27 +1243,27 @@ __global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int to
         for (int w = 0; w < 3; w++) {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                acc0[r] += partial[(w * 32 + r) * 64 + lane];
-                acc1[r] += partial[(w * 32 + 16 + r) * 64 + lane];
+                acc[0][r] += partial[(w * 32 + r) * 64 + lane];
+                acc[1][r] += partial[(w * 32 + 16 + r) * 64 + lane];
             }
         }
     }
     if (!active) return;
-    // epilogue: the lane holds column n of its two tiles; register r is row 8 (r / 4) + 4 h + r % 4
+    // epilogue: the lane holds column n of its tiles; register r is row 8 (r / 4) + 4 h + r % 4
 #pragma unroll
     for (int r = 0; r < 16; r++) {
         const int m = 8 * (r >> 2) + 4 * h + (r & 3);
         if (m >= rows_here) continue;
         const float rs = src_scale[m];
         if (MODE == PF_GEMM_GATE_UP) {
-            if (row_a >= limit) continue;
-            const float v = pf_silu(acc0[r] * rs) * (acc1[r] * rs);
-            if (shared) a.shared_act[(size_t)(m0 + m) * inter + row_a] = v;
-            else a.act[(size_t)(first + m0 + m) * inter + row_a] = v;
+            if (row0 >= limit) continue;
+            const float v = pf_silu(acc[0][r] * rs) * (acc[1][r] * rs);
+            if (shared) a.shared_act[(size_t)(m0 + m) * inter + row0] = v;
+            else a.act[(size_t)(first + m0 + m) * inter + row0] = v;
         } else {
             float *out = a.down + (size_t)(first + m0 + m) * a.hidden;
-            if (row_a < limit) out[row_a] = acc0[r] * rs;
-            if (row_b < limit) out[row_b] = acc1[r] * rs;
+#pragma unroll
+            for (int q = 0; q < S; q++) if (row0 + 32 * q < limit) out[row0 + 32 * q] = acc[q][r] * rs;
         }
     }
 }
