@@ -103,6 +103,56 @@ __device__ __forceinline__ bool pf_output_commit(const PfKernelArgs &a, int t, i
     return ok;
 }
 
+// The same for four neighbouring columns, 16 bytes at a time where every row of the target starts on a 16-byte boundary
+// (pf_output_quads, uniform).
+__device__ __forceinline__ bool pf_output_quads(const PfKernelArgs &a) {
+    if (!a.hc_residual) return (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 && a.y_pitch % 4 == 0;
+    return (reinterpret_cast<uintptr_t>(a.hc_residual) & 15) == 0 && a.hc_token_pitch % 4 == 0 && a.hc_stream_pitch % 4 == 0;
+}
+struct PfOutputQuad { float4 r[PF_HC_FOLD_MAX]; };
+__device__ __forceinline__ void pf_output_quad_prefetch(const PfKernelArgs &a, int t, int n, bool quads, PfOutputQuad &q) {
+    if (!a.hc_residual) return;
+    const float *r = a.hc_residual + (size_t)t * a.hc_token_pitch + n;
+#pragma unroll
+    for (int h = 0; h < PF_HC_FOLD_MAX; h++) {
+        if (h >= a.hc_streams) continue;
+        const float *s = r + (size_t)h * a.hc_stream_pitch;
+        q.r[h] = quads ? *reinterpret_cast<const float4 *>(s) : make_float4(s[0], s[1], s[2], s[3]);
+    }
+}
+__device__ __forceinline__ void pf_store_quad(float *at, const float4 &v, bool quads) {
+    if (quads) { *reinterpret_cast<float4 *>(at) = v; return; }
+    at[0] = v.x; at[1] = v.y; at[2] = v.z; at[3] = v.w;
+}
+__device__ __forceinline__ bool pf_finite(const float4 &v) { return pf_finite(v.x) && pf_finite(v.y) && pf_finite(v.z) && pf_finite(v.w); }
+__device__ __forceinline__ bool pf_output_quad_commit(const PfKernelArgs &a, int t, int n, bool quads, const float4 &value, const PfOutputQuad &q) {
+#pragma clang fp contract(off)
+    if (!a.hc_residual) {
+        pf_store_quad(a.y + (size_t)t * a.y_pitch + n, value, quads);
+        return pf_finite(value);
+    }
+    bool ok = true;
+    float *r = a.hc_residual + (size_t)t * a.hc_token_pitch + n;
+    const float *w = a.hc_inject + (size_t)t * a.hc_streams;
+#pragma unroll
+    for (int h = 0; h < PF_HC_FOLD_MAX; h++) {
+        if (h >= a.hc_streams) continue;
+        const float px = w[h] * value.x, py = w[h] * value.y, pz = w[h] * value.z, pw = w[h] * value.w;
+        const float4 result = make_float4(q.r[h].x + px, q.r[h].y + py, q.r[h].z + pz, q.r[h].w + pw);
+        pf_store_quad(r + (size_t)h * a.hc_stream_pitch, result, quads);
+        ok &= pf_finite(result);
+    }
+    return ok;
+}
+
+// Threads of a workgroup that takes a row of `quads` 16-byte pieces in rounds: as few rounds as 320 threads allow, and the
+// fewest whole waves for that many rounds (640 pieces: two rounds of 320 threads instead of two and a half of 256).
+#define PF_ROW_THREADS 320
+inline unsigned pf_row_threads(unsigned quads) {
+    const unsigned rounds = (quads + PF_ROW_THREADS - 1) / PF_ROW_THREADS;
+    return rounds ? ((quads + rounds - 1) / rounds + 63) / 64 * 64 : 64;
+}
+
 struct PfHipMoe {
     PfHipMoeDesc desc;
     uint8_t *w[8];
