@@ -223,7 +223,7 @@ void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hip
 }
 
 // ---- router logits by FP32 MFMA ----------------------------------------------------------------
-// Workgroup = one 32-token x 32-expert tile, its four waves a quarter of the columns each (the
+// Workgroup = a tile of 32 TR tokens x 32 TC experts, its eight waves an eighth of the columns each (the
 // partial tiles are added in wave order).  Also writes the routing tolerance's bound on the sum of
 // squared products, max(x)^2 * |w_e|^2.  (The shared router's logit comes from pf_k_rows_to_half.)
 //
@@ -239,73 +239,88 @@ void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hip
 // wave's alone, so no barrier is needed before the partial tiles meet.
 typedef float float4v __attribute__((ext_vector_type(4)));
 #define PF_ROUTER_PITCH 36   // floats between rows of a staged piece: eight neighbouring lanes' 16-byte reads cover all banks
-__global__ void __launch_bounds__(256) pf_k_pf_router(PfKernelArgs a, int tokens) {
-    __shared__ float partial[3][16][64];
-    __shared__ __align__(16) float staged[4][2][32 * PF_ROUTER_PITCH];   // [wave][x | w][row][column]
+#define PF_ROUTER_WAVES 8
+#define PF_ROUTER_LDS(TR, TC) (PF_ROUTER_WAVES * ((TR) + (TC)) * 32 * PF_ROUTER_PITCH * 4)
+// Bound by the matrix cores (two thirds of a wave's life at 2048 tokens, the rest waits for first loads and the sums at the
+// end).  1024 tokens, 512 experts, rows of 2048: 28.1 us with 64 x 32 tiles, 30.7 with 32 x 32 (a workgroup reads 96 rows
+// for two of their tiles, instead of 128); 2048 tokens, rows of 2560: 66.8 us, 67.7.
+template <int TR, int TC>
+__global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_waves_per_eu(2))) pf_k_pf_router(PfKernelArgs a, int tokens) {
+    extern __shared__ __align__(16) float router_lds[];   // [wave][x rows, then experts][column]; later the waves' partial tiles
     const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = threadIdx.x >> 6;
-    const int t0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
+    const int t0 = blockIdx.x * 32 * TR, e0 = blockIdx.y * 32 * TC;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.route_flags[0] = 0;   // the routing's list starts empty
     const int i = lane & 31, kk = lane >> 5;
-    // the four waves split the rows' 128-byte lines (hidden is a multiple of 32)
-    const int lines = H / 32, l0 = lines * wave / 4, l1 = lines * (wave + 1) / 4;
+    // the waves split the rows' 128-byte lines (hidden is a multiple of 32)
+    const int lines = H / 32, l0 = lines * wave / PF_ROUTER_WAVES, l1 = lines * (wave + 1) / PF_ROUTER_WAVES;
     const int lr = lane >> 3, piece = lane & 7;   // fetch: row within a group of eight, 16-byte piece of the line
-    const float4v *xsrc[4], *wsrc[4];
+    constexpr int ROWS = 4 * (TR + TC);           // groups of eight rows
+    const float4v *src[ROWS];
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const int t = min(t0 + 8 * g + lr, tokens - 1), e = min(e0 + 8 * g + lr, E - 1);
-        xsrc[g] = reinterpret_cast<const float4v *>(a.x + (size_t)t * a.x_pitch) + piece;
-        wsrc[g] = reinterpret_cast<const float4v *>(a.w[0] + (size_t)e * H * 4) + piece;
+    for (int g = 0; g < ROWS; g++) {
+        const int r = 8 * g + lr;
+        src[g] = (g < 4 * TR ? reinterpret_cast<const float4v *>(a.x + (size_t)min(t0 + r, tokens - 1) * a.x_pitch)
+                             : reinterpret_cast<const float4v *>(a.w[0] + (size_t)min(e0 + r - 32 * TR, E - 1) * H * 4)) + piece;
     }
-    float *xs = staged[wave][0], *ws = staged[wave][1];
-    float16v acc = {0};
-    if (l0 < l1) {
-        float4v xg[4], wg[4];
+    float *mine = router_lds + (size_t)wave * (TR + TC) * 32 * PF_ROUTER_PITCH;
+    float16v acc[TR][TC];
 #pragma unroll
-        for (int g = 0; g < 4; g++) { xg[g] = xsrc[g][8 * l0]; wg[g] = wsrc[g][8 * l0]; }
+    for (int r = 0; r < TR; r++)
+#pragma unroll
+        for (int c = 0; c < TC; c++) acc[r][c] = float16v{0};
+    if (l0 < l1) {
+        float4v fetched[ROWS];
+#pragma unroll
+        for (int g = 0; g < ROWS; g++) fetched[g] = src[g][8 * l0];
         for (int l = l0; l < l1; l++) {
             // the piece fetched last into LDS (after the reads of the piece before it, in the wave's program order),
             // then the next one's loads on their way (the last step fetches its own piece again; two pieces ahead
             // measured no faster)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                *reinterpret_cast<float4v *>(xs + (8 * g + lr) * PF_ROUTER_PITCH + 4 * piece) = xg[g];
-                *reinterpret_cast<float4v *>(ws + (8 * g + lr) * PF_ROUTER_PITCH + 4 * piece) = wg[g];
-            }
+            for (int g = 0; g < ROWS; g++) *reinterpret_cast<float4v *>(mine + (8 * g + lr) * PF_ROUTER_PITCH + 4 * piece) = fetched[g];
             const int next = l + 1 < l1 ? l + 1 : l;
 #pragma unroll
-            for (int g = 0; g < 4; g++) { xg[g] = xsrc[g][8 * next]; wg[g] = wsrc[g][8 * next]; }
-            float4v xv[4], wv[4];
+            for (int g = 0; g < ROWS; g++) fetched[g] = src[g][8 * next];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                xv[c] = *reinterpret_cast<const float4v *>(xs + i * PF_ROUTER_PITCH + 4 * (2 * c + kk));
-                wv[c] = *reinterpret_cast<const float4v *>(ws + i * PF_ROUTER_PITCH + 4 * (2 * c + kk));
-            }
+            for (int s = 0; s < 4; s++) {
+                float4v v[TR + TC];
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[c].x, wv[c].x, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[c].y, wv[c].y, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[c].z, wv[c].z, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[c].w, wv[c].w, acc, 0, 0, 0);
+                for (int q = 0; q < TR + TC; q++)
+                    v[q] = *reinterpret_cast<const float4v *>(mine + (32 * q + i) * PF_ROUTER_PITCH + 4 * (2 * s + kk));
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int r = 0; r < TR; r++)
+#pragma unroll
+                        for (int c = 0; c < TC; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[r][k], v[TR + c][k], acc[r][c], 0, 0, 0);
             }
         }
     }
-    if (wave > 0) {
+    __syncthreads();   // the staged pieces have been read
+    constexpr int REGS = 16 * TR * TC;
 #pragma unroll
-        for (int r = 0; r < 16; r++) partial[wave - 1][r][lane] = acc[r];
-    }
+    for (int r = 0; r < REGS; r++) router_lds[(wave * REGS + r) * 64 + lane] = acc[r / 16 / TC][r / 16 % TC][r % 16];
     __syncthreads();
-    if (wave > 0) return;
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = ((acc[r] + partial[0][r][lane]) + partial[1][r][lane]) + partial[2][r][lane];
-    const int col = e0 + i;   // this lane's expert
-    const float wn = col < E ? a.w_norm2[col] : 0.0f;
+    for (int q = 0; q < REGS / PF_ROUTER_WAVES; q++) {   // added in wave order
+        const int r = wave + PF_ROUTER_WAVES * q;
+        float logit = router_lds[r * 64 + lane];
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int row = t0 + 8 * (r >> 2) + 4 * kk + (r & 3);
+        for (int w = 1; w < PF_ROUTER_WAVES; w++) logit += router_lds[(w * REGS + r) * 64 + lane];
+        const int row = t0 + 32 * (r / 16 / TC) + 8 * ((r & 15) >> 2) + 4 * kk + (r & 3), col = e0 + 32 * (r / 16 % TC) + i;
         if (row >= tokens || col >= E) continue;
-        a.logits[(size_t)row * E + col] = acc[r];
-        a.logit_ssq[(size_t)row * E + col] = a.x_max2[row] * wn;
+        a.logits[(size_t)row * E + col] = logit;
+        a.logit_ssq[(size_t)row * E + col] = a.x_max2[row] * a.w_norm2[col];
     }
+}
+template <int TR, int TC>
+static void launch_router(const PfKernelArgs &a, int tokens, hipStream_t stream) {
+    static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_router<TR, TC>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       PF_ROUTER_LDS(TR, TC)) == hipSuccess;   // more than the default 64 KB
+    (void)configured;
+    const dim3 grid((tokens + 32 * TR - 1) / (32 * TR), (a.experts + 32 * TC - 1) / (32 * TC));
+    hipLaunchKernelGGL((pf_k_pf_router<TR, TC>), grid, dim3(64 * PF_ROUTER_WAVES), PF_ROUTER_LDS(TR, TC), stream, a, tokens);
 }
 
 // ---- grouped product ------------------------------------------------------------------------------
@@ -1391,7 +1406,14 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     // tile of full depth, and 544 workgroups do not spread evenly over 256 compute units, 512 do)
     hipLaunchKernelGGL(pf_k_rows_to_half, dim3(tokens), dim3(256), 0, stream, a.x, a.x_pitch, H, (half_t *)a.x16, a.x_scale,
                        a.x_max2, a.error_word, reinterpret_cast<const float *>(a.w[7]), a.shared_scale);
-    hipLaunchKernelGGL(pf_k_pf_router, dim3((tokens + 31) / 32, (E + 31) / 32), dim3(256), 0, stream, a, tokens);
+    // the tile whose rounds over the chip are the least matrix work, the larger of two equal ones
+    auto work = [&](int tr, int tc) {
+        const long tiles = (long)((tokens + 32 * tr - 1) / (32 * tr)) * ((E + 32 * tc - 1) / (32 * tc));
+        return (tiles + 255) / 256 * tr * tc;
+    };
+    if (work(2, 2) <= work(2, 1) && work(2, 2) <= work(1, 1)) launch_router<2, 2>(a, tokens, stream);
+    else if (work(2, 1) <= work(1, 1)) launch_router<2, 1>(a, tokens, stream);
+    else launch_router<1, 1>(a, tokens, stream);
     if (last < 2) return;
     // stage 2: routes and grouping
     pf_launch_route(a, tokens, stream);
