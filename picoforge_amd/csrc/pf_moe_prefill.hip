@@ -22,6 +22,7 @@
 // order and the 2^-22 activation rounding only.
 #include "pf_moe_internal.h"
 #include "pf_upload_addr.h"
+#include "pf_plain_walk.h"
 
 typedef _Float16 half_t;
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -1130,26 +1131,23 @@ __device__ __forceinline__ void plain_product(const PlainBatch<PF_Q2_K, S> &w, c
     }
 }
 
-#define PLAIN_CHUNK 512                     // activation columns staged per pass (256, three workgroups a compute unit: slower)
+#define PLAIN_CHUNK PF_PLAIN_CHUNK          // activation columns staged per pass (256, three workgroups a compute unit: slower)
 #define PLAIN_PITCH (PLAIN_CHUNK + 8)       // halfs between staged rows: 16 bytes of padding spread the rows over the banks
 #define PLAIN_SUMS (PLAIN_CHUNK / 16 + 8)   // halfs between the rows' sums over 16 columns
 #define PLAIN_TILE_BYTES (2 * 32 * PLAIN_PITCH * 2)
 #define PLAIN_LDS (PLAIN_TILE_BYTES + 2 * 32 * PLAIN_SUMS * 2)
 
 // Stages PLAIN_CHUNK columns of the tile's 32 activation rows (high and low parts), one 1 KB row part per load instruction, and
-// multiplies them, pass after pass.  A wave takes every `parts`-th batch starting with batch `part`: with parts > 1 the waves
-// of a workgroup share one pair of rows and their partial sums are added afterwards.
+// multiplies them, pass after pass (pf_plain_walk.h).  A wave takes every `parts`-th batch of the row starting with batch
+// `part`: with parts > 1 the waves of a workgroup share one pair of rows and their partial sums are added afterwards.
 struct PlainTile { half_t *tile, *sums; const half_t *a16; const uint32_t *src_row; int a_cols; };
 template <int FMT, int S>
 __device__ __forceinline__ void plain_passes(const PlainTile &a, const PlainRow (&rows)[S], bool active, int part, int parts, float16v (&acc)[S]) {
     typedef PlainBatch<FMT, S> Batch;
     const int lane = pf_lane(), wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
-    const int batches = (a.a_cols + Batch::COLS - 1) / Batch::COLS;
     const half_t *ahi = a.tile + (size_t)n * PLAIN_PITCH, *alo = ahi + 32 * PLAIN_PITCH;
     Batch w, next;
-    if (active && part < batches) next.load(rows, part, h);   // on their way while the first columns are staged
-    for (int c0 = 0; c0 < a.a_cols; c0 += PLAIN_CHUNK) {
-        const int cols = min(PLAIN_CHUNK, a.a_cols - c0);
+    auto stage = [&](int c0, int cols) {
         if (c0) __syncthreads();   // the previous pass has been consumed
         // 64 row parts (32 rows, high and low) over the four waves; a lane moves 16 bytes of each
 #pragma unroll 4
@@ -1181,14 +1179,9 @@ __device__ __forceinline__ void plain_passes(const PlainTile &a, const PlainRow 
             }
             __syncthreads();
         }
-        if (!active) continue;
-        for (int k0 = Batch::COLS * part; k0 < cols; k0 += Batch::COLS * parts) {
-            w = next;
-            const int after = (c0 + k0) / Batch::COLS + parts;
-            if (after < batches) next.load(rows, after, h);
-            plain_product(w, ahi, alo, a.sums + (size_t)n * PLAIN_SUMS, 32 * PLAIN_SUMS, k0, cols, h, acc);
-        }
-    }
+    };
+    pf_plain_walk(a.a_cols, Batch::COLS, part, parts, active, stage, [&](int batch) { next.load(rows, batch, h); }, [&] { w = next; },
+                  [&](int k0, int cols) { plain_product(w, ahi, alo, a.sums + (size_t)n * PLAIN_SUMS, 32 * PLAIN_SUMS, k0, cols, h, acc); });
 }
 
 // grid: (row tiles the list can hold) x slabs; 4 waves.  Items whose tensors are in a format of the ring

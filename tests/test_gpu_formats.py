@@ -207,3 +207,19 @@ def test_full_size_profile_layers(product, oracle, profile):
         _, yg, idsg, wg = layer.forward(x)
         assert_parity(y, ids, w, yg, idsg, wg, label="chunk against the general kernels")
     print(f"  max abs err {worst:.2e}", flush=True)
+
+
+# a shared expert in Q2_K, whose gate and up products split their columns over the four waves of a workgroup: a round of
+# staged columns holds two of its 256-blocks, fewer than the waves (one round, two, a last one half full, four, five)
+@pytest.mark.parametrize("gtype", [abi.GGUF_Q4_K, abi.GGUF_IQ2_XXS])
+@pytest.mark.parametrize("h", [512, 768, 1024, 2048, 2560])
+def test_prefill_kernels_with_a_q2k_shared_expert(product, oracle, h, gtype):
+    print(f"case prefill type={gtype}, shared expert Q2_K, h={h}", flush=True)
+    cfg = abi.moe_config(h, 16, 4, 256, 256)
+    weights, x = make_layer_inputs(cfg, gtype, 37, seed=h + gtype, shared_type=abi.GGUF_Q2_K)
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, 37) as layer:
+        assert product.hip.moe_kernel_family(*layer.device_handles(), 37) == 2, "the prefill kernels do not cover this layer"
+        for tokens in (5, 37):
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"h={h} T={tokens}")
