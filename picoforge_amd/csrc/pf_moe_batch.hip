@@ -555,9 +555,15 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
     for (int w = 0; w < 16; w++) sum += staged[w][0][64 * wave + lane];   // register `wave` of every wave, in wave order
     const int t = t0 + 4 * kk + (wave & 3), e = e0 + i;
     if (t < tokens && e < E) {
-        (wave < 4 ? a.logits : a.logit_ssq)[(size_t)t * E + e] = sum;
-        // a nonfinite activation makes every product with it nonfinite, and a sum with such a term stays so
-        if (!pf_finite(sum)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
+        if (wave < 4) {
+            a.logits[(size_t)t * E + e] = sum;
+            // a nonfinite activation makes every product with it nonfinite, and a sum with such a term stays so
+            if (!pf_finite(sum)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
+        } else {
+            // the squares of finite values beyond 1.8e19 are infinite (times a zero: NaN) where the logit is finite: a
+            // tolerance without bound, so that the token is routed in serial order
+            a.logit_ssq[(size_t)t * E + e] = pf_finite(sum) ? sum : INFINITY;
+        }
     }
 }
 

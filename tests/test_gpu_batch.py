@@ -36,3 +36,24 @@ def test_batches_of_a_few_rows_per_expert(product, oracle, h, e, k, i, s, physic
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
         np.testing.assert_array_equal(y, layer.forward(x[:tokens])[1], err_msg="not deterministic")
+
+
+@pytest.mark.parametrize("router", [0.0, 1e-19])
+def test_activations_whose_squares_overflow(product, oracle, router):
+    """A finite activation of 2e19 that the router and the experts all but ignore: its square is infinite, the logits, the
+    routes and the outputs are ordinary.  router: the magnitude of the router's weights in its column (0: inf * 0 in the
+    sums of squares; 1e-19: an infinite sum, products of about two)."""
+    cfg = abi.moe_config(512, 32, 6, 256, 256)
+    weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, 65, seed=23)
+    rows = weights.raw[0].view(np.float32).reshape(cfg.experts, cfg.hidden_size)
+    rows[:, 0] = router * np.linspace(-1.0, 1.0, cfg.experts, dtype=np.float32)
+    weights.raw[7].view(np.float32)[0] = 0.0
+    for j in (1, 2, 4, 5):
+        weights.raw[j].reshape(-1, cfg.hidden_size // 256, 144)[:, 0] = 0   # the first 256 columns of gate and up
+    x[::3, 0] = 2e19
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, 65) as layer:
+        for tokens in (33, 65):
+            print(f"case squares overflow, router {router}, {tokens} tokens", flush=True)
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
