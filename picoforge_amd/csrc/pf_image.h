@@ -1,5 +1,5 @@
-// Digit images of activation rows and the scalar pieces of the block formats that the kernels with integer products share
-// (pf_moe_decode.hip, pf_moe_batch.hip).
+// Digit images of the decode kernels' activation rows (pf_moe_decode.hip), and the lane moves and scalar pieces of the block
+// formats that they share with the other kernels with integer products (pf_moe_batch.hip, whose images are finer).
 #pragma once
 #include "pf_moe_internal.h"
 

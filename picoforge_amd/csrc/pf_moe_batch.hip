@@ -8,18 +8,21 @@
 //   pf_k_batch_gate_up   gate and up products of 32 units, SwiGLU, the activation rows' digit images (expert order)
 //   pf_k_batch_down      down products of 128 output rows, FP32, in expert order (pf_k_pf_combine adds them up)
 //
-// Arithmetic: the decode kernels'.  Activations are digit images (24-bit integers per 32-group as three balanced base-256
-// digits), weight codes signed bytes, the group's dot product exact in integers, the group's scale and minimum applied in
-// FP32.  The integer products run on v_mfma_i32_32x32x32_i8, one instruction per 32-group:
+// Arithmetic: as the decode kernels', on finer images.  Activations are digit images: integers relative to a power of two
+// per 32-group, 2^-29 of its largest magnitude's binade, as four balanced base-256 digits (a 32-bit value within 2^6 of the
+// largest is exact, a smaller one is off by at most 2^-30 of it).  Weight codes are signed bytes, the group's dot product
+// exact in integers, the group's scale and minimum applied in FP32.  With the decode kernels' three digits the activation
+// rows' rounding showed: 60 tokens of an IQ2_XXS layer 2.9e-7 off the result in 64 bits (2-norm) where FP32 sums of FP32
+// rows (the general kernels) are 2.4e-7 off, now 1.9e-7; 101 tokens of the q2 profile 322 -> 328 us.  The integer products run on v_mfma_i32_32x32x32_i8, one instruction per 32-group:
 //
 //   A (rows)     lane (m = lane % 32, h = lane / 32): digit plane m % 4 of the chunk's token m / 4, bytes 16 h .. 16 h + 15
-//                of the group (plane 3 repeats plane 2; its results are not looked at)
+//                of the group
 //   B (columns)  lane (n = lane % 32, h): weight row n's codes 16 h .. 16 h + 15 of the group
 //   D            lane (n, h), register 4 q + p: weight row n, token 2 q + h, plane p
 //
-// so the three planes of a (row, token) sum meet in one lane, the lane's weight row is the one whose scales it holds, and a
+// so the planes of a (row, token) sum meet in one lane, the lane's weight row is the one whose scales it holds, and a
 // chunk of up to 2 q tokens only recombines q of the four register quads.  Per 32 x 32 weights: 6 (Q4_K) to 28 (MXFP4)
-// vector instructions for the codes, about 5 for the scales, 7 per quad -- against 36 per token for the dot-product
+// vector instructions for the codes, about 5 for the scales, 8 per quad -- against 36 per token for the dot-product
 // instructions of the decode kernels and about 75, whatever the rows, for the FP16 product of the prefill kernels.
 #include "pf_moe_internal.h"
 #include "pf_image.h"
@@ -219,9 +222,9 @@ template <bool ROWS> struct BatchRows<PF_Q2_K, ROWS> {
 // ---- a chunk's rows against a piece ------------------------------------------------------------------
 struct BatchFactor { float step, sum; };   // a (token, group)'s step, and step * sum of the group's integers
 
-__device__ __forceinline__ float batch_value(const int16v &d, int q) {
-    return fmaf(65536.0f, (float)d[4 * q + 2], (float)(d[4 * q] + (d[4 * q + 1] << 8)));
-}
+// the upper and the lower pair of planes of a sum: at most 28 bits each
+__device__ __forceinline__ float batch_upper(const int16v &d, int q) { return (float)(d[4 * q + 2] + (d[4 * q + 3] << 8)); }
+__device__ __forceinline__ float batch_lower(const int16v &d, int q) { return (float)(d[4 * q] + (d[4 * q + 1] << 8)); }
 
 // acc[s][q] += the products of set s's piece with tokens 2 q + h of the chunk
 template <int FMT, bool ROWS, int SETS, int QUADS>
@@ -244,10 +247,13 @@ __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS
 #pragma unroll
             for (int q = 0; q < QUADS; q++) {
                 const BatchFactor f = factors[16 * q + g];
-                if (Rows::MIN_OPERAND) {
-                    acc[s][q] = fmaf(f.step, fmaf(scale, batch_value(d[s], q), -minimum * batch_value(m[s], q)), acc[s][q]);
+                if (Rows::MIN_OPERAND) {   // the two products nearly cancel: their difference pair by pair, the upper one's with what its product lost
+                    const float mu = batch_upper(m[s], q), product = minimum * mu;
+                    const float upper = fmaf(scale, batch_upper(d[s], q), -product) - fmaf(minimum, mu, -product);
+                    const float lower = fmaf(scale, batch_lower(d[s], q), -minimum * batch_lower(m[s], q));
+                    acc[s][q] = fmaf(f.step, fmaf(65536.0f, upper, lower), acc[s][q]);
                 } else {
-                    acc[s][q] = fmaf(f.step * batch_value(d[s], q), scale, acc[s][q]);
+                    acc[s][q] = fmaf(f.step * fmaf(65536.0f, batch_upper(d[s], q), batch_lower(d[s], q)), scale, acc[s][q]);
                     if (Rows::MINIMA) acc[s][q] = fmaf(-f.sum, minimum, acc[s][q]);
                 }
             }
@@ -261,17 +267,17 @@ __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS
 template <int GROUPS>
 __device__ __forceinline__ void batch_operands(int4v (&x)[GROUPS], BatchFactor *factors, const uint32_t *images, uint32_t at, uint32_t factor_at,
                                                int piece, int groups, int lane) {
-    const uint32_t mine = at + 8 * (uint32_t)min(lane & 3, PF_IMG_PLANES - 1) + 4 * (uint32_t)(lane >> 5);
+    const uint32_t mine = at + 8 * (uint32_t)(lane & 3) + 4 * (uint32_t)(lane >> 5);
 #pragma unroll
     for (int g = 0; g < GROUPS; g++) {
-        const uint32_t *group = images + PF_IMG_GROUP * min(GROUPS * piece + g, groups - 1);   // uniform
+        const uint32_t *group = images + PF_BIMG_GROUP * min(GROUPS * piece + g, groups - 1);   // uniform
         x[g] = *reinterpret_cast<const int4v *>(group + mine);
     }
     const int fg = GROUPS * piece + (lane & 7), last = min(fg, groups - 1);
-    const float step = fg < groups ? __uint_as_float((images + PF_IMG_GROUP * groups)[factor_at + (uint32_t)last]) : 0.0f;
-    const int sum = (int)(images + (PF_IMG_GROUP + 1) * groups)[factor_at + (uint32_t)last];
+    const float step = fg < groups ? __uint_as_float((images + PF_BIMG_GROUP * groups)[factor_at + (uint32_t)last]) : 0.0f;
+    const float sum = fg < groups ? __uint_as_float((images + (PF_BIMG_GROUP + 1) * groups)[factor_at + (uint32_t)last]) : 0.0f;
     pf_wave_lds_fence();   // the piece before has been read
-    factors[lane] = BatchFactor{step, step * (float)sum};
+    factors[lane] = BatchFactor{step, sum};
     pf_wave_lds_fence();
 }
 
@@ -365,6 +371,57 @@ __device__ __forceinline__ void batch_stage_tables(uint32_t *tables, const PfKer
     __syncthreads();
 }
 
+// A group's step (the power of two that puts its largest magnitude m between 2^29 and 2^30, or the smallest normal one) and
+// the step's inverse.
+__device__ __forceinline__ void batch_step(float m, float &step, float &inv) {
+    const int exponent = max((int)(__float_as_uint(m) >> 23) - 29, 1);
+    step = __uint_as_float((uint32_t)exponent << 23);
+    inv = __uint_as_float((uint32_t)(254 - exponent) << 23);
+}
+// balanced base-256 digits of q, lowest first
+__device__ __forceinline__ void batch_digits(int q, int (&d)[PF_BIMG_PLANES]) {
+#pragma unroll
+    for (int p = 0; p + 1 < PF_BIMG_PLANES; p++) {
+        d[p] = ((q + 128) & 255) - 128;
+        q = (q - d[p]) >> 8;
+    }
+    d[PF_BIMG_PLANES - 1] = q;
+}
+// the sum of a group's integers (36 bits) from the sums of their upper and lower 16 bits
+__device__ __forceinline__ float batch_sum(int upper, int lower) { return fmaf(65536.0f, (float)upper, (float)lower); }
+
+// Thread j of a group of four neighbouring lanes: the eight values 8j..8j+7 of a K-vector into its image.
+__device__ __forceinline__ void batch_image_chunk(uint32_t *img, const float (&v)[8], int j, int K) {
+    float m = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; c++) m = fmaxf(m, fabsf(v[c]));
+    m = fmaxf(m, __int_as_float(dpp_quad_xor1(__float_as_int(m))));
+    m = fmaxf(m, __int_as_float(dpp_quad_xor2(__float_as_int(m))));
+    float step, inv;
+    batch_step(m, step, inv);
+    uint32_t w[PF_BIMG_PLANES][2] = {};
+    int upper = 0, lower = 0;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const int q = __float2int_rn(v[c] * inv);
+        upper += q >> 16;
+        lower += q & 0xffff;
+        int d[PF_BIMG_PLANES];
+        batch_digits(q, d);
+#pragma unroll
+        for (int p = 0; p < PF_BIMG_PLANES; p++) w[p][c >> 2] |= (uint32_t)(d[p] & 255) << (8 * (c & 3));
+    }
+    upper += dpp_quad_xor1(upper); upper += dpp_quad_xor2(upper);
+    lower += dpp_quad_xor1(lower); lower += dpp_quad_xor2(lower);
+    const int g = j >> 2, at = PF_BIMG_GROUP * g + 2 * (j & 3);
+#pragma unroll
+    for (int p = 0; p < PF_BIMG_PLANES; p++) { img[at + 8 * p] = w[p][0]; img[at + 8 * p + 1] = w[p][1]; }
+    if ((j & 3) == 0) {
+        img[PF_BIMG_GROUP * (K / 32) + g] = __float_as_uint(step);
+        img[(PF_BIMG_GROUP + 1) * (K / 32) + g] = __float_as_uint(step * batch_sum(upper, lower));
+    }
+}
+
 // Lanes 0..31 and 32..63, one value each: group g of two K-vectors' images (store: whether the lane's vector exists).
 __device__ __forceinline__ void batch_image_group(uint32_t *img, float v, int g, int K, int lane, bool store) {
     float m = fabsf(v);
@@ -372,21 +429,22 @@ __device__ __forceinline__ void batch_image_group(uint32_t *img, float v, int g,
     for (int k = 0; k < 4; k++) m = fmaxf(m, __int_as_float(dpp_row_step(__float_as_int(m), k)));
     m = fmaxf(m, __shfl_xor(m, 16));
     float step, inv;
-    group_step2(m, step, inv);
+    batch_step(m, step, inv);
     const int q = __float2int_rn(v * inv);
-    int sum = q;
+    int upper = q >> 16, lower = q & 0xffff;
 #pragma unroll
-    for (int k = 0; k < 4; k++) sum += dpp_row_step(sum, k);
-    sum += __shfl_xor(sum, 16);
-    int d[PF_IMG_PLANES];
-    image_digits(q, d);
+    for (int k = 0; k < 4; k++) { upper += dpp_row_step(upper, k); lower += dpp_row_step(lower, k); }
+    upper += __shfl_xor(upper, 16);
+    lower += __shfl_xor(lower, 16);
+    int d[PF_BIMG_PLANES];
+    batch_digits(q, d);
     if (!store) return;
-    uint8_t *bytes = reinterpret_cast<uint8_t *>(img + PF_IMG_GROUP * g);
+    uint8_t *bytes = reinterpret_cast<uint8_t *>(img + PF_BIMG_GROUP * g);
 #pragma unroll
-    for (int p = 0; p < PF_IMG_PLANES; p++) bytes[32 * p + (lane & 31)] = (uint8_t)d[p];
+    for (int p = 0; p < PF_BIMG_PLANES; p++) bytes[32 * p + (lane & 31)] = (uint8_t)d[p];
     if ((lane & 31) == 0) {
-        img[PF_IMG_GROUP * (K / 32) + g] = __float_as_uint(step);
-        img[(PF_IMG_GROUP + 1) * (K / 32) + g] = (uint32_t)sum;
+        img[PF_BIMG_GROUP * (K / 32) + g] = __float_as_uint(step);
+        img[(PF_BIMG_GROUP + 1) * (K / 32) + g] = __float_as_uint(step * batch_sum(upper, lower));
     }
 }
 
@@ -410,8 +468,8 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
     if (32 * tile >= I) return;
     if (batch_tables<FMT>()) batch_stage_tables(tables, a);
     const int groups = a.hidden / 32, K = a.top_k;
-    const uint32_t words = (uint32_t)pf_image2_words(a.hidden);
-    const size_t act_words = pf_image2_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    const uint32_t words = (uint32_t)pf_batch_image_words(a.hidden);
+    const size_t act_words = pf_batch_image_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
     for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         float acc[2][4] = {};
@@ -458,7 +516,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) p
     const int tile = 4 * blockIdx.x + wave;
     if (32 * tile >= H) return;
     const int groups = (it.shared ? a.shared_inter : a.inter) / 32;
-    const uint32_t words = (uint32_t)pf_image2_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    const uint32_t words = (uint32_t)pf_batch_image_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
     for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         auto image_at = [&](int r) { return (uint32_t)(it.first + c0 + r) * words; };
@@ -481,6 +539,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) p
 // a workgroup waits for memory once, and small tiles spread a few tokens over the chip (a 32 x 32 tile keeps a compute
 // unit's matrix cores busy for 7 us, this one for 2 + 2).  A line goes through the wave's own LDS because a product step
 // wants element k of row i from lane (i, k).  The sums of squares (the routing's tolerance) are products of the squares.
+// A logit is summed in four chains a wave and in pairs over the waves: the routes' share of the block's error is then what
+// the other routers' is (8e-8 of the result, 14e-8 with one chain).
 // The last row of workgroups takes a token a wave: its digit image, and the shared router's logit and sigmoid.
 // Measured at a width of 2560: 101 tokens 37 -> 12.7 us, against the decode kernels' router in groups of four tokens (32
 // tokens of width 2048: 14.0 -> 9.6).
@@ -497,7 +557,8 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
         float z = 0.0f;
         for (int j = lane; j < H / 8; j += 64) {
             const float4v p = row[2 * j], q = row[2 * j + 1], u = gate[2 * j], v = gate[2 * j + 1];
-            image2_chunk(a.ximg + (size_t)t * pf_image2_words(H), make_float4(p.x, p.y, p.z, p.w), make_float4(q.x, q.y, q.z, q.w), j, H);
+            const float both[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+            batch_image_chunk(a.ximg + (size_t)t * pf_batch_image_words(H), both, j, H);
 #pragma unroll
             for (int c = 0; c < 4; c++) z = fmaf(p[c], u[c], fmaf(q[c], v[c], z));
         }
@@ -523,7 +584,7 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
         }
     }
     float *xs = staged[wave][0], *ws = staged[wave][1];
-    float4v acc = {0}, sq = {0};
+    float4v part[4] = {}, sq = {0};   // four chains of the logits' sums: a chain's rounding grows with its length
 #pragma unroll
     for (int l = 0; l < ROUTER_LINES; l++) {
         if (l0 + l >= l1) break;
@@ -540,19 +601,25 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
             const float4v w = *reinterpret_cast<const float4v *>(ws + i * ROUTER_PITCH + 16 * c + 4 * kk);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[k], w[k], acc, 0, 0, 0);
+                part[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[k], w[k], part[k], 0, 0, 0);
                 sq = __builtin_amdgcn_mfma_f32_16x16x4f32(x[k] * x[k], w[k] * w[k], sq, 0, 0, 0);
             }
         }
     }
+    const float4v acc = (part[0] + part[1]) + (part[2] + part[3]);
     pf_wave_lds_fence();
 #pragma unroll
     for (int r = 0; r < 4; r++) { xs[64 * r + lane] = acc[r]; xs[64 * (4 + r) + lane] = sq[r]; }   // the wave's own part of LDS: 512 floats
     __syncthreads();
     if (wave >= 8) return;
-    float sum = 0.0f;
+    float sums[16];   // register `wave` of every wave, added in pairs
 #pragma unroll
-    for (int w = 0; w < 16; w++) sum += staged[w][0][64 * wave + lane];   // register `wave` of every wave, in wave order
+    for (int w = 0; w < 16; w++) sums[w] = staged[w][0][64 * wave + lane];
+#pragma unroll
+    for (int n = 8; n; n /= 2)
+#pragma unroll
+        for (int w = 0; w < n; w++) sums[w] = sums[2 * w] + sums[2 * w + 1];
+    const float sum = sums[0];
     const int t = t0 + 4 * kk + (wave & 3), e = e0 + i;
     if (t < tokens && e < E) {
         if (wave < 4) {

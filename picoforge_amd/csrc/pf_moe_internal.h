@@ -33,8 +33,10 @@ struct PfKernelArgs {
     float *act;                      // general path [tokens * top_k, inter]; decode path [unique, tokens, inter]
     float *shared_act;               // [tokens, shared_inter]
     float *shared_scale;             // [tokens] sigmoid of the shared router logit
-    uint32_t *ximg, *aimg;           // decode path, tile-ordered Q4_K: digit images (pf_image2_words) of the token rows, written
-                                     // by kernel 1, and of the activation rows [unique, tokens] then [tokens] shared, by kernel 2
+    uint32_t *ximg, *aimg;           // decode path: digit images (pf_image2_words) of the token rows, written by kernel 1, and of the
+                                     // activation rows [unique, tokens] then [tokens] shared, by kernel 2; a few rows per expert:
+                                     // images (pf_batch_image_words) of the token rows, and of the pairs' activation rows in expert
+                                     // order, then the shared expert's
     uint32_t *uniq;                  // decode path: [0] count, then ids[P], then pair->unique[P], then token masks[P]
     // decode path, one token, the expert stage in one launch (null: three kernels): the workgroups' activation lines
     // (FUSE_REPLICAS copies) and the counter whose value tags a forward's lines, incremented by the router kernel
@@ -180,6 +182,11 @@ struct PfHipMoe {
 #define PF_IMG_PLANES 3                       // signed byte digits per value: 24 bits
 #define PF_IMG_GROUP (8 * PF_IMG_PLANES)      // dwords of one 32-group's digits
 __host__ __device__ constexpr size_t pf_image2_words(size_t K) { return (K / 32) * (PF_IMG_GROUP + 2); }
+// The image of the kernels for a few rows per expert (pf_moe_batch.hip): four digits, a power of two as the step, and the
+// step times the sum of the integers as a float in place of the sum.
+#define PF_BIMG_PLANES 4
+#define PF_BIMG_GROUP (8 * PF_BIMG_PLANES)
+__host__ __device__ constexpr size_t pf_batch_image_words(size_t K) { return (K / 32) * (PF_BIMG_GROUP + 2); }
 
 struct PfHipWork {
     const PfHipMoe *moe;
