@@ -2,15 +2,13 @@
 #include "pf_moe_internal.h"
 #include "pf_moe_debug.h"
 #include "pf_host_calls.h"
+#include "pf_host_rows.h"
 #include "../../include/pf_iq2_codes.h"
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
-#include <atomic>
-#include <condition_variable>
 #include <mutex>
 #include <new>
-#include <thread>
 
 static thread_local char g_error[256] = "";
 
@@ -574,170 +572,34 @@ static hipError_t await_results(const HostBlock &b, const HostResults &r) {
     return hipStreamSynchronize(nullptr);
 }
 
-// Longer batches pass through a ring of PF_RING_SLOTS page-locked pieces that follows the block: the CPU fills or empties
-// some pieces while the others are on their way.  (A hipMemcpy2D on the caller's pageable rows moves them row by row, each
-// with a wait of its own: 777 rows of 8 KB each way took 24.9 ms.)  A piece is large enough that its transfer hides the
-// enqueueing.  One CPU copies at about a fifth of what the link carries, so the pieces are dealt to a few threads.
-#define PF_RING_SLOTS 8
-#define PF_RING_BYTES ((size_t)512 * 1024)
-#define PF_CREW_HELPERS 3                            // besides the calling thread
-#define PF_CREW_FROM ((size_t)1024 * 1024)           // bytes that are worth waking them for (10 to 20 us)
-
-// The helpers, one crew for the process: started with the first workspace that takes longer batches, ended with the last.
-// A call that finds the crew at work for another one copies alone.
-struct CopyCrew {
-    std::mutex busy, lock;
-    std::condition_variable wake, done;
-    std::thread thread[PF_CREW_HELPERS];
-    int helpers = 0, running = 0;
-    unsigned long round = 0;
-    bool quit = false;
-    void (*part)(void *, int, int) = nullptr;
-    void *job = nullptr;
-    void serve(int worker) {
-        unsigned long seen = 0;
-        std::unique_lock<std::mutex> hold(lock);
-        for (;;) {
-            wake.wait(hold, [&] { return quit || round != seen; });
-            if (quit) return;
-            seen = round;
-            hold.unlock();
-            part(job, worker, helpers + 1);
-            hold.lock();
-            if (--running == 0) done.notify_one();
-        }
-    }
-    CopyCrew() {
-        for (; helpers < PF_CREW_HELPERS; helpers++) {
-            try { thread[helpers] = std::thread([this, h = helpers] { serve(h + 1); }); } catch (...) { break; }
-        }
-    }
-    ~CopyCrew() {
-        { std::lock_guard<std::mutex> hold(lock); quit = true; }
-        wake.notify_all();
-        for (int h = 0; h < helpers; h++) thread[h].join();
-    }
-    // part(job, worker, workers) by every worker; the calling thread is worker 0
-    void run(void (*f)(void *, int, int), void *j) {
-        { std::lock_guard<std::mutex> hold(lock); part = f; job = j; running = helpers; round++; }
-        wake.notify_all();
-        f(j, 0, helpers + 1);
-        std::unique_lock<std::mutex> hold(lock);
-        done.wait(hold, [&] { return running == 0; });
-    }
-};
-static std::mutex g_crew_lock;
-static CopyCrew *g_crew = nullptr;
-static int g_crew_users = 0;
-static void crew_retain() {
-    std::lock_guard<std::mutex> hold(g_crew_lock);
-    if (g_crew_users++ == 0) g_crew = new (std::nothrow) CopyCrew();
-}
-static void crew_release() {
-    CopyCrew *last = nullptr;
-    {
-        std::lock_guard<std::mutex> hold(g_crew_lock);
-        if (--g_crew_users == 0) { last = g_crew; g_crew = nullptr; }
-    }
-    delete last;
-}
-
-// Rows between the caller's memory (a pitch) and dense device rows.  Piece p goes to worker p % workers, whose own slots its
-// pieces take in turn.
-struct RingJob {
-    PfHipWork *w;
-    uint8_t *device;
-    uint8_t *host;          // the caller's rows
-    size_t pitch, row_bytes, rows, step, pieces;
-    int device_id;
-    bool check;             // in: look for values that are not finite
-    std::atomic<int> error, nonfinite;
-    size_t rows_of(size_t p) const { return rows - p * step < step ? rows - p * step : step; }
-    static int slot_of(size_t p, int workers) {
-        const int per = PF_RING_SLOTS / workers;
-        return (int)(p % workers) * per + (int)(p / workers % per);
-    }
-    void fail(hipError_t e) { int none = 0; if (e != hipSuccess) error.compare_exchange_strong(none, (int)e); }
-};
-static void rows_in(void *dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
-    for (size_t r = 0; r < rows; r++) memcpy((uint8_t *)dst + r * row_bytes, (const uint8_t *)src + r * src_pitch, row_bytes);
-}
-static void rows_out(void *dst, size_t dst_pitch, const void *src, size_t row_bytes, size_t rows) {
-    for (size_t r = 0; r < rows; r++) memcpy((uint8_t *)dst + r * dst_pitch, (const uint8_t *)src + r * row_bytes, row_bytes);
-}
-// whether n floats are finite: an exponent of all ones carries into the sign bit
-static bool finite_floats(const void *p, size_t n) {
-    const uint8_t *bytes = static_cast<const uint8_t *>(p);
-    uint32_t carry = 0;
-    for (size_t i = 0; i < n; i++) {
-        uint32_t bits;
-        memcpy(&bits, bytes + 4 * i, 4);
-        carry |= (bits & 0x7fffffffu) + 0x00800000u;
-    }
-    return !(carry >> 31);
-}
-// A piece on its way, by a kernel that addresses the page-locked memory: 35 GB/s and no wait between engine and kernels,
-// where copies of this size brought 22 GB/s out of the device.
-static void ring_transfer(RingJob *j, int slot, void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
-    if (bytes % 16 == 0) {
-        const uint8_t *ring = j->w->ring;
+// Longer batches pass through the workspace's ring of page-locked pieces (pf_host_rows.h).  A piece travels by a kernel that
+// addresses the page-locked memory: 35 GB/s and no wait between engine and kernels, where copies of this size brought 22 GB/s
+// out of the device.
+static int ring_bind(void *, int device) { return (int)hipSetDevice(device); }
+static int ring_wait(void *work, int slot) { return (int)hipEventSynchronize(static_cast<PfHipWork *>(work)->ring_event[slot]); }
+static int ring_send(void *work, int slot, void *dst, const void *src, size_t bytes, bool in) {
+    PfHipWork *w = static_cast<PfHipWork *>(work);
+    hipError_t e;
+    if (ring_by_kernel(dst, src, bytes)) {
         auto on_device = [&](const void *p) {   // a piece by its device address
             const uint8_t *b = static_cast<const uint8_t *>(p);
-            return b >= ring && b < ring + PF_RING_SLOTS * PF_RING_BYTES ? j->w->host_device + (b - j->w->host) : const_cast<uint8_t *>(b);
+            return b >= w->ring && b < w->ring + PF_RING_SLOTS * PF_RING_BYTES ? w->host_device + (b - w->host) : const_cast<uint8_t *>(b);
         };
         hipLaunchKernelGGL(pf_k_copy_rows, dim3((unsigned)((bytes / 16 + 255) / 256)), dim3(256), 0, nullptr, reinterpret_cast<const uint4 *>(on_device(src)),
                            reinterpret_cast<uint4 *>(on_device(dst)), (int)(bytes / 16));
-        j->fail(hipGetLastError());
+        e = hipGetLastError();
     } else {
-        j->fail(hipMemcpyAsync(dst, src, bytes, kind, nullptr));
+        e = hipMemcpyAsync(dst, src, bytes, in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, nullptr);
     }
-    j->fail(hipEventRecord(j->w->ring_event[slot], nullptr));
-}
-static void ring_in_part(void *job, int worker, int workers) {
-    RingJob *j = static_cast<RingJob *>(job);
-    if (worker) j->fail(hipSetDevice(j->device_id));
-    for (size_t p = worker; p < j->pieces && !j->error.load() && !j->nonfinite.load(); p += workers) {
-        const int slot = RingJob::slot_of(p, workers);
-        const size_t r = p * j->step, n = j->rows_of(p);
-        uint8_t *piece = j->w->ring + slot * PF_RING_BYTES;
-        j->fail(hipEventSynchronize(j->w->ring_event[slot]));   // the piece's last transfer (none yet: returns at once)
-        rows_in(piece, j->host + r * j->pitch, j->pitch, j->row_bytes, n);
-        if (j->check && !finite_floats(piece, n * j->row_bytes / 4)) { j->nonfinite = 1; return; }
-        ring_transfer(j, slot, j->device + r * j->row_bytes, piece, n * j->row_bytes, hipMemcpyHostToDevice);
-    }
-}
-static void ring_send_out(RingJob *j, size_t p, int workers) {
-    const int slot = RingJob::slot_of(p, workers);
-    ring_transfer(j, slot, j->w->ring + slot * PF_RING_BYTES, j->device + p * j->step * j->row_bytes, j->rows_of(p) * j->row_bytes, hipMemcpyDeviceToHost);
-}
-static void ring_out_part(void *job, int worker, int workers) {   // the first PF_RING_SLOTS pieces are on their way
-    RingJob *j = static_cast<RingJob *>(job);
-    if (worker) j->fail(hipSetDevice(j->device_id));
-    const size_t ahead = (size_t)(PF_RING_SLOTS / workers) * workers;
-    for (size_t p = worker; p < j->pieces && !j->error.load(); p += workers) {
-        const int slot = RingJob::slot_of(p, workers);
-        j->fail(hipEventSynchronize(j->w->ring_event[slot]));
-        if (j->error.load()) break;
-        rows_out(j->host + p * j->step * j->pitch, j->pitch, j->w->ring + slot * PF_RING_BYTES, j->row_bytes, j->rows_of(p));
-        if (p + ahead < j->pieces) ring_send_out(j, p + ahead, workers);
-    }
+    const hipError_t recorded = hipEventRecord(w->ring_event[slot], nullptr);
+    return (int)(e != hipSuccess ? e : recorded);
 }
 
 static bool through_ring(const PfHipWork *w, size_t row_bytes) { return w->ring && row_bytes <= PF_RING_BYTES; }
 static void ring_job(RingJob *j, PfHipWork *w, void *device, const void *host, size_t pitch, size_t row_bytes, size_t rows) {
-    j->w = w; j->device = (uint8_t *)device; j->host = (uint8_t *)const_cast<void *>(host);
-    j->pitch = pitch; j->row_bytes = row_bytes; j->rows = rows;
-    j->step = PF_RING_BYTES / row_bytes;
-    j->pieces = (rows + j->step - 1) / j->step;
-    j->device_id = 0;
-    (void)hipGetDevice(&j->device_id);
-    j->check = false;
-    j->error = 0; j->nonfinite = 0;
-}
-// The crew if the rows are worth it and it is free (its `busy` is then held), else null.
-static CopyCrew *crew_for(const RingJob &j) {
-    CopyCrew *crew = j.row_bytes * j.rows >= PF_CREW_FROM ? g_crew : nullptr;   // (a workspace with a ring keeps it alive)
-    return crew && crew->helpers && PF_RING_SLOTS % (crew->helpers + 1) == 0 && crew->busy.try_lock() ? crew : nullptr;
+    int device_id = 0;
+    (void)hipGetDevice(&device_id);
+    j->open({w, device_id, ring_bind, ring_wait, ring_send}, w->ring, device, host, pitch, row_bytes, rows);
 }
 // The caller's rows into device rows, enqueued on the default stream; they have been read when this returns.  nonfinite (may
 // be null): set where a row holds a value that is not finite; what has been sent by then is of no account.
@@ -751,8 +613,7 @@ static hipError_t rows_to_device(PfHipWork *w, void *d_dst, const void *src, siz
     RingJob j;
     ring_job(&j, w, d_dst, src, src_pitch, row_bytes, rows);
     j.check = nonfinite != nullptr;
-    if (CopyCrew *crew = crew_for(j)) { crew->run(ring_in_part, &j); crew->busy.unlock(); }
-    else ring_in_part(&j, 0, 1);
+    ring_rows_in(&j);
     if (nonfinite) *nonfinite = j.nonfinite.load() != 0;
     return (hipError_t)j.error.load();
 }
@@ -1162,13 +1023,9 @@ static int long_results(PfHipWork *work, float *y, size_t y_pitch_bytes, uint32_
     RingJob j;
     ring_job(&j, work, work->y, y, y_pitch_bytes, H * 4, tokens);
     CopyCrew *crew = crew_for(j);
-    const int workers = crew ? crew->helpers + 1 : 1;
-    for (size_t p = 0; p < j.pieces && p < PF_RING_SLOTS; p++) ring_send_out(&j, p, workers);
+    ring_start_out(&j, crew);
     const hipError_t e = await_results(b, r);
-    const bool fine = e == hipSuccess && !j.error.load() && !*r.error_word;
-    if (fine && crew) crew->run(ring_out_part, &j);
-    else if (fine) ring_out_part(&j, 0, 1);
-    if (crew) crew->busy.unlock();
+    ring_rows_out(&j, crew, e == hipSuccess && !*r.error_word);
     HIP_TRY(e);
     HIP_TRY((hipError_t)j.error.load());
     *error_word = *r.error_word;
