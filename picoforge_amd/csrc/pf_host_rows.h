@@ -134,8 +134,11 @@ static inline bool finite_floats(const void *p, size_t n) {
     }
     return !(carry >> 31);
 }
-// Whether a transfer goes by the kernel that moves 16 bytes a thread, else by a copy.
-static inline bool ring_by_kernel(const void *, const void *, size_t bytes) { return bytes % 16 == 0; }
+// Whether a transfer goes by the kernel that moves 16 bytes a thread, else by a copy.  A piece of the ring starts on a 16-byte
+// boundary; a piece's device rows do not where a row is no multiple of 16 bytes.
+static inline bool ring_by_kernel(const void *dst, const void *src, size_t bytes) {
+    return bytes % 16 == 0 && ((uintptr_t)dst | (uintptr_t)src) % 16 == 0;
+}
 
 static inline void ring_in_part(void *job, int worker, int workers) {
     RingJob *j = static_cast<RingJob *>(job);

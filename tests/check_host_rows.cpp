@@ -2,8 +2,8 @@
 // sanitizers by tests/test_host_rows.py.  A "device" is a thread that carries out the enqueued transfers one after the other,
 // as a stream does, so that a piece filled or emptied before its transfer has ended is a race the thread sanitizer sees.
 // Several callers, each with a ring and device rows of its own, send rows in, have the device negate them and fetch them back,
-// at once: the crew is busy for some of them, and comes and goes as callers open and close.  Every row must arrive, and nothing
-// between the rows of a pitch may be touched.
+// at once: the crew is busy for some of them, and comes and goes as callers open and close.  Every 16-byte transfer must start
+// on 16-byte boundaries, every row must arrive, and nothing between the rows of a pitch may be touched.
 #include <stdio.h>
 #include <stdlib.h>
 #include <math.h>
@@ -64,6 +64,10 @@ static int dev_wait(void *self, int slot) {
 static int dev_send(void *self, int slot, void *dst, const void *src, size_t bytes, bool) {
     Device *d = static_cast<Device *>(self);
     { std::lock_guard<std::mutex> hold(d->lock); if (d->sends++ == d->fail_at) return 7; }
+    if (ring_by_kernel(dst, src, bytes)) {   // 16 bytes a thread
+        expect(bytes % 16 == 0, "a 16-byte transfer of another length");
+        expect(((uintptr_t)dst | (uintptr_t)src) % 16 == 0, "a 16-byte transfer off a 16-byte boundary");
+    }
     const unsigned long at = d->enqueue([=] { memcpy(dst, src, bytes); });
     std::lock_guard<std::mutex> hold(d->lock);
     d->slot_at[slot] = at;

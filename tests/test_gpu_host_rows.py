@@ -30,3 +30,13 @@ def test_rows_through_block_ring_and_crew(product, oracle, hidden, batches):
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
             _, y2, _, _ = layer.forward(x[:tokens], want_routes=False)
             np.testing.assert_array_equal(y, y2)
+
+
+def test_pieces_that_start_off_a_16_byte_boundary(product, oracle):
+    """Rows of 132 bytes (33 F32 columns, the general kernels): the second piece of the ring starts 12 bytes off a 16-byte
+    boundary of the device rows, and its 4 rows are a multiple of 16 bytes long."""
+    cfg = abi.moe_config(33, 8, 2, 32, 32)
+    tokens = 512 * 1024 // 132 + 4
+    weights, x = make_layer_inputs(cfg, abi.GGUF_F32, tokens, seed=33, std=0.1)
+    want = forward_with(oracle, cfg, weights, x)
+    assert_parity(*forward_with(product, cfg, weights, x), *want, label=f"hidden 33, {tokens} tokens")
