@@ -102,6 +102,7 @@ WORKLOADS = {
 # what the kernels compute in (every product exact; the result differs from the reference's serial f32 sums by the
 # rounding of the activations and by the order of the additions; observed error <= 1e-5 against a bar of 1e-3)
 DTYPE_DECODE = "i32 dot products of 24-bit block-fixed-point activations with integer weight codes, f32 scales and sums"
+DTYPE_BATCH = "i32 matrix-core products of 30-bit block-fixed-point activations (int8 digits) with integer weight codes, f32 scales and sums"
 DTYPE_PREFILL = "f16 matrix-core products of exact-integer weight operands with two-part f16 activations, f32 accumulation"
 HEADLINE = "q4k_decode"
 ALL_CONFIGS = ["iq2xxs_decode", "q4k_verify4", "q4k_prefill1024", "q4k_stack48"]
@@ -119,6 +120,10 @@ GENERAL_STAGES = ["pf_k_pre (router logits, shared gate/up + SwiGLU, shared gate
                   "routing (top-k, serial-order re-routes)",
                   "pf_k_gate_up (routed gate/up + SwiGLU)",
                   "pf_k_down_combine (routed and shared down products, combine)"]
+BATCH_STAGES = ["pf_k_batch_router (router logits by FP32 MFMA, digit images of x)",
+                "routing + grouping (top-k, serial-order re-routes, histogram/scan/placement)",
+                "pf_k_batch_gate_up (gate/up + SwiGLU by int8 MFMA, digit images of the activations)",
+                "pf_k_batch_down + pf_k_pf_combine (down by int8 MFMA, slot-ordered combine)"]
 PREFILL_STAGES = ["pf_k_rows_to_half + pf_k_pf_router (fp16 copy of x, router logits by FP32 MFMA)",
                   "routing + grouping (top-k, serial-order re-routes, histogram/scan/stable placement)",
                   "pf_k_pf_gemm<gate_up> (grouped gate/up + SwiGLU by FP16 MFMA, then fp16 copy of the activations)",
@@ -313,8 +318,8 @@ def run_layer(args, ctx, name, steps, warmup, cpu_seconds):
     # groups of every forward; a group's duration is the difference between consecutive plans (it includes
     # the dispatch gap before it, as a profiler's start-to-end time of a dependent kernel does).
     family = hip.moe_kernel_family(moe, work, tokens)
-    prefill = family == 2 or (family == 0 and chunk_inputs)   # accounted as a chunk: bytes of the grouped products, tokens per second
-    names = {0: GENERAL_STAGES, 1: DECODE_STAGES, 2: PREFILL_STAGES}[family]
+    prefill = family == 2 or (family != 1 and chunk_inputs)   # accounted as a chunk: bytes of the grouped products, tokens per second
+    names = {0: GENERAL_STAGES, 1: DECODE_STAGES, 2: PREFILL_STAGES, 3: BATCH_STAGES}[family]
     if family == 1 and hip.moe_decode_launches(moe, work, tokens) == 2:
         names = FUSED_DECODE_STAGES
     if family == 1 and hip.moe_decode_launches(moe, work, tokens) == 4:
@@ -355,7 +360,7 @@ def run_layer(args, ctx, name, steps, warmup, cpu_seconds):
         flops = sum(stage_flops)
         extra = {"prefill_tokens_per_s": round(tokens / (ms_per_step * 1e-3), 1),
                  "flops_per_step": flops,
-                 "mfma_frac_of_fp16_dense_peak": round(flops / (ms_per_step * 1e-3) / 1e12 / MFMA_F16_PEAK_TFLOPS, 4),
+                 **({"mfma_frac_of_fp16_dense_peak": round(flops / (ms_per_step * 1e-3) / 1e12 / MFMA_F16_PEAK_TFLOPS, 4)} if family == 2 else {}),
                  "stage_tflops": {names[j].split()[0]: round(stage_flops[j] / (stage_us[j] * 1e-6) / 1e12, 1)
                                   for j in (0, 2, 3)},
                  "binding_roofline": "hbm: about 80 flop per weight byte at this chunk size, below the MFMA ridge"}
@@ -365,7 +370,7 @@ def run_layer(args, ctx, name, steps, warmup, cpu_seconds):
                        unique * lb["down"] + lb["shared_down"]]
         if len(names) == 2:
             stage_bytes = [stage_bytes[0], stage_bytes[1] + stage_bytes[2]]
-        if family == 1 and len(names) == 4:   # the routing launch reads the tokens' logits and their noise terms
+        if family in (1, 3) and len(names) == 4:   # the routing launch reads the tokens' logits and their noise terms
             stage_bytes = [stage_bytes[0], tokens * cfg.experts * 8, stage_bytes[1], stage_bytes[2]]
         if family == 0:
             stage_bytes = [lb["routers"] + lb["shared_gate_up"], tokens * cfg.experts * 8, unique * lb["gate_up"],
@@ -419,7 +424,7 @@ def run_layer(args, ctx, name, steps, warmup, cpu_seconds):
         "ms_per_step_p10_p90": [round(timing["p10"], 6), round(timing["p90"], 6)],
         "timed_replays": timing["replays"], "timed_ms": round(timing["timed_ms"], 2),
         "higher_is_better": False, "scaling": "weak", "vs_baseline": None,
-        "dtype": DTYPE_DECODE if not prefill else DTYPE_PREFILL,
+        "dtype": {1: DTYPE_DECODE, 2: DTYPE_PREFILL, 3: DTYPE_BATCH}.get(family, DTYPE_PREFILL if prefill else DTYPE_DECODE),
         "data": "synthetic",
         "config": {"workload": f"one MoE layer, hidden {cfg.hidden_size}, {cfg.experts} experts, top-{cfg.top_k}, "
                                f"intermediate {cfg.intermediate}, shared {cfg.shared_intermediate}; "

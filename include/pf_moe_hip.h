@@ -80,10 +80,11 @@ int pf_hip_moe_forward_device(const PfHipMoe *moe, PfHipWork *work, const float 
 int pf_hip_moe_forward_static(const PfHipMoe *moe, const float *d_x, size_t x_pitch, float *d_y,
                               size_t y_pitch, uint32_t *d_ids, float *d_route_weights,
                               uint32_t *d_error_word, size_t tokens, void *stream);
-/* Which kernels a forward of `tokens` tokens runs on this layer and workspace: 1 the
- * decode kernels (1..4 tokens, 1..16 with the tile-ordered copies; supported shapes and formats),
- * 2 the matrix-core prefill kernels, 0 the general kernels (any shape and format mix).  A streamed
- * layer: 1 for the batches its decode kernels take when the pool keeps Q4_K slots in the tile order. */
+/* Which kernels a forward of `tokens` tokens (rows 16-byte aligned) runs on this layer and workspace:
+ * 1 the decode kernels, 3 the kernels for a few rows per expert, 2 the matrix-core prefill kernels,
+ * 0 the general kernels (any shape and format mix).  Which of the first three depends on the batch's
+ * (token, expert) pairs and the layer's experts and formats.  A streamed layer, given a pool with
+ * tile-ordered slots: 1 up to 16 tokens, 3 up to 400, else 0. */
 int pf_hip_moe_kernel_family(const PfHipMoe *moe, const PfHipWork *work, size_t tokens);
 /* Dependent launches of such a forward on the decode kernels: 3 (router logits; routing, gate/up and
  * SwiGLU; down products and combine), or 2 where one launch takes the whole expert stage (one token,

@@ -144,6 +144,7 @@ class HipShim:
         bind("pf_hip_work_full_reroutes", C.c_int, vp, u32p)
         bind("pf_hip_work_clear_status", C.c_int, vp)
         bind("pf_hip_work_force_general", None, vp, C.c_int)
+        bind("pf_hip_work_force_grouped", None, vp, C.c_int)
         bind("pf_hip_work_limit_kernels", None, vp, C.c_int)
         bind("pf_hip_work_check_guards", C.c_int, vp, P(C.c_int), P(C.c_int))
         bind("pf_hip_moe_forward_host", C.c_int, vp, vp, vp, sz, vp, sz, vp, sz, vp, sz, sz, u32p)

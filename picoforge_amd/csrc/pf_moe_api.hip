@@ -775,6 +775,7 @@ extern "C" int pf_hip_work_check_guards(PfHipWork *w, int *damaged, int *first) 
 }
 
 extern "C" void pf_hip_work_force_general(PfHipWork *w, int on) { if (w) w->force_general = on; }
+extern "C" void pf_hip_work_force_grouped(PfHipWork *w, int on) { if (w) w->force_grouped = on; }
 extern "C" void pf_hip_work_limit_kernels(PfHipWork *w, int count) { if (w) w->stage_limit = count > 0 ? count : 0; }
 
 static PfKernelArgs make_args(const PfHipMoe *m, PfHipWork *w, const float *d_x, size_t x_pitch, float *d_y,
@@ -842,6 +843,18 @@ static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
     }
 }
 
+// The kernels a resident layer's batch runs where its rows are 16-byte aligned (else: the general kernels).
+enum Family { FAMILY_GENERAL, FAMILY_DECODE, FAMILY_GROUPED, FAMILY_BATCH };   // as pf_hip_moe_kernel_family reports them
+static Family kernel_family(const PfHipMoe *moe, const PfHipWork *work, size_t tokens) {
+    const bool grouped = moe->prefill_ready && work->down && tokens > PF_DECODE_MAX_TOKENS;
+    if (work->force_general) return FAMILY_GENERAL;
+    if (work->force_grouped && grouped) return FAMILY_GROUPED;
+    const BatchRange range = batch_range(moe, work);
+    if (moe->decode_ready && tokens <= range.pair_to) return FAMILY_DECODE;
+    if (moe->decode_ready && tokens <= range.batch_to) return FAMILY_BATCH;
+    return grouped ? FAMILY_GROUPED : FAMILY_GENERAL;
+}
+
 static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_x, size_t x_pitch, float *d_y,
                            size_t y_pitch, size_t tokens, const HcTarget *hc, hipStream_t s) {
     const PfHipMoeDesc *d = &moe->desc;
@@ -856,12 +869,12 @@ static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_
         return PF_HIP_E_UNSUPPORTED;
     }
     const bool aligned = (x_pitch % 4 == 0) && ((uintptr_t)d_x % 16 == 0);
-    const BatchRange range = batch_range(moe, work);
-    if (moe->decode_ready && tokens <= range.pair_to && aligned && !work->force_general) {
+    const Family family = aligned ? kernel_family(moe, work, tokens) : FAMILY_GENERAL;
+    if (family == FAMILY_DECODE) {
         pf_launch_decode(a, (int)tokens, s, work->stage_limit);
-    } else if (moe->decode_ready && tokens <= range.batch_to && aligned && !work->force_general) {
+    } else if (family == FAMILY_BATCH) {
         pf_launch_batch(a, (int)tokens, s, work->stage_limit);
-    } else if (moe->prefill_ready && work->down && tokens > PF_DECODE_MAX_TOKENS && aligned && !work->force_general) {
+    } else if (family == FAMILY_GROUPED) {
         pf_launch_prefill(a, (int)tokens, s, work->stage_limit);
     } else {
         // the general kernels stage one token's activations in LDS
@@ -876,15 +889,27 @@ static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_
     return PF_HIP_OK;
 }
 
-// Which kernels a forward of `tokens` tokens (rows 16-byte aligned) runs: 1 the decode kernels,
-// 2 the matrix-core prefill kernels, 0 the general kernels.
+// Short batches of a streamed layer whose pool regions hold tile-ordered slots where the format has a tile order (all three of
+// a layer of one format throughout; gate and up of the checkpoint profiles, whose down slots stay row by row) run the tile
+// decode kernels: kernel 1 and the routing kernels in the first call, kernels 2 and 3 reading the pairs' slots in the second.
+static uint32_t streamed_mask(const PfHipMoe *moe) { return moe->stream_decode <= 2 ? 7u : 3u; }
+static bool streamed_decode(const PfHipMoe *moe, const PfHipWork *work, size_t tokens, uint32_t tiled_mask) {
+    return moe->stream_decode && tiled_mask == streamed_mask(moe) && tokens <= PF_TILE_DECODE_MAX_TOKENS && !work->force_general;
+}
+
+// Longer batches of such a layer: the kernels for a few rows per expert.
+static bool streamed_batch(const PfHipMoe *moe, const PfHipWork *work, size_t tokens, uint32_t tiled_mask) {
+    return moe->stream_decode && tiled_mask == streamed_mask(moe) && work->down && tokens > PF_TILE_DECODE_MAX_TOKENS && tokens <= PF_BATCH_MAX_TOKENS &&
+           !work->force_general;
+}
+
 extern "C" int pf_hip_moe_kernel_family(const PfHipMoe *moe, const PfHipWork *work, size_t tokens) {
-    if (!moe || !work || work->force_general) return 0;
-    if (moe->streamed) return moe->stream_decode && tokens <= PF_TILE_DECODE_MAX_TOKENS ? 1 : 0;   // given a pool with tile-ordered slots
-    const BatchRange range = batch_range(moe, work);
-    if (moe->decode_ready && (tokens <= range.pair_to || (range.batch_to && tokens <= PF_TILE_DECODE_MAX_TOKENS))) return 1;
-    if (moe->prefill_ready && work->down && tokens > PF_DECODE_MAX_TOKENS) return 2;
-    return 0;
+    if (!moe || !work) return FAMILY_GENERAL;
+    if (moe->streamed) {   // given a pool with tile-ordered slots
+        const uint32_t mask = streamed_mask(moe);
+        return streamed_decode(moe, work, tokens, mask) ? FAMILY_DECODE : streamed_batch(moe, work, tokens, mask) ? FAMILY_BATCH : FAMILY_GENERAL;
+    }
+    return kernel_family(moe, work, tokens);
 }
 
 extern "C" int pf_hip_moe_decode_launches(const PfHipMoe *moe, const PfHipWork *work, size_t tokens) {
@@ -1125,21 +1150,6 @@ static bool slot_plan(uint32_t gguf_type, size_t k_storage, size_t n_out, size_t
         p->scale_offset = 0;
     }
     return true;
-}
-
-// Short batches of a streamed layer whose Q4_K pool regions hold tile-ordered slots (all three of a Q4_K layer; gate and
-// up of the q4 checkpoint profile, whose MXFP4 down slots stay row by row) run the tile decode kernels: kernel 1 and the
-// routing kernels in the first call, kernels 2 and 3 reading the pairs' slots in the second.
-static bool streamed_decode(const PfHipMoe *moe, const PfHipWork *work, size_t tokens, uint32_t tiled_mask) {
-    const uint32_t wanted = moe->stream_decode <= 2 ? 7u : 3u;   // one format throughout: all three regions; a profile: gate and up
-    return moe->stream_decode && tiled_mask == wanted && tokens <= PF_TILE_DECODE_MAX_TOKENS && !work->force_general;
-}
-
-// Longer batches of such a layer: the kernels for a few rows per expert.
-static bool streamed_batch(const PfHipMoe *moe, const PfHipWork *work, size_t tokens, uint32_t tiled_mask) {
-    const uint32_t wanted = moe->stream_decode <= 2 ? 7u : 3u;
-    return moe->stream_decode && tiled_mask == wanted && work->down && tokens > PF_TILE_DECODE_MAX_TOKENS && tokens <= PF_BATCH_MAX_TOKENS &&
-           !work->force_general;
 }
 
 extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes,

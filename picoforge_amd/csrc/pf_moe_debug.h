@@ -9,6 +9,9 @@ extern "C" {
 
 /* Tests: route every batch size through the general kernels (on != 0) instead of the specialised ones. */
 void pf_hip_work_force_general(PfHipWork *work, int on);
+/* The matrix-core prefill kernels on every batch they take (more than 4 tokens of a layer they cover), whatever else would
+ * run there. */
+void pf_hip_work_force_grouped(PfHipWork *work, int on);
 
 /* Every later forward on this workspace enqueues only the first `count` of its dependent kernel groups (decode
  * path: its kernels; other paths: four groups; 0 = all; results are then incomplete).  A measuring program times

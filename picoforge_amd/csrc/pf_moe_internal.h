@@ -205,6 +205,7 @@ struct PfHipWork {
     uint32_t call;                  // number of the host-pointer call in progress (the block holds the last one published)
     int stage_limit;                // profiling: launch only the first so many kernels of a forward; 0 = all
     int force_general;               // tests: run the general kernels even where the decode path applies
+    int force_grouped;               // tests: run the grouped product on every batch it takes
     size_t guard, guard_at[40];      // diagnostics (PF_WORK_GUARD=1): bytes of pattern behind each buffer, and where
 };
 

@@ -180,6 +180,10 @@ class MoeLayer:
         """Route every batch size through the general kernels (tests of both kernel families)."""
         self.api.hip.work_force_general(self.api.device_work(self.work), 1 if on else 0)
 
+    def force_grouped(self, on=True):
+        """The matrix-core prefill kernels on every batch they take (tests)."""
+        self.api.hip.work_force_grouped(self.api.device_work(self.work), 1 if on else 0)
+
     def serial_order_reroutes(self):
         count = C.c_uint32()
         self.api.hip.work_exact_rows(self.api.device_work(self.work), C.byref(count))

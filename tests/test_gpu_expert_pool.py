@@ -207,8 +207,9 @@ def test_streamed_layer_on_the_decode_kernels(product, oracle, tmp_path, expert_
     gate and up with an MXFP4 down tensor, IQ2_XXS gate and up with a Q2_K one; the shared expert Q8_0) -- streamed
     through a pool that was told its formats: the Q4_K and IQ2_XXS slots are kept in the tile order and batches of up to
     16 tokens run the decode kernels on them (the router kernel and the routing in the first device call, the expert
-    kernels on the pairs' slots in the second); longer batches run the general kernels on the same slots.  56 slots for
-    64 experts: evictions on the way."""
+    kernels on the pairs' slots in the second), longer batches the kernels for a few rows per expert; the general kernels,
+    which take what is longer still, read the same slots where they are asked for.  56 slots for 64 experts: evictions on
+    the way."""
     cfg = abi.moe_config(512, 64, 4, 256, 256)
     tokens = 40
     weights, x = make_layer_inputs(cfg, expert_type, tokens, seed=67)
@@ -236,9 +237,11 @@ def test_streamed_layer_on_the_decode_kernels(product, oracle, tmp_path, expert_
     with pf.MoeLayer(product, cfg, weights, tokens, handle=handle) as layer:
         moe, work = layer.device_handles()
         assert product.hip.moe_kernel_family(moe, work, 1) == 1 and product.hip.moe_kernel_family(moe, work, 16) == 1
-        assert product.hip.moe_kernel_family(moe, work, 17) == 0
-        for first, count in ((0, 1), (1, 1), (2, 4), (6, 16), (22, 3), (0, 16), (20, 18), (25, 15)):
-            print(f"  streamed rows {first}..{first + count}", flush=True)
+        assert product.hip.moe_kernel_family(moe, work, 17) == 3
+        for first, count, general in ((0, 1, 0), (1, 1, 0), (2, 4, 0), (6, 16, 0), (22, 3, 0), (0, 16, 0), (20, 18, 0), (20, 18, 1), (3, 5, 1), (25, 15, 0)):
+            print(f"  streamed rows {first}..{first + count}" + (" on the general kernels" if general else ""), flush=True)
+            layer.force_general(general)
+            assert product.hip.moe_kernel_family(moe, work, count) == (0 if general else 1 if count <= 16 else 3)
             rows = np.ascontiguousarray(x[first:first + count])
             y = np.full((count, cfg.hidden_size), -99.0, np.float32)
             ids = np.full((count, cfg.top_k), 0xFFFFFFFF, np.uint32)

@@ -76,7 +76,7 @@ def test_decode_kernels_on_batches_of_up_to_sixteen_tokens(product, oracle, h, e
     x[9] = x[8]                                   # two identical tokens share every expert
     want = forward_with(oracle, cfg, weights, x)
     with pf.MoeLayer(product, cfg, weights, 16) as layer:
-        if product.hip.moe_kernel_family(*layer.device_handles(), 16) != 1:
+        if product.hip.moe_kernel_family(*layer.device_handles(), 16) not in (1, 3):
             pytest.skip("batches of 16 tokens of this layer run the prefill kernels")
         for tokens in (5, 6, 7, 9, 13, 16):
             print(f"  tokens={tokens}", flush=True)
@@ -105,6 +105,11 @@ def test_prefill_kernels_match_oracle_and_general_kernels(product, oracle, h, e,
         print(f"  max abs err {worst:.2e}, serial-order reroutes {layer.serial_order_reroutes()}", flush=True)
         _, y2, ids2, _ = layer.forward(x)
         np.testing.assert_array_equal(y, y2, err_msg="prefill path is not deterministic")
+        layer.force_grouped()                     # whatever else takes so few tokens
+        assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == 2, "the prefill kernels do not cover this layer"
+        _, y, ids, w = layer.forward(x)
+        assert_parity(y, ids, w, *want, label=f"grouped product T={tokens}")
+        np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="prefill path is not deterministic")
         layer.force_general()
         _, y, ids, w = layer.forward(x)
         assert_parity(y, ids, w, *want, label="general kernels on a prefill shape")
@@ -118,15 +123,22 @@ def test_prefill_from_row_order_when_the_tile_ordered_copy_is_switched_off(produ
     want = forward_with(oracle, cfg, weights, x)
     with pf.MoeLayer(product, cfg, weights, 70) as layer:
         _, y_tiled, _, _ = layer.forward(x)
+        layer.force_grouped()
+        _, y_grouped, _, _ = layer.forward(x)
     monkeypatch.setenv("PF_MOE_PREFILL_COPY", "0")
     with pf.MoeLayer(product, cfg, weights, 70) as layer:
         bytes_without = product.hip.moe_bytes(layer.device_handles()[0])
-        _, y, ids, w = layer.forward(x)
+        _, y, ids, w = layer.forward(x)           # (the kernels for a few rows per expert: they read either order too)
+        layer.force_grouped()
+        assert product.hip.moe_kernel_family(*layer.device_handles(), 70) == 2
+        _, yg, idsg, wg = layer.forward(x)
     monkeypatch.delenv("PF_MOE_PREFILL_COPY")
     with pf.MoeLayer(product, cfg, weights, 70) as layer:
         bytes_with = product.hip.moe_bytes(layer.device_handles()[0])
     assert_parity(y, ids, w, *want, label="prefill from the row order")
     np.testing.assert_array_equal(y, y_tiled, err_msg="the two weight orders give different results")
+    assert_parity(yg, idsg, wg, *want, label="grouped product from the row order")
+    np.testing.assert_array_equal(yg, y_grouped, err_msg="the two weight orders give different results")
     assert bytes_with == bytes_without
 
 
@@ -171,9 +183,13 @@ def test_full_size_prefill_rows_match_oracle(product, oracle, gtype):
     with pf.MoeLayer(product, cfg, weights, 48) as layer:
         _, y, ids, w = layer.forward(x)
         assert_parity(y[:6], ids[:6], w[:6], *want, label="full-size prefill")
+        layer.force_grouped()
+        _, yp, idsp, wp = layer.forward(x)
+        assert_parity(yp[:6], idsp[:6], wp[:6], *want, label="full-size grouped product")
         layer.force_general()
         _, yg, idsg, wg = layer.forward(x)
         assert_parity(y, ids, w, yg, idsg, wg, label="prefill against general kernels, all 48 rows")
+        assert_parity(yp, idsp, wp, yg, idsg, wg, label="grouped product against general kernels, all 48 rows")
 
 
 LARGER_PREFILL = [
@@ -353,6 +369,9 @@ def test_crowds_of_near_equal_experts(product, oracle, clones):
         assert_parity(y, ids, w, want[0][:16], want[1][:16], want[2][:16], label=f"crowd of {clones}, 16 tokens")
         _, y, ids, w = layer.forward(x)
         assert_parity(y, ids, w, *want, label=f"crowd of {clones}, chunk")
+        layer.force_grouped()
+        _, y, ids, w = layer.forward(x)
+        assert_parity(y, ids, w, *want, label=f"crowd of {clones}, grouped product")
         reroutes, full = layer.serial_order_reroutes(), layer.full_reroutes()
         print(f"  crowd of {clones}: {reroutes} re-routed, {full} the long way", flush=True)
         assert reroutes >= tokens

@@ -59,17 +59,18 @@ def test_a_layer_outlives_its_file(tmp_path, product, oracle):
     (dict(hidden=2560, experts=128, top_k=10, inter=640, shared=640, streams=4), 768),     # the checkpoints' widths
 ], ids=["benchmark-size", "checkpoint-widths"])
 def test_a_full_width_layer_from_a_file(tmp_path, product, oracle, dims, physical):
-    """The decode kernels at 1 and 4 tokens and the matrix-core kernels at 48 tokens must be the ones that run
-    on a layer that came out of a file, at the benchmarks' widths and at the checkpoints' own (Q2_K down padded)."""
+    """The decode kernels at 1 and 4 tokens, the kernels for a few rows per expert at 48 and the matrix-core kernels where they
+    are asked for at 48 must be the ones that run on a layer that came out of a file, at the benchmarks' widths and at the checkpoints' own (Q2_K down padded)."""
     print(f"case layer from a file, profile q2, hidden {dims['hidden']}", flush=True)
     mf = gf.ModelFile(profile="q2", kinds=("gdn",), mtp=0, dims=dims, moe_only=True, seed=9, std=0.02)
     mf.write(tmp_path / "layer.gguf")
     with GgufFile(product, mf.path) as f:
         assert f.moe_model().moe.down_physical == physical and f.moe_weights(0).nbytes > 150e6
-        for count, family in ((1, 1), (4, 1), (48, 2)):
+        for count, family in ((1, 1), (4, 1), (48, 3), (48, 2)):
             x = tokens_for(dims["hidden"], count, 40 + count)
             with f.moe_layer(0, count) as mine, f.moe_layer(0, count, api=oracle) as cpu:
                 moe, work = mine.device_handles()
+                mine.force_grouped(family == 2)
                 assert product.hip.moe_kernel_family(moe, work, count) == family
                 _, y, ids, w = mine.forward(x)
                 _, y_ref, ids_ref, w_ref = cpu.forward(x[:8])

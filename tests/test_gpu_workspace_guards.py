@@ -3,8 +3,8 @@
 A workspace created with PF_WORK_GUARD=1 has 4096 bytes of a fixed pattern behind each of its buffers (logits,
 routes, activations, digit images, union tables, the prefill path's fp16 forms and grouping tables, ...).  The
 layers of the checkpoint profiles and of the single-format configurations, at the benchmark widths and at the
-checkpoints' widths, run batches of 1, 4 and 16 tokens (decode kernels), 48 tokens (matrix cores) and the
-general kernels; afterwards every guard must still hold the pattern, and the outputs must match the CPU path."""
+checkpoints' widths, run batches of 1, 4 and 16 tokens (decode kernels), 48 tokens (the kernels for a few
+rows per expert, and the grouped product) and the general kernels; afterwards every guard must still hold the pattern, and the outputs must match the CPU path."""
 import ctypes as C
 
 import numpy as np
@@ -53,6 +53,9 @@ def test_no_kernel_writes_beyond_its_workspace_buffer(product, oracle, monkeypat
                 print(f"guards: {label}, 48 tokens", flush=True)
                 layer.forward(x)
                 assert guards(product, layer) == (0, -1), f"{label}: a guard was overwritten by the 48-token forward"
+                layer.force_grouped()
+                layer.forward(x)
+                assert guards(product, layer) == (0, -1), f"{label}: a guard was overwritten by the 48-token grouped product"
                 layer.force_general()
                 layer.forward(x[:5])
                 assert guards(product, layer) == (0, -1), f"{label}: a guard was overwritten by the general kernels"
