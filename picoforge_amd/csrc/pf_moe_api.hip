@@ -444,10 +444,10 @@ static Carve plan_work(const PfHipMoeDesc *d, size_t cap, bool fused = false, si
     {   // digit images of the decode path: the token rows; the activation rows of every (unique expert, token) and the shared expert's
         const size_t widest = I > d->shared_inter ? I : d->shared_inter;
         const size_t rows = Td * K * Td + Td > Tt * (K + 1) ? Td * K * Td + Td : Tt * (K + 1);
-        const size_t batch = one_format && prefill ? Tt : 0;   // tokens of a batch of pf_moe_batch.hip, whose images are larger
-        want[W_XIMG] = (batch ? batch * pf_batch_image_words(H) : Tt * pf_image2_words(H)) * 4;
+        const size_t batch = one_format && prefill ? Tt : 0;   // tokens of a batch of pf_moe_batch.hip, whose images are larger in a streamed layer
+        want[W_XIMG] = (batch ? batch * pf_batch_image_words(4, H) : Tt * pf_image2_words(H)) * 4;
         want[W_AIMG] = rows * pf_image2_words(widest) * 4;
-        if (want[W_AIMG] < batch * (K + 1) * pf_batch_image_words(widest) * 4) want[W_AIMG] = batch * (K + 1) * pf_batch_image_words(widest) * 4;
+        if (want[W_AIMG] < batch * (K + 1) * pf_batch_image_words(4, widest) * 4) want[W_AIMG] = batch * (K + 1) * pf_batch_image_words(4, widest) * 4;
     }
     // prefill path: fp16 copies, per-row scales, down products in expert order, grouping tables
     const size_t Tp = prefill ? T : 0, Is = d->shared_inter;
@@ -1175,7 +1175,7 @@ extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *wo
         return PF_HIP_E_UNSUPPORTED;
     }
     if (streamed_batch(moe, work, tokens, tiled_mask)) {
-        pf_launch_batch_router(a, (int)tokens, nullptr);
+        pf_launch_batch_router(a, (int)tokens, 4, nullptr);
         pf_launch_dec_route(a, (int)tokens, nullptr);
     } else if (streamed_decode(moe, work, tokens, tiled_mask)) {
         pf_launch_dec_router(a, (int)tokens, (int)((moe->desc.experts + 3) / 4), nullptr);

@@ -8,21 +8,27 @@
 //   pf_k_batch_gate_up   gate and up products of 32 units, SwiGLU, the activation rows' digit images (expert order)
 //   pf_k_batch_down      down products of 128 output rows, FP32, in expert order (pf_k_pf_combine adds them up)
 //
-// Arithmetic: as the decode kernels', on finer images.  Activations are digit images: integers relative to a power of two
-// per 32-group, 2^-29 of its largest magnitude's binade, as four balanced base-256 digits (a 32-bit value within 2^6 of the
-// largest is exact, a smaller one is off by at most 2^-30 of it).  Weight codes are signed bytes, the group's dot product
-// exact in integers, the group's scale and minimum applied in FP32.  With the decode kernels' three digits the activation
-// rows' rounding showed: 60 tokens of an IQ2_XXS layer 2.9e-7 off the result in 64 bits (2-norm) where FP32 sums of FP32
-// rows (the general kernels) are 2.4e-7 off, now 1.9e-7; 101 tokens of the q2 profile 322 -> 328 us.  The integer products run on v_mfma_i32_32x32x32_i8, one instruction per 32-group:
+// Arithmetic: the decode kernels'.  Activations are digit images (integers per 32-group as balanced base-256 digits), weight
+// codes signed bytes, the group's dot product exact in integers, the group's scale and minimum applied in FP32.  PLANES digits:
+//
+//   3   resident layers: the decode kernels' 24 bits relative to the group's largest magnitude
+//   4   streamed layers, whose batches would otherwise run on FP32 rows (the general kernels): 30 bits and a power of two as the
+//       step, 2^-29 of the binade of the group's largest magnitude, so that a value within 2^6 of it is exact, a smaller one
+//       off by at most 2^-30 of it, and no group vanishes
+//
+// Distance to the result in 64 bits, 60 tokens of an IQ2_XXS layer (2-norm; normal rows, and rows with a few channels 300 times
+// larger): three digits 2.9e-7 and 3.8e-7, four 1.9e-7 and 1.9e-7; the grouped product of prefill 4.1e-7 and 11e-7, the general
+// kernels 2.4e-7 and 2.6e-7.  The fourth digit costs 1 to 3 % of a kernel's time (another addition per sum, a third more
+// image to read).  The integer products run on v_mfma_i32_32x32x32_i8, one instruction per 32-group:
 //
 //   A (rows)     lane (m = lane % 32, h = lane / 32): digit plane m % 4 of the chunk's token m / 4, bytes 16 h .. 16 h + 15
-//                of the group
+//                of the group (with three planes, plane 3 repeats plane 2; its results are not looked at)
 //   B (columns)  lane (n = lane % 32, h): weight row n's codes 16 h .. 16 h + 15 of the group
 //   D            lane (n, h), register 4 q + p: weight row n, token 2 q + h, plane p
 //
 // so the planes of a (row, token) sum meet in one lane, the lane's weight row is the one whose scales it holds, and a
 // chunk of up to 2 q tokens only recombines q of the four register quads.  Per 32 x 32 weights: 6 (Q4_K) to 28 (MXFP4)
-// vector instructions for the codes, about 5 for the scales, 8 per quad -- against 36 per token for the dot-product
+// vector instructions for the codes, about 5 for the scales, 7 or 8 per quad -- against 36 per token for the dot-product
 // instructions of the decode kernels and about 75, whatever the rows, for the FP16 product of the prefill kernels.
 #include "pf_moe_internal.h"
 #include "pf_image.h"
@@ -222,12 +228,17 @@ template <bool ROWS> struct BatchRows<PF_Q2_K, ROWS> {
 // ---- a chunk's rows against a piece ------------------------------------------------------------------
 struct BatchFactor { float step, sum; };   // a (token, group)'s step, and step * sum of the group's integers
 
-// the upper and the lower pair of planes of a sum: at most 28 bits each
-__device__ __forceinline__ float batch_upper(const int16v &d, int q) { return (float)(d[4 * q + 2] + (d[4 * q + 3] << 8)); }
+// A sum from its planes, in two parts of at most 28 bits: its value is 65536 upper + lower.
+template <int PLANES> __device__ __forceinline__ float batch_upper(const int16v &d, int q) {
+    return (float)(PLANES == 4 ? d[4 * q + 2] + (d[4 * q + 3] << 8) : d[4 * q + 2]);
+}
 __device__ __forceinline__ float batch_lower(const int16v &d, int q) { return (float)(d[4 * q] + (d[4 * q + 1] << 8)); }
+template <int PLANES> __device__ __forceinline__ float batch_value(const int16v &d, int q) {
+    return fmaf(65536.0f, batch_upper<PLANES>(d, q), batch_lower(d, q));
+}
 
 // acc[s][q] += the products of set s's piece with tokens 2 q + h of the chunk
-template <int FMT, bool ROWS, int SETS, int QUADS>
+template <int FMT, bool ROWS, int PLANES, int SETS, int QUADS>
 __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS], const int4v (&x)[BatchRows<FMT, ROWS>::GROUPS], const BatchFactor *factors,
                                             int here, const uint32_t *tables, float (&acc)[SETS][4]) {
     typedef BatchRows<FMT, ROWS> Rows;
@@ -247,13 +258,15 @@ __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS
 #pragma unroll
             for (int q = 0; q < QUADS; q++) {
                 const BatchFactor f = factors[16 * q + g];
-                if (Rows::MIN_OPERAND) {   // the two products nearly cancel: their difference pair by pair, the upper one's with what its product lost
-                    const float mu = batch_upper(m[s], q), product = minimum * mu;
-                    const float upper = fmaf(scale, batch_upper(d[s], q), -product) - fmaf(minimum, mu, -product);
+                if (Rows::MIN_OPERAND && PLANES == 4) {   // the two products nearly cancel: their difference part by part, the upper one's with what its product lost
+                    const float mu = batch_upper<PLANES>(m[s], q), product = minimum * mu;
+                    const float upper = fmaf(scale, batch_upper<PLANES>(d[s], q), -product) - fmaf(minimum, mu, -product);
                     const float lower = fmaf(scale, batch_lower(d[s], q), -minimum * batch_lower(m[s], q));
                     acc[s][q] = fmaf(f.step, fmaf(65536.0f, upper, lower), acc[s][q]);
+                } else if (Rows::MIN_OPERAND) {
+                    acc[s][q] = fmaf(f.step, fmaf(scale, batch_value<PLANES>(d[s], q), -minimum * batch_value<PLANES>(m[s], q)), acc[s][q]);
                 } else {
-                    acc[s][q] = fmaf(f.step * fmaf(65536.0f, batch_upper(d[s], q), batch_lower(d[s], q)), scale, acc[s][q]);
+                    acc[s][q] = fmaf(f.step * batch_value<PLANES>(d[s], q), scale, acc[s][q]);
                     if (Rows::MINIMA) acc[s][q] = fmaf(-f.sum, minimum, acc[s][q]);
                 }
             }
@@ -264,18 +277,18 @@ __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS
 // The chunk's activation operands of a piece and the piece's factors into the wave's LDS (factors[8 * token + group]).
 // at, factor_at: the dword offsets in `images` of the images of the lane's token (lane % 32) / 4, and lane / 8.  Groups
 // beyond the row's last repeat it with a factor of zero.
-template <int GROUPS>
+template <int PLANES, int GROUPS>
 __device__ __forceinline__ void batch_operands(int4v (&x)[GROUPS], BatchFactor *factors, const uint32_t *images, uint32_t at, uint32_t factor_at,
                                                int piece, int groups, int lane) {
-    const uint32_t mine = at + 8 * (uint32_t)(lane & 3) + 4 * (uint32_t)(lane >> 5);
+    const uint32_t mine = at + 8 * (uint32_t)min(lane & 3, PLANES - 1) + 4 * (uint32_t)(lane >> 5);
 #pragma unroll
     for (int g = 0; g < GROUPS; g++) {
-        const uint32_t *group = images + PF_BIMG_GROUP * min(GROUPS * piece + g, groups - 1);   // uniform
+        const uint32_t *group = images + 8 * PLANES * min(GROUPS * piece + g, groups - 1);   // uniform
         x[g] = *reinterpret_cast<const int4v *>(group + mine);
     }
     const int fg = GROUPS * piece + (lane & 7), last = min(fg, groups - 1);
-    const float step = fg < groups ? __uint_as_float((images + PF_BIMG_GROUP * groups)[factor_at + (uint32_t)last]) : 0.0f;
-    const float sum = fg < groups ? __uint_as_float((images + (PF_BIMG_GROUP + 1) * groups)[factor_at + (uint32_t)last]) : 0.0f;
+    const float step = fg < groups ? __uint_as_float((images + 8 * PLANES * groups)[factor_at + (uint32_t)last]) : 0.0f;
+    const float sum = fg < groups ? __uint_as_float((images + (8 * PLANES + 1) * groups)[factor_at + (uint32_t)last]) : 0.0f;
     pf_wave_lds_fence();   // the piece before has been read
     factors[lane] = BatchFactor{step, sum};
     pf_wave_lds_fence();
@@ -291,7 +304,7 @@ __device__ __forceinline__ int batch_lane() {
 }
 
 // image_at(r): dword offset in `images` of the image of the chunk's row r
-template <int FMT, bool ROWS, int SETS, typename ImageAt>
+template <int FMT, bool ROWS, int PLANES, int SETS, typename ImageAt>
 __device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&tensor)[SETS], size_t e, int tile, int first_piece, int piece_step,
                                             int groups, const uint32_t *images, ImageAt image_at, BatchFactor *factors, int rows,
                                             const uint32_t *tables, float (&acc)[SETS][4]) {
@@ -310,14 +323,14 @@ __device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&t
     for (int piece = first_piece; piece < pieces; piece += piece_step) {
         const int lane = batch_lane();
         int4v x[Rows::GROUPS];
-        batch_operands<Rows::GROUPS>(x, factors, images, at, factor_at, piece, groups, lane);
+        batch_operands<PLANES, Rows::GROUPS>(x, factors, images, at, factor_at, piece, groups, lane);
 #pragma unroll
         for (int s = 0; s < SETS; s++) w[s].open();
         const BatchFactor *mine = factors + 8 * (lane >> 5);
         const int here = groups - Rows::GROUPS * piece;
-        if (rows <= 2) batch_piece<FMT, ROWS, SETS, 1>(w, x, mine, here, tables, acc);
-        else if (rows <= 4) batch_piece<FMT, ROWS, SETS, 2>(w, x, mine, here, tables, acc);
-        else batch_piece<FMT, ROWS, SETS, 4>(w, x, mine, here, tables, acc);
+        if (rows <= 2) batch_piece<FMT, ROWS, PLANES, SETS, 1>(w, x, mine, here, tables, acc);
+        else if (rows <= 4) batch_piece<FMT, ROWS, PLANES, SETS, 2>(w, x, mine, here, tables, acc);
+        else batch_piece<FMT, ROWS, PLANES, SETS, 4>(w, x, mine, here, tables, acc);
         if (piece + piece_step < pieces) {
             const int lane = batch_lane();
 #pragma unroll
@@ -333,7 +346,7 @@ struct BatchItem {
     int token0;           // shared expert: the first row's token
     size_t e;             // where the expert's weights are: its id, or its pool slot
 };
-__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, int tokens, uint32_t tile, BatchItem &it) {
+__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t tile, BatchItem &it) {
     const uint32_t count = a.tiles[0];
     const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[tile];   // {expert, first row, rows, first row within the expert}
     if (tile >= count) return false;
@@ -371,81 +384,83 @@ __device__ __forceinline__ void batch_stage_tables(uint32_t *tables, const PfKer
     __syncthreads();
 }
 
-// A group's step (the power of two that puts its largest magnitude m between 2^29 and 2^30, or the smallest normal one) and
-// the step's inverse.
-__device__ __forceinline__ void batch_step(float m, float &step, float &inv) {
-    const int exponent = max((int)(__float_as_uint(m) >> 23) - 29, 1);
-    step = __uint_as_float((uint32_t)exponent << 23);
-    inv = __uint_as_float((uint32_t)(254 - exponent) << 23);
+// A group's step and its inverse.  Four planes: the power of two that puts the largest magnitude m between 2^29 and 2^30, or the
+// smallest normal one.
+template <int PLANES> __device__ __forceinline__ void batch_step(float m, float &step, float &inv) {
+    if constexpr (PLANES == 3) {
+        group_step2(m, step, inv);
+    } else {
+        const int exponent = max((int)(__float_as_uint(m) >> 23) - 29, 1);
+        step = __uint_as_float((uint32_t)exponent << 23);
+        inv = __uint_as_float((uint32_t)(254 - exponent) << 23);
+    }
 }
 // balanced base-256 digits of q, lowest first
-__device__ __forceinline__ void batch_digits(int q, int (&d)[PF_BIMG_PLANES]) {
+template <int PLANES> __device__ __forceinline__ void batch_digits(int q, int (&d)[PLANES]) {
 #pragma unroll
-    for (int p = 0; p + 1 < PF_BIMG_PLANES; p++) {
+    for (int p = 0; p + 1 < PLANES; p++) {
         d[p] = ((q + 128) & 255) - 128;
         q = (q - d[p]) >> 8;
     }
-    d[PF_BIMG_PLANES - 1] = q;
+    d[PLANES - 1] = q;
 }
-// the sum of a group's integers (36 bits) from the sums of their upper and lower 16 bits
-__device__ __forceinline__ float batch_sum(int upper, int lower) { return fmaf(65536.0f, (float)upper, (float)lower); }
+// What a vector's group ends with: the step, and the step times the sum of its integers (at most 36 bits, from the sums of
+// their upper and lower 16 bits).
+template <int PLANES> __device__ __forceinline__ void batch_image_end(uint32_t *img, int g, int K, float step, int upper, int lower) {
+    img[8 * PLANES * (K / 32) + g] = __float_as_uint(step);
+    img[(8 * PLANES + 1) * (K / 32) + g] = __float_as_uint(step * fmaf(65536.0f, (float)upper, (float)lower));
+}
 
 // Thread j of a group of four neighbouring lanes: the eight values 8j..8j+7 of a K-vector into its image.
-__device__ __forceinline__ void batch_image_chunk(uint32_t *img, const float (&v)[8], int j, int K) {
+template <int PLANES> __device__ __forceinline__ void batch_image_chunk(uint32_t *img, const float (&v)[8], int j, int K) {
     float m = 0.0f;
 #pragma unroll
     for (int c = 0; c < 8; c++) m = fmaxf(m, fabsf(v[c]));
     m = fmaxf(m, __int_as_float(dpp_quad_xor1(__float_as_int(m))));
     m = fmaxf(m, __int_as_float(dpp_quad_xor2(__float_as_int(m))));
     float step, inv;
-    batch_step(m, step, inv);
-    uint32_t w[PF_BIMG_PLANES][2] = {};
+    batch_step<PLANES>(m, step, inv);
+    uint32_t w[PLANES][2] = {};
     int upper = 0, lower = 0;
 #pragma unroll
     for (int c = 0; c < 8; c++) {
         const int q = __float2int_rn(v[c] * inv);
         upper += q >> 16;
         lower += q & 0xffff;
-        int d[PF_BIMG_PLANES];
-        batch_digits(q, d);
+        int d[PLANES];
+        batch_digits<PLANES>(q, d);
 #pragma unroll
-        for (int p = 0; p < PF_BIMG_PLANES; p++) w[p][c >> 2] |= (uint32_t)(d[p] & 255) << (8 * (c & 3));
+        for (int p = 0; p < PLANES; p++) w[p][c >> 2] |= (uint32_t)(d[p] & 255) << (8 * (c & 3));
     }
     upper += dpp_quad_xor1(upper); upper += dpp_quad_xor2(upper);
     lower += dpp_quad_xor1(lower); lower += dpp_quad_xor2(lower);
-    const int g = j >> 2, at = PF_BIMG_GROUP * g + 2 * (j & 3);
+    const int g = j >> 2, at = 8 * PLANES * g + 2 * (j & 3);
 #pragma unroll
-    for (int p = 0; p < PF_BIMG_PLANES; p++) { img[at + 8 * p] = w[p][0]; img[at + 8 * p + 1] = w[p][1]; }
-    if ((j & 3) == 0) {
-        img[PF_BIMG_GROUP * (K / 32) + g] = __float_as_uint(step);
-        img[(PF_BIMG_GROUP + 1) * (K / 32) + g] = __float_as_uint(step * batch_sum(upper, lower));
-    }
+    for (int p = 0; p < PLANES; p++) { img[at + 8 * p] = w[p][0]; img[at + 8 * p + 1] = w[p][1]; }
+    if ((j & 3) == 0) batch_image_end<PLANES>(img, g, K, step, upper, lower);
 }
 
 // Lanes 0..31 and 32..63, one value each: group g of two K-vectors' images (store: whether the lane's vector exists).
-__device__ __forceinline__ void batch_image_group(uint32_t *img, float v, int g, int K, int lane, bool store) {
+template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t *img, float v, int g, int K, int lane, bool store) {
     float m = fabsf(v);
 #pragma unroll
     for (int k = 0; k < 4; k++) m = fmaxf(m, __int_as_float(dpp_row_step(__float_as_int(m), k)));
     m = fmaxf(m, __shfl_xor(m, 16));
     float step, inv;
-    batch_step(m, step, inv);
+    batch_step<PLANES>(m, step, inv);
     const int q = __float2int_rn(v * inv);
     int upper = q >> 16, lower = q & 0xffff;
 #pragma unroll
     for (int k = 0; k < 4; k++) { upper += dpp_row_step(upper, k); lower += dpp_row_step(lower, k); }
     upper += __shfl_xor(upper, 16);
     lower += __shfl_xor(lower, 16);
-    int d[PF_BIMG_PLANES];
-    batch_digits(q, d);
+    int d[PLANES];
+    batch_digits<PLANES>(q, d);
     if (!store) return;
-    uint8_t *bytes = reinterpret_cast<uint8_t *>(img + PF_BIMG_GROUP * g);
+    uint8_t *bytes = reinterpret_cast<uint8_t *>(img + 8 * PLANES * g);
 #pragma unroll
-    for (int p = 0; p < PF_BIMG_PLANES; p++) bytes[32 * p + (lane & 31)] = (uint8_t)d[p];
-    if ((lane & 31) == 0) {
-        img[PF_BIMG_GROUP * (K / 32) + g] = __float_as_uint(step);
-        img[(PF_BIMG_GROUP + 1) * (K / 32) + g] = __float_as_uint(step * batch_sum(upper, lower));
-    }
+    for (int p = 0; p < PLANES; p++) bytes[32 * p + (lane & 31)] = (uint8_t)d[p];
+    if ((lane & 31) == 0) batch_image_end<PLANES>(img, g, K, step, upper, lower);
 }
 
 // blockIdx.x: 32 units; blockIdx.y: row tile.  The workgroup's waves share K (a 256-block each, in turn); their partial
@@ -456,20 +471,20 @@ __device__ __forceinline__ void batch_image_group(uint32_t *img, float v, int g,
 // two waves with four (both slower), the operands past the registers through LDS (slower: LDS becomes the bottleneck for
 // IQ2_XXS), one matrix a wave at twice the occupancy (85 us).
 #define BATCH_WAVES 4
-template <int FMT, int FMTS, bool ROWS>
-__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(3))) pf_k_batch_gate_up(PfKernelArgs a, int tokens) {
+template <int FMT, int FMTS, bool ROWS, int PLANES>
+__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(3))) pf_k_batch_gate_up(PfKernelArgs a) {
     __shared__ float partial[BATCH_WAVES][2][4][64];
     __shared__ BatchFactor factors[BATCH_WAVES][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
     BatchItem it;
-    if (!batch_item(a, tokens, blockIdx.y, it)) return;
+    if (!batch_item(a, blockIdx.y, it)) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int tile = blockIdx.x, I = it.shared ? a.shared_inter : a.inter;
     if (32 * tile >= I) return;
     if (batch_tables<FMT>()) batch_stage_tables(tables, a);
     const int groups = a.hidden / 32, K = a.top_k;
-    const uint32_t words = (uint32_t)pf_batch_image_words(a.hidden);
-    const size_t act_words = pf_batch_image_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    const uint32_t words = (uint32_t)pf_batch_image_words(PLANES, a.hidden);
+    const size_t act_words = pf_batch_image_words(PLANES, a.inter > a.shared_inter ? a.inter : a.shared_inter);
     for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         float acc[2][4] = {};
@@ -478,8 +493,8 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
             const uint32_t row = (uint32_t)(c0 + r);
             return (it.shared ? (uint32_t)it.token0 + row : a.row_to_pair[(uint32_t)it.first + row] / (uint32_t)K) * words;
         };
-        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS, 2>(a, tensor, 0, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
-        else batch_chunk<FMT, ROWS, 2>(a, tensor, it.e, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
+        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS, PLANES, 2>(a, tensor, 0, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
+        else batch_chunk<FMT, ROWS, PLANES, 2>(a, tensor, it.e, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
         const int lane = batch_lane();
 #pragma unroll
         for (int q = 0; q < 4; q++)
@@ -498,32 +513,32 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
             const float act = pf_silu(gate) * up;
             const int r = 2 * q + (lane >> 5);
             if (r < rows && !pf_finite(act)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
-            batch_image_group(a.aimg + (size_t)(it.first + c0 + min(r, rows - 1)) * act_words, act, tile, I, lane, r < rows);
+            batch_image_group<PLANES>(a.aimg + (size_t)(it.first + c0 + min(r, rows - 1)) * act_words, act, tile, I, lane, r < rows);
         }
         if (c0 + BATCH_ROWS < it.rows) __syncthreads();   // the sums have been read
     }
 }
 
 // blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert
-template <int FMT, int FMTS, bool ROWS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, int tokens) {
+template <int FMT, int FMTS, bool ROWS, int PLANES>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a) {
     __shared__ BatchFactor factors[4][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
     BatchItem it;
-    if (!batch_item(a, tokens, blockIdx.y, it)) return;
+    if (!batch_item(a, blockIdx.y, it)) return;
     if (batch_tables<FMT>()) batch_stage_tables(tables, a);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), H = a.hidden;
     const int tile = 4 * blockIdx.x + wave;
     if (32 * tile >= H) return;
     const int groups = (it.shared ? a.shared_inter : a.inter) / 32;
-    const uint32_t words = (uint32_t)pf_batch_image_words(a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    const uint32_t words = (uint32_t)pf_batch_image_words(PLANES, a.inter > a.shared_inter ? a.inter : a.shared_inter);
     for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         auto image_at = [&](int r) { return (uint32_t)(it.first + c0 + r) * words; };
         float acc[1][4] = {};
         const int tensor[1] = {it.shared ? 6 : 3};
-        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS || FMTS == PF_Q8_0, 1>(a, tensor, 0, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
-        else batch_chunk<FMT, ROWS, 1>(a, tensor, it.e, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
+        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS || FMTS == PF_Q8_0, PLANES, 1>(a, tensor, 0, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
+        else batch_chunk<FMT, ROWS, PLANES, 1>(a, tensor, it.e, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
         const int lane = batch_lane();
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -547,6 +562,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) p
 typedef float float4v __attribute__((ext_vector_type(4)));
 #define ROUTER_LINES 5      // 32-column lines a wave holds: hidden <= 2560
 #define ROUTER_PITCH 36     // floats between rows of a staged line: neighbouring lanes' 16-byte reads cover all banks
+template <int PLANES>
 __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int tokens) {
     __shared__ __align__(16) float staged[16][2][16 * ROUTER_PITCH];
     const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -558,7 +574,7 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
         for (int j = lane; j < H / 8; j += 64) {
             const float4v p = row[2 * j], q = row[2 * j + 1], u = gate[2 * j], v = gate[2 * j + 1];
             const float both[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
-            batch_image_chunk(a.ximg + (size_t)t * pf_batch_image_words(H), both, j, H);
+            batch_image_chunk<PLANES>(a.ximg + (size_t)t * pf_batch_image_words(PLANES, H), both, j, H);
 #pragma unroll
             for (int c = 0; c < 4; c++) z = fmaf(p[c], u[c], fmaf(q[c], v[c], z));
         }
@@ -634,26 +650,28 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
     }
 }
 
-void pf_launch_batch_router(const PfKernelArgs &a, int tokens, hipStream_t stream) {
-    hipLaunchKernelGGL(pf_k_batch_router, dim3((tokens + 15) / 16, (a.experts + 15) / 16 + 1), dim3(1024), 0, stream, a, tokens);
+void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, hipStream_t stream) {
+    const dim3 grid((tokens + 15) / 16, (a.experts + 15) / 16 + 1);
+    hipLaunchKernelGGL(planes == 4 ? pf_k_batch_router<4> : pf_k_batch_router<3>, grid, dim3(1024), 0, stream, a, tokens);
 }
 
 // ---- dispatch --------------------------------------------------------------------------------------
-template <int FG, int FD, int FS, bool ROWS>
+template <int FG, int FD, int FS, bool ROWS, int PLANES>
 static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile_cap, hipStream_t stream, int last) {
     const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
-    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a, tokens);
+    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a);
     if (last < 4) return;
-    hipLaunchKernelGGL((pf_k_batch_down<FD, FS, ROWS>), dim3((a.hidden + 127) / 128, tile_cap), dim3(256), 0, stream, a, tokens);
+    hipLaunchKernelGGL((pf_k_batch_down<FD, FS, ROWS, PLANES>), dim3((a.hidden + 127) / 128, tile_cap), dim3(256), 0, stream, a);
 }
 
 template <int FG, int FD, int FS>
 static void launch_batch_experts(const PfKernelArgs &a, int tokens, unsigned tile_cap, hipStream_t stream, int last) {
     // a layer keeps the tile-ordered copies of its gate and up tensors (and a one-format layer those of its down tensors,
-    // the profiles those of the shared gate and up) or none of them
+    // the profiles those of the shared gate and up) or none of them; a streamed layer's pool keeps its slots that way
     const bool tiled = (FG == PF_Q4_K ? a.wt[1] && a.wt[2] : a.wi[1] && a.wi[2]) && (FS != PF_Q8_0 || (a.wq[4] && a.wq[5]));
-    if (tiled) launch_batch_format<FG, FD, FS, false>(a, tokens, tile_cap, stream, last);
-    else launch_batch_format<FG, FD, FS, true>(a, tokens, tile_cap, stream, last);
+    if (a.slots) launch_batch_format<FG, FD, FS, false, 4>(a, tokens, tile_cap, stream, last);
+    else if (tiled) launch_batch_format<FG, FD, FS, false, 3>(a, tokens, tile_cap, stream, last);
+    else launch_batch_format<FG, FD, FS, true, 3>(a, tokens, tile_cap, stream, last);
 }
 
 void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stream, int last) {
@@ -671,7 +689,7 @@ void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stre
 
 void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit) {
     const int last = stage_limit ? stage_limit : 4;
-    pf_launch_batch_router(a, tokens, stream);
+    pf_launch_batch_router(a, tokens, 3, stream);
     if (last < 2) return;
     pf_launch_dec_route(a, tokens, stream);
     pf_launch_group(a, a.ids, tokens, stream);

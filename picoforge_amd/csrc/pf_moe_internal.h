@@ -182,11 +182,9 @@ struct PfHipMoe {
 #define PF_IMG_PLANES 3                       // signed byte digits per value: 24 bits
 #define PF_IMG_GROUP (8 * PF_IMG_PLANES)      // dwords of one 32-group's digits
 __host__ __device__ constexpr size_t pf_image2_words(size_t K) { return (K / 32) * (PF_IMG_GROUP + 2); }
-// The image of the kernels for a few rows per expert (pf_moe_batch.hip): four digits, a power of two as the step, and the
-// step times the sum of the integers as a float in place of the sum.
-#define PF_BIMG_PLANES 4
-#define PF_BIMG_GROUP (8 * PF_BIMG_PLANES)
-__host__ __device__ constexpr size_t pf_batch_image_words(size_t K) { return (K / 32) * (PF_BIMG_GROUP + 2); }
+// The image of the kernels for a few rows per expert (pf_moe_batch.hip): three or four digits, and the step times the sum of
+// the integers as a float in place of the sum.
+__host__ __device__ constexpr size_t pf_batch_image_words(int planes, size_t K) { return (K / 32) * (8 * planes + 2); }
 
 struct PfHipWork {
     const PfHipMoe *moe;
@@ -277,7 +275,7 @@ size_t pf_prefill_half_row(int cols);   // halfs per row of the fp16 form of a m
 int pf_prefill_max_tiles(int tokens, int experts, int top_k);
 // pf_moe_batch.hip: a few rows per expert, for the layers of the tile decode kernels
 void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
-void pf_launch_batch_router(const PfKernelArgs &a, int tokens, hipStream_t stream);
+void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, hipStream_t stream);
 void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stream, int last);
 // pf_moe_hc.hip
 void pf_launch_hc_read(const float *d_normed, size_t n_token_pitch, size_t n_stream_pitch, const float *d_logits,

@@ -8,7 +8,6 @@ import picoforge_amd as pf
 from picoforge_amd import abi
 
 from helpers import assert_parity, forward_with, make_layer_inputs
-from test_oracle_packed import np_iq2
 
 pytestmark = pytest.mark.gpu
 
@@ -58,48 +57,3 @@ def test_activations_whose_squares_overflow(product, oracle, router):
             print(f"case squares overflow, router {router}, {tokens} tokens", flush=True)
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
-
-
-def forward64(cfg, weights, x, ids):
-    """The block in 64 bits for an IQ2_XXS layer (its decoded values are exact in 32), routes renormalised over ids."""
-    h, i, e = cfg.hidden_size, cfg.intermediate, cfg.experts
-    x = x.astype(np.float64)
-    router, gate_row = (weights.raw[j].view(np.float32).astype(np.float64) for j in (0, 7))
-    gate, up, down, shared_gate, shared_up, shared_down = (np_iq2(weights.raw[j], h if j not in (3, 6) else i).astype(np.float64) for j in range(1, 7))
-
-    def expert(rows, g, u, d):
-        z = rows @ g.T
-        return (z / (1.0 + np.exp(-z)) * (rows @ u.T)) @ d.T
-
-    z = np.take_along_axis(x @ router.reshape(e, h).T, ids.astype(np.int64), 1)
-    w = np.exp(z - z.max(1, keepdims=True))
-    w /= w.sum(1, keepdims=True)
-    y = expert(x, shared_gate, shared_up, shared_down) / (1.0 + np.exp(-(x @ gate_row)))[:, None]
-    for k in range(e):
-        t, slot = np.nonzero(ids == k)
-        y[t] += w[t, slot][:, None] * expert(x[t], gate[k * i:(k + 1) * i], up[k * i:(k + 1) * i], down[k * h:(k + 1) * h])
-    return y
-
-
-@pytest.mark.parametrize("kind", ["normal", "outliers", "lognormal"])
-def test_as_close_to_64_bits_as_sums_in_32(product, kind):
-    """The integer products on digit images lose no more than the general kernels, which sum FP32 activations times decoded
-    weights in FP32 (measured: 0.7 to 0.8 of their distance; with three digits it was 1.2 to 1.6 of it)."""
-    print(f"case precision {kind}", flush=True)
-    cfg = abi.moe_config(2048, 24, 4, 512, 512)
-    weights, x = make_layer_inputs(cfg, abi.GGUF_IQ2_XXS, 60, seed=11)
-    rng = np.random.default_rng(3)
-    if kind == "outliers":
-        x[:, rng.choice(2048, 8, replace=False)] *= 300.0     # a few channels hundreds of times larger
-    if kind == "lognormal":
-        x *= np.exp(2.0 * rng.standard_normal(x.shape)).astype(np.float32)
-    x = pf.rms_normalise(x)
-    with pf.MoeLayer(product, cfg, weights, 60) as layer:
-        _, y, ids, _ = layer.forward(x)
-        layer.force_general()
-        _, y_general, ids_general, _ = layer.forward(x)
-    np.testing.assert_array_equal(ids, ids_general)
-    want = forward64(cfg, weights, x, ids)
-    off, off_general = (np.linalg.norm(a - want) / np.linalg.norm(want) for a in (y, y_general))
-    print(f"  off by {off:.2e}, the general kernels by {off_general:.2e}", flush=True)
-    assert off <= off_general
