@@ -4,8 +4,8 @@
 #include "../../include/pf_moe_hip.h"
 
 #define PF_DECODE_MAX_TOKENS 4
-#define PF_TILE_DECODE_MAX_TOKENS 16   // Q4_K layers whose tile-ordered copies are kept: one token per grid row
-
+#define PF_TILE_DECODE_MAX_TOKENS 16   // layers whose tile-ordered copies are kept, and pool slots: one token per grid row
+#define PF_PAIR_MAX_TOKENS 32          // ... of one format throughout, resident
 #define PF_BATCH_MAX_TOKENS 400        // the kernels for a few rows per expert (pf_moe_batch.hip)
 
 // Everything a kernel needs, passed by value.  Weight index order is

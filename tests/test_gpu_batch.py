@@ -57,3 +57,22 @@ def test_activations_whose_squares_overflow(product, oracle, router):
             print(f"case squares overflow, router {router}, {tokens} tokens", flush=True)
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
+
+
+# (experts, top-k, format, last batch of the decode kernels, last of the kernels for a few rows per expert)
+LINES = [(16, 4, abi.GGUF_Q4_K, 32, 250), (64, 8, abi.GGUF_Q4_K, 29, 128), (128, 8, abi.GGUF_IQ2_XXS, 28, 247), (64, 8, "q2", 6, 139),
+         (128, 8, "q4", 9, 144)]
+
+
+@pytest.mark.parametrize("e,k,fmt,pair_to,batch_to", LINES)
+def test_batches_on_both_sides_of_the_lines_between_the_kernels(product, oracle, e, k, fmt, pair_to, batch_to):
+    """The lines go by pairs and experts; a token more on either side of one is another kernel family's and the same block."""
+    print(f"case lines {fmt} e={e} k={k}", flush=True)
+    cfg = abi.moe_config(512, e, k, 256, 256)
+    weights, x = make_layer_inputs(cfg, fmt, batch_to + 1, seed=e + k)
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, batch_to + 1) as layer:
+        for tokens, family in ((pair_to, 1), (pair_to + 1, 3), (batch_to, 3), (batch_to + 1, 2)):
+            assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == family, tokens
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
