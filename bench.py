@@ -59,7 +59,11 @@ WORKLOADS = {
     "q4k_verify8": dict(type=abi.GGUF_Q4_K, tokens=8, steps=500, warmup=50,
                         label="Q4_K experts, 8-token batch of the same process (each token about half of its neighbour's experts)"),
     "q4k_verify16": dict(type=abi.GGUF_Q4_K, tokens=16, steps=250, warmup=25,
-                         label="Q4_K experts, 16-token batch of the same process: the longest the decode kernels take"),
+                         label="Q4_K experts, 16-token batch of the same process: the longest the decode kernels take of a profile or of pool slots"),
+    "q4k_batch64": dict(type=abi.GGUF_Q4_K, tokens=64, steps=64, warmup=10,
+                        label="Q4_K experts, 64 tokens at once, Zipf(1.1) expert popularity"),
+    "q2ckpt_batch101": dict(type="q2", tokens=101, steps=64, warmup=10, dims=CKPT_Q2,
+                            label="checkpoint profile Q2 at the checkpoints' widths, 101 tokens at once, Zipf(1.1) expert popularity"),
     "q4k_prefill1024": dict(type=abi.GGUF_Q4_K, tokens=1024, steps=20, warmup=5, label="Q4_K experts, " + PREFILL_LABEL),
     "q4k_prefill2048": dict(type=abi.GGUF_Q4_K, tokens=2048, steps=20, warmup=5,
                             label="Q4_K experts, " + PREFILL_LABEL.replace("1024", "2048") + " (the chunk size of the 48-layer stack)"),
@@ -102,7 +106,7 @@ WORKLOADS = {
 # what the kernels compute in (every product exact; the result differs from the reference's serial f32 sums by the
 # rounding of the activations and by the order of the additions; observed error <= 1e-5 against a bar of 1e-3)
 DTYPE_DECODE = "i32 dot products of 24-bit block-fixed-point activations with integer weight codes, f32 scales and sums"
-DTYPE_BATCH = "i32 matrix-core products of 30-bit block-fixed-point activations (int8 digits) with integer weight codes, f32 scales and sums"
+DTYPE_BATCH = "i32 matrix-core products of 24-bit block-fixed-point activations (int8 digits) with integer weight codes, f32 scales and sums"
 DTYPE_PREFILL = "f16 matrix-core products of exact-integer weight operands with two-part f16 activations, f32 accumulation"
 HEADLINE = "q4k_decode"
 ALL_CONFIGS = ["iq2xxs_decode", "q4k_verify4", "q4k_prefill1024", "q4k_stack48"]
@@ -363,7 +367,7 @@ def run_layer(args, ctx, name, steps, warmup, cpu_seconds):
                  **({"mfma_frac_of_fp16_dense_peak": round(flops / (ms_per_step * 1e-3) / 1e12 / MFMA_F16_PEAK_TFLOPS, 4)} if family == 2 else {}),
                  "stage_tflops": {names[j].split()[0]: round(stage_flops[j] / (stage_us[j] * 1e-6) / 1e12, 1)
                                   for j in (0, 2, 3)},
-                 "binding_roofline": "hbm: about 80 flop per weight byte at this chunk size, below the MFMA ridge"}
+                 "binding_roofline": f"hbm: {flops / alg_bytes:.0f} flop per byte at this chunk size, below the MFMA ridge"}
     else:
         alg_bytes = workloads.algorithmic_bytes_per_token(wl["type"], unique_experts=unique, cfg=cfg)
         stage_bytes = [lb["routers"], unique * lb["gate_up"] + lb["shared_gate_up"],

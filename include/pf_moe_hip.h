@@ -58,6 +58,10 @@ void pf_hip_moe_destroy(PfHipMoe *moe);
 /* Total HBM bytes held by the layer. */
 size_t pf_hip_moe_bytes(const PfHipMoe *moe);
 
+/* Device bytes of a workspace.  A workspace also holds page-locked host memory for host-pointer
+ * forwards: the rows and results of up to 64 tokens, and with a token_cap beyond 64 the cap's ids and
+ * route weights and a ring of 4 MB; the first such workspace of a process starts three threads that
+ * copy rows, the last one destroyed ends them. */
 size_t pf_hip_work_bytes(const PfHipMoeDesc *desc, size_t token_cap);
 int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWork **out);
 void pf_hip_work_destroy(PfHipWork *work);
@@ -116,9 +120,11 @@ int pf_hip_work_clear_status(PfHipWork *work);
 /* Host-buffer forward used by qwen4_moe_forward: copies x in, runs the forward,
  * copies y (and ids/weights when non-NULL) out, returns the error word.  Pitches
  * in bytes.  Outputs are written only when the error word is zero.  Batches of up
- * to 16 tokens go through a pinned host block the workspace owns (one enqueued copy
- * in, output rows written into the block by the kernels, one enqueued copy for the
- * error word, ids and weights, one wait); longer ones use a blocking copy per buffer. */
+ * to 64 tokens go through a pinned host block the workspace owns (a kernel brings the
+ * rows in, the output rows are written into the block by the last kernel, one more
+ * kernel publishes error word, ids and weights, and the call polls for its number);
+ * longer ones pass through a ring of page-locked pieces that the calling thread and,
+ * from 1 MB of rows on, three helper threads fill and empty. */
 int pf_hip_moe_forward_host(const PfHipMoe *moe, PfHipWork *work, const float *x,
                             size_t x_pitch_bytes, float *y, size_t y_pitch_bytes,
                             uint32_t *ids, size_t ids_pitch_bytes, float *weights,
@@ -223,7 +229,8 @@ int pf_hip_exact_combine_host(const float *down, const uint64_t *pair_to_row, co
  * three of a layer that is Q4_K or IQ2_XXS throughout, gate and up of one in a checkpoint profile (Q4_K with
  * an MXFP4 down tensor, IQ2_XXS with a Q2_K one; Q8_0 shared expert) -- batches of up to 16 tokens run the
  * decode kernels on the slots (the first call the router kernel and the routing, the second the expert
- * kernels); otherwise the general kernels, which read either order. */
+ * kernels), batches of up to 400 those for a few rows per expert; otherwise the general kernels, which
+ * read either order. */
 int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *work, const float *x, size_t x_pitch_bytes,
                                    size_t tokens, uint32_t tiled_mask, uint32_t *ids, uint32_t *error_word);
 int pf_hip_moe_experts_streamed_host(const PfHipMoe *moe, PfHipWork *work, const void *const regions[3],

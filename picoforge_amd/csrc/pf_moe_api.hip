@@ -411,8 +411,8 @@ static Carve plan_work(const PfHipMoeDesc *d, size_t cap, bool fused = false, si
     memset(&c, 0, sizeof c);
     const size_t T = cap ? cap : 1, E = d->experts, K = d->top_k, H = d->hidden, I = d->inter;
     const size_t Td = T < PF_DECODE_MAX_TOKENS ? T : PF_DECODE_MAX_TOKENS;   // tokens per decode launch
-    // ... and per launch of the kernels for tile-ordered Q4_K (whether the copies are kept is not known here)
-    // (one format throughout, or a checkpoint profile: Q8_0 shared expert)
+    // ... and per launch of the kernels on tile-ordered weights (whether the copies are kept is not known here): one format
+    // throughout, or a checkpoint profile (Q8_0 shared expert)
     bool one_format = (d->type[1] == PF_Q4_K || d->type[1] == PF_IQ2_XXS) && d->type[2] == d->type[1];
     for (int t = 4; t <= 6; t++) one_format &= d->type[t] == d->type[1] || d->type[t] == PF_Q8_0;
     // ... and per batch of the kernels for a few rows per expert, which share the images
@@ -523,7 +523,7 @@ static bool through_host_block(const PfHipWork *w, size_t tokens) { return w->ho
 
 // A short batch's rows come in and its results go out by kernels that address the block, not by copies: a copy runs on a
 // copy engine, and each change between engine and kernels waits for a signal (a one-token call of a 2048-wide layer with
-// both copies and a wait for the stream 34.7 us, so 30.1).
+// both copies and a wait for the stream 34.7 us, so 32.2).
 __global__ void pf_k_copy_rows(const uint4 *src, uint4 *dst, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
@@ -1148,7 +1148,8 @@ extern "C" int pf_host_finite(const float *x, size_t pitch_bytes, size_t rows, s
 // Two calls with the caller's pool in between.  The first runs the router and the routing and returns the pairs'
 // expert ids; the caller makes those experts resident (qw4_pool_acquire) and passes the pool's device regions and
 // the pairs' slots to the second, which runs the expert products and the combine reading rows at
-// region + slot * expert_bytes.  The general kernels serve both: streaming is bound by the reads that fill the pool.
+// region + slot * expert_bytes.  Short batches run the decode kernels in both, longer ones the kernels for a few rows per
+// expert, and what neither takes (streamed_decode, streamed_batch) the general kernels.
 extern "C" int pf_hip_pool_slot_tiled(uint32_t gguf_type, size_t n_out) {
     return (gguf_type == PF_Q4_K || gguf_type == PF_IQ2_XXS) && n_out % 32 == 0;
 }

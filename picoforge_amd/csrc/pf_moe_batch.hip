@@ -467,7 +467,7 @@ template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t
 // sums meet in LDS and are added in wave order, a wave per pair of rows.
 // Bound by the chain a workgroup lives through (item, weights, products, the same for a second 256-block, sums): three
 // workgroups a compute unit keep 120 KB on their way, 3.9 TB/s of weights at 32 tokens (77 us for 283 MB; the 32-row FP16
-// product took 79, at 101 tokens of the q2 profile 309 against 180).  Measured and left out: eight waves with a block each,
+// product took 79, at 101 tokens of the q2 profile 309 against 187).  Measured and left out: eight waves with a block each,
 // two waves with four (both slower), the operands past the registers through LDS (slower: LDS becomes the bottleneck for
 // IQ2_XXS), one matrix a wave at twice the occupancy (85 us).
 #define BATCH_WAVES 4

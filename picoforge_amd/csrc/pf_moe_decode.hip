@@ -2391,8 +2391,8 @@ static void launch_down(const PfKernelArgs &a, dim3 grid, dim3 block, size_t lds
         launch_down_bounded<FD, FS, NT, SPL, 1024>(a, grid, block, lds, stream, row_blocks, rows_per_block, image_pitch);
 }
 
-// Layers the kernels whose lanes are weight rows take, one token per grid row, for up to PF_TILE_DECODE_MAX_TOKENS
-// tokens: every expert tensor Q4_K, or every one IQ2_XXS, with its tile-ordered copy kept; the two checkpoint profiles
+// Layers the kernels whose lanes are weight rows take, one token per grid row, for up to PF_PAIR_MAX_TOKENS tokens
+// (PF_TILE_DECODE_MAX_TOKENS of a checkpoint profile and of pool slots): every expert tensor Q4_K, or every one IQ2_XXS, with its tile-ordered copy kept; the two checkpoint profiles
 // with the tile-ordered copies of their routed gate and up tensors and of the shared expert's Q8_0 gate and up (their
 // down tensors are read row by row).  Returns the combination as decode_combination numbers it, 0 for other layers.
 #if PF_DECODE_PART == 0

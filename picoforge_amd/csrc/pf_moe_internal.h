@@ -165,13 +165,14 @@ struct PfHipMoe {
     size_t total_bytes;
     bool decode_ready;               // shapes and formats the specialised decode kernels cover
     bool prefill_ready;              // shapes and formats the matrix-core prefill kernels cover
-    int stream_decode;               // a streamed layer whose short batches run the tile decode kernels on pool slots: 1 Q4_K
-                                     // throughout, 4 the q4 checkpoint profile (0: the general kernels serve every batch)
+    int stream_decode;               // a streamed layer whose batches run the tile decode kernels and those for a few rows per
+                                     // expert on pool slots: 1 Q4_K, 2 IQ2_XXS throughout, 3, 4 the q2, q4 checkpoint profile
+                                     // (0: the general kernels serve every batch)
     float *w_norm2;                  // [experts] squared norm of each router row
     float *router_t;                 // [slab of 64 experts][hidden / 4][64][4] copy of the router
-    uint8_t *w_tiled[8];             // tile-ordered second copy of the expert tensors for the prefill path (or null)
-    uint8_t *w_itile[8];             // tile-ordered second copy of IQ2_XXS expert tensors for the decode path (or null)
-    uint8_t *w_qtile[8];             // tile-ordered second copy of the Q8_0 shared gate and up tensors (or null)
+    uint8_t *w_tiled[8];             // Q4_K expert tensors in tile order, for every kernel family (or null)
+    uint8_t *w_itile[8];             // tile-ordered second copy of IQ2_XXS expert tensors, decode and few rows per expert (or null)
+    uint8_t *w_qtile[8];             // tile-ordered second copy of the Q8_0 shared gate and up tensors, the same (or null)
     bool streamed;                   // the routed tensors are not resident: forwards read them from an expert pool
 };
 

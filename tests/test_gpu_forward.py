@@ -228,15 +228,15 @@ def test_decode_unnormalised_weights_and_repeat_calls(product, oracle, norm):
             assert_parity(y, ids, w, *want, label=f"norm={norm}")
 
 
-@pytest.mark.parametrize("tokens", [1, 5, 16, 17])
+@pytest.mark.parametrize("tokens", [1, 5, 16, 17, 65, 600])
 def test_host_pointer_forward_with_padded_rows_and_without_routes(product, tokens):
-    """Batches of up to 16 tokens pass through the workspace's pinned block (the output rows are written into it by the
-    kernels, ids and weights arrive in one copy), longer ones through one copy per buffer: both must place rows at the
-    caller's pitches, leave the padding alone and give the same rows with and without the routes asked for."""
+    """Batches of up to 64 tokens pass through the workspace's pinned block (the output rows are written into it by the
+    kernels, ids and weights by one more), longer ones through a ring of pieces, from 1 MB on by several threads: all must
+    place rows at the caller's pitches, leave the padding alone and give the same rows with and without the routes asked for."""
     cfg = abi.moe_config(512, 64, 4, 256, 256)
     weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, tokens, seed=31)
     h, k = cfg.hidden_size, cfg.top_k
-    with pf.MoeLayer(product, cfg, weights, 32) as layer:
+    with pf.MoeLayer(product, cfg, weights, max(32, tokens)) as layer:
         _, y0, ids0, w0 = layer.forward(x)
         _, y1, _, _ = layer.forward(x, want_routes=False)
         assert np.array_equal(y0, y1)

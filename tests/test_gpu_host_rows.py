@@ -1,5 +1,7 @@
 """Host-pointer forwards on both sides of each way rows travel: the page-locked block (up to 64 tokens), the ring of pieces by
 one thread, and by the crew (from 1 MB); a value that is not finite in the last row is found before anything is written."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -40,3 +42,33 @@ def test_pieces_that_start_off_a_16_byte_boundary(product, oracle):
     weights, x = make_layer_inputs(cfg, abi.GGUF_F32, tokens, seed=33, std=0.1)
     want = forward_with(oracle, cfg, weights, x)
     assert_parity(*forward_with(product, cfg, weights, x), *want, label=f"hidden 33, {tokens} tokens")
+
+
+def test_two_workspaces_at_once(product):
+    """Two threads, each with a layer and a workspace of its own, on batches that are worth the crew: whoever finds it at work
+    for the other copies alone, and every call's rows are what the call gives by itself."""
+    cfg = abi.moe_config(512, 16, 3, 256, 256)
+    layers, inputs, alone, wrong = [], [], [], []
+    for seed in (5, 6):
+        weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, 900, seed=seed)
+        layers.append(pf.MoeLayer(product, cfg, weights, 900))
+        inputs.append((x, x[:600]))
+        alone.append([layers[-1].forward(rows)[1:] for rows in inputs[-1]])
+
+    def calls(which):
+        try:
+            for turn in range(12):
+                got = layers[which].forward(inputs[which][turn % 2])[1:]
+                if not all(np.array_equal(a, b) for a, b in zip(got, alone[which][turn % 2])):
+                    wrong.append((which, turn))
+        except Exception as e:   # a thread's error would be lost
+            wrong.append((which, repr(e)))
+
+    threads = [threading.Thread(target=calls, args=(which,)) for which in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for layer in layers:
+        layer.close()
+    assert not wrong, wrong
