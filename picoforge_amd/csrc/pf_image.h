@@ -19,13 +19,13 @@ __device__ __forceinline__ void group_step2(float m, float &step, float &inv) {
     step = none ? 0.0f : m * (1.0f / PF_IMG_TOP);
 }
 // balanced base-256 digits of q, lowest first (each in -128..127)
-__device__ __forceinline__ void image_digits(int q, int (&d)[PF_IMG_PLANES]) {
+template <int PLANES> __device__ __forceinline__ void image_digits(int q, int (&d)[PLANES]) {
 #pragma unroll
-    for (int p = 0; p + 1 < PF_IMG_PLANES; p++) {
+    for (int p = 0; p + 1 < PLANES; p++) {
         d[p] = ((q + 128) & 255) - 128;
         q = (q - d[p]) >> 8;
     }
-    d[PF_IMG_PLANES - 1] = q;
+    d[PLANES - 1] = q;
 }
 // the integer dot product from its per-plane parts (float: three planes leave 32 bits)
 __device__ __forceinline__ float image_value(const int (&part)[PF_IMG_PLANES]) {

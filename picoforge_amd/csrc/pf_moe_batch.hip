@@ -17,7 +17,7 @@
 //       off by at most 2^-30 of it, and no group vanishes
 //
 // Distance to the result in 64 bits, 60 tokens of an IQ2_XXS layer (2-norm; normal rows, and rows with a few channels 300 times
-// larger): three digits 2.9e-7 and 3.8e-7, four 1.9e-7 and 1.9e-7; the grouped product of prefill 4.1e-7 and 11e-7, the general
+// larger): three digits 2.8e-7 and 3.8e-7, four 1.9e-7 and 1.9e-7; the grouped product of prefill 4.1e-7 and 11e-7, the general
 // kernels 2.4e-7 and 2.6e-7.  The fourth digit costs 1 to 3 % of a kernel's time (another addition per sum, a third more
 // image to read).  The integer products run on v_mfma_i32_32x32x32_i8, one instruction per 32-group:
 //
@@ -226,7 +226,7 @@ template <bool ROWS> struct BatchRows<PF_Q2_K, ROWS> {
 };
 
 // ---- a chunk's rows against a piece ------------------------------------------------------------------
-struct BatchFactor { float step, sum; };   // a (token, group)'s step, and step * sum of the group's integers
+struct BatchFactor { float step, sum; };   // a (token, group)'s step, and the sum of the group's integers
 
 // A sum from its planes, in two parts of at most 28 bits: its value is 65536 upper + lower.
 template <int PLANES> __device__ __forceinline__ float batch_upper(const int16v &d, int q) {
@@ -265,9 +265,10 @@ __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS
                     acc[s][q] = fmaf(f.step, fmaf(65536.0f, upper, lower), acc[s][q]);
                 } else if (Rows::MIN_OPERAND) {
                     acc[s][q] = fmaf(f.step, fmaf(scale, batch_value<PLANES>(d[s], q), -minimum * batch_value<PLANES>(m[s], q)), acc[s][q]);
+                } else if (Rows::MINIMA) {
+                    acc[s][q] = fmaf(f.step, fmaf(scale, batch_value<PLANES>(d[s], q), -minimum * f.sum), acc[s][q]);
                 } else {
                     acc[s][q] = fmaf(f.step * batch_value<PLANES>(d[s], q), scale, acc[s][q]);
-                    if (Rows::MINIMA) acc[s][q] = fmaf(-f.sum, minimum, acc[s][q]);
                 }
             }
         }
@@ -395,20 +396,11 @@ template <int PLANES> __device__ __forceinline__ void batch_step(float m, float 
         inv = __uint_as_float((uint32_t)(254 - exponent) << 23);
     }
 }
-// balanced base-256 digits of q, lowest first
-template <int PLANES> __device__ __forceinline__ void batch_digits(int q, int (&d)[PLANES]) {
-#pragma unroll
-    for (int p = 0; p + 1 < PLANES; p++) {
-        d[p] = ((q + 128) & 255) - 128;
-        q = (q - d[p]) >> 8;
-    }
-    d[PLANES - 1] = q;
-}
-// What a vector's group ends with: the step, and the step times the sum of its integers (at most 36 bits, from the sums of
-// their upper and lower 16 bits).
+// What a vector's group ends with: the step, and the sum of its integers (at most 36 bits, from the sums of their upper and
+// lower 16 bits).
 template <int PLANES> __device__ __forceinline__ void batch_image_end(uint32_t *img, int g, int K, float step, int upper, int lower) {
     img[8 * PLANES * (K / 32) + g] = __float_as_uint(step);
-    img[(8 * PLANES + 1) * (K / 32) + g] = __float_as_uint(step * fmaf(65536.0f, (float)upper, (float)lower));
+    img[(8 * PLANES + 1) * (K / 32) + g] = __float_as_uint(fmaf(65536.0f, (float)upper, (float)lower));
 }
 
 // Thread j of a group of four neighbouring lanes: the eight values 8j..8j+7 of a K-vector into its image.
@@ -428,7 +420,7 @@ template <int PLANES> __device__ __forceinline__ void batch_image_chunk(uint32_t
         upper += q >> 16;
         lower += q & 0xffff;
         int d[PLANES];
-        batch_digits<PLANES>(q, d);
+        image_digits(q, d);
 #pragma unroll
         for (int p = 0; p < PLANES; p++) w[p][c >> 2] |= (uint32_t)(d[p] & 255) << (8 * (c & 3));
     }
@@ -455,7 +447,7 @@ template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t
     upper += __shfl_xor(upper, 16);
     lower += __shfl_xor(lower, 16);
     int d[PLANES];
-    batch_digits<PLANES>(q, d);
+    image_digits(q, d);
     if (!store) return;
     uint8_t *bytes = reinterpret_cast<uint8_t *>(img + 8 * PLANES * g);
 #pragma unroll

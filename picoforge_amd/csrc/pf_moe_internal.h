@@ -183,8 +183,8 @@ struct PfHipMoe {
 #define PF_IMG_PLANES 3                       // signed byte digits per value: 24 bits
 #define PF_IMG_GROUP (8 * PF_IMG_PLANES)      // dwords of one 32-group's digits
 __host__ __device__ constexpr size_t pf_image2_words(size_t K) { return (K / 32) * (PF_IMG_GROUP + 2); }
-// The image of the kernels for a few rows per expert (pf_moe_batch.hip): three or four digits, and the step times the sum of
-// the integers as a float in place of the sum.
+// The image of the kernels for a few rows per expert (pf_moe_batch.hip): three or four digits, and the sum of the integers
+// as a float.
 __host__ __device__ constexpr size_t pf_batch_image_words(int planes, size_t K) { return (K / 32) * (8 * planes + 2); }
 
 struct PfHipWork {
