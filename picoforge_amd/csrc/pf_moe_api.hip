@@ -831,8 +831,9 @@ struct HcTarget {   // residual streams to inject into instead of writing y
 // alone: with fewer experts the same tokens are more rows an expert.  Swept over E (top-k) = 16 (4), 32 (6), 64, 128, 256 (8),
 // 512 (10), uniform and Zipf(1.1) popularity, 5 to 400 tokens, the widths of the measured layer (one format throughout) and of
 // the checkpoints (profiles); P at the crossing, by E:
-//   pairs -> few rows      Q4_K 224 at 64, beyond 32 tokens elsewhere; IQ2_XXS 172, 165, 216 at 32, 64, 128; the profiles, whose down
-//                          kernel is slower per pair: q2 35 to 57 at any E, q4 61, 69, 54, 92, 113, 142
+//   pairs -> few rows      one format: Q4_K 224 at 64, beyond 32 tokens elsewhere; IQ2_XXS 172, 165, 216 at 32, 64, 128.  The profiles'
+//                          lines lie beyond their crossings (q2 35 to 57 pairs at any E, q4 54 to 142) at 10 and 16 tokens:
+//                          the decode kernels are closer to the result in 64 bits (2.9e-7 against 3.1e-7 and 3.3e-7)
 //   few rows -> grouped    one format 988..1000, 1002..1058, 929..1128, 1977..2167, 2376..2608, 3626..4000; q2 866..890, 918..925,
 //                          970..1678, 1659..2022, 2222..2731, 4000; q4 749..829, 797..853, 717..761, 1282..1344, 1877..2154, 3032..3285
 //   the same, IQ2_XXS gate and up rows as they are stored (slower to read for the few-row kernels)
@@ -841,8 +842,9 @@ struct HcTarget {   // residual streams to inject into instead of writing y
 // The grouped product's time hardly grows until its tiles fill the chip more than once, so up to 64 experts the line is a
 // number of pairs; from there it pays for every expert met and the few-row kernels for every eight rows.  A rule on tokens
 // that fits 512 experts (32 / 240 for Q4_K, 32 / 320, 10 / 400, 16 / 400) is up to 1.42 times slower than the better side with
-// 64: 320 tokens of an IQ2_XXS layer 189 us against 133.  With this rule no size measured is above 1.12 (1.21 in short
-// batches whose neighbours share half of their experts, which meet fewer of them).
+// 64: 320 tokens of an IQ2_XXS layer 189 us against 133.  With this rule no size from 17 tokens on is above 1.10
+// (1.20 in batches whose neighbours share half of their experts, which meet fewer of them).  The q4 line stays above the
+// crossing at 512 experts (1.10 at 400 tokens): the few-row kernels are closer to 64 bits, 3.3e-7 against 5.4e-7.
 struct BatchRange { size_t pair_to, batch_to; };
 static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
     const int combination = pf_decode_tile_layer(moe->desc, moe->w_tiled, moe->w_itile, moe->w_qtile);
@@ -850,18 +852,17 @@ static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
     if (!work->down || !moe->prefill_ready) return {short_to, 0};   // the workspace was planned without the grouping's tables
     const size_t E = moe->desc.experts, K = moe->desc.top_k;
     const bool q4k = moe->desc.type[1] == PF_Q4_K, throughout = moe->desc.type[3] == moe->desc.type[1];
-    size_t pairs = 0, most_tokens = PF_DECODE_MAX_TOKENS;   // no tile-ordered copies: the segment kernels take four tokens
-    if (combination && throughout) { pairs = (q4k ? 200 : 160) + E / 2; most_tokens = PF_PAIR_MAX_TOKENS; }
-    else if (combination) { pairs = q4k ? 55 + E / 6 : 50; most_tokens = PF_TILE_DECODE_MAX_TOKENS; }
-    const size_t by_pairs = pairs / K > PF_DECODE_MAX_TOKENS ? pairs / K : PF_DECODE_MAX_TOKENS;
     auto within = [](size_t low, size_t v, size_t high) { return v < low ? low : v > high ? high : v; };
+    size_t pair_to = PF_DECODE_MAX_TOKENS;   // no tile-ordered copies: the segment kernels take four tokens
+    if (combination && throughout) pair_to = within(PF_TILE_DECODE_MAX_TOKENS, ((q4k ? 200 : 160) + E / 2) / K, PF_PAIR_MAX_TOKENS);
+    else if (combination) pair_to = q4k ? PF_TILE_DECODE_MAX_TOKENS : 10;
     size_t most;
     if (throughout && (q4k || combination)) most = within(1000, 16 * E, 1400 + 9 * E / 2);
     else if (throughout) most = within(570, 10 * E, 900 + 9 * E / 2);
-    else if (q4k) most = within(800, 450 + 11 * E / 2, SIZE_MAX);
+    else if (q4k) most = within(800, 350 + 36 * E / 5, SIZE_MAX);
     else if (combination) most = within(850, 700 + 13 * E / 2, SIZE_MAX);
     else most = within(570, 300 + 21 * E / 4, SIZE_MAX);
-    return {by_pairs < most_tokens ? by_pairs : most_tokens, most / K < PF_BATCH_MAX_TOKENS ? most / K : PF_BATCH_MAX_TOKENS};
+    return {pair_to, most / K < PF_BATCH_MAX_TOKENS ? most / K : PF_BATCH_MAX_TOKENS};
 }
 
 // The kernels a resident layer's batch runs where its rows are 16-byte aligned (else: the general kernels).

@@ -60,8 +60,8 @@ def test_activations_whose_squares_overflow(product, oracle, router):
 
 
 # (experts, top-k, format, last batch of the decode kernels, last of the kernels for a few rows per expert)
-LINES = [(16, 4, abi.GGUF_Q4_K, 32, 250), (64, 8, abi.GGUF_Q4_K, 29, 128), (128, 8, abi.GGUF_IQ2_XXS, 28, 247), (64, 8, "q2", 6, 139),
-         (128, 8, "q4", 9, 144)]
+LINES = [(16, 4, abi.GGUF_Q4_K, 32, 250), (64, 8, abi.GGUF_Q4_K, 29, 128), (128, 8, abi.GGUF_IQ2_XXS, 28, 247), (64, 8, "q2", 10, 139),
+         (128, 8, "q4", 16, 158)]
 
 
 @pytest.mark.parametrize("e,k,fmt,pair_to,batch_to", LINES)
