@@ -310,10 +310,11 @@ def forward64(cfg, weights, x, ids):
 
 
 @pytest.mark.parametrize("kind", ["normal", "outliers", "lognormal"])
-def test_streamed_batches_are_as_close_to_64_bits_as_sums_in_32(product, tmp_path, kind):
+def test_streamed_batches_are_as_close_to_64_bits_as_sums_in_32(product, tmp_path, monkeypatch, kind):
     """The integer products on digit images that take a streamed batch of 17 tokens and more lose no more than the general
     kernels, which sum FP32 activations times decoded weights in FP32 (measured: 0.7 to 0.8 of their distance; three digits
-    instead of four 1.2 to 1.6 of it)."""
+    instead of four 1.2 to 1.6 of it).  The larger images fill the buffers planned for them and no more."""
+    monkeypatch.setenv("PF_WORK_GUARD", "1")
     print(f"case precision {kind}", flush=True)
     cfg = abi.moe_config(2048, 24, 4, 512, 512)
     weights, x = make_layer_inputs(cfg, abi.GGUF_IQ2_XXS, 60, seed=11)
@@ -344,6 +345,9 @@ def test_streamed_batches_are_as_close_to_64_bits_as_sums_in_32(product, tmp_pat
             assert product.forward_streamed(layer.handle, pool, 0, abi.f32_view(x), abi.f32_view(y), C.byref(routes), layer.work,
                                             C.byref(layer.err)) == abi.QW4_OK, layer.err.detail
             outputs.append((y, ids))
+            damaged, first = C.c_int(), C.c_int()
+            assert product.hip.work_check_guards(product.device_work(layer.work), C.byref(damaged), C.byref(first)) == 0
+            assert (damaged.value, first.value) == (0, -1), "a guard was overwritten"
     product.pool_destroy(pool)
     os.close(fd)
     np.testing.assert_array_equal(outputs[0][1], outputs[1][1])
