@@ -2,10 +2,11 @@
 // its rows, in one place for the kernel and for the host-side check (tests/check_plain_walk.cpp).
 //
 // A row's columns pass in rounds of PF_PLAIN_CHUNK staged activation columns; a batch is `batch_cols` columns of weights
-// (PF_PLAIN_CHUNK is whole batches of every format).  A wave takes every `parts`-th batch of the whole row, from batch `part`
-// on, and requests a batch's successor before it multiplies it.  Batches are counted over the whole row and not within a
-// round: a round of the 256-column format holds two batches, fewer than the four waves of a split workgroup, so a wave's next
-// batch lies a round or two further on.
+// (PF_PLAIN_CHUNK is whole batches of every format).  The waves that share a row take its batches in turn, and each requests
+// its next batch before it multiplies the present one.  No more waves take part than a round holds batches, so that a wave's
+// batches lie equally in every round: two of the four waves of a split workgroup for the 256-column format, whose batches a
+// wave would otherwise meet in every other round only.  (Counting the batches over the whole row, so that all four take part,
+// costs the other formats 2 % of the launch: the compiler then forms every batch's address anew.)
 #pragma once
 
 #define PF_PLAIN_CHUNK 512
@@ -22,17 +23,19 @@
 template <class Stage, class Request, class Take, class Multiply>
 PF_WALK_FN void pf_plain_walk(int a_cols, int batch_cols, int part, int parts, bool active, Stage stage, Request request, Take take,
                               Multiply multiply) {
-    const int batches = (a_cols + batch_cols - 1) / batch_cols;
-    int batch = part;
-    if (active && batch < batches) request(batch);   // on its way while the first columns are staged
+    const int batches = (a_cols + batch_cols - 1) / batch_cols, held = PF_PLAIN_CHUNK / batch_cols;
+    const int stride = held >= 4 || parts < held ? parts : held;   // (at most four waves share a row)
+    const bool takes = active && part < stride;
+    if (takes && part < batches) request(part);   // on its way while the first columns are staged
     for (int c0 = 0; c0 < a_cols; c0 += PF_PLAIN_CHUNK) {
         const int cols = a_cols - c0 < PF_PLAIN_CHUNK ? a_cols - c0 : PF_PLAIN_CHUNK;
         stage(c0, cols);
-        if (!active) continue;
-        for (; batch * batch_cols < c0 + cols; batch += parts) {
+        if (!takes) continue;
+        for (int k0 = batch_cols * part; k0 < cols; k0 += batch_cols * stride) {
             take();
-            if (batch + parts < batches) request(batch + parts);
-            multiply(batch * batch_cols - c0, cols);
+            const int after = (c0 + k0) / batch_cols + stride;
+            if (after < batches) request(after);
+            multiply(k0, cols);
         }
     }
 }
