@@ -897,7 +897,14 @@ static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_
     } else if (family == FAMILY_BATCH) {
         pf_launch_batch(a, (int)tokens, s, work->stage_limit);
     } else if (family == FAMILY_GROUPED) {
-        pf_launch_prefill(a, (int)tokens, s, work->stage_limit);
+        // the grouped product addresses a chunk's activation rows with 32 bits: beyond that in pieces, whole row tiles each
+        const size_t piece = pf_prefill_most_tokens((int)d->hidden);
+        for (size_t t = 0; t < tokens; t += piece) {
+            PfKernelArgs b = a;
+            b.x += t * a.x_pitch; b.y += t * a.y_pitch; b.ids += t * d->top_k; b.route_weights += t * d->top_k;
+            if (b.hc_residual) { b.hc_residual += t * a.hc_token_pitch; b.hc_inject += t * a.hc_streams; }
+            pf_launch_prefill(b, (int)(tokens - t < piece ? tokens - t : piece), s, work->stage_limit);
+        }
     } else {
         // the general kernels stage one token's activations in LDS
         const size_t lds_route = ((size_t)d->hidden + 3 * (size_t)d->experts) * 4;

@@ -274,6 +274,7 @@ void pf_launch_q4k_tile(const uint8_t *d_src, uint8_t *d_dst, size_t rows, int b
 void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hipStream_t stream);
 size_t pf_prefill_half_row(int cols);   // halfs per row of the fp16 form of a matrix with `cols` columns
 int pf_prefill_max_tiles(int tokens, int experts, int top_k);
+size_t pf_prefill_most_tokens(int hidden);   // that one launch of pf_launch_prefill takes
 // pf_moe_batch.hip: a few rows per expert, for the layers of the tile decode kernels
 void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
 void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, hipStream_t stream);

@@ -26,8 +26,11 @@
 
 typedef _Float16 half_t;
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 typedef float float16v __attribute__((ext_vector_type(16)));
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 
 // halfs per row of a converted matrix: high parts, low parts, per 256-block the 16 group-sum halfs
 // [even groups: 4 high, 4 low][odd groups: 4 high, 4 low]
@@ -327,500 +330,388 @@ static void launch_router(const PfKernelArgs &a, int tokens, hipStream_t stream)
 // ---- grouped product ------------------------------------------------------------------------------
 enum { PF_GEMM_GATE_UP = 0, PF_GEMM_DOWN = 1 };
 
-// Workgroup = one 32-row tile of an expert against 64 NW weight rows: NW compute waves, each
-// with two 32-row weight tiles (gate + up of 32 units, or 2 x 32 down rows), and 1 + NW / 4 loader
-// waves.
+// Workgroup = one 32-row tile of an expert against 32 GW weight rows: eight waves, each with one 32-row weight tile (the gate and
+// the up tiles of 128 units, or 256 down rows); a down workgroup goes over several such slabs.
 //
-// Only the loader waves issue global loads.  They move the operands of one stage (64 of the K
-// columns) straight into LDS, 16 bytes per lane, up to four stages ahead of the products, through
-// a ring of five slots: with one workgroup per compute unit that keeps about 100 KB on their way;
-// a wave counts at most 63 loads, so the stream is split over three loaders (activations; the
-// weight runs of compute waves 0-3; of 4-7).  A stalled memory pipeline holds up the loaders, never the waves that feed the matrix
-// cores.  One workgroup barrier per stage hands the landed slot to the compute waves and the slot
-// they have just left back to the loaders.
+// A wave takes its weights straight from memory into registers, 16 bytes a lane and whole cache lines an instruction, and
+// requests the bytes of the next 256-block into the registers that the products have just left: 4 to 5 KB a wave on their way
+// at any time, and no wave waits for another one's.  The activation rows are what the waves share: a block's 256 columns in LDS,
+// two copies in turn, the next block's requested straight into the other copy.  One barrier a 256-block.  A wave with one tile
+// keeps to 128 registers, so two workgroups, four waves a SIMD, share a compute unit: while one unpacks a block's headers, adds
+// its block up or waits, the others feed the matrix core.
 //
-//   slot   [0, A_PART)            high parts of the 32 activation rows, 128 bytes each: four images
-//                                 of eight rows, chunk-major (16-byte chunk c of row r at 128 c + 16 r)
-//          [A_PART, 2 A_PART)     low parts likewise
-//          [SLOT_W, +2 NW KB)     the stage's 32-byte nibble run of every weight row: per tile the
-//                                 first halves of the 32 rows, then the second halves
-//   once per 256-block: the 16-byte block headers of the 2 NW tiles, the activation rows' group sums
+// Bound by power and by the bytes together: at 1024 tokens of the benchmark's Q4_K layer (640 row tiles, 604 MB of gate and up
+// weights) the card draws 1.28 kW and its clock falls to 1.8 GHz; without the memory reads the launch takes 137 us, without
+// the products 157, as it is 177.  Before, with loader waves that moved every operand through a ring in LDS and a barrier every
+// 64 columns, it took 201; the down launch 103 against 109, IQ2_XXS (777 tokens) 156 + 92 against 201 + 102, Q4_K rows of 2560
+// against 640 units (2048 tokens; units in slabs of 128, not 256) 375 against 477.
 //
-// IQ2_XXS differs in the weight bytes only: a row's stage is 16 bytes (two 32-groups of four grid
-// indices and one word of signs and scale), so a wave's two tiles are one 1 KB image
-// [tile][row][16 bytes]; per 256-block a row brings its fp16 scale (the dword around it); the
-// 256 x 8 magnitude grid and the 128 sign masks sit in LDS behind the ring.
+//   copy   [part: high, low][64 columns][eight rows][16-byte chunk of the 64 columns][row][16 bytes]
 //
-// Matrix-core operands.  Lane (n = lane % 32, h = lane / 32) holds column n (a weight row) and
-// supplies K slots 8h..8h+7.  In stage j, step t, these are the codes 8t..8t+7 of group 2j + h
-// (h = 0: the low nibbles of the run, h = 1: the high nibbles), so a lane needs the scale and the
-// minimum of one group per stage, and activation columns 64 j + 32 h + 8 t + 0..7.
-#define NW 8                               // compute waves per workgroup
-#define NL (1 + NW / 4)                    // loader waves
-#define RING_SLOTS 5
-#define A_GROUP 1152                       // bytes between eight-row images: 1 KB + 128, neighbours start on opposite bank halves
-#define A_PART (4 * A_GROUP)
-#define SLOT_W (2 * A_PART)
-#define SLOT_BYTES (SLOT_W + 2 * NW * 1024)
-#define HDR_OFF (RING_SLOTS * SLOT_BYTES)
-#define BLOCK_BYTES (2 * NW * 512 + 1024)   // per 256-block: headers, then sums; two copies (blocks alternate)
-#define SUMS_OFF (HDR_OFF + 2 * NW * 512)
-#define GEMM_LDS (HDR_OFF + 2 * BLOCK_BYTES)   // 146 432 bytes with 8 compute waves: one workgroup per compute unit
+// Tiles of experts with at most 16 rows put the low parts of their rows into the tile's other 16 rows (PARTS = 1): one product
+// instead of two, half of the operand reads and of the copy.
+//
+// Matrix-core operands.  Lane (n = lane % 32, h = lane / 32) holds column n (a weight row) and supplies K slots 8h..8h+7.  Which
+// columns of the block those are is free as long as the activations' lanes take the same ones.  Q4_K: a lane loads half h of a
+// run's 32 nibble bytes, steps 0 and 1 are the low nibbles (group 2j, columns 16h..16h+15 of it), steps 2 and 3 the high
+// nibbles (group 2j + 1).  IQ2_XXS: a lane loads the 8 bytes of group 2j + h, a step is one of its four grid entries.
+#define GW 8                                   // waves per workgroup
+#define GEMM_IMAGE 1152                        // between eight-row images of 64 columns: 1 KB + 128, neighbours start on opposite bank halves
+#define GEMM_PART_BYTES (16 * GEMM_IMAGE)      // one part of 32 rows x 256 columns
+#define GEMM_COPY_BYTES (2 * GEMM_PART_BYTES)
+#define GEMM_LDS (2 * GEMM_COPY_BYTES)
 #define IQ2_GRID_OFF GEMM_LDS                  // IQ2_XXS: 256 grid entries of 8 magnitudes, then 128 masks of 8 fp16 sign bits
 #define IQ2_SIGN_OFF (IQ2_GRID_OFF + 2048)
 #define GEMM_LDS_IQ2 (IQ2_SIGN_OFF + 2048)
-static_assert(RING_SLOTS == 5 && NW % 4 == 0, "the loaders' wait counts below assume three younger stages on their way");
 
 __device__ __forceinline__ void to_lds(const void *global, unsigned char *lds) {
     __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint32_t *>(global), reinterpret_cast<uint32_t *>(lds), 16, 0, 0);
 }
 
-__device__ __forceinline__ void to_lds_dword(const void *global, unsigned char *lds) {   // 4 bytes per lane, lane l at lds + 4 l
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint32_t *>(global), reinterpret_cast<uint32_t *>(lds), 4, 0, 0);
-}
-
-__device__ __forceinline__ void stage_barrier() {
+// Barrier between the uses of an LDS copy: the wave's own LDS accesses are over, of its loads from memory the youngest LATER may
+// still be on their way.
+template <int LATER> __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((LATER & 15) | (LATER >> 4) << 14 | 0x70);   // vmcnt(LATER) lgkmcnt(0), in a form that the compiler counts with
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
 
-struct GemmTarget {   // one work item of the grouped product: a 32-row tile of an expert against one slab of weight rows
+// A buffer whose reads beyond `bytes` give zero and cost no memory access.
+typedef __amdgpu_buffer_rsrc_t PfBuffer;
+typedef __attribute__((address_space(3))) unsigned char lds_byte;
+__device__ __forceinline__ PfBuffer pf_buffer(const void *base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+#define PF_NOWHERE 0xC0000000u   // an offset beyond every buffer: none is larger
+
+struct GemmItem {   // a 32-row tile of an expert
     bool shared;
-    int first, count, inter, kblocks, a_cols, slab;
-    int m0, rows_here;    // first row of the tile within the expert's rows, rows in it
-    int waves;            // compute waves whose weight rows exist (the last slab of a narrow matrix has fewer)
-    uint32_t zero_row;    // index of the all-zero row that ends the fp16 form of the activation matrix
-    uint32_t row_bytes;   // of the weight tensor(s)
-    uint32_t wave_rows;   // weight rows between the tiles of consecutive compute waves
-    bool tiled;           // weights in the tile order of pf_k_q4k_tile (else GGUF row order)
-    const uint8_t *w0, *w1;   // first weight row of compute wave 0's two tiles
-    const uint16_t *s0, *s1;  // IQ2_XXS: the tensors' fp16 block scales, and the index of the tiles' first row's first scale
-    uint32_t sidx0, sidx1, bpr;
-    const half_t *a16;
-    const float *a_scale;
+    int expert, first, m0, rows_here;   // first row of the tile in expert order and within the expert, rows in it
+    int inter;
 };
 
-// Work item q -> (row tile, slab).  Workgroups go to the eight XCDs round robin by index and a
-// workgroup's items are a multiple of eight apart.  The tile list is cut into groups of GEMM_XCD_TILES
-// consecutive tiles and the groups dealt to the XCDs in turn; the items of a group (its tiles' slabs)
-// get numbers eight apart: neighbouring workgroups of one XCD, one L2, at the same time.  The slabs of
-// a row tile read the same activation rows, and the row tiles of one expert, neighbours in the list,
-// the same weights: fetched once from memory where they fall into one group.  False: nothing to do
-// for q.  Every wave of the workgroup evaluates this for itself, with the same result.
+// Work item q -> (row tile, slab group).  Workgroups go to the eight XCDs round robin by index.  The tile list is cut into groups of
+// GEMM_XCD_TILES consecutive tiles and the groups dealt to the XCDs in turn; the items of a group (its tiles' slabs) get numbers
+// eight apart: neighbouring workgroups of one XCD, one L2, at the same time.  The slabs of a row tile read the same
+// activation rows, and the row tiles of one expert, neighbours in the list, the same weights: fetched once from memory where
+// they fall into one group.  False: nothing to do for q.
 #define GEMM_XCD_TILES 8
-template <int MODE, int FMT>
-__device__ __forceinline__ bool gemm_item(const PfKernelArgs &a, int tokens, int slabs, uint32_t q, GemmTarget &g) {
-    const int E = a.experts, K = a.top_k;
+__device__ __forceinline__ bool gemm_item(const PfKernelArgs &a, int slabs, uint32_t q, GemmItem &g, int &slab) {
     const uint32_t xcd = q % 8, turn = q / 8, r = turn / slabs;
     const uint32_t tile = GEMM_XCD_TILES * ((r / GEMM_XCD_TILES) * 8 + xcd) + r % GEMM_XCD_TILES;
     if (tile >= a.tiles[0]) return false;
-    const uint32_t entry = a.tiles[1 + tile];
-    const int expert = entry & 0xffffu;
-    g.m0 = 32 * (int)(entry >> 16);
-    g.slab = turn % slabs;
-    g.shared = expert == E;
-    const int P = tokens * K;
-    g.first = g.shared ? P : (int)a.offsets[expert];
-    g.count = g.shared ? tokens : (int)a.offsets[expert + 1] - g.first;
-    if (g.count <= g.m0) return false;
-    g.rows_here = min(32, g.count - g.m0);
+    const uint4 item = reinterpret_cast<const uint4 *>(a.items)[tile];
+    slab = turn % slabs;
+    g.expert = (int)item.x; g.first = (int)item.y; g.rows_here = (int)item.z; g.m0 = (int)item.w;
+    g.shared = g.expert == a.experts;
     g.inter = g.shared ? a.shared_inter : a.inter;
-    const size_t ex = g.shared ? 0 : (size_t)expert;
-    if (a.type[MODE == PF_GEMM_GATE_UP ? (g.shared ? 4 : 1) : (g.shared ? 6 : 3)] != (uint32_t)FMT)
-        return false;   // another format: the plain grouped product takes the item
-    if (MODE == PF_GEMM_GATE_UP) {
-        const int tg = g.shared ? 4 : 1;
-        if (32 * NW * g.slab >= g.inter) return false;
-        g.row_bytes = (uint32_t)a.row_bytes[tg];
-        g.tiled = a.wt[tg] != nullptr;
-        g.w0 = (g.tiled ? a.wt[tg] : a.w[tg]) + ex * a.expert_bytes[tg] + (size_t)(32 * NW * g.slab) * g.row_bytes;
-        g.w1 = (g.tiled ? a.wt[tg + 1] : a.w[tg + 1]) + ex * a.expert_bytes[tg + 1] + (size_t)(32 * NW * g.slab) * g.row_bytes;
-        if (FMT == PF_IQ2_XXS) {
-            g.bpr = (uint32_t)a.blocks_per_row[tg];
-            g.s0 = reinterpret_cast<const uint16_t *>(a.w[tg] + a.scale_offset[tg]);
-            g.s1 = reinterpret_cast<const uint16_t *>(a.w[tg + 1] + a.scale_offset[tg + 1]);
-            g.sidx0 = g.sidx1 = (uint32_t)((ex * a.n_out[tg] + 32 * NW * g.slab) * g.bpr);
-        }
-        g.wave_rows = 32;
-        g.waves = min(NW, (g.inter - 32 * NW * g.slab) / 32);
-        g.kblocks = a.hidden / 256; g.a_cols = a.hidden;
-        g.a16 = reinterpret_cast<const half_t *>(a.x16); g.a_scale = a.x_scale;
-        g.zero_row = a.token_cap;
-    } else {
-        const int td = g.shared ? 6 : 3;
-        if (64 * NW * g.slab >= a.hidden) return false;
-        g.row_bytes = (uint32_t)a.row_bytes[td];
-        g.tiled = a.wt[td] != nullptr;
-        g.w0 = (g.tiled ? a.wt[td] : a.w[td]) + ex * a.expert_bytes[td] + (size_t)(64 * NW * g.slab) * g.row_bytes;
-        g.w1 = g.w0 + (size_t)32 * g.row_bytes;
-        if (FMT == PF_IQ2_XXS) {
-            g.bpr = (uint32_t)a.blocks_per_row[td];
-            g.s0 = g.s1 = reinterpret_cast<const uint16_t *>(a.w[td] + a.scale_offset[td]);
-            g.sidx0 = (uint32_t)((ex * a.n_out[td] + 64 * NW * g.slab) * g.bpr);
-            g.sidx1 = g.sidx0 + 32 * g.bpr;
-        }
-        g.wave_rows = 64;
-        g.waves = min(NW, (a.hidden - 64 * NW * g.slab) / 64);
-        g.kblocks = g.inter / 256; g.a_cols = g.inter;
-        g.a16 = reinterpret_cast<const half_t *>(g.shared ? a.sact16 : a.act16);
-        g.a_scale = g.shared ? a.sact_scale : a.act_scale;
-        g.zero_row = g.shared ? a.token_cap : a.token_cap * (uint32_t)K;
-    }
     return true;
 }
 
-// first item at or after q (stepping by the grid size) that has work; false when the list is exhausted
-template <int MODE, int FMT>
-__device__ __forceinline__ bool gemm_next_item(const PfKernelArgs &a, int tokens, int slabs, uint32_t items, uint32_t &q,
-                                               GemmTarget &g) {
-    for (; q < items; q += gridDim.x)
-        if (gemm_item<MODE, FMT>(a, tokens, slabs, q, g)) return true;
-    return false;
-}
-
-// Loads of the stages that may still be on their way when stage s is handed over: the younger
-// stages issued so far, at most three.  Three consecutive stages hold one that opens a 256-block
-// (and carries `block_loads` more) unless stage s opens one itself; fewer than three only happens
-// at the end, inside the last block.
-#define WAIT_YOUNGER(younger, opens, per_stage, block_loads)                             \
-    do {                                                                                 \
-        if ((younger) >= 3 && (opens)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (per_stage) + (block_loads)) : "memory"); \
-        else if ((younger) >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (per_stage)) : "memory");        \
-        else if ((younger) == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (per_stage)) : "memory");        \
-        else if ((younger) == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(1 * (per_stage)) : "memory");        \
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                            \
-    } while (0)
-
-// A loader wave.  ROLE 0 moves the activation images and the group sums (and leaves the rows'
-// scales for the epilogue); ROLE q >= 1 the weight runs and block headers of compute waves
-// 4 (q - 1) .. 4 (q - 1) + 3.  It walks the workgroup's items as one stream of stages, up to
-// RING_SLOTS - 1 stages ahead of the compute waves, also across item boundaries: the ring never
-// drains between items.  Every workgroup barrier here pairs with one of gemm_compute.
-template <int MODE, int FMT, int ROLE>
-__device__ __forceinline__ void gemm_loader(const PfKernelArgs &a, int tokens, int slabs, uint32_t items, unsigned char *ring,
-                                            float (*row_scale)[32]) {
-    const int lane = pf_lane(), K = a.top_k;
-    GemmTarget g;
-    uint32_t q = blockIdx.x;
-    bool more = gemm_next_item<MODE, FMT>(a, tokens, slabs, items, q, g);
-    int kb = 0, j = 0, slot_index = 0, block_parity = 0, item_index = 0;
-    uint32_t a_off[4] = {0, 0, 0, 0}, a_live[4] = {0, 0, 0, 0}, s_off = 0, s_live = 0, w_off = 0, h_off = 0, block_step = 0,
-             run0 = 0, run_step = 0;
-    size_t wave_bytes = 0;
-    auto open_item = [&]() {   // per-lane source offsets of the item the issue cursor has reached
-        if (ROLE == 0) {
-            // activation images: instruction i carries rows 8i..8i+7, lane = 8 * chunk + row.  The
-            // lanes of rows beyond the tile's last all read the first 16 bytes of the matrix's
-            // all-zero row, whatever the stage: one cache line serves them (a_live masks the
-            // stage's column offset away), so padding costs no memory traffic.
-            const uint32_t a_pitch = (uint32_t)pf_half_row(g.a_cols);
-            auto source_row = [&](int m) -> uint32_t {
-                if (m >= g.rows_here) return g.zero_row;
-                if (g.shared) return (uint32_t)(g.m0 + m);
-                return MODE == PF_GEMM_GATE_UP ? a.row_to_pair[g.first + g.m0 + m] / (uint32_t)K : (uint32_t)(g.first + g.m0 + m);
-            };
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int m = 8 * i + (lane & 7);
-                a_live[i] = m < g.rows_here ? 0xffffffffu : 0u;
-                a_off[i] = source_row(m) * a_pitch + (8u * (uint32_t)(lane >> 3) & a_live[i]);
-            }
-            const uint32_t mine = source_row(lane & 31);
-            s_live = (lane & 31) < g.rows_here ? 0xffffffffu : 0u;
-            s_off = mine * a_pitch + ((2u * (uint32_t)g.a_cols + 8u * (uint32_t)(lane >> 5)) & s_live);
-            // the rows' scales for the epilogue of this item (read many barriers later; four copies
-            // in turn, because this wave may open the item after next before the epilogue of the
-            // current one is over)
-            if (lane < 32) row_scale[item_index & 3][lane] = (lane < g.rows_here) ? g.a_scale[mine] : 0.0f;
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        } else if (FMT == PF_IQ2_XXS) {
-            // lane = 32 * (tile of the wave's pair) + row: the row's two groups of the stage, and per
-            // block the dword that holds the row's fp16 scale
-            w_off = (uint32_t)(lane & 31) * g.row_bytes;
-            h_off = (uint32_t)(lane & 31) * g.bpr;
-            wave_bytes = (size_t)g.wave_rows * g.row_bytes;
-        } else {
-            // weight runs: lane = 32 * half + row; headers: lane = 32 * (tile of the wave's pair) + row.
-            // Tile order: a 32-row tile's 256-block is 4608 consecutive bytes, the 32 headers, then per
-            // run the 1 KB image exactly as it lands in LDS; row order: 144-byte blocks at the row pitch.
-            w_off = g.tiled ? 16u * (uint32_t)lane : (uint32_t)(lane & 31) * g.row_bytes + 16u * (uint32_t)(lane >> 5);
-            h_off = g.tiled ? 16u * (uint32_t)(lane & 31) : (uint32_t)(lane & 31) * g.row_bytes;
-            block_step = g.tiled ? 4608u : 144u; run0 = g.tiled ? 512u : 16u; run_step = g.tiled ? 1024u : 32u;
-            wave_bytes = (size_t)g.wave_rows * g.row_bytes;
-        }
-        item_index++;
-    };
-    auto issue = [&]() {   // the stage under the issue cursor, then advance the cursor
-        unsigned char *slot = ring + slot_index * SLOT_BYTES;
-        unsigned char *block = ring + block_parity * BLOCK_BYTES;
-        if (ROLE == 0) {
-            const uint32_t high = 256u * (uint32_t)kb + 64u * (uint32_t)j, low = high + (uint32_t)g.a_cols;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                to_lds(g.a16 + a_off[i] + (high & a_live[i]), slot + i * A_GROUP);
-                to_lds(g.a16 + a_off[i] + (low & a_live[i]), slot + A_PART + i * A_GROUP);
-            }
-            if (j == 0) to_lds(g.a16 + s_off + (16u * (uint32_t)kb & s_live), block + SUMS_OFF);
-        } else if (FMT == PF_IQ2_XXS) {
-            const uint8_t *tile = (lane >> 5) ? g.w1 : g.w0;
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int v = 4 * (ROLE - 1) + c, vv = min(v, g.waves - 1);   // a wave without rows repeats the last one's
-                to_lds(tile + (size_t)vv * wave_bytes + w_off + 64u * (uint32_t)kb + 16u * (uint32_t)j, slot + SLOT_W + v * 1024);
-            }
-            if (j == 0) {
-                const uint16_t *scales = (lane >> 5) ? g.s1 : g.s0;
-                const uint32_t first = (lane >> 5) ? g.sidx1 : g.sidx0;
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int v = 4 * (ROLE - 1) + c, vv = min(v, g.waves - 1);
-                    const uint32_t at = first + (uint32_t)vv * g.wave_rows * g.bpr + h_off + (uint32_t)kb;
-                    to_lds_dword(scales + (at & ~1u), block + HDR_OFF + v * 256);
-                }
-            }
-        } else {
-            const uint32_t run = block_step * (uint32_t)kb + run0 + run_step * (uint32_t)j;
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int v = 4 * (ROLE - 1) + c;
-                const size_t at = (size_t)min(v, g.waves - 1) * wave_bytes;   // a wave without rows repeats the last one's
-                to_lds(g.w0 + at + run + w_off, slot + SLOT_W + (2 * v) * 1024);
-                to_lds(g.w1 + at + run + w_off, slot + SLOT_W + (2 * v + 1) * 1024);
-            }
-            if (j == 0) {
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int v = 4 * (ROLE - 1) + c;
-                    const size_t at = (size_t)min(v, g.waves - 1) * wave_bytes;
-                    to_lds(((lane >> 5) ? g.w1 : g.w0) + at + block_step * (uint32_t)kb + h_off, block + HDR_OFF + v * 1024);
-                }
-            }
-        }
-        slot_index = slot_index + 1 == RING_SLOTS ? 0 : slot_index + 1;
-        if (++j == 4) {
-            j = 0;
-            block_parity ^= 1;
-            if (++kb == g.kblocks) {
-                kb = 0;
-                q += gridDim.x;
-                more = gemm_next_item<MODE, FMT>(a, tokens, slabs, items, q, g);
-                if (more) open_item();
-            }
-        }
-    };
-    if (more) open_item();
-    // Before the barrier of stage s its loads have landed (loads complete in order).  After it,
-    // the slot of stage s - 1 is free for stage s + RING_SLOTS - 1.  A stage that opens a block also
-    // brings its headers and sums, into the copy that the block before the previous one used.
-    int issued = 0;
-    while (issued < RING_SLOTS - 1 && more) { issue(); issued++; }
-    for (int s = 0; s < issued; s++) {
-        const int younger = issued - s - 1;   // at most RING_SLOTS - 2
-        const bool opens = (s & 3) != 0;      // one of stages s + 1 .. s + 3 opens a block
-        if (ROLE == 0) WAIT_YOUNGER(younger, opens, 8, 1);
-        else if (FMT == PF_IQ2_XXS) WAIT_YOUNGER(younger, opens, 4, 4);
-        else WAIT_YOUNGER(younger, opens, 8, 4);
-        stage_barrier();
-        if (more) { issue(); issued++; }
-    }
-}
-
-// 6-bit scale and minimum of group 2 jj + h (h per lane) from the 12 packed bytes of a block
-// header (src/qwen4_packed.c:88-91)
-__device__ __forceinline__ void q4_scale_min(const uint4 &hdr, int jj, int h, uint32_t &sc, uint32_t &mn) {
-    const int sh = 16 * (jj & 1) + 8 * h;
-    if (jj < 2) {
-        sc = (hdr.y >> sh) & 63u;
-        mn = (hdr.z >> sh) & 63u;
+// One expert's tensor as a wave reads it: the buffers and what the lanes add to an offset in them.  Tile order keeps a 32-row
+// tile's 256-block together, row order a row's blocks.
+struct GemmRows {
+    const uint8_t *base, *head;         // codes, and block headers (the same bytes except for IQ2_XXS in row order: half scales)
+    uint32_t bytes, head_bytes;
+    uint32_t lane_at, head_at;          // per lane: of its codes, of its row's block header
+    uint32_t tile_step, block_step, run_step, head_tile_step, head_step;
+};
+template <int FMT> __device__ __forceinline__ GemmRows gemm_rows(const PfKernelArgs &a, int t, size_t expert) {
+    const uint32_t n = pf_lane() & 31, h = pf_lane() >> 5, row_bytes = (uint32_t)a.row_bytes[t], blocks = (uint32_t)a.blocks_per_row[t];
+    const bool tiled = FMT == PF_IQ2_XXS ? a.wi[t] != nullptr : a.wt[t] != nullptr;
+    GemmRows r;
+    if (FMT == PF_IQ2_XXS && tiled) {
+        r.bytes = (uint32_t)pf_i2t_expert_bytes(a.n_out[t], (int)blocks);
+        r.base = a.wi[t] + expert * r.bytes;
+        r.lane_at = 16 * n + 8 * h; r.head_at = 2048 + 2 * n;
+        r.block_step = r.head_step = PF_I2T_CHUNK; r.run_step = 512;
+        r.tile_step = r.head_tile_step = blocks * PF_I2T_CHUNK;
+    } else if (FMT == PF_IQ2_XXS) {   // payloads of all experts, then their scales
+        r.bytes = (uint32_t)a.expert_bytes[t]; r.head_bytes = 2 * (uint32_t)a.n_out[t] * blocks;
+        r.base = a.w[t] + expert * r.bytes;
+        r.head = a.w[t] + a.scale_offset[t] + expert * r.head_bytes;
+        r.lane_at = n * row_bytes + 8 * h; r.head_at = 2 * n * blocks;
+        r.block_step = 64; r.head_step = 2; r.run_step = 16;
+        r.tile_step = 32 * row_bytes; r.head_tile_step = 64 * blocks;
+        return r;
     } else {
-        const uint32_t hi = (hdr.w >> sh) & 255u, lo_s = (hdr.y >> sh) & 255u, lo_m = (hdr.z >> sh) & 255u;
-        sc = (hi & 15u) | ((lo_s & 192u) >> 2);
-        mn = (hi >> 4) | ((lo_m & 192u) >> 2);
+        r.bytes = (uint32_t)a.expert_bytes[t];
+        r.base = (tiled ? a.wt[t] : a.w[t]) + expert * a.expert_bytes[t];
+        r.tile_step = r.head_tile_step = 32 * row_bytes;
+        r.lane_at = tiled ? 512 + 512 * h + 16 * n : 16 + n * row_bytes + 16 * h;
+        r.head_at = tiled ? 16 * n : n * row_bytes;
+        r.block_step = r.head_step = tiled ? 4608 : 144; r.run_step = tiled ? 1024 : 32;
     }
+    r.head = r.base; r.head_bytes = r.bytes;
+    return r;
 }
 
-// eight codes (the nibbles under mask in two dwords) times the group's scale, exact in fp16: a
-// nibble under the exponent byte 0x64 reads as 1024 + q (low nibble) or 1024 + 16 q (high nibble,
-// left in place), and (1024 + q) * s - 1024 * s = q * s, (1024 + 16 q) * (s / 16) - 64 s = q * s;
-// s2 and c are the pair of constants that belongs to the lane's nibble position
-__device__ __forceinline__ half8v q4_scaled_codes(uint32_t w0, uint32_t w1, uint32_t mask, half2v s2, half2v c) {
-    const uint32_t q0 = w0 & mask, q1 = w1 & mask;
-    const uint32_t bias = 0x64646464u;
-    const half2v p0 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, q0, 0x04010400u));
-    const half2v p1 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, q0, 0x04030402u));
-    const half2v p2 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, q1, 0x04010400u));
-    const half2v p3 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, q1, 0x04030402u));
-    const half2v v0 = p0 * s2 - c, v1 = p1 * s2 - c, v2 = p2 * s2 - c, v3 = p3 * s2 - c;
-    return half8v{v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
+// Four nibbles (those under mask in a dword) times the group's scale as fp16 operands, exact: a nibble alone in a half is the
+// subnormal q 2^-24 (16 q 2^-24 where a high nibble stays in place), s2 the scale times 2^10 (2^6) in both halves, the product
+// q s 2^-14, a normal number.  The fold takes the 2^-14 away again.
+__device__ __forceinline__ half4v q4_scaled_codes(uint32_t w, uint32_t mask, half2v s2) {
+    const uint32_t q = w & mask;
+    const half2v v0 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0u, q, 0x0C010C00u)) * s2;
+    const half2v v1 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0u, q, 0x0C030C02u)) * s2;
+    return half4v{v0.x, v0.y, v1.x, v1.y};
 }
 
-// A compute wave: all K against its two weight tiles.  A 256-block's result is
-// d * P - dmin * Q with P = sum (scale * code) x and Q = sum_g min_g * (sum of x over group g).
-// slot_off and block_parity carry the ring position from one item to the next.
-__device__ __forceinline__ void gemm_compute(const unsigned char *ring, int kblocks, float16v &acc0, float16v &acc1, int &slot_off,
-                                             int &block_parity) {
-    const int lane = pf_lane(), wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
-    const uint32_t mask = h ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
-    const half_t unit = h ? (half_t)0.0625f : (half_t)1.0f;
-    const int bias_shift = h ? 6 : 10;
-    const unsigned char *a_lane = ring + (n >> 3) * A_GROUP + (4 * h) * 128 + (n & 7) * 16;
-    const unsigned char *w_lane = ring + SLOT_W + (2 * wave) * 1024 + n * 16;
+__device__ __forceinline__ half8v join(half4v a, half4v b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+
+// A wave's weight tile over one 256-block: the bytes as they were loaded (code[run], head), and what the block's headers say (open).
+// The block is sixteen steps of one matrix-core operand: step i is step i % 4 of run i / 4, against the 16-byte column chunk
+// chunk(i) + chunk_h h of the run's 64 columns.
+template <int FMT> struct GemmBlock;
+template <> struct GemmBlock<PF_Q4_K> {
+    uint4v code[4], head;
+    half2v scale[4];         // groups 2j and 2j + 1: times 2^10 and 2^6
+    float d, low;            // factors of the products (2^14 d) and of the minima's sums
+    static __device__ __forceinline__ constexpr int chunk(int i) { return 4 * ((i & 3) >> 1) + (i & 1); }
+    static constexpr int chunk_h = 2;
+    static constexpr int requests = 6;   // of a block: its headers, the rows' sums, four runs
+    __device__ __forceinline__ void request_run(int j, const PfBuffer &b, const GemmRows &r, uint32_t at) {
+        code[j] = __builtin_amdgcn_raw_buffer_load_b128(b, (int)r.lane_at, (int)(at + (uint32_t)j * r.run_step), 0);
+    }
+    __device__ __forceinline__ void request_head(const PfBuffer &b, const GemmRows &r, uint32_t at) {
+        head = __builtin_amdgcn_raw_buffer_load_b128(b, (int)r.head_at, (int)at, 0);
+    }
+    // Scales and minima of all eight groups (src/qwen4_packed.c:88-91), four bytes at a time; returns the minima as the operand
+    // of the product with the rows' group sums: K slots 8h..8h+3 hold the high parts of groups h, 2 + h, 4 + h, 6 + h, slots
+    // 8h+4..8h+7 their low parts, so the four minima appear once against each.
+    __device__ __forceinline__ half8v open() {
+        const uint4v w = head;
+        const half2v dm = __builtin_bit_cast(half2v, w.x);
+        d = (float)dm.x * 16384.0f; low = (float)dm.y;
+        const uint32_t s03 = w.y & 0x3F3F3F3Fu, s47 = (w.w & 0x0F0F0F0Fu) | ((w.y >> 2) & 0x30303030u);
+        const uint32_t m03 = w.z & 0x3F3F3F3Fu, m47 = ((w.w >> 4) & 0x0F0F0F0Fu) | ((w.z >> 2) & 0x30303030u);
+        const uint32_t bias = 0x64646464u;   // a byte under the exponent byte 0x64 is 1024 + byte
+        const half2v k = {(half_t)1024.0f, (half_t)1024.0f}, up = {(half_t)1024.0f, (half_t)64.0f};
+        scale[0] = (__builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, s03, 0x04010400u)) - k) * up;
+        scale[1] = (__builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, s03, 0x04030402u)) - k) * up;
+        scale[2] = (__builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, s47, 0x04010400u)) - k) * up;
+        scale[3] = (__builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, s47, 0x04030402u)) - k) * up;
+        const uint32_t mine = __builtin_amdgcn_perm(m47, m03, pf_lane() >> 5 ? 0x07050301u : 0x06040200u);
+        const half2v a = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, mine, 0x04010400u)) - k;
+        const half2v b = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, mine, 0x04030402u)) - k;
+        return half8v{a.x, a.y, b.x, b.y, a.x, a.y, b.x, b.y};
+    }
+    __device__ __forceinline__ half8v operand(int i, const lds_byte *) const {
+        const int j = i >> 2, t = i & 3;
+        const half_t f = t < 2 ? scale[j].x : scale[j].y;
+        const uint32_t mask = t < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
+        return join(q4_scaled_codes(code[j][2 * (t & 1)], mask, half2v{f, f}), q4_scaled_codes(code[j][2 * (t & 1) + 1], mask, half2v{f, f}));
+    }
+};
+// IQ2_XXS (src/qwen4_packed.c:95-121): a weight is d / 8 * (2 s + 1) * magnitude * sign with a 4-bit s per 32-group, magnitudes 8,
+// 25 or 43 from the grid and d per 256-block, so (2 s + 1) * magnitude <= 1333 is an exact fp16 operand: a magnitude byte under the
+// exponent byte 0x64 reads as 1024 + m, (1024 + m) * (2 s + 1) - 1024 * (2 s + 1) = m * (2 s + 1) in one fused step, and the sign is
+// a bit flip.  A 256-block's result is (d / 8) * P; there are no minima.
+template <> struct GemmBlock<PF_IQ2_XXS> {
+    uint2v code[4];
+    uint16_t head;
+    float d, low;
+    static __device__ __forceinline__ constexpr int chunk(int i) { return i & 3; }
+    static constexpr int chunk_h = 4;
+    static constexpr int requests = 5;
+    __device__ __forceinline__ void request_run(int j, const PfBuffer &b, const GemmRows &r, uint32_t at) {
+        code[j] = __builtin_amdgcn_raw_buffer_load_b64(b, (int)r.lane_at, (int)(at + (uint32_t)j * r.run_step), 0);
+    }
+    __device__ __forceinline__ void request_head(const PfBuffer &b, const GemmRows &r, uint32_t at) {
+        head = __builtin_amdgcn_raw_buffer_load_b16(b, (int)r.head_at, (int)at, 0);
+    }
+    __device__ __forceinline__ void open() { d = (float)__builtin_bit_cast(half_t, head) * 0.125f; }
+    __device__ __forceinline__ half8v operand(int i, const lds_byte *tables) const {
+        const uint2v g = code[i >> 2];
+        const uint32_t f = 2u * (g.y >> 28) + 1u;
+        const half_t sf = (half_t)(int)f, kf = (half_t)(int)(1024u * f);
+        const half2v s2 = {sf, sf}, c = {kf, kf};
+        const uint2v m = *reinterpret_cast<const __attribute__((address_space(3))) uint2v *>(tables + 8u * ((g.x >> (8 * (i & 3))) & 255u));
+        const uint4v flip = *reinterpret_cast<const __attribute__((address_space(3))) uint4v *>(tables + 2048 + 16u * ((g.y >> (7 * (i & 3))) & 127u));
+        const uint32_t bias = 0x64646464u;
+        const half2v p0 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.x, 0x04010400u));
+        const half2v p1 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.x, 0x04030402u));
+        const half2v p2 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.y, 0x04010400u));
+        const half2v p3 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.y, 0x04030402u));
+        const half2v v0 = p0 * s2 - c, v1 = p1 * s2 - c, v2 = p2 * s2 - c, v3 = p3 * s2 - c;
+        const uint4v bits = {__builtin_bit_cast(uint32_t, v0) ^ flip.x, __builtin_bit_cast(uint32_t, v1) ^ flip.y,
+                             __builtin_bit_cast(uint32_t, v2) ^ flip.z, __builtin_bit_cast(uint32_t, v3) ^ flip.w};
+        return __builtin_bit_cast(half8v, bits);
+    }
+};
+
+// What a wave's requests read of its item.
+struct GemmSource {
+    PfBuffer weights, heads, x[2];
+    GemmRows rows;
+    uint32_t a_at[2], sum_at;   // per lane: of the rows it copies, of the group sums of its operand row
+    // Copies columns 64 (wave / 2) .. + 63 of the operand rows 16 (wave % 2) .. + 15.
+    __device__ __forceinline__ void request_rows(int wave, int kb, lds_byte *to) const {
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(x[p], to + p * GEMM_PART_BYTES + (2 * wave + i) * GEMM_IMAGE, 16, (int)a_at[i], 512 * kb, 0, 0);
+        asm volatile("" ::: "memory");   // what is requested from here on is younger
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
+
+// One 256-block of a wave's tile.  from, to: the copies of this block's rows (at the lane's) and of the next one's.  at, head_at: the
+// wave's tile in its expert's tensor, at the next block.
+template <int FMT, int PARTS>
+__device__ __forceinline__ void gemm_block(GemmBlock<FMT> &w, half8v &sums, const GemmSource &src, uint32_t at, uint32_t head_at, int next_kb, int wave,
+                                           const lds_byte *__restrict from, lds_byte *__restrict to, const lds_byte *__restrict tables, float16v &acc) {
     const float16v zero = {0};
-    for (int kb = 0; kb < kblocks; kb++) {
-        float16v part0 = zero, part1 = zero, q0 = zero, q1 = zero;
-        float d0 = 0.0f, m0 = 0.0f, d1 = 0.0f, m1 = 0.0f;
-        half2v s2[2][4], c2[2][4];
+    src.request_rows(wave, next_kb, to);
+    if constexpr (FMT == PF_Q4_K) {
+        const float16v q = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, w.open(), zero, 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            stage_barrier();
-            const unsigned char *slot_a = a_lane + slot_off, *slot_w = w_lane + slot_off;
-            slot_off = slot_off + SLOT_BYTES == RING_SLOTS * SLOT_BYTES ? 0 : slot_off + SLOT_BYTES;
-            // every LDS operand of the stage is requested up front (they return in order: the first
-            // product waits for the weight runs and one fragment pair, the rest arrive under way)
-            const uint4 wa0 = *reinterpret_cast<const uint4 *>(slot_w), wb0 = *reinterpret_cast<const uint4 *>(slot_w + 512);
-            const uint4 wa1 = *reinterpret_cast<const uint4 *>(slot_w + 1024), wb1 = *reinterpret_cast<const uint4 *>(slot_w + 1536);
-            half8v ah[4], al[4];
+        for (int r = 0; r < 16; r++) acc[r] = fmaf(-w.low, q[r], acc[r]);
+    } else {
+        w.open();
+    }
+    const float d = w.d;
+    w.request_head(src.heads, src.rows, head_at);
+    if (FMT == PF_Q4_K) sums = __builtin_bit_cast(half8v, __builtin_amdgcn_raw_buffer_load_b128(src.x[0], (int)src.sum_at, 32 * next_kb, 0));
+    float16v part = zero;
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                ah[t] = *reinterpret_cast<const half8v *>(slot_a + 128 * t);
-                al[t] = *reinterpret_cast<const half8v *>(slot_a + A_PART + 128 * t);
+    for (int i = 0; i < 16; i++) {
+        half8v x[PARTS];
+#pragma unroll
+        for (int p = 0; p < PARTS; p++)
+            x[p] = *reinterpret_cast<const __attribute__((address_space(3))) half8v *>(from + p * GEMM_PART_BYTES + (i >> 2) * 4 * GEMM_IMAGE + GemmBlock<FMT>::chunk(i) * 128);
+        const half8v b = w.operand(i, tables);
+#pragma unroll
+        for (int p = 0; p < PARTS; p++) part = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[p], b, part, 0, 0, 0);
+        if ((i & 3) == 3) { w.request_run(i >> 2, src.weights, src.rows, at); __builtin_amdgcn_sched_barrier(0); }
+    }
+    lds_barrier<GemmBlock<FMT>::requests>();   // the next block's rows are there; its weights, requested after them, may not be
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = fmaf(d, part[r], acc[r]);
+}
+
+// The slabs [slab0, slab1) of a row tile.  PARTS = 2: high and low parts of up to 32 rows; 1: both parts of up to 16 rows as one
+// 32-row operand (row 16 + m: the low part of row m).
+template <int MODE, int FMT, int PARTS>
+__device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem &g, int slab0, int slab1, lds_byte *lds) {
+    const int lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, h = lane >> 5;
+    const int K = a.top_k, a_cols = MODE == PF_GEMM_GATE_UP ? a.hidden : g.inter, kblocks = a_cols / 256;
+    // weights: gate tiles of the first four waves, up tiles of the others; a wave beyond the matrix's last rows repeats them
+    const int t = MODE == PF_GEMM_GATE_UP ? (g.shared ? 4 : 1) + (wave >> 2) : g.shared ? 6 : 3;
+    const int last_tile = (MODE == PF_GEMM_GATE_UP ? g.inter : a.hidden) / 32 - 1;
+    auto tile_of = [&](int slab) -> int { return MODE == PF_GEMM_GATE_UP ? 4 * slab + (wave & 3) : GW * slab + wave; };
+    GemmSource src;
+    src.rows = gemm_rows<FMT>(a, t, g.shared ? 0 : (size_t)g.expert);
+    src.weights = pf_buffer(src.rows.base, src.rows.bytes);
+    src.heads = pf_buffer(src.rows.head, src.rows.head_bytes);
+    GemmBlock<FMT> w;
+    {   // the first block's are on their way while the rows are looked up
+        const uint32_t tile = (uint32_t)min(tile_of(slab0), last_tile);
+        w.request_head(src.heads, src.rows, tile * src.rows.head_tile_step);
+#pragma unroll
+        for (int j = 0; j < 4; j++) w.request_run(j, src.weights, src.rows, tile * src.rows.tile_step);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // activation rows: the tile's own rows (down, and the shared expert's tokens) or gathered by token
+    const bool gathered = MODE == PF_GEMM_GATE_UP && !g.shared;
+    const uint32_t a_pitch = 2u * (uint32_t)pf_half_row(a_cols);   // bytes
+    const int row0 = gathered ? 0 : g.shared ? g.m0 : g.first;
+    const uint8_t *base = reinterpret_cast<const uint8_t *>(MODE == PF_GEMM_GATE_UP ? a.x16 : g.shared ? a.sact16 : a.act16) + (size_t)row0 * a_pitch;
+    const uint32_t bytes = gathered ? (uint32_t)min((size_t)a.token_cap * a_pitch, (size_t)PF_NOWHERE) : (uint32_t)g.rows_here * a_pitch;
+    src.x[0] = pf_buffer(base, bytes);
+    src.x[1] = pf_buffer(base + 2 * (size_t)a_cols, PARTS == 2 ? bytes - 2 * (uint32_t)a_cols : 0);
+    const uint32_t mine = gathered ? a.row_to_pair[g.first + min(n, g.rows_here - 1)] / (uint32_t)K : (uint32_t)min(n, g.rows_here - 1);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int v = 16 * (wave & 1) + 8 * i + (lane & 7), m = PARTS == 1 ? v & 15 : v;
+        const uint32_t row = __shfl(mine, m), low = PARTS == 1 && v >= 16 ? 2u * (uint32_t)a_cols : 0u;
+        src.a_at[i] = m < g.rows_here ? row * a_pitch + low + 128u * (uint32_t)(wave >> 1) + 16u * (uint32_t)(lane >> 3) : PF_NOWHERE;
+    }
+    src.sum_at = n < g.rows_here ? mine * a_pitch + 4u * (uint32_t)a_cols + 16u * (uint32_t)h : PF_NOWHERE;
+    const float scale_mine = (MODE == PF_GEMM_GATE_UP ? a.x_scale : g.shared ? a.sact_scale : a.act_scale)[row0 + (int)mine];
+    src.request_rows(wave, 0, lds);
+    half8v sums;
+    if (FMT == PF_Q4_K) sums = __builtin_bit_cast(half8v, __builtin_amdgcn_raw_buffer_load_b128(src.x[0], (int)src.sum_at, 0, 0));
+    lds_barrier<0>();
+    const lds_byte *take = lds + (n >> 3) * GEMM_IMAGE + GemmBlock<FMT>::chunk_h * h * 128 + (n & 7) * 16;
+    float16v acc = {0};
+    int copy = 0, kb = 0, slab = slab0;
+    for (int left = (slab1 - slab0) * kblocks; left; left--) {
+        const bool wraps = kb + 1 == kblocks;
+        const int next_kb = wraps ? 0 : kb + 1;
+        const uint32_t tile = (uint32_t)min(tile_of(wraps ? slab + 1 : slab), last_tile);
+        if (left == 1) { src.weights = pf_buffer(src.rows.base, 0); src.heads = pf_buffer(src.rows.head, 0); }   // no block is left to request
+        gemm_block<FMT, PARTS>(w, sums, src, tile * src.rows.tile_step + (uint32_t)next_kb * src.rows.block_step,
+                               tile * src.rows.head_tile_step + (uint32_t)next_kb * src.rows.head_step, next_kb, wave, take + copy * GEMM_COPY_BYTES,
+                               lds + (copy ^ 1) * GEMM_COPY_BYTES, lds + IQ2_GRID_OFF, acc);
+        copy ^= 1;
+        kb = next_kb;
+        if (!wraps) continue;
+        // epilogue: the lane holds column n of its tile; register r is row 8 (r / 4) + 4 h + r % 4
+        constexpr int REGS = 8 * PARTS;
+        const bool exist = tile_of(slab) <= last_tile;
+        int row_in_4 = 4 * h, col = n;
+        asm volatile("" : "+v"(row_in_4), "+v"(col));   // what follows from them is formed here, not kept in registers through the products
+        float v[REGS];
+#pragma unroll
+        for (int r = 0; r < REGS; r++) v[r] = (PARTS == 1 ? acc[r] + acc[r + 8] : acc[r]) * __shfl(scale_mine, 8 * (r >> 2) + row_in_4 + (r & 3));
+        if (MODE == PF_GEMM_GATE_UP) {   // (one slab) the gate waves hand their rows to the up waves through LDS
+            __attribute__((address_space(3))) float *meet = reinterpret_cast<__attribute__((address_space(3))) float *>(lds) + (wave & 3) * 1024 + lane;
+            if (wave < 4) {
+#pragma unroll
+                for (int r = 0; r < REGS; r++) meet[64 * r] = pf_silu(v[r]);
             }
-            if (j == 0) {
-                const unsigned char *block = ring + block_parity * BLOCK_BYTES;
-                block_parity ^= 1;
-                const uint4 hdr0 = *reinterpret_cast<const uint4 *>(block + HDR_OFF + (2 * wave) * 512 + n * 16);
-                const uint4 hdr1 = *reinterpret_cast<const uint4 *>(block + HDR_OFF + (2 * wave + 1) * 512 + n * 16);
-                const half8v as = *reinterpret_cast<const half8v *>(block + SUMS_OFF + lane * 16);
-                asm volatile("" ::: "memory");   // the requests stay above the arithmetic
-                // the hardware conversion is exact for every binary16 value, subnormals included
-                const half2v dm0 = __builtin_bit_cast(half2v, hdr0.x), dm1 = __builtin_bit_cast(half2v, hdr1.x);
-                d0 = (float)dm0.x; m0 = (float)dm0.y; d1 = (float)dm1.x; m1 = (float)dm1.y;
-                half_t min0[4], min1[4];
+            lds_barrier<0>();
+            if (wave < 4 || !exist) return;
+            float *out = (g.shared ? a.shared_act + (size_t)g.m0 * g.inter : a.act + (size_t)g.first * g.inter) + 32 * tile_of(slab) + col;
 #pragma unroll
-                for (int jj = 0; jj < 4; jj++) {
-                    uint32_t sc, mn;
-                    q4_scale_min(hdr0, jj, h, sc, mn);
-                    min0[jj] = (half_t)(int)mn;
-                    const half_t s0 = (half_t)(int)sc * unit, k0 = (half_t)(int)(sc << bias_shift);
-                    s2[0][jj] = half2v{s0, s0};
-                    c2[0][jj] = half2v{k0, k0};
-                    q4_scale_min(hdr1, jj, h, sc, mn);
-                    min1[jj] = (half_t)(int)mn;
-                    const half_t s1 = (half_t)(int)sc * unit, k1 = (half_t)(int)(sc << bias_shift);
-                    s2[1][jj] = half2v{s1, s1};
-                    c2[1][jj] = half2v{k1, k1};
-                }
-                // Q: K slots 8h..8h+3 hold the high parts of the sums of the lane's four groups,
-                // 8h+4..8h+7 the low parts; the four minima appear once against each
-                const half8v mv0 = {min0[0], min0[1], min0[2], min0[3], min0[0], min0[1], min0[2], min0[3]};
-                const half8v mv1 = {min1[0], min1[1], min1[2], min1[3], min1[0], min1[1], min1[2], min1[3]};
-                q0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(as, mv0, zero, 0, 0, 0);
-                q1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(as, mv1, zero, 0, 0, 0);
+            for (int r = 0; r < REGS; r++) {
+                const int m = 8 * (r >> 2) + row_in_4 + (r & 3);
+                if (m < g.rows_here) out[(size_t)m * g.inter] = meet[64 * r] * v[r];
             }
-            asm volatile("" ::: "memory");
-            const uint32_t w0[8] = {wa0.x, wa0.y, wa0.z, wa0.w, wb0.x, wb0.y, wb0.z, wb0.w};
-            const uint32_t w1[8] = {wa1.x, wa1.y, wa1.z, wa1.w, wb1.x, wb1.y, wb1.z, wb1.w};
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const half8v b0 = q4_scaled_codes(w0[2 * t], w0[2 * t + 1], mask, s2[0][j], c2[0][j]);
-                const half8v b1 = q4_scaled_codes(w1[2 * t], w1[2 * t + 1], mask, s2[1][j], c2[1][j]);
-                part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t], b0, part0, 0, 0, 0);
-                part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t], b1, part1, 0, 0, 0);
-                part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[t], b0, part0, 0, 0, 0);
-                part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[t], b1, part1, 0, 0, 0);
-            }
-            if (j == 0) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    acc0[r] = fmaf(-m0, q0[r], acc0[r]);
-                    acc1[r] = fmaf(-m1, q1[r], acc1[r]);
-                }
-            }
+            return;
         }
+        float *out = a.down + (size_t)g.first * a.hidden + 32 * tile_of(slab) + col;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            acc0[r] = fmaf(d0, part0[r], acc0[r]);
-            acc1[r] = fmaf(d1, part1[r], acc1[r]);
+        for (int r = 0; r < REGS; r++) {
+            const int m = 8 * (r >> 2) + row_in_4 + (r & 3);
+            if (m < g.rows_here && exist) out[(size_t)m * a.hidden] = v[r];
         }
+        acc = float16v{0};
+        slab++;
     }
 }
 
-// The same for IQ2_XXS tiles (src/qwen4_packed.c:95-121): a weight is d / 8 * (2 s + 1) * magnitude * sign with a
-// 4-bit s per 32-group, magnitudes 8, 25 or 43 from the grid and d per 256-block, so
-// (2 s + 1) * magnitude <= 1333 is an exact fp16 operand: a magnitude byte under the exponent byte
-// 0x64 reads as 1024 + m, (1024 + m) * (2 s + 1) - 1024 * (2 s + 1) = m * (2 s + 1) in one fused step,
-// and the sign is a bit flip.  A 256-block's result is (d / 8) * P.  Lane (n, h) takes group 2 j + h in
-// stage j: step t is its grid entry t (8 weights) with the 7 sign bits t of the group's second word.
-// sidx0 / sidx1 / bpr locate the rows' fp16 block scales (which half of the loaded dword is theirs).
-__device__ __forceinline__ void gemm_compute_iq2(const unsigned char *ring, int kblocks, float16v &acc0, float16v &acc1,
-                                                 int &slot_off, int &block_parity, uint32_t sidx0, uint32_t sidx1, uint32_t bpr,
-                                                 int wave_rows) {
-    const int lane = pf_lane(), wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
-    const unsigned char *a_lane = ring + (n >> 3) * A_GROUP + (4 * h) * 128 + (n & 7) * 16;
-    const unsigned char *w_lane = ring + SLOT_W + wave * 1024 + n * 16 + 8 * h;
-    const uint2 *grid = reinterpret_cast<const uint2 *>(ring + IQ2_GRID_OFF);
-    const uint4 *signs = reinterpret_cast<const uint4 *>(ring + IQ2_SIGN_OFF);
-    // index of this lane's rows' first scale; the loader fetched the dword around scale index + kb
-    const uint32_t row0 = sidx0 + ((uint32_t)wave * wave_rows + n) * bpr, row1 = sidx1 + ((uint32_t)wave * wave_rows + n) * bpr;
-    const float16v zero = {0};
-    for (int kb = 0; kb < kblocks; kb++) {
-        float16v part0 = zero, part1 = zero;
-        float d0 = 0.0f, d1 = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            stage_barrier();
-            const unsigned char *slot_a = a_lane + slot_off, *slot_w = w_lane + slot_off;
-            slot_off = slot_off + SLOT_BYTES == RING_SLOTS * SLOT_BYTES ? 0 : slot_off + SLOT_BYTES;
-            const uint2 g0 = *reinterpret_cast<const uint2 *>(slot_w), g1 = *reinterpret_cast<const uint2 *>(slot_w + 512);
-            half8v ah[4], al[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                ah[t] = *reinterpret_cast<const half8v *>(slot_a + 128 * t);
-                al[t] = *reinterpret_cast<const half8v *>(slot_a + A_PART + 128 * t);
-            }
-            if (j == 0) {
-                const unsigned char *block = ring + block_parity * BLOCK_BYTES;
-                block_parity ^= 1;
-                const uint32_t pair0 = *reinterpret_cast<const uint32_t *>(block + HDR_OFF + wave * 256 + 4 * n);
-                const uint32_t pair1 = *reinterpret_cast<const uint32_t *>(block + HDR_OFF + wave * 256 + 128 + 4 * n);
-                const uint32_t bits0 = ((row0 + (uint32_t)kb) & 1u) ? pair0 >> 16 : pair0 & 0xffffu;
-                const uint32_t bits1 = ((row1 + (uint32_t)kb) & 1u) ? pair1 >> 16 : pair1 & 0xffffu;
-                d0 = (float)__builtin_bit_cast(half_t, (unsigned short)bits0) * 0.125f;
-                d1 = (float)__builtin_bit_cast(half_t, (unsigned short)bits1) * 0.125f;
-            }
-            asm volatile("" ::: "memory");   // the requests stay above the arithmetic
-            const half_t s0 = (half_t)(int)(2u * (g0.y >> 28) + 1u), s1 = (half_t)(int)(2u * (g1.y >> 28) + 1u);
-            const half_t k0 = (half_t)(int)(1024u * (2u * (g0.y >> 28) + 1u)), k1 = (half_t)(int)(1024u * (2u * (g1.y >> 28) + 1u));
-            const half2v s20 = {s0, s0}, s21 = {s1, s1}, c20 = {k0, k0}, c21 = {k1, k1};
-            auto codes = [&](const uint2 &g, int t, half2v s2, half2v c) -> half8v {
-                const uint2 m = grid[(g.x >> (8 * t)) & 255u];
-                const uint4 flip = signs[(g.y >> (7 * t)) & 127u];
-                const uint32_t bias = 0x64646464u;
-                const half2v p0 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.x, 0x04010400u));
-                const half2v p1 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.x, 0x04030402u));
-                const half2v p2 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.y, 0x04010400u));
-                const half2v p3 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, m.y, 0x04030402u));
-                const half2v v0 = p0 * s2 - c, v1 = p1 * s2 - c, v2 = p2 * s2 - c, v3 = p3 * s2 - c;
-                const uint4 bits = {__builtin_bit_cast(uint32_t, v0) ^ flip.x, __builtin_bit_cast(uint32_t, v1) ^ flip.y,
-                                    __builtin_bit_cast(uint32_t, v2) ^ flip.z, __builtin_bit_cast(uint32_t, v3) ^ flip.w};
-                return __builtin_bit_cast(half8v, bits);
-            };
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const half8v b0 = codes(g0, t, s20, c20), b1 = codes(g1, t, s21, c21);
-                part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t], b0, part0, 0, 0, 0);
-                part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t], b1, part1, 0, 0, 0);
-                part0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[t], b0, part0, 0, 0, 0);
-                part1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[t], b1, part1, 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            acc0[r] = fmaf(d0, part0[r], acc0[r]);
-            acc1[r] = fmaf(d1, part1[r], acc1[r]);
+// slabs: workgroups that share a row tile; per: slabs that each of them takes (gate and up: one).
+template <int MODE, int FMT>
+__global__ void __launch_bounds__(64 * GW, 4) pf_k_pf_gemm(PfKernelArgs a, int slabs, int per) {
+    extern __shared__ __align__(16) unsigned char gemm_lds[];
+    GemmItem g;
+    int slab;
+    if (!gemm_item(a, slabs, blockIdx.x, g, slab)) return;
+    if (a.type[MODE == PF_GEMM_GATE_UP ? (g.shared ? 4 : 1) : (g.shared ? 6 : 3)] != (uint32_t)FMT) return;   // the plain kernel's
+    const int width = MODE == PF_GEMM_GATE_UP ? 16 * GW : 32 * GW, all = ((MODE == PF_GEMM_GATE_UP ? g.inter : a.hidden) + width - 1) / width;
+    const int slab0 = slab * per, slab1 = min(slab0 + per, all);
+    if (slab0 >= slab1) return;
+    if (FMT == PF_IQ2_XXS) {
+        // grid magnitudes, and for every 7-bit sign field the fp16 sign bits of its eight weights (the eighth sign makes the number
+        // of negative weights even)
+        if (threadIdx.x < 256) reinterpret_cast<uint64_t *>(gemm_lds + IQ2_GRID_OFF)[threadIdx.x] = a.iq2_grid[threadIdx.x];
+        else if (threadIdx.x < 384) {
+            const uint32_t s7 = threadIdx.x - 256, s8 = s7 | ((__popc(s7) & 1u) << 7);
+            uint4 flip;
+            flip.x = ((s8 >> 0) & 1u) << 15 | ((s8 >> 1) & 1u) << 31;
+            flip.y = ((s8 >> 2) & 1u) << 15 | ((s8 >> 3) & 1u) << 31;
+            flip.z = ((s8 >> 4) & 1u) << 15 | ((s8 >> 5) & 1u) << 31;
+            flip.w = ((s8 >> 6) & 1u) << 15 | ((s8 >> 7) & 1u) << 31;
+            reinterpret_cast<uint4 *>(gemm_lds + IQ2_SIGN_OFF)[s7] = flip;
         }
     }
+    // by the expert's rows, not the tile's: which of them a tile holds differs from run to run, and the two add up in another order
+    lds_byte *lds = (lds_byte *)gemm_lds;
+    if (g.m0 == 0 && g.rows_here <= 16) gemm_tile<MODE, FMT, 1>(a, g, slab0, slab1, lds);
+    else gemm_tile<MODE, FMT, 2>(a, g, slab0, slab1, lds);
 }
 
 // Histogram of the routed pairs.  counts[] is zero on entry: the workspace starts zeroed and
@@ -832,9 +723,10 @@ __global__ void pf_k_pf_count(const uint32_t *ids, int pairs, int E, uint32_t *c
 
 // One workgroup: exclusive scan of counts[E] into offsets[E + 1], and the row tiles: every
 // expert's rows (the shared expert = expert E with all tokens) cut into tiles of 32; tiles[0] =
-// count, tiles[1 + i] = expert | (tile index within the expert) << 16.  Leaves counts[] zero.
+// count, tiles[1 + i] = expert | (tile index within the expert) << 16, items[i] = {expert, first row, rows, first row
+// within the expert}.  Leaves counts[] zero.
 __global__ void __launch_bounds__(256) pf_k_pf_scan_tiles(uint32_t *counts, int E, int tokens, uint32_t *offsets,
-                                                          uint32_t *tiles) {
+                                                          uint32_t *tiles, uint4 *items) {
     __shared__ uint32_t rows_before[256], tiles_before[256];
     const int tid = threadIdx.x, per = (E + 1 + 255) / 256, lo = tid * per, hi = min(E + 1, lo + per);
     uint32_t rows = 0, ntiles = 0;
@@ -867,76 +759,16 @@ __global__ void __launch_bounds__(256) pf_k_pf_scan_tiles(uint32_t *counts, int 
     uint32_t row = rows_before[tid], at = tiles_before[tid];
     for (int e = lo; e < hi; e++) {
         const uint32_t c = e < E ? counts[e] : (uint32_t)tokens, n = (c + 31u) / 32u;
+        for (uint32_t i = 0; i < n; i++) {
+            tiles[1 + at + i] = (uint32_t)e | (i << 16);
+            items[at + i] = make_uint4((uint32_t)e, row + 32u * i, min(32u, c - 32u * i), 32u * i);
+        }
         if (e < E) {
             offsets[e] = row;
             row += c;
             counts[e] = 0;
         }
-        for (uint32_t i = 0; i < n; i++) tiles[1 + at + i] = (uint32_t)e | (i << 16);
         at += n;
-    }
-}
-
-// One workgroup per compute unit; workgroup b takes items b, b + grid, b + 2 grid, ...
-template <int MODE, int FMT>
-__global__ void __launch_bounds__(64 * (NW + NL), 3) pf_k_pf_gemm(PfKernelArgs a, int tokens, int slabs) {
-    extern __shared__ __align__(16) unsigned char ring[];
-    __shared__ float row_scale[4][32];
-    const int lane = pf_lane(), wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
-    const uint32_t items = (a.tiles[0] + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES) * (uint32_t)slabs;
-    if (FMT == PF_IQ2_XXS) {
-        // grid magnitudes, and for every 7-bit sign field the fp16 sign bits of its eight weights
-        // (the eighth sign makes the number of negative weights even)
-        if (threadIdx.x < 256) reinterpret_cast<uint64_t *>(ring + IQ2_GRID_OFF)[threadIdx.x] = a.iq2_grid[threadIdx.x];
-        if (threadIdx.x >= 256 && threadIdx.x < 384) {
-            const uint32_t s7 = threadIdx.x - 256, s8 = s7 | ((__popc(s7) & 1u) << 7);
-            uint4 flip;
-            flip.x = ((s8 >> 0) & 1u) << 15 | ((s8 >> 1) & 1u) << 31;
-            flip.y = ((s8 >> 2) & 1u) << 15 | ((s8 >> 3) & 1u) << 31;
-            flip.z = ((s8 >> 4) & 1u) << 15 | ((s8 >> 5) & 1u) << 31;
-            flip.w = ((s8 >> 6) & 1u) << 15 | ((s8 >> 7) & 1u) << 31;
-            reinterpret_cast<uint4 *>(ring + IQ2_SIGN_OFF)[s7] = flip;
-        }
-        __syncthreads();
-    }
-    if (wave >= NW) {
-        __builtin_amdgcn_s_setprio(3);   // the loaders issue little and everything waits for it
-        if (wave == NW) gemm_loader<MODE, FMT, 0>(a, tokens, slabs, items, ring, row_scale);
-        else if (wave == NW + 1) gemm_loader<MODE, FMT, 1>(a, tokens, slabs, items, ring, row_scale);
-        else gemm_loader<MODE, FMT, 2>(a, tokens, slabs, items, ring, row_scale);
-        return;
-    }
-    GemmTarget g;
-    int slot_off = 0, block_parity = 0, item_index = 0;
-    uint32_t q = blockIdx.x;
-    while (gemm_next_item<MODE, FMT>(a, tokens, slabs, items, q, g)) {
-        float16v acc0 = {0}, acc1 = {0};
-        if (FMT == PF_IQ2_XXS)
-            gemm_compute_iq2(ring, g.kblocks, acc0, acc1, slot_off, block_parity, g.sidx0, g.sidx1, g.bpr, (int)g.wave_rows);
-        else
-            gemm_compute(ring, g.kblocks, acc0, acc1, slot_off, block_parity);
-        // epilogue: the lane holds column n of its tiles; register r is row 8 (r / 4) + 4 h + r % 4
-        const float *scales = row_scale[item_index & 3];
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int m = 8 * (r >> 2) + 4 * h + (r & 3);
-            if (m >= g.rows_here || wave >= g.waves) continue;
-            const float rs = scales[m];
-            if (MODE == PF_GEMM_GATE_UP) {
-                const int unit = 32 * NW * g.slab + 32 * wave + n;
-                const float gate = acc0[r] * rs, up = acc1[r] * rs;
-                const float v = pf_silu(gate) * up;
-                if (g.shared) a.shared_act[(size_t)(g.m0 + m) * g.inter + unit] = v;
-                else a.act[(size_t)(g.first + g.m0 + m) * g.inter + unit] = v;
-            } else {
-                const int r0 = 64 * NW * g.slab + 64 * wave + n;
-                float *out = a.down + (size_t)(g.first + g.m0 + m) * a.hidden;
-                out[r0] = acc0[r] * rs;
-                out[r0 + 32] = acc1[r] * rs;
-            }
-        }
-        item_index++;
-        q += gridDim.x;
     }
 }
 
@@ -1341,31 +1173,30 @@ bool pf_prefill_supported(const PfHipMoeDesc &d) {
         (d.type[3] == PF_Q2_K && d.down_physical % 256))
         return false;
     if (d.top_k > 64 || d.top_k >= d.experts || d.experts >= 65535) return false;
+    if ((size_t)d.hidden * (d.inter > d.shared_inter ? d.inter : d.shared_inter) > PF_NOWHERE || pf_prefill_most_tokens((int)d.hidden) == 0)
+        return false;   // one expert's tensor, one token's row by 32-bit offsets
     return true;
 }
 
 size_t pf_prefill_half_row(int cols) { return pf_half_row(cols); }
+size_t pf_prefill_most_tokens(int hidden) { return PF_NOWHERE / (2 * pf_half_row(hidden)) / 32 * 32; }
 // sum over experts of ceil(rows / 32) <= pairs / 32 + experts, plus the shared expert's tiles
 int pf_prefill_max_tiles(int tokens, int experts, int top_k) {
     return (int)(((size_t)tokens * top_k) / 32 + experts + (tokens + 31) / 32 + 1);
 }
 
+// The tile list's length is only known on the device: a workgroup beyond it ends at once.
 template <int MODE, int FMT>
-static void launch_gemm(const PfKernelArgs &a, int tokens, int slabs, hipStream_t stream) {
+static void launch_gemm(const PfKernelArgs &a, unsigned tile_cap, int width, int cols, hipStream_t stream) {
     const size_t lds = FMT == PF_IQ2_XXS ? GEMM_LDS_IQ2 : GEMM_LDS;
-    static bool configured = false;   // once per instantiation: more than the default 64 KB of dynamic LDS
-    static int grid = 0;
-    if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_gemm<MODE, FMT>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        int device = 0, units = 0;
-        (void)hipGetDevice(&device);
-        (void)hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device);
-        grid = units >= 8 ? units / 8 * 8 : 8;   // one workgroup per compute unit (its LDS), a multiple of the XCD count
-        configured = true;
-    }
-    // the item count is only known on the device: every workgroup walks the list from its own index
-    hipLaunchKernelGGL((pf_k_pf_gemm<MODE, FMT>), dim3(grid), dim3(64 * (NW + NL)), lds, stream, a, tokens, slabs);
+    static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_gemm<MODE, FMT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int)lds) == hipSuccess;   // more than the default 64 KB
+    (void)configured;
+    const int rows = MODE == PF_GEMM_GATE_UP ? 16 * GW : 32 * GW, all = (width + rows - 1) / rows;
+    const int per = MODE == PF_GEMM_GATE_UP ? 1 : max(1, min(all, 8 / max(1, cols / 256)));
+    const int slabs = (all + per - 1) / per;
+    const unsigned tiles = (tile_cap + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES);
+    hipLaunchKernelGGL((pf_k_pf_gemm<MODE, FMT>), dim3(tiles * slabs), dim3(64 * GW), lds, stream, a, slabs, per);
 }
 
 template <int MODE>
@@ -1384,7 +1215,8 @@ void pf_launch_group(const PfKernelArgs &a, const uint32_t *ids, int tokens, hip
     const int E = a.experts, P = tokens * a.top_k;
     if (pf_launch_group_fused(ids, P, E, tokens, a.offsets, a.tiles, const_cast<uint32_t *>(a.items), a.pair_to_row, a.row_to_pair, stream)) return;
     hipLaunchKernelGGL(pf_k_pf_count, dim3((P + 255) / 256), dim3(256), 0, stream, ids, P, E, a.counts);
-    hipLaunchKernelGGL(pf_k_pf_scan_tiles, dim3(1), dim3(256), 0, stream, a.counts, E, tokens, a.offsets, a.tiles);
+    hipLaunchKernelGGL(pf_k_pf_scan_tiles, dim3(1), dim3(256), 0, stream, a.counts, E, tokens, a.offsets, a.tiles,
+                       reinterpret_cast<uint4 *>(const_cast<uint32_t *>(a.items)));
     pf_launch_group_place(ids, P, E, a.offsets, a.pair_to_row, a.row_to_pair, stream);
 }
 void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream) {
@@ -1418,8 +1250,8 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     const bool iq2 = a.type[1] == PF_IQ2_XXS;
     const uint32_t ring_fmt = a.type[1];
     const unsigned tile_cap = (unsigned)pf_prefill_max_tiles(tokens, E, K);
-    if (iq2) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS>(a, tokens, (gi + 32 * NW - 1) / (32 * NW), stream);
-    else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K>(a, tokens, (gi + 32 * NW - 1) / (32 * NW), stream);
+    if (iq2) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS>(a, tile_cap, gi, H, stream);
+    else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K>(a, tile_cap, gi, H, stream);
     // only the shared expert's tiles (tokens / 32 of them) are left for this launch: columns split over the waves
     if (a.type[4] != ring_fmt) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, stream);
     const int widest = I > Is ? I : Is;
@@ -1435,8 +1267,8 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     if (last < 4) return;
     // stage 4: down and combine
     if (a.type[3] == ring_fmt || a.type[6] == ring_fmt) {
-        if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS>(a, tokens, (H + 64 * NW - 1) / (64 * NW), stream);
-        else launch_gemm<PF_GEMM_DOWN, PF_Q4_K>(a, tokens, (H + 64 * NW - 1) / (64 * NW), stream);
+        if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS>(a, tile_cap, H, gi, stream);
+        else launch_gemm<PF_GEMM_DOWN, PF_Q4_K>(a, tile_cap, H, gi, stream);
     }
     if (a.type[3] != ring_fmt || a.type[6] != ring_fmt) launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, tile_cap, (H + 255) / 256, 0, stream);
     pf_launch_combine(a, tokens, stream);
