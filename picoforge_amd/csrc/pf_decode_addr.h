@@ -155,6 +155,12 @@ PF_HD size_t pf_i2t_chunk_at(size_t expert_bytes, size_t e, int row_tile, int kb
 PF_HD size_t pf_i2t_scale_at(int row_in_tile) { return 2048 + 2 * (size_t)row_in_tile; }
 PF_HD size_t pf_i2t_piece_at(int run, int row_in_tile) { return (size_t)run * 512 + 16 * (size_t)row_in_tile; }
 
+// ---- tile-ordered MXFP4 (the routed down projection, for the grouped product; 32 rows x one unit of 128 weights = 2176 bytes:
+// the rows' 16-byte blocks, block by block, then the rows' four scale bytes each) ----
+PF_HD size_t pf_mxt_expert_bytes(int n_out, int units) { return (size_t)(n_out / 32) * units * PF_I2T_CHUNK; }
+PF_HD size_t pf_mxt_piece_at(int block, int row_in_tile) { return (size_t)block * 512 + 16 * (size_t)row_in_tile; }
+PF_HD size_t pf_mxt_scales_at(int row_in_tile) { return 2048 + 4 * (size_t)row_in_tile; }
+
 // ---- tile-ordered Q8_0 (the shared expert of the checkpoint profiles; 32 rows x one 64-weight run = 2176 bytes: the
 // rows' 64 code bytes as four 16-byte pieces, piece by piece, then the rows' two half scales each, then padding) ----
 PF_HD size_t pf_q8t_expert_bytes(int n_out, int runs) { return (size_t)(n_out / 32) * runs * PF_I2T_CHUNK; }

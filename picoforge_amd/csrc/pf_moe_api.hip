@@ -265,6 +265,14 @@ extern "C" int pf_hip_moe_create(const PfHipMoeDesc *desc, const void *const hos
                     m->total_bytes += m->bytes[a];
                 }
             }
+            if (e == hipSuccess && pf_mx_down_takes(*desc)) {   // its block-scaled product reads whole lines of this copy
+                const size_t bytes = pf_mxt_expert_bytes((int)n_out[3], m->blocks_per_row[3] / 4) * experts[3];
+                e = hipMalloc((void **)&m->w_mxtile, bytes);
+                if (e == hipSuccess) {
+                    pf_launch_mx_tile(m->w[3], m->w[3] + m->scale_offset[3], m->w_mxtile, (size_t)n_out[3] * experts[3], m->blocks_per_row[3], nullptr);
+                    m->total_bytes += bytes;
+                }
+            }
             if (e == hipSuccess) e = hipDeviceSynchronize();
             if (e != hipSuccess) {
                 pf_set_error("tile-ordered weights", e);
@@ -393,6 +401,7 @@ extern "C" void pf_hip_moe_destroy(PfHipMoe *m) {
     for (int a = 0; a < 8; a++) if (m->w_tiled[a]) (void)hipFree(m->w_tiled[a]);
     for (int a = 0; a < 8; a++) if (m->w_itile[a]) (void)hipFree(m->w_itile[a]);
     for (int a = 0; a < 8; a++) if (m->w_qtile[a]) (void)hipFree(m->w_qtile[a]);
+    if (m->w_mxtile) (void)hipFree(m->w_mxtile);
     free(m);
 }
 
@@ -812,6 +821,7 @@ static PfKernelArgs make_args(const PfHipMoe *m, PfHipWork *w, const float *d_x,
     a.token_cap = (uint32_t)w->cap;
     a.router_t = m->router_t;
     for (int j = 0; j < 8; j++) { a.wt[j] = m->w_tiled[j]; a.wi[j] = m->w_itile[j]; a.wq[j] = m->w_qtile[j]; }
+    a.wm = m->w_mxtile;
     return a;
 }
 

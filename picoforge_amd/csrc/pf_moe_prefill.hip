@@ -23,14 +23,12 @@
 #include "pf_moe_internal.h"
 #include "pf_upload_addr.h"
 #include "pf_plain_walk.h"
+#include "pf_grouped.h"
+#include "pf_mx_rows.h"
 
-typedef _Float16 half_t;
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
-typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 
 // halfs per row of a converted matrix: high parts, low parts, per 256-block the 16 group-sum halfs
 // [even groups: 4 high, 4 low][odd groups: 4 high, 4 low]
@@ -197,12 +195,15 @@ __device__ __forceinline__ void rows_to_half_short(size_t block, const float *sr
 }
 
 // Two matrices of such rows in one launch (the routed and the shared activation rows): workgroups [0, blocks_a) take
-// the first, the others the second.
-template <int PARTS>
+// the first, the others the second.  DIGITS: the first as the digit rows of pf_moe_mx.hip (of at most 1024 values).
+template <int PARTS, bool DIGITS>
 __global__ void __launch_bounds__(256) pf_k_rows_to_half_short2(const float *src_a, int cols_a, size_t rows_a, half_t *dst_a, float *scale_a,
                                                                 unsigned blocks_a, const float *src_b, int cols_b, size_t rows_b,
                                                                 half_t *dst_b, float *scale_b, uint32_t *error_word) {
-    if (blockIdx.x < blocks_a) rows_to_half_short<PARTS>(blockIdx.x, src_a, (size_t)cols_a, cols_a, rows_a, dst_a, scale_a, nullptr, error_word);
+    if (blockIdx.x < blocks_a) {
+        if (DIGITS) pf_rows_to_digits(blockIdx.x, src_a, cols_a, rows_a, reinterpret_cast<uint32_t *>(dst_a), scale_a, error_word);
+        else rows_to_half_short<PARTS>(blockIdx.x, src_a, (size_t)cols_a, cols_a, rows_a, dst_a, scale_a, nullptr, error_word);
+    }
     else rows_to_half_short<PARTS>(blockIdx.x - blocks_a, src_b, (size_t)cols_b, cols_b, rows_b, dst_b, scale_b, nullptr, error_word);
 }
 
@@ -366,47 +367,6 @@ enum { PF_GEMM_GATE_UP = 0, PF_GEMM_DOWN = 1 };
 
 __device__ __forceinline__ void to_lds(const void *global, unsigned char *lds) {
     __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint32_t *>(global), reinterpret_cast<uint32_t *>(lds), 16, 0, 0);
-}
-
-// Barrier between the uses of an LDS copy: the wave's own LDS accesses are over, of its loads from memory the youngest LATER may
-// still be on their way.
-template <int LATER> __device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((LATER & 15) | (LATER >> 4) << 14 | 0x70);   // vmcnt(LATER) lgkmcnt(0), in a form that the compiler counts with
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-// A buffer whose reads beyond `bytes` give zero and cost no memory access.
-typedef __amdgpu_buffer_rsrc_t PfBuffer;
-typedef __attribute__((address_space(3))) unsigned char lds_byte;
-__device__ __forceinline__ PfBuffer pf_buffer(const void *base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-#define PF_NOWHERE 0xC0000000u   // an offset beyond every buffer: none is larger
-
-struct GemmItem {   // a 32-row tile of an expert
-    bool shared;
-    int expert, first, m0, rows_here;   // first row of the tile in expert order and within the expert, rows in it
-    int inter;
-};
-
-// Work item q -> (row tile, slab group).  Workgroups go to the eight XCDs round robin by index.  The tile list is cut into groups of
-// GEMM_XCD_TILES consecutive tiles and the groups dealt to the XCDs in turn; the items of a group (its tiles' slabs) get numbers
-// eight apart: neighbouring workgroups of one XCD, one L2, at the same time.  The slabs of a row tile read the same
-// activation rows, and the row tiles of one expert, neighbours in the list, the same weights: fetched once from memory where
-// they fall into one group.  False: nothing to do for q.
-#define GEMM_XCD_TILES 8
-__device__ __forceinline__ bool gemm_item(const PfKernelArgs &a, int slabs, uint32_t q, GemmItem &g, int &slab) {
-    const uint32_t xcd = q % 8, turn = q / 8, r = turn / slabs;
-    const uint32_t tile = GEMM_XCD_TILES * ((r / GEMM_XCD_TILES) * 8 + xcd) + r % GEMM_XCD_TILES;
-    if (tile >= a.tiles[0]) return false;
-    const uint4 item = reinterpret_cast<const uint4 *>(a.items)[tile];
-    slab = turn % slabs;
-    g.expert = (int)item.x; g.first = (int)item.y; g.rows_here = (int)item.z; g.m0 = (int)item.w;
-    g.shared = g.expert == a.experts;
-    g.inter = g.shared ? a.shared_inter : a.inter;
-    return true;
 }
 
 // One expert's tensor as a wave reads it: the buffers and what the lanes add to an offset in them.  Tile order keeps a 32-row
@@ -1022,7 +982,7 @@ __device__ __forceinline__ void plain_passes(const PlainTile &a, const PlainRow 
 // partial sums meet in LDS and wave 0 adds them in wave order.  For matrices with few row tiles (the
 // shared expert) that gives four times as many workgroups.
 template <int MODE>
-__global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int tokens, int slabs, int split) {
+__global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int tokens, int slabs, int split, int shared_only) {
     extern __shared__ __align__(16) unsigned char plain_lds[];
     __shared__ uint32_t src_row[32];
     __shared__ float src_scale[32];
@@ -1030,7 +990,7 @@ __global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int to
     const int lane = pf_lane(), wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
     const int E = a.experts, K = a.top_k, P = tokens * K;
     const uint32_t all = a.tiles[0], slab = blockIdx.x % slabs;
-    const uint32_t item_tile = blockIdx.x / slabs + (split ? all - (uint32_t)((tokens + 31) / 32) : 0u);   // the shared expert's tiles are the list's last
+    const uint32_t item_tile = blockIdx.x / slabs + (shared_only ? all - (uint32_t)((tokens + 31) / 32) : 0u);   // the shared expert's tiles are the list's last
     if (item_tile >= all) return;
     const uint32_t entry = a.tiles[1 + item_tile];
     const int expert = entry & 0xffffu, m0 = 32 * (int)(entry >> 16);
@@ -1200,14 +1160,14 @@ static void launch_gemm(const PfKernelArgs &a, unsigned tile_cap, int width, int
 }
 
 template <int MODE>
-static void launch_gemm_plain(const PfKernelArgs &a, int tokens, unsigned tile_cap, int slabs, int split, hipStream_t stream) {
+static void launch_gemm_plain(const PfKernelArgs &a, int tokens, unsigned tile_cap, int slabs, int split, bool shared_only, hipStream_t stream) {
     static bool configured = false;   // once per instantiation: more than the default 64 KB of dynamic LDS
     if (!configured) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_gemm_plain<MODE>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, PLAIN_LDS);
         configured = true;
     }
-    hipLaunchKernelGGL(pf_k_pf_gemm_plain<MODE>, dim3(tile_cap * slabs), dim3(256), PLAIN_LDS, stream, a, tokens, slabs, split);
+    hipLaunchKernelGGL(pf_k_pf_gemm_plain<MODE>, dim3(tile_cap * slabs), dim3(256), PLAIN_LDS, stream, a, tokens, slabs, split, (int)shared_only);
 }
 
 // the pairs by expert: offsets, row tiles, pair <-> row
@@ -1253,11 +1213,13 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     if (iq2) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS>(a, tile_cap, gi, H, stream);
     else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K>(a, tile_cap, gi, H, stream);
     // only the shared expert's tiles (tokens / 32 of them) are left for this launch: columns split over the waves
-    if (a.type[4] != ring_fmt) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, stream);
+    if (a.type[4] != ring_fmt) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, true, stream);
     const int widest = I > Is ? I : Is;
+    const bool digits = a.wm && widest <= 1024;   // the routed rows as digits
     if (widest <= 1024 && P > 0 && tokens > 0) {
-        const unsigned blocks_a = (unsigned)((P + 3) / 4), blocks_b = (unsigned)((tokens + 3) / 4);
-        hipLaunchKernelGGL(widest <= 512 ? pf_k_rows_to_half_short2<1> : pf_k_rows_to_half_short2<2>, dim3(blocks_a + blocks_b), dim3(256), 0,
+        const unsigned rows_a = digits ? 4u * pf_mx_rows_a_wave(I) : 4u, blocks_a = ((unsigned)P + rows_a - 1) / rows_a, blocks_b = (unsigned)((tokens + 3) / 4);
+        hipLaunchKernelGGL(digits ? (widest <= 512 ? pf_k_rows_to_half_short2<1, true> : pf_k_rows_to_half_short2<2, true>)
+                                  : (widest <= 512 ? pf_k_rows_to_half_short2<1, false> : pf_k_rows_to_half_short2<2, false>), dim3(blocks_a + blocks_b), dim3(256), 0,
                            stream, a.act, I, (size_t)P, (half_t *)a.act16, a.act_scale, blocks_a, a.shared_act, Is, (size_t)tokens,
                            (half_t *)a.sact16, a.sact_scale, a.error_word);
     } else {
@@ -1270,6 +1232,8 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
         if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS>(a, tile_cap, H, gi, stream);
         else launch_gemm<PF_GEMM_DOWN, PF_Q4_K>(a, tile_cap, H, gi, stream);
     }
-    if (a.type[3] != ring_fmt || a.type[6] != ring_fmt) launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, tile_cap, (H + 255) / 256, 0, stream);
+    if (digits) pf_launch_mx_down(a, tile_cap, stream);
+    if (digits ? a.type[6] != ring_fmt : a.type[3] != ring_fmt || a.type[6] != ring_fmt)
+        launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, digits ? (unsigned)((tokens + 31) / 32) : tile_cap, (H + 255) / 256, 0, digits, stream);
     pf_launch_combine(a, tokens, stream);
 }

@@ -1,6 +1,6 @@
 // What one thread of an upload kernel moves, as functions that compile for the host as well: the kernels that lay a
 // layer's tensors out in device memory (the scale/payload split of IQ2_XXS, Q8_0 and MXFP4, the tile orders of Q4_K,
-// IQ2_XXS and Q8_0) call them for their addresses, and a host-side test walks every thread of every launch and checks
+// IQ2_XXS, Q8_0 and MXFP4) call them for their addresses, and a host-side test walks every thread of every launch and checks
 // that each read ends inside the source buffer and each write inside the destination allocation.
 #pragma once
 #include "pf_decode_addr.h"
@@ -109,6 +109,29 @@ PF_HD PfMove pf_q8_tile_move(size_t i, size_t rows, int blocks_per_row) {
         m.width = 2; m.from = 1;          // two half scales, 2 bytes each, written as one dword
         m.src = 2 * b; m.src2_used = true; m.src2 = 2 * (b + 1);
         m.dst = chunk * PF_I2T_CHUNK + pf_q8t_scales_at(row);
+    }
+    return m;
+}
+
+// ---- MXFP4 into tile order (pf_k_mx_tile): per (32-row tile, unit of four blocks) chunk 128 piece threads and 32 scale threads ----
+PF_HD size_t pf_mx_tile_threads(size_t rows, int blocks_per_row) { return rows / 32 * (size_t)(blocks_per_row / 4) * 160; }
+PF_HD PfMove pf_mx_tile_move(size_t i, size_t rows, int blocks_per_row) {
+    PfMove m = {};
+    const size_t per_chunk = 128 + 32;
+    const int units = blocks_per_row / 4;
+    const size_t chunk = i / per_chunk, tile = chunk / units, unit = chunk % units;
+    if (chunk >= rows / 32 * (size_t)units) return m;
+    const int p = (int)(i % per_chunk), row = p & 31;
+    const size_t block = (32 * tile + row) * blocks_per_row + 4 * unit;   // the row's first of the unit
+    m.active = true;
+    if (p < 128) {
+        m.width = 16; m.from = 0;
+        m.src = 16 * (block + (p >> 5));
+        m.dst = chunk * PF_I2T_CHUNK + pf_mxt_piece_at(p >> 5, row);
+    } else {
+        m.width = 4; m.from = 1;
+        m.src = block;
+        m.dst = chunk * PF_I2T_CHUNK + pf_mxt_scales_at(row);
     }
     return m;
 }

@@ -1,6 +1,6 @@
 // Host-side walk over every thread of every kernel that lays a layer's tensors out in device memory at
 // pf_hip_moe_create (and when a pool stores an expert): the scale/payload split of IQ2_XXS, Q8_0 and MXFP4, the
-// tile orders of Q4_K, IQ2_XXS and Q8_0.  Compiled with g++ by tests/test_upload_addresses.py; includes the
+// tile orders of Q4_K, IQ2_XXS, Q8_0 and MXFP4.  Compiled with g++ by tests/test_upload_addresses.py; includes the
 // header the kernels take their addresses from (picoforge_amd/csrc/pf_upload_addr.h), so what is checked here is
 // what the device executes.  For each tensor of a layer it walks the launch as the library makes it -- every
 // thread of the rounded-up grid -- and checks that each read ends inside the source buffer, each write inside the
@@ -92,6 +92,14 @@ int main(int argc, char **argv) {
             const Buffer tiled = {"tile-ordered IQ2_XXS", bytes, 0, 0, bytes};
             walk("pf_k_iq2_tile", pf_iq2_tile_threads(rows, p.blocks_per_row), [&](size_t i) { return pf_iq2_tile_move(i, rows, p.blocks_per_row); },
                  device, tiled, nullptr);
+        } else if (type[a] == PF_MXFP4 && a == 3 && k_storage[a] % 128 == 0) {
+            const size_t bytes = pf_mxt_expert_bytes((int)n_out[a], p.blocks_per_row / 4) * experts;
+            const Buffer tiled = {"tile-ordered MXFP4", bytes, 0, 0, bytes};
+            std::vector<unsigned char> written(bytes);
+            walk("pf_k_mx_tile", pf_mx_tile_threads(rows, p.blocks_per_row), [&](size_t i) { return pf_mx_tile_move(i, rows, p.blocks_per_row); },
+                 device, tiled, &written);
+            for (size_t b = 0; b < written.size(); b++)
+                if (written[b] != 1) { complain("pf_k_mx_tile", "leaves a byte unwritten", 0, b, 1, bytes); break; }
         } else if (type[a] == PF_Q8_0 && experts == 1 && k_storage[a] % 64 == 0 && (a == 4 || a == 5)) {
             const size_t bytes = pf_q8t_expert_bytes((int)n_out[a], (int)(k_storage[a] / 64));
             const Buffer tiled = {"tile-ordered Q8_0", bytes, 0, 0, bytes};

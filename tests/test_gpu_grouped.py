@@ -31,7 +31,7 @@ def steered(cfg, fmt, seed):
 @pytest.mark.parametrize("h,i,s,physical,fmt", [
     (256, 256, 512, None, abi.GGUF_Q4_K), (768, 512, 256, None, abi.GGUF_Q4_K), (256, 256, 512, None, abi.GGUF_IQ2_XXS),
     (768, 512, 256, None, abi.GGUF_IQ2_XXS), (512, 384, 128, 512, "q2"), (512, 384, 128, None, "q4"), (2560, 640, 640, 768, "q2"),
-    (2560, 640, 640, None, "q4"),
+    (2560, 640, 640, None, "q4"), (256, 128, 128, None, "q4"), (512, 256, 512, None, "q4"), (256, 512, 128, None, "q4"), (256, 768, 128, None, "q4"),
 ])
 def test_row_counts_around_the_tiles(product, oracle, monkeypatch, h, i, s, physical, fmt, copy):
     print(f"case grouped rows {fmt} h={h} i={i} s={s} tile-ordered copies {copy}", flush=True)
