@@ -35,11 +35,11 @@ struct GemmItem {   // a 32-row tile of an expert
 // GEMM_XCD_TILES consecutive tiles and the groups dealt to the XCDs in turn; the items of a group (its tiles' slabs) get numbers
 // eight apart: neighbouring workgroups of one XCD, one L2, at the same time.  The slabs of a row tile read the same
 // activation rows, and the row tiles of one expert, neighbours in the list, the same weights: fetched once from memory where
-// they fall into one group.  False: nothing to do for q.
+// they fall into one group.  skip: tiles left out at the list's start.  False: nothing to do for q.
 #define GEMM_XCD_TILES 8
-__device__ __forceinline__ bool gemm_item(const PfKernelArgs &a, int slabs, uint32_t q, GemmItem &g, int &slab) {
+__device__ __forceinline__ bool gemm_item(const PfKernelArgs &a, int slabs, uint32_t q, GemmItem &g, int &slab, uint32_t skip = 0) {
     const uint32_t xcd = q % 8, turn = q / 8, r = turn / slabs;
-    const uint32_t tile = GEMM_XCD_TILES * ((r / GEMM_XCD_TILES) * 8 + xcd) + r % GEMM_XCD_TILES;
+    const uint32_t tile = GEMM_XCD_TILES * ((r / GEMM_XCD_TILES) * 8 + xcd) + r % GEMM_XCD_TILES + skip;
     if (tile >= a.tiles[0]) return false;
     const uint4 item = reinterpret_cast<const uint4 *>(a.items)[tile];
     slab = turn % slabs;

@@ -376,11 +376,27 @@ struct GemmRows {
     uint32_t bytes, head_bytes;
     uint32_t lane_at, head_at;          // per lane: of its codes, of its row's block header
     uint32_t tile_step, block_step, run_step, head_tile_step, head_step;
+    uint32_t group_step, head_run_step; // Q8_0: between the two groups of a run, between the runs' scale pairs
 };
 template <int FMT> __device__ __forceinline__ GemmRows gemm_rows(const PfKernelArgs &a, int t, size_t expert) {
     const uint32_t n = pf_lane() & 31, h = pf_lane() >> 5, row_bytes = (uint32_t)a.row_bytes[t], blocks = (uint32_t)a.blocks_per_row[t];
-    const bool tiled = FMT == PF_IQ2_XXS ? a.wi[t] != nullptr : a.wt[t] != nullptr;
+    const bool tiled = FMT == PF_IQ2_XXS ? a.wi[t] != nullptr : FMT == PF_Q8_0 ? a.wq[t] != nullptr : a.wt[t] != nullptr;
     GemmRows r;
+    if (FMT == PF_Q8_0 && tiled) {   // (a tensor of one expert)
+        r.bytes = (uint32_t)pf_q8t_expert_bytes(a.n_out[t], (int)blocks / 2);
+        r.base = a.wq[t];
+        r.lane_at = 512 * h + 16 * n; r.head_at = 2048 + 4 * n;
+        r.group_step = 1024; r.run_step = r.head_run_step = PF_I2T_CHUNK; r.block_step = r.head_step = 4 * PF_I2T_CHUNK;
+        r.tile_step = r.head_tile_step = blocks / 2 * PF_I2T_CHUNK;
+    } else if (FMT == PF_Q8_0) {     // payloads of all experts, then their scales
+        r.bytes = (uint32_t)a.expert_bytes[t]; r.head_bytes = 2 * (uint32_t)a.n_out[t] * blocks;
+        r.base = a.w[t] + expert * r.bytes;
+        r.head = a.w[t] + a.scale_offset[t] + expert * r.head_bytes;
+        r.lane_at = n * row_bytes + 16 * h; r.head_at = 2 * n * blocks;
+        r.group_step = 32; r.run_step = 64; r.head_run_step = 4; r.block_step = 256; r.head_step = 16;
+        r.tile_step = 32 * row_bytes; r.head_tile_step = 64 * blocks;
+        return r;
+    } else
     if (FMT == PF_IQ2_XXS && tiled) {
         r.bytes = (uint32_t)pf_i2t_expert_bytes(a.n_out[t], (int)blocks);
         r.base = a.wi[t] + expert * r.bytes;
@@ -500,6 +516,46 @@ template <> struct GemmBlock<PF_IQ2_XXS> {
     }
 };
 
+// eight bytes as eight halfs, exact: a byte under the exponent byte 0x64 reads as 1024 + byte
+__device__ __forceinline__ half8v half8_of_bytes(uint32_t b0, uint32_t b1, half_t offset) {
+    const uint32_t bias = 0x64646464u;
+    const half2v c = {offset, offset};
+    const half2v v0 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b0, 0x04010400u)) - c;
+    const half2v v1 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b0, 0x04030402u)) - c;
+    const half2v v2 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b1, 0x04010400u)) - c;
+    const half2v v3 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b1, 0x04030402u)) - c;
+    return half8v{v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
+}
+// signed bytes: flip the sign bit, read as unsigned, take 128 more away
+__device__ __forceinline__ half8v half8_of_signed_bytes(uint32_t b0, uint32_t b1) {
+    return half8_of_bytes(b0 ^ 0x80808080u, b1 ^ 0x80808080u, (half_t)1152.0f);
+}
+
+// Q8_0: signed code bytes, a half scale per 32-group: a group's partial sums times its scale.  Lane (n, h) loads bytes 16h..16h+15 of a
+// group; step i is half i % 2 of its bytes in group i / 2 of the block.  Half scales are no integers, so they stay out of the
+// operand.  The shared expert of the checkpoint profiles: its gate and up tiles ride with the routed ones' launch (2048 tokens of 2560 x
+// 640: 411 us, against 377 and 90 for a launch of the plain kernel), its down tiles are a launch of 38 us (plain kernel: 50).
+template <> struct GemmBlock<PF_Q8_0> {
+    uint4v code[8];
+    uint32_t head[4];   // of a run: its two groups' scales
+    static __device__ __forceinline__ constexpr int chunk(int i) { return 4 * ((i & 3) >> 1) + (i & 1); }
+    static constexpr int chunk_h = 2;
+    static constexpr int requests = 12;
+    __device__ __forceinline__ void request_run(int j, const PfBuffer &b, const PfBuffer &heads, const GemmRows &r, uint32_t at, uint32_t head_at) {
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+            code[2 * j + e] = __builtin_amdgcn_raw_buffer_load_b128(b, (int)r.lane_at, (int)(at + (uint32_t)j * r.run_step + (uint32_t)e * r.group_step), 0);
+        head[j] = __builtin_amdgcn_raw_buffer_load_b32(heads, (int)r.head_at, (int)(head_at + (uint32_t)j * r.head_run_step), 0);
+    }
+    __device__ __forceinline__ float scale(int g) const {
+        return (float)__builtin_bit_cast(half_t, (unsigned short)((g & 1) ? head[g >> 1] >> 16 : head[g >> 1] & 0xffffu));
+    }
+    __device__ __forceinline__ half8v operand(int i) const {
+        const uint4v c = code[i >> 1];
+        return half8_of_signed_bytes(c[2 * (i & 1)], c[2 * (i & 1) + 1]);
+    }
+};
+
 // What a wave's requests read of its item.
 struct GemmSource {
     PfBuffer weights, heads, x[2];
@@ -551,12 +607,45 @@ __device__ __forceinline__ void gemm_block(GemmBlock<FMT> &w, half8v &sums, cons
     for (int r = 0; r < 16; r++) acc[r] = fmaf(d, part[r], acc[r]);
 }
 
+// The same for Q8_0, whose groups are added up one by one, the even and the odd ones apart (a row of sums half as long); groups: 8, or 4 in the last block of a row of an odd number of 128 columns.
+template <int PARTS>
+__device__ __forceinline__ void gemm_block_q8(GemmBlock<PF_Q8_0> &w, const GemmSource &src, uint32_t at, uint32_t head_at, int next_kb, int groups, int wave,
+                                              const lds_byte *__restrict from, lds_byte *__restrict to, float16v (&acc)[2]) {
+    const float16v zero = {0};
+    src.request_rows(wave, next_kb, to);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (2 * j < groups) {   // (uniform)
+#pragma unroll
+            for (int g = 2 * j; g < 2 * j + 2; g++) {
+                float16v part = zero;
+#pragma unroll
+                for (int i = 2 * g; i < 2 * g + 2; i++) {
+                    const half8v b = w.operand(i);
+#pragma unroll
+                    for (int p = 0; p < PARTS; p++) {
+                        const half8v x = *reinterpret_cast<const __attribute__((address_space(3))) half8v *>(from + p * GEMM_PART_BYTES + j * 4 * GEMM_IMAGE +
+                                                                                                             GemmBlock<PF_Q8_0>::chunk(i) * 128);
+                        part = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, b, part, 0, 0, 0);
+                    }
+                }
+                const float d = w.scale(g);
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[g & 1][r] = fmaf(d, part[r], acc[g & 1][r]);
+            }
+        }
+        w.request_run(j, src.weights, src.heads, src.rows, at, head_at);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier<GemmBlock<PF_Q8_0>::requests>();
+}
+
 // The slabs [slab0, slab1) of a row tile.  PARTS = 2: high and low parts of up to 32 rows; 1: both parts of up to 16 rows as one
 // 32-row operand (row 16 + m: the low part of row m).
 template <int MODE, int FMT, int PARTS>
 __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem &g, int slab0, int slab1, lds_byte *lds) {
     const int lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, h = lane >> 5;
-    const int K = a.top_k, a_cols = MODE == PF_GEMM_GATE_UP ? a.hidden : g.inter, kblocks = a_cols / 256;
+    const int K = a.top_k, a_cols = MODE == PF_GEMM_GATE_UP ? a.hidden : g.inter, kblocks = (a_cols + 255) / 256;
     // weights: gate tiles of the first four waves, up tiles of the others; a wave beyond the matrix's last rows repeats them
     const int t = MODE == PF_GEMM_GATE_UP ? (g.shared ? 4 : 1) + (wave >> 2) : g.shared ? 6 : 3;
     const int last_tile = (MODE == PF_GEMM_GATE_UP ? g.inter : a.hidden) / 32 - 1;
@@ -568,9 +657,14 @@ __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem 
     GemmBlock<FMT> w;
     {   // the first block's are on their way while the rows are looked up
         const uint32_t tile = (uint32_t)min(tile_of(slab0), last_tile);
-        w.request_head(src.heads, src.rows, tile * src.rows.head_tile_step);
+        if constexpr (FMT == PF_Q8_0) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) w.request_run(j, src.weights, src.rows, tile * src.rows.tile_step);
+            for (int j = 0; j < 4; j++) w.request_run(j, src.weights, src.heads, src.rows, tile * src.rows.tile_step, tile * src.rows.head_tile_step);
+        } else {
+            w.request_head(src.heads, src.rows, tile * src.rows.head_tile_step);
+#pragma unroll
+            for (int j = 0; j < 4; j++) w.request_run(j, src.weights, src.rows, tile * src.rows.tile_step);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
     // activation rows: the tile's own rows (down, and the shared expert's tokens) or gathered by token
@@ -595,21 +689,28 @@ __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem 
     if (FMT == PF_Q4_K) sums = __builtin_bit_cast(half8v, __builtin_amdgcn_raw_buffer_load_b128(src.x[0], (int)src.sum_at, 0, 0));
     lds_barrier<0>();
     const lds_byte *take = lds + (n >> 3) * GEMM_IMAGE + GemmBlock<FMT>::chunk_h * h * 128 + (n & 7) * 16;
-    float16v acc = {0};
+    float16v acc = {0}, apart[2] = {{0}, {0}};
     int copy = 0, kb = 0, slab = slab0;
     for (int left = (slab1 - slab0) * kblocks; left; left--) {
         const bool wraps = kb + 1 == kblocks;
         const int next_kb = wraps ? 0 : kb + 1;
         const uint32_t tile = (uint32_t)min(tile_of(wraps ? slab + 1 : slab), last_tile);
         if (left == 1) { src.weights = pf_buffer(src.rows.base, 0); src.heads = pf_buffer(src.rows.head, 0); }   // no block is left to request
-        gemm_block<FMT, PARTS>(w, sums, src, tile * src.rows.tile_step + (uint32_t)next_kb * src.rows.block_step,
-                               tile * src.rows.head_tile_step + (uint32_t)next_kb * src.rows.head_step, next_kb, wave, take + copy * GEMM_COPY_BYTES,
-                               lds + (copy ^ 1) * GEMM_COPY_BYTES, lds + IQ2_GRID_OFF, acc);
+        const uint32_t at = tile * src.rows.tile_step + (uint32_t)next_kb * src.rows.block_step;
+        const uint32_t head_at = tile * src.rows.head_tile_step + (uint32_t)next_kb * src.rows.head_step;
+        const lds_byte *from = take + copy * GEMM_COPY_BYTES;
+        lds_byte *to = lds + (copy ^ 1) * GEMM_COPY_BYTES;
+        if constexpr (FMT == PF_Q8_0) gemm_block_q8<PARTS>(w, src, at, head_at, next_kb, min(8, (a_cols - 256 * kb) / 32), wave, from, to, apart);
+        else gemm_block<FMT, PARTS>(w, sums, src, at, head_at, next_kb, wave, from, to, lds + IQ2_GRID_OFF, acc);
         copy ^= 1;
         kb = next_kb;
         if (!wraps) continue;
         // epilogue: the lane holds column n of its tile; register r is row 8 (r / 4) + 4 h + r % 4
         constexpr int REGS = 8 * PARTS;
+        if (FMT == PF_Q8_0) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) { acc[r] = apart[0][r] + apart[1][r]; apart[0][r] = apart[1][r] = 0.0f; }
+        }
         const bool exist = tile_of(slab) <= last_tile;
         int row_in_4 = 4 * h, col = n;
         asm volatile("" : "+v"(row_in_4), "+v"(col));   // what follows from them is formed here, not kept in registers through the products
@@ -643,18 +744,19 @@ __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem 
     }
 }
 
-// slabs: workgroups that share a row tile; per: slabs that each of them takes (gate and up: one).
-template <int MODE, int FMT>
-__global__ void __launch_bounds__(64 * GW, 4) pf_k_pf_gemm(PfKernelArgs a, int slabs, int per) {
+// FMT, SHARED: the routed tensors' format and the shared expert's.  slabs: workgroups that share a row tile; per: slabs that each of
+// them takes (gate and up: one); skip_routed: only the shared expert's tiles, the list's last, of this many tokens (0: all).
+template <int MODE, int FMT, int SHARED>
+__global__ void __launch_bounds__(64 * GW, 4) pf_k_pf_gemm(PfKernelArgs a, int slabs, int per, int skip_routed) {
     extern __shared__ __align__(16) unsigned char gemm_lds[];
     GemmItem g;
     int slab;
-    if (!gemm_item(a, slabs, blockIdx.x, g, slab)) return;
-    if (a.type[MODE == PF_GEMM_GATE_UP ? (g.shared ? 4 : 1) : (g.shared ? 6 : 3)] != (uint32_t)FMT) return;   // the plain kernel's
+    if (!gemm_item(a, slabs, blockIdx.x, g, slab, skip_routed ? a.tiles[0] - (uint32_t)(skip_routed + 31) / 32 : 0)) return;
+    if (a.type[MODE == PF_GEMM_GATE_UP ? (g.shared ? 4 : 1) : (g.shared ? 6 : 3)] != (uint32_t)(g.shared ? SHARED : FMT)) return;   // the plain kernel's
     const int width = MODE == PF_GEMM_GATE_UP ? 16 * GW : 32 * GW, all = ((MODE == PF_GEMM_GATE_UP ? g.inter : a.hidden) + width - 1) / width;
     const int slab0 = slab * per, slab1 = min(slab0 + per, all);
     if (slab0 >= slab1) return;
-    if (FMT == PF_IQ2_XXS) {
+    if (FMT == PF_IQ2_XXS && (SHARED == FMT || !g.shared)) {
         // grid magnitudes, and for every 7-bit sign field the fp16 sign bits of its eight weights (the eighth sign makes the number
         // of negative weights even)
         if (threadIdx.x < 256) reinterpret_cast<uint64_t *>(gemm_lds + IQ2_GRID_OFF)[threadIdx.x] = a.iq2_grid[threadIdx.x];
@@ -670,7 +772,13 @@ __global__ void __launch_bounds__(64 * GW, 4) pf_k_pf_gemm(PfKernelArgs a, int s
     }
     // by the expert's rows, not the tile's: which of them a tile holds differs from run to run, and the two add up in another order
     lds_byte *lds = (lds_byte *)gemm_lds;
-    if (g.m0 == 0 && g.rows_here <= 16) gemm_tile<MODE, FMT, 1>(a, g, slab0, slab1, lds);
+    const bool narrow = g.m0 == 0 && g.rows_here <= 16;
+    if (SHARED != FMT && g.shared) {
+        if (narrow) gemm_tile<MODE, SHARED, 1>(a, g, slab0, slab1, lds);
+        else gemm_tile<MODE, SHARED, 2>(a, g, slab0, slab1, lds);
+        return;
+    }
+    if (narrow) gemm_tile<MODE, FMT, 1>(a, g, slab0, slab1, lds);
     else gemm_tile<MODE, FMT, 2>(a, g, slab0, slab1, lds);
 }
 
@@ -743,21 +851,6 @@ __global__ void __launch_bounds__(256) pf_k_pf_scan_tiles(uint32_t *counts, int 
 // multiply the group's partial sums; Q2_K folds its 4-bit scale into the operand (scale * code
 // <= 45) and obtains sum(min * x) from a second product with the minimum as the operand, as
 // d * P - dmin * Q per 256-block.
-
-// eight bytes as eight halfs, exact: a byte under the exponent byte 0x64 reads as 1024 + byte
-__device__ __forceinline__ half8v half8_of_bytes(uint32_t b0, uint32_t b1, half_t offset) {
-    const uint32_t bias = 0x64646464u;
-    const half2v c = {offset, offset};
-    const half2v v0 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b0, 0x04010400u)) - c;
-    const half2v v1 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b0, 0x04030402u)) - c;
-    const half2v v2 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b1, 0x04010400u)) - c;
-    const half2v v3 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b1, 0x04030402u)) - c;
-    return half8v{v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
-}
-// signed bytes: flip the sign bit, read as unsigned, take 128 more away
-__device__ __forceinline__ half8v half8_of_signed_bytes(uint32_t b0, uint32_t b1) {
-    return half8_of_bytes(b0 ^ 0x80808080u, b1 ^ 0x80808080u, (half_t)1152.0f);
-}
 
 // Eight E2M1 codes (one per byte of two dwords, in the low nibble) as halfs holding twice their value:
 // 0, 1, 2, 3, 4, 6, 8, 12 are 0x0000, 0x3C00, 0x4000, 0x4200, 0x4400, 0x4600, 0x4800, 0x4A00, so a byte
@@ -976,13 +1069,16 @@ __device__ __forceinline__ void plain_passes(const PlainTile &a, const PlainRow 
                   [&](int k0, int cols) { plain_product(w, ahi, alo, a.sums + (size_t)n * PLAIN_SUMS, 32 * PLAIN_SUMS, k0, cols, h, acc); });
 }
 
+// which: all items of the list, the shared expert's (the grid: its tiles alone), or the routed experts'.
+enum { PLAIN_ALL, PLAIN_SHARED, PLAIN_ROUTED };
+
 // grid: (row tiles the list can hold) x slabs; 4 waves.  Items whose tensors are in a format of the ring
 // kernel are skipped here, as the ring kernel skips these.
 // split != 0 (gate/up only): the four waves share 32 units and take a quarter of the columns each; their
 // partial sums meet in LDS and wave 0 adds them in wave order.  For matrices with few row tiles (the
 // shared expert) that gives four times as many workgroups.
 template <int MODE>
-__global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int tokens, int slabs, int split, int shared_only) {
+__global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int tokens, int slabs, int split, int which) {
     extern __shared__ __align__(16) unsigned char plain_lds[];
     __shared__ uint32_t src_row[32];
     __shared__ float src_scale[32];
@@ -990,11 +1086,12 @@ __global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int to
     const int lane = pf_lane(), wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
     const int E = a.experts, K = a.top_k, P = tokens * K;
     const uint32_t all = a.tiles[0], slab = blockIdx.x % slabs;
-    const uint32_t item_tile = blockIdx.x / slabs + (shared_only ? all - (uint32_t)((tokens + 31) / 32) : 0u);   // the shared expert's tiles are the list's last
+    const uint32_t item_tile = blockIdx.x / slabs + (which == PLAIN_SHARED ? all - (uint32_t)((tokens + 31) / 32) : 0u);   // the shared expert's tiles are the list's last
     if (item_tile >= all) return;
     const uint32_t entry = a.tiles[1 + item_tile];
     const int expert = entry & 0xffffu, m0 = 32 * (int)(entry >> 16);
     const bool shared = expert == E;
+    if (which == PLAIN_ROUTED && shared) return;
     const int first = shared ? P : (int)a.offsets[expert];
     const int count = shared ? tokens : (int)a.offsets[expert + 1] - first;
     if (count <= m0) return;
@@ -1145,29 +1242,31 @@ int pf_prefill_max_tiles(int tokens, int experts, int top_k) {
     return (int)(((size_t)tokens * top_k) / 32 + experts + (tokens + 31) / 32 + 1);
 }
 
-// The tile list's length is only known on the device: a workgroup beyond it ends at once.
-template <int MODE, int FMT>
-static void launch_gemm(const PfKernelArgs &a, unsigned tile_cap, int width, int cols, hipStream_t stream) {
+// The tile list's length is only known on the device: a workgroup beyond it ends at once.  shared_tokens: the shared expert's tiles only
+// (one slab a workgroup, they are few).
+template <int MODE, int FMT, int SHARED>
+static void launch_gemm(const PfKernelArgs &a, unsigned tile_cap, int width, int cols, int shared_tokens, hipStream_t stream) {
     const size_t lds = FMT == PF_IQ2_XXS ? GEMM_LDS_IQ2 : GEMM_LDS;
-    static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_gemm<MODE, FMT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_gemm<MODE, FMT, SHARED>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        (int)lds) == hipSuccess;   // more than the default 64 KB
     (void)configured;
     const int rows = MODE == PF_GEMM_GATE_UP ? 16 * GW : 32 * GW, all = (width + rows - 1) / rows;
-    const int per = MODE == PF_GEMM_GATE_UP ? 1 : max(1, min(all, 8 / max(1, cols / 256)));
+    const int per = MODE == PF_GEMM_GATE_UP || shared_tokens ? 1 : max(1, min(all, 8 / max(1, cols / 256)));
     const int slabs = (all + per - 1) / per;
+    if (shared_tokens) tile_cap = (unsigned)(shared_tokens + 31) / 32;
     const unsigned tiles = (tile_cap + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES);
-    hipLaunchKernelGGL((pf_k_pf_gemm<MODE, FMT>), dim3(tiles * slabs), dim3(64 * GW), lds, stream, a, slabs, per);
+    hipLaunchKernelGGL((pf_k_pf_gemm<MODE, FMT, SHARED>), dim3(tiles * slabs), dim3(64 * GW), lds, stream, a, slabs, per, shared_tokens);
 }
 
 template <int MODE>
-static void launch_gemm_plain(const PfKernelArgs &a, int tokens, unsigned tile_cap, int slabs, int split, bool shared_only, hipStream_t stream) {
+static void launch_gemm_plain(const PfKernelArgs &a, int tokens, unsigned tile_cap, int slabs, int split, int which, hipStream_t stream) {
     static bool configured = false;   // once per instantiation: more than the default 64 KB of dynamic LDS
     if (!configured) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_gemm_plain<MODE>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, PLAIN_LDS);
         configured = true;
     }
-    hipLaunchKernelGGL(pf_k_pf_gemm_plain<MODE>, dim3(tile_cap * slabs), dim3(256), PLAIN_LDS, stream, a, tokens, slabs, split, (int)shared_only);
+    hipLaunchKernelGGL(pf_k_pf_gemm_plain<MODE>, dim3(tile_cap * slabs), dim3(256), PLAIN_LDS, stream, a, tokens, slabs, split, which);
 }
 
 // the pairs by expert: offsets, row tiles, pair <-> row
@@ -1210,10 +1309,13 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     const bool iq2 = a.type[1] == PF_IQ2_XXS;
     const uint32_t ring_fmt = a.type[1];
     const unsigned tile_cap = (unsigned)pf_prefill_max_tiles(tokens, E, K);
-    if (iq2) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS>(a, tile_cap, gi, H, stream);
-    else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K>(a, tile_cap, gi, H, stream);
+    const bool q8 = a.type[4] == PF_Q8_0;   // the shared expert of the checkpoint profiles
+    if (iq2 && q8) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS, PF_Q8_0>(a, tile_cap, gi, H, 0, stream);
+    else if (iq2) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS, PF_IQ2_XXS>(a, tile_cap, gi, H, 0, stream);
+    else if (q8) launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q8_0>(a, tile_cap, gi, H, 0, stream);
+    else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q4_K>(a, tile_cap, gi, H, 0, stream);
     // only the shared expert's tiles (tokens / 32 of them) are left for this launch: columns split over the waves
-    if (a.type[4] != ring_fmt) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, true, stream);
+    if (a.type[4] != ring_fmt && !q8) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, PLAIN_SHARED, stream);
     const int widest = I > Is ? I : Is;
     const bool digits = a.wm && widest <= 1024;   // the routed rows as digits
     if (widest <= 1024 && P > 0 && tokens > 0) {
@@ -1229,11 +1331,14 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     if (last < 4) return;
     // stage 4: down and combine
     if (a.type[3] == ring_fmt || a.type[6] == ring_fmt) {
-        if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS>(a, tile_cap, H, gi, stream);
-        else launch_gemm<PF_GEMM_DOWN, PF_Q4_K>(a, tile_cap, H, gi, stream);
+        if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS, PF_IQ2_XXS>(a, tile_cap, H, gi, 0, stream);
+        else launch_gemm<PF_GEMM_DOWN, PF_Q4_K, PF_Q4_K>(a, tile_cap, H, gi, 0, stream);
     }
     if (digits) pf_launch_mx_down(a, tile_cap, stream);
-    if (digits ? a.type[6] != ring_fmt : a.type[3] != ring_fmt || a.type[6] != ring_fmt)
-        launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, digits ? (unsigned)((tokens + 31) / 32) : tile_cap, (H + 255) / 256, 0, digits, stream);
+    const bool plain_routed = a.type[3] != ring_fmt && !digits, q8_shared = a.type[6] == PF_Q8_0, plain_shared = a.type[6] != ring_fmt && !q8_shared;
+    if (plain_routed || plain_shared)
+        launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, plain_routed ? tile_cap : (unsigned)((tokens + 31) / 32), (H + 255) / 256, 0,
+                                        !plain_routed ? PLAIN_SHARED : q8_shared ? PLAIN_ROUTED : PLAIN_ALL, stream);
+    if (q8_shared) launch_gemm<PF_GEMM_DOWN, PF_Q8_0, PF_Q8_0>(a, tile_cap, H, Is, tokens, stream);
     pf_launch_combine(a, tokens, stream);
 }
