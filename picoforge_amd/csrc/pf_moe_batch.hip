@@ -30,7 +30,7 @@
 // chunk of up to 2 q tokens only recombines q of the four register quads.  Per 32 x 32 weights: 6 (Q4_K) to 28 (MXFP4)
 // vector instructions for the codes, about 5 for the scales, 7 or 8 per quad -- against 36 per token for the dot-product
 // instructions of the decode kernels and about 75, whatever the rows, for the FP16 product of the prefill kernels.
-#include "pf_moe_internal.h"
+#include "pf_grouped.h"
 #include "pf_image.h"
 #include "pf_route_device.h"
 
@@ -52,7 +52,7 @@ template <bool ROWS> struct BatchRows<PF_Q4_K, ROWS> {   // in tile order a 64-w
     uint4 hdr, q[4];
     uint32_t sc[2], mn[2];
     float d, dmin;
-    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane) {
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane, const uint32_t *) {
         if constexpr (!ROWS) {
             const uint8_t *chunk = a.wt[t] + pf_q4t_chunk_at(a.expert_bytes[t], e, tile, a.blocks_per_row[t], piece);
             hdr = *reinterpret_cast<const uint4 *>(chunk + pf_q4t_header_at(lane & 31));
@@ -91,7 +91,7 @@ template <bool ROWS> struct BatchRows<PF_IQ2_XXS, ROWS> {   // in tile order, el
     uint4 q[4];
     uint32_t dbits;
     float d;
-    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane) {
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane, const uint32_t *) {
         const int kblocks = a.blocks_per_row[t];
         if constexpr (!ROWS) {
             const uint8_t *chunk = a.wi[t] + pf_i2t_chunk_at(pf_i2t_expert_bytes(a.n_out[t], kblocks), e, tile, kblocks, piece);
@@ -127,7 +127,7 @@ template <bool ROWS> struct BatchRows<PF_Q8_0, ROWS> {   // the checkpoint profi
     static constexpr bool MINIMA = false, MIN_OPERAND = false;
     uint4 q[4];
     uint32_t d2[2];
-    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane) {
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane, const uint32_t *) {
         if constexpr (!ROWS) {
             const int runs = a.blocks_per_row[t] / 2, h = lane >> 5;
 #pragma unroll
@@ -158,21 +158,34 @@ template <bool ROWS> struct BatchRows<PF_Q8_0, ROWS> {   // the checkpoint profi
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
 };
 
-template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // row by row: a lane reads its row's whole block and keeps the low or the high nibbles
+template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // in tile order, else row by row: a lane reads its row's whole block and keeps the low or the high nibbles
     static constexpr int GROUPS = 8;
     static constexpr bool MINIMA = false, MIN_OPERAND = false;
     uint4 q[8];
-    uint32_t e2[4];
-    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane) {
-        const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
-        const uint8_t *codes = a.w[t] + row0 * a.row_bytes[t], *scales = a.w[t] + a.scale_offset[t] + row0 * (size_t)a.blocks_per_row[t];
-        const uint32_t code_at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t], scale_at = (uint32_t)(lane & 31) * (uint32_t)a.blocks_per_row[t];
+    uint32_t e2[ROWS ? 4 : 2];
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane, const uint32_t *) {
+        if constexpr (!ROWS) {
+            const int units = groups / 4;
+            const uint8_t *rows = a.wm + e * pf_mxt_expert_bytes(a.n_out[t], units) + (size_t)tile * units * PF_I2T_CHUNK;   // uniform
+            const uint32_t code_at = 16 * (uint32_t)(lane & 31), scale_at = 4 * (uint32_t)(lane & 31);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int g = min(GROUPS * piece + 2 * r, groups - 2);
-            q[2 * r] = *reinterpret_cast<const uint4 *>((codes + 16 * g) + code_at);
-            q[2 * r + 1] = *reinterpret_cast<const uint4 *>((codes + 16 * (g + 1)) + code_at);
-            e2[r] = *reinterpret_cast<const uint16_t *>((scales + g) + scale_at);
+            for (int u = 0; u < 2; u++) {
+                const uint8_t *chunk = rows + (size_t)min(2 * piece + u, units - 1) * PF_I2T_CHUNK;
+#pragma unroll
+                for (int g = 0; g < 4; g++) q[4 * u + g] = *reinterpret_cast<const uint4 *>((chunk + 512 * g) + code_at);
+                e2[u] = *reinterpret_cast<const uint32_t *>((chunk + 2048) + scale_at);
+            }
+        } else {
+            const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
+            const uint8_t *codes = a.w[t] + row0 * a.row_bytes[t], *scales = a.w[t] + a.scale_offset[t] + row0 * (size_t)a.blocks_per_row[t];
+            const uint32_t code_at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t], scale_at = (uint32_t)(lane & 31) * (uint32_t)a.blocks_per_row[t];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int g = min(GROUPS * piece + 2 * r, groups - 2);
+                q[2 * r] = *reinterpret_cast<const uint4 *>((codes + 16 * g) + code_at);
+                q[2 * r + 1] = *reinterpret_cast<const uint4 *>((codes + 16 * (g + 1)) + code_at);
+                e2[r] = *reinterpret_cast<const uint16_t *>((scales + g) + scale_at);
+            }
         }
     }
     __device__ __forceinline__ void open() {}
@@ -181,26 +194,32 @@ template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // row by row: a lane 
         return int4v{e2m1_twice4(q[g].x >> s), e2m1_twice4(q[g].y >> s), e2m1_twice4(q[g].z >> s), e2m1_twice4(q[g].w >> s)};
     }
     __device__ __forceinline__ int4v min_operand(int) const { return int4v{0, 0, 0, 0}; }
-    __device__ __forceinline__ float scale(int g) const { return 0.5f * pf_e8m0_scale((e2[g >> 1] >> (8 * (g & 1))) & 255u); }   // the integers are twice the values
+    __device__ __forceinline__ float scale(int g) const {    // the integers are twice the values
+        return 0.5f * pf_e8m0_scale(ROWS ? (e2[g >> 1] >> (8 * (g & 1))) & 255u : (e2[g >> 2] >> (8 * (g & 3))) & 255u);
+    }
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
 };
 
-// Q2_K, row by row: a lane's half of a group is one sub-group of 16, so its 4-bit scale goes into the codes (at most 45) and
-// its 4-bit minimum is an operand of its own (the sum of the activations of a sub-group is a product with it).
+// Q2_K: a lane's half of a group is one sub-group of 16, so its 4-bit scale goes into the codes (at most 45) and its 4-bit
+// minimum is an operand of its own (the sum of the activations of a sub-group is a product with it).  ROWS: from memory, a
+// dword of 32 rows at a time; else from the wave's copy of the whole tile in LDS (batch_stage_rows).
 template <bool ROWS> struct BatchRows<PF_Q2_K, ROWS> {
     static constexpr int GROUPS = 8;
     static constexpr bool MINIMA = true, MIN_OPERAND = true;
     uint32_t q[8], sm[4], dd;
     float d, dmin;
-    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane) {
+    __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int, int lane, const uint32_t *stage) {
         const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
-        const uint32_t *blocks = reinterpret_cast<const uint32_t *>(a.w[t] + row0 * a.row_bytes[t] + 84 * (size_t)piece);
         const uint32_t at = (uint32_t)(lane & 31) * (uint32_t)(a.row_bytes[t] / 4), code_at = at + 4 + 4 * (uint32_t)(lane >> 5);
+        auto take = [&](const uint32_t *blocks) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) sm[i] = blocks[at + i];
+            for (int i = 0; i < 4; i++) sm[i] = blocks[at + i];
 #pragma unroll
-        for (int i = 0; i < 8; i++) q[i] = blocks[code_at + 8 * (i >> 2) + (i & 3)];
-        dd = blocks[at + 20];
+            for (int i = 0; i < 8; i++) q[i] = blocks[code_at + 8 * (i >> 2) + (i & 3)];
+            dd = blocks[at + 20];
+        };
+        if constexpr (!ROWS) take(stage + 21 * piece);
+        else take(reinterpret_cast<const uint32_t *>(a.w[t] + row0 * a.row_bytes[t] + 84 * (size_t)piece));
     }
     __device__ __forceinline__ void open() { d = half_bits(dd & 0xffffu); dmin = half_bits(dd >> 16); }
     __device__ __forceinline__ uint32_t scale_min(int g) const {   // byte 2 g + h
@@ -308,7 +327,7 @@ __device__ __forceinline__ int batch_lane() {
 template <int FMT, bool ROWS, int PLANES, int SETS, typename ImageAt>
 __device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&tensor)[SETS], size_t e, int tile, int first_piece, int piece_step,
                                             int groups, const uint32_t *images, ImageAt image_at, BatchFactor *factors, int rows,
-                                            const uint32_t *tables, float (&acc)[SETS][4]) {
+                                            const uint32_t *tables, float (&acc)[SETS][4], const uint32_t *stage = nullptr) {
     typedef BatchRows<FMT, ROWS> Rows;
     const int pieces = (groups + Rows::GROUPS - 1) / Rows::GROUPS;
     if (first_piece >= pieces) return;
@@ -317,7 +336,7 @@ __device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&t
     {
         const int lane = batch_lane();
 #pragma unroll
-        for (int s = 0; s < SETS; s++) w[s].load(a, tensor[s], e, tile, first_piece, groups, lane);   // on their way while the rows are looked up
+        for (int s = 0; s < SETS; s++) w[s].load(a, tensor[s], e, tile, first_piece, groups, lane, stage);   // on their way while the rows are looked up
         at = image_at(min((lane & 31) >> 2, rows - 1));
         factor_at = image_at(min(lane >> 3, rows - 1));
     }
@@ -335,7 +354,7 @@ __device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&t
         if (piece + piece_step < pieces) {
             const int lane = batch_lane();
 #pragma unroll
-            for (int s = 0; s < SETS; s++) w[s].load(a, tensor[s], e, tile, piece + piece_step, groups, lane);
+            for (int s = 0; s < SETS; s++) w[s].load(a, tensor[s], e, tile, piece + piece_step, groups, lane, stage);
         }
     }
 }
@@ -458,13 +477,17 @@ template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t
 // blockIdx.x: 32 units; blockIdx.y: row tile.  The workgroup's waves share K (a 256-block each, in turn); their partial
 // sums meet in LDS and are added in wave order, a wave per pair of rows.
 // Bound by the chain a workgroup lives through (item, weights, products, the same for a second 256-block, sums): three
-// workgroups a compute unit keep 120 KB on their way, 3.9 TB/s of weights at 32 tokens (77 us for 283 MB; the 32-row FP16
-// product took 79, at 101 tokens of the q2 profile 309 against 187).  Measured and left out: eight waves with a block each,
-// two waves with four (both slower), the operands past the registers through LDS (slower: LDS becomes the bottleneck for
+// workgroups a compute unit keep 120 KB on their way, 3.9 TB/s of weights at 32 tokens (72 us for 283 MB).  IQ2_XXS, whose
+// table look-ups lengthen the chain and whose weights are half the bytes, is held to the registers of four workgroups a compute
+// unit: 101 tokens of the q2 profile 178 -> 163 us, 24 tokens 82 -> 74; Q4_K spills at that (175 -> 199 us).  With the weights
+// read from a cache the two take 138 and 124 us of these: the products' chain, not the memory, is the longer part.  Measured and left out: eight waves with a block each,
+// five waves for rows of ten blocks (1.4 times slower: every workgroup's fifth wave meets the same SIMD), two
+// waves with four (slower), the next block's weights asked for before the products (no gain, the rows' operands wait behind
+// them), the operands past the registers through LDS (slower: LDS becomes the bottleneck for
 // IQ2_XXS), one matrix a wave at twice the occupancy (85 us).
 #define BATCH_WAVES 4
 template <int FMT, int FMTS, bool ROWS, int PLANES>
-__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(3))) pf_k_batch_gate_up(PfKernelArgs a) {
+__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a) {
     __shared__ float partial[BATCH_WAVES][2][4][64];
     __shared__ BatchFactor factors[BATCH_WAVES][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
@@ -511,11 +534,28 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
     }
 }
 
-// blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert
+// A tile of Q2_K rows of at most BATCH_STAGE_BYTES into the wave's LDS, as it lies in memory.  A row's blocks are 84 bytes, so
+// lanes that read the same dword of 32 rows touch a line each, 64 accesses for 128 bytes: at 101 tokens of the checkpoints'
+// width the kernel stood at 1.9 TB/s (138 us).  The tile is one run of bytes, asked for at once, and in LDS rows of an odd
+// number of dwords meet no bank twice: 104 us (24 tokens 67 -> 53).  Rows of more than three blocks stay on the loads by row.
+#define BATCH_STAGE_BYTES (32 * 3 * 84)
+__device__ __forceinline__ void batch_stage_rows(uint32_t *stage, const PfKernelArgs &a, int t, size_t e, int tile) {
+    const uint32_t bytes = 32 * (uint32_t)a.row_bytes[t];
+    const PfBuffer rows = pf_buffer(a.w[t] + (e * (size_t)a.n_out[t] + (size_t)(32 * tile)) * a.row_bytes[t], bytes);
+#pragma unroll
+    for (int i = 0; i < (BATCH_STAGE_BYTES + 1023) / 1024; i++)   // beyond the tile: zeros, without an access
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_byte *)stage + 1024 * i, 16, 1024 * i + 16 * pf_lane(), 0, 0, 0);
+}
+
+// blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert.  Bound by the products' chain of a wave
+// (with the weights in a cache 90 us of 104 for Q2_K, 97 of 120 for MXFP4, 101 tokens); MXFP4 took 157 us from rows, whose
+// 16-byte blocks are a line each, and takes 120 from the tile-ordered copy that the grouped product keeps.
 template <int FMT, int FMTS, bool ROWS, int PLANES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a) {
+    constexpr bool STAGED = FMT == PF_Q2_K && !ROWS;
     __shared__ BatchFactor factors[4][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
+    __shared__ __align__(16) uint32_t staged[STAGED ? 4 : 1][STAGED ? 2048 : 4];
     BatchItem it;
     if (!batch_item(a, blockIdx.y, it)) return;
     if (batch_tables<FMT>()) batch_stage_tables(tables, a);
@@ -524,13 +564,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) p
     if (32 * tile >= H) return;
     const int groups = (it.shared ? a.shared_inter : a.inter) / 32;
     const uint32_t words = (uint32_t)pf_batch_image_words(PLANES, a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    uint32_t *stage = staged[STAGED ? wave : 0];
+    if (STAGED && !it.shared) {
+        batch_stage_rows(stage, a, 3, it.e, tile);
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the wave's own copy is there
+        pf_wave_lds_fence();
+    }
     for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         auto image_at = [&](int r) { return (uint32_t)(it.first + c0 + r) * words; };
         float acc[1][4] = {};
         const int tensor[1] = {it.shared ? 6 : 3};
         if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS || FMTS == PF_Q8_0, PLANES, 1>(a, tensor, 0, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
-        else batch_chunk<FMT, ROWS, PLANES, 1>(a, tensor, it.e, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
+        else batch_chunk<FMT, ROWS, PLANES, 1>(a, tensor, it.e, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc, stage);
         const int lane = batch_lane();
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -653,7 +699,13 @@ static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile
     const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
     hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a);
     if (last < 4) return;
-    hipLaunchKernelGGL((pf_k_batch_down<FD, FS, ROWS, PLANES>), dim3((a.hidden + 127) / 128, tile_cap), dim3(256), 0, stream, a);
+    // down rows: as gate and up where the layer has one format; MXFP4 in tile order where the layer keeps that copy (resident
+    // ones), Q2_K by whole tiles where they fit a wave's LDS
+    const dim3 grid((a.hidden + 127) / 128, tile_cap);
+    constexpr bool either = FD == PF_Q2_K || (FD == PF_MXFP4 && PLANES == 3);
+    const bool other = FD == PF_Q2_K ? 32 * a.row_bytes[3] <= BATCH_STAGE_BYTES : a.wm != nullptr;
+    if (either && other) hipLaunchKernelGGL((pf_k_batch_down<FD, FS, either ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a);
 }
 
 template <int FG, int FD, int FS>

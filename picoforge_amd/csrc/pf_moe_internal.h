@@ -20,7 +20,7 @@ struct PfKernelArgs {
     const uint8_t *wt[8];            // Q4_K expert tensors in tile order for the grouped product (null: not kept)
     const uint8_t *wi[8];            // IQ2_XXS expert tensors in tile order for the decode kernels (null: not kept)
     const uint8_t *wq[8];            // Q8_0 tensors (the profiles' shared gate and up) in tile order (null: not kept)
-    const uint8_t *wm;               // the routed down tensor, MXFP4, in tile order for the grouped product (null: not kept)
+    const uint8_t *wm;               // the routed down tensor, MXFP4, in tile order for the grouped product and the few-row kernels (null: not kept)
     const float *router_t;           // router as [slab of 64 experts][hidden / 4][64][4] (serial-order re-routing)
     const uint64_t *iq2_grid;        // 256 x 8 magnitudes, device memory
     const uint32_t *iq2_signed;      // 2 x 4096 words: four signed magnitudes per (grid entry, sign nibble)

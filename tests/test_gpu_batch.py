@@ -59,6 +59,25 @@ def test_activations_whose_squares_overflow(product, oracle, router):
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
 
 
+@pytest.mark.parametrize("h,i,physical,fmt,copy", [
+    (512, 256, 256, "q2", "1"), (512, 384, 512, "q2", "1"), (768, 640, 768, "q2", "1"), (512, 896, 1024, "q2", "1"),   # three blocks a row fit the copy in LDS
+    (512, 256, None, "q4", "1"), (512, 384, None, "q4", "1"), (512, 512, None, "q4", "1"), (768, 640, None, "q4", "1"),
+    (512, 768, None, "q4", "1"), (768, 640, None, "q4", "0"),   # no tile-ordered copy: rows
+])
+def test_down_rows_by_tile_and_by_row(product, oracle, monkeypatch, h, i, physical, fmt, copy):
+    """The orders of the profiles' down weights, at two to five units of 128 columns and one to four blocks a row."""
+    print(f"case batch down {fmt} h={h} i={i} down stored {physical or i} wide, tile-ordered copies {copy}", flush=True)
+    monkeypatch.setenv("PF_MOE_PREFILL_COPY", copy)
+    cfg = abi.moe_config(h, 24, 3, i, i, down_physical=physical)
+    weights, x = make_layer_inputs(cfg, fmt, 40, seed=h + i)
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, 40) as layer:
+        for tokens in (17, 40):
+            assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == 3
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
+
+
 # (experts, top-k, format, last batch of the decode kernels, last of the kernels for a few rows per expert)
 LINES = [(16, 4, abi.GGUF_Q4_K, 32, 250), (64, 8, abi.GGUF_Q4_K, 29, 128), (128, 8, abi.GGUF_IQ2_XXS, 28, 247), (64, 8, "q2", 10, 139),
          (128, 8, "q4", 16, 158)]
