@@ -27,6 +27,7 @@
 #include "pf_route_fast.h"
 #include "pf_route_fix.h"
 #include "pf_upload_addr.h"
+#include "pf_mx_rows.h"
 
 #ifdef PF_TIMING
 #define STAMP(i) do { if (blockIdx.x == PF_TIMING && threadIdx.x == 0) reinterpret_cast<unsigned long long *>(a.exact_rows + 2)[i] = wall_clock64(); } while (0)
@@ -1718,6 +1719,116 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FMT =
     }
 }
 
+// ---- kernel 3 of the q4 profile for batches: the block-scaled matrix instruction ----------------------
+#if PF_DECODE_PART == 3
+// The activation rows as digit rows (pf_mx_rows.h), in place.
+__global__ void __launch_bounds__(256) pf_k_dec_rows_to_digits(PfKernelArgs a, size_t rows) {
+    pf_rows_to_digits(blockIdx.x, a.act, a.inter, rows, reinterpret_cast<uint32_t *>(a.act), nullptr, a.error_word);
+}
+
+// A workgroup takes 32 output rows of one token, a wave per slot, then two for the shared expert's rows of 16.
+// v_mfma_scale_f32_16x16x128_f8f6f4: a unit of 128 columns an instruction, the five planes of the slot's digit row as rows 0..4 of the
+// left operand (rows beyond repeat the last and are not looked at), 16 weight rows as MXFP4 stores them on the right: no vector
+// instruction for a weight, where pf_k_dec_down_q4t unpacks and multiplies 64 weights a lane in about 100.  A sum's planes meet at the
+// end, smallest first.  Bound by the two rounds of workgroups that a batch is and their chain (expert, rows, sums): 13 tokens of the
+// checkpoints' widths read 100 MB in 29 us (16 rows a workgroup 38 us, 64 rows 27; without the shared expert 25).
+template <int UNITS>   // of 128 columns
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) pf_k_dec_down_mx(PfKernelArgs a) {
+    __shared__ float partial[16][32];
+    extern __shared__ int lds[];   // twice the shared expert's image and 16 rows' products
+    const int token = (int)blockIdx.y;
+    q4t_at_token(a, token);
+    const int K = a.top_k, lane = pf_lane(), n = lane & 15, kb = lane >> 4;
+    const int s = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int n_base = 32 * (int)blockIdx.x;
+    const PfScalarWords ids = (PfScalarWords)(uintptr_t)a.ids, rws = (PfScalarWords)(uintptr_t)a.route_weights;
+    float rw[16];
+#pragma unroll
+    for (int slot = 0; slot < 16; slot++) rw[slot] = slot < K ? __uint_as_float(rws[slot]) : 0.0f;
+    const float shared_scale = __uint_as_float(((PfScalarWords)(uintptr_t)a.shared_scale)[0]);
+    PfOutputRegs out_regs;
+    if (threadIdx.x < 32) pf_output_prefetch(a, token, n_base + threadIdx.x, out_regs);
+    if (s >= K) {
+        const int part = s - K, Is = a.shared_inter, words = (int)pf_image2_words(Is) + 16 * (Is / 64);
+        const size_t widest = a.inter > Is ? a.inter : Is;
+        uint32_t *mine = reinterpret_cast<uint32_t *>(lds) + part * words;
+        down_wave<PF_Q8_0>(a, 6, 0u, Is, Is, n_base + 16 * part, 16, a.aimg + (size_t)K * pf_image2_words(widest), mine, nullptr,
+                           reinterpret_cast<float *>(mine + pf_image2_words(Is)), partial[K] + 16 * part);
+    } else {
+        uint32_t e = ids[s];
+        if (e >= (uint32_t)a.experts) {   // only reachable with nonfinite logits
+            if (lane == 0) atomicOr(a.error_word, PF_HIP_ERR_BOUNDS | PF_HIP_ERR_NONFINITE);
+            e = 0;
+        }
+        const uint8_t *rows = a.wm + e * pf_mxt_expert_bytes(a.n_out[3], UNITS) + (size_t)(n_base >> 5) * UNITS * PF_I2T_CHUNK;
+        const uint32_t row = (uint32_t)(n_base & 16) + n, code_at = 512 * kb + 16 * row, scale_at = 2048 + 4 * row;
+        uint4v w[2][UNITS];
+        uint32_t ws[2][UNITS];
+#pragma unroll
+        for (int u = 0; u < UNITS; u++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                w[t][u] = *reinterpret_cast<const uint4v *>(rows + (u * PF_I2T_CHUNK + 256 * t) + code_at);
+                ws[t][u] = *reinterpret_cast<const uint32_t *>(rows + (u * PF_I2T_CHUNK + 64 * t) + scale_at);
+            }
+        const uint8_t *line = reinterpret_cast<const uint8_t *>(a.act + (size_t)s * a.inter);
+        const uint32_t plane = min(n, PF_MX_PLANES - 1), group = PF_MX_LINE * kb;
+        float4v acc[2] = {};
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            const uint8_t *unit = line + 4 * PF_MX_LINE * u;
+            const uint4v first = *reinterpret_cast<const uint4v *>(unit + (group + 16 * plane));
+            const uint2v rest = *reinterpret_cast<const uint2v *>(unit + (group + PF_MX_TAIL_AT(plane)));
+            const int scale = unit[group + PF_MX_SCALE_AT(plane)];
+            const int8v x = {(int)first.x, (int)first.y, (int)first.z, (int)first.w, (int)rest.x, (int)rest.y, 0, 0};
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const uint4v c = w[t][u];
+                const int8v b = {(int)c.x, (int)c.y, (int)c.z, (int)c.w, 0, 0, 0, 0};
+                acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(x, b, acc[t], 2, 4, 0, scale, 0, (int)(ws[t][u] >> (8 * kb)));
+            }
+        }
+        const float back = __uint_as_float((uint32_t)line[PF_MX_EXPONENT_AT] << 23);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {   // register r of lanes 16 i ..: plane 4 i + r
+            const float last = __shfl(acc[t][0], 16 + n);
+            if (lane < 16) partial[s][16 * t + n] = ((((last + acc[t][3]) + acc[t][2]) + acc[t][1]) + acc[t][0]) * back;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 32) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int slot = 0; slot < 15; slot++)   // slot order, as src/qwen4_moe.c:362-372
+            if (slot < K) sum += rw[slot] * partial[slot][threadIdx.x];
+        const float y = sum + shared_scale * partial[K][threadIdx.x];
+        if (!pf_output_commit(a, token, n_base + threadIdx.x, y, out_regs)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
+    }
+}
+
+// From five tokens on (checkpoint widths, the rows' conversion of 5 us included): 4 tokens 18.1 us against 19.5, and a launch more;
+// 8 tokens 25 against 38, 13 tokens 35 against 62, 16 tokens 39 against 73.
+#define DOWN_MX_FROM 5
+template <int UNITS> static void launch_down_mx_units(const PfKernelArgs &a, int tokens, hipStream_t stream) {
+    const size_t lds = 2 * (size_t)(pf_image2_words(a.shared_inter) + 16 * (a.shared_inter / 64)) * 4;
+    hipLaunchKernelGGL(pf_k_dec_down_mx<UNITS>, dim3(a.hidden / 32, tokens), dim3(64 * (a.top_k + 2)), lds, stream, a);
+}
+static bool down_mx_applies(const PfKernelArgs &a, int tokens) {
+    return tokens >= DOWN_MX_FROM && a.wm && a.top_k + 2 <= 16;   // at most 1024 threads
+}
+static void launch_down_mx(const PfKernelArgs &a, int tokens, hipStream_t stream) {
+    const size_t rows = (size_t)tokens * a.top_k, block = 4 * pf_mx_rows_a_wave(a.inter);
+    hipLaunchKernelGGL(pf_k_dec_rows_to_digits, dim3((unsigned)((rows + block - 1) / block)), dim3(256), 0, stream, a, rows);
+    switch (a.inter / 128) {
+    case 1: launch_down_mx_units<1>(a, tokens, stream); break;
+    case 2: launch_down_mx_units<2>(a, tokens, stream); break;
+    case 3: launch_down_mx_units<3>(a, tokens, stream); break;
+    case 4: launch_down_mx_units<4>(a, tokens, stream); break;
+    default: launch_down_mx_units<5>(a, tokens, stream);   // a layer keeps the copy up to 640 columns
+    }
+}
+#endif
+
 // ---- kernel 3 for batches of six tokens and more, tensors in tile order -------------------------------
 // A workgroup takes 64 output rows of one token, a wave per slot (the last wave the shared expert), a lane per row: the
 // 64 lanes of a wave share the run they are at, so the activation digits are scalar operands read from the digit image
@@ -2472,6 +2583,12 @@ static void launch_q4t_experts(const PfKernelArgs &a, int tokens, hipStream_t st
             return;
         }
     }
+#if PF_DECODE_PART == 3
+    if (!POOL && down_mx_applies(a, tokens)) {
+        launch_down_mx(a, tokens, stream);
+        return;
+    }
+#endif
     const size_t widest = I > Is ? I : Is;
     constexpr bool GRID = FD == PF_IQ2_XXS || FS == PF_IQ2_XXS;
     // rows per workgroup: eight in the tile order; for down tensors kept row by row the fewest that leave no more

@@ -20,8 +20,6 @@
 #include "pf_mx_rows.h"
 #include "pf_upload_addr.h"
 
-typedef int int8v __attribute__((ext_vector_type(8)));
-
 template <int UNITS>   // of 128 columns
 __global__ void __launch_bounds__(256, 2) pf_k_mx_down(PfKernelArgs a, int slabs, int per) {
     extern __shared__ __align__(16) unsigned char mx_lds[];

@@ -6,14 +6,19 @@
 // leave 2^-25 of the binade of the group's largest magnitude (the two-part halfs of the other grouped products: 2^-23 of the
 // value, and not under 2^-25 of the row's).
 //
-// 128 bytes a group: 16 bytes of each plane's 24 (chunks 0..4), the planes' other 8 bytes, then the five scale bytes and padding.  A slot
-// order within the group that follows MXFP4's nibbles: slot 2 i is column i, slot 2 i + 1 column 16 + i.
+// 128 bytes a group: 16 bytes of each plane's 24 (chunks 0..4), the planes' other 8 bytes, then the five scale bytes, the
+// row's exponent and padding.  A slot order within the group that follows MXFP4's nibbles: slot 2 i is column i, slot 2 i + 1 column 16 + i.
 #pragma once
 #include "pf_grouped.h"
 
 #define PF_MX_PLANES 5
+#define PF_MX_TAIL_AT(plane) (80 + 8 * (plane))
+#define PF_MX_SCALE_AT(plane) (120 + (plane))
+#define PF_MX_EXPONENT_AT 125
 #define PF_MX_LINE 128   // bytes of a group; a row of K values takes 4 K bytes
 
+typedef int int8v __attribute__((ext_vector_type(8)));
+typedef float float4v __attribute__((ext_vector_type(4)));
 typedef float float32v __attribute__((ext_vector_type(32)));
 typedef uint32_t uint6v __attribute__((ext_vector_type(6)));
 
@@ -32,7 +37,7 @@ __device__ __forceinline__ float32v pf_from_e2m3(const uint6v &q, float scale) {
 
 // A lane per group; a wave takes as many whole rows as its lanes hold groups (cols at most 1024, a multiple of 32).
 __host__ __device__ constexpr int pf_mx_rows_a_wave(int cols) { return 64 / (cols / 32); }
-__device__ __forceinline__ void pf_rows_to_digits(size_t block, const float *src, int cols, size_t rows, uint32_t *dst, float *scale_out, uint32_t *error_word) {
+__device__ __forceinline__ void pf_rows_to_digits(size_t block, const float *src, int cols, size_t rows, uint32_t *dst, float *scale_out, uint32_t *error_word) {   // dst may be src: a lane writes the bytes that it has read
     const int lane = pf_lane(), groups = cols / 32, at = lane / groups, group = lane - at * groups, together = pf_mx_rows_a_wave(cols);
     const size_t row = (block * 4 + (threadIdx.x >> 6)) * together + at;
     const bool mine = at < together && row < rows;
@@ -69,12 +74,12 @@ __device__ __forceinline__ void pf_rows_to_digits(size_t block, const float *src
         for (int i = 0; i < 16; i++) { a[i] -= back[2 * i]; b[i] -= back[2 * i + 1]; }
     }
     if (!mine) return;
-    if (group == 0) scale_out[row] = __int_as_float((e + 1) << 23);
+    if (group == 0 && scale_out) scale_out[row] = __int_as_float((e + 1) << 23);
     uint4v *line = reinterpret_cast<uint4v *>(dst + row * cols + 32 * group);
 #pragma unroll
     for (int p = 0; p < PF_MX_PLANES; p++) line[p] = uint4v{plane[p][0], plane[p][1], plane[p][2], plane[p][3]};
     line[5] = uint4v{plane[0][4], plane[0][5], plane[1][4], plane[1][5]};
     line[6] = uint4v{plane[2][4], plane[2][5], plane[3][4], plane[3][5]};
     const uint32_t s0 = (uint32_t)(127 + E - 2);   // plane p: 5 p less
-    line[7] = uint4v{plane[4][4], plane[4][5], s0 * 0x01010101u - 0x0F0A0500u, s0 - 20u};
+    line[7] = uint4v{plane[4][4], plane[4][5], s0 * 0x01010101u - 0x0F0A0500u, (s0 - 20u) | (uint32_t)(e + 1) << 8};
 }

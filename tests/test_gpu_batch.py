@@ -95,3 +95,26 @@ def test_batches_on_both_sides_of_the_lines_between_the_kernels(product, oracle,
             assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == family, tokens
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
+
+
+@pytest.mark.parametrize("h,i,s,k,copy", [
+    (512, 256, 256, 6, "1"), (768, 384, 384, 1, "1"), (512, 512, 640, 14, "1"), (512, 256, 256, 15, "1"), (2560, 640, 640, 10, "1"), (1024, 768, 256, 4, "1"),   # 768: no copy
+    (2560, 640, 640, 10, "0"),
+])
+def test_short_batches_of_the_q4_profile(product, oracle, monkeypatch, h, i, s, k, copy):
+    """The decode kernels' down projections of MXFP4 rows: on the block-scaled matrix instruction where the layer keeps the
+    tile-ordered copy, from the batch size on where that pays; two to five units of 128 columns, one to fifteen slots."""
+    print(f"case short q4 batches h={h} i={i} s={s} k={k} tile-ordered copies {copy}", flush=True)
+    monkeypatch.setenv("PF_MOE_PREFILL_COPY", copy)
+    cfg = abi.moe_config(h, 32, k, i, s)
+    weights, x = make_layer_inputs(cfg, "q4", 16, seed=h + i + k)
+    x[3] = 0.0
+    x[4, : h // 2] *= 1e-4
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, 16) as layer:
+        for tokens in (1, 2, 3, 4, 5, 16):
+            assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == (1 if copy == "1" or tokens <= 4 else 3)
+            print(f"  tokens={tokens}", flush=True)
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
+        np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
