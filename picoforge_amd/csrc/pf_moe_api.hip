@@ -503,6 +503,7 @@ static void carve_work(PfHipWork *w, const Carve &c, uint8_t *base);
 // write the output rows straight into the block.
 #define PF_HOST_BLOCK_TOKENS 64   // (beyond, a byte over the link costs a kernel more than it costs a copy engine)
 #define PF_HOST_HEAD_BYTES 256
+#define PF_RING_ARRIVED 62   // word of exact_rows that counts a ring piece's workgroups (zero, as the workspace is at first)
 struct HostBlock {
     uint8_t *head;
     uint32_t *ids, *slots;
@@ -524,7 +525,8 @@ static HostBlock host_block(const PfHipMoeDesc *d, size_t cap, uint8_t *base) {
     b.slots_offset = at;
     b.slots = (uint32_t *)(base + at); at += pairs;
     b.published_offset = at;
-    b.published = (uint32_t *)(base + at); at += 256;
+    b.published = (uint32_t *)(base + at); at += 64 * (1 + PF_RING_SLOTS);   // and the ring's words (ring_word)
+    at = (at + 255) & ~(size_t)255;
     b.bytes = at;
     return b;
 }
@@ -537,11 +539,40 @@ __global__ void pf_k_copy_rows(const uint4 *src, uint4 *dst, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = src[i];
 }
+// A piece of a longer batch's ring, and its number into the slot's word on the host.  (An event after every piece is a packet of
+// its own that nothing overlaps, 5.5 us beside the 10 to 14 of 512 KB.  A fence in every wave instead of one for 16 KB makes them
+// 20.)  A call of 777 tokens of width 2048 829 -> 760 us, of 1024 of width 2560 1280 -> 1190.  arrived: zero between the launches,
+// which follow each other on one stream.
+__global__ void __launch_bounds__(256) pf_k_copy_piece(const uint4 *src, uint4 *dst, int n, uint32_t *arrived, uint32_t *word, uint32_t number, int out) {
+    const int i0 = (int)(blockIdx.x * 1024 + threadIdx.x);   // four loads on their way, and a fence for 16 KB
+    uint4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = src[min(i0 + 256 * k, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (i0 + 256 * k < n) dst[i0 + 256 * k] = v[k];
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the wave's own stores have been taken
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (out) __threadfence_system();   // in: a stored value has been read, and only the stream's next kernel looks at it
+    if (__hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
+    __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 struct PublishParts { const uint32_t *src[3]; uint32_t *dst[3]; int words[3]; };
 // One workgroup: the parts, then (everything before it has reached the host's memory) the call's number.
-__global__ void __launch_bounds__(256) pf_k_publish(PublishParts p, uint32_t *published, uint32_t call) {
-    for (int j = 0; j < 3; j++)
-        for (int i = threadIdx.x; i < p.words[j]; i += 256) p.dst[j][i] = p.src[j][i];
+// THREADS: 256 for the block's batches, 1024 and 16 bytes a thread for longer ones (777 tokens 24 -> 14 us; the shorter ones'
+// call is 0.8 us longer that way).
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS) pf_k_publish(PublishParts p, uint32_t *published, uint32_t call) {
+    for (int j = 0; j < 3; j++) {
+        int first = 0;
+        if (THREADS > 256 && ((uintptr_t)p.src[j] | (uintptr_t)p.dst[j]) % 16 == 0) {
+            first = p.words[j] / 4 * 4;
+            for (int i = threadIdx.x; i < first / 4; i += THREADS) reinterpret_cast<uint4 *>(p.dst[j])[i] = reinterpret_cast<const uint4 *>(p.src[j])[i];
+        }
+        for (int i = first + threadIdx.x; i < p.words[j]; i += THREADS) p.dst[j][i] = p.src[j][i];
+    }
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(published, call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -560,7 +591,7 @@ struct HostResults { const uint32_t *error_word, *ids; const float *weights; uin
 static hipError_t publish_results(PfHipWork *w, const HostBlock &b, size_t tokens, bool want_ids, bool want_weights, HostResults *r) {
     const int pairs = (int)(tokens * w->moe->desc.top_k);
     const bool in_block = tokens <= PF_HOST_BLOCK_TOKENS;
-    uint8_t *const ids = in_block ? (uint8_t *)b.ids : w->routes, *const weights = in_block ? (uint8_t *)b.weights : w->routes + 4 * (size_t)pairs;
+    uint8_t *const ids = in_block ? (uint8_t *)b.ids : w->routes, *const weights = in_block ? (uint8_t *)b.weights : w->routes + 16 * (((size_t)pairs + 3) / 4);
     r->error_word = (const uint32_t *)b.head;
     r->ids = (const uint32_t *)ids;
     r->weights = (const float *)weights;
@@ -569,7 +600,7 @@ static hipError_t publish_results(PfHipWork *w, const HostBlock &b, size_t token
     p.src[0] = w->error_word; p.dst[0] = (uint32_t *)w->host_device; p.words[0] = 1;
     p.src[1] = w->ids; p.dst[1] = (uint32_t *)(w->host_device + (ids - w->host)); p.words[1] = want_ids ? pairs : 0;
     p.src[2] = (const uint32_t *)w->route_weights; p.dst[2] = (uint32_t *)(w->host_device + (weights - w->host)); p.words[2] = want_weights ? pairs : 0;
-    hipLaunchKernelGGL(pf_k_publish, dim3(1), dim3(256), 0, nullptr, p, (uint32_t *)(w->host_device + b.published_offset), r->call);
+    hipLaunchKernelGGL(in_block ? pf_k_publish<256> : pf_k_publish<1024>, dim3(1), dim3(in_block ? 256 : 1024), 0, nullptr, p, (uint32_t *)(w->host_device + b.published_offset), r->call);
     return hipGetLastError();
 }
 // The number is polled for as long as a short batch can take; then the stream is waited for, which also reports its errors.
@@ -582,10 +613,22 @@ static hipError_t await_results(const HostBlock &b, const HostResults &r) {
 }
 
 // Longer batches pass through the workspace's ring of page-locked pieces (pf_host_rows.h).  A piece travels by a kernel that
-// addresses the page-locked memory: 35 GB/s and no wait between engine and kernels, where copies of this size brought 22 GB/s
-// out of the device.
+// addresses the page-locked memory: 38 GB/s and no wait between engine and kernels, where copies of this size brought 22 GB/s
+// out of the device.  With eight threads, or pieces of 256 KB, nothing is faster (777 rows of 8 KB: 770, 775 and 850 us).
 static int ring_bind(void *, int device) { return (int)hipSetDevice(device); }
-static int ring_wait(void *work, int slot) { return (int)hipEventSynchronize(static_cast<PfHipWork *>(work)->ring_event[slot]); }
+static uint32_t *ring_word(const PfHipWork *w, int slot) {   // in the block: behind the published call's number, a line each
+    return host_block(&w->moe->desc, w->cap, w->host).published + 16 * (slot + 1);
+}
+static int ring_wait(void *work, int slot) {
+    PfHipWork *w = static_cast<PfHipWork *>(work);
+    if (!w->ring_number[slot]) return (int)hipEventSynchronize(w->ring_event[slot]);
+    const uint32_t *word = ring_word(w, slot);
+    for (int turn = 0; turn < 400000; turn++) {
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == w->ring_number[slot]) return 0;
+        __builtin_ia32_pause();
+    }
+    return (int)hipStreamSynchronize(nullptr);   // long past a piece's time; also reports the stream's errors
+}
 static int ring_send(void *work, int slot, void *dst, const void *src, size_t bytes, bool in) {
     PfHipWork *w = static_cast<PfHipWork *>(work);
     hipError_t e;
@@ -594,12 +637,16 @@ static int ring_send(void *work, int slot, void *dst, const void *src, size_t by
             const uint8_t *b = static_cast<const uint8_t *>(p);
             return b >= w->ring && b < w->ring + PF_RING_SLOTS * PF_RING_BYTES ? w->host_device + (b - w->host) : const_cast<uint8_t *>(b);
         };
-        hipLaunchKernelGGL(pf_k_copy_rows, dim3((unsigned)((bytes / 16 + 255) / 256)), dim3(256), 0, nullptr, reinterpret_cast<const uint4 *>(on_device(src)),
-                           reinterpret_cast<uint4 *>(on_device(dst)), (int)(bytes / 16));
-        e = hipGetLastError();
-    } else {
-        e = hipMemcpyAsync(dst, src, bytes, in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, nullptr);
+        uint32_t number = w->ring_sent[slot] + 1;
+        if (!number) number = 1;   // 0: no kernel's
+        w->ring_sent[slot] = w->ring_number[slot] = number;
+        hipLaunchKernelGGL(pf_k_copy_piece, dim3((unsigned)((bytes / 16 + 1023) / 1024)), dim3(256), 0, nullptr, reinterpret_cast<const uint4 *>(on_device(src)),
+                           reinterpret_cast<uint4 *>(on_device(dst)), (int)(bytes / 16), w->exact_rows + PF_RING_ARRIVED,
+                           (uint32_t *)(w->host_device + ((uint8_t *)ring_word(w, slot) - w->host)), number, in ? 0 : 1);
+        return (int)hipGetLastError();
     }
+    w->ring_number[slot] = 0;
+    e = hipMemcpyAsync(dst, src, bytes, in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, nullptr);
     const hipError_t recorded = hipEventRecord(w->ring_event[slot], nullptr);
     return (int)(e != hipSuccess ? e : recorded);
 }
@@ -652,7 +699,7 @@ extern "C" int pf_hip_work_create(const PfHipMoe *moe, size_t token_cap, PfHipWo
     // waits once, for the last of them (without the block the forwards fall back to one blocking copy per buffer)
     const size_t block = host_block(&moe->desc, token_cap, nullptr).bytes;
     const bool long_batches = token_cap > PF_HOST_BLOCK_TOKENS;
-    const size_t routes = long_batches ? (2 * token_cap * moe->desc.top_k * 4 + 255) & ~(size_t)255 : 0;   // ids and weights of a longer batch
+    const size_t routes = long_batches ? (2 * token_cap * moe->desc.top_k * 4 + 16 + 255) & ~(size_t)255 : 0;   // ids and weights of a longer batch
     if (hipHostMalloc((void **)&w->host, block + routes + (long_batches ? PF_RING_SLOTS * PF_RING_BYTES : 0), hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         w->host = nullptr;

@@ -202,7 +202,9 @@ struct PfHipWork {
     uint8_t *host_device;           // the same block as the kernels address it (they write the output rows straight into it)
     uint8_t *ring;                  // page-locked pieces behind the block, for host-pointer forwards of longer batches (null: none)
     uint8_t *routes;                // page-locked ids and route weights of a longer batch, between the block and the ring
-    hipEvent_t ring_event[8];      // a piece's last transfer
+    hipEvent_t ring_event[8];      // a piece's last transfer, where a copy engine makes it (ring_number 0)
+    uint32_t ring_number[8];       // else: the number that its kernel leaves in the slot's word of the block
+    uint32_t ring_sent[8];         // numbers given out
     uint32_t call;                  // number of the host-pointer call in progress (the block holds the last one published)
     int stage_limit;                // profiling: launch only the first so many kernels of a forward; 0 = all
     int force_general;               // tests: run the general kernels even where the decode path applies

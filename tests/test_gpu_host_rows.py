@@ -72,3 +72,25 @@ def test_two_workspaces_at_once(product):
     for layer in layers:
         layer.close()
     assert not wrong, wrong
+
+
+@pytest.mark.parametrize("hidden,k", [(256, 1), (768, 3), (2560, 5)])
+def test_pieces_of_every_length_call_after_call(product, hidden, k):
+    """Last pieces of less than a kernel's 16 KB, of a whole number of them and of more, slots taken again within a call and by
+    the next one; ids and weights of a longer batch at every remainder of four."""
+    step = 512 * 1024 // (4 * hidden)
+    cfg = abi.moe_config(hidden, 12, k, 256, 256)
+    most = 9 * step + 3
+    weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, most, seed=hidden + k)
+    with pf.MoeLayer(product, cfg, weights, most) as layer:
+        layer.force_general()
+        _, y, ids, w = layer.forward(x[:300])
+        for tokens in (65, 66, 67, 68, step, step + 1, 2 * step - 1, 8 * step + 4, most, 65, 9 * step):
+            print(f"case pieces hidden={hidden} tokens={tokens}", flush=True)
+            _, yt, idst, wt = layer.forward(x[:tokens])
+            n = min(tokens, 300)
+            np.testing.assert_array_equal(yt[:n], y[:n])
+            np.testing.assert_array_equal(idst[:n], ids[:n])
+            np.testing.assert_array_equal(wt[:n], w[:n])
+            _, again, _, _ = layer.forward(x[:tokens])
+            np.testing.assert_array_equal(yt, again)
