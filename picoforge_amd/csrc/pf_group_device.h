@@ -1,0 +1,124 @@
+// Grouping of a batch's pairs by expert in one workgroup: the part that pf_moe_route.hip (alone in a launch) and
+// pf_moe_prefill.hip (beside the activation rows' conversion) share.
+#pragma once
+#include "pf_device.h"
+
+// One workgroup of 1024 threads: counts the pairs per expert in LDS, scans the counts (offsets, and the row tiles:
+// tiles[0] = count, tiles[1 + i] = expert | tile index << 16, items[i] = {expert, first row, rows, first row within the expert}; the shared expert = expert E with every token, as
+// pf_k_pf_scan_tiles lists them), and hands every pair the next free row of its expert through an LDS cursor.  The rows
+// of an expert are therefore in no particular order (pf_k_group_place keeps them in pair order): every row of the
+// grouped products is computed on its own and found again through pair_to_row, so the order changes no result, and a
+// walk over all pairs per expert, which the order costs, took three times as long as everything else here.
+#define GROUP_FUSED_MAX_PAIRS 32768
+#define GROUP_FUSED_MAX_EXPERTS 2047
+//
+// Bound by one compute unit's chain of loads, LDS atomics and stores.  An expert has GROUP_COPIES counters, a lane's by its number,
+// so that a popular one's pairs do not queue for one word, and the rows' pairs are collected in LDS and written in order: scattered
+// stores are a cache line each.  Beside the conversion of the rows (pf_k_pf_group_rows) 20480 pairs 27.7 -> 24.6 us, 10240 16.1 -> 14.2
+// (Zipf 1.1, 512 experts).
+#define GROUP_COPIES 8
+#define GROUP_FUSED_LDS ((GROUP_COPIES * GROUP_FUSED_MAX_EXPERTS + GROUP_FUSED_MAX_PAIRS / 2) * 4)   // 128 KB, at most
+// words of fused_lds: the counters, then the pair of every row in 16 bits
+__host__ __device__ constexpr size_t pf_group_lds_words(int pairs, int E) { return (size_t)GROUP_COPIES * E + (pairs + 7) / 8 * 4; }
+__device__ __forceinline__ void pf_group_block(uint32_t *fused_lds, const uint32_t *ids, int pairs, int E, int tokens, uint32_t *offsets,
+                                               uint32_t *tiles, uint4 *items, uint32_t *pair_to_row, uint32_t *row_to_pair) {
+    __shared__ uint32_t wave_rows[16], wave_tiles[16];
+    const int tid = threadIdx.x, quads = pairs / 4;
+    uint32_t *counts = fused_lds;   // [expert][copy]; later the next free row
+    uint16_t *pair_of = reinterpret_cast<uint16_t *>(fused_lds + (size_t)GROUP_COPIES * E);
+    for (int i = tid; i < GROUP_COPIES * E; i += 1024) counts[i] = 0;
+    // four pairs a thread and step (ids on a 16-byte boundary), all of a thread's asked for at once and kept for the second walk; the
+    // ragged end pair by pair
+    constexpr int STEPS = GROUP_FUSED_MAX_PAIRS / 4 / 1024;
+    uint4 four[STEPS];
+#pragma unroll
+    for (int k = 0; k < STEPS; k++)
+        if (1024 * k < quads) four[k] = reinterpret_cast<const uint4 *>(ids)[min(tid + 1024 * k, quads - 1)];
+    const int tail = 4 * quads + tid;   // at most three pairs
+    const uint32_t last = tail < pairs ? ids[tail] : 0xffffffffu;
+    uint32_t *mine = counts + tid % GROUP_COPIES;
+    __syncthreads();
+    auto count = [&](uint32_t id) { if (id < (uint32_t)E) atomicAdd(&mine[GROUP_COPIES * id], 1u); };
+#pragma unroll
+    for (int k = 0; k < STEPS; k++) {
+        if (tid + 1024 * k >= quads) break;
+        count(four[k].x); count(four[k].y); count(four[k].z); count(four[k].w);
+    }
+    count(last);
+    __syncthreads();
+    // exclusive scan of the counts (rows) and of the row-tile counts, thread t owning `per` consecutive experts
+    const int per = (E + 1 + 1023) / 1024, lo = tid * per, hi = min(E + 1, lo + per);
+    auto rows_of = [&](int e) {
+        if (e == E) return (uint32_t)tokens;
+        uint32_t c = 0;
+#pragma unroll
+        for (int r = 0; r < GROUP_COPIES; r++) c += counts[GROUP_COPIES * e + r];
+        return c;
+    };
+    uint32_t rows = 0, ntiles = 0;
+    for (int e = lo; e < hi; e++) {
+        const uint32_t c = rows_of(e);
+        if (e < E) rows += c;
+        ntiles += (c + 31u) / 32u;
+    }
+    // inclusive scan over the 1024 threads: within a wave by shuffles, then the sixteen waves' totals through LDS
+    const int lane = pf_lane(), wave = tid >> 6;
+    uint32_t run_rows = rows, run_tiles = ntiles;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t up_rows = __shfl_up(run_rows, d), up_tiles = __shfl_up(run_tiles, d);
+        if (lane >= d) { run_rows += up_rows; run_tiles += up_tiles; }
+    }
+    if (lane == 63) { wave_rows[wave] = run_rows; wave_tiles[wave] = run_tiles; }
+    __syncthreads();
+    uint32_t placed = 0;   // pairs of experts there are
+    for (int w = 0; w < 16; w++) {
+        if (w < wave) { run_rows += wave_rows[w]; run_tiles += wave_tiles[w]; }
+        placed += wave_rows[w];
+    }
+    if (tid == 1023) {
+        offsets[E] = run_rows;
+        tiles[0] = run_tiles;
+    }
+    uint32_t row = run_rows - rows, at = run_tiles - ntiles;
+    for (int e = lo; e < hi; e++) {
+        const uint32_t c = rows_of(e), n = (c + 31u) / 32u;
+        for (uint32_t i = 0; i < n; i++) {
+            tiles[1 + at + i] = (uint32_t)e | (i << 16);
+            items[at + i] = make_uint4((uint32_t)e, (e < E ? row : (uint32_t)pairs) + 32u * i, min(32u, c - 32u * i), 32u * i);
+        }
+        at += n;
+        if (e == E) break;
+        offsets[e] = row;
+#pragma unroll
+        for (int r = 0; r < GROUP_COPIES; r++) {
+            const uint32_t here = counts[GROUP_COPIES * e + r];
+            counts[GROUP_COPIES * e + r] = row;
+            row += here;
+        }
+    }
+    __syncthreads();
+    auto place = [&](uint32_t id, int p) -> uint32_t {
+        if (id >= (uint32_t)E) return 0u;   // only with nonfinite logits
+        const uint32_t r = atomicAdd(&mine[GROUP_COPIES * id], 1u);
+        pair_of[r] = (uint16_t)p;
+        return r;
+    };
+#pragma unroll
+    for (int k = 0; k < STEPS; k++) {
+        const int q = tid + 1024 * k;
+        if (q >= quads) break;
+        const uint4 v = four[k];
+        uint4 r;
+        r.x = place(v.x, 4 * q); r.y = place(v.y, 4 * q + 1); r.z = place(v.z, 4 * q + 2); r.w = place(v.w, 4 * q + 3);
+        reinterpret_cast<uint4 *>(pair_to_row)[q] = r;
+    }
+    if (tail < pairs) pair_to_row[tail] = place(last, tail);
+    __syncthreads();
+    for (uint32_t q = tid; 4 * q + 3 < placed; q += 1024) {
+        const uint2 v = reinterpret_cast<const uint2 *>(pair_of)[q];
+        reinterpret_cast<uint4 *>(row_to_pair)[q] = make_uint4(v.x & 0xffffu, v.x >> 16, v.y & 0xffffu, v.y >> 16);
+    }
+    const uint32_t rest = (placed & ~3u) + tid;
+    if (tid < 4 && rest < placed) row_to_pair[rest] = pair_of[rest];
+}

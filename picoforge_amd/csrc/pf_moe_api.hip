@@ -409,7 +409,7 @@ extern "C" size_t pf_hip_moe_bytes(const PfHipMoe *m) { return m ? m->total_byte
 
 // workspace layout: buffers carved from one allocation, each 256-byte aligned
 enum { W_LOGITS, W_SSQ, W_ERR, W_IDS, W_RW, W_ACT, W_SACT, W_SSCALE, W_X, W_Y, W_SLOTS, W_UNIQ, W_EXACT, W_FLAGS, W_XIMG, W_AIMG,
-       W_FLINES, W_FGEN, W_X16, W_ACT16, W_SACT16, W_XSCALE, W_ACTSCALE, W_SACTSCALE, W_XMAX2, W_DOWN, W_COUNTS, W_OFFSETS,
+       W_FLINES, W_FGEN, W_X16, W_ACT16, W_SACT16, W_XSCALE, W_ACTSCALE, W_SACTSCALE, W_DOWN, W_COUNTS, W_OFFSETS,
        W_P2R, W_R2P, W_GROUPBAD, W_TILES, W_ITEMS, W_COUNT };
 #define PF_GUARD_BYTES 4096
 struct Carve { size_t offset[W_COUNT], size[W_COUNT], total; bool fused; size_t guard; };
@@ -467,7 +467,6 @@ static Carve plan_work(const PfHipMoeDesc *d, size_t cap, bool fused = false, si
     want[W_XSCALE] = Tp * 4;
     want[W_ACTSCALE] = Tp * K * 4;
     want[W_SACTSCALE] = Tp * 4;
-    want[W_XMAX2] = Tp * 4;
     want[W_DOWN] = (Tp * K + Tp) * H * 4;
     want[W_COUNTS] = prefill ? E * 4 : 0;
     want[W_OFFSETS] = prefill ? (E + 1) * 4 : 0;
@@ -752,7 +751,6 @@ static void carve_work(PfHipWork *w, const Carve &c, uint8_t *base) {
         w->x_scale = (float *)(base + c.offset[W_XSCALE]);
         w->act_scale = (float *)(base + c.offset[W_ACTSCALE]);
         w->sact_scale = (float *)(base + c.offset[W_SACTSCALE]);
-        w->x_max2 = (float *)(base + c.offset[W_XMAX2]);
         w->down = (float *)(base + c.offset[W_DOWN]);
         w->counts = (uint32_t *)(base + c.offset[W_COUNTS]);
         w->offsets = (uint32_t *)(base + c.offset[W_OFFSETS]);
@@ -861,7 +859,7 @@ static PfKernelArgs make_args(const PfHipMoe *m, PfHipWork *w, const float *d_x,
     a.fuse_lines = w->fuse_lines; a.fuse_gen = w->fuse_gen;
     a.error_word = w->error_word; a.exact_rows = w->exact_rows; a.route_flags = w->route_flags;
     a.x16 = w->x16; a.act16 = w->act16; a.sact16 = w->sact16;
-    a.x_scale = w->x_scale; a.act_scale = w->act_scale; a.sact_scale = w->sact_scale; a.x_max2 = w->x_max2;
+    a.x_scale = w->x_scale; a.act_scale = w->act_scale; a.sact_scale = w->sact_scale;
     a.w_norm2 = m->w_norm2; a.down = w->down;
     a.counts = w->counts; a.offsets = w->offsets; a.pair_to_row = w->pair_to_row; a.row_to_pair = w->row_to_pair;
     a.group_bad = w->group_bad; a.tiles = w->tiles; a.items = w->items;

@@ -55,7 +55,6 @@ struct PfKernelArgs {
     uint16_t *x16, *act16, *sact16;  // fp16 forms of x, act (pairs in expert order), shared act: per row the high
                                      // parts, the low parts, then 8 + 8 group-sum parts per 256 columns
     float *x_scale, *act_scale, *sact_scale;   // per row: the power of two the fp16 form was divided by
-    float *x_max2;                   // [tokens] largest squared magnitude of the row
     const float *w_norm2;            // [experts] squared norm of each router row
     float *down;                     // [pairs + tokens, hidden] down products in expert order, then the shared expert's
     uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles;
@@ -196,7 +195,7 @@ struct PfHipWork {
     float *logits, *logit_ssq, *route_weights, *act, *shared_act, *shared_scale, *x, *y;
     uint32_t *ids, *uniq, *error_word, *exact_rows, *route_flags, *slots, *fuse_lines, *fuse_gen;
     uint16_t *x16, *act16, *sact16;  // prefill buffers (allocated when cap exceeds the decode path's batch)
-    float *x_scale, *act_scale, *sact_scale, *x_max2, *down;
+    float *x_scale, *act_scale, *sact_scale, *down;
     uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles, *items;
     uint8_t *host;                  // pinned host block for the host-pointer forwards of short batches (null: not available)
     uint8_t *host_device;           // the same block as the kernels address it (they write the output rows straight into it)
@@ -272,6 +271,7 @@ void pf_launch_block_split(const uint8_t *d_gguf, uint8_t *d_payload, uint8_t *d
 // pf_moe_prefill.hip
 bool pf_prefill_supported(const PfHipMoeDesc &d);
 void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
+bool pf_group_fits(const uint32_t *d_ids, int pairs, int experts);   // one workgroup groups them
 void pf_launch_group(const PfKernelArgs &a, const uint32_t *ids, int tokens, hipStream_t stream);
 void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream);
 void pf_launch_q4k_tile(const uint8_t *d_src, uint8_t *d_dst, size_t rows, int blocks_per_row, hipStream_t stream);

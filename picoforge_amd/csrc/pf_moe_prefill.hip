@@ -25,6 +25,7 @@
 #include "pf_plain_walk.h"
 #include "pf_grouped.h"
 #include "pf_mx_rows.h"
+#include "pf_group_device.h"
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
@@ -57,23 +58,21 @@ void pf_launch_q4k_tile(const uint8_t *d_src, uint8_t *d_dst, size_t rows, int b
 // threads form one 32-group.
 // gate (may be null): a row of `cols` weights; gate_out[row] = sigmoid(row . gate), the shared router's scale (four
 // partial sums a lane, lanes and waves added in a fixed order).
-__global__ void __launch_bounds__(256) pf_k_rows_to_half(const float *src, size_t src_pitch, int cols, half_t *dst,
-                                                         float *scale_out, float *max2_out, uint32_t *error_word,
-                                                         const float *gate, float *gate_out) {
-    __shared__ float part[4];
-    __shared__ float dots[4];
+// tid: 0..255 of the row's threads; part, dots: four floats of LDS of theirs; store: whether the row is one to write (every
+// thread of the workgroup comes along: barriers)
+__device__ __forceinline__ void row_to_half(size_t row, bool store, int tid, float *part, float *dots, const float *src, size_t src_pitch, int cols, half_t *dst,
+                                            float *scale_out, uint32_t *error_word, const float *gate, float *gate_out) {
     float dot = 0.0f;
-    const size_t row = blockIdx.x;
     const float *s = src + row * src_pitch;
     float m = 0.0f;
     bool bad = false;
-    for (int c = threadIdx.x; c < cols; c += blockDim.x) {
+    for (int c = tid; c < cols; c += 256) {
         const float v = s[c];
         bad |= !pf_finite(v);
         m = fmaxf(m, fabsf(v));
     }
     m = pf_wave_max(m);
-    if (pf_lane() == 0) part[threadIdx.x >> 6] = m;
+    if (pf_lane() == 0) part[tid >> 6] = m;
     if (__any(bad) && pf_lane() == 0) atomicOr(error_word, PF_HIP_ERR_NONFINITE);
     __syncthreads();
     m = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
@@ -82,7 +81,7 @@ __global__ void __launch_bounds__(256) pf_k_rows_to_half(const float *src, size_
     const float scale = __int_as_float((e + 1) << 23);        // 2^(e-126)
     const float inv = __int_as_float((253 - e) << 23);        // 2^(126-e)
     half_t *out = dst + row * pf_half_row(cols);
-    for (int j = threadIdx.x; j < cols / 8; j += blockDim.x) {
+    for (int j = tid; j < cols / 8; j += 256) {
         const float4 a = reinterpret_cast<const float4 *>(s)[2 * j], b = reinterpret_cast<const float4 *>(s)[2 * j + 1];
         const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         if (gate) {
@@ -99,11 +98,13 @@ __global__ void __launch_bounds__(256) pf_k_rows_to_half(const float *src, size_
             lo[c] = l;
             sum += (float)h + (float)l;
         }
-        *reinterpret_cast<half8v *>(out + 8 * j) = hi;
-        *reinterpret_cast<half8v *>(out + cols + 8 * j) = lo;
+        if (store) {
+            *reinterpret_cast<half8v *>(out + 8 * j) = hi;
+            *reinterpret_cast<half8v *>(out + cols + 8 * j) = lo;
+        }
         sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0xB1, 0xF, 0xF, true));   // quad xor 1
         sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x4E, 0xF, 0xF, true));   // quad xor 2
-        if ((j & 3) == 0) {
+        if ((j & 3) == 0 && store) {
             const int g = j >> 2;
             const half_t sh = (half_t)sum, sl = (half_t)(sum - (float)sh);
             half_t *sums = out + 2 * cols + 16 * (g >> 3) + 8 * (g & 1) + ((g & 7) >> 1);
@@ -113,18 +114,37 @@ __global__ void __launch_bounds__(256) pf_k_rows_to_half(const float *src, size_
     }
     if (gate) {   // uniform
         dot = pf_wave_sum(dot);
-        if (pf_lane() == 0) dots[threadIdx.x >> 6] = dot;
+        if (pf_lane() == 0) dots[tid >> 6] = dot;
         __syncthreads();
-        if (threadIdx.x == 0) {
+        if (tid == 0 && store) {
             const float z = (dots[0] + dots[1]) + (dots[2] + dots[3]);
             gate_out[row] = pf_sigmoid(z);
             if (!pf_finite(z)) atomicOr(error_word, PF_HIP_ERR_NONFINITE);
         }
     }
-    if (threadIdx.x == 0) {
-        scale_out[row] = scale;
-        if (max2_out) max2_out[row] = m * m;
+    if (tid == 0 && store) scale_out[row] = scale;
+}
+__global__ void __launch_bounds__(256) pf_k_rows_to_half(const float *src, size_t src_pitch, int cols, half_t *dst, float *scale_out,
+                                                         uint32_t *error_word, const float *gate, float *gate_out) {
+    __shared__ float part[4], dots[4];
+    row_to_half(blockIdx.x, true, threadIdx.x, part, dots, src, src_pitch, cols, dst, scale_out, error_word, gate, gate_out);
+}
+
+// Workgroup 0 groups the pairs (pf_group_device.h), the others convert the chunk's rows, four each: the grouping, one workgroup's
+// chain, leaves the rest of the chip idle, and the conversion fits in beside it.  Apart they took 14.3 and 10.7 us (1024 tokens of
+// width 2048), 21.9 and 12.5 (2048 of width 2560), together 14.2 and 24.6; the router finds the rows' largest magnitudes itself for
+// another 1.5.
+__global__ void __launch_bounds__(1024) pf_k_pf_group_rows(PfKernelArgs a, int tokens) {
+    extern __shared__ __align__(16) uint32_t group_lds[];
+    if (blockIdx.x == 0) {
+        pf_group_block(group_lds, a.ids, tokens * a.top_k, a.experts, tokens, a.offsets, a.tiles, reinterpret_cast<uint4 *>(const_cast<uint32_t *>(a.items)),
+                       a.pair_to_row, a.row_to_pair);
+        return;
     }
+    __shared__ float part[4][4], dots[4][4];
+    const int team = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)), row = 4 * ((int)blockIdx.x - 1) + team;
+    row_to_half(min(row, tokens - 1), row < tokens, threadIdx.x & 255, part[team], dots[team], a.x, a.x_pitch, a.hidden, (half_t *)a.x16, a.x_scale,
+                a.error_word, reinterpret_cast<const float *>(a.w[7]), a.shared_scale);
 }
 
 // The same for rows of at most 512 PARTS values (the activation rows): one wave per row, four rows per workgroup, the row
@@ -208,10 +228,10 @@ __global__ void __launch_bounds__(256) pf_k_rows_to_half_short2(const float *src
 }
 
 static void launch_rows_to_half(const float *src, size_t src_pitch, int cols, size_t rows, half_t *dst, float *scale_out,
-                                float *max2_out, uint32_t *error_word, hipStream_t stream) {
+                                uint32_t *error_word, hipStream_t stream) {
     if (rows == 0) return;
     hipLaunchKernelGGL(pf_k_rows_to_half, dim3((unsigned)rows), dim3(256), 0, stream, src, src_pitch, cols, dst, scale_out,
-                       max2_out, error_word, (const float *)nullptr, (float *)nullptr);
+                       error_word, (const float *)nullptr, (float *)nullptr);
 }
 
 // squared norm of every router row (once, at upload)
@@ -252,9 +272,11 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 template <int TR, int TC>
 __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_waves_per_eu(2))) pf_k_pf_router(PfKernelArgs a, int tokens) {
     extern __shared__ __align__(16) float router_lds[];   // [wave][x rows, then experts][column]; later the waves' partial tiles
+    __shared__ uint32_t largest[32 * TR];                 // the rows' largest magnitudes, as bits
     const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = threadIdx.x >> 6;
     const int t0 = blockIdx.x * 32 * TR, e0 = blockIdx.y * 32 * TC;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.route_flags[0] = 0;   // the routing's list starts empty
+    if (threadIdx.x < 32 * TR) largest[threadIdx.x] = 0;
     const int i = lane & 31, kk = lane >> 5;
     // the waves split the rows' 128-byte lines (hidden is a multiple of 32)
     const int lines = H / 32, l0 = lines * wave / PF_ROUTER_WAVES, l1 = lines * (wave + 1) / PF_ROUTER_WAVES;
@@ -273,6 +295,7 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
     for (int r = 0; r < TR; r++)
 #pragma unroll
         for (int c = 0; c < TC; c++) acc[r][c] = float16v{0};
+    float most[4 * TR] = {};
     if (l0 < l1) {
         float4v fetched[ROWS];
 #pragma unroll
@@ -283,6 +306,11 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
             // measured no faster)
 #pragma unroll
             for (int g = 0; g < ROWS; g++) *reinterpret_cast<float4v *>(mine + (8 * g + lr) * PF_ROUTER_PITCH + 4 * piece) = fetched[g];
+#pragma unroll
+            for (int g = 0; g < 4 * TR; g++) {
+                const float4v v = fetched[g];
+                most[g] = fmaxf(most[g], fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+            }
             const int next = l + 1 < l1 ? l + 1 : l;
 #pragma unroll
             for (int g = 0; g < ROWS; g++) fetched[g] = src[g][8 * next];
@@ -303,6 +331,8 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
         }
     }
     __syncthreads();   // the staged pieces have been read
+#pragma unroll
+    for (int g = 0; g < 4 * TR; g++) atomicMax(&largest[8 * g + lr], __float_as_uint(most[g]));
     constexpr int REGS = 16 * TR * TC;
 #pragma unroll
     for (int r = 0; r < REGS; r++) router_lds[(wave * REGS + r) * 64 + lane] = acc[r / 16 / TC][r / 16 % TC][r % 16];
@@ -316,7 +346,8 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
         const int row = t0 + 32 * (r / 16 / TC) + 8 * ((r & 15) >> 2) + 4 * kk + (r & 3), col = e0 + 32 * (r / 16 % TC) + i;
         if (row >= tokens || col >= E) continue;
         a.logits[(size_t)row * E + col] = logit;
-        a.logit_ssq[(size_t)row * E + col] = a.x_max2[row] * a.w_norm2[col];
+        const float m = __uint_as_float(largest[row - t0]);
+        a.logit_ssq[(size_t)row * E + col] = m * m * a.w_norm2[col];
     }
 }
 template <int TR, int TC>
@@ -1285,11 +1316,7 @@ void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream) {
 void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit) {
     const int H = a.hidden, E = a.experts, K = a.top_k, I = a.inter, Is = a.shared_inter, P = tokens * K;
     const int last = stage_limit ? stage_limit : 4;
-    // stage 1: fp16 parts of x, router logits
-    // (the shared router's column rides with the conversion: as a column of the router product it cost a 17th column
-    // tile of full depth, and 544 workgroups do not spread evenly over 256 compute units, 512 do)
-    hipLaunchKernelGGL(pf_k_rows_to_half, dim3(tokens), dim3(256), 0, stream, a.x, a.x_pitch, H, (half_t *)a.x16, a.x_scale,
-                       a.x_max2, a.error_word, reinterpret_cast<const float *>(a.w[7]), a.shared_scale);
+    // stage 1: router logits
     // the tile whose rounds over the chip are the least matrix work, the larger of two equal ones
     auto work = [&](int tr, int tc) {
         const long tiles = (long)((tokens + 32 * tr - 1) / (32 * tr)) * ((E + 32 * tc - 1) / (32 * tc));
@@ -1299,9 +1326,20 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     else if (work(2, 1) <= work(1, 1)) launch_router<2, 1>(a, tokens, stream);
     else launch_router<1, 1>(a, tokens, stream);
     if (last < 2) return;
-    // stage 2: routes and grouping
+    // stage 2: routes, grouping, fp16 parts of x
+    // (the shared router's column rides with the conversion: as a column of the router product it cost a 17th column
+    // tile of full depth, and 544 workgroups do not spread evenly over 256 compute units, 512 do)
     pf_launch_route(a, tokens, stream);
-    pf_launch_group(a, a.ids, tokens, stream);
+    if (pf_group_fits(a.ids, P, E)) {
+        static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_group_rows), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                           GROUP_FUSED_LDS) == hipSuccess;
+        (void)configured;
+        hipLaunchKernelGGL(pf_k_pf_group_rows, dim3(1 + (unsigned)(tokens + 3) / 4), dim3(1024), pf_group_lds_words(P, E) * sizeof(uint32_t), stream, a, tokens);
+    } else {
+        hipLaunchKernelGGL(pf_k_rows_to_half, dim3(tokens), dim3(256), 0, stream, a.x, a.x_pitch, H, (half_t *)a.x16, a.x_scale, a.error_word,
+                           reinterpret_cast<const float *>(a.w[7]), a.shared_scale);
+        pf_launch_group(a, a.ids, tokens, stream);
+    }
     if (last < 3) return;
     // stage 3: gate/up + SwiGLU, then fp16 parts of the activation rows
     // the ring kernel takes the items whose tensors are in the routed gate's format, the plain kernel the rest
@@ -1325,8 +1363,8 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
                            stream, a.act, I, (size_t)P, (half_t *)a.act16, a.act_scale, blocks_a, a.shared_act, Is, (size_t)tokens,
                            (half_t *)a.sact16, a.sact_scale, a.error_word);
     } else {
-        launch_rows_to_half(a.act, (size_t)I, I, (size_t)P, (half_t *)a.act16, a.act_scale, nullptr, a.error_word, stream);
-        launch_rows_to_half(a.shared_act, (size_t)Is, Is, (size_t)tokens, (half_t *)a.sact16, a.sact_scale, nullptr, a.error_word, stream);
+        launch_rows_to_half(a.act, (size_t)I, I, (size_t)P, (half_t *)a.act16, a.act_scale, a.error_word, stream);
+        launch_rows_to_half(a.shared_act, (size_t)Is, Is, (size_t)tokens, (half_t *)a.sact16, a.sact_scale, a.error_word, stream);
     }
     if (last < 4) return;
     // stage 4: down and combine

@@ -10,6 +10,7 @@
 #include "pf_route_device.h"
 #include "pf_route_fast.h"
 #include "pf_route_fix.h"
+#include "pf_group_device.h"
 
 #define ROUTE_MAX_FAST_EXPERTS 1024
 
@@ -375,91 +376,24 @@ void pf_launch_group_place(const uint32_t *d_ids, int pairs, int experts, const 
                        d_pair_to_row, d_row_to_pair);
 }
 
-// ---- grouping in one launch (the prefill path) ---------------------------------------------------------
-// One workgroup of 1024 threads: counts the pairs per expert in LDS, scans the counts (offsets, and the row tiles:
-// tiles[0] = count, tiles[1 + i] = expert | tile index << 16, items[i] = {expert, first row, rows, first row within the expert}; the shared expert = expert E with every token, as
-// pf_k_pf_scan_tiles lists them), and hands every pair the next free row of its expert through an LDS cursor.  The rows
-// of an expert are therefore in no particular order (pf_k_group_place keeps them in pair order): every row of the
-// grouped products is computed on its own and found again through pair_to_row, so the order changes no result, and a
-// walk over all pairs per expert, which the order costs, took three times as long as everything else here.
-#define GROUP_FUSED_MAX_PAIRS 32768
-#define GROUP_FUSED_MAX_EXPERTS 2047
+// ---- grouping in one launch (pf_group_device.h) ---------------------------------------------------------
 __global__ void __launch_bounds__(1024) pf_k_group_fused(const uint32_t *ids, int pairs, int E, int tokens, uint32_t *offsets,
                                                          uint32_t *tiles, uint4 *items, uint32_t *pair_to_row, uint32_t *row_to_pair) {
     extern __shared__ __align__(16) uint32_t fused_lds[];
-    __shared__ uint32_t wave_rows[16], wave_tiles[16];
-    const int tid = threadIdx.x, quads = pairs / 4;
-    uint32_t *counts = fused_lds, *cursor = counts + (E + 1);
-    for (int e = tid; e <= E; e += 1024) counts[e] = 0;
-    __syncthreads();
-    // four pairs a thread and step (ids on a 16-byte boundary), the ragged end pair by pair
-    for (int q = tid; q < quads; q += 1024) {
-        const uint4 v = reinterpret_cast<const uint4 *>(ids)[q];
-        if (v.x < (uint32_t)E) atomicAdd(&counts[v.x], 1u);
-        if (v.y < (uint32_t)E) atomicAdd(&counts[v.y], 1u);
-        if (v.z < (uint32_t)E) atomicAdd(&counts[v.z], 1u);
-        if (v.w < (uint32_t)E) atomicAdd(&counts[v.w], 1u);
-    }
-    for (int p = 4 * quads + tid; p < pairs; p += 1024) {
-        const uint32_t id = ids[p];
-        if (id < (uint32_t)E) atomicAdd(&counts[id], 1u);
-    }
-    __syncthreads();
-    // exclusive scan of the counts (rows) and of the row-tile counts, thread t owning `per` consecutive experts
-    const int per = (E + 1 + 1023) / 1024, lo = tid * per, hi = min(E + 1, lo + per);
-    uint32_t rows = 0, ntiles = 0;
-    for (int e = lo; e < hi; e++) {
-        const uint32_t c = e < E ? counts[e] : (uint32_t)tokens;
-        if (e < E) rows += c;
-        ntiles += (c + 31u) / 32u;
-    }
-    // inclusive scan over the 1024 threads: within a wave by shuffles, then the sixteen waves' totals through LDS
-    const int lane = pf_lane(), wave = tid >> 6;
-    uint32_t run_rows = rows, run_tiles = ntiles;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t up_rows = __shfl_up(run_rows, d), up_tiles = __shfl_up(run_tiles, d);
-        if (lane >= d) { run_rows += up_rows; run_tiles += up_tiles; }
-    }
-    if (lane == 63) { wave_rows[wave] = run_rows; wave_tiles[wave] = run_tiles; }
-    __syncthreads();
-    for (int w = 0; w < wave; w++) { run_rows += wave_rows[w]; run_tiles += wave_tiles[w]; }
-    if (tid == 1023) {
-        offsets[E] = run_rows;
-        tiles[0] = run_tiles;
-    }
-    uint32_t row = run_rows - rows, at = run_tiles - ntiles;
-    for (int e = lo; e < hi; e++) {
-        const uint32_t c = e < E ? counts[e] : (uint32_t)tokens, n = (c + 31u) / 32u;
-        if (e < E) {
-            cursor[e] = row;
-            offsets[e] = row;
-        }
-        for (uint32_t i = 0; i < n; i++) {
-            tiles[1 + at + i] = (uint32_t)e | (i << 16);
-            items[at + i] = make_uint4((uint32_t)e, (e < E ? row : (uint32_t)pairs) + 32u * i, min(32u, c - 32u * i), 32u * i);
-        }
-        if (e < E) row += c;
-        at += n;
-    }
-    __syncthreads();
-    auto place = [&](uint32_t id, int p) {
-        if (id >= (uint32_t)E) return;
-        const uint32_t r = atomicAdd(&cursor[id], 1u);
-        pair_to_row[p] = r;
-        row_to_pair[r] = (uint32_t)p;
-    };
-    for (int q = tid; q < quads; q += 1024) {
-        const uint4 v = reinterpret_cast<const uint4 *>(ids)[q];
-        place(v.x, 4 * q); place(v.y, 4 * q + 1); place(v.z, 4 * q + 2); place(v.w, 4 * q + 3);
-    }
-    for (int p = 4 * quads + tid; p < pairs; p += 1024) place(ids[p], p);
+    pf_group_block(fused_lds, ids, pairs, E, tokens, offsets, tiles, items, pair_to_row, row_to_pair);
+}
+
+bool pf_group_fits(const uint32_t *d_ids, int pairs, int experts) {
+    return pairs > 0 && pairs <= GROUP_FUSED_MAX_PAIRS && experts <= GROUP_FUSED_MAX_EXPERTS && (reinterpret_cast<uintptr_t>(d_ids) & 15) == 0;
 }
 
 bool pf_launch_group_fused(const uint32_t *d_ids, int pairs, int experts, int tokens, uint32_t *d_offsets, uint32_t *d_tiles,
                            uint32_t *d_items, uint32_t *d_pair_to_row, uint32_t *d_row_to_pair, hipStream_t stream) {
-    if (pairs <= 0 || pairs > GROUP_FUSED_MAX_PAIRS || experts > GROUP_FUSED_MAX_EXPERTS || (reinterpret_cast<uintptr_t>(d_ids) & 15)) return false;
-    const size_t lds = 2 * ((size_t)experts + 1) * sizeof(uint32_t);
+    if (!pf_group_fits(d_ids, pairs, experts)) return false;
+    const size_t lds = pf_group_lds_words(pairs, experts) * sizeof(uint32_t);
+    static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_group_fused), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       GROUP_FUSED_LDS) == hipSuccess;   // more than the default 64 KB
+    (void)configured;
     hipLaunchKernelGGL(pf_k_group_fused, dim3(1), dim3(1024), lds, stream, d_ids, pairs, experts, tokens, d_offsets, d_tiles,
                        reinterpret_cast<uint4 *>(d_items), d_pair_to_row, d_row_to_pair);
     return true;

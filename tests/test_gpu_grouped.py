@@ -48,6 +48,26 @@ def test_row_counts_around_the_tiles(product, oracle, monkeypatch, h, i, s, phys
         np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
 
 
+@pytest.mark.parametrize("tokens,e,k", [(4096, 16, 8), (2049, 300, 7), (1023, 40, 3), (131, 9, 1)])
+def test_pairs_that_one_workgroup_groups(product, tokens, e, k):
+    """Up to 32768 pairs (128 KB of LDS), at every remainder of four, beside rows that do not fill the last workgroup; an expert
+    that every token has."""
+    print(f"case grouped, {tokens} tokens of {k} pairs, {e} experts", flush=True)
+    cfg = abi.moe_config(256, e, k, 256, 256)
+    weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, tokens, seed=tokens + e)
+    x[:, 0] = 1.0
+    weights.raw[0].view(np.float32).reshape(e, 256)[e // 2, 0] = 9.0
+    x[::7] *= 1e-3
+    with pf.MoeLayer(product, cfg, weights, len(x)) as layer:
+        layer.force_grouped()
+        _, y, ids, w = layer.forward(x)
+        np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
+        layer.force_general()
+        _, yg, idsg, wg = layer.forward(x)
+    assert (ids == e // 2).any(axis=1).mean() > 0.8
+    assert_parity(y, ids, w, yg, idsg, wg, label="grouped product against general kernels")
+
+
 def test_more_pairs_than_one_workgroup_groups(product):
     """Beyond 32768 pairs the row tiles come from the kernels that count, scan and place one after the other."""
     print("case grouped, 4100 tokens of 8 pairs", flush=True)
