@@ -1260,7 +1260,7 @@ extern "C" int pf_hip_moe_route_streamed_host(const PfHipMoe *moe, PfHipWork *wo
         return PF_HIP_E_UNSUPPORTED;
     }
     if (streamed_batch(moe, work, tokens, tiled_mask)) {
-        pf_launch_batch_router(a, (int)tokens, 4, nullptr);
+        pf_launch_batch_router(a, (int)tokens, 4, false, nullptr);
         pf_launch_dec_route(a, (int)tokens, nullptr);
     } else if (streamed_decode(moe, work, tokens, tiled_mask)) {
         pf_launch_dec_router(a, (int)tokens, (int)((moe->desc.experts + 3) / 4), nullptr);

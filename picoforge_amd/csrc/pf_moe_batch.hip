@@ -416,14 +416,14 @@ template <int PLANES> __device__ __forceinline__ void batch_step(float m, float 
     }
 }
 // What a vector's group ends with: the step, and the sum of its integers (at most 36 bits, from the sums of their upper and
-// lower 16 bits).
-template <int PLANES> __device__ __forceinline__ void batch_image_end(uint32_t *img, int g, int K, float step, int upper, int lower) {
+// lower 16 bits); WHOLE: as the decode kernels keep it, three planes' 29 bits as an integer.
+template <int PLANES, bool WHOLE = false> __device__ __forceinline__ void batch_image_end(uint32_t *img, int g, int K, float step, int upper, int lower) {
     img[8 * PLANES * (K / 32) + g] = __float_as_uint(step);
-    img[(8 * PLANES + 1) * (K / 32) + g] = __float_as_uint(fmaf(65536.0f, (float)upper, (float)lower));
+    img[(8 * PLANES + 1) * (K / 32) + g] = WHOLE ? (uint32_t)(65536 * upper + lower) : __float_as_uint(fmaf(65536.0f, (float)upper, (float)lower));
 }
 
 // Thread j of a group of four neighbouring lanes: the eight values 8j..8j+7 of a K-vector into its image.
-template <int PLANES> __device__ __forceinline__ void batch_image_chunk(uint32_t *img, const float (&v)[8], int j, int K) {
+template <int PLANES, bool WHOLE> __device__ __forceinline__ void batch_image_chunk(uint32_t *img, const float (&v)[8], int j, int K) {
     float m = 0.0f;
 #pragma unroll
     for (int c = 0; c < 8; c++) m = fmaxf(m, fabsf(v[c]));
@@ -448,7 +448,7 @@ template <int PLANES> __device__ __forceinline__ void batch_image_chunk(uint32_t
     const int g = j >> 2, at = 8 * PLANES * g + 2 * (j & 3);
 #pragma unroll
     for (int p = 0; p < PLANES; p++) { img[at + 8 * p] = w[p][0]; img[at + 8 * p + 1] = w[p][1]; }
-    if ((j & 3) == 0) batch_image_end<PLANES>(img, g, K, step, upper, lower);
+    if ((j & 3) == 0) batch_image_end<PLANES, WHOLE>(img, g, K, step, upper, lower);
 }
 
 // Lanes 0..31 and 32..63, one value each: group g of two K-vectors' images (store: whether the lane's vector exists).
@@ -600,7 +600,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) p
 typedef float float4v __attribute__((ext_vector_type(4)));
 #define ROUTER_LINES 5      // 32-column lines a wave holds: hidden <= 2560
 #define ROUTER_PITCH 36     // floats between rows of a staged line: neighbouring lanes' 16-byte reads cover all banks
-template <int PLANES>
+template <int PLANES, bool WHOLE>   // WHOLE: the decode kernels' images
 __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int tokens) {
     __shared__ __align__(16) float staged[16][2][16 * ROUTER_PITCH];
     const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -608,15 +608,16 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
         const int t = 16 * blockIdx.x + wave;
         if (t >= tokens) return;
         const float4v *row = reinterpret_cast<const float4v *>(a.x + (size_t)t * a.x_pitch), *gate = reinterpret_cast<const float4v *>(a.w[7]);
-        float z = 0.0f;
+        float4v zp = {0}, zq = {0};   // eight chains, as above
         for (int j = lane; j < H / 8; j += 64) {
             const float4v p = row[2 * j], q = row[2 * j + 1], u = gate[2 * j], v = gate[2 * j + 1];
             const float both[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
-            batch_image_chunk<PLANES>(a.ximg + (size_t)t * pf_batch_image_words(PLANES, H), both, j, H);
+            batch_image_chunk<PLANES, WHOLE>(a.ximg + (size_t)t * pf_batch_image_words(PLANES, H), both, j, H);
 #pragma unroll
-            for (int c = 0; c < 4; c++) z = fmaf(p[c], u[c], fmaf(q[c], v[c], z));
+            for (int c = 0; c < 4; c++) { zp[c] = fmaf(p[c], u[c], zp[c]); zq[c] = fmaf(q[c], v[c], zq[c]); }
         }
-        z = pf_wave_sum(z);
+        zp += zq;
+        const float z = pf_wave_sum((zp.x + zp.y) + (zp.z + zp.w));
         if (lane == 0) {
             a.shared_scale[t] = pf_sigmoid(z);
             if (!pf_finite(z)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
@@ -688,9 +689,11 @@ __global__ void __launch_bounds__(1024) pf_k_batch_router(PfKernelArgs a, int to
     }
 }
 
-void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, hipStream_t stream) {
+bool pf_batch_router_takes(int hidden) { return hidden % 32 == 0 && hidden <= 16 * 32 * ROUTER_LINES; }
+void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, bool whole, hipStream_t stream) {
     const dim3 grid((tokens + 15) / 16, (a.experts + 15) / 16 + 1);
-    hipLaunchKernelGGL(planes == 4 ? pf_k_batch_router<4> : pf_k_batch_router<3>, grid, dim3(1024), 0, stream, a, tokens);
+    auto *const kernel = whole ? pf_k_batch_router<3, true> : planes == 4 ? pf_k_batch_router<4, false> : pf_k_batch_router<3, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(1024), 0, stream, a, tokens);
 }
 
 // ---- dispatch --------------------------------------------------------------------------------------
@@ -733,7 +736,7 @@ void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stre
 
 void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit) {
     const int last = stage_limit ? stage_limit : 4;
-    pf_launch_batch_router(a, tokens, 3, stream);
+    pf_launch_batch_router(a, tokens, 3, false, stream);
     if (last < 2) return;
     pf_launch_dec_route(a, tokens, stream);
     pf_launch_group(a, a.ids, tokens, stream);

@@ -285,7 +285,8 @@ void pf_launch_mx_tile(const uint8_t *d_payload, const uint8_t *d_scales, uint8_
 void pf_launch_mx_down(const PfKernelArgs &a, unsigned tile_cap, hipStream_t stream);
 // pf_moe_batch.hip: a few rows per expert, for the layers of the tile decode kernels
 void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
-void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, hipStream_t stream);
+bool pf_batch_router_takes(int hidden);
+void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, bool whole, hipStream_t stream);   // whole: with the decode kernels' images
 void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stream, int last);
 // pf_moe_hc.hip
 void pf_launch_hc_read(const float *d_normed, size_t n_token_pitch, size_t n_stream_pitch, const float *d_logits,

@@ -118,3 +118,19 @@ def test_short_batches_of_the_q4_profile(product, oracle, monkeypatch, h, i, s, 
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
         np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
+
+
+@pytest.mark.parametrize("h,e,k,fmt", [(512, 70, 6, abi.GGUF_Q4_K), (2560, 33, 4, abi.GGUF_Q4_K), (768, 100, 5, abi.GGUF_IQ2_XXS), (2048, 512, 3, abi.GGUF_IQ2_XXS)])
+def test_decode_kernels_on_either_side_of_the_matrix_router(product, oracle, h, e, k, fmt):
+    """Up to 16 tokens the decode kernels' own router, from 17 on tiles of 16 tokens and experts, whose images they read."""
+    print(f"case decode router {fmt} h={h} e={e} k={k}", flush=True)
+    cfg = abi.moe_config(h, e, k, 256, 256)
+    weights, x = make_layer_inputs(cfg, fmt, 32, seed=h + e)
+    x[3] = 0.0
+    x[20] *= 1e-4
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, 32) as layer:
+        for tokens in (16, 17, 25, 32):
+            assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == 1
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
