@@ -95,7 +95,8 @@ int pf_hip_moe_kernel_family(const PfHipMoe *moe, const PfHipWork *work, size_t 
  * Q4_K or IQ2_XXS throughout, a workspace created with PF_MOE_DECODE_FUSED=1 in the environment, a
  * device with a compute unit per workgroup: an option, slower than the three kernels where it was
  * measured), or 4 where the routing runs in a launch of its own between the router logits and a
- * gate/up kernel that is given the experts (three tokens or more on the tile-ordered kernels).
+ * gate/up kernel that is given the experts (three tokens or more on the tile-ordered kernels; what
+ * converts the activation rows ahead of an MXFP4 down product counts as part of that).
  * 0: the forward runs other kernels. */
 int pf_hip_moe_decode_launches(const PfHipMoe *moe, const PfHipWork *work, size_t tokens);
 /* Device pointers into the workspace, valid after a forward: expert ids

@@ -50,8 +50,8 @@ PF_HD bool pf_tensor_place(uint32_t type, size_t k_storage, size_t n_out, size_t
     p->n_out = (int)n_out;
     p->blocks_per_row = (int)blocks_per_row;
     if (head) {
-        // every block's payload (64, 32 or 16 bytes), then every block's scale; four bytes of slack because the prefill
-        // loader reads the dword around a scale
+        // every block's payload (64, 32 or 16 bytes), then every block's scale; four bytes of slack for a reader
+        // that takes the dword around a scale
         const size_t payload = size - head;
         p->row_bytes = blocks_per_row * payload;
         p->scale_offset = (blocks_per_row * rows * payload + 255) & ~(size_t)255;

@@ -252,9 +252,9 @@ extern "C" int pf_hip_moe_create(const PfHipMoeDesc *desc, const void *const hos
             pf_hip_moe_destroy(m);
             return e == hipErrorOutOfMemory ? PF_HIP_E_MEMORY : PF_HIP_E_RUNTIME;
         }
-        // Second, tile-ordered copy of the expert tensors: the grouped product then reads whole cache
-        // lines once instead of 32-byte pieces of lines it meets again a stage later.  It doubles the
-        // expert bytes; PF_MOE_PREFILL_COPY=0 does without it (the same kernels read the row order).
+        // Second, tile-ordered copy of the expert tensors: a load of the grouped product, and of the decode kernels whose lanes
+        // are weight rows, is then whole cache lines instead of 16 bytes of 32 rows.  It doubles the expert bytes;
+        // PF_MOE_PREFILL_COPY=0 does without it (the grouped product reads the row order).
         const char *copy = getenv("PF_MOE_PREFILL_COPY");
         if (!copy || strcmp(copy, "0") != 0) {
             for (int a = 1; a <= 6 && e == hipSuccess; a++) {
@@ -263,14 +263,6 @@ extern "C" int pf_hip_moe_create(const PfHipMoeDesc *desc, const void *const hos
                 if (e == hipSuccess) {
                     pf_launch_q4k_tile(m->w[a], m->w_tiled[a], (size_t)n_out[a] * experts[a], m->blocks_per_row[a], nullptr);
                     m->total_bytes += m->bytes[a];
-                }
-            }
-            if (e == hipSuccess && pf_mx_down_takes(*desc)) {   // its block-scaled product reads whole lines of this copy
-                const size_t bytes = pf_mxt_expert_bytes((int)n_out[3], m->blocks_per_row[3] / 4) * experts[3];
-                e = hipMalloc((void **)&m->w_mxtile, bytes);
-                if (e == hipSuccess) {
-                    pf_launch_mx_tile(m->w[3], m->w[3] + m->scale_offset[3], m->w_mxtile, (size_t)n_out[3] * experts[3], m->blocks_per_row[3], nullptr);
-                    m->total_bytes += bytes;
                 }
             }
             if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -316,6 +308,25 @@ extern "C" int pf_hip_moe_create(const PfHipMoeDesc *desc, const void *const hos
                 pf_hip_moe_destroy(m);
                 return e == hipErrorOutOfMemory ? PF_HIP_E_MEMORY : PF_HIP_E_RUNTIME;
             }
+        }
+    }
+    // The routed MXFP4 down tensor in tile order, for the block-scaled products and the few-row kernels.  Where there is no
+    // memory left for it they read the rows (a layer that fits without the copy is not refused for it).
+    if (m->prefill_ready && pf_mx_down_takes(*desc)) {
+        const char *copy = getenv("PF_MOE_PREFILL_COPY");
+        const size_t bytes = pf_mxt_expert_bytes((int)n_out[3], m->blocks_per_row[3] / 4) * experts[3];
+        if ((!copy || strcmp(copy, "0") != 0) && hipMalloc((void **)&m->w_mxtile, bytes) == hipSuccess) {
+            pf_launch_mx_tile(m->w[3], m->w[3] + m->scale_offset[3], m->w_mxtile, (size_t)n_out[3] * experts[3], m->blocks_per_row[3], nullptr);
+            m->total_bytes += bytes;
+            const hipError_t e = hipDeviceSynchronize();
+            if (e != hipSuccess) {
+                pf_set_error("tile-ordered weights", e);
+                pf_hip_moe_destroy(m);
+                return PF_HIP_E_RUNTIME;
+            }
+        } else {
+            (void)hipGetLastError();
+            m->w_mxtile = nullptr;
         }
     }
     // A streamed layer that is Q4_K throughout, or in the q4 checkpoint profile (Q4_K gate and up, MXFP4 down, Q8_0 shared

@@ -1,14 +1,13 @@
 // Prefill path: a chunk of tokens through one MoE layer as grouped matrix products on the
 // matrix cores.
 //
-//   pf_k_rows_to_half   f32 rows -> power-of-two scaled fp16 pairs (high + low part) and the
-//                       per-32-group sums, the scale, max^2, finite check
 //   pf_k_pf_router      router logits [T, E] by FP32 MFMA
-//   routing, grouping   the kernels of pf_moe_route.hip (serial-order re-route of close tokens,
-//                       histogram / scan / stable placement)
+//   routing             the kernels of pf_moe_route.hip (serial-order re-route of close tokens)
+//   pf_k_pf_group_rows  grouping of the pairs (pf_group_device.h); beside it f32 rows -> power-of-two scaled fp16
+//                       pairs (high + low part) and the per-32-group sums, the scale, finite check
 //   pf_k_pf_gemm        grouped product over the rows of each expert (the shared expert is
 //                       expert E with every token) on v_mfma_f32_32x32x16_f16; gate/up with
-//                       the SwiGLU epilogue, or down
+//                       the SwiGLU epilogue, or down (routed MXFP4 down rows: pf_moe_mx.hip)
 //   pf_k_pf_combine     slot-ordered weighted sum of the down rows, then the shared branch
 //
 // Numerics.  A Q4_K weight is d * (scale * code) - dmin * min (src/qwen4_packed.c:86-93) with
@@ -37,7 +36,7 @@ typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 __host__ __device__ constexpr size_t pf_half_row(int cols) { return 2 * (size_t)cols + 16 * (((size_t)cols + 255) / 256); }
 
 // ---- Q4_K tensors in tile order (once, at upload) ---------------------------------------------
-// The grouped product's loader moves one 32-row tile's share of a 256-block per instruction group.
+// A wave of the grouped product takes a 32-row tile's share of a 256-block at a time.
 // In GGUF row order that is 32 pieces a row pitch apart; here the same bytes are regrouped so that
 // it is 4608 consecutive bytes: [32 headers of 16 bytes][run 0..3: 16-byte halves 0 of the 32 rows,
 // then halves 1].  One thread per 16-byte piece; rows is a multiple of 32.
@@ -250,7 +249,7 @@ void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hip
 // ---- router logits by FP32 MFMA ----------------------------------------------------------------
 // Workgroup = a tile of 32 TR tokens x 32 TC experts, its eight waves an eighth of the columns each (the
 // partial tiles are added in wave order).  Also writes the routing tolerance's bound on the sum of
-// squared products, max(x)^2 * |w_e|^2.  (The shared router's logit comes from pf_k_rows_to_half.)
+// squared products, max(x)^2 * |w_e|^2.  (The shared router's logit comes with the rows' conversion.)
 //
 // Operands.  A product step wants, from lane (i, kk), element k = kk of row i: fetched like that
 // from global memory, every load instruction touches 32 rows, and the address unit, which takes a
@@ -872,10 +871,10 @@ __global__ void __launch_bounds__(256) pf_k_pf_scan_tiles(uint32_t *counts, int 
 }
 
 // ---- the grouped product for the other formats of real checkpoints --------------------------------
-// Q8_0 (shared expert), Q2_K and MXFP4 (routed down projections) have no operand path in the ring
-// kernel above.  This kernel computes the same items with the same operands' arithmetic (exact
+// Q2_K, and MXFP4 and Q8_0 where the kernels made for them do not apply, have no operand path in the kernel
+// above.  This kernel computes the same items with the same operands' arithmetic (exact
 // integer weight operands in fp16, two-part fp16 activations, FP32 accumulation, scales applied to
-// the partial sums in FP32) but without the LDS ring: a workgroup is one row tile against one slab
+// the partial sums in FP32): a workgroup is one row tile against one slab
 // of 4 x 32 (gate/up) or 4 x 64 (down) weight rows, a wave takes its operands straight from global
 // memory (the activation fragments are shared through the caches by the four waves and the slabs).
 // Group scales that are not integers (Q8_0: a half per 32 weights; MXFP4: a power of two per 32)
@@ -1103,8 +1102,8 @@ __device__ __forceinline__ void plain_passes(const PlainTile &a, const PlainRow 
 // which: all items of the list, the shared expert's (the grid: its tiles alone), or the routed experts'.
 enum { PLAIN_ALL, PLAIN_SHARED, PLAIN_ROUTED };
 
-// grid: (row tiles the list can hold) x slabs; 4 waves.  Items whose tensors are in a format of the ring
-// kernel are skipped here, as the ring kernel skips these.
+// grid: (row tiles the list can hold) x slabs; 4 waves.  Items whose tensors are in a format of pf_k_pf_gemm
+// are skipped here, as that kernel skips these.
 // split != 0 (gate/up only): the four waves share 32 units and take a quarter of the columns each; their
 // partial sums meet in LDS and wave 0 adds them in wave order.  For matrices with few row tiles (the
 // shared expert) that gives four times as many workgroups.
@@ -1245,14 +1244,14 @@ __global__ void __launch_bounds__(PF_ROW_THREADS) pf_k_pf_combine(PfKernelArgs a
 }
 
 // ---- dispatch --------------------------------------------------------------------------------------
-// Routed gate and up in Q4_K or IQ2_XXS (the ring kernel's operand paths); the routed down tensor and the
-// shared expert's three tensors in that same format or in Q2_K, MXFP4, Q8_0 (the plain grouped product).
+// Routed gate and up in Q4_K or IQ2_XXS (pf_k_pf_gemm's operand paths); the routed down tensor and the
+// shared expert's three tensors in that same format or in Q2_K, MXFP4, Q8_0.
 bool pf_prefill_supported(const PfHipMoeDesc &d) {
     const uint32_t g = d.type[1];
     auto covered = [&](uint32_t t) { return t == g || t == PF_Q8_0 || t == PF_Q2_K || t == PF_MXFP4; };
     if ((g != PF_Q4_K && g != PF_IQ2_XXS) || d.type[2] != g || !covered(d.type[3])) return false;
     if (d.type[5] != d.type[4] || !covered(d.type[4]) || !covered(d.type[6])) return false;
-    // widths: whole 256-blocks where the ring kernel reads them; where the plain kernel takes a down projection, whole
+    // widths: whole 256-blocks where pf_k_pf_gemm reads the gate's format; where the plain kernel takes a down projection, whole
     // 128-column halves (the checkpoints' 640), and only Q2_K may be stored wider than its logical width
     auto width_ok = [&](uint32_t type, uint32_t k) { return k % (type == g ? 256u : 128u) == 0; };
     if (d.hidden % 256 || d.inter % 32 || d.shared_inter % 32 || !width_ok(d.type[3], d.inter) || !width_ok(d.type[6], d.shared_inter))
@@ -1342,10 +1341,10 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     }
     if (last < 3) return;
     // stage 3: gate/up + SwiGLU, then fp16 parts of the activation rows
-    // the ring kernel takes the items whose tensors are in the routed gate's format, the plain kernel the rest
+    // pf_k_pf_gemm takes the items whose tensors are in the routed gate's format and the Q8_0 shared expert, the plain kernel the rest
     const int gi = I > Is ? I : Is;
     const bool iq2 = a.type[1] == PF_IQ2_XXS;
-    const uint32_t ring_fmt = a.type[1];
+    const uint32_t gate_fmt = a.type[1];
     const unsigned tile_cap = (unsigned)pf_prefill_max_tiles(tokens, E, K);
     const bool q8 = a.type[4] == PF_Q8_0;   // the shared expert of the checkpoint profiles
     if (iq2 && q8) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS, PF_Q8_0>(a, tile_cap, gi, H, 0, stream);
@@ -1353,7 +1352,7 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     else if (q8) launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q8_0>(a, tile_cap, gi, H, 0, stream);
     else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q4_K>(a, tile_cap, gi, H, 0, stream);
     // only the shared expert's tiles (tokens / 32 of them) are left for this launch: columns split over the waves
-    if (a.type[4] != ring_fmt && !q8) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, PLAIN_SHARED, stream);
+    if (a.type[4] != gate_fmt && !q8) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, PLAIN_SHARED, stream);
     const int widest = I > Is ? I : Is;
     const bool digits = a.wm && widest <= 1024;   // the routed rows as digits
     if (widest <= 1024 && P > 0 && tokens > 0) {
@@ -1368,12 +1367,12 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     }
     if (last < 4) return;
     // stage 4: down and combine
-    if (a.type[3] == ring_fmt || a.type[6] == ring_fmt) {
+    if (a.type[3] == gate_fmt || a.type[6] == gate_fmt) {
         if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS, PF_IQ2_XXS>(a, tile_cap, H, gi, 0, stream);
         else launch_gemm<PF_GEMM_DOWN, PF_Q4_K, PF_Q4_K>(a, tile_cap, H, gi, 0, stream);
     }
     if (digits) pf_launch_mx_down(a, tile_cap, stream);
-    const bool plain_routed = a.type[3] != ring_fmt && !digits, q8_shared = a.type[6] == PF_Q8_0, plain_shared = a.type[6] != ring_fmt && !q8_shared;
+    const bool plain_routed = a.type[3] != gate_fmt && !digits, q8_shared = a.type[6] == PF_Q8_0, plain_shared = a.type[6] != gate_fmt && !q8_shared;
     if (plain_routed || plain_shared)
         launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, plain_routed ? tile_cap : (unsigned)((tokens + 31) / 32), (H + 255) / 256, 0,
                                         !plain_routed ? PLAIN_SHARED : q8_shared ? PLAIN_ROUTED : PLAIN_ALL, stream);
