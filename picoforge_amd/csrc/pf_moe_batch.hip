@@ -6,7 +6,8 @@
 // weights come from memory once, and once in registers serve eight rows at a time.
 //
 //   pf_k_batch_gate_up   gate and up products of 32 units, SwiGLU, the activation rows' digit images (expert order)
-//   pf_k_batch_down      down products of 128 output rows, FP32, in expert order (pf_k_pf_combine adds them up)
+//   pf_k_batch_down      down products of 128 output rows, FP32, in expert order (pf_k_pf_combine adds them up); of the q4
+//                        profile with a tile-ordered copy the shared expert's only, the routed ones by pf_k_mx_down
 //
 // Arithmetic: the decode kernels'.  Activations are digit images (integers per 32-group as balanced base-256 digits), weight
 // codes signed bytes, the group's dot product exact in integers, the group's scale and minimum applied in FP32.  PLANES digits:
@@ -158,34 +159,21 @@ template <bool ROWS> struct BatchRows<PF_Q8_0, ROWS> {   // the checkpoint profi
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
 };
 
-template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // in tile order, else row by row: a lane reads its row's whole block and keeps the low or the high nibbles
+template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // row by row: a lane reads its row's whole block and keeps the low or the high nibbles
     static constexpr int GROUPS = 8;
     static constexpr bool MINIMA = false, MIN_OPERAND = false;
     uint4 q[8];
-    uint32_t e2[ROWS ? 4 : 2];
+    uint32_t e2[4];
     __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane, const uint32_t *) {
-        if constexpr (!ROWS) {
-            const int units = groups / 4;
-            const uint8_t *rows = a.wm + e * pf_mxt_expert_bytes(a.n_out[t], units) + (size_t)tile * units * PF_I2T_CHUNK;   // uniform
-            const uint32_t code_at = 16 * (uint32_t)(lane & 31), scale_at = 4 * (uint32_t)(lane & 31);
+        const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
+        const uint8_t *codes = a.w[t] + row0 * a.row_bytes[t], *scales = a.w[t] + a.scale_offset[t] + row0 * (size_t)a.blocks_per_row[t];
+        const uint32_t code_at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t], scale_at = (uint32_t)(lane & 31) * (uint32_t)a.blocks_per_row[t];
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const uint8_t *chunk = rows + (size_t)min(2 * piece + u, units - 1) * PF_I2T_CHUNK;
-#pragma unroll
-                for (int g = 0; g < 4; g++) q[4 * u + g] = *reinterpret_cast<const uint4 *>((chunk + 512 * g) + code_at);
-                e2[u] = *reinterpret_cast<const uint32_t *>((chunk + 2048) + scale_at);
-            }
-        } else {
-            const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
-            const uint8_t *codes = a.w[t] + row0 * a.row_bytes[t], *scales = a.w[t] + a.scale_offset[t] + row0 * (size_t)a.blocks_per_row[t];
-            const uint32_t code_at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t], scale_at = (uint32_t)(lane & 31) * (uint32_t)a.blocks_per_row[t];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int g = min(GROUPS * piece + 2 * r, groups - 2);
-                q[2 * r] = *reinterpret_cast<const uint4 *>((codes + 16 * g) + code_at);
-                q[2 * r + 1] = *reinterpret_cast<const uint4 *>((codes + 16 * (g + 1)) + code_at);
-                e2[r] = *reinterpret_cast<const uint16_t *>((scales + g) + scale_at);
-            }
+        for (int r = 0; r < 4; r++) {
+            const int g = min(GROUPS * piece + 2 * r, groups - 2);
+            q[2 * r] = *reinterpret_cast<const uint4 *>((codes + 16 * g) + code_at);
+            q[2 * r + 1] = *reinterpret_cast<const uint4 *>((codes + 16 * (g + 1)) + code_at);
+            e2[r] = *reinterpret_cast<const uint16_t *>((scales + g) + scale_at);
         }
     }
     __device__ __forceinline__ void open() {}
@@ -194,9 +182,7 @@ template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // in tile order, else
         return int4v{e2m1_twice4(q[g].x >> s), e2m1_twice4(q[g].y >> s), e2m1_twice4(q[g].z >> s), e2m1_twice4(q[g].w >> s)};
     }
     __device__ __forceinline__ int4v min_operand(int) const { return int4v{0, 0, 0, 0}; }
-    __device__ __forceinline__ float scale(int g) const {    // the integers are twice the values
-        return 0.5f * pf_e8m0_scale(ROWS ? (e2[g >> 1] >> (8 * (g & 1))) & 255u : (e2[g >> 2] >> (8 * (g & 3))) & 255u);
-    }
+    __device__ __forceinline__ float scale(int g) const {  return 0.5f * pf_e8m0_scale((e2[g >> 1] >> (8 * (g & 1))) & 255u); }   // the integers are twice the values
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
 };
 
@@ -366,7 +352,7 @@ struct BatchItem {
     int token0;           // shared expert: the first row's token
     size_t e;             // where the expert's weights are: its id, or its pool slot
 };
-__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t tile, BatchItem &it) {
+__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t tile, BatchItem &it) {   // false: no such item
     const uint32_t count = a.tiles[0];
     const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[tile];   // {expert, first row, rows, first row within the expert}
     if (tile >= count) return false;
@@ -486,6 +472,13 @@ template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t
 // them), the operands past the registers through LDS (slower: LDS becomes the bottleneck for
 // IQ2_XXS), one matrix a wave at twice the occupancy (85 us).
 #define BATCH_WAVES 4
+// The q4 profile's routed down projection runs on the block-scaled product (pf_k_mx_down), as a chunk's, where the layer keeps that
+// copy: its activation rows leave the gate and up kernel as FP32 and become digit rows.  On the integers 101 tokens of the checkpoints'
+// widths took 157 us row by row and 120 from the copy; now 84, 7 for the rows and 14 for the shared expert's down projection.  24
+// tokens 77 -> 39 + 5 + 12, 300 tokens 229 -> 98 + 9 + 23.
+template <int FMT, int FMTS, int PLANES> __host__ __device__ __forceinline__ bool batch_down_scaled(const PfKernelArgs &a) {
+    return FMT == PF_Q4_K && FMTS == PF_Q8_0 && PLANES == 3 && a.wm != nullptr;
+}
 template <int FMT, int FMTS, bool ROWS, int PLANES>
 __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a) {
     __shared__ float partial[BATCH_WAVES][2][4][64];
@@ -500,6 +493,7 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
     const int groups = a.hidden / 32, K = a.top_k;
     const uint32_t words = (uint32_t)pf_batch_image_words(PLANES, a.hidden);
     const size_t act_words = pf_batch_image_words(PLANES, a.inter > a.shared_inter ? a.inter : a.shared_inter);
+    const bool rows_only = batch_down_scaled<FMT, FMTS, PLANES>(a) && !it.shared;   // the down projection takes digit rows
     for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         float acc[2][4] = {};
@@ -528,7 +522,12 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
             const float act = pf_silu(gate) * up;
             const int r = 2 * q + (lane >> 5);
             if (r < rows && !pf_finite(act)) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
-            batch_image_group<PLANES>(a.aimg + (size_t)(it.first + c0 + min(r, rows - 1)) * act_words, act, tile, I, lane, r < rows);
+            const size_t row = (size_t)(it.first + c0 + min(r, rows - 1));
+            if (rows_only) {
+                if (r < rows) a.act[row * I + 32 * tile + (lane & 31)] = act;
+            } else {
+                batch_image_group<PLANES>(a.aimg + row * act_words, act, tile, I, lane, r < rows);
+            }
         }
         if (c0 + BATCH_ROWS < it.rows) __syncthreads();   // the sums have been read
     }
@@ -548,16 +547,17 @@ __device__ __forceinline__ void batch_stage_rows(uint32_t *stage, const PfKernel
 }
 
 // blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert.  Bound by the products' chain of a wave
-// (with the weights in a cache 90 us of 104 for Q2_K, 97 of 120 for MXFP4, 101 tokens); MXFP4 took 157 us from rows, whose
-// 16-byte blocks are a line each, and takes 120 from the tile-ordered copy that the grouped product keeps.
+// (with the weights in a cache 90 us of 104 for Q2_K, 101 tokens).
+// last: the list's last items, the shared expert's, a chunk of rows a workgroup (blockIdx.z): alone in a launch a
+// tile's four chunks one after the other took 35 us, side by side 14 (101 tokens).
 template <int FMT, int FMTS, bool ROWS, int PLANES>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, int last) {
     constexpr bool STAGED = FMT == PF_Q2_K && !ROWS;
     __shared__ BatchFactor factors[4][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
     __shared__ __align__(16) uint32_t staged[STAGED ? 4 : 1][STAGED ? 2048 : 4];
     BatchItem it;
-    if (!batch_item(a, blockIdx.y, it)) return;
+    if (!batch_item(a, last ? a.tiles[0] - 1 - blockIdx.y : blockIdx.y, it)) return;
     if (batch_tables<FMT>()) batch_stage_tables(tables, a);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), H = a.hidden;
     const int tile = 4 * blockIdx.x + wave;
@@ -570,7 +570,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) p
         __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the wave's own copy is there
         pf_wave_lds_fence();
     }
-    for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
+    for (int c0 = BATCH_ROWS * blockIdx.z; c0 < it.rows; c0 += BATCH_ROWS * gridDim.z) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         auto image_at = [&](int r) { return (uint32_t)(it.first + c0 + r) * words; };
         float acc[1][4] = {};
@@ -702,13 +702,18 @@ static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile
     const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
     hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a);
     if (last < 4) return;
-    // down rows: as gate and up where the layer has one format; MXFP4 in tile order where the layer keeps that copy (resident
-    // ones), Q2_K by whole tiles where they fit a wave's LDS
     const dim3 grid((a.hidden + 127) / 128, tile_cap);
-    constexpr bool either = FD == PF_Q2_K || (FD == PF_MXFP4 && PLANES == 3);
-    const bool other = FD == PF_Q2_K ? 32 * a.row_bytes[3] <= BATCH_STAGE_BYTES : a.wm != nullptr;
-    if (either && other) hipLaunchKernelGGL((pf_k_batch_down<FD, FS, either ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a);
+    if (FD == PF_MXFP4 && batch_down_scaled<FG, FS, PLANES>(a)) {
+        pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
+        pf_launch_mx_down(a, tile_cap, stream);
+        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, (tokens + 31) / 32, 32 / BATCH_ROWS), dim3(256), 0, stream, a, 1);
+        return;
+    }
+    // down rows: as gate and up where the layer has one format; Q2_K by whole tiles where they fit a wave's LDS
+    constexpr bool q2 = FD == PF_Q2_K;
+    if (q2 && 32 * a.row_bytes[3] <= BATCH_STAGE_BYTES)
+        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, q2 ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, 0);
+    else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, 0);
 }
 
 template <int FG, int FD, int FS>

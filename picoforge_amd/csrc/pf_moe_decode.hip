@@ -1721,11 +1721,6 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FMT =
 
 // ---- kernel 3 of the q4 profile for batches: the block-scaled matrix instruction ----------------------
 #if PF_DECODE_PART == 3
-// The activation rows as digit rows (pf_mx_rows.h), in place.
-__global__ void __launch_bounds__(256) pf_k_dec_rows_to_digits(PfKernelArgs a, size_t rows) {
-    pf_rows_to_digits(blockIdx.x, a.act, a.inter, rows, reinterpret_cast<uint32_t *>(a.act), nullptr, a.error_word);
-}
-
 // A workgroup takes 32 output rows of one token, a wave per slot, then two for the shared expert's rows of 16.
 // v_mfma_scale_f32_16x16x128_f8f6f4: a unit of 128 columns an instruction, the five planes of the slot's digit row as rows 0..4 of the
 // left operand (rows beyond repeat the last and are not looked at), 16 weight rows as MXFP4 stores them on the right: no vector
@@ -1817,8 +1812,7 @@ static bool down_mx_applies(const PfKernelArgs &a, int tokens) {
     return tokens >= DOWN_MX_FROM && a.wm && a.top_k + 2 <= 16;   // at most 1024 threads
 }
 static void launch_down_mx(const PfKernelArgs &a, int tokens, hipStream_t stream) {
-    const size_t rows = (size_t)tokens * a.top_k, block = 4 * pf_mx_rows_a_wave(a.inter);
-    hipLaunchKernelGGL(pf_k_dec_rows_to_digits, dim3((unsigned)((rows + block - 1) / block)), dim3(256), 0, stream, a, rows);
+    pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act), nullptr, a.error_word, stream);   // in place
     switch (a.inter / 128) {
     case 1: launch_down_mx_units<1>(a, tokens, stream); break;
     case 2: launch_down_mx_units<2>(a, tokens, stream); break;

@@ -20,7 +20,7 @@ struct PfKernelArgs {
     const uint8_t *wt[8];            // Q4_K expert tensors in tile order for the grouped product (null: not kept)
     const uint8_t *wi[8];            // IQ2_XXS expert tensors in tile order for the decode kernels (null: not kept)
     const uint8_t *wq[8];            // Q8_0 tensors (the profiles' shared gate and up) in tile order (null: not kept)
-    const uint8_t *wm;               // the routed down tensor, MXFP4, in tile order for the grouped product and the few-row kernels (null: not kept)
+    const uint8_t *wm;               // the routed down tensor, MXFP4, in tile order for the block-scaled products (null: not kept)
     const float *router_t;           // router as [slab of 64 experts][hidden / 4][64][4] (serial-order re-routing)
     const uint64_t *iq2_grid;        // 256 x 8 magnitudes, device memory
     const uint32_t *iq2_signed;      // 2 x 4096 words: four signed magnitudes per (grid entry, sign nibble)
@@ -281,6 +281,7 @@ int pf_prefill_max_tiles(int tokens, int experts, int top_k);
 size_t pf_prefill_most_tokens(int hidden);   // that one launch of pf_launch_prefill takes
 // pf_moe_mx.hip: the routed MXFP4 down projection of a chunk, from rows of digits (pf_mx_rows.h) instead of halfs
 bool pf_mx_down_takes(const PfHipMoeDesc &d);
+void pf_launch_rows_to_digits(const float *d_src, int cols, size_t rows, uint32_t *d_dst, float *d_scales, uint32_t *d_error, hipStream_t stream);
 void pf_launch_mx_tile(const uint8_t *d_payload, const uint8_t *d_scales, uint8_t *d_dst, size_t rows, int blocks_per_row, hipStream_t stream);
 void pf_launch_mx_down(const PfKernelArgs &a, unsigned tile_cap, hipStream_t stream);
 // pf_moe_batch.hip: a few rows per expert, for the layers of the tile decode kernels

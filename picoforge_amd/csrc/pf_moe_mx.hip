@@ -151,3 +151,12 @@ void pf_launch_mx_down(const PfKernelArgs &a, unsigned tile_cap, hipStream_t str
     default: launch<5>(a, tiles, stream); break;
     }
 }
+
+// Activation rows as digit rows, for batches (a chunk's come with the shared expert's halfs).  dst may be src; scales may be null.
+__global__ void __launch_bounds__(256) pf_k_rows_to_digits(const float *src, int cols, size_t rows, uint32_t *dst, float *scales, uint32_t *error_word) {
+    pf_rows_to_digits(blockIdx.x, src, cols, rows, dst, scales, error_word);
+}
+void pf_launch_rows_to_digits(const float *d_src, int cols, size_t rows, uint32_t *d_dst, float *d_scales, uint32_t *d_error, hipStream_t stream) {
+    const size_t block = 4 * (size_t)pf_mx_rows_a_wave(cols);
+    if (rows) hipLaunchKernelGGL(pf_k_rows_to_digits, dim3((unsigned)((rows + block - 1) / block)), dim3(256), 0, stream, d_src, cols, rows, d_dst, d_scales, d_error);
+}
