@@ -1099,8 +1099,8 @@ __device__ __forceinline__ void plain_passes(const PlainTile &a, const PlainRow 
                   [&](int k0, int cols) { plain_product(w, ahi, alo, a.sums + (size_t)n * PLAIN_SUMS, 32 * PLAIN_SUMS, k0, cols, h, acc); });
 }
 
-// which: all items of the list, the shared expert's (the grid: its tiles alone), or the routed experts'.
-enum { PLAIN_ALL, PLAIN_SHARED, PLAIN_ROUTED };
+// which: all items of the list, or the shared expert's (the grid: its tiles alone).
+enum { PLAIN_ALL, PLAIN_SHARED };
 
 // grid: (row tiles the list can hold) x slabs; 4 waves.  Items whose tensors are in a format of pf_k_pf_gemm
 // are skipped here, as that kernel skips these.
@@ -1121,7 +1121,6 @@ __global__ void __launch_bounds__(256) pf_k_pf_gemm_plain(PfKernelArgs a, int to
     const uint32_t entry = a.tiles[1 + item_tile];
     const int expert = entry & 0xffffu, m0 = 32 * (int)(entry >> 16);
     const bool shared = expert == E;
-    if (which == PLAIN_ROUTED && shared) return;
     const int first = shared ? P : (int)a.offsets[expert];
     const int count = shared ? tokens : (int)a.offsets[expert + 1] - first;
     if (count <= m0) return;
@@ -1372,10 +1371,13 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
         else launch_gemm<PF_GEMM_DOWN, PF_Q4_K, PF_Q4_K>(a, tile_cap, H, gi, 0, stream);
     }
     if (digits) pf_launch_mx_down(a, tile_cap, stream);
-    const bool plain_routed = a.type[3] != gate_fmt && !digits, q8_shared = a.type[6] == PF_Q8_0, plain_shared = a.type[6] != gate_fmt && !q8_shared;
+    // (beside routed items of the plain kernel a Q8_0 shared expert's cost nothing: in a launch of its own it made the down stage of
+    // the q2 profile's 1024-token chunk 169 us instead of 157, at the checkpoints' widths 291 instead of 271)
+    const bool plain_routed = a.type[3] != gate_fmt && !digits, q8_shared = a.type[6] == PF_Q8_0 && !plain_routed;
+    const bool plain_shared = a.type[6] != gate_fmt && !q8_shared;
     if (plain_routed || plain_shared)
         launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, plain_routed ? tile_cap : (unsigned)((tokens + 31) / 32), (H + 255) / 256, 0,
-                                        !plain_routed ? PLAIN_SHARED : q8_shared ? PLAIN_ROUTED : PLAIN_ALL, stream);
+                                        plain_routed ? PLAIN_ALL : PLAIN_SHARED, stream);
     if (q8_shared) launch_gemm<PF_GEMM_DOWN, PF_Q8_0, PF_Q8_0>(a, tile_cap, H, Is, tokens, stream);
     pf_launch_combine(a, tokens, stream);
 }
