@@ -3,6 +3,7 @@
 #include "pf_moe_debug.h"
 #include "pf_host_calls.h"
 #include "pf_host_rows.h"
+#include "pf_piece_order.h"
 #include "../../include/pf_iq2_codes.h"
 #include <stdio.h>
 #include <stdlib.h>
@@ -553,6 +554,13 @@ __global__ void pf_k_copy_rows(const uint4 *src, uint4 *dst, int n) {
 // its own that nothing overlaps, 5.5 us beside the 10 to 14 of 512 KB.  A fence in every wave instead of one for 16 KB makes them
 // 20.)  A call of 777 tokens of width 2048 829 -> 760 us, of 1024 of width 2560 1280 -> 1190.  arrived: zero between the launches,
 // which follow each other on one stream.
+struct PieceOps {
+    uint32_t *arrived, *word;
+    __device__ void fence() { __threadfence_system(); }
+    __device__ uint32_t arrive() { return __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ void clear() { __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ void publish(uint32_t number) { __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+};
 __global__ void __launch_bounds__(256) pf_k_copy_piece(const uint4 *src, uint4 *dst, int n, uint32_t *arrived, uint32_t *word, uint32_t number, int out) {
     const int i0 = (int)(blockIdx.x * 1024 + threadIdx.x);   // four loads on their way, and a fence for 16 KB
     uint4 v[4];
@@ -564,10 +572,7 @@ __global__ void __launch_bounds__(256) pf_k_copy_piece(const uint4 *src, uint4 *
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the wave's own stores have been taken
     __syncthreads();
     if (threadIdx.x != 0) return;
-    if (out) __threadfence_system();   // in: a stored value has been read, and only the stream's next kernel looks at it
-    if (__hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
-    __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    pf_piece_done(PieceOps{arrived, word}, gridDim.x, number, out != 0);
 }
 struct PublishParts { const uint32_t *src[3]; uint32_t *dst[3]; int words[3]; };
 // One workgroup: the parts, then (everything before it has reached the host's memory) the call's number.
