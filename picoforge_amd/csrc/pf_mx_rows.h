@@ -1,10 +1,12 @@
 // Digit rows: the activation rows of the MXFP4 down projection as operands of v_mfma_scale_f32_32x32x64_f8f6f4 (pf_moe_mx.hip).
 //
-// A row is divided by a power of two so that its largest magnitude lies in [0.5, 1).  Per group of 32 values with largest
+// A row whose largest magnitude m is outside [2^-61, 2^60) is divided by the power of two that brings it there, other rows are taken
+// as they are: a product with a block scale of 2^125 or 2^-127 is then no larger or smaller on its way than the result.  (Rows
+// divided down to [0.5, 1) overflowed on scales that small rows made up for.)  Per group of 32 values with largest
 // magnitude below 2^E, plane p is what planes 0 .. p - 1 leave, rounded to a six-bit float (two exponent, three mantissa bits)
 // times 2^(E - 2 - 5 p): a remainder is below 4 of its plane's steps, the rounding leaves an eighth of a step at most, so five planes
 // leave 2^-25 of the binade of the group's largest magnitude (the two-part halfs of the other grouped products: 2^-23 of the
-// value, and not under 2^-25 of the row's).
+// value, and not under 2^-25 of the row's).  E is -100 at least, 39 binades under the smallest m.
 //
 // 128 bytes a group: 16 bytes of each plane's 24 (chunks 0..4), the planes' other 8 bytes, then the five scale bytes, the
 // row's exponent and padding.  A slot order within the group that follows MXFP4's nibbles: slot 2 i is column i, slot 2 i + 1 column 16 + i.
@@ -57,9 +59,9 @@ __device__ __forceinline__ void pf_rows_to_digits(size_t block, const float *src
     float m = most;   // of the row: each step doubles the groups, in a ring, that a lane has seen
 #pragma unroll
     for (int d = 1; d < 32; d <<= 1) m = fmaxf(m, __shfl(m, at * groups + (group + d) % groups));
-    int e = (__float_as_int(m) >> 23) & 255;                  // m in [2^(e-127), 2^(e-126))
-    e = (e == 0 || e == 255) ? 126 : min(e, 252);             // zero, subnormal or nonfinite row: scale 1
-    const float inv = __int_as_float((253 - e) << 23);        // 2^(126-e)
+    const int binade = ((__float_as_int(m) >> 23) & 255) - 126;   // m in [2^(binade-1), 2^binade); a nonfinite row: 129
+    const int shift = max(binade - 60, min(binade + 60, 0));
+    const float inv = __int_as_float((127 - shift) << 23);
     const int E = max(((__float_as_int(most * inv) >> 23) & 255) - 126, -100);
 #pragma unroll
     for (int i = 0; i < 16; i++) { a[i] *= inv; b[i] *= inv; }
@@ -74,12 +76,12 @@ __device__ __forceinline__ void pf_rows_to_digits(size_t block, const float *src
         for (int i = 0; i < 16; i++) { a[i] -= back[2 * i]; b[i] -= back[2 * i + 1]; }
     }
     if (!mine) return;
-    if (group == 0 && scale_out) scale_out[row] = __int_as_float((e + 1) << 23);
+    if (group == 0 && scale_out) scale_out[row] = __int_as_float((127 + shift) << 23);
     uint4v *line = reinterpret_cast<uint4v *>(dst + row * cols + 32 * group);
 #pragma unroll
     for (int p = 0; p < PF_MX_PLANES; p++) line[p] = uint4v{plane[p][0], plane[p][1], plane[p][2], plane[p][3]};
     line[5] = uint4v{plane[0][4], plane[0][5], plane[1][4], plane[1][5]};
     line[6] = uint4v{plane[2][4], plane[2][5], plane[3][4], plane[3][5]};
     const uint32_t s0 = (uint32_t)(127 + E - 2);   // plane p: 5 p less
-    line[7] = uint4v{plane[4][4], plane[4][5], s0 * 0x01010101u - 0x0F0A0500u, (s0 - 20u) | (uint32_t)(e + 1) << 8};
+    line[7] = uint4v{plane[4][4], plane[4][5], s0 * 0x01010101u - 0x0F0A0500u, (s0 - 20u) | (uint32_t)(127 + shift) << 8};
 }

@@ -229,3 +229,31 @@ def test_prefill_kernels_with_a_q2k_shared_expert(product, oracle, h, gtype):
         for tokens in (5, 37):
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"h={h} T={tokens}")
+
+
+@pytest.mark.parametrize("x_scale,exponent", [(2.0 ** -30, 252), (2.0 ** 20, 0), (2.0 ** 20, 3)])
+def test_mxfp4_down_scales_near_the_ends_of_their_range(product, oracle, x_scale, exponent):
+    """Block scales of 2^125, 2^-127 and 2^-124 against activation rows small or large enough that every product and the result are
+    ordinary numbers, on each kernel family's batches (the shared expert, of ordinary scales, adds nothing: its down rows are zero)."""
+    print(f"case mxfp4 scales 2^{exponent - 127}, activations times {x_scale}", flush=True)
+    cfg = abi.moe_config(512, 24, 3, 256, 256)
+    weights, x = make_layer_inputs(cfg, "q4", 40, seed=exponent + 5)
+    blocks = weights.raw[3].reshape(-1, 17)
+    blocks[:, 0] = exponent
+    weights.raw[6].reshape(-1, 34)[:, :2] = 0
+    x *= np.float32(x_scale)
+    want = forward_with(oracle, cfg, weights, x)
+    assert np.isfinite(want[0]).all() and (np.abs(want[0]).max(axis=1) > 2.0 ** -120).all()
+    largest = np.abs(want[0]).max(axis=1, keepdims=True)
+    with pf.MoeLayer(product, cfg, weights, 40) as layer:
+        for tokens, family in ((1, 1), (4, 1), (5, 1), (16, 1), (17, 3), (40, 3), (40, 2), (40, 0)):
+            print(f"  tokens={tokens} family={family}", flush=True)
+            layer.force_grouped(family == 2)
+            layer.force_general(family == 0)
+            assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == family
+            _, y, ids, w = layer.forward(x[:tokens])
+            np.testing.assert_array_equal(ids, want[1][:tokens])
+            np.testing.assert_allclose(w, want[2][:tokens], atol=2e-6, rtol=2e-5)
+            error = np.abs(y.astype(np.float64) - want[0][:tokens]).max(axis=1)
+            print(f"    error {(error / largest[:tokens, 0]).max():.2e} of the row's largest", flush=True)
+            assert (error <= 1e-5 * largest[:tokens, 0]).all()   # 32-bit sums of 256 products and three slots
