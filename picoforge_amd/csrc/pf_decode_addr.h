@@ -155,11 +155,21 @@ PF_HD size_t pf_i2t_chunk_at(size_t expert_bytes, size_t e, int row_tile, int kb
 PF_HD size_t pf_i2t_scale_at(int row_in_tile) { return 2048 + 2 * (size_t)row_in_tile; }
 PF_HD size_t pf_i2t_piece_at(int run, int row_in_tile) { return (size_t)run * 512 + 16 * (size_t)row_in_tile; }
 
-// ---- tile-ordered MXFP4 (the routed down projection, for the grouped product; 32 rows x one unit of 128 weights = 2176 bytes:
+// ---- tile-ordered MXFP4 (the routed down projection, in place of its rows; 32 rows x one unit of 128 weights = 2176 bytes:
 // the rows' 16-byte blocks, block by block, then the rows' four scale bytes each) ----
 PF_HD size_t pf_mxt_expert_bytes(int n_out, int units) { return (size_t)(n_out / 32) * units * PF_I2T_CHUNK; }
 PF_HD size_t pf_mxt_piece_at(int block, int row_in_tile) { return (size_t)block * 512 + 16 * (size_t)row_in_tile; }
 PF_HD size_t pf_mxt_scales_at(int row_in_tile) { return 2048 + 4 * (size_t)row_in_tile; }
+// a lane's 64-weight segment of row n of an expert, as pf_segment_spans gives it, from the expert's start: two blocks, then their two
+// scale bytes
+struct PfSpan32 { uint32_t at, width; };
+PF_HD void pf_mxt_segment_spans(int units, int n, int seg, PfSpan32 out[3]) {
+    const uint32_t chunk = (uint32_t)((n >> 5) * units + (seg >> 1)) * PF_I2T_CHUNK;
+    const int row_in_tile = n & 31, block = 2 * (seg & 1);
+    out[0] = {chunk + (uint32_t)pf_mxt_piece_at(block, row_in_tile), 16};
+    out[1] = {chunk + (uint32_t)pf_mxt_piece_at(block + 1, row_in_tile), 16};
+    out[2] = {chunk + (uint32_t)pf_mxt_scales_at(row_in_tile) + (uint32_t)block, 2};
+}
 
 // ---- tile-ordered Q8_0 (the shared expert of the checkpoint profiles; 32 rows x one 64-weight run = 2176 bytes: the
 // rows' 64 code bytes as four 16-byte pieces, piece by piece, then the rows' two half scales each, then padding) ----

@@ -311,20 +311,26 @@ extern "C" int pf_hip_moe_create(const PfHipMoeDesc *desc, const void *const hos
             }
         }
     }
-    // The routed MXFP4 down tensor in tile order, for the block-scaled products and the few-row kernels.  Where there is no
-    // memory left for it they read the rows (a layer that fits without the copy is not refused for it).
-    if (m->prefill_ready && pf_mx_down_takes(*desc)) {
+    // The routed MXFP4 down tensor in tile order, which every kernel family reads, in place of its rows: a layer takes no more
+    // memory for it.  Where there is none left for the two while the one is made from the other, and with PF_MOE_PREFILL_COPY=0,
+    // the rows stay.
+    // (The decode kernels on segments of rows read the rows: no layer of these widths runs them with the other copies kept.)
+    const bool segments = m->decode_ready && pf_decode_tile_layer(m->desc, m->w_tiled, m->w_itile, m->w_qtile) == 0;
+    if (m->prefill_ready && !segments && pf_mx_down_takes(*desc)) {
         const char *copy = getenv("PF_MOE_PREFILL_COPY");
         const size_t bytes = pf_mxt_expert_bytes((int)n_out[3], m->blocks_per_row[3] / 4) * experts[3];
         if ((!copy || strcmp(copy, "0") != 0) && hipMalloc((void **)&m->w_mxtile, bytes) == hipSuccess) {
             pf_launch_mx_tile(m->w[3], m->w[3] + m->scale_offset[3], m->w_mxtile, (size_t)n_out[3] * experts[3], m->blocks_per_row[3], nullptr);
-            m->total_bytes += bytes;
             const hipError_t e = hipDeviceSynchronize();
             if (e != hipSuccess) {
                 pf_set_error("tile-ordered weights", e);
                 pf_hip_moe_destroy(m);
                 return PF_HIP_E_RUNTIME;
             }
+            (void)hipFree(m->w[3]);
+            m->w[3] = nullptr;
+            m->total_bytes += bytes;
+            m->total_bytes -= m->bytes[3];
         } else {
             (void)hipGetLastError();
             m->w_mxtile = nullptr;

@@ -191,8 +191,15 @@ __device__ __forceinline__ void wseg_load<PF_Q8_0>(WSeg<PF_Q8_0> &w, const PfKer
     w.d2 = *reinterpret_cast<const uint32_t *>(a.w[t] + sp[1].at);
 }
 
-// MXFP4, device layout (16 nibble bytes per block, scale bytes apart): a segment is two blocks
+// MXFP4, device layout (16 nibble bytes per block, scale bytes apart) and in tile order: a segment is two blocks
 template <> struct WSeg<PF_MXFP4> { uint4 q[2]; uint32_t e2; };
+__device__ __forceinline__ void wseg_load_tiled(WSeg<PF_MXFP4> &w, const uint8_t *expert, int units, int n, int seg) {
+    PfSpan32 sp[3];
+    pf_mxt_segment_spans(units, n, seg, sp);
+    w.q[0] = *reinterpret_cast<const uint4 *>(expert + sp[0].at);
+    w.q[1] = *reinterpret_cast<const uint4 *>(expert + sp[1].at);
+    w.e2 = *reinterpret_cast<const uint16_t *>(expert + sp[2].at);
+}
 template <>
 __device__ __forceinline__ void wseg_load<PF_MXFP4>(WSeg<PF_MXFP4> &w, const PfKernelArgs &a, int t, size_t e, size_t n,
                                                     int seg) {
@@ -1518,7 +1525,7 @@ __device__ __forceinline__ float down_dot(const TileItem<PF_IQ2_XXS> &w, int, co
     return half_bits(dbits) * 0.125f * (acc[0] + acc[1]);
 }
 
-// The formats kept row by row (the profiles' down tensors): a lane's run is the segment the loaders above fetch; lanes
+// The profiles' down tensors: a lane's run is the segment the loaders above fetch; row by row lanes
 // r * 8 + part, so that the eight runs of a row are neighbouring lanes and neighbouring bytes.
 struct GroupDigits {   // one 32-group from the slot's image in LDS
     uint32_t dg[PF_IMG_GROUP];
@@ -1610,7 +1617,7 @@ template <int F> __host__ __device__ constexpr bool tile_ordered() { return F ==
 
 // One wave's rows of its slot (eight in the tile order): partial_row[0..rows).  tensor: 3 (the slot's expert e) or 6 (the
 // shared expert); I: the logical width, k_stored: the stored one; dots: rows * I / 64 floats of LDS of the wave's own.
-template <int F>
+template <int F, bool POOL = false>
 __device__ __forceinline__ void down_wave(const PfKernelArgs &a, int tensor, uint32_t e, int I, int k_stored, int n_base, int rows,
                                           const uint32_t *image, uint32_t *mine, uint32_t *tables, float *dots, float *partial_row) {
     const int lane = pf_lane(), runs = I / 64, groups = I / 32;
@@ -1649,7 +1656,20 @@ __device__ __forceinline__ void down_wave(const PfKernelArgs &a, int tensor, uin
         // row, neighbouring bytes, and a row count that does not divide 64 (ten for a hidden width of 2560) leaves no
         // lane idle but in the last step.  The products meet in LDS; a lane per row adds its runs in order.
         const int items = rows * runs;
-        for (int item = lane; item < items; item += 64) {
+        bool tiled = false;
+        if constexpr (F == PF_MXFP4 && !POOL) {
+            tiled = a.wm != nullptr;
+            const int units = runs / 2;
+            const uint8_t *expert = a.wm + (size_t)e * pf_mxt_expert_bytes(a.hidden, units);
+            for (int item = lane; tiled && item < items; item += 64) {   // neighbouring lanes are neighbouring rows
+                const int run = item / rows, r = item - run * rows;
+                WSeg<F> w;
+                wseg_load_tiled(w, expert, units, n_base + r, run);
+                if (!fenced) { pf_wave_lds_fence(); fenced = true; }
+                dots[r * runs + run] = down_dot(w, mine, run, groups);
+            }
+        }
+        for (int item = lane; !tiled && item < items; item += 64) {
             const int r = item / runs, run = item - r * runs;
             WSeg<F> w;
             wseg_load<F>(w, a, tensor, e, (size_t)(n_base + r), run);
@@ -1671,7 +1691,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FMT =
     __shared__ float partial[17][16];
     extern __shared__ int lds[];   // IQ2_XXS: the waves' magnitude grids; [slot][image words of the widest activation row]; [slot][rows * runs] products
     constexpr bool GRID = FMT == PF_IQ2_XXS || FMTS == PF_IQ2_XXS;
-    pf_args_now(a.ids, a.route_weights, a.shared_scale, a.aimg, a.hc_residual, a.wt[3], a.wt[6], a.w[3], a.w[6], a.expert_bytes[3],
+    pf_args_now(a.ids, a.route_weights, a.shared_scale, a.aimg, a.hc_residual, a.wt[3], a.wt[6], a.w[3], a.w[6], a.wm, a.expert_bytes[3],
                 a.shared_inter, a.down_physical, a.hc_streams, a.error_word, rows);
     const int token = (int)blockIdx.y;
     q4t_at_token(a, token);
@@ -1680,7 +1700,11 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FMT =
     uint32_t *tables = reinterpret_cast<uint32_t *>(lds) + (GRID ? 512 * s : 0);
     int *images = lds + (GRID ? 512 * (K + 1) : 0);
     const bool shared = s == K;
-    const int n_base = rows * (int)blockIdx.x;
+    // MXFP4 in tile order: neighbouring rows' workgroups on one XCD, whose L2 then reads a line once that several of them need (ten
+    // rows, one token of 2560 x 640: 20.7 -> 19.9 us a layer)
+    int block = (int)blockIdx.x;
+    if (FMT == PF_MXFP4 && !POOL && a.wm && gridDim.x % 8 == 0) block = (block & 7) * (int)(gridDim.x / 8) + (block >> 3);
+    const int n_base = rows * block;
     const size_t widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
     float *dots = reinterpret_cast<float *>(images + (size_t)(K + 1) * pf_image2_words(widest)) + (size_t)s * rows * (widest / 64);
     // the slot's expert and the combine's operands through the scalar cache
@@ -1706,7 +1730,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(FMT =
     const uint32_t *image = a.aimg + (size_t)s * pf_image2_words(widest);   // slot = unique expert with one token; the shared expert's follows
     uint32_t *mine = reinterpret_cast<uint32_t *>(images) + (size_t)s * pf_image2_words(widest);
     if (shared) down_wave<FMTS>(a, 6, 0u, a.shared_inter, a.shared_inter, n_base, rows, image, mine, tables, dots, partial[s]);
-    else down_wave<FMT>(a, 3, e, a.inter, a.down_physical, n_base, rows, image, mine, tables, dots, partial[s]);
+    else down_wave<FMT, POOL>(a, 3, e, a.inter, a.down_physical, n_base, rows, image, mine, tables, dots, partial[s]);
     __syncthreads();
     const int n = n_base + threadIdx.x;
     if ((int)threadIdx.x < rows && n < H) {
@@ -2505,8 +2529,8 @@ static void launch_down(const PfKernelArgs &a, dim3 grid, dim3 block, size_t lds
 
 // Layers the kernels whose lanes are weight rows take, one token per grid row, for up to PF_PAIR_MAX_TOKENS tokens
 // (PF_TILE_DECODE_MAX_TOKENS of a checkpoint profile and of pool slots): every expert tensor Q4_K, or every one IQ2_XXS, with its tile-ordered copy kept; the two checkpoint profiles
-// with the tile-ordered copies of their routed gate and up tensors and of the shared expert's Q8_0 gate and up (their
-// down tensors are read row by row).  Returns the combination as decode_combination numbers it, 0 for other layers.
+// with the tile-ordered copies of their routed gate and up tensors and of the shared expert's Q8_0 gate and up (of their
+// down tensors the routed MXFP4 one is read in tile order or row by row, the others row by row).  Returns the combination as decode_combination numbers it, 0 for other layers.
 #if PF_DECODE_PART == 0
 int pf_decode_tile_layer(const PfHipMoeDesc &d, const uint8_t *const q4k_tiled[8], const uint8_t *const iq2_tiled[8],
                          const uint8_t *const q8_tiled[8]) {
@@ -2592,13 +2616,16 @@ static void launch_q4t_experts(const PfKernelArgs &a, int tokens, hipStream_t st
 #endif
     const size_t widest = I > Is ? I : Is;
     constexpr bool GRID = FD == PF_IQ2_XXS || FS == PF_IQ2_XXS;
-    // rows per workgroup: eight in the tile order; for down tensors kept row by row the fewest that leave no more
-    // workgroups than compute units (256 on this GPU), so that a hidden width of 2560 runs ten rows in one round
+    // rows per workgroup: eight in the tile order; for the profiles' down tensors the fewest that leave no more
+    // workgroups than compute units (256 on this GPU), so that a hidden width of 2560 runs ten rows in one round.  Of MXFP4 in
+    // tile order, where sixteen rows are whole lines, sixteen from four tokens on (2048 x 512, 4 tokens 39.7 -> 36.6 us, 5
+    // 46.8 -> 45.2; 2560 x 640 62.4 -> 61.7, 67.2 -> 66.9; 3 tokens of six slots 26.4 -> 27.5)
     int rows = 8;
     if (!tile_ordered<FD>() && !tile_ordered<FS>()) {
         rows = (H + 255) / 256;
         while (rows < 16 && H % rows) rows++;
         if (H % rows || rows > 16) rows = 8;
+        if (FD == PF_MXFP4 && !POOL && a.wm && tokens >= 4) rows = 16;
     }
     static bool configured = false;   // once per instantiation: more than the default 64 KB of dynamic LDS
     if (!configured) {

@@ -20,7 +20,7 @@ struct PfKernelArgs {
     const uint8_t *wt[8];            // Q4_K expert tensors in tile order for the grouped product (null: not kept)
     const uint8_t *wi[8];            // IQ2_XXS expert tensors in tile order for the decode kernels (null: not kept)
     const uint8_t *wq[8];            // Q8_0 tensors (the profiles' shared gate and up) in tile order (null: not kept)
-    const uint8_t *wm;               // the routed down tensor, MXFP4, in tile order for the block-scaled products (null: not kept)
+    const uint8_t *wm;               // the routed down tensor, MXFP4, in tile order, in place of w[3] (null: rows)
     const float *router_t;           // router as [slab of 64 experts][hidden / 4][64][4] (serial-order re-routing)
     const uint64_t *iq2_grid;        // 256 x 8 magnitudes, device memory
     const uint32_t *iq2_signed;      // 2 x 4096 words: four signed magnitudes per (grid entry, sign nibble)
@@ -173,7 +173,7 @@ struct PfHipMoe {
     uint8_t *w_tiled[8];             // Q4_K expert tensors in tile order, for every kernel family (or null)
     uint8_t *w_itile[8];             // tile-ordered second copy of IQ2_XXS expert tensors, decode and few rows per expert (or null)
     uint8_t *w_qtile[8];             // tile-ordered second copy of the Q8_0 shared gate and up tensors, the same (or null)
-    uint8_t *w_mxtile;               // tile-ordered second copy of an MXFP4 routed down tensor, for the grouped product (or null)
+    uint8_t *w_mxtile;               // an MXFP4 routed down tensor in tile order, in place of w[3] (or null)
     bool streamed;                   // the routed tensors are not resident: forwards read them from an expert pool
 };
 

@@ -216,6 +216,16 @@ __device__ __forceinline__ float dot_row_mxfp4(const uint8_t *payload, const uin
     return acc;
 }
 
+__device__ __forceinline__ float dot_row_mxfp4_tiled(const uint8_t *expert, int n, const float *x, int nblk, int lane) {
+    float acc = 0.0f;
+    for (int b = lane; b < nblk; b += PF_WAVE) {
+        PfSpan32 sp[3];
+        pf_mxt_segment_spans(nblk / 4, n, b >> 1, sp);
+        acc += dot_row_mxfp4(expert + ((b & 1) ? sp[1].at : sp[0].at), expert + sp[2].at + (b & 1), x + 32 * b, 1, 0);
+    }
+    return acc;
+}
+
 // Q2_K (GGUF bytes): lane l takes the group of 16 values l of the row: 16 code bytes of one bit plane,
 // one scale | min << 4 byte.  Group g of a block: half g / 8, plane (g % 8) / 2, bytes (g % 2) * 16 ...
 __device__ __forceinline__ float dot_row_q2k(const uint8_t *row, const float *x, int nblk, int lane) {
@@ -261,7 +271,10 @@ __device__ __forceinline__ float dot_tensor_row(const PfKernelArgs &a, int t, si
     case PF_Q8_0:
         v = dot_row_q8(row, reinterpret_cast<const uint16_t *>(scales) + first_block, x, a.blocks_per_row[t], lane);
         break;
-    case PF_MXFP4: v = dot_row_mxfp4(row, scales + first_block, x, a.blocks_per_row[t], lane); break;
+    case PF_MXFP4:
+        v = a.w[t] ? dot_row_mxfp4(row, scales + first_block, x, a.blocks_per_row[t], lane)
+                   : dot_row_mxfp4_tiled(a.wm + e * pf_mxt_expert_bytes(a.n_out[t], a.blocks_per_row[t] / 4), (int)n, x, a.blocks_per_row[t], lane);
+        break;
     default:
         v = a.w[t] ? dot_row_iq2(row, reinterpret_cast<const uint16_t *>(scales) + first_block, x, a.blocks_per_row[t], lane, grid)
                    : dot_row_iq2_tiled(a.wi[t] + e * pf_i2t_expert_bytes(a.n_out[t], a.blocks_per_row[t]), (int)n, x,

@@ -1353,7 +1353,7 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     // only the shared expert's tiles (tokens / 32 of them) are left for this launch: columns split over the waves
     if (a.type[4] != gate_fmt && !q8) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, PLAIN_SHARED, stream);
     const int widest = I > Is ? I : Is;
-    const bool digits = a.wm && widest <= 1024;   // the routed rows as digits
+    const bool digits = a.wm != nullptr;   // the routed rows as digits (they are of at most 640 values)
     if (widest <= 1024 && P > 0 && tokens > 0) {
         const unsigned rows_a = digits ? 4u * pf_mx_rows_a_wave(I) : 4u, blocks_a = ((unsigned)P + rows_a - 1) / rows_a, blocks_b = (unsigned)((tokens + 3) / 4);
         hipLaunchKernelGGL(digits ? (widest <= 512 ? pf_k_rows_to_half_short2<1, true> : pf_k_rows_to_half_short2<2, true>)
@@ -1361,7 +1361,8 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
                            stream, a.act, I, (size_t)P, (half_t *)a.act16, a.act_scale, blocks_a, a.shared_act, Is, (size_t)tokens,
                            (half_t *)a.sact16, a.sact_scale, a.error_word);
     } else {
-        launch_rows_to_half(a.act, (size_t)I, I, (size_t)P, (half_t *)a.act16, a.act_scale, a.error_word, stream);
+        if (digits) pf_launch_rows_to_digits(a.act, I, (size_t)P, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
+        else launch_rows_to_half(a.act, (size_t)I, I, (size_t)P, (half_t *)a.act16, a.act_scale, a.error_word, stream);
         launch_rows_to_half(a.shared_act, (size_t)Is, Is, (size_t)tokens, (half_t *)a.sact16, a.sact_scale, a.error_word, stream);
     }
     if (last < 4) return;

@@ -142,6 +142,20 @@ int main(int argc, char **argv) {
                 }
         }
     }
+    // the tile-ordered MXFP4 down tensor: every row's 64-weight segments
+    if (type[3] == PF_MXFP4 && H % 32 == 0 && phys % 128 == 0) {
+        const int units = phys / 128;
+        PfTensorPlace copy = place[3];
+        copy.expert_bytes = pf_mxt_expert_bytes(H, units);
+        copy.bytes = copy.expert_bytes * experts[3];
+        for (size_t e : some_experts)
+            for (int n = 0; n < H; n++)
+                for (int seg = 0; seg < 2 * units; seg++) {
+                    PfSpan32 sp[3];
+                    pf_mxt_segment_spans(units, n, seg, sp);
+                    for (int i = 0; i < 3; i++) check("tile segment", 3, copy, {e * copy.expert_bytes + sp[i].at, sp[i].width}, i < 2 ? 16 : 2, e, n, seg);
+                }
+    }
     // the tile-ordered Q8_0 copies of the profiles' shared gate and up tensors: one chunk per 64-weight run, addressed by
     // the gate/up kernel as four chunks per 256-block
     for (int a : {4, 5}) {

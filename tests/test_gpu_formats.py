@@ -257,3 +257,30 @@ def test_mxfp4_down_scales_near_the_ends_of_their_range(product, oracle, x_scale
             error = np.abs(y.astype(np.float64) - want[0][:tokens]).max(axis=1)
             print(f"    error {(error / largest[:tokens, 0]).max():.2e} of the row's largest", flush=True)
             assert (error <= 1e-5 * largest[:tokens, 0]).all()   # 32-bit sums of 256 products and three slots
+
+
+@pytest.mark.parametrize("h,i,s,k", [(512, 256, 256, 3), (768, 640, 1152, 2), (2560, 512, 640, 10), (512, 512, 2048, 12)])
+def test_mxfp4_down_rows_are_kept_once(product, oracle, monkeypatch, h, i, s, k):
+    """Device memory holds the routed MXFP4 down tensor in one order, and every kernel family reads it there with the results that it
+    gives from the rows (a chunk's products are other ones)."""
+    cfg = abi.moe_config(h, 24, k, i, s)
+    weights, x = make_layer_inputs(cfg, "q4", 40, seed=h + i + s)
+    want = forward_with(oracle, cfg, weights, x)
+    got, held = {}, {}
+    for copy in ("0", "1"):
+        monkeypatch.setenv("PF_MOE_PREFILL_COPY", copy)
+        with pf.MoeLayer(product, cfg, weights, 40) as layer:
+            moe, work = layer.device_handles()
+            held[copy] = product.hip.moe_bytes(moe)
+            for tokens, family in ((1, 1), (2, 1), (3, 1), (4, 1), (16, None), (40, 3), (40, 2), (40, 0)):
+                print(f"case mxfp4 down h={h} i={i} s={s} tile order {copy} tokens={tokens} family={family}", flush=True)
+                layer.force_grouped(family == 2)
+                layer.force_general(family == 0)
+                assert family is None or product.hip.moe_kernel_family(moe, work, tokens) == family
+                _, y, ids, w = layer.forward(x[:tokens])
+                assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens} family {family}")
+                if family == 0:
+                    assert copy == "0" or np.array_equal(y, got[tokens, family])
+                got[tokens, family] = y
+    second = weights.raw[1].size + weights.raw[2].size + (weights.raw[4].size + weights.raw[5].size) * 17 // 16   # Q4_K gate and up, Q8_0 shared ones
+    assert held["1"] - held["0"] <= second + 8 * 256
