@@ -312,14 +312,14 @@ extern "C" int pf_hip_moe_create(const PfHipMoeDesc *desc, const void *const hos
         }
     }
     // The routed MXFP4 down tensor in tile order, which every kernel family reads, in place of its rows: a layer takes no more
-    // memory for it.  Where there is none left for the two while the one is made from the other, and with PF_MOE_PREFILL_COPY=0,
-    // the rows stay.
+    // memory for it.  Where there is none left for the two while the one is made from the other, and with PF_MOE_PREFILL_COPY=0 or
+    // PF_MOE_MXFP4_ROWS=1, the rows stay.
     // (The decode kernels on segments of rows read the rows: no layer of these widths runs them with the other copies kept.)
     const bool segments = m->decode_ready && pf_decode_tile_layer(m->desc, m->w_tiled, m->w_itile, m->w_qtile) == 0;
     if (m->prefill_ready && !segments && pf_mx_down_takes(*desc)) {
-        const char *copy = getenv("PF_MOE_PREFILL_COPY");
+        const char *copy = getenv("PF_MOE_PREFILL_COPY"), *rows = getenv("PF_MOE_MXFP4_ROWS");
         const size_t bytes = pf_mxt_expert_bytes((int)n_out[3], m->blocks_per_row[3] / 4) * experts[3];
-        if ((!copy || strcmp(copy, "0") != 0) && hipMalloc((void **)&m->w_mxtile, bytes) == hipSuccess) {
+        if ((!copy || strcmp(copy, "0") != 0) && (!rows || rows[0] != '1') && hipMalloc((void **)&m->w_mxtile, bytes) == hipSuccess) {
             pf_launch_mx_tile(m->w[3], m->w[3] + m->scale_offset[3], m->w_mxtile, (size_t)n_out[3] * experts[3], m->blocks_per_row[3], nullptr);
             const hipError_t e = hipDeviceSynchronize();
             if (e != hipSuccess) {
