@@ -2484,11 +2484,17 @@ static void launch_gate_up(const PfKernelArgs &a, dim3 grid, size_t lds, hipStre
 
 void pf_launch_dec_router(const PfKernelArgs &a, int tokens, int router_blocks, hipStream_t stream);
 #if PF_DECODE_PART == 0
-// From 17 tokens on, the second tile of 16, the few-row kernels' router on the matrix cores (rows of 2048: 16 tokens 9.4 us both ways,
-// 24 tokens 9.3 against 11.6, 32 tokens 9.6 against 14.6; 8 tokens 8.8 against 6.6).
+// From 17 tokens on, the second tile of 16, and where tokens times experts give its tiles of 16 x 16 enough of the chip, the few-row
+// kernels' router on the matrix cores.  The other one's time grows with the tokens and the experts, this one's is a workgroup's, so
+// the line is a product; a forward with it against without, us:
+//   rows of 2048   512 experts 17 tokens 76.8 : 78.7, 32 tokens 114.9 : 119.7   384: 20 73.6 : 73.3, 24 81.7 : 83.9
+//                  256: 24 77.8 : 76.7, 32 100.9 : 100.8   128: 17 64.7 : 61.7, 32 95.9 : 94.0   64: 17 60.7 : 58.0
+//   2560           512: 17 82.5 : 83.1, 24 112.8 : 115.4   256: 32 124.9 : 123.9   128: 32 94.4 : 91.8
+//   1024           512: 17 45.8 : 48.4   256: 28 41.0 : 41.3, 32 43.7 : 46.7   128: 28 40.3 : 39.8
 #define DEC_ROUTER_MFMA_FROM 17
+#define DEC_ROUTER_MFMA_LOGITS 8192
 void pf_launch_dec_router(const PfKernelArgs &a, int tokens, int router_blocks, hipStream_t stream) {
-    if (tokens >= DEC_ROUTER_MFMA_FROM && pf_batch_router_takes(a.hidden)) {
+    if (tokens >= DEC_ROUTER_MFMA_FROM && tokens * a.experts >= DEC_ROUTER_MFMA_LOGITS && pf_batch_router_takes(a.hidden)) {
         pf_launch_batch_router(a, tokens, 3, true, stream);
         return;
     }

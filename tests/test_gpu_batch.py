@@ -120,9 +120,10 @@ def test_short_batches_of_the_q4_profile(product, oracle, monkeypatch, h, i, s, 
         np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
 
 
-@pytest.mark.parametrize("h,e,k,fmt", [(512, 70, 6, abi.GGUF_Q4_K), (2560, 33, 4, abi.GGUF_Q4_K), (768, 100, 5, abi.GGUF_IQ2_XXS), (2048, 512, 3, abi.GGUF_IQ2_XXS)])
+@pytest.mark.parametrize("h,e,k,fmt", [(512, 70, 6, abi.GGUF_Q4_K), (2560, 33, 4, abi.GGUF_Q4_K), (768, 100, 5, abi.GGUF_IQ2_XXS), (2048, 512, 3, abi.GGUF_IQ2_XXS),
+                                       (512, 300, 6, abi.GGUF_Q4_K), (2560, 257, 4, abi.GGUF_Q4_K), (768, 500, 5, abi.GGUF_IQ2_XXS)])   # 32, 32, 17 tokens on
 def test_decode_kernels_on_either_side_of_the_matrix_router(product, oracle, h, e, k, fmt):
-    """Up to 16 tokens the decode kernels' own router, from 17 on tiles of 16 tokens and experts, whose images they read."""
+    """Up to 16 tokens or 8192 logits the decode kernels' own router, beyond them tiles of 16 tokens and experts, whose images they read."""
     print(f"case decode router {fmt} h={h} e={e} k={k}", flush=True)
     cfg = abi.moe_config(h, e, k, 256, 256)
     weights, x = make_layer_inputs(cfg, fmt, 32, seed=h + e)
