@@ -19,6 +19,7 @@
 #include "pf_grouped.h"
 #include "pf_mx_rows.h"
 #include "pf_upload_addr.h"
+#include "pf_item_order.h"
 
 template <int UNITS>   // of 128 columns
 __global__ void __launch_bounds__(256, 2) pf_k_mx_down(PfKernelArgs a, int slabs, int per) {
@@ -134,21 +135,21 @@ void pf_launch_mx_tile(const uint8_t *d_payload, const uint8_t *d_scales, uint8_
     hipLaunchKernelGGL(pf_k_mx_tile, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, d_payload, d_scales, d_dst, rows, blocks_per_row);
 }
 
-template <int UNITS> static void launch(const PfKernelArgs &a, unsigned tiles, hipStream_t stream) {
-    const int lds = 32 * 4 * 128 * UNITS, all = a.hidden / 256, per = max(1, min(all, 5)), slabs = (all + per - 1) / per;
+template <int UNITS> static void launch(const PfKernelArgs &a, unsigned tile_cap, hipStream_t stream) {
+    const unsigned tiles = (tile_cap + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES);
+    const int lds = 32 * 4 * 128 * UNITS, all = a.hidden / 256, per = pf_slabs_each(all, 5, tile_cap), slabs = (all + per - 1) / per;
     static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_mx_down<UNITS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
     (void)configured;   // more than the default 64 KB
     hipLaunchKernelGGL(pf_k_mx_down<UNITS>, dim3(tiles * slabs), dim3(256), lds, stream, a, slabs, per);
 }
 // the routed experts' down products, from the digit rows in act16
 void pf_launch_mx_down(const PfKernelArgs &a, unsigned tile_cap, hipStream_t stream) {
-    const unsigned tiles = (tile_cap + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES);
     switch (a.inter / 128) {
-    case 1: launch<1>(a, tiles, stream); break;
-    case 2: launch<2>(a, tiles, stream); break;
-    case 3: launch<3>(a, tiles, stream); break;
-    case 4: launch<4>(a, tiles, stream); break;
-    default: launch<5>(a, tiles, stream); break;
+    case 1: launch<1>(a, tile_cap, stream); break;
+    case 2: launch<2>(a, tile_cap, stream); break;
+    case 3: launch<3>(a, tile_cap, stream); break;
+    case 4: launch<4>(a, tile_cap, stream); break;
+    default: launch<5>(a, tile_cap, stream); break;
     }
 }
 

@@ -23,6 +23,7 @@
 #include "pf_upload_addr.h"
 #include "pf_plain_walk.h"
 #include "pf_grouped.h"
+#include "pf_item_order.h"
 #include "pf_mx_rows.h"
 #include "pf_group_device.h"
 
@@ -1280,7 +1281,7 @@ static void launch_gemm(const PfKernelArgs &a, unsigned tile_cap, int width, int
                                                        (int)lds) == hipSuccess;   // more than the default 64 KB
     (void)configured;
     const int rows = MODE == PF_GEMM_GATE_UP ? 16 * GW : 32 * GW, all = (width + rows - 1) / rows;
-    const int per = MODE == PF_GEMM_GATE_UP || shared_tokens ? 1 : max(1, min(all, 8 / max(1, cols / 256)));
+    const int per = MODE == PF_GEMM_GATE_UP || shared_tokens ? 1 : pf_slabs_each(all, max(1, 8 / max(1, cols / 256)), tile_cap);
     const int slabs = (all + per - 1) / per;
     if (shared_tokens) tile_cap = (unsigned)(shared_tokens + 31) / 32;
     const unsigned tiles = (tile_cap + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES);
