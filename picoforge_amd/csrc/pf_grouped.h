@@ -2,6 +2,7 @@
 // uses of an LDS copy, work items.
 #pragma once
 #include "pf_moe_internal.h"
+#include "pf_item_order.h"
 
 typedef _Float16 half_t;
 typedef float float16v __attribute__((ext_vector_type(16)));
@@ -31,18 +32,13 @@ struct GemmItem {   // a 32-row tile of an expert
     int inter;
 };
 
-// Work item q -> (row tile, slab group).  Workgroups go to the eight XCDs round robin by index.  The tile list is cut into groups of
-// GEMM_XCD_TILES consecutive tiles and the groups dealt to the XCDs in turn; the items of a group (its tiles' slabs) get numbers
-// eight apart: neighbouring workgroups of one XCD, one L2, at the same time.  The slabs of a row tile read the same
-// activation rows, and the row tiles of one expert, neighbours in the list, the same weights: fetched once from memory where
-// they fall into one group.  skip: tiles left out at the list's start.  False: nothing to do for q.
-#define GEMM_XCD_TILES 8
-__device__ __forceinline__ bool gemm_item(const PfKernelArgs &a, int slabs, uint32_t q, GemmItem &g, int &slab, uint32_t skip = 0) {
-    const uint32_t xcd = q % 8, turn = q / 8, r = turn / slabs;
-    const uint32_t tile = GEMM_XCD_TILES * ((r / GEMM_XCD_TILES) * 8 + xcd) + r % GEMM_XCD_TILES + skip;
-    if (tile >= a.tiles[0]) return false;
-    const uint4 item = reinterpret_cast<const uint4 *>(a.items)[tile];
-    slab = turn % slabs;
+// The item that number q of the launch is (pf_item_order.h); shared: the shared expert's row tiles, the list's last; skip: tiles at
+// the list's start that the launch leaves out.  False: nothing to do for q.
+__device__ __forceinline__ bool gemm_item(const PfKernelArgs &a, int slabs, int shift, uint32_t q, uint32_t routed, uint32_t shared, uint32_t skip, GemmItem &g, int &slab) {
+    const PfItemPlace p = pf_item_place(q, slabs, shift, routed, shared);
+    if (!p.any) return false;
+    const uint4 item = reinterpret_cast<const uint4 *>(a.items)[skip + p.tile];
+    slab = p.slab;
     g.expert = (int)item.x; g.first = (int)item.y; g.rows_here = (int)item.z; g.m0 = (int)item.w;
     g.shared = g.expert == a.experts;
     g.inter = g.shared ? a.shared_inter : a.inter;

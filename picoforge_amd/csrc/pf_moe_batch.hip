@@ -705,7 +705,7 @@ static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile
     const dim3 grid((a.hidden + 127) / 128, tile_cap);
     if (FD == PF_MXFP4 && batch_down_scaled<FG, FS, PLANES>(a)) {
         pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
-        pf_launch_mx_down(a, tile_cap, stream);
+        pf_launch_mx_down(a, tokens, tile_cap - (unsigned)(tokens + 31) / 32, stream);
         hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, (tokens + 31) / 32, 32 / BATCH_ROWS), dim3(256), 0, stream, a, 1);
         return;
     }

@@ -283,7 +283,7 @@ size_t pf_prefill_most_tokens(int hidden);   // that one launch of pf_launch_pre
 bool pf_mx_down_takes(const PfHipMoeDesc &d);
 void pf_launch_rows_to_digits(const float *d_src, int cols, size_t rows, uint32_t *d_dst, float *d_scales, uint32_t *d_error, hipStream_t stream);
 void pf_launch_mx_tile(const uint8_t *d_payload, const uint8_t *d_scales, uint8_t *d_dst, size_t rows, int blocks_per_row, hipStream_t stream);
-void pf_launch_mx_down(const PfKernelArgs &a, unsigned tile_cap, hipStream_t stream);
+void pf_launch_mx_down(const PfKernelArgs &a, int tokens, unsigned routed_cap, hipStream_t stream);
 // pf_moe_batch.hip: a few rows per expert, for the layers of the tile decode kernels
 void pf_launch_batch(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
 bool pf_batch_router_takes(int hidden);

@@ -19,15 +19,14 @@
 #include "pf_grouped.h"
 #include "pf_mx_rows.h"
 #include "pf_upload_addr.h"
-#include "pf_item_order.h"
 
 template <int UNITS>   // of 128 columns
-__global__ void __launch_bounds__(256, 2) pf_k_mx_down(PfKernelArgs a, int slabs, int per) {
+__global__ void __launch_bounds__(256, 2) pf_k_mx_down(PfKernelArgs a, int slabs, int per, int shift, uint32_t shared_tiles) {
     extern __shared__ __align__(16) unsigned char mx_lds[];
     lds_byte *lds = (lds_byte *)mx_lds;
     GemmItem g;
     int slab;
-    if (!gemm_item(a, slabs, blockIdx.x, g, slab) || g.shared) return;
+    if (!gemm_item(a, slabs, shift, blockIdx.x, a.tiles[0] - shared_tiles, 0, 0, g, slab)) return;   // the routed tiles, ahead of the shared expert's
     constexpr int K = 128 * UNITS;
     const int lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, h = lane >> 5;
     const int slab1 = min((slab + 1) * per, a.hidden / 256);
@@ -135,21 +134,20 @@ void pf_launch_mx_tile(const uint8_t *d_payload, const uint8_t *d_scales, uint8_
     hipLaunchKernelGGL(pf_k_mx_tile, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, d_payload, d_scales, d_dst, rows, blocks_per_row);
 }
 
-template <int UNITS> static void launch(const PfKernelArgs &a, unsigned tile_cap, hipStream_t stream) {
-    const unsigned tiles = (tile_cap + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES);
-    const int lds = 32 * 4 * 128 * UNITS, all = a.hidden / 256, per = pf_slabs_each(all, 5, tile_cap), slabs = (all + per - 1) / per;
+template <int UNITS> static void launch(const PfKernelArgs &a, int tokens, unsigned routed_cap, hipStream_t stream) {
+    const int lds = 32 * 4 * 128 * UNITS, all = a.hidden / 256, per = pf_slabs_each(all, 5, routed_cap), slabs = (all + per - 1) / per, shift = pf_group_shift(routed_cap);
     static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_mx_down<UNITS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
     (void)configured;   // more than the default 64 KB
-    hipLaunchKernelGGL(pf_k_mx_down<UNITS>, dim3(tiles * slabs), dim3(256), lds, stream, a, slabs, per);
+    hipLaunchKernelGGL(pf_k_mx_down<UNITS>, dim3(pf_item_numbers(slabs, shift, routed_cap, 0)), dim3(256), lds, stream, a, slabs, per, shift, (uint32_t)(tokens + 31) / 32);
 }
-// the routed experts' down products, from the digit rows in act16
-void pf_launch_mx_down(const PfKernelArgs &a, unsigned tile_cap, hipStream_t stream) {
+// the routed experts' down products, from the digit rows in act16; routed_cap: their row tiles, at most
+void pf_launch_mx_down(const PfKernelArgs &a, int tokens, unsigned routed_cap, hipStream_t stream) {
     switch (a.inter / 128) {
-    case 1: launch<1>(a, tile_cap, stream); break;
-    case 2: launch<2>(a, tile_cap, stream); break;
-    case 3: launch<3>(a, tile_cap, stream); break;
-    case 4: launch<4>(a, tile_cap, stream); break;
-    default: launch<5>(a, tile_cap, stream); break;
+    case 1: launch<1>(a, tokens, routed_cap, stream); break;
+    case 2: launch<2>(a, tokens, routed_cap, stream); break;
+    case 3: launch<3>(a, tokens, routed_cap, stream); break;
+    case 4: launch<4>(a, tokens, routed_cap, stream); break;
+    default: launch<5>(a, tokens, routed_cap, stream); break;
     }
 }
 

@@ -23,7 +23,6 @@
 #include "pf_upload_addr.h"
 #include "pf_plain_walk.h"
 #include "pf_grouped.h"
-#include "pf_item_order.h"
 #include "pf_mx_rows.h"
 #include "pf_group_device.h"
 
@@ -776,13 +775,14 @@ __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem 
 }
 
 // FMT, SHARED: the routed tensors' format and the shared expert's.  slabs: workgroups that share a row tile; per: slabs that each of
-// them takes (gate and up: one); skip_routed: only the shared expert's tiles, the list's last, of this many tokens (0: all).
+// them takes (gate and up: one); shift: of the groups of tiles; shared_tiles: the shared expert's; only_shared: of them alone.
 template <int MODE, int FMT, int SHARED>
-__global__ void __launch_bounds__(64 * GW, 4) pf_k_pf_gemm(PfKernelArgs a, int slabs, int per, int skip_routed) {
+__global__ void __launch_bounds__(64 * GW, 4) pf_k_pf_gemm(PfKernelArgs a, int slabs, int per, int shift, uint32_t shared_tiles, int only_shared) {
     extern __shared__ __align__(16) unsigned char gemm_lds[];
     GemmItem g;
     int slab;
-    if (!gemm_item(a, slabs, blockIdx.x, g, slab, skip_routed ? a.tiles[0] - (uint32_t)(skip_routed + 31) / 32 : 0)) return;
+    const uint32_t routed = a.tiles[0] - shared_tiles;
+    if (!gemm_item(a, slabs, shift, blockIdx.x, only_shared ? 0 : routed, shared_tiles, only_shared ? routed : 0, g, slab)) return;
     if (a.type[MODE == PF_GEMM_GATE_UP ? (g.shared ? 4 : 1) : (g.shared ? 6 : 3)] != (uint32_t)(g.shared ? SHARED : FMT)) return;   // the plain kernel's
     const int width = MODE == PF_GEMM_GATE_UP ? 16 * GW : 32 * GW, all = ((MODE == PF_GEMM_GATE_UP ? g.inter : a.hidden) + width - 1) / width;
     const int slab0 = slab * per, slab1 = min(slab0 + per, all);
@@ -1272,20 +1272,21 @@ int pf_prefill_max_tiles(int tokens, int experts, int top_k) {
     return (int)(((size_t)tokens * top_k) / 32 + experts + (tokens + 31) / 32 + 1);
 }
 
-// The tile list's length is only known on the device: a workgroup beyond it ends at once.  shared_tokens: the shared expert's tiles only
-// (one slab a workgroup, they are few).
+// The tile list's length is only known on the device: a workgroup beyond it ends at once.  routed_cap: routed row tiles, at most (0: the
+// shared expert's only, one slab a workgroup, they are few).
 template <int MODE, int FMT, int SHARED>
-static void launch_gemm(const PfKernelArgs &a, unsigned tile_cap, int width, int cols, int shared_tokens, hipStream_t stream) {
+static void launch_gemm(const PfKernelArgs &a, int tokens, unsigned routed_cap, int width, int cols, hipStream_t stream) {
     const size_t lds = FMT == PF_IQ2_XXS ? GEMM_LDS_IQ2 : GEMM_LDS;
     static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_gemm<MODE, FMT, SHARED>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        (int)lds) == hipSuccess;   // more than the default 64 KB
     (void)configured;
     const int rows = MODE == PF_GEMM_GATE_UP ? 16 * GW : 32 * GW, all = (width + rows - 1) / rows;
-    const int per = MODE == PF_GEMM_GATE_UP || shared_tokens ? 1 : pf_slabs_each(all, max(1, 8 / max(1, cols / 256)), tile_cap);
+    const unsigned shared = (unsigned)(tokens + 31) / 32;
+    const int per = MODE == PF_GEMM_GATE_UP || !routed_cap ? 1 : pf_slabs_each(all, max(1, 8 / max(1, cols / 256)), routed_cap + shared);
     const int slabs = (all + per - 1) / per;
-    if (shared_tokens) tile_cap = (unsigned)(shared_tokens + 31) / 32;
-    const unsigned tiles = (tile_cap + 8u * GEMM_XCD_TILES - 1u) / (8u * GEMM_XCD_TILES) * (8u * GEMM_XCD_TILES);
-    hipLaunchKernelGGL((pf_k_pf_gemm<MODE, FMT, SHARED>), dim3(tiles * slabs), dim3(64 * GW), lds, stream, a, slabs, per, shared_tokens);
+    const int shift = pf_group_shift(routed_cap);
+    hipLaunchKernelGGL((pf_k_pf_gemm<MODE, FMT, SHARED>), dim3(pf_item_numbers(slabs, shift, routed_cap, shared)), dim3(64 * GW), lds, stream, a, slabs, per,
+                       shift, shared, routed_cap ? 0 : 1);
 }
 
 template <int MODE>
@@ -1345,14 +1346,14 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     const int gi = I > Is ? I : Is;
     const bool iq2 = a.type[1] == PF_IQ2_XXS;
     const uint32_t gate_fmt = a.type[1];
-    const unsigned tile_cap = (unsigned)pf_prefill_max_tiles(tokens, E, K);
+    const unsigned shared_tiles = (unsigned)(tokens + 31) / 32, routed_cap = (unsigned)pf_prefill_max_tiles(tokens, E, K) - shared_tiles;
     const bool q8 = a.type[4] == PF_Q8_0;   // the shared expert of the checkpoint profiles
-    if (iq2 && q8) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS, PF_Q8_0>(a, tile_cap, gi, H, 0, stream);
-    else if (iq2) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS, PF_IQ2_XXS>(a, tile_cap, gi, H, 0, stream);
-    else if (q8) launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q8_0>(a, tile_cap, gi, H, 0, stream);
-    else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q4_K>(a, tile_cap, gi, H, 0, stream);
+    if (iq2 && q8) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS, PF_Q8_0>(a, tokens, routed_cap, gi, H, stream);
+    else if (iq2) launch_gemm<PF_GEMM_GATE_UP, PF_IQ2_XXS, PF_IQ2_XXS>(a, tokens, routed_cap, gi, H, stream);
+    else if (q8) launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q8_0>(a, tokens, routed_cap, gi, H, stream);
+    else launch_gemm<PF_GEMM_GATE_UP, PF_Q4_K, PF_Q4_K>(a, tokens, routed_cap, gi, H, stream);
     // only the shared expert's tiles (tokens / 32 of them) are left for this launch: columns split over the waves
-    if (a.type[4] != gate_fmt && !q8) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, (unsigned)((tokens + 31) / 32), (Is + 31) / 32, 1, PLAIN_SHARED, stream);
+    if (a.type[4] != gate_fmt && !q8) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, shared_tiles, (Is + 31) / 32, 1, PLAIN_SHARED, stream);
     const int widest = I > Is ? I : Is;
     const bool digits = a.wm != nullptr;   // the routed rows as digits (they are of at most 640 values)
     if (widest <= 1024 && P > 0 && tokens > 0) {
@@ -1369,17 +1370,17 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     if (last < 4) return;
     // stage 4: down and combine
     if (a.type[3] == gate_fmt || a.type[6] == gate_fmt) {
-        if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS, PF_IQ2_XXS>(a, tile_cap, H, gi, 0, stream);
-        else launch_gemm<PF_GEMM_DOWN, PF_Q4_K, PF_Q4_K>(a, tile_cap, H, gi, 0, stream);
+        if (iq2) launch_gemm<PF_GEMM_DOWN, PF_IQ2_XXS, PF_IQ2_XXS>(a, tokens, routed_cap, H, gi, stream);
+        else launch_gemm<PF_GEMM_DOWN, PF_Q4_K, PF_Q4_K>(a, tokens, routed_cap, H, gi, stream);
     }
-    if (digits) pf_launch_mx_down(a, tile_cap, stream);
+    if (digits) pf_launch_mx_down(a, tokens, routed_cap, stream);
     // (beside routed items of the plain kernel a Q8_0 shared expert's cost nothing: in a launch of its own it made the down stage of
     // the q2 profile's 1024-token chunk 169 us instead of 157, at the checkpoints' widths 291 instead of 271)
     const bool plain_routed = a.type[3] != gate_fmt && !digits, q8_shared = a.type[6] == PF_Q8_0 && !plain_routed;
     const bool plain_shared = a.type[6] != gate_fmt && !q8_shared;
     if (plain_routed || plain_shared)
-        launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, plain_routed ? tile_cap : (unsigned)((tokens + 31) / 32), (H + 255) / 256, 0,
+        launch_gemm_plain<PF_GEMM_DOWN>(a, tokens, plain_routed ? routed_cap + shared_tiles : shared_tiles, (H + 255) / 256, 0,
                                         plain_routed ? PLAIN_ALL : PLAIN_SHARED, stream);
-    if (q8_shared) launch_gemm<PF_GEMM_DOWN, PF_Q8_0, PF_Q8_0>(a, tile_cap, H, Is, tokens, stream);
+    if (q8_shared) launch_gemm<PF_GEMM_DOWN, PF_Q8_0, PF_Q8_0>(a, tokens, 0, H, Is, stream);
     pf_launch_combine(a, tokens, stream);
 }

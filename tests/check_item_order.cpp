@@ -1,6 +1,7 @@
 // Host-side check of how the grouped products' launches cut their work (picoforge_amd/csrc/pf_item_order.h).  Compiled with g++ by
 // tests/test_item_order.py.  Exit status 1 on a violation.
 #include <stdio.h>
+#include <vector>
 #include "../picoforge_amd/csrc/pf_item_order.h"
 
 static int bad = 0;
@@ -23,7 +24,37 @@ static void slabs() {
             }
 }
 
+// every item once, and no XCD with more than its share of the routed groups or the shared expert's tiles
+static void places() {
+    const uint32_t routed_of[] = {0, 1, 7, 8, 9, 63, 64, 65, 75, 640, 1001}, shared_of[] = {0, 1, 5, 8, 9, 11, 24, 64};
+    for (uint32_t routed : routed_of)
+        for (uint32_t shared : shared_of)
+            for (int slabs = 1; slabs <= 12; slabs++)
+                for (uint32_t more : {0u, 40u, 300u}) {   // the numbers are for an upper bound of the routed tiles
+                    const int shift = pf_group_shift(routed + more);
+                    const uint32_t tiles = routed + shared, numbers = pf_item_numbers(slabs, shift, routed + more, shared);
+                    std::vector<int> times((size_t)tiles * slabs);
+                    uint32_t routed_on[PF_XCDS] = {}, shared_on[PF_XCDS] = {};
+                    for (uint32_t q = 0; q < numbers; q++) {
+                        const PfItemPlace p = pf_item_place(q, slabs, shift, routed, shared);
+                        if (!p.any) continue;
+                        expect(p.tile < tiles && p.slab >= 0 && p.slab < slabs, "an item that is not there", (int)routed, (int)shared, (int)q);
+                        if (p.tile >= tiles || p.slab < 0 || p.slab >= slabs) continue;
+                        times[(size_t)p.tile * slabs + p.slab]++;
+                        (p.tile < routed ? routed_on : shared_on)[q % PF_XCDS]++;
+                    }
+                    for (int t : times) expect(t == 1, "an item left out or taken twice", (int)routed, (int)shared, slabs);
+                    for (int x = 0; x < PF_XCDS; x++) {   // an XCD's part: no more than a group above the least, and of them all
+                        expect(shared_on[x] <= ((shared + PF_XCDS - 1) / PF_XCDS + (1u << shift)) * slabs, "the shared expert on few XCDs", (int)routed, (int)shared, (int)shared_on[x]);
+                        expect(routed_on[x] <= (routed / PF_XCDS + (1u << shift)) * slabs, "routed tiles on few XCDs", (int)routed, (int)shared, (int)routed_on[x]);
+                        expect(routed_on[x] + shared_on[x] <= (tiles / PF_XCDS + (1u << shift) + 1) * slabs, "tiles on few XCDs", (int)routed, (int)shared, x);
+                    }
+                    if (routed >= 8 && more == 0) expect(1u << shift <= (routed + 63) / 64, "groups larger than an eighth of an XCD's part", (int)routed, shift, 0);
+                }
+}
+
 int main() {
     slabs();
+    places();
     return bad != 0;
 }
