@@ -55,3 +55,15 @@ PF_HD uint32_t pf_item_numbers(int slabs, int shift, uint32_t routed, uint32_t s
     const uint32_t deal = PF_XCDS << shift;
     return ((routed + deal - 1) / deal * deal + (shared + PF_XCDS - 1) / PF_XCDS * PF_XCDS) * (uint32_t)slabs;   // (no XCD has more)
 }
+
+// Which MXFP4 down projections of a layer that keeps them in tile order run on the block-scaled product.  It saves work for every weight
+// and row, and costs launches of its own (the rows' conversion 3 to 5 us; in the few-row kernels the shared expert's part as well).
+//
+// Batches of the decode kernels: the work is a pair's rows.  Forwards on the other kernel and on this, us: 5 tokens of 4 slots, 2048 x
+// 512 (21e6) 27.0 : 29.7, 8 of 8, 1024 x 512 (34e6) 29.3 : 32.4, 6 of 8, 2048 x 512 (50e6) 37.5 : 39.4, 5 of 10, 2560 x 640 (82e6)
+// 59.8 : 54.8, 16 of 10 (262e6) 136.0 : 117.5.  Of 480 batches of 8 to 512 experts, 1 to 10 slots and eight widths none is more than
+// 7 % slower than on the other side of the line.
+#define PF_DOWN_SCALED_FROM 5   // 4 tokens of 10 slots, 2560 x 640: 18.1 us of down projection against 19.5, and a launch more
+PF_HD bool pf_decode_down_scaled(int tokens, int top_k, int hidden, int inter) {
+    return tokens >= PF_DOWN_SCALED_FROM && (size_t)tokens * top_k * hidden * inter >= 55000000u;
+}

@@ -1825,24 +1825,21 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(6))) 
     }
 }
 
-// From five tokens on (checkpoint widths, the rows' conversion of 5 us included): 4 tokens 18.1 us against 19.5, and a launch more;
-// 8 tokens 25 against 38, 13 tokens 35 against 62, 16 tokens 39 against 73.
-#define DOWN_MX_FROM 5
+// (checkpoint widths, the rows' conversion of 5 us included: 8 tokens 25 us against 38, 13 tokens 35 against 62, 16 tokens 39 against 73)
 template <int UNITS> static void launch_down_mx_units(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     const size_t lds = 2 * (size_t)(pf_image2_words(a.shared_inter) + 16 * (a.shared_inter / 64)) * 4;
     hipLaunchKernelGGL(pf_k_dec_down_mx<UNITS>, dim3(a.hidden / 32, tokens), dim3(64 * (a.top_k + 2)), lds, stream, a);
 }
 static bool down_mx_applies(const PfKernelArgs &a, int tokens) {
-    return tokens >= DOWN_MX_FROM && a.wm && a.top_k + 2 <= 16;   // at most 1024 threads
+    return a.wm && a.top_k + 2 <= 16 && pf_decode_down_scaled(tokens, a.top_k, a.hidden, a.inter);   // (a workgroup has 1024 threads at most)
 }
 static void launch_down_mx(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act), nullptr, a.error_word, stream);   // in place
     switch (a.inter / 128) {
-    case 1: launch_down_mx_units<1>(a, tokens, stream); break;
     case 2: launch_down_mx_units<2>(a, tokens, stream); break;
     case 3: launch_down_mx_units<3>(a, tokens, stream); break;
     case 4: launch_down_mx_units<4>(a, tokens, stream); break;
-    default: launch_down_mx_units<5>(a, tokens, stream);   // a layer keeps the copy up to 640 columns
+    default: launch_down_mx_units<5>(a, tokens, stream);   // (decode layers are 256 columns and more, the tile order is kept up to 640)
     }
 }
 #endif
@@ -2624,14 +2621,14 @@ static void launch_q4t_experts(const PfKernelArgs &a, int tokens, hipStream_t st
     constexpr bool GRID = FD == PF_IQ2_XXS || FS == PF_IQ2_XXS;
     // rows per workgroup: eight in the tile order; for the profiles' down tensors the fewest that leave no more
     // workgroups than compute units (256 on this GPU), so that a hidden width of 2560 runs ten rows in one round.  Of MXFP4 in
-    // tile order, where sixteen rows are whole lines, sixteen from four tokens on (2048 x 512, 4 tokens 39.7 -> 36.6 us, 5
-    // 46.8 -> 45.2; 2560 x 640 62.4 -> 61.7, 67.2 -> 66.9; 3 tokens of six slots 26.4 -> 27.5)
+    // tile order, where sixteen rows are whole lines, sixteen from four tokens and sixteen pairs on (2048 x 512, 4 tokens 39.7 -> 36.6 us, 5
+    // 46.8 -> 45.2; 2560 x 640 62.4 -> 61.7, 67.2 -> 66.9; 3 tokens of six slots 26.4 -> 27.5, 5 tokens of two 30.5 -> 32.3)
     int rows = 8;
     if (!tile_ordered<FD>() && !tile_ordered<FS>()) {
         rows = (H + 255) / 256;
         while (rows < 16 && H % rows) rows++;
         if (H % rows || rows > 16) rows = 8;
-        if (FD == PF_MXFP4 && !POOL && a.wm && tokens >= 4) rows = 16;
+        if (FD == PF_MXFP4 && !POOL && a.wm && tokens >= 4 && tokens * a.top_k >= 16) rows = 16;
     }
     static bool configured = false;   // once per instantiation: more than the default 64 KB of dynamic LDS
     if (!configured) {

@@ -53,7 +53,15 @@ static void places() {
                 }
 }
 
+// batches that are clearly faster on one of the two down projections
+static void decode_down() {
+    expect(!pf_decode_down_scaled(5, 2, 768, 256) && !pf_decode_down_scaled(8, 2, 2048, 512) && !pf_decode_down_scaled(5, 4, 2048, 512), "small batches", 0, 0, 0);
+    expect(pf_decode_down_scaled(5, 10, 2560, 640) && pf_decode_down_scaled(13, 10, 2560, 640) && pf_decode_down_scaled(8, 8, 2048, 512), "large batches", 0, 0, 0);
+    expect(!pf_decode_down_scaled(4, 10, 2560, 640), "four tokens", 0, 0, 0);
+}
+
 int main() {
+    decode_down();
     slabs();
     places();
     return bad != 0;

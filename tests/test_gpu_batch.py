@@ -99,11 +99,12 @@ def test_batches_on_both_sides_of_the_lines_between_the_kernels(product, oracle,
 
 @pytest.mark.parametrize("h,i,s,k,copy", [
     (512, 256, 256, 6, "1"), (768, 384, 384, 1, "1"), (512, 512, 640, 14, "1"), (512, 256, 256, 15, "1"), (2560, 640, 640, 10, "1"), (1024, 768, 256, 4, "1"),   # 768: no copy
+    (2048, 256, 256, 14, "1"), (2048, 384, 640, 12, "1"), (2048, 512, 512, 10, "1"),   # the largest on the block-scaled product
     (2560, 640, 640, 10, "0"),
 ])
 def test_short_batches_of_the_q4_profile(product, oracle, monkeypatch, h, i, s, k, copy):
     """The decode kernels' down projections of MXFP4 rows: on the block-scaled matrix instruction where the layer keeps the
-    tile-ordered copy, from the batch size on where that pays; two to five units of 128 columns, one to fifteen slots."""
+    tile order, from the work on where that pays; two to five units of 128 columns, one to fifteen slots."""
     print(f"case short q4 batches h={h} i={i} s={s} k={k} tile-ordered copies {copy}", flush=True)
     monkeypatch.setenv("PF_MOE_PREFILL_COPY", copy)
     cfg = abi.moe_config(h, 32, k, i, s)

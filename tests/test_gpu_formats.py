@@ -231,12 +231,13 @@ def test_prefill_kernels_with_a_q2k_shared_expert(product, oracle, h, gtype):
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"h={h} T={tokens}")
 
 
+@pytest.mark.parametrize("h,i,s", [(512, 256, 256), (2048, 640, 1024)])   # the second: 16 tokens and batches on the block-scaled product
 @pytest.mark.parametrize("x_scale,exponent", [(2.0 ** -30, 252), (2.0 ** 20, 0), (2.0 ** 20, 3)])
-def test_mxfp4_down_scales_near_the_ends_of_their_range(product, oracle, x_scale, exponent):
+def test_mxfp4_down_scales_near_the_ends_of_their_range(product, oracle, x_scale, exponent, h, i, s):
     """Block scales of 2^125, 2^-127 and 2^-124 against activation rows small or large enough that every product and the result are
     ordinary numbers, on each kernel family's batches (the shared expert, of ordinary scales, adds nothing: its down rows are zero)."""
-    print(f"case mxfp4 scales 2^{exponent - 127}, activations times {x_scale}", flush=True)
-    cfg = abi.moe_config(512, 24, 3, 256, 256)
+    print(f"case mxfp4 scales 2^{exponent - 127}, activations times {x_scale}, {h} x {i}", flush=True)
+    cfg = abi.moe_config(h, 24, 3, i, s)
     weights, x = make_layer_inputs(cfg, "q4", 40, seed=exponent + 5)
     blocks = weights.raw[3].reshape(-1, 17)
     blocks[:, 0] = exponent
@@ -256,7 +257,7 @@ def test_mxfp4_down_scales_near_the_ends_of_their_range(product, oracle, x_scale
             np.testing.assert_allclose(w, want[2][:tokens], atol=2e-6, rtol=2e-5)
             error = np.abs(y.astype(np.float64) - want[0][:tokens]).max(axis=1)
             print(f"    error {(error / largest[:tokens, 0]).max():.2e} of the row's largest", flush=True)
-            assert (error <= 1e-5 * largest[:tokens, 0]).all()   # 32-bit sums of 256 products and three slots
+            assert (error <= 1e-5 * largest[:tokens, 0]).all()   # 32-bit sums of at most 640 products and three slots
 
 
 @pytest.mark.parametrize("h,i,s,k", [(512, 256, 256, 3), (768, 640, 1152, 2), (2560, 512, 640, 10), (512, 512, 2048, 12)])
