@@ -6,8 +6,8 @@
 // weights come from memory once, and once in registers serve eight rows at a time.
 //
 //   pf_k_batch_gate_up   gate and up products of 32 units, SwiGLU, the activation rows' digit images (expert order)
-//   pf_k_batch_down      down products of 128 output rows, FP32, in expert order (pf_k_pf_combine adds them up); of the q4
-//                        profile with a tile-ordered copy the shared expert's only, the routed ones by pf_k_mx_down
+//   pf_k_batch_down      down products of 128 output rows, FP32, in expert order (pf_k_pf_combine adds them up); of larger batches
+//                        of the q4 profile the shared expert's only, the routed ones by pf_k_mx_down
 //
 // Arithmetic: the decode kernels'.  Activations are digit images (integers per 32-group as balanced base-256 digits), weight
 // codes signed bytes, the group's dot product exact in integers, the group's scale and minimum applied in FP32.  PLANES digits:
@@ -159,21 +159,26 @@ template <bool ROWS> struct BatchRows<PF_Q8_0, ROWS> {   // the checkpoint profi
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
 };
 
-template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // row by row: a lane reads its row's whole block and keeps the low or the high nibbles
+template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // in tile order or row by row: a lane reads its row's whole block and keeps the low or the high nibbles
     static constexpr int GROUPS = 8;
     static constexpr bool MINIMA = false, MIN_OPERAND = false;
     uint4 q[8];
     uint32_t e2[4];
     __device__ __forceinline__ void load(const PfKernelArgs &a, int t, size_t e, int tile, int piece, int groups, int lane, const uint32_t *) {
         const size_t row0 = e * (size_t)a.n_out[t] + (size_t)(32 * tile);
-        const uint8_t *codes = a.w[t] + row0 * a.row_bytes[t], *scales = a.w[t] + a.scale_offset[t] + row0 * (size_t)a.blocks_per_row[t];
-        const uint32_t code_at = (uint32_t)(lane & 31) * (uint32_t)a.row_bytes[t], scale_at = (uint32_t)(lane & 31) * (uint32_t)a.blocks_per_row[t];
+        const int units = groups / 4;
+        const uint8_t *codes = ROWS ? a.w[t] + row0 * a.row_bytes[t] : a.wm + row0 / 32 * units * PF_I2T_CHUNK;
+        const uint8_t *scales = a.w[t] + a.scale_offset[t] + row0 * (size_t)a.blocks_per_row[t];   // (ROWS)
+        const uint32_t code_at = (uint32_t)(lane & 31) * (ROWS ? (uint32_t)a.row_bytes[t] : 16u);
+        const uint32_t scale_at = (uint32_t)(lane & 31) * (ROWS ? (uint32_t)a.blocks_per_row[t] : 4u);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int g = min(GROUPS * piece + 2 * r, groups - 2);
-            q[2 * r] = *reinterpret_cast<const uint4 *>((codes + 16 * g) + code_at);
-            q[2 * r + 1] = *reinterpret_cast<const uint4 *>((codes + 16 * (g + 1)) + code_at);
-            e2[r] = *reinterpret_cast<const uint16_t *>((scales + g) + scale_at);
+            const uint8_t *unit = codes + (g >> 2) * PF_I2T_CHUNK;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                q[2 * r + i] = *reinterpret_cast<const uint4 *>((ROWS ? codes + 16 * (g + i) : unit + pf_mxt_piece_at((g & 3) + i, 0)) + code_at);
+            e2[r] = *reinterpret_cast<const uint16_t *>((ROWS ? scales + g : unit + pf_mxt_scales_at(0) + (g & 3)) + scale_at);
         }
     }
     __device__ __forceinline__ void open() {}
@@ -182,7 +187,7 @@ template <bool ROWS> struct BatchRows<PF_MXFP4, ROWS> {   // row by row: a lane 
         return int4v{e2m1_twice4(q[g].x >> s), e2m1_twice4(q[g].y >> s), e2m1_twice4(q[g].z >> s), e2m1_twice4(q[g].w >> s)};
     }
     __device__ __forceinline__ int4v min_operand(int) const { return int4v{0, 0, 0, 0}; }
-    __device__ __forceinline__ float scale(int g) const {  return 0.5f * pf_e8m0_scale((e2[g >> 1] >> (8 * (g & 1))) & 255u); }   // the integers are twice the values
+    __device__ __forceinline__ float scale(int g) const { return 0.5f * pf_e8m0_scale((e2[g >> 1] >> (8 * (g & 1))) & 255u); }   // the integers are twice the values
     __device__ __forceinline__ float minimum(int) const { return 0.0f; }
 };
 
@@ -472,15 +477,9 @@ template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t
 // them), the operands past the registers through LDS (slower: LDS becomes the bottleneck for
 // IQ2_XXS), one matrix a wave at twice the occupancy (85 us).
 #define BATCH_WAVES 4
-// The q4 profile's routed down projection runs on the block-scaled product (pf_k_mx_down), as a chunk's, where the layer keeps that
-// copy: its activation rows leave the gate and up kernel as FP32 and become digit rows.  On the integers 101 tokens of the checkpoints'
-// widths took 157 us row by row and 120 from the copy; now 84, 7 for the rows and 14 for the shared expert's down projection.  24
-// tokens 77 -> 39 + 5 + 12, 300 tokens 229 -> 98 + 9 + 23.
-template <int FMT, int FMTS, int PLANES> __host__ __device__ __forceinline__ bool batch_down_scaled(const PfKernelArgs &a) {
-    return FMT == PF_Q4_K && FMTS == PF_Q8_0 && PLANES == 3 && a.wm != nullptr;
-}
+// float_rows: the routed experts' activation rows leave the kernel as FP32 (they become digit rows for pf_k_mx_down), else as images.
 template <int FMT, int FMTS, bool ROWS, int PLANES>
-__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a) {
+__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a, int float_rows) {
     __shared__ float partial[BATCH_WAVES][2][4][64];
     __shared__ BatchFactor factors[BATCH_WAVES][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
@@ -493,7 +492,7 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
     const int groups = a.hidden / 32, K = a.top_k;
     const uint32_t words = (uint32_t)pf_batch_image_words(PLANES, a.hidden);
     const size_t act_words = pf_batch_image_words(PLANES, a.inter > a.shared_inter ? a.inter : a.shared_inter);
-    const bool rows_only = batch_down_scaled<FMT, FMTS, PLANES>(a) && !it.shared;   // the down projection takes digit rows
+    const bool rows_only = float_rows && !it.shared;
     for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         float acc[2][4] = {};
@@ -700,19 +699,24 @@ void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, bool 
 template <int FG, int FD, int FS, bool ROWS, int PLANES>
 static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile_cap, hipStream_t stream, int last) {
     const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
-    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a);
+    // The q4 profile's routed down projection on the block-scaled product, as a chunk's, where the work is worth its launches: on the
+    // integers 101 tokens of the checkpoints' widths took 157 us row by row and 120 in tile order, there 84, 7 for the rows and 14 for the
+    // shared expert's down projection.  24 tokens 77 -> 39 + 5 + 12, 300 tokens 229 -> 98 + 9 + 23.
+    const bool scaled = FD == PF_MXFP4 && PLANES == 3 && a.wm && pf_batch_down_scaled(tokens, a.experts, a.top_k, a.hidden, a.inter, a.shared_inter);
+    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a, scaled ? 1 : 0);
     if (last < 4) return;
     const dim3 grid((a.hidden + 127) / 128, tile_cap);
-    if (FD == PF_MXFP4 && batch_down_scaled<FG, FS, PLANES>(a)) {
+    if (scaled) {
         pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
         pf_launch_mx_down(a, tokens, tile_cap - (unsigned)(tokens + 31) / 32, stream);
         hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, (tokens + 31) / 32, 32 / BATCH_ROWS), dim3(256), 0, stream, a, 1);
         return;
     }
-    // down rows: as gate and up where the layer has one format; Q2_K by whole tiles where they fit a wave's LDS
-    constexpr bool q2 = FD == PF_Q2_K;
-    if (q2 && 32 * a.row_bytes[3] <= BATCH_STAGE_BYTES)
-        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, q2 ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, 0);
+    // down rows: as gate and up where the layer has one format; Q2_K by whole tiles where they fit a wave's LDS, MXFP4 in tile order
+    // where the layer keeps that
+    constexpr bool either = FD == PF_Q2_K || (FD == PF_MXFP4 && PLANES == 3);
+    const bool lines = FD == PF_Q2_K ? 32 * a.row_bytes[3] <= BATCH_STAGE_BYTES : a.wm != nullptr;
+    if (either && lines) hipLaunchKernelGGL((pf_k_batch_down<FD, FS, either ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, 0);
     else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, 0);
 }
 

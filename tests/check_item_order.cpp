@@ -60,7 +60,15 @@ static void decode_down() {
     expect(!pf_decode_down_scaled(4, 10, 2560, 640), "four tokens", 0, 0, 0);
 }
 
+static void batch_down() {
+    expect(!pf_batch_down_scaled(17, 8, 2, 2048, 512, 512) && !pf_batch_down_scaled(400, 32, 2, 768, 256, 256) && !pf_batch_down_scaled(24, 128, 8, 512, 256, 256),
+           "small batches", 0, 0, 0);
+    expect(pf_batch_down_scaled(17, 512, 10, 2560, 640, 640) && pf_batch_down_scaled(101, 512, 10, 2560, 640, 640) && pf_batch_down_scaled(32, 32, 4, 1024, 512, 512),
+           "large batches", 0, 0, 0);
+}
+
 int main() {
+    batch_down();
     decode_down();
     slabs();
     places();
