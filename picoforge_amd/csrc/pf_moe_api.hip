@@ -904,24 +904,21 @@ struct HcTarget {   // residual streams to inject into instead of writing y
 //   up to batch_to   the kernels for a few rows per expert, which read an expert once for the batch and multiply its rows in
 //                    eights
 //   beyond           the grouped product of 32-row tiles
-// The lines lie where both sides measured the same, and follow the batch's pairs P and the layer's experts E, not its tokens
-// alone: with fewer experts the same tokens are more rows an expert.  Swept over E (top-k) = 16 (4), 32 (6), 64, 128, 256 (8),
-// 512 (10), uniform and Zipf(1.1) popularity, 5 to 400 tokens, the widths of the measured layer (one format throughout) and of
-// the checkpoints (profiles); P at the crossing, by E:
-//   pairs -> few rows      one format: Q4_K 224 at 64, beyond 32 tokens elsewhere; IQ2_XXS 172, 165, 216 at 32, 64, 128.  The profiles'
-//                          lines lie beyond their crossings (q2 35 to 57 pairs at any E, q4 54 to 142) at 10 and 16 tokens:
-//                          the decode kernels are closer to the result in 64 bits (2.9e-7 against 3.1e-7 and 3.3e-7)
-//   few rows -> grouped    one format 988..1000, 1002..1058, 929..1128, 1977..2167, 2376..2608, 3626..4000; q2 866..890, 918..925,
-//                          970..1678, 1659..2022, 2222..2731, 4000; q4 749..829, 797..853, 717..761, 1282..1344, 1877..2154, 3032..3285
-//   the same, IQ2_XXS gate and up rows as they are stored (slower to read for the few-row kernels)
-//                          572..589, 613..682, 533..563, 1430..1446, 1981..2033, 2004..3191; q2 573..632, 701..769, 459..535, 1008,
-//                          1552..1622, 2826..3196
-// The grouped product's time hardly grows until its tiles fill the chip more than once, so up to 64 experts the line is a
-// number of pairs; from there it pays for every expert met and the few-row kernels for every eight rows.  A rule on tokens
-// that fits 512 experts (32 / 240 for Q4_K, 32 / 320, 10 / 400, 16 / 400) is up to 1.42 times slower than the better side with
-// 64: 320 tokens of an IQ2_XXS layer 189 us against 133.  With this rule no size from 17 tokens on is above 1.10
-// (1.20 in batches whose neighbours share half of their experts, which meet fewer of them).  The q4 line stays above the
-// crossing at 512 experts (1.10 at 400 tokens): the few-row kernels are closer to 64 bits, 3.3e-7 against 5.4e-7.
+// The lines follow the batch's pairs P and the layer's experts E, not its tokens alone: with fewer experts the same tokens are more rows
+// an expert.  Up to 64 experts the second is a number of pairs, from there it pays for every expert met; a rule on tokens that fits
+// 512 experts (32 / 240 for Q4_K, 32 / 320, 10 / 400, 16 / 400) is 1.42 times slower than the better side with 64.
+// They were drawn where two sides took the same time, on earlier kernels.  Swept again over E (top-k) = 16 (4), 32 (6), 64, 128, 256
+// (8), 512 (10), uniform and Zipf(1.1) popularity, 5 to 420 tokens, the widths of the measured layer (one format throughout) and of the
+// checkpoints (profiles), the present kernels cross at
+//   pairs -> few rows      one format: Q4_K 224 pairs at 64 experts, beyond 32 tokens elsewhere; IQ2_XXS 192, 160, 224 at 32, 64, 128.
+//                          q2 from 32 to 64 pairs on, up to 1.30 beyond the crossing (8 tokens, 64 experts); q4 not up to 16 tokens,
+//                          but at 64 experts, 16
+//   few rows -> grouped    one format 112, 168, 136 to 192, 80 to 224, 136 to 2000, 280 to 3200 pairs; q2 112, 168, 400, 1000, 2560, 4000; q4
+//                          160, 240, 512, 512, 400, 280
+// so a batch just under the second line is 1.02 to 1.27 times slower than on the grouped product (125 tokens, 64 experts, Zipf 1.27;
+// 400 tokens of the q4 profile, 512 experts 1.21).  Both lines stay: the side that they keep is the one nearer to the result in 64
+// bits (60 tokens, decode kernels / few rows / grouped product: Q4_K 3.1 / 3.2 / 7.1e-7, IQ2_XXS 2.6 / 2.8 / 4.2e-7, q2 2.9 / 3.1 /
+// 4.4e-7, q4 2.6 / 2.8 / 4.8e-7).
 struct BatchRange { size_t pair_to, batch_to; };
 static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
     const int combination = pf_decode_tile_layer(moe->desc, moe->w_tiled, moe->w_itile, moe->w_qtile);
