@@ -30,9 +30,8 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 
-// halfs per row of a converted matrix: high parts, low parts, per 256-block the 16 group-sum halfs
+// halfs per row of the fp16 form: high parts, low parts, per (started) 256 columns the 16 group-sum halfs
 // [even groups: 4 high, 4 low][odd groups: 4 high, 4 low]
-// halfs per row of the fp16 form: high parts, low parts, 16 group-sum parts per (started) 256 columns
 __host__ __device__ constexpr size_t pf_half_row(int cols) { return 2 * (size_t)cols + 16 * (((size_t)cols + 255) / 256); }
 
 // ---- Q4_K tensors in tile order (once, at upload) ---------------------------------------------
@@ -151,7 +150,7 @@ __global__ void __launch_bounds__(1024) pf_k_pf_group_rows(PfKernelArgs a, int t
 // of its four waves only took part in the maximum: 22528 rows of 640 values took 36.2 us (routed) + 8.8 (shared), 21.6 so.
 template <int PARTS>
 __device__ __forceinline__ void rows_to_half_short(size_t block, const float *src, size_t src_pitch, int cols, size_t rows, half_t *dst,
-                                                   float *scale_out, float *max2_out, uint32_t *error_word) {
+                                                   float *scale_out, uint32_t *error_word) {
     const size_t row = block * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int lane = pf_lane();
@@ -207,10 +206,7 @@ __device__ __forceinline__ void rows_to_half_short(size_t block, const float *sr
             sums[4] = sl;
         }
     }
-    if (lane == 0) {
-        scale_out[row] = scale;
-        if (max2_out) max2_out[row] = m * m;
-    }
+    if (lane == 0) scale_out[row] = scale;
 }
 
 // Two matrices of such rows in one launch (the routed and the shared activation rows): workgroups [0, blocks_a) take
@@ -221,9 +217,9 @@ __global__ void __launch_bounds__(256) pf_k_rows_to_half_short2(const float *src
                                                                 half_t *dst_b, float *scale_b, uint32_t *error_word) {
     if (blockIdx.x < blocks_a) {
         if (DIGITS) pf_rows_to_digits(blockIdx.x, src_a, cols_a, rows_a, reinterpret_cast<uint32_t *>(dst_a), scale_a, error_word);
-        else rows_to_half_short<PARTS>(blockIdx.x, src_a, (size_t)cols_a, cols_a, rows_a, dst_a, scale_a, nullptr, error_word);
+        else rows_to_half_short<PARTS>(blockIdx.x, src_a, (size_t)cols_a, cols_a, rows_a, dst_a, scale_a, error_word);
     }
-    else rows_to_half_short<PARTS>(blockIdx.x - blocks_a, src_b, (size_t)cols_b, cols_b, rows_b, dst_b, scale_b, nullptr, error_word);
+    else rows_to_half_short<PARTS>(blockIdx.x - blocks_a, src_b, (size_t)cols_b, cols_b, rows_b, dst_b, scale_b, error_word);
 }
 
 static void launch_rows_to_half(const float *src, size_t src_pitch, int cols, size_t rows, half_t *dst, float *scale_out,
@@ -637,7 +633,8 @@ __device__ __forceinline__ void gemm_block(GemmBlock<FMT> &w, half8v &sums, cons
     for (int r = 0; r < 16; r++) acc[r] = fmaf(d, part[r], acc[r]);
 }
 
-// The same for Q8_0, whose groups are added up one by one, the even and the odd ones apart (a row of sums half as long); groups: 8, or 4 in the last block of a row of an odd number of 128 columns.
+// The same for Q8_0, whose groups are added up one by one, the even and the odd ones apart (a row of sums half as long); groups: 8,
+// or 4 in the last block of a row of an odd number of 128 columns.
 template <int PARTS>
 __device__ __forceinline__ void gemm_block_q8(GemmBlock<PF_Q8_0> &w, const GemmSource &src, uint32_t at, uint32_t head_at, int next_kb, int groups, int wave,
                                               const lds_byte *__restrict from, lds_byte *__restrict to, float16v (&acc)[2]) {
