@@ -917,8 +917,8 @@ struct HcTarget {   // residual streams to inject into instead of writing y
 //                          160, 240, 512, 512, 400, 280
 // so a batch just under the second line is 1.02 to 1.27 times slower than on the grouped product (125 tokens, 64 experts, Zipf 1.27;
 // 400 tokens of the q4 profile, 512 experts 1.21).  Both lines stay: the side that they keep is the one nearer to the result in 64
-// bits (60 tokens, decode kernels / few rows / grouped product: Q4_K 3.1 / 3.2 / 7.1e-7, IQ2_XXS 2.6 / 2.8 / 4.2e-7, q2 2.9 / 3.1 /
-// 4.4e-7, q4 2.6 / 2.8 / 4.8e-7).
+// bits (60 tokens, 24 experts, decode kernels / few rows / grouped product: Q4_K 3.2 / 3.2 / 6.7e-7, IQ2_XXS 2.6 / 2.8 / 4.0e-7, q2
+// 2.7 / 3.0 / 4.8e-7, q4 2.7 / 2.8 / 4.4e-7).
 struct BatchRange { size_t pair_to, batch_to; };
 static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
     const int combination = pf_decode_tile_layer(moe->desc, moe->w_tiled, moe->w_itile, moe->w_qtile);
