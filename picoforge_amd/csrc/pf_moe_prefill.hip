@@ -368,10 +368,10 @@ enum { PF_GEMM_GATE_UP = 0, PF_GEMM_DOWN = 1 };
 // its block up or waits, the others feed the matrix core.
 //
 // Bound by power and by the bytes together: at 1024 tokens of the benchmark's Q4_K layer (640 row tiles, 604 MB of gate and up
-// weights) the card draws 1.28 kW and its clock falls to 1.8 GHz; without the memory reads the launch takes 137 us, without
-// the products 157, as it is 177.  Before, with loader waves that moved every operand through a ring in LDS and a barrier every
-// 64 columns, it took 201; the down launch 103 against 109, IQ2_XXS (777 tokens) 156 + 92 against 201 + 102, Q4_K rows of 2560
-// against 640 units (2048 tokens; units in slabs of 128, not 256) 375 against 477.
+// weights) the card draws 1.28 kW and its clock falls to 1.8 GHz; repeated by itself the launch takes 177 us, without the memory reads
+// 137, without the products 157.  Before, loader waves moved every operand through a ring in LDS with a barrier every 64 columns.
+// Traced within forwards, in turn, gate and up / down, us, before and now (units in slabs of 128, not 256): 1024 tokens 222 / 122 ->
+// 207 / 117, 2048 tokens 317 / 168 -> 304 / 173, IQ2_XXS, 777 tokens 229 / 116 -> 184 / 106.
 //
 //   copy   [part: high, low][64 columns][eight rows][16-byte chunk of the 64 columns][row][16 bytes]
 //
@@ -560,7 +560,7 @@ __device__ __forceinline__ half8v half8_of_signed_bytes(uint32_t b0, uint32_t b1
 // Q8_0: signed code bytes, a half scale per 32-group: a group's partial sums times its scale.  Lane (n, h) loads bytes 16h..16h+15 of a
 // group; step i is half i % 2 of its bytes in group i / 2 of the block.  Half scales are no integers, so they stay out of the
 // operand.  The shared expert of the checkpoint profiles: its gate and up tiles ride with the routed ones' launch (2048 tokens of 2560 x
-// 640: 411 us, against 377 and 90 for a launch of the plain kernel), its down tiles are a launch of 38 us (plain kernel: 50).
+// 640, the q4 profile: 433 us traced, before 490 and 90 for a launch of the plain kernel), its down tiles are a launch of 39 us.
 template <> struct GemmBlock<PF_Q8_0> {
     uint4v code[8];
     uint32_t head[4];   // of a run: its two groups' scales
