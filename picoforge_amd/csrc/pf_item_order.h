@@ -19,35 +19,34 @@ PF_HD int pf_slabs_each(int all, int most, unsigned tiles) {
 // into groups of consecutive ones and the groups dealt to the XCDs in turn; the items of a group (its tiles' slabs) get numbers eight
 // apart: neighbouring workgroups of one XCD, one L2, at the same time.  The slabs of a row tile read the same activation rows, and the
 // row tiles of one expert, neighbours in the list, the same weights: fetched once from memory where they fall into one group.  Groups
-// are of eight tiles where that leaves every XCD eight of them, else smaller, so that a short list is spread over the chip.  The shared
-// expert's tiles, the list's last, follow one by one: first on the XCDs that have a group less than the others, then on all.
-// (Groups of eight whatever the list, the shared expert's among them: eight routed tiles were one XCD's, 257 tokens' shared tiles two XCDs'.
-// 7 tokens of a Q4_K layer of 8 experts, 4096 x 1536, 143 us, now 89; the q4 profile, 32 experts of 2560 x 768 beside a shared expert of
+// are of eight tiles where that leaves every XCD eight of them, else smaller, so that a short list is spread over the chip.  (Groups of
+// eight whatever the list, the shared expert's among them: eight routed tiles were one XCD's, 257 tokens' shared tiles two XCDs'.  7
+// tokens of a Q4_K layer of 8 experts, 4096 x 1536, 143 us, now 89; the q4 profile, 32 experts of 2560 x 768 beside a shared expert of
 // 3072, 257 tokens 394, now 274.)
+// The shared expert's tiles, the list's last, are dealt one by one, first to the XCDs that have a group less than the others, then to
+// all, and are an XCD's first: a profile's Q8_0 tile takes longer than a routed one and at the list's end it was the launch's (q4 profile,
+// 64 experts of 3072 x 1024, sixteen slots, 55 tokens 235 us a forward, now 226; 8 experts of 4096 x 1536, 450 tokens 267, now 223).
 #define PF_XCDS 8
 PF_HD int pf_group_shift(uint32_t routed) { return routed >= 512 ? 3 : routed >= 256 ? 2 : routed >= 128 ? 1 : 0; }
 struct PfItemPlace { bool any; uint32_t tile; int slab; };
 PF_HD PfItemPlace pf_item_place(uint32_t q, int slabs, int shift, uint32_t routed, uint32_t shared) {
-    const uint32_t xcd = q % PF_XCDS, turn = q / PF_XCDS, each = 1u << shift, groups = (routed + each - 1) >> shift, full = groups / PF_XCDS, more = groups % PF_XCDS;
+    const uint32_t xcd = q % PF_XCDS, turn = q / PF_XCDS, each = 1u << shift, groups = (routed + each - 1) >> shift, more = groups % PF_XCDS;
+    const uint32_t lacking = more ? PF_XCDS - more : 0, gap = lacking << shift;   // XCDs with a group less than the first `more`; their free places
     uint32_t r = turn / (uint32_t)slabs;   // the XCD's tile
     PfItemPlace p;
     p.slab = (int)(turn % (uint32_t)slabs);
-    const uint32_t before = (xcd < more ? full + 1 : full) << shift;   // its places for routed tiles
-    if (r < before) {
-        p.tile = (((r >> shift) * PF_XCDS + xcd) << shift) + (r & (each - 1));
-        p.any = p.tile < routed;
+    // its shared tiles: number r of the gap is lacking * r + own, beyond the gap every eighth
+    auto count = [](uint32_t first, uint32_t end, uint32_t step) { return first < end ? (end - first - 1) / step + 1 : 0u; };
+    const bool fills = lacking && xcd >= more;
+    const uint32_t in_gap = fills ? count(xcd - more, shared < gap ? shared : gap, lacking) : 0, mine = in_gap + count(gap + xcd, shared, PF_XCDS);
+    if (r < mine) {
+        p.tile = routed + (r < in_gap ? lacking * r + xcd - more : gap + PF_XCDS * (r - in_gap) + xcd);
+        p.any = true;
         return p;
     }
-    r -= before;
-    uint32_t s = PF_XCDS * r + xcd;
-    if (more) {
-        const uint32_t lacking = PF_XCDS - more;
-        if (xcd < more) s += lacking << shift;
-        else if (r < each) s = lacking * r + xcd - more;
-        else s += (lacking << shift) - PF_XCDS * each;
-    }
-    p.tile = routed + s;
-    p.any = s < shared;
+    r -= mine;
+    p.tile = (((r >> shift) * PF_XCDS + xcd) << shift) + (r & (each - 1));
+    p.any = p.tile < routed;
     return p;
 }
 // numbers that cover up to `routed` tiles and `shared` more

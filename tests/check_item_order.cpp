@@ -34,10 +34,12 @@ static void places() {
                     const int shift = pf_group_shift(routed + more);
                     const uint32_t tiles = routed + shared, numbers = pf_item_numbers(slabs, shift, routed + more, shared);
                     std::vector<int> times((size_t)tiles * slabs);
-                    uint32_t routed_on[PF_XCDS] = {}, shared_on[PF_XCDS] = {};
+                    uint32_t routed_on[PF_XCDS] = {}, shared_on[PF_XCDS] = {}, routed_seen[PF_XCDS] = {};
                     for (uint32_t q = 0; q < numbers; q++) {
                         const PfItemPlace p = pf_item_place(q, slabs, shift, routed, shared);
                         if (!p.any) continue;
+                        if (p.tile < routed) routed_seen[q % PF_XCDS] = 1;
+                        else expect(!routed_seen[q % PF_XCDS], "a shared tile behind a routed one", (int)routed, (int)shared, (int)q);
                         expect(p.tile < tiles && p.slab >= 0 && p.slab < slabs, "an item that is not there", (int)routed, (int)shared, (int)q);
                         if (p.tile >= tiles || p.slab < 0 || p.slab >= slabs) continue;
                         times[(size_t)p.tile * slabs + p.slab]++;
