@@ -240,12 +240,16 @@ extern "C" int pf_hip_moe_create(const PfHipMoeDesc *desc, const void *const hos
         m->total_bytes += slab_floats * sizeof(float);
     }
     m->decode_ready = !m->streamed && pf_decode_supported(*desc);
-    // prefill path: squared norms of the router rows (the routing tolerance's bound)
+    // prefill path: squared norms of the router rows (the routing tolerance's bound), the router as operands
     m->prefill_ready = !m->streamed && pf_prefill_supported(*desc);
     if (m->prefill_ready) {
+        const size_t parts = pf_router_parts_bytes((int)E, (int)h);
         hipError_t e = hipMalloc((void **)&m->w_norm2, E * sizeof(float));
+        if (e == hipSuccess) e = hipMalloc((void **)&m->router_parts, parts);
         if (e == hipSuccess) {
             pf_launch_row_norm2(reinterpret_cast<const float *>(m->w[0]), (int)E, (int)h, m->w_norm2, nullptr);
+            pf_launch_router_parts(reinterpret_cast<const float *>(m->w[0]), (int)E, (int)h, m->router_parts, nullptr);
+            m->total_bytes += parts;
             e = hipDeviceSynchronize();
         }
         if (e != hipSuccess) {
@@ -415,6 +419,7 @@ extern "C" void pf_hip_moe_destroy(PfHipMoe *m) {
     if (!m) return;
     for (int a = 0; a < 8; a++) if (m->w[a]) (void)hipFree(m->w[a]);
     if (m->w_norm2) (void)hipFree(m->w_norm2);
+    if (m->router_parts) (void)hipFree(m->router_parts);
     if (m->router_t) (void)hipFree(m->router_t);
     for (int a = 0; a < 8; a++) if (m->w_tiled[a]) (void)hipFree(m->w_tiled[a]);
     for (int a = 0; a < 8; a++) if (m->w_itile[a]) (void)hipFree(m->w_itile[a]);
@@ -882,7 +887,7 @@ static PfKernelArgs make_args(const PfHipMoe *m, PfHipWork *w, const float *d_x,
     a.error_word = w->error_word; a.exact_rows = w->exact_rows; a.route_flags = w->route_flags;
     a.x16 = w->x16; a.act16 = w->act16; a.sact16 = w->sact16;
     a.x_scale = w->x_scale; a.act_scale = w->act_scale; a.sact_scale = w->sact_scale;
-    a.w_norm2 = m->w_norm2; a.down = w->down;
+    a.w_norm2 = m->w_norm2; a.router_parts = m->router_parts; a.down = w->down;
     a.counts = w->counts; a.offsets = w->offsets; a.pair_to_row = w->pair_to_row; a.row_to_pair = w->row_to_pair;
     a.group_bad = w->group_bad; a.tiles = w->tiles; a.items = w->items;
     a.token_cap = (uint32_t)w->cap;
@@ -964,7 +969,7 @@ static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_
         snprintf(g_error, sizeof g_error, "the layer's routed experts are not resident: forward it through an expert pool");
         return PF_HIP_E_UNSUPPORTED;
     }
-    const bool aligned = (x_pitch % 4 == 0) && ((uintptr_t)d_x % 16 == 0);
+    const bool aligned = (x_pitch % 4 == 0) && ((uintptr_t)d_x % 16 == 0) && x_pitch < (size_t)1 << 27;   // (eight rows by 32-bit offsets)
     const Family family = aligned ? kernel_family(moe, work, tokens) : FAMILY_GENERAL;
     if (family == FAMILY_DECODE) {
         pf_launch_decode(a, (int)tokens, s, work->stage_limit);

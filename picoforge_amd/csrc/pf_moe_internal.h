@@ -56,6 +56,7 @@ struct PfKernelArgs {
                                      // parts, the low parts, then 8 + 8 group-sum parts per 256 columns
     float *x_scale, *act_scale, *sact_scale;   // per row: the power of two the fp16 form was divided by
     const float *w_norm2;            // [experts] squared norm of each router row
+    const uint8_t *router_parts;     // router as operands of the chunks' logits (pf_k_router_parts)
     float *down;                     // [pairs + tokens, hidden] down products in expert order, then the shared expert's
     uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles;
     const uint32_t *items;           // row tiles as {expert, first row, rows, first row within the expert} (pf_k_group_fused)
@@ -169,6 +170,7 @@ struct PfHipMoe {
                                      // expert on pool slots: 1 Q4_K, 2 IQ2_XXS throughout, 3, 4 the q2, q4 checkpoint profile
                                      // (0: the general kernels serve every batch)
     float *w_norm2;                  // [experts] squared norm of each router row
+    uint8_t *router_parts;           // router as bf16 parts in operand order
     float *router_t;                 // [slab of 64 experts][hidden / 4][64][4] copy of the router
     uint8_t *w_tiled[8];             // Q4_K expert tensors in tile order, for every kernel family (or null)
     uint8_t *w_itile[8];             // tile-ordered second copy of IQ2_XXS expert tensors, decode and few rows per expert (or null)
@@ -276,6 +278,8 @@ void pf_launch_group(const PfKernelArgs &a, const uint32_t *ids, int tokens, hip
 void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream);
 void pf_launch_q4k_tile(const uint8_t *d_src, uint8_t *d_dst, size_t rows, int blocks_per_row, hipStream_t stream);
 void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hipStream_t stream);
+size_t pf_router_parts_bytes(int experts, int cols);
+void pf_launch_router_parts(const float *d_w, int experts, int cols, void *d_out, hipStream_t stream);
 size_t pf_prefill_half_row(int cols);   // halfs per row of the fp16 form of a matrix with `cols` columns
 int pf_prefill_max_tiles(int tokens, int experts, int top_k);
 size_t pf_prefill_most_tokens(int hidden);   // that one launch of pf_launch_prefill takes

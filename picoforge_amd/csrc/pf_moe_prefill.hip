@@ -1,7 +1,7 @@
 // Prefill path: a chunk of tokens through one MoE layer as grouped matrix products on the
 // matrix cores.
 //
-//   pf_k_pf_router      router logits [T, E] by FP32 MFMA
+//   pf_k_pf_router      router logits [T, E], both factors as three bf16 parts
 //   routing             the kernels of pf_moe_route.hip (serial-order re-route of close tokens)
 //   pf_k_pf_group_rows  grouping of the pairs (pf_group_device.h); beside it f32 rows -> power-of-two scaled fp16
 //                       pairs (high + low part) and the per-32-group sums, the scale, finite check
@@ -242,33 +242,78 @@ void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hip
     hipLaunchKernelGGL(pf_k_row_norm2, dim3(rows), dim3(64), 0, stream, d_w, cols, d_out);
 }
 
-// ---- router logits by FP32 MFMA ----------------------------------------------------------------
+// ---- router logits by three bf16 parts of every factor -----------------------------------------
 // Workgroup = a tile of 32 TR tokens x 32 TC experts, its eight waves an eighth of the columns each (the
 // partial tiles are added in wave order).  Also writes the routing tolerance's bound on the sum of
 // squared products, max(x)^2 * |w_e|^2.  (The shared router's logit comes with the rows' conversion.)
 //
-// Operands.  A product step wants, from lane (i, kk), element k = kk of row i: fetched like that
-// from global memory, every load instruction touches 32 rows, and the address unit, which takes a
-// cache line at a time, sets the pace (the kernel took 3.3 times the matrix cores' time at the
-// benchmark shape).
-// Instead a wave fetches a 32-column piece of its 32 + 32 rows as eight instructions of eight whole
-// 128-byte lines each (lane = 8 * row + 16-byte piece), stores it into LDS of its own at a row
-// pitch of 144 bytes, and reads its operands from there, 16 bytes a lane: columns
-// 4 (2 c + kk) .. + 3 for steps 4 c .. 4 c + 3, the same pairing for both operands.  The next
-// piece's global loads are on their way while the current one is multiplied; the LDS is the
-// wave's alone, so no barrier is needed before the partial tiles meet.
+// A value is h + m + l exactly: h its upper eight significant bits (cut off, so that the largest floats do not round up to
+// infinity), m the rest rounded to eight, l what that leaves.  Of the nine products of two values six are formed, exact in
+// the FP32 sums; the three left out are below 2^-23 of the product together, and l's sign is as good as random.
+//
+// The experts' parts are made once, at upload, in the order in which a wave takes them as operands (pf_k_router_parts): 1 KB an
+// instruction, no conversion.  A row of x is fetched in 32-column pieces, whole 128-byte lines (lane = 8 * row + 16-byte piece),
+// passes through LDS of the wave's own (row pitch 144 bytes; no barrier) because a product step wants columns 8 h .. 8 h + 7 of row i
+// from lane (i, h), and is split there, a step ahead of its products.
+//
+// Bound by what the L2 hands out: 2048 tokens of width 2560 against 512 experts are 420 MB of operands in 41 us traced.  On the FP32
+// instruction, whose products alone take 34, it was 75; with both factors split in the kernel 53, bound by the vector instructions.
+// 1024 tokens of width 2048: 25.4 us (FP32 38); tiles of 64 x 32 instead of 32 x 64 27.1, two pieces ahead no faster.  Error
+// against 64 bits (2-norm; 2047, 1025, 600, 460 tokens): 3.2, 3.5, 2.5, 3.4e-7, on FP32 3.8, 4.1, 2.9, 3.9e-7.
 typedef float float4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+struct RouterParts { uint4v part[3]; };
+__device__ __forceinline__ uint32_t router_round2(float a, float b) {   // (whole vectors are converted a value at a time)
+    typedef float float2v __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2v{a, b}, bf16x2));
+}
+__device__ __forceinline__ RouterParts router_parts(float4v a, float4v b) {
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    RouterParts r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t u = __float_as_uint(x[2 * i]), v = __float_as_uint(x[2 * i + 1]);
+        const float u1 = x[2 * i] - __uint_as_float(u & 0xffff0000u), v1 = x[2 * i + 1] - __uint_as_float(v & 0xffff0000u);
+        const uint32_t middle = router_round2(u1, v1);
+        r.part[0][i] = __builtin_amdgcn_perm(v, u, 0x07060302u);
+        r.part[1][i] = middle;
+        r.part[2][i] = router_round2(u1 - __uint_as_float(middle << 16), v1 - __uint_as_float(middle & 0xffff0000u));
+    }
+    return r;
+}
+
+// Router rows [experts][cols] -> [tile of 32][16 columns][part][lane (i, h): row i, columns 8 h .. 8 h + 7][8 bf16]; rows beyond the
+// last are zeros.  A thread per lane of a step.
+__global__ void __launch_bounds__(256) pf_k_router_parts(const float *w, int experts, int cols, uint4v *out, size_t threads) {
+    const size_t id = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (id >= threads) return;
+    const size_t step = id >> 6, tile = step / (size_t)(cols / 16);
+    const int lane = (int)(id & 63), row = (int)(32 * tile) + (lane & 31), c = 16 * (int)(step % (size_t)(cols / 16)) + 8 * (lane >> 5);
+    float4v a = {0}, b = {0};
+    if (row < experts) {
+        const float4v *src = reinterpret_cast<const float4v *>(w + (size_t)row * cols + c);
+        a = src[0]; b = src[1];
+    }
+    const RouterParts r = router_parts(a, b);
+#pragma unroll
+    for (int p = 0; p < 3; p++) out[(3 * step + p) * 64 + lane] = r.part[p];
+}
+size_t pf_router_parts_bytes(int experts, int cols) { return (size_t)((experts + 31) / 32) * 32 * cols * 6; }
+void pf_launch_router_parts(const float *d_w, int experts, int cols, void *d_out, hipStream_t stream) {
+    const size_t threads = (size_t)((experts + 31) / 32) * (size_t)(cols / 16) * 64;
+    hipLaunchKernelGGL(pf_k_router_parts, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, d_w, experts, cols, reinterpret_cast<uint4v *>(d_out), threads);
+}
+
 #define PF_ROUTER_PITCH 36   // floats between rows of a staged piece: eight neighbouring lanes' 16-byte reads cover all banks
 #define PF_ROUTER_WAVES 8
-#define PF_ROUTER_LDS(TR, TC) (PF_ROUTER_WAVES * ((TR) + (TC)) * 32 * PF_ROUTER_PITCH * 4)
-// Bound by the matrix cores (two thirds of a wave's life at 2048 tokens, the rest waits for first loads and the sums at the
-// end).  1024 tokens, 512 experts, rows of 2048: 28.1 us with 64 x 32 tiles, 30.7 with 32 x 32 (a workgroup reads 96 rows
-// for two of their tiles, instead of 128); 2048 tokens, rows of 2560: 66.8 us, 67.7.
+// the staged pieces, later the partial tiles
+constexpr int router_lds_bytes(int tr, int tc) { return PF_ROUTER_WAVES * 128 * tr * (32 * tc > PF_ROUTER_PITCH ? 32 * tc : PF_ROUTER_PITCH); }
 template <int TR, int TC>
 __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_waves_per_eu(2))) pf_k_pf_router(PfKernelArgs a, int tokens) {
-    extern __shared__ __align__(16) float router_lds[];   // [wave][x rows, then experts][column]; later the waves' partial tiles
+    extern __shared__ __align__(16) float router_lds[];   // [wave][x row][column]; later the waves' partial tiles
     __shared__ uint32_t largest[32 * TR];                 // the rows' largest magnitudes, as bits
-    const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = threadIdx.x >> 6;
+    const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t0 = blockIdx.x * 32 * TR, e0 = blockIdx.y * 32 * TC;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.route_flags[0] = 0;   // the routing's list starts empty
     if (threadIdx.x < 32 * TR) largest[threadIdx.x] = 0;
@@ -276,58 +321,100 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
     // the waves split the rows' 128-byte lines (hidden is a multiple of 32)
     const int lines = H / 32, l0 = lines * wave / PF_ROUTER_WAVES, l1 = lines * (wave + 1) / PF_ROUTER_WAVES;
     const int lr = lane >> 3, piece = lane & 7;   // fetch: row within a group of eight, 16-byte piece of the line
-    constexpr int ROWS = 4 * (TR + TC);           // groups of eight rows
-    const float4v *src[ROWS];
+    constexpr int GROUPS = 4 * TR;                // of eight rows
+    // a buffer per eight x rows, one for the experts' parts; rows beyond the last are zeros
+    PfBuffer x_rows[GROUPS];
 #pragma unroll
-    for (int g = 0; g < ROWS; g++) {
-        const int r = 8 * g + lr;
-        src[g] = (g < 4 * TR ? reinterpret_cast<const float4v *>(a.x + (size_t)min(t0 + r, tokens - 1) * a.x_pitch)
-                             : reinterpret_cast<const float4v *>(a.w[0] + (size_t)min(e0 + r - 32 * TR, E - 1) * H * 4)) + piece;
+    for (int g = 0; g < GROUPS; g++) {
+        const int first = t0 + 8 * g, rows = min(max(tokens - first, 0), 8);
+        x_rows[g] = pf_buffer(a.x + (size_t)min(first, tokens - 1) * a.x_pitch, rows ? (uint32_t)(((size_t)(rows - 1) * a.x_pitch + H) * 4) : 0);
     }
-    float *mine = router_lds + (size_t)wave * (TR + TC) * 32 * PF_ROUTER_PITCH;
+    const uint32_t tile_bytes = 192u * (uint32_t)H;
+    const PfBuffer experts = pf_buffer(a.router_parts + (size_t)(e0 / 32) * tile_bytes, (uint32_t)min(TC, (E - e0 + 31) / 32) * tile_bytes);
+    const int x_at = (int)((uint32_t)lr * (uint32_t)a.x_pitch * 4u + 16u * (uint32_t)piece), w_at = 16 * lane;
+    float *mine = router_lds + (size_t)wave * TR * 32 * PF_ROUTER_PITCH;
     float16v acc[TR][TC];
 #pragma unroll
     for (int r = 0; r < TR; r++)
 #pragma unroll
         for (int c = 0; c < TC; c++) acc[r][c] = float16v{0};
-    float most[4 * TR] = {};
+    float most[GROUPS] = {};
+    float4v fetched[GROUPS], raw[TR][2];
+    RouterParts x[2][TR], w[2][TC];   // of the two steps of 16 columns that a piece is
+    auto fetch = [&](int l) {
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) fetched[g] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(x_rows[g], x_at, 128 * min(l, l1 - 1), 0));
+    };
+    auto request = [&](int step, int l) {
+#pragma unroll
+        for (int c = 0; c < TC; c++)
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+                w[step][c].part[p] = __builtin_amdgcn_raw_buffer_load_b128(experts, w_at, (int)((uint32_t)c * tile_bytes + 3072u * (uint32_t)(2 * min(l, l1 - 1) + step) + 1024u * p), 0);
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+            const float4v v = fetched[g];
+            *reinterpret_cast<float4v *>(mine + (8 * g + lr) * PF_ROUTER_PITCH + 4 * piece) = v;
+            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most[g]) : "v"(v.x), "v"(v.y));   // (fmaxf spends an instruction on quieting every operand)
+            asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most[g]) : "v"(v.z), "v"(v.w));
+        }
+    };
+    auto take = [&](int step) {
+#pragma unroll
+        for (int q = 0; q < TR; q++) {
+            const float *at = mine + (32 * q + i) * PF_ROUTER_PITCH + 16 * step + 8 * kk;
+            raw[q][0] = *reinterpret_cast<const float4v *>(at);
+            raw[q][1] = *reinterpret_cast<const float4v *>(at + 4);
+        }
+    };
+    // step's products, the other step's rows split meanwhile: a few vector instructions behind every product
+    auto products = [&](int step) {
+#pragma unroll
+        for (int q = 0; q < TR; q++) x[step ^ 1][q] = router_parts(raw[q][0], raw[q][1]);
+#pragma unroll
+        for (int p = 0; p < 6; p++) {   // l h, h l, m m, m h, h m, h h
+            constexpr int px[6] = {2, 0, 1, 1, 0, 0}, pw[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int r = 0; r < TR; r++)
+#pragma unroll
+                for (int c = 0; c < TC; c++)
+                    acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x[step][r].part[px[p]]), __builtin_bit_cast(bf16x8, w[step][c].part[pw[p]]), acc[r][c], 0, 0, 0);
+        }
+#pragma unroll
+        for (int m = 0; m < 6 * TR * TC; m++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                               // a product
+            __builtin_amdgcn_sched_group_barrier(0x002, (46 * TR + 6 * TR * TC - 1) / (6 * TR * TC), 0);   // vector instructions
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
     if (l0 < l1) {
-        float4v fetched[ROWS];
+        fetch(l0);
+        request(0, l0);
+        request(1, l0);
+        stage();
+        fetch(l0 + 1);
+        take(0);
 #pragma unroll
-        for (int g = 0; g < ROWS; g++) fetched[g] = src[g][8 * l0];
+        for (int q = 0; q < TR; q++) x[0][q] = router_parts(raw[q][0], raw[q][1]);
+        take(1);
         for (int l = l0; l < l1; l++) {
-            // the piece fetched last into LDS (after the reads of the piece before it, in the wave's program order),
-            // then the next one's loads on their way (the last step fetches its own piece again; two pieces ahead
-            // measured no faster)
-#pragma unroll
-            for (int g = 0; g < ROWS; g++) *reinterpret_cast<float4v *>(mine + (8 * g + lr) * PF_ROUTER_PITCH + 4 * piece) = fetched[g];
-#pragma unroll
-            for (int g = 0; g < 4 * TR; g++) {
-                const float4v v = fetched[g];
-                most[g] = fmaxf(most[g], fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-            }
-            const int next = l + 1 < l1 ? l + 1 : l;
-#pragma unroll
-            for (int g = 0; g < ROWS; g++) fetched[g] = src[g][8 * next];
+            products(0);
+            request(0, l + 1);
+            stage();   // the next piece
+            fetch(l + 2);
+            take(0);
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                float4v v[TR + TC];
-#pragma unroll
-                for (int q = 0; q < TR + TC; q++)
-                    v[q] = *reinterpret_cast<const float4v *>(mine + (32 * q + i) * PF_ROUTER_PITCH + 4 * (2 * s + kk));
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-#pragma unroll
-                    for (int r = 0; r < TR; r++)
-#pragma unroll
-                        for (int c = 0; c < TC; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[r][k], v[TR + c][k], acc[r][c], 0, 0, 0);
-            }
+            products(1);
+            request(1, l + 1);
+            take(1);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     __syncthreads();   // the staged pieces have been read
 #pragma unroll
-    for (int g = 0; g < 4 * TR; g++) atomicMax(&largest[8 * g + lr], __float_as_uint(most[g]));
+    for (int g = 0; g < GROUPS; g++) atomicMax(&largest[8 * g + lr], __float_as_uint(most[g]));
     constexpr int REGS = 16 * TR * TC;
 #pragma unroll
     for (int r = 0; r < REGS; r++) router_lds[(wave * REGS + r) * 64 + lane] = acc[r / 16 / TC][r / 16 % TC][r % 16];
@@ -337,7 +424,7 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
         const int r = wave + PF_ROUTER_WAVES * q;
         float logit = router_lds[r * 64 + lane];
 #pragma unroll
-        for (int w = 1; w < PF_ROUTER_WAVES; w++) logit += router_lds[(w * REGS + r) * 64 + lane];
+        for (int v = 1; v < PF_ROUTER_WAVES; v++) logit += router_lds[(v * REGS + r) * 64 + lane];
         const int row = t0 + 32 * (r / 16 / TC) + 8 * ((r & 15) >> 2) + 4 * kk + (r & 3), col = e0 + 32 * (r / 16 % TC) + i;
         if (row >= tokens || col >= E) continue;
         a.logits[(size_t)row * E + col] = logit;
@@ -348,10 +435,10 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
 template <int TR, int TC>
 static void launch_router(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_router<TR, TC>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       PF_ROUTER_LDS(TR, TC)) == hipSuccess;   // more than the default 64 KB
+                                                       router_lds_bytes(TR, TC)) == hipSuccess;   // more than the default 64 KB
     (void)configured;
     const dim3 grid((tokens + 32 * TR - 1) / (32 * TR), (a.experts + 32 * TC - 1) / (32 * TC));
-    hipLaunchKernelGGL((pf_k_pf_router<TR, TC>), grid, dim3(64 * PF_ROUTER_WAVES), PF_ROUTER_LDS(TR, TC), stream, a, tokens);
+    hipLaunchKernelGGL((pf_k_pf_router<TR, TC>), grid, dim3(64 * PF_ROUTER_WAVES), router_lds_bytes(TR, TC), stream, a, tokens);
 }
 
 // ---- grouped product ------------------------------------------------------------------------------
@@ -1314,13 +1401,13 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     const int H = a.hidden, E = a.experts, K = a.top_k, I = a.inter, Is = a.shared_inter, P = tokens * K;
     const int last = stage_limit ? stage_limit : 4;
     // stage 1: router logits
-    // the tile whose rounds over the chip are the least matrix work, the larger of two equal ones
+    // the tile whose rounds over the chip are the least matrix work, the larger of two equal ones (it reads less per product)
     auto work = [&](int tr, int tc) {
         const long tiles = (long)((tokens + 32 * tr - 1) / (32 * tr)) * ((E + 32 * tc - 1) / (32 * tc));
         return (tiles + 255) / 256 * tr * tc;
     };
-    if (work(2, 2) <= work(2, 1) && work(2, 2) <= work(1, 1)) launch_router<2, 2>(a, tokens, stream);
-    else if (work(2, 1) <= work(1, 1)) launch_router<2, 1>(a, tokens, stream);
+    if (work(2, 2) <= work(1, 2) && work(2, 2) <= work(1, 1)) launch_router<2, 2>(a, tokens, stream);
+    else if (work(1, 2) <= work(1, 1)) launch_router<1, 2>(a, tokens, stream);
     else launch_router<1, 1>(a, tokens, stream);
     if (last < 2) return;
     // stage 2: routes, grouping, fp16 parts of x

@@ -1,4 +1,4 @@
-"""GPU parity of the prefill router's tiles (32 x 32, 64 x 32, 64 x 64 tokens by experts) against the CPU oracle, at counts of
+"""GPU parity of the prefill router's tiles (32 x 32, 32 x 64, 64 x 64 tokens by experts) against the CPU oracle, at counts of
 tokens and experts that are no whole tiles, with activation rows of up to 512 values and wider ones."""
 import numpy as np
 import pytest
@@ -24,3 +24,37 @@ def test_router_tiles(product, oracle, e, i, tokens):
         _, y, ids, w = layer.forward(x)
         assert_parity(y, ids, w, *want[:3], label=f"e={e} T={tokens}")
         np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
+
+
+@pytest.mark.parametrize("e,i,tokens", CASES)
+def test_router_logits(product, e, i, tokens):
+    """The logits themselves against 64 bits, on rows of very different sizes.  Bound: every product keeps 2^-23 of itself (the three
+    products of parts that are left out), a logit is six products' sums a 16-column step of a wave's eighth of the row, at most twelve
+    steps' roundings here, and seven more additions, each off by at most 2^-23 of the sum of the magnitudes."""
+    hidden = 256
+    cfg = abi.moe_config(hidden, e, 4, i, i)
+    weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, tokens, seed=e + tokens)
+    scale = np.exp2(np.random.default_rng(e).integers(-60, 61, tokens)).astype(np.float32)
+    scale[[0, tokens - 1]] = 1.0, 2.0 ** 100
+    x = np.ascontiguousarray(x * scale[:, None])
+    x[1, 7] = np.finfo(np.float32).max   # rounded to eight bits it would be infinite
+    router = weights.raw[0].view(np.float32).reshape(e, hidden).astype(np.float64)
+    want, size = x.astype(np.float64) @ router.T, np.abs(x.astype(np.float64)) @ np.abs(router.T)
+    hip = product.hip
+    with pf.MoeLayer(product, cfg, weights, tokens) as layer:
+        moe, work = layer.device_handles()
+        assert hip.moe_kernel_family(moe, work, tokens) == 2
+        d_x, d_y = hip.to_device(x), hip.to_device(np.zeros_like(x))
+        try:
+            print(f"router logits e={e} tokens={tokens}", flush=True)
+            hip.work_limit_kernels(work, 1)   # the first stage alone
+            hip.check(hip.moe_forward_device(moe, work, d_x, hidden, d_y, hidden, tokens, None), "forward")
+            hip.check(hip.synchronize(), "wait")
+            got = hip.from_device(hip.work_logits(work), (tokens, e), np.float32)
+        finally:
+            hip.work_limit_kernels(work, 0)
+            hip.free(d_x)
+            hip.free(d_y)
+    error = np.abs(got - want) / size
+    print(f"largest error {error.max():.2e} of the magnitudes' sum", flush=True)
+    assert error.max() <= (1 + 12 + 7) * 2.0 ** -23
