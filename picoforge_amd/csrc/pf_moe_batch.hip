@@ -357,10 +357,12 @@ struct BatchItem {
     int token0;           // shared expert: the first row's token
     size_t e;             // where the expert's weights are: its id, or its pool slot
 };
-__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t tile, BatchItem &it) {   // false: no such item
+// Number q of a launch.  The list's last `shared` items, the shared expert's, come first: theirs are 32 rows, four chunks one after the
+// other, and at the launch's end they were its end (101 tokens of the q2 profile 283 us a forward, now 248).  False: no such item.
+__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t q, uint32_t shared, BatchItem &it) {
     const uint32_t count = a.tiles[0];
-    const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[tile];   // {expert, first row, rows, first row within the expert}
-    if (tile >= count) return false;
+    const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[q < shared ? count - shared + q : q - shared];   // {expert, first row, rows, first row within the expert}
+    if (q >= count) return false;
     const int expert = (int)entry.x;
     it.shared = expert == a.experts;
     it.first = (int)entry.y;
@@ -479,12 +481,12 @@ template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t
 #define BATCH_WAVES 4
 // float_rows: the routed experts' activation rows leave the kernel as FP32 (they become digit rows for pf_k_mx_down), else as images.
 template <int FMT, int FMTS, bool ROWS, int PLANES>
-__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a, int float_rows) {
+__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a, uint32_t shared_items, int float_rows) {
     __shared__ float partial[BATCH_WAVES][2][4][64];
     __shared__ BatchFactor factors[BATCH_WAVES][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
     BatchItem it;
-    if (!batch_item(a, blockIdx.y, it)) return;
+    if (!batch_item(a, blockIdx.y, shared_items, it)) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int tile = blockIdx.x, I = it.shared ? a.shared_inter : a.inter;
     if (32 * tile >= I) return;
@@ -547,16 +549,16 @@ __device__ __forceinline__ void batch_stage_rows(uint32_t *stage, const PfKernel
 
 // blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert.  Bound by the products' chain of a wave
 // (with the weights in a cache 90 us of 104 for Q2_K, 101 tokens).
-// last: the list's last items, the shared expert's, a chunk of rows a workgroup (blockIdx.z): alone in a launch a
+// Alone in a launch (blockIdx.y below shared_items) the shared expert's items are a chunk of rows a workgroup (blockIdx.z): a
 // tile's four chunks one after the other took 35 us, side by side 14 (101 tokens).
 template <int FMT, int FMTS, bool ROWS, int PLANES>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, int last) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, uint32_t shared_items) {
     constexpr bool STAGED = FMT == PF_Q2_K && !ROWS;
     __shared__ BatchFactor factors[4][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
     __shared__ __align__(16) uint32_t staged[STAGED ? 4 : 1][STAGED ? 2048 : 4];
     BatchItem it;
-    if (!batch_item(a, last ? a.tiles[0] - 1 - blockIdx.y : blockIdx.y, it)) return;
+    if (!batch_item(a, blockIdx.y, shared_items, it)) return;
     if (batch_tables<FMT>()) batch_stage_tables(tables, a);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), H = a.hidden;
     const int tile = 4 * blockIdx.x + wave;
@@ -703,21 +705,22 @@ static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile
     // integers 101 tokens of the checkpoints' widths took 157 us row by row and 120 in tile order, there 84, 7 for the rows and 14 for the
     // shared expert's down projection.  24 tokens 77 -> 39 + 5 + 12, 300 tokens 229 -> 98 + 9 + 23.
     const bool scaled = FD == PF_MXFP4 && PLANES == 3 && a.wm && pf_batch_down_scaled(tokens, a.experts, a.top_k, a.hidden, a.inter, a.shared_inter);
-    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a, scaled ? 1 : 0);
+    const unsigned shared = (unsigned)(tokens + 31) / 32;
+    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a, shared, scaled ? 1 : 0);
     if (last < 4) return;
     const dim3 grid((a.hidden + 127) / 128, tile_cap);
     if (scaled) {
         pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
-        pf_launch_mx_down(a, tokens, tile_cap - (unsigned)(tokens + 31) / 32, stream);
-        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, (tokens + 31) / 32, 32 / BATCH_ROWS), dim3(256), 0, stream, a, 1);
+        pf_launch_mx_down(a, tokens, tile_cap - shared, stream);
+        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, shared, 32 / BATCH_ROWS), dim3(256), 0, stream, a, shared);
         return;
     }
     // down rows: as gate and up where the layer has one format; Q2_K by whole tiles where they fit a wave's LDS, MXFP4 in tile order
     // where the layer keeps that
     constexpr bool either = FD == PF_Q2_K || (FD == PF_MXFP4 && PLANES == 3);
     const bool lines = FD == PF_Q2_K ? 32 * a.row_bytes[3] <= BATCH_STAGE_BYTES : a.wm != nullptr;
-    if (either && lines) hipLaunchKernelGGL((pf_k_batch_down<FD, FS, either ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, 0);
-    else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, 0);
+    if (either && lines) hipLaunchKernelGGL((pf_k_batch_down<FD, FS, either ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, shared);
+    else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, shared);
 }
 
 template <int FG, int FD, int FS>
