@@ -4,14 +4,20 @@
 #include "pf_device.h"
 
 // One workgroup of 1024 threads: counts the pairs per expert in LDS, scans the counts (offsets, and the row tiles:
-// tiles[0] = count, tiles[1 + i] = expert | tile index << 16, items[i] = {expert, first row, rows, first row within the expert}; the shared expert = expert E with every token, as
-// pf_k_pf_scan_tiles lists them), and hands every pair the next free row of its expert through an LDS cursor.  The rows
+// tiles[0] = count, tiles[1 + i] = expert | tile index << 16, items[i] = {expert, first row, rows, first row within the expert}; the
+// shared expert = expert E with every token, the list's last), and hands every pair the next free row of its expert through an LDS cursor.  The rows
 // of an expert are therefore in no particular order (pf_k_group_place keeps them in pair order): every row of the
 // grouped products is computed on its own and found again through pair_to_row, so the order changes no result, and a
 // walk over all pairs per expert, which the order costs, took three times as long as everything else here.
 #define GROUP_FUSED_MAX_PAIRS 32768
 #define GROUP_FUSED_MAX_EXPERTS 2047
 //
+// The list's order.  The few-row kernels take a tile in chunks of eight rows, one after the other: the tiles of experts with more than 24
+// rows come first, then more than 16, more than 8, the others (101 tokens of the q2 profile, gate and up 156 -> 146 us traced, down 99 ->
+// 94).  CHUNK: the grouped product's tiles stay in the experts' order, where those that wait for memory and those that wait
+// for the matrix cores are mixed, but for the experts of no more than half of the average rows, the shortest items, which come last: in any
+// order a launch ended with whatever the list ended with (1024 tokens of the Q4_K layer 361 -> 357 us a forward, 2048 of the q4 profile
+// 836 -> 830; by classes as above 367 and 828, experts of several tiles first 366 and 867).
 // Bound by one compute unit's chain of loads, LDS atomics and stores.  An expert has GROUP_COPIES counters, a lane's by its number,
 // so that a popular one's pairs do not queue for one word, and the rows' pairs are collected in LDS and written in order: scattered
 // stores are a cache line each.  Beside the conversion of the rows (pf_k_pf_group_rows) 20480 pairs 27.7 -> 24.6 us, 10240 16.1 -> 14.2
@@ -20,9 +26,11 @@
 #define GROUP_FUSED_LDS ((GROUP_COPIES * GROUP_FUSED_MAX_EXPERTS + GROUP_FUSED_MAX_PAIRS / 2) * 4)   // 128 KB, at most
 // words of fused_lds: the counters, then the pair of every row in 16 bits
 __host__ __device__ constexpr size_t pf_group_lds_words(int pairs, int E) { return (size_t)GROUP_COPIES * E + (pairs + 7) / 8 * 4; }
+template <bool CHUNK>
 __device__ __forceinline__ void pf_group_block(uint32_t *fused_lds, const uint32_t *ids, int pairs, int E, int tokens, uint32_t *offsets,
                                                uint32_t *tiles, uint4 *items, uint32_t *pair_to_row, uint32_t *row_to_pair) {
-    __shared__ uint32_t wave_rows[16], wave_tiles[16];
+    __shared__ uint32_t wave_rows[16];
+    __shared__ uint64_t wave_tiles[16];
     const int tid = threadIdx.x, quads = pairs / 4;
     uint32_t *counts = fused_lds;   // [expert][copy]; later the next free row
     uint16_t *pair_of = reinterpret_cast<uint16_t *>(fused_lds + (size_t)GROUP_COPIES * E);
@@ -55,40 +63,51 @@ __device__ __forceinline__ void pf_group_block(uint32_t *fused_lds, const uint32
         for (int r = 0; r < GROUP_COPIES; r++) c += counts[GROUP_COPIES * e + r];
         return c;
     };
-    uint32_t rows = 0, ntiles = 0;
-    for (int e = lo; e < hi; e++) {
+    // the routed tiles of each class, 16 bits each
+    const uint32_t few = (uint32_t)pairs / (2 * (uint32_t)E);
+    auto class_at = [&](uint32_t c) { return CHUNK ? (c > few ? 0 : 16) : c > 24u ? 0 : c > 16u ? 16 : c > 8u ? 32 : 48; };
+    uint32_t rows = 0;
+    uint64_t ntiles = 0;
+    for (int e = lo; e < min(hi, E); e++) {
         const uint32_t c = rows_of(e);
-        if (e < E) rows += c;
-        ntiles += (c + 31u) / 32u;
+        rows += c;
+        ntiles += (uint64_t)((c + 31u) / 32u) << class_at(c);
     }
     // inclusive scan over the 1024 threads: within a wave by shuffles, then the sixteen waves' totals through LDS
     const int lane = pf_lane(), wave = tid >> 6;
-    uint32_t run_rows = rows, run_tiles = ntiles;
+    uint32_t run_rows = rows;
+    uint64_t run_tiles = ntiles;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t up_rows = __shfl_up(run_rows, d), up_tiles = __shfl_up(run_tiles, d);
+        const uint32_t up_rows = __shfl_up(run_rows, d);
+        const uint64_t up_tiles = (uint64_t)__shfl_up((uint32_t)(run_tiles >> 32), d) << 32 | __shfl_up((uint32_t)run_tiles, d);
         if (lane >= d) { run_rows += up_rows; run_tiles += up_tiles; }
     }
     if (lane == 63) { wave_rows[wave] = run_rows; wave_tiles[wave] = run_tiles; }
     __syncthreads();
     uint32_t placed = 0;   // pairs of experts there are
+    uint64_t listed = 0;
     for (int w = 0; w < 16; w++) {
         if (w < wave) { run_rows += wave_rows[w]; run_tiles += wave_tiles[w]; }
         placed += wave_rows[w];
+        listed += wave_tiles[w];
     }
+    const uint64_t until = listed + (listed << 16) + (listed << 32) + (listed << 48);   // the tiles of the classes up to each
+    const uint32_t routed = (uint32_t)(until >> 48);
     if (tid == 1023) {
         offsets[E] = run_rows;
-        tiles[0] = run_tiles;
+        tiles[0] = routed + ((uint32_t)tokens + 31u) / 32u;
     }
-    uint32_t row = run_rows - rows, at = run_tiles - ntiles;
+    uint32_t row = run_rows - rows;
+    uint64_t before = run_tiles - ntiles + (until - listed);
     for (int e = lo; e < hi; e++) {
-        const uint32_t c = rows_of(e), n = (c + 31u) / 32u;
+        const uint32_t c = rows_of(e), n = (c + 31u) / 32u, at = e < E ? (uint32_t)(before >> class_at(c)) & 0xffffu : routed;
         for (uint32_t i = 0; i < n; i++) {
             tiles[1 + at + i] = (uint32_t)e | (i << 16);
             items[at + i] = make_uint4((uint32_t)e, (e < E ? row : (uint32_t)pairs) + 32u * i, min(32u, c - 32u * i), 32u * i);
         }
-        at += n;
         if (e == E) break;
+        before += (uint64_t)n << class_at(c);
         offsets[e] = row;
 #pragma unroll
         for (int r = 0; r < GROUP_COPIES; r++) {

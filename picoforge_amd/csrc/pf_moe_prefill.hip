@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) pf_k_rows_to_half(const float *src, size_
 __global__ void __launch_bounds__(1024) pf_k_pf_group_rows(PfKernelArgs a, int tokens) {
     extern __shared__ __align__(16) uint32_t group_lds[];
     if (blockIdx.x == 0) {
-        pf_group_block(group_lds, a.ids, tokens * a.top_k, a.experts, tokens, a.offsets, a.tiles, reinterpret_cast<uint4 *>(const_cast<uint32_t *>(a.items)),
+        pf_group_block<true>(group_lds, a.ids, tokens * a.top_k, a.experts, tokens, a.offsets, a.tiles, reinterpret_cast<uint4 *>(const_cast<uint32_t *>(a.items)),
                        a.pair_to_row, a.row_to_pair);
         return;
     }

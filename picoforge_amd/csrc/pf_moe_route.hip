@@ -380,7 +380,7 @@ void pf_launch_group_place(const uint32_t *d_ids, int pairs, int experts, const 
 __global__ void __launch_bounds__(1024) pf_k_group_fused(const uint32_t *ids, int pairs, int E, int tokens, uint32_t *offsets,
                                                          uint32_t *tiles, uint4 *items, uint32_t *pair_to_row, uint32_t *row_to_pair) {
     extern __shared__ __align__(16) uint32_t fused_lds[];
-    pf_group_block(fused_lds, ids, pairs, E, tokens, offsets, tiles, items, pair_to_row, row_to_pair);
+    pf_group_block<false>(fused_lds, ids, pairs, E, tokens, offsets, tiles, items, pair_to_row, row_to_pair);
 }
 
 bool pf_group_fits(const uint32_t *d_ids, int pairs, int experts) {

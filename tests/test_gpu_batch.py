@@ -136,3 +136,36 @@ def test_decode_kernels_on_either_side_of_the_matrix_router(product, oracle, h, 
             assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == 1
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"T={tokens}")
+
+
+ROWS = [1, 24, 7, 8, 9, 0, 16, 17, 33, 25, 32, 65]
+
+
+def steered(cfg, fmt, rows, seed):
+    """A layer whose router sends rows[e] tokens to expert e."""
+    expert = np.repeat(np.arange(len(rows)), rows)
+    np.random.default_rng(seed).shuffle(expert)
+    weights, x = make_layer_inputs(cfg, fmt, len(expert), seed=seed)
+    router = weights.raw[0].view(np.float32).reshape(cfg.experts, cfg.hidden_size)
+    router *= 0.01
+    x[:, :cfg.experts] = 0.0
+    router[np.arange(cfg.experts), np.arange(cfg.experts)] = 5.0
+    x[np.arange(len(expert)), expert] = 2.0
+    return weights, x, expert
+
+
+@pytest.mark.parametrize("h,i,s,physical,fmt", [
+    (512, 256, 512, None, abi.GGUF_Q4_K), (512, 256, 256, None, abi.GGUF_IQ2_XXS), (512, 384, 256, 512, "q2"), (512, 384, 256, None, "q4")])
+def test_experts_of_every_row_count(product, oracle, h, i, s, physical, fmt):
+    """Experts of no row up to three row tiles in one batch: the item list's classes (up to 8, 16, 24 rows, more) with an expert on
+    either side of each, and a shared expert of eight tiles ahead of them."""
+    print(f"case few rows, every row count, {fmt} h={h} i={i} s={s}", flush=True)
+    cfg = abi.moe_config(h, len(ROWS), 1, i, s, down_physical=physical)
+    weights, x, expert = steered(cfg, fmt, ROWS, seed=h + i + s)
+    want = forward_with(oracle, cfg, weights, x)
+    np.testing.assert_array_equal(want[1][:, 0], expert)
+    with pf.MoeLayer(product, cfg, weights, len(x)) as layer:
+        assert product.hip.moe_kernel_family(*layer.device_handles(), len(x)) == 3
+        _, y, ids, w = layer.forward(x)
+        assert_parity(y, ids, w, *want, label=f"{fmt}")
+        np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
