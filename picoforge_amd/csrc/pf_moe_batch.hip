@@ -247,12 +247,16 @@ template <int PLANES> __device__ __forceinline__ float batch_value(const int16v 
     return fmaf(65536.0f, batch_upper<PLANES>(d, q), batch_lower(d, q));
 }
 
-// acc[s][q] += the products of set s's piece with tokens 2 q + h of the chunk
-template <int FMT, bool ROWS, int PLANES, int SETS, int QUADS>
+// acc[s][q] += the products of set s's piece with tokens 2 q + h of the chunk.  OWN: the piece is added up by itself first, as a chain's
+// rounding grows with its length; in layers of one format (24 tokens 2.90 -> 2.72e-7 from 64 bits for IQ2_XXS, 3.16 -> 3.10 for Q4_K: no
+// further than the decode kernels).  The profiles' kernels have no registers for it (101 tokens of the q2 profile 3 % slower).
+template <int FMT, bool ROWS, int PLANES, int SETS, int QUADS, bool OWN>
 __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS], const int4v (&x)[BatchRows<FMT, ROWS>::GROUPS], const BatchFactor *factors,
                                             int here, const uint32_t *tables, float (&acc)[SETS][4]) {
     typedef BatchRows<FMT, ROWS> Rows;
     const int16v zero = {0};
+    float own[SETS][4] = {};
+    auto &part = *(OWN ? &own : &acc);
 #pragma unroll
     for (int g = 0; g < Rows::GROUPS; g++) {
         if (g >= here) break;   // the ragged end of a row
@@ -272,17 +276,22 @@ __device__ __forceinline__ void batch_piece(const BatchRows<FMT, ROWS> (&w)[SETS
                     const float mu = batch_upper<PLANES>(m[s], q), product = minimum * mu;
                     const float upper = fmaf(scale, batch_upper<PLANES>(d[s], q), -product) - fmaf(minimum, mu, -product);
                     const float lower = fmaf(scale, batch_lower(d[s], q), -minimum * batch_lower(m[s], q));
-                    acc[s][q] = fmaf(f.step, fmaf(65536.0f, upper, lower), acc[s][q]);
+                    part[s][q] = fmaf(f.step, fmaf(65536.0f, upper, lower), part[s][q]);
                 } else if (Rows::MIN_OPERAND) {
-                    acc[s][q] = fmaf(f.step, fmaf(scale, batch_value<PLANES>(d[s], q), -minimum * batch_value<PLANES>(m[s], q)), acc[s][q]);
+                    part[s][q] = fmaf(f.step, fmaf(scale, batch_value<PLANES>(d[s], q), -minimum * batch_value<PLANES>(m[s], q)), part[s][q]);
                 } else if (Rows::MINIMA) {
-                    acc[s][q] = fmaf(f.step, fmaf(scale, batch_value<PLANES>(d[s], q), -minimum * f.sum), acc[s][q]);
+                    part[s][q] = fmaf(f.step, fmaf(scale, batch_value<PLANES>(d[s], q), -minimum * f.sum), part[s][q]);
                 } else {
-                    acc[s][q] = fmaf(f.step * batch_value<PLANES>(d[s], q), scale, acc[s][q]);
+                    part[s][q] = fmaf(f.step * batch_value<PLANES>(d[s], q), scale, part[s][q]);
                 }
             }
         }
     }
+    if (!OWN) return;
+#pragma unroll
+    for (int s = 0; s < SETS; s++)
+#pragma unroll
+        for (int q = 0; q < QUADS; q++) acc[s][q] += own[s][q];
 }
 
 // The chunk's activation operands of a piece and the piece's factors into the wave's LDS (factors[8 * token + group]).
@@ -315,7 +324,7 @@ __device__ __forceinline__ int batch_lane() {
 }
 
 // image_at(r): dword offset in `images` of the image of the chunk's row r
-template <int FMT, bool ROWS, int PLANES, int SETS, typename ImageAt>
+template <int FMT, bool ROWS, int PLANES, bool OWN, int SETS, typename ImageAt>
 __device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&tensor)[SETS], size_t e, int tile, int first_piece, int piece_step,
                                             int groups, const uint32_t *images, ImageAt image_at, BatchFactor *factors, int rows,
                                             const uint32_t *tables, float (&acc)[SETS][4], const uint32_t *stage = nullptr) {
@@ -339,9 +348,9 @@ __device__ __forceinline__ void batch_chunk(const PfKernelArgs &a, const int (&t
         for (int s = 0; s < SETS; s++) w[s].open();
         const BatchFactor *mine = factors + 8 * (lane >> 5);
         const int here = groups - Rows::GROUPS * piece;
-        if (rows <= 2) batch_piece<FMT, ROWS, PLANES, SETS, 1>(w, x, mine, here, tables, acc);
-        else if (rows <= 4) batch_piece<FMT, ROWS, PLANES, SETS, 2>(w, x, mine, here, tables, acc);
-        else batch_piece<FMT, ROWS, PLANES, SETS, 4>(w, x, mine, here, tables, acc);
+        if (rows <= 2) batch_piece<FMT, ROWS, PLANES, SETS, 1, OWN>(w, x, mine, here, tables, acc);
+        else if (rows <= 4) batch_piece<FMT, ROWS, PLANES, SETS, 2, OWN>(w, x, mine, here, tables, acc);
+        else batch_piece<FMT, ROWS, PLANES, SETS, 4, OWN>(w, x, mine, here, tables, acc);
         if (piece + piece_step < pieces) {
             const int lane = batch_lane();
 #pragma unroll
@@ -357,17 +366,19 @@ struct BatchItem {
     int token0;           // shared expert: the first row's token
     size_t e;             // where the expert's weights are: its id, or its pool slot
 };
-// Number q of a launch.  The list's last `shared` items, the shared expert's, come first: theirs are 32 rows, four chunks one after the
-// other, and at the launch's end they were its end (101 tokens of the q2 profile 283 us a forward, now 248).  False: no such item.
+// Number q of a launch.  The shared expert's rows, the list's last items, come first and a chunk of eight a number: `shared` numbers.  (As
+// row tiles, four chunks one after the other, at the list's end they were a launch's end: 101 tokens of the q2 profile 283 us a forward, first
+// 248; for a layer of few experts they were as long as all else.)  False: no such item.
 __device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t q, uint32_t shared, BatchItem &it) {
-    const uint32_t count = a.tiles[0];
-    const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[q < shared ? count - shared + q : q - shared];   // {expert, first row, rows, first row within the expert}
-    if (q >= count) return false;
+    const uint32_t count = a.tiles[0], routed = count - (shared + 3) / 4;
+    const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[q < shared ? routed + q / 4 : q - shared];   // {expert, first row, rows, first row within the expert}
+    if (q >= shared + routed) return false;
+    const int chunk = q < shared ? BATCH_ROWS * (int)(q % 4) : 0;
     const int expert = (int)entry.x;
     it.shared = expert == a.experts;
-    it.first = (int)entry.y;
-    it.rows = (int)entry.z;
-    it.token0 = (int)entry.w;
+    it.first = (int)entry.y + chunk;
+    it.rows = q < shared ? min(BATCH_ROWS, (int)entry.z - chunk) : (int)entry.z;
+    it.token0 = (int)entry.w + chunk;
     it.e = it.shared ? 0 : (size_t)expert;
     if (a.slots && !it.shared) {   // expert streaming: the rows of an expert share its pool slot
         uint32_t slot = a.slots[a.row_to_pair[it.first]];
@@ -503,8 +514,8 @@ __global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_
             const uint32_t row = (uint32_t)(c0 + r);
             return (it.shared ? (uint32_t)it.token0 + row : a.row_to_pair[(uint32_t)it.first + row] / (uint32_t)K) * words;
         };
-        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS, PLANES, 2>(a, tensor, 0, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
-        else batch_chunk<FMT, ROWS, PLANES, 2>(a, tensor, it.e, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
+        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS, PLANES, false>(a, tensor, 0, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
+        else batch_chunk<FMT, ROWS, PLANES, FMT == FMTS>(a, tensor, it.e, tile, wave, BATCH_WAVES, groups, a.ximg, image_at, factors[wave], rows, tables, acc);
         const int lane = batch_lane();
 #pragma unroll
         for (int q = 0; q < 4; q++)
@@ -549,8 +560,6 @@ __device__ __forceinline__ void batch_stage_rows(uint32_t *stage, const PfKernel
 
 // blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert.  Bound by the products' chain of a wave
 // (with the weights in a cache 90 us of 104 for Q2_K, 101 tokens).
-// Alone in a launch (blockIdx.y below shared_items) the shared expert's items are a chunk of rows a workgroup (blockIdx.z): a
-// tile's four chunks one after the other took 35 us, side by side 14 (101 tokens).
 template <int FMT, int FMTS, bool ROWS, int PLANES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, uint32_t shared_items) {
     constexpr bool STAGED = FMT == PF_Q2_K && !ROWS;
@@ -571,13 +580,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) p
         __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the wave's own copy is there
         pf_wave_lds_fence();
     }
-    for (int c0 = BATCH_ROWS * blockIdx.z; c0 < it.rows; c0 += BATCH_ROWS * gridDim.z) {
+    for (int c0 = 0; c0 < it.rows; c0 += BATCH_ROWS) {
         const int rows = min(BATCH_ROWS, it.rows - c0);
         auto image_at = [&](int r) { return (uint32_t)(it.first + c0 + r) * words; };
         float acc[1][4] = {};
         const int tensor[1] = {it.shared ? 6 : 3};
-        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS || FMTS == PF_Q8_0, PLANES, 1>(a, tensor, 0, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
-        else batch_chunk<FMT, ROWS, PLANES, 1>(a, tensor, it.e, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc, stage);
+        if (FMT != FMTS && it.shared) batch_chunk<FMTS, ROWS || FMTS == PF_Q8_0, PLANES, false>(a, tensor, 0, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc);
+        else batch_chunk<FMT, ROWS, PLANES, FMT == FMTS>(a, tensor, it.e, tile, 0, 1, groups, a.aimg, image_at, factors[wave], rows, tables, acc, stage);
         const int lane = batch_lane();
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -699,20 +708,20 @@ void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, bool 
 
 // ---- dispatch --------------------------------------------------------------------------------------
 template <int FG, int FD, int FS, bool ROWS, int PLANES>
-static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile_cap, hipStream_t stream, int last) {
+static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned routed_cap, hipStream_t stream, int last) {
     const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
     // The q4 profile's routed down projection on the block-scaled product, as a chunk's, where the work is worth its launches: on the
     // integers 101 tokens of the checkpoints' widths took 157 us row by row and 120 in tile order, there 84, 7 for the rows and 14 for the
     // shared expert's down projection.  24 tokens 77 -> 39 + 5 + 12, 300 tokens 229 -> 98 + 9 + 23.
     const bool scaled = FD == PF_MXFP4 && PLANES == 3 && a.wm && pf_batch_down_scaled(tokens, a.experts, a.top_k, a.hidden, a.inter, a.shared_inter);
-    const unsigned shared = (unsigned)(tokens + 31) / 32;
-    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, tile_cap), dim3(64 * BATCH_WAVES), 0, stream, a, shared, scaled ? 1 : 0);
+    const unsigned shared = (unsigned)(tokens + BATCH_ROWS - 1) / BATCH_ROWS;
+    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, shared + routed_cap), dim3(64 * BATCH_WAVES), 0, stream, a, shared, scaled ? 1 : 0);
     if (last < 4) return;
-    const dim3 grid((a.hidden + 127) / 128, tile_cap);
+    const dim3 grid((a.hidden + 127) / 128, shared + routed_cap);
     if (scaled) {
         pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
-        pf_launch_mx_down(a, tokens, tile_cap - shared, stream);
-        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, shared, 32 / BATCH_ROWS), dim3(256), 0, stream, a, shared);
+        pf_launch_mx_down(a, tokens, routed_cap, stream);
+        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, shared), dim3(256), 0, stream, a, shared);
         return;
     }
     // down rows: as gate and up where the layer has one format; Q2_K by whole tiles where they fit a wave's LDS, MXFP4 in tile order
@@ -724,20 +733,18 @@ static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned tile
 }
 
 template <int FG, int FD, int FS>
-static void launch_batch_experts(const PfKernelArgs &a, int tokens, unsigned tile_cap, hipStream_t stream, int last) {
+static void launch_batch_experts(const PfKernelArgs &a, int tokens, unsigned routed_cap, hipStream_t stream, int last) {
     // a layer keeps the tile-ordered copies of its gate and up tensors (and a one-format layer those of its down tensors,
     // the profiles those of the shared gate and up) or none of them; a streamed layer's pool keeps its slots that way
     const bool tiled = (FG == PF_Q4_K ? a.wt[1] && a.wt[2] : a.wi[1] && a.wi[2]) && (FS != PF_Q8_0 || (a.wq[4] && a.wq[5]));
-    if (a.slots) launch_batch_format<FG, FD, FS, false, 4>(a, tokens, tile_cap, stream, last);
-    else if (tiled) launch_batch_format<FG, FD, FS, false, 3>(a, tokens, tile_cap, stream, last);
-    else launch_batch_format<FG, FD, FS, true, 3>(a, tokens, tile_cap, stream, last);
+    if (a.slots) launch_batch_format<FG, FD, FS, false, 4>(a, tokens, routed_cap, stream, last);
+    else if (tiled) launch_batch_format<FG, FD, FS, false, 3>(a, tokens, routed_cap, stream, last);
+    else launch_batch_format<FG, FD, FS, true, 3>(a, tokens, routed_cap, stream, last);
 }
 
 void pf_launch_batch_experts(const PfKernelArgs &a, int tokens, hipStream_t stream, int last) {
     // row tiles there can be: an expert with rows has at least one
-    const int pairs = tokens * a.top_k;
-    unsigned cap = (unsigned)pf_prefill_max_tiles(tokens, a.experts, a.top_k), few = (unsigned)(pairs + (tokens + 31) / 32);
-    if (few < cap) cap = few;
+    const unsigned pairs = (unsigned)(tokens * a.top_k), most = (unsigned)(pf_prefill_max_tiles(tokens, a.experts, a.top_k) - (tokens + 31) / 32), cap = min(pairs, most);
     switch (a.type[1] == PF_Q4_K ? (a.type[3] == PF_Q4_K ? 1 : 4) : (a.type[3] == PF_IQ2_XXS ? 2 : 3)) {
     case 1: launch_batch_experts<PF_Q4_K, PF_Q4_K, PF_Q4_K>(a, tokens, cap, stream, last); break;
     case 2: launch_batch_experts<PF_IQ2_XXS, PF_IQ2_XXS, PF_IQ2_XXS>(a, tokens, cap, stream, last); break;
