@@ -4,8 +4,12 @@
 //
 // The CPU fills or empties some pieces while the others are on their way.  (A hipMemcpy2D on the caller's pageable rows moves
 // them row by row, each with a wait of its own: 777 rows of 8 KB each way took 24.9 ms.)  A piece is large enough that its
-// transfer hides the enqueueing.  One CPU copies at about a fifth of what the link carries, so the pieces are dealt to a few
-// threads.
+// transfer hides the enqueueing.  One CPU copies at about a fifth of what the link carries, so a few threads share the copying,
+// and they share every piece: parts of it go to whoever is free, in order.  (With whole pieces dealt to the threads the first
+// transfer started, and the last piece's copy ended, when one thread had copied 512 KB, 55 us each.)  A piece is a quarter of
+// the rows, between 256 KB and 1 MB: a kernel moves 512 KB at 35 GB/s, 1 MB at 38 in and 44 out, all of 6 MB at 42 and 51, and
+// the first piece's copy and the last one's hide behind nothing.  A call of 777 rows of 8 KB 706 -> 686 us, with pieces of
+// 512 KB 696; calls of 300 rows with pieces of 256 KB 472, of a quarter 432.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
@@ -17,7 +21,8 @@
 #include <thread>
 
 #define PF_RING_SLOTS 8
-#define PF_RING_BYTES ((size_t)512 * 1024)
+#define PF_RING_BYTES ((size_t)1024 * 1024)          // a piece at most
+#define PF_RING_PARTS 16                             // of a piece, each copied by one thread
 #define PF_CREW_HELPERS 3                            // besides the calling thread
 #define PF_CREW_FROM ((size_t)1024 * 1024)           // bytes that are worth waking them for (10 to 20 us)
 
@@ -90,8 +95,8 @@ struct RingCarrier {
     int (*send)(void *self, int slot, void *dst, const void *src, size_t bytes, bool in);   // enqueues the slot's next transfer
 };
 
-// Rows between the caller's memory (a pitch) and dense device rows.  Piece p goes to worker p % workers, whose own slots its
-// pieces take in turn.
+// Rows between the caller's memory (a pitch) and dense device rows.  Piece p has slot p % PF_RING_SLOTS; its parts are handed
+// out in order, piece after piece, and who ends a piece's last part sends it (in) or the slot's next one (out).
 struct RingJob {
     RingCarrier carrier;
     uint8_t *ring, *device;
@@ -99,23 +104,52 @@ struct RingJob {
     size_t pitch, row_bytes, rows, step, pieces;
     bool check;             // in: look for values that are not finite
     std::atomic<int> error, nonfinite;
+    std::atomic<size_t> next;                                       // part to hand out
+    std::atomic<size_t> sent[PF_RING_SLOTS], ended[PF_RING_SLOTS];  // a slot's pieces that have been sent; its parts that have been copied
     void open(const RingCarrier &c, uint8_t *pieces_at, void *device_rows, const void *host_rows, size_t host_pitch, size_t bytes, size_t count) {
         carrier = c; ring = pieces_at; device = (uint8_t *)device_rows; host = (uint8_t *)const_cast<void *>(host_rows);
         pitch = host_pitch; row_bytes = bytes; rows = count;
-        step = PF_RING_BYTES / row_bytes;
+        const size_t quarter = rows * row_bytes / 4, least = PF_RING_BYTES / 4;
+        const size_t bytes_a_piece = quarter < least ? least : quarter < PF_RING_BYTES ? quarter : PF_RING_BYTES;
+        step = (row_bytes <= bytes_a_piece ? bytes_a_piece : PF_RING_BYTES) / row_bytes;
         pieces = (rows + step - 1) / step;
         check = false;
-        error = 0; nonfinite = 0;
+        error = 0; nonfinite = 0; next = 0;
+        for (int s = 0; s < PF_RING_SLOTS; s++) { sent[s] = 0; ended[s] = 0; }
     }
     size_t rows_of(size_t p) const { return rows - p * step < step ? rows - p * step : step; }
-    static int slot_of(size_t p, int workers) {
-        const int per = PF_RING_SLOTS / workers;
-        return (int)(p % workers) * per + (int)(p / workers % per);
-    }
+    static int slot_of(size_t p) { return (int)(p % PF_RING_SLOTS); }
+    bool stopped() const { return error.load() != 0 || nonfinite.load() != 0; }
     void fail(int e) { int none = 0; if (e) error.compare_exchange_strong(none, e); }
     void bind(int worker) { if (worker) fail(carrier.bind(carrier.self, carrier.device)); }
-    void wait(int slot) { fail(carrier.wait(carrier.self, slot)); }
-    void send(int slot, void *dst, const void *src, size_t bytes, bool in) { fail(carrier.send(carrier.self, slot, dst, src, bytes, in)); }
+    void send(size_t p, bool in) {
+        const int slot = slot_of(p);
+        uint8_t *piece = ring + slot * PF_RING_BYTES, *there = device + p * step * row_bytes;
+        fail(carrier.send(carrier.self, slot, in ? there : piece, in ? piece : there, rows_of(p) * row_bytes, in));
+        sent[slot].fetch_add(1);
+    }
+    // The next part: of piece p, rows [first, last) of it; false when there is none left or the job has stopped.
+    struct Part { size_t p, first, last; };
+    bool take(Part *part) {
+        const size_t q = next.fetch_add(1), share = (step + PF_RING_PARTS - 1) / PF_RING_PARTS;
+        part->p = q / PF_RING_PARTS;
+        if (part->p >= pieces || stopped()) return false;
+        const size_t n = rows_of(part->p), from = q % PF_RING_PARTS * share;
+        part->first = from < n ? from : n;
+        part->last = from + share < n ? from + share : n;
+        return true;
+    }
+    // Until `count` pieces have been sent through the slot and the last of them has arrived; false when the job stops.  (The
+    // parts before this one are all in other threads' hands, so the piece is sent without this thread.)
+    bool await(int slot, size_t count) {
+        while (sent[slot].load() < count) {
+            if (stopped()) return false;
+            std::this_thread::yield();
+        }
+        fail(carrier.wait(carrier.self, slot));
+        return !stopped();
+    }
+    bool ends_piece(size_t p) { return ended[slot_of(p)].fetch_add(1) + 1 == PF_RING_PARTS * (p / PF_RING_SLOTS + 1); }
 };
 static inline void rows_in(void *dst, const void *src, size_t src_pitch, size_t row_bytes, size_t rows) {
     for (size_t r = 0; r < rows; r++) memcpy((uint8_t *)dst + r * row_bytes, (const uint8_t *)src + r * src_pitch, row_bytes);
@@ -140,40 +174,34 @@ static inline bool ring_by_kernel(const void *dst, const void *src, size_t bytes
     return bytes % 16 == 0 && ((uintptr_t)dst | (uintptr_t)src) % 16 == 0;
 }
 
-static inline void ring_in_part(void *job, int worker, int workers) {
+static inline void ring_in_part(void *job, int worker, int) {
     RingJob *j = static_cast<RingJob *>(job);
     j->bind(worker);
-    for (size_t p = worker; p < j->pieces && !j->error.load() && !j->nonfinite.load(); p += workers) {
-        const int slot = RingJob::slot_of(p, workers);
-        const size_t r = p * j->step, n = j->rows_of(p);
-        uint8_t *piece = j->ring + slot * PF_RING_BYTES;
-        j->wait(slot);
-        rows_in(piece, j->host + r * j->pitch, j->pitch, j->row_bytes, n);
-        if (j->check && !finite_floats(piece, n * j->row_bytes / 4)) { j->nonfinite = 1; return; }
-        j->send(slot, j->device + r * j->row_bytes, piece, n * j->row_bytes, true);
+    for (RingJob::Part t; j->take(&t);) {
+        const int slot = RingJob::slot_of(t.p);
+        uint8_t *to = j->ring + slot * PF_RING_BYTES + t.first * j->row_bytes;
+        if (!j->await(slot, t.p / PF_RING_SLOTS)) return;
+        rows_in(to, j->host + (t.p * j->step + t.first) * j->pitch, j->pitch, j->row_bytes, t.last - t.first);
+        if (j->check && !finite_floats(to, (t.last - t.first) * j->row_bytes / 4)) { j->nonfinite = 1; return; }
+        if (j->ends_piece(t.p)) j->send(t.p, true);
     }
 }
-static inline void ring_send_out(RingJob *j, size_t p, int workers) {
-    const int slot = RingJob::slot_of(p, workers);
-    j->send(slot, j->ring + slot * PF_RING_BYTES, j->device + p * j->step * j->row_bytes, j->rows_of(p) * j->row_bytes, false);
-}
-static inline void ring_out_part(void *job, int worker, int workers) {   // the first PF_RING_SLOTS pieces are on their way
+static inline void ring_out_part(void *job, int worker, int) {   // the first PF_RING_SLOTS pieces are on their way
     RingJob *j = static_cast<RingJob *>(job);
     j->bind(worker);
-    const size_t ahead = (size_t)(PF_RING_SLOTS / workers) * workers;
-    for (size_t p = worker; p < j->pieces && !j->error.load(); p += workers) {
-        const int slot = RingJob::slot_of(p, workers);
-        j->wait(slot);
-        if (j->error.load()) break;
-        rows_out(j->host + p * j->step * j->pitch, j->pitch, j->ring + slot * PF_RING_BYTES, j->row_bytes, j->rows_of(p));
-        if (p + ahead < j->pieces) ring_send_out(j, p + ahead, workers);
+    for (RingJob::Part t; j->take(&t);) {
+        const int slot = RingJob::slot_of(t.p);
+        if (!j->await(slot, t.p / PF_RING_SLOTS + 1)) return;
+        rows_out(j->host + (t.p * j->step + t.first) * j->pitch, j->pitch, j->ring + slot * PF_RING_BYTES + t.first * j->row_bytes, j->row_bytes,
+                 t.last - t.first);
+        if (j->ends_piece(t.p) && t.p + PF_RING_SLOTS < j->pieces) j->send(t.p + PF_RING_SLOTS, false);
     }
 }
 
 // The crew if the rows are worth it and it is free (its `busy` is then held), else null.
 static inline CopyCrew *crew_for(const RingJob &j) {
     CopyCrew *crew = j.row_bytes * j.rows >= PF_CREW_FROM ? g_crew : nullptr;   // (a workspace with a ring keeps it alive)
-    return crew && crew->helpers && PF_RING_SLOTS % (crew->helpers + 1) == 0 && crew->busy.try_lock() ? crew : nullptr;
+    return crew && crew->helpers && crew->busy.try_lock() ? crew : nullptr;
 }
 // In: the caller's rows have been read, and their transfers enqueued, when this returns.
 static inline void ring_rows_in(RingJob *j) {
@@ -182,9 +210,8 @@ static inline void ring_rows_in(RingJob *j) {
 }
 // Out: the first pieces' transfers enqueued; then, where the call went well, every row into the caller's memory.  crew: from
 // crew_for, given back by ring_rows_out.
-static inline void ring_start_out(RingJob *j, CopyCrew *crew) {
-    const int workers = crew ? crew->helpers + 1 : 1;
-    for (size_t p = 0; p < j->pieces && p < PF_RING_SLOTS; p++) ring_send_out(j, p, workers);
+static inline void ring_start_out(RingJob *j, CopyCrew *) {
+    for (size_t p = 0; p < j->pieces && p < PF_RING_SLOTS; p++) j->send(p, false);
 }
 static inline void ring_rows_out(RingJob *j, CopyCrew *crew, bool fine) {
     fine = fine && !j->error.load();

@@ -639,8 +639,8 @@ static hipError_t await_results(const HostBlock &b, const HostResults &r) {
 }
 
 // Longer batches pass through the workspace's ring of page-locked pieces (pf_host_rows.h).  A piece travels by a kernel that
-// addresses the page-locked memory: 38 GB/s and no wait between engine and kernels, where copies of this size brought 22 GB/s
-// out of the device.  With eight threads, or pieces of 256 KB, nothing is faster (777 rows of 8 KB: 770, 775 and 850 us).
+// addresses the page-locked memory: 38 to 44 GB/s and no wait between engine and kernels, where copies of this size brought 22 GB/s
+// out of the device.
 static int ring_bind(void *, int device) { return (int)hipSetDevice(device); }
 static uint32_t *ring_word(const PfHipWork *w, int slot) {   // in the block: behind the published call's number, a line each
     return host_block(&w->moe->desc, w->cap, w->host).published + 16 * (slot + 1);
