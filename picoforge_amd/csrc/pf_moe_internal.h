@@ -59,7 +59,7 @@ struct PfKernelArgs {
     const uint8_t *router_parts;     // router as operands of the chunks' logits (pf_k_router_parts)
     float *down;                     // [pairs + tokens, hidden] down products in expert order, then the shared expert's
     uint32_t *counts, *offsets, *pair_to_row, *row_to_pair, *group_bad, *tiles;
-    const uint32_t *items;           // row tiles as {expert, first row, rows, first row within the expert} (pf_k_group_fused)
+    const uint32_t *items;           // row tiles as {expert, first row, rows, first row within the expert} (pf_group_scan)
     // injection into hyper-connection streams in place of writing y (null: y is written)
     float *hc_residual;              // [tokens, streams, hidden], pitches in floats
     const float *hc_inject;          // [tokens, streams], dense

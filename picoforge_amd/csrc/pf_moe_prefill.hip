@@ -64,10 +64,30 @@ __device__ __forceinline__ void row_to_half(size_t row, bool store, int tid, flo
     const float *s = src + row * src_pitch;
     float m = 0.0f;
     bool bad = false;
-    for (int c = tid; c < cols; c += 256) {
-        const float v = s[c];
-        bad |= !pf_finite(v);
-        m = fmaxf(m, fabsf(v));
+    constexpr int HELD = 2;   // pieces of eight values that a thread keeps between the maximum and the conversion; rows of more are read twice
+    float kept[HELD][8];
+    auto take = [&](int j, float (&v)[8]) {
+        const float4 a = reinterpret_cast<const float4 *>(s)[2 * j], b = reinterpret_cast<const float4 *>(s)[2 * j + 1];
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    };
+    auto look = [&](int j, const float (&v)[8]) {   // the maximum, and the shared router's sum
+#pragma unroll
+        for (int c = 0; c < 8; c++) { bad |= !pf_finite(v[c]); m = fmaxf(m, fabsf(v[c])); }
+        if (gate) {
+            const float4 ga = reinterpret_cast<const float4 *>(gate)[2 * j], gb = reinterpret_cast<const float4 *>(gate)[2 * j + 1];
+            dot += ((v[0] * ga.x + v[1] * ga.y) + (v[2] * ga.z + v[3] * ga.w)) + ((v[4] * gb.x + v[5] * gb.y) + (v[6] * gb.z + v[7] * gb.w));
+        }
+    };
+#pragma unroll
+    for (int p = 0; p < HELD; p++)
+        if (tid + 256 * p < cols / 8) take(tid + 256 * p, kept[p]);
+#pragma unroll
+    for (int p = 0; p < HELD; p++)
+        if (tid + 256 * p < cols / 8) look(tid + 256 * p, kept[p]);
+    for (int j = tid + 256 * HELD; j < cols / 8; j += 256) {
+        float v[8];
+        take(j, v);
+        look(j, v);
     }
     m = pf_wave_max(m);
     if (pf_lane() == 0) part[tid >> 6] = m;
@@ -79,13 +99,7 @@ __device__ __forceinline__ void row_to_half(size_t row, bool store, int tid, flo
     const float scale = __int_as_float((e + 1) << 23);        // 2^(e-126)
     const float inv = __int_as_float((253 - e) << 23);        // 2^(126-e)
     half_t *out = dst + row * pf_half_row(cols);
-    for (int j = tid; j < cols / 8; j += 256) {
-        const float4 a = reinterpret_cast<const float4 *>(s)[2 * j], b = reinterpret_cast<const float4 *>(s)[2 * j + 1];
-        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        if (gate) {
-            const float4 ga = reinterpret_cast<const float4 *>(gate)[2 * j], gb = reinterpret_cast<const float4 *>(gate)[2 * j + 1];
-            dot += ((a.x * ga.x + a.y * ga.y) + (a.z * ga.z + a.w * ga.w)) + ((b.x * gb.x + b.y * gb.y) + (b.z * gb.z + b.w * gb.w));
-        }
+    auto convert = [&](int j, const float (&v)[8]) {
         half8v hi, lo;
         float sum = 0.0f;
 #pragma unroll
@@ -109,6 +123,14 @@ __device__ __forceinline__ void row_to_half(size_t row, bool store, int tid, flo
             sums[0] = sh;
             sums[4] = sl;
         }
+    };
+#pragma unroll
+    for (int p = 0; p < HELD; p++)
+        if (tid + 256 * p < cols / 8) convert(tid + 256 * p, kept[p]);
+    for (int j = tid + 256 * HELD; j < cols / 8; j += 256) {
+        float v[8];
+        take(j, v);
+        convert(j, v);
     }
     if (gate) {   // uniform
         dot = pf_wave_sum(dot);
@@ -128,19 +150,18 @@ __global__ void __launch_bounds__(256) pf_k_rows_to_half(const float *src, size_
     row_to_half(blockIdx.x, true, threadIdx.x, part, dots, src, src_pitch, cols, dst, scale_out, error_word, gate, gate_out);
 }
 
-// Workgroup 0 groups the pairs (pf_group_device.h), the others convert the chunk's rows, four each: the grouping, one workgroup's
-// chain, leaves the rest of the chip idle, and the conversion fits in beside it.  Apart they took 14.3 and 10.7 us (1024 tokens of
-// width 2048), 21.9 and 12.5 (2048 of width 2560), together 14.2 and 24.6; the router finds the rows' largest magnitudes itself for
-// another 1.5.
-__global__ void __launch_bounds__(1024) pf_k_pf_group_rows(PfKernelArgs a, int tokens) {
+// The first workgroups group the pairs, 1024 each: every one counts all pairs for itself, those before its own apart (pf_group_pairs),
+// and the first writes the lists.  The others convert the chunk's rows, four each.  1024 tokens of width 2048 12.5 us, 2048 of width 2560
+// 16.5; with one workgroup for all pairs, and rows read twice, 15.3 and 24.8.
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) pf_k_pf_group_rows(PfKernelArgs a, int tokens, int place_blocks) {
     extern __shared__ __align__(16) uint32_t group_lds[];
-    if (blockIdx.x == 0) {
-        pf_group_block<true>(group_lds, a.ids, tokens * a.top_k, a.experts, tokens, a.offsets, a.tiles, reinterpret_cast<uint4 *>(const_cast<uint32_t *>(a.items)),
+    if ((int)blockIdx.x < place_blocks) {
+        pf_group_pairs(group_lds, a.ids, tokens * a.top_k, a.experts, tokens, (int)blockIdx.x, a.offsets, a.tiles, reinterpret_cast<uint4 *>(const_cast<uint32_t *>(a.items)),
                        a.pair_to_row, a.row_to_pair);
         return;
     }
     __shared__ float part[4][4], dots[4][4];
-    const int team = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)), row = 4 * ((int)blockIdx.x - 1) + team;
+    const int team = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)), row = 4 * ((int)blockIdx.x - place_blocks) + team;
     row_to_half(min(row, tokens - 1), row < tokens, threadIdx.x & 255, part[team], dots[team], a.x, a.x_pitch, a.hidden, (half_t *)a.x16, a.x_scale,
                 a.error_word, reinterpret_cast<const float *>(a.w[7]), a.shared_scale);
 }
@@ -1411,9 +1432,11 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     pf_launch_route(a, tokens, stream);
     if (pf_group_fits(a.ids, P, E)) {
         static const bool configured = hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_pf_group_rows), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                           GROUP_FUSED_LDS) == hipSuccess;
+                                                           GROUP_PAIRS_LDS) == hipSuccess;
         (void)configured;
-        hipLaunchKernelGGL(pf_k_pf_group_rows, dim3(1 + (unsigned)(tokens + 3) / 4), dim3(1024), pf_group_lds_words(P, E) * sizeof(uint32_t), stream, a, tokens);
+        const unsigned place_blocks = (unsigned)(P + 1023) / 1024;
+        hipLaunchKernelGGL(pf_k_pf_group_rows, dim3(place_blocks + (unsigned)(tokens + 3) / 4), dim3(1024), 2 * GROUP_COPIES * pf_group_pitch(E) * sizeof(uint32_t), stream, a, tokens,
+                           (int)place_blocks);
     } else {
         hipLaunchKernelGGL(pf_k_rows_to_half, dim3(tokens), dim3(256), 0, stream, a.x, a.x_pitch, H, (half_t *)a.x16, a.x_scale, a.error_word,
                            reinterpret_cast<const float *>(a.w[7]), a.shared_scale);

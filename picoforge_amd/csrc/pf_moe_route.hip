@@ -9,25 +9,89 @@
 #include "pf_moe_internal.h"
 #include "pf_route_device.h"
 #include "pf_route_fast.h"
-#include "pf_route_fix.h"
+#include "pf_route_fix_many.h"
 #include "pf_group_device.h"
 
 #define ROUTE_MAX_FAST_EXPERTS 1024
 
-// ---- fast routing inside a forward (general path) --------------------------------
+// ---- routing inside a forward: chunks and the general path --------------------------------------
+// A workgroup routes up to sixteen tokens, a wave each, and then those of them whose best logits are too close, together
+// (pf_route_fix_many.h): the candidates of all of them, as many as there are lanes, share the chain's wave, which costs the same for
+// one token as for five.  exact_rows[0] counts the tokens routed again, exact_rows[1] those of them that went the long way.
+// Bound by that chain, a dependent addition a column.  1024 tokens of width 2048 25 us traced, 2048 of width 2560 26, where a launch
+// that routed and one that routed again, a workgroup a flagged token, took 8.2 + 22.6 and 9.1 + 23.9.  (Handing every pair its rank among its
+// expert's here, by additions to a counter an expert in memory, took 10 us: a popular one's queue.)
+#define ROUTE_TOKENS 16
+#define ROUTE_UNFLAGGED 0xffffffffu
 template <int NPL>
-__global__ void __launch_bounds__(64) pf_k_route_fast(PfKernelArgs a) {
-    const int t = blockIdx.x, lane = threadIdx.x, E = a.experts, K = a.top_k;
-    PfRouteResult r = pf_route_fast_wave<NPL>(a.logits + (size_t)t * E, a.logit_ssq + (size_t)t * E, E, K,
-                                              a.norm_topk != 0, a.hidden, lane);
-    if (r.bad && lane == 0) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
-    if (lane < K) {
-        a.ids[(size_t)t * K + lane] = r.id;
-        a.route_weights[(size_t)t * K + lane] = r.weight;
+__global__ void __launch_bounds__(1024) pf_k_route_tokens(PfKernelArgs a, int tokens) {
+    extern __shared__ __align__(16) float route_lds[];   // the two chunk buffers, then the long way's 3 E floats
+    __shared__ uint32_t cand[ROUTE_TOKENS][PF_WAVE], list[PF_WAVE], found[ROUTE_TOKENS], ids[ROUTE_TOKENS * PF_WAVE];
+    __shared__ float weights[ROUTE_TOKENS * PF_WAVE], sums[PF_WAVE];
+    __shared__ uint32_t again[ROUTE_TOKENS];   // 0: settled at once, 1: by the candidates, 2: the long way
+    const int E = a.experts, K = a.top_k, H = a.hidden, picks = K < E ? K : E, lane = pf_lane();
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), grid = (int)gridDim.x;
+    const int here = (tokens - (int)blockIdx.x + grid - 1) / grid;   // tokens blockIdx.x, + grid, ...: flagged neighbours go to several workgroups
+    const bool norm = a.norm_topk != 0;
+    const float *router = reinterpret_cast<const float *>(a.w[0]);
+    auto token = [&](int w) { return (size_t)((int)blockIdx.x + w * grid); };
+    const size_t at = token(min(wave, here - 1)) * E;   // this wave's token's logits
+    if (wave < here) {
+        const PfRouteResult r = pf_route_fast_wave<NPL>(a.logits + at, a.logit_ssq + at, E, K, norm, H, lane);
+        if (r.bad && lane == 0) atomicOr(a.error_word, PF_HIP_ERR_NONFINITE);
+        if (lane < K) { ids[wave * K + lane] = r.id; weights[wave * K + lane] = r.weight; }
+        uint32_t count = ROUTE_UNFLAGGED;
+        if (r.close) {
+            float v[NPL], s2[NPL];
+            pf_load_row<NPL>(a.logits + at, E, lane, -INFINITY, v);
+            pf_load_row<NPL>(a.logit_ssq + at, E, lane, 0.0f, s2);
+            count = (uint32_t)pf_fix_candidates<NPL>(v, s2, r.kth, r.best, E, picks, H, pf_fix_by_pieces(router, H), cand[wave], lane);
+        }
+        if (lane == 0) { found[wave] = count; again[wave] = count == ROUTE_UNFLAGGED ? 0u : 2u; }
     }
-    if (lane == 0 && r.close) {   // onto the list of tokens to route again in serial order: [0] count, then the tokens
-        const uint32_t at = atomicAdd(a.route_flags, 1u);
-        a.route_flags[1 + at] = (uint32_t)t;
+    __syncthreads();
+    // the flagged tokens in turn, as many at a time as their candidates fit the chain's lanes
+    for (int w = 0; w < here;) {
+        int n = 0, mine = -1, count = 0;
+        for (; w < here; w++) {
+            const uint32_t c = found[w];
+            if (c == ROUTE_UNFLAGGED || c == 0u) continue;
+            if (n + (int)c > PF_WAVE) break;
+            if (w == wave) { mine = n; count = (int)c; }
+            n += (int)c;
+        }
+        if (n == 0) break;
+        if (mine >= 0 && lane < count) list[mine + lane] = (uint32_t)wave << 16 | cand[wave][lane];
+        __syncthreads();
+        const float logit = pf_fix_sums(n, H, route_lds, [&](int r) { return router + (size_t)(list[r] & 0xffffu) * H; },
+                                        [&](int r, int k) { return pf_fix_values(a.x + token((int)(list[r] >> 16)) * a.x_pitch, k); }, wave, lane);
+        if (wave == 0) sums[lane] = logit;
+        __syncthreads();
+        if (mine >= 0) {
+            float v[NPL];
+            pf_load_row<NPL>(a.logits + at, E, lane, -INFINITY, v);
+            const bool active = lane < count;
+            const bool settled = pf_fix_finish<NPL>(count, active ? cand[wave][lane] : 0u, active ? sums[mine + lane] : 0.0f, v, E, picks, norm,
+                                                    ids + wave * K, weights + wave * K, lane);
+            if (lane == 0 && settled) again[wave] = 1u;
+        }
+    }
+    __syncthreads();
+    for (int w = 0; w < here; w++) {
+        if (again[w] != 2u) continue;   // the same for every thread
+        pf_fix_long_way(router, a.x + token(w) * a.x_pitch, E, K, norm, H, route_lds, route_lds + 2 * PF_FIX_CHUNK_FLOATS, ids + w * K,
+                        weights + w * K, wave, lane);
+        __syncthreads();
+    }
+    if ((int)threadIdx.x < here && again[threadIdx.x]) {
+        atomicAdd(a.exact_rows, 1u);
+        if (again[threadIdx.x] == 2u) atomicAdd(a.exact_rows + 1, 1u);
+    }
+    const int p = threadIdx.x;
+    if (p < here * K) {   // at most 16 * 62
+        const size_t to = token(p / K) * K + p % K;
+        a.ids[to] = ids[p];
+        a.route_weights[to] = weights[p];
     }
 }
 
@@ -150,27 +214,6 @@ __global__ void __launch_bounds__(64) pf_k_route_fix_select(PfKernelArgs a) {
     }
 }
 
-// The listed tokens, one wave each: only the experts whose order is in doubt are summed again in serial order
-// (pf_route_fix.h); a token that this does not settle is routed the long way by the same wave.  exact_rows[0]
-// counts the listed tokens, exact_rows[1] those that went the long way.
-template <int NPL>
-__global__ void __launch_bounds__(1024) pf_k_route_fix(PfKernelArgs a) {
-    extern __shared__ float fix_floats[];
-    const int E = a.experts, K = a.top_k, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t listed = a.route_flags[0];
-    for (uint32_t item = blockIdx.x; item < listed; item += gridDim.x) {
-        const int t = (int)a.route_flags[1 + item];
-        const int how = pf_route_fix_block<NPL>(reinterpret_cast<const float *>(a.w[0]), a.x + (size_t)t * a.x_pitch,
-                                                a.logits + (size_t)t * E, a.logit_ssq + (size_t)t * E, E, K, a.norm_topk != 0,
-                                                a.hidden, fix_floats, a.ids + (size_t)t * K, a.route_weights + (size_t)t * K,
-                                                wave, lane);
-        if (threadIdx.x == 0) {
-            atomicAdd(a.exact_rows, 1u);
-            if (how == 2) atomicAdd(a.exact_rows + 1, 1u);
-        }
-    }
-}
-
 // Every token through the exact path (expert counts the fast kernel cannot hold): the full list.
 __global__ void pf_k_flag_all(uint32_t *list, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -179,38 +222,32 @@ __global__ void pf_k_flag_all(uint32_t *list, int n) {
 }
 
 template <int NPL>
-static void launch_route_fix(const PfKernelArgs &a, int workers, size_t lds, hipStream_t stream) {
+static void launch_route_tokens(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     static bool configured = false;   // once per instantiation: more than the default 64 KB of dynamic LDS
     if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_route_fix<NPL>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  144 * 1024);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(pf_k_route_tokens<NPL>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
         configured = true;
     }
-    hipLaunchKernelGGL(pf_k_route_fix<NPL>, dim3(workers), dim3(1024), lds, stream, a);
+    // a workgroup a compute unit (its LDS and threads leave room for no second one) while sixteen tokens each suffice
+    const int per = min(ROUTE_TOKENS, (tokens + 255) / 256);
+    const size_t lds = (2 * PF_FIX_CHUNK_FLOATS + 3 * (size_t)a.experts) * sizeof(float);
+    hipLaunchKernelGGL(pf_k_route_tokens<NPL>, dim3((tokens + per - 1) / per), dim3(1024), lds, stream, a, tokens);
 }
 
 bool pf_route_needs_slabs(int experts, int top_k) { return experts > ROUTE_MAX_FAST_EXPERTS || top_k >= PF_WAVE - 1; }
 
 void pf_launch_route(const PfKernelArgs &a, int tokens, hipStream_t stream) {
     const int npl = (a.experts + PF_WAVE - 1) / PF_WAVE;
-    if (pf_route_needs_slabs(a.experts, a.top_k))   // the fast routing keeps top_k + 2 keys, one per lane
-        hipLaunchKernelGGL(pf_k_flag_all, dim3((tokens + 255) / 256), dim3(256), 0, stream, a.route_flags, tokens);
-    else if (npl <= 1) hipLaunchKernelGGL(pf_k_route_fast<1>, dim3(tokens), dim3(64), 0, stream, a);
-    else if (npl <= 2) hipLaunchKernelGGL(pf_k_route_fast<2>, dim3(tokens), dim3(64), 0, stream, a);
-    else if (npl <= 4) hipLaunchKernelGGL(pf_k_route_fast<4>, dim3(tokens), dim3(64), 0, stream, a);
-    else if (npl <= 8) hipLaunchKernelGGL(pf_k_route_fast<8>, dim3(tokens), dim3(64), 0, stream, a);
-    else hipLaunchKernelGGL(pf_k_route_fast<16>, dim3(tokens), dim3(64), 0, stream, a);
-    // the listed tokens are few: a fixed number of workgroups walks the list
-    const int workers = tokens < 256 ? tokens : 256;
-    if (!pf_route_needs_slabs(a.experts, a.top_k)) {
-        const size_t lds = pf_route_fix_lds_floats(a.hidden, a.experts) * sizeof(float);
-        if (npl <= 1) launch_route_fix<1>(a, workers, lds, stream);
-        else if (npl <= 2) launch_route_fix<2>(a, workers, lds, stream);
-        else if (npl <= 4) launch_route_fix<4>(a, workers, lds, stream);
-        else if (npl <= 8) launch_route_fix<8>(a, workers, lds, stream);
-        else launch_route_fix<16>(a, workers, lds, stream);
+    if (!pf_route_needs_slabs(a.experts, a.top_k)) {   // the fast routing keeps top_k + 2 keys, one per lane
+        if (npl <= 1) launch_route_tokens<1>(a, tokens, stream);
+        else if (npl <= 2) launch_route_tokens<2>(a, tokens, stream);
+        else if (npl <= 4) launch_route_tokens<4>(a, tokens, stream);
+        else if (npl <= 8) launch_route_tokens<8>(a, tokens, stream);
+        else launch_route_tokens<16>(a, tokens, stream);
         return;
     }
+    hipLaunchKernelGGL(pf_k_flag_all, dim3((tokens + 255) / 256), dim3(256), 0, stream, a.route_flags, tokens);
+    const int workers = tokens < 256 ? tokens : 256;
     // more experts than a wave's registers hold: every token is listed and all its logits are summed serially
     const size_t fix_lds = (size_t)FIX_RING * FIX_BATCH * 1024 + (size_t)a.hidden * sizeof(float);
     static bool configured = false;   // more than the default 64 KB of dynamic LDS
@@ -380,7 +417,7 @@ void pf_launch_group_place(const uint32_t *d_ids, int pairs, int experts, const 
 __global__ void __launch_bounds__(1024) pf_k_group_fused(const uint32_t *ids, int pairs, int E, int tokens, uint32_t *offsets,
                                                          uint32_t *tiles, uint4 *items, uint32_t *pair_to_row, uint32_t *row_to_pair) {
     extern __shared__ __align__(16) uint32_t fused_lds[];
-    pf_group_block<false>(fused_lds, ids, pairs, E, tokens, offsets, tiles, items, pair_to_row, row_to_pair);
+    pf_group_block(fused_lds, ids, pairs, E, tokens, offsets, tiles, items, pair_to_row, row_to_pair);
 }
 
 bool pf_group_fits(const uint32_t *d_ids, int pairs, int experts) {

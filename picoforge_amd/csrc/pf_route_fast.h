@@ -66,6 +66,7 @@ struct PfRouteResult {
     float weight;    // lane r < top_k: route weight of slot r
     bool close;      // uniform: some adjacent pair of the k+1 best logits is within tolerance
     bool bad;        // uniform: a nonfinite logit was seen
+    float best, kth; // uniform: the largest and the smallest of the top_k chosen logits (pf_route_fast_wave)
 };
 
 // One round of extraction: the largest remaining value of the wave, its holder and register.
@@ -256,6 +257,8 @@ __device__ __forceinline__ PfRouteResult pf_route_fast_wave(const float *z_row, 
     pf_route_finish_wave(my_z, my_s2, K, rounds, norm, hidden, total, top_all, lane, out.weight, out.close);
     out.close |= ambiguous;
     out.bad = bad;
+    out.best = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_z), 0));
+    out.kth = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_z), (K < E ? K : E) - 1));
     return out;
 }
 
