@@ -485,7 +485,7 @@ static Carve plan_work(const PfHipMoeDesc *d, size_t cap, bool fused = false, si
     const size_t Tp = prefill ? T : 0, Is = d->shared_inter;
     // one more row each, never written after the workspace's initial memset: the all-zero row
     want[W_X16] = prefill ? (Tp + 1) * pf_prefill_half_row((int)H) * 2 : 0;
-    want[W_ACT16] = prefill ? (Tp * K + 1) * pf_prefill_half_row((int)I) * 2 : 0;
+    want[W_ACT16] = prefill ? (Tp * K + 1) * pf_prefill_act_row(*d) * 2 : 0;
     want[W_SACT16] = prefill ? (Tp + 1) * pf_prefill_half_row((int)Is) * 2 : 0;
     want[W_XSCALE] = Tp * 4;
     want[W_ACTSCALE] = Tp * K * 4;

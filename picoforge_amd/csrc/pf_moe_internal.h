@@ -281,6 +281,7 @@ void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hip
 size_t pf_router_parts_bytes(int experts, int cols);
 void pf_launch_router_parts(const float *d_w, int experts, int cols, void *d_out, hipStream_t stream);
 size_t pf_prefill_half_row(int cols);   // halfs per row of the fp16 form of a matrix with `cols` columns
+size_t pf_prefill_act_row(const PfHipMoeDesc &d);   // of the routed activation rows
 int pf_prefill_max_tiles(int tokens, int experts, int top_k);
 size_t pf_prefill_most_tokens(int hidden);   // that one launch of pf_launch_prefill takes
 // pf_moe_mx.hip: the routed MXFP4 down projection of a chunk, from rows of digits (pf_mx_rows.h) instead of halfs

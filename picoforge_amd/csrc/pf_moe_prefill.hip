@@ -33,6 +33,8 @@ typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 // halfs per row of the fp16 form: high parts, low parts, per (started) 256 columns the 16 group-sum halfs
 // [even groups: 4 high, 4 low][odd groups: 4 high, 4 low]
 __host__ __device__ constexpr size_t pf_half_row(int cols) { return 2 * (size_t)cols + 16 * (((size_t)cols + 255) / 256); }
+// the same with the sums of 16 columns, as Q2_K's minima want them: per started 256 columns 16 high, 16 low halfs
+__host__ __device__ constexpr size_t pf_half_row16(int cols) { return 2 * (size_t)cols + 32 * (((size_t)cols + 255) / 256); }
 
 // ---- Q4_K tensors in tile order (once, at upload) ---------------------------------------------
 // A wave of the grouped product takes a 32-row tile's share of a 256-block at a time.
@@ -169,7 +171,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) 
 // The same for rows of at most 512 PARTS values (the activation rows): one wave per row, four rows per workgroup, the row
 // read once -- a lane keeps its 8 PARTS values between the maximum and the conversion.  With a workgroup per row three
 // of its four waves only took part in the maximum: 22528 rows of 640 values took 36.2 us (routed) + 8.8 (shared), 21.6 so.
-template <int PARTS>
+template <int PARTS, bool SUMS16>
 __device__ __forceinline__ void rows_to_half_short(size_t block, const float *src, size_t src_pitch, int cols, size_t rows, half_t *dst,
                                                    float *scale_out, uint32_t *error_word) {
     const size_t row = block * 4 + (threadIdx.x >> 6);
@@ -198,7 +200,7 @@ __device__ __forceinline__ void rows_to_half_short(size_t block, const float *sr
     e = (e == 0 || e == 255) ? 126 : min(e, 252);             // zero, subnormal or nonfinite row: scale 1
     const float scale = __int_as_float((e + 1) << 23);        // 2^(e-126)
     const float inv = __int_as_float((253 - e) << 23);        // 2^(126-e)
-    half_t *out = dst + row * pf_half_row(cols);
+    half_t *out = dst + row * (SUMS16 ? pf_half_row16(cols) : pf_half_row(cols));
 #pragma unroll
     for (int p = 0; p < PARTS; p++) {
         const int j = 64 * p + lane;
@@ -218,6 +220,15 @@ __device__ __forceinline__ void rows_to_half_short(size_t block, const float *sr
             *reinterpret_cast<half8v *>(out + cols + 8 * j) = lo;
         }
         sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0xB1, 0xF, 0xF, true));   // quad xor 1
+        if (SUMS16) {
+            if (mine && (j & 1) == 0) {
+                const half_t sh = (half_t)sum, sl = (half_t)(sum - (float)sh);
+                half_t *sums = out + 2 * cols + 32 * (j >> 5) + ((j & 31) >> 1);
+                sums[0] = sh;
+                sums[16] = sl;
+            }
+            continue;
+        }
         sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x4E, 0xF, 0xF, true));   // quad xor 2
         if (mine && (j & 3) == 0) {
             const int g = j >> 2;
@@ -231,16 +242,18 @@ __device__ __forceinline__ void rows_to_half_short(size_t block, const float *sr
 }
 
 // Two matrices of such rows in one launch (the routed and the shared activation rows): workgroups [0, blocks_a) take
-// the first, the others the second.  DIGITS: the first as the digit rows of pf_moe_mx.hip (of at most 1024 values).
-template <int PARTS, bool DIGITS>
+// the first, the others the second.  The first as KIND says: with the sums of 32 or of 16 columns, or as the digit rows of pf_moe_mx.hip
+// (of at most 1024 values).
+enum RowKind { ROWS_SUMS32, ROWS_SUMS16, ROWS_DIGITS };
+template <int PARTS, RowKind KIND>
 __global__ void __launch_bounds__(256) pf_k_rows_to_half_short2(const float *src_a, int cols_a, size_t rows_a, half_t *dst_a, float *scale_a,
                                                                 unsigned blocks_a, const float *src_b, int cols_b, size_t rows_b,
                                                                 half_t *dst_b, float *scale_b, uint32_t *error_word) {
     if (blockIdx.x < blocks_a) {
-        if (DIGITS) pf_rows_to_digits(blockIdx.x, src_a, cols_a, rows_a, reinterpret_cast<uint32_t *>(dst_a), scale_a, error_word);
-        else rows_to_half_short<PARTS>(blockIdx.x, src_a, (size_t)cols_a, cols_a, rows_a, dst_a, scale_a, error_word);
+        if (KIND == ROWS_DIGITS) pf_rows_to_digits(blockIdx.x, src_a, cols_a, rows_a, reinterpret_cast<uint32_t *>(dst_a), scale_a, error_word);
+        else rows_to_half_short<PARTS, KIND == ROWS_SUMS16>(blockIdx.x, src_a, (size_t)cols_a, cols_a, rows_a, dst_a, scale_a, error_word);
     }
-    else rows_to_half_short<PARTS>(blockIdx.x - blocks_a, src_b, (size_t)cols_b, cols_b, rows_b, dst_b, scale_b, error_word);
+    else rows_to_half_short<PARTS, false>(blockIdx.x - blocks_a, src_b, (size_t)cols_b, cols_b, rows_b, dst_b, scale_b, error_word);
 }
 
 static void launch_rows_to_half(const float *src, size_t src_pitch, int cols, size_t rows, half_t *dst, float *scale_out,
@@ -545,6 +558,12 @@ template <int FMT> __device__ __forceinline__ GemmRows gemm_rows(const PfKernelA
         r.block_step = 64; r.head_step = 2; r.run_step = 16;
         r.tile_step = 32 * row_bytes; r.head_tile_step = 64 * blocks;
         return r;
+    } else if (FMT == PF_Q2_K) {   // GGUF rows
+        r.bytes = (uint32_t)a.expert_bytes[t];
+        r.base = a.w[t] + expert * a.expert_bytes[t];
+        r.lane_at = n * row_bytes + 16 + 16 * h; r.head_at = n * row_bytes + 68 * h;
+        r.block_step = r.head_step = 84; r.run_step = 32;
+        r.tile_step = r.head_tile_step = 32 * row_bytes;
     } else {
         r.bytes = (uint32_t)a.expert_bytes[t];
         r.base = (tiled ? a.wt[t] : a.w[t]) + expert * a.expert_bytes[t];
@@ -658,6 +677,58 @@ __device__ __forceinline__ half8v half8_of_bytes(uint32_t b0, uint32_t b1, half_
     const half2v v3 = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, b1, 0x04030402u)) - c;
     return half8v{v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
 }
+
+// Q2_K (src/qwen4_packed.c:106-121): a weight is d * scale * code - dmin * min with a 4-bit scale and minimum for 16 columns and a
+// 2-bit code, so scale * code <= 45 is an exact fp16 operand, made as Q4_K's are (the code stays where it is in its byte, the scale brings
+// the power of four), and the minima are the operand of a product with the rows' sums of 16 columns.  Lane (n, h) loads bytes
+// 16h..16h+15 of both halves of a block's codes; step i is the eight bytes i % 2 of them at bits 2 (i / 2 % 4), its columns those of Q4_K.
+// Rows are read where they lie, 84 bytes a block: an instruction touches 32 lines or more for 512 to 1024 bytes, and the L2's lines
+// bound the kernel.  So a block's three loads follow each other while its lines are there (apart 276 us for 1500 tokens of the
+// checkpoints' widths, together 257), and the scales and the two factors are one load, the lower lanes' and the upper ones' (254).
+// On the plain kernel it took 339, 239 -> 162 for 500 tokens, 164 -> 119 for 1000 of 2048 x 512; the distance to 64 bits is the same
+// (4.9e-7 at 2560 x 640).  A block's loads asked for half a block earlier, in registers of their own: 24 of them spilled, 320.
+template <> struct GemmBlock<PF_Q2_K> {
+    uint4v code[2], head;    // head: the scales in lanes 0..31, the block's last 16 bytes in lanes 32..63
+    half2v scale[4];         // of a 64-column run: the scales of its two groups' halves h, times 2^10 and 2^8, or 2^6 and 2^4
+    float d, low;
+    static __device__ __forceinline__ constexpr int chunk(int i) { return 4 * ((i & 3) >> 1) + (i & 1); }
+    static constexpr int chunk_h = 2;
+    static constexpr int requests = 5;   // of a block: the rows' sums (two), its header, two halves of codes
+    __device__ __forceinline__ void request_half(int j, const PfBuffer &b, const GemmRows &r, uint32_t at) {
+        code[j] = __builtin_amdgcn_raw_buffer_load_b128(b, (int)r.lane_at, (int)(at + (uint32_t)j * r.run_step), 0);
+    }
+    __device__ __forceinline__ void request_head(const PfBuffer &b, const GemmRows &r, uint32_t at) {
+        head = __builtin_amdgcn_raw_buffer_load_b128(b, (int)r.head_at, (int)at, 0);
+    }
+    // Returns the minima of sub-groups 8h..8h+7 as an operand.
+    __device__ __forceinline__ half8v open() {
+        uint32_t sc[4], dm = 0;   // the lower lanes' words and the upper lanes' last one, in all lanes
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const auto halves = __builtin_amdgcn_permlane32_swap(head[c], head[c], false, false);
+            sc[c] = halves[0];
+            if (c == 3) dm = halves[1];
+        }
+        const half2v both = __builtin_bit_cast(half2v, dm);
+        d = (float)both.x * 16384.0f; low = (float)both.y;
+        const bool second = pf_lane() >> 5;
+        const uint32_t bias = 0x64646464u;   // a byte under the exponent byte 0x64 is 1024 + byte
+        const half2v k = {(half_t)1024.0f, (half_t)1024.0f}, up0 = {(half_t)1024.0f, (half_t)256.0f}, up1 = {(half_t)64.0f, (half_t)16.0f};
+#pragma unroll
+        for (int half = 0; half < 2; half++) {   // sub-groups h, 2 + h, 4 + h, 6 + h of the half
+            const uint32_t mine = __builtin_amdgcn_perm(sc[2 * half + 1], sc[2 * half], second ? 0x07050301u : 0x06040200u) & 0x0F0F0F0Fu;
+            scale[2 * half] = (__builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, mine, 0x04010400u)) - k) * up0;
+            scale[2 * half + 1] = (__builtin_bit_cast(half2v, __builtin_amdgcn_perm(bias, mine, 0x04030402u)) - k) * up1;
+        }
+        return half8_of_bytes(((second ? sc[2] : sc[0]) >> 4) & 0x0F0F0F0Fu, ((second ? sc[3] : sc[1]) >> 4) & 0x0F0F0F0Fu, (half_t)1024.0f);
+    }
+    __device__ __forceinline__ half8v operand(int i) const {
+        const half_t f = (i & 2) ? scale[i >> 2].y : scale[i >> 2].x;
+        const uint32_t mask = 0x03030303u << (2 * ((i >> 1) & 3));
+        return join(q4_scaled_codes(code[i >> 3][2 * (i & 1)], mask, half2v{f, f}), q4_scaled_codes(code[i >> 3][2 * (i & 1) + 1], mask, half2v{f, f}));
+    }
+};
+
 // signed bytes: flip the sign bit, read as unsigned, take 128 more away
 __device__ __forceinline__ half8v half8_of_signed_bytes(uint32_t b0, uint32_t b1) {
     return half8_of_bytes(b0 ^ 0x80808080u, b1 ^ 0x80808080u, (half_t)1152.0f);
@@ -703,6 +774,12 @@ struct GemmSource {
         asm volatile("" ::: "memory");   // what is requested from here on is younger
         __builtin_amdgcn_sched_barrier(0);
     }
+    // The operand row's sums of 16 columns of a block, high and low parts; of columns that do not exist: zeros.
+    __device__ __forceinline__ void request_sums16(half8v (&sums)[2], int kb, bool whole) const {
+        const uint32_t mine = whole || pf_lane() < 32 ? sum_at : PF_NOWHERE;
+#pragma unroll
+        for (int p = 0; p < 2; p++) sums[p] = __builtin_bit_cast(half8v, __builtin_amdgcn_raw_buffer_load_b128(x[0], (int)mine, 64 * kb + 32 * p, 0));
+    }
 };
 
 // One 256-block of a wave's tile.  from, to: the copies of this block's rows (at the lane's) and of the next one's.  at, head_at: the
@@ -735,6 +812,45 @@ __device__ __forceinline__ void gemm_block(GemmBlock<FMT> &w, half8v &sums, cons
         if ((i & 3) == 3) { w.request_run(i >> 2, src.weights, src.rows, at); __builtin_amdgcn_sched_barrier(0); }
     }
     lds_barrier<GemmBlock<FMT>::requests>();   // the next block's rows are there; its weights, requested after them, may not be
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = fmaf(d, part[r], acc[r]);
+}
+
+// The same for Q2_K.  whole: the block's 256 columns exist, else its first 128 (next_whole: the next block's).
+template <int PARTS>
+__device__ __forceinline__ void gemm_block_q2(GemmBlock<PF_Q2_K> &w, half8v (&sums)[2], const GemmSource &src, uint32_t at, uint32_t head_at, int next_kb,
+                                              bool whole, bool next_whole, int wave, const lds_byte *__restrict from, lds_byte *__restrict to, float16v &acc) {
+    const float16v zero = {0};
+    src.request_rows(wave, next_kb, to);
+    const half8v minima = w.open();
+    float16v q = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[0], minima, zero, 0, 0, 0);
+    q = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[1], minima, q, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = fmaf(-w.low, q[r], acc[r]);
+    const float d = w.d;
+    src.request_sums16(sums, next_kb, next_whole);
+    float16v part = zero;
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        if (half == 0 || whole) {   // (uniform)
+#pragma unroll
+            for (int i = 8 * half; i < 8 * half + 8; i++) {
+                const half8v b = w.operand(i);
+#pragma unroll
+                for (int p = 0; p < PARTS; p++) {
+                    const half8v x = *reinterpret_cast<const __attribute__((address_space(3))) half8v *>(from + p * GEMM_PART_BYTES + (i >> 2) * 4 * GEMM_IMAGE +
+                                                                                                         GemmBlock<PF_Q2_K>::chunk(i) * 128);
+                    part = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, b, part, 0, 0, 0);
+                }
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    w.request_head(src.heads, src.rows, head_at);
+    w.request_half(0, src.weights, src.rows, at);
+    w.request_half(1, src.weights, src.rows, at);
+    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier<GemmBlock<PF_Q2_K>::requests>();
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = fmaf(d, part[r], acc[r]);
 }
@@ -795,14 +911,19 @@ __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem 
             for (int j = 0; j < 4; j++) w.request_run(j, src.weights, src.heads, src.rows, tile * src.rows.tile_step, tile * src.rows.head_tile_step);
         } else {
             w.request_head(src.heads, src.rows, tile * src.rows.head_tile_step);
+            if constexpr (FMT == PF_Q2_K) {
+                w.request_half(0, src.weights, src.rows, tile * src.rows.tile_step);
+                w.request_half(1, src.weights, src.rows, tile * src.rows.tile_step);
+            } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) w.request_run(j, src.weights, src.rows, tile * src.rows.tile_step);
+                for (int j = 0; j < 4; j++) w.request_run(j, src.weights, src.rows, tile * src.rows.tile_step);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     }
     // activation rows: the tile's own rows (down, and the shared expert's tokens) or gathered by token
     const bool gathered = MODE == PF_GEMM_GATE_UP && !g.shared;
-    const uint32_t a_pitch = 2u * (uint32_t)pf_half_row(a_cols);   // bytes
+    const uint32_t a_pitch = 2u * (uint32_t)(FMT == PF_Q2_K ? pf_half_row16(a_cols) : pf_half_row(a_cols));   // bytes
     const int row0 = gathered ? 0 : g.shared ? g.m0 : g.first;
     const uint8_t *base = reinterpret_cast<const uint8_t *>(MODE == PF_GEMM_GATE_UP ? a.x16 : g.shared ? a.sact16 : a.act16) + (size_t)row0 * a_pitch;
     const uint32_t bytes = gathered ? (uint32_t)min((size_t)a.token_cap * a_pitch, (size_t)PF_NOWHERE) : (uint32_t)g.rows_here * a_pitch;
@@ -818,8 +939,10 @@ __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem 
     src.sum_at = n < g.rows_here ? mine * a_pitch + 4u * (uint32_t)a_cols + 16u * (uint32_t)h : PF_NOWHERE;
     const float scale_mine = (MODE == PF_GEMM_GATE_UP ? a.x_scale : g.shared ? a.sact_scale : a.act_scale)[row0 + (int)mine];
     src.request_rows(wave, 0, lds);
-    half8v sums;
+    half8v sums, sums16[2];
+    auto whole = [&](int kb) { return 256 * kb + 256 <= a_cols; };   // (widths are whole halves of a block)
     if (FMT == PF_Q4_K) sums = __builtin_bit_cast(half8v, __builtin_amdgcn_raw_buffer_load_b128(src.x[0], (int)src.sum_at, 0, 0));
+    if (FMT == PF_Q2_K) src.request_sums16(sums16, 0, whole(0));
     lds_barrier<0>();
     const lds_byte *take = lds + (n >> 3) * GEMM_IMAGE + GemmBlock<FMT>::chunk_h * h * 128 + (n & 7) * 16;
     float16v acc = {0}, apart[2] = {{0}, {0}};
@@ -834,6 +957,7 @@ __device__ __forceinline__ void gemm_tile(const PfKernelArgs &a, const GemmItem 
         const lds_byte *from = take + copy * GEMM_COPY_BYTES;
         lds_byte *to = lds + (copy ^ 1) * GEMM_COPY_BYTES;
         if constexpr (FMT == PF_Q8_0) gemm_block_q8<PARTS>(w, src, at, head_at, next_kb, min(8, (a_cols - 256 * kb) / 32), wave, from, to, apart);
+        else if constexpr (FMT == PF_Q2_K) gemm_block_q2<PARTS>(w, sums16, src, at, head_at, next_kb, whole(kb), whole(next_kb), wave, from, to, acc);
         else gemm_block<FMT, PARTS>(w, sums, src, at, head_at, next_kb, wave, from, to, lds + IQ2_GRID_OFF, acc);
         copy ^= 1;
         kb = next_kb;
@@ -1365,7 +1489,15 @@ bool pf_prefill_supported(const PfHipMoeDesc &d) {
     return true;
 }
 
+// A Q2_K down projection beside a Q8_0 shared expert's on pf_k_pf_gemm: activation rows that the conversion holds in registers (at most
+// 1024 values).  The others are the plain kernel's, 1.3 to 1.5 times slower.
+static bool pf_q2_down(const uint32_t *type, int inter, int shared_inter) {
+    return type[3] == PF_Q2_K && type[6] == PF_Q8_0 && inter <= 1024 && shared_inter <= 1024;
+}
 size_t pf_prefill_half_row(int cols) { return pf_half_row(cols); }
+size_t pf_prefill_act_row(const PfHipMoeDesc &d) {
+    return pf_q2_down(d.type, (int)d.inter, (int)d.shared_inter) ? pf_half_row16((int)d.inter) : pf_half_row((int)d.inter);
+}
 size_t pf_prefill_most_tokens(int hidden) { return PF_NOWHERE / (2 * pf_half_row(hidden)) / 32 * 32; }
 // sum over experts of ceil(rows / 32) <= pairs / 32 + experts, plus the shared expert's tiles
 int pf_prefill_max_tiles(int tokens, int experts, int top_k) {
@@ -1458,11 +1590,13 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
     if (a.type[4] != gate_fmt && !q8) launch_gemm_plain<PF_GEMM_GATE_UP>(a, tokens, shared_tiles, (Is + 31) / 32, 1, PLAIN_SHARED, stream);
     const int widest = I > Is ? I : Is;
     const bool digits = a.wm != nullptr;   // the routed rows as digits (they are of at most 640 values)
+    const bool q2_down = pf_q2_down(a.type, I, Is);
     if (widest <= 1024 && P > 0 && tokens > 0) {
         const unsigned rows_a = digits ? 4u * pf_mx_rows_a_wave(I) : 4u, blocks_a = ((unsigned)P + rows_a - 1) / rows_a, blocks_b = (unsigned)((tokens + 3) / 4);
-        hipLaunchKernelGGL(digits ? (widest <= 512 ? pf_k_rows_to_half_short2<1, true> : pf_k_rows_to_half_short2<2, true>)
-                                  : (widest <= 512 ? pf_k_rows_to_half_short2<1, false> : pf_k_rows_to_half_short2<2, false>), dim3(blocks_a + blocks_b), dim3(256), 0,
-                           stream, a.act, I, (size_t)P, (half_t *)a.act16, a.act_scale, blocks_a, a.shared_act, Is, (size_t)tokens,
+        hipLaunchKernelGGL(digits ? (widest <= 512 ? pf_k_rows_to_half_short2<1, ROWS_DIGITS> : pf_k_rows_to_half_short2<2, ROWS_DIGITS>)
+                           : q2_down ? (widest <= 512 ? pf_k_rows_to_half_short2<1, ROWS_SUMS16> : pf_k_rows_to_half_short2<2, ROWS_SUMS16>)
+                                     : (widest <= 512 ? pf_k_rows_to_half_short2<1, ROWS_SUMS32> : pf_k_rows_to_half_short2<2, ROWS_SUMS32>),
+                           dim3(blocks_a + blocks_b), dim3(256), 0, stream, a.act, I, (size_t)P, (half_t *)a.act16, a.act_scale, blocks_a, a.shared_act, Is, (size_t)tokens,
                            (half_t *)a.sact16, a.sact_scale, a.error_word);
     } else {
         if (digits) pf_launch_rows_to_digits(a.act, I, (size_t)P, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
@@ -1476,6 +1610,11 @@ void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, in
         else launch_gemm<PF_GEMM_DOWN, PF_Q4_K, PF_Q4_K>(a, tokens, routed_cap, H, gi, stream);
     }
     if (digits) pf_launch_mx_down(a, tokens, routed_cap, stream);
+    if (q2_down) {
+        launch_gemm<PF_GEMM_DOWN, PF_Q2_K, PF_Q8_0>(a, tokens, routed_cap, H, gi, stream);
+        pf_launch_combine(a, tokens, stream);
+        return;
+    }
     // (beside routed items of the plain kernel a Q8_0 shared expert's cost nothing: in a launch of its own it made the down stage of
     // the q2 profile's 1024-token chunk 169 us instead of 157, at the checkpoints' widths 291 instead of 271)
     const bool plain_routed = a.type[3] != gate_fmt && !digits, q8_shared = a.type[6] == PF_Q8_0 && !plain_routed;
