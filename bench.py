@@ -128,7 +128,7 @@ BATCH_STAGES = ["pf_k_batch_router (router logits by FP32 MFMA, digit images of 
                 "routing + grouping (top-k, serial-order re-routes, histogram/scan/placement)",
                 "pf_k_batch_gate_up (gate/up + SwiGLU by int8 MFMA, digit images of the activations)",
                 "pf_k_batch_down + pf_k_pf_combine (down by int8 MFMA, slot-ordered combine)"]
-PREFILL_STAGES = ["pf_k_pf_router (router logits by FP32 MFMA)",
+PREFILL_STAGES = ["pf_k_pf_router (router logits by MFMA on bf16 parts)",
                   "routing + grouping (top-k, serial-order re-routes, histogram/scan/placement beside the fp16 copy of x)",
                   "pf_k_pf_gemm<gate_up> (grouped gate/up + SwiGLU by FP16 MFMA, then fp16 copy of the activations)",
                   "pf_k_pf_gemm<down> + pf_k_pf_combine (grouped down by FP16 MFMA, slot-ordered combine)"]

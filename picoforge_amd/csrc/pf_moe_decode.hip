@@ -25,7 +25,7 @@
 #include "pf_image.h"
 #include "pf_route_device.h"
 #include "pf_route_fast.h"
-#include "pf_route_fix.h"
+#include "pf_route_fix_many.h"
 #include "pf_upload_addr.h"
 #include "pf_mx_rows.h"
 
@@ -1141,7 +1141,8 @@ __global__ void __launch_bounds__(1024) pf_k_dec_gate_up_q4t(PfKernelArgs a, int
 // registers, which leave room for one workgroup per compute unit only.  So the tokens are routed first, one workgroup
 // each (a flagged token is routed again once, not by every workgroup of its grid row), and kernel 2 takes its expert
 // from the ids: eight waves, at most 64 registers a lane and a few KB of LDS, four workgroups per compute unit, some
-// computing while the others wait for their weights.
+// computing while the others wait for their weights.  101 tokens, some of them flagged: 21.5 us traced; 25 with the k best looked for again and
+// rows asked for when they are put down (pf_route_fix_block).
 template <int NPL>
 __global__ void __launch_bounds__(1024) pf_k_dec_route(PfKernelArgs a) {
     extern __shared__ int lds[];
@@ -1155,14 +1156,19 @@ __global__ void __launch_bounds__(1024) pf_k_dec_route(PfKernelArgs a) {
     const int parts = min(8, (E + 63) / 64), chunk = (E + parts - 1) / parts, rounds = K + 1;
     if (wave < parts) pf_route_stage1<NPL1>(a.logits, a.logit_ssq, E, wave, chunk, rounds, norm, &R.cands[0], lane);
     __syncthreads();
+    float kth = 0.0f, best_z = 0.0f;
     if (wave == 0) {
         const PfRouteResult r = pf_route_stage2(&R.cands[0], parts, K, rounds, norm, H, lane);
         if (lane < K) { R.ids[lane] = r.id; R.weights[lane] = r.weight; }
         if (lane == 0) { R.close[0] = r.close ? 1u : 0u; R.nonfinite[0] = r.bad ? 1u : 0u; }
+        kth = r.kth; best_z = r.best;
     }
     __syncthreads();
     if (R.close[0]) {
-        q4t_route_fix<NPL>(reinterpret_cast<const float *>(a.w[0]), a.x, a.logits, a.logit_ssq, E, K, norm, H, 0, &R);
+        const int how = pf_fix_token<NPL>(reinterpret_cast<const float *>(a.w[0]), a.x, a.logits, a.logit_ssq, kth, best_z, E, K, norm, H,
+                                          reinterpret_cast<float *>(lds), R.ids, R.weights, wave, lane);
+        if (threadIdx.x == 0) { R.close_mask = (uint32_t)how; R.bad = R.nonfinite[0]; }
+        __syncthreads();
     } else {
         if (threadIdx.x == 0) { R.close_mask = 0; R.bad = R.nonfinite[0]; }
         __syncthreads();

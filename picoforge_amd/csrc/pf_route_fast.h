@@ -66,7 +66,7 @@ struct PfRouteResult {
     float weight;    // lane r < top_k: route weight of slot r
     bool close;      // uniform: some adjacent pair of the k+1 best logits is within tolerance
     bool bad;        // uniform: a nonfinite logit was seen
-    float best, kth; // uniform: the largest and the smallest of the top_k chosen logits (pf_route_fast_wave)
+    float best, kth; // uniform: the largest and the smallest of the top_k chosen logits
 };
 
 // One round of extraction: the largest remaining value of the wave, its holder and register.
@@ -401,5 +401,7 @@ __device__ __forceinline__ PfRouteResult pf_route_stage2(PfRouteCands *c, int pa
     pf_route_finish_wave(my_z, my_s2, K, rounds, norm, hidden, total, top_all, lane, out.weight, out.close);
     out.id = my_id;
     out.bad = bad;
+    out.best = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_z), 0));
+    out.kth = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_z), min(K, rounds) - 1));
     return out;
 }

@@ -1,7 +1,7 @@
 // Re-routing of several flagged tokens by the waves of one workgroup: the steps of pf_route_fix.h (candidates, serial sums, order, the
 // long way) one by one, so that the candidates of several tokens can share the chain's wave, a lane each, and their rows are asked for a
-// chunk before their products are put down.  pf_route_fix_block has the same steps for one token in a form of its own: built from these
-// it moved the decode kernels' code, 0.5 to 1.5 % of a token's four layers (65.8 us against 66.8).
+// chunk before their products are put down.  pf_route_fix_block has the same steps in a form of its own: built from these
+// it moved the one-token kernels' code, 0.5 to 1.5 % of a token's four layers (65.8 us against 66.8).
 #pragma once
 #include "pf_route_fix.h"
 
@@ -158,4 +158,36 @@ __device__ __forceinline__ void pf_fix_long_way(const float *router, const float
     }
     __syncthreads();
     if (wave == 0) pf_route_exact_wave(z, z + E, z + 2 * E, E, K, norm, ids_out, w_out, lane);
+}
+
+// One token, called by every wave of a workgroup of PF_FIX_THREADS threads, whose routing knows the smallest and the largest of the k
+// best logits (wave 0).  lds: 68 + 2 PF_FIX_CHUNK_FLOATS + 3 E floats; the rest as pf_route_fix_block.
+template <int NPL>
+__device__ __forceinline__ int pf_fix_token(const float *router, const float *x, const float *z_row, const float *ssq_row, float kth, float best_z, int E,
+                                            int K, bool norm, int H, float *lds, uint32_t *ids_out, float *w_out, int wave, int lane) {
+    uint32_t *cand = reinterpret_cast<uint32_t *>(lds), *hand = cand + 64;   // hand[0]: candidates (0: the long way), hand[1]: outcome
+    float *stage = lds + 68;
+    const int picks = K < E ? K : E;
+    float v[NPL];
+    int count = 0;
+    if (wave == 0) {
+        float s2[NPL];
+        pf_load_row<NPL>(z_row, E, lane, -INFINITY, v);
+        pf_load_row<NPL>(ssq_row, E, lane, 0.0f, s2);
+        count = pf_fix_candidates<NPL>(v, s2, kth, best_z, E, picks, H, pf_fix_by_pieces(router, H), cand, lane);
+        if (lane == 0) hand[0] = (uint32_t)count;
+    }
+    __syncthreads();
+    const int n = (int)hand[0];
+    float logit = 0.0f;
+    if (n > 0) logit = pf_fix_sums(n, H, stage, [&](int r) { return router + (size_t)cand[r] * H; }, [&](int, int k) { return pf_fix_values(x, k); }, wave, lane);
+    if (wave == 0) {
+        const bool settled = n > 0 && pf_fix_finish<NPL>(count, lane < count ? cand[lane] : 0u, logit, v, E, picks, norm, ids_out, w_out, lane);
+        if (lane == 0) hand[1] = settled ? 1u : 2u;
+    }
+    __syncthreads();
+    const int how = (int)hand[1];
+    if (how == 2) pf_fix_long_way(router, x, E, K, norm, H, stage, stage + 2 * PF_FIX_CHUNK_FLOATS, ids_out, w_out, wave, lane);
+    __syncthreads();
+    return how;
 }
