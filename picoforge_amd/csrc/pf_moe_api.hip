@@ -4,6 +4,7 @@
 #include "pf_host_calls.h"
 #include "pf_host_rows.h"
 #include "pf_piece_order.h"
+#include "pf_router_addr.h"
 #include "../../include/pf_iq2_codes.h"
 #include <stdio.h>
 #include <stdlib.h>

@@ -278,7 +278,6 @@ void pf_launch_group(const PfKernelArgs &a, const uint32_t *ids, int tokens, hip
 void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream);
 void pf_launch_q4k_tile(const uint8_t *d_src, uint8_t *d_dst, size_t rows, int blocks_per_row, hipStream_t stream);
 void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hipStream_t stream);
-size_t pf_router_parts_bytes(int experts, int cols);
 void pf_launch_router_parts(const float *d_w, int experts, int cols, void *d_out, hipStream_t stream);
 size_t pf_prefill_half_row(int cols);   // halfs per row of the fp16 form of a matrix with `cols` columns
 size_t pf_prefill_act_row(const PfHipMoeDesc &d);   // of the routed activation rows

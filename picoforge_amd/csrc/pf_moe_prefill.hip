@@ -23,6 +23,7 @@
 #include "pf_upload_addr.h"
 #include "pf_plain_walk.h"
 #include "pf_grouped.h"
+#include "pf_router_addr.h"
 #include "pf_mx_rows.h"
 #include "pf_group_device.h"
 
@@ -333,9 +334,8 @@ __global__ void __launch_bounds__(256) pf_k_router_parts(const float *w, int exp
 #pragma unroll
     for (int p = 0; p < 3; p++) out[(3 * step + p) * 64 + lane] = r.part[p];
 }
-size_t pf_router_parts_bytes(int experts, int cols) { return (size_t)((experts + 31) / 32) * 32 * cols * 6; }
 void pf_launch_router_parts(const float *d_w, int experts, int cols, void *d_out, hipStream_t stream) {
-    const size_t threads = (size_t)((experts + 31) / 32) * (size_t)(cols / 16) * 64;
+    const size_t threads = (size_t)pf_router_tiles(experts) * (size_t)(cols / 16) * 64;
     hipLaunchKernelGGL(pf_k_router_parts, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, d_w, experts, cols, reinterpret_cast<uint4v *>(d_out), threads);
 }
 
@@ -356,16 +356,16 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
     const int lines = H / 32, l0 = lines * wave / PF_ROUTER_WAVES, l1 = lines * (wave + 1) / PF_ROUTER_WAVES;
     const int lr = lane >> 3, piece = lane & 7;   // fetch: row within a group of eight, 16-byte piece of the line
     constexpr int GROUPS = 4 * TR;                // of eight rows
-    // a buffer per eight x rows, one for the experts' parts; rows beyond the last are zeros
+    // a buffer per eight x rows, rows beyond the last zeros; one for the experts' parts, which no load leaves (a buffer's bound is not
+    // compared with the scalar part of an offset)
     PfBuffer x_rows[GROUPS];
 #pragma unroll
     for (int g = 0; g < GROUPS; g++) {
         const int first = t0 + 8 * g, rows = min(max(tokens - first, 0), 8);
         x_rows[g] = pf_buffer(a.x + (size_t)min(first, tokens - 1) * a.x_pitch, rows ? (uint32_t)(((size_t)(rows - 1) * a.x_pitch + H) * 4) : 0);
     }
-    const uint32_t tile_bytes = 192u * (uint32_t)H;
-    const PfBuffer experts = pf_buffer(a.router_parts + (size_t)(e0 / 32) * tile_bytes, (uint32_t)min(TC, (E - e0 + 31) / 32) * tile_bytes);
-    const int x_at = (int)((uint32_t)lr * (uint32_t)a.x_pitch * 4u + 16u * (uint32_t)piece), w_at = 16 * lane;
+    const PfBuffer experts = pf_buffer(a.router_parts + pf_router_tile_at(e0 / 32, H), (uint32_t)min(TC, pf_router_tiles(E) - e0 / 32) * (uint32_t)pf_router_tile_at(1, H));
+    const int x_at = (int)((uint32_t)lr * (uint32_t)a.x_pitch * 4u + 16u * (uint32_t)piece);
     float *mine = router_lds + (size_t)wave * TR * 32 * PF_ROUTER_PITCH;
     float16v acc[TR][TC];
 #pragma unroll
@@ -381,10 +381,12 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
     };
     auto request = [&](int step, int l) {
 #pragma unroll
-        for (int c = 0; c < TC; c++)
+        for (int c = 0; c < TC; c++) {
+            const int tile = pf_router_tile_read(E, e0 / 32, c);
 #pragma unroll
             for (int p = 0; p < 3; p++)
-                w[step][c].part[p] = __builtin_amdgcn_raw_buffer_load_b128(experts, w_at, (int)((uint32_t)c * tile_bytes + 3072u * (uint32_t)(2 * min(l, l1 - 1) + step) + 1024u * p), 0);
+                w[step][c].part[p] = __builtin_amdgcn_raw_buffer_load_b128(experts, (int)pf_router_part_at(0, 0, 0, 0, lane), (int)pf_router_part_at(tile, H, 2 * min(l, l1 - 1) + step, p, 0), 0);
+        }
     };
     auto stage = [&]() {
 #pragma unroll

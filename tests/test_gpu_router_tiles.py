@@ -58,3 +58,17 @@ def test_router_logits(product, e, i, tokens):
     error = np.abs(got - want) / size
     print(f"largest error {error.max():.2e} of the magnitudes' sum", flush=True)
     assert error.max() <= (1 + 12 + 7) * 2.0 ** -23
+
+
+@pytest.mark.parametrize("e,tokens", [(480, 600), (160, 1700), (480, 1700)])
+def test_odd_number_of_expert_tiles(product, oracle, e, tokens):
+    """Workgroups of two tiles of 32 experts with one tile left for the last of them."""
+    print(f"case router tiles, odd e={e} tokens={tokens}", flush=True)
+    cfg = abi.moe_config(256, e, 4, 256, 256)
+    weights, few = make_layer_inputs(cfg, abi.GGUF_Q4_K, 97, seed=e)
+    row = np.arange(tokens) % 97
+    want = [a[row] for a in forward_with(oracle, cfg, weights, few)[:3]]
+    with pf.MoeLayer(product, cfg, weights, tokens) as layer:
+        layer.force_grouped()
+        _, y, ids, w = layer.forward(few[row])
+        assert_parity(y, ids, w, *want, label=f"e={e} T={tokens}")
