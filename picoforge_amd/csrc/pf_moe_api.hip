@@ -978,7 +978,7 @@ static int forward_enqueue(const PfHipMoe *moe, PfHipWork *work, const float *d_
         snprintf(g_error, sizeof g_error, "the layer's routed experts are not resident: forward it through an expert pool");
         return PF_HIP_E_UNSUPPORTED;
     }
-    const bool aligned = (x_pitch % 4 == 0) && ((uintptr_t)d_x % 16 == 0) && x_pitch < (size_t)1 << 27;   // (eight rows by 32-bit offsets)
+    const bool aligned = (x_pitch % 4 == 0) && ((uintptr_t)d_x % 16 == 0);
     const Family family = aligned ? kernel_family(moe, work, tokens) : FAMILY_GENERAL;
     if (family == FAMILY_DECODE) {
         pf_launch_decode(a, (int)tokens, s, work->stage_limit);

@@ -356,16 +356,12 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
     const int lines = H / 32, l0 = lines * wave / PF_ROUTER_WAVES, l1 = lines * (wave + 1) / PF_ROUTER_WAVES;
     const int lr = lane >> 3, piece = lane & 7;   // fetch: row within a group of eight, 16-byte piece of the line
     constexpr int GROUPS = 4 * TR;                // of eight rows
-    // a buffer per eight x rows, rows beyond the last zeros; one for the experts' parts, which no load leaves (a buffer's bound is not
-    // compared with the scalar part of an offset)
-    PfBuffer x_rows[GROUPS];
+    // the x rows by their addresses, in place of those beyond the last token the last one again; the experts' parts in a buffer that no
+    // load leaves (its bound is not compared with the scalar part of an offset)
+    const float4v *x_row[GROUPS];
 #pragma unroll
-    for (int g = 0; g < GROUPS; g++) {
-        const int first = t0 + 8 * g, rows = min(max(tokens - first, 0), 8);
-        x_rows[g] = pf_buffer(a.x + (size_t)min(first, tokens - 1) * a.x_pitch, rows ? (uint32_t)(((size_t)(rows - 1) * a.x_pitch + H) * 4) : 0);
-    }
+    for (int g = 0; g < GROUPS; g++) x_row[g] = reinterpret_cast<const float4v *>(a.x + (size_t)min(t0 + 8 * g + lr, tokens - 1) * a.x_pitch) + piece;
     const PfBuffer experts = pf_buffer(a.router_parts + pf_router_tile_at(e0 / 32, H), (uint32_t)min(TC, pf_router_tiles(E) - e0 / 32) * (uint32_t)pf_router_tile_at(1, H));
-    const int x_at = (int)((uint32_t)lr * (uint32_t)a.x_pitch * 4u + 16u * (uint32_t)piece);
     float *mine = router_lds + (size_t)wave * TR * 32 * PF_ROUTER_PITCH;
     float16v acc[TR][TC];
 #pragma unroll
@@ -377,7 +373,7 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
     RouterParts x[2][TR], w[2][TC];   // of the two steps of 16 columns that a piece is
     auto fetch = [&](int l) {
 #pragma unroll
-        for (int g = 0; g < GROUPS; g++) fetched[g] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(x_rows[g], x_at, 128 * min(l, l1 - 1), 0));
+        for (int g = 0; g < GROUPS; g++) fetched[g] = x_row[g][8 * min(l, l1 - 1)];
     };
     auto request = [&](int step, int l) {
 #pragma unroll
