@@ -282,20 +282,25 @@ void pf_launch_row_norm2(const float *d_w, int rows, int cols, float *d_out, hip
 // partial tiles are added in wave order).  Also writes the routing tolerance's bound on the sum of
 // squared products, max(x)^2 * |w_e|^2.  (The shared router's logit comes with the rows' conversion.)
 //
-// A value is h + m + l exactly: h its upper eight significant bits (cut off, so that the largest floats do not round up to
-// infinity), m the rest rounded to eight, l what that leaves.  Of the nine products of two values six are formed, exact in
-// the FP32 sums; the three left out are below 2^-23 of the product together, and l's sign is as good as random.
+// A value is h + m + l exactly: h its upper eight significant bits, rounded (but never to infinity: the largest floats keep theirs),
+// m the rest rounded to eight, l what that leaves, |m| <= 2^-8 and |l| <= 2^-17 of the value.  Of the nine products of two values six are
+// formed, exact in the FP32 sums; the three left out are below 2^-24 (1 + 2^-10) of the product together, what rounding it to FP32
+// takes, as the reference does before it adds: the routing tolerance (pf_route_finish_wave) needs no more than that.
 //
 // The experts' parts are made once, at upload, in the order in which a wave takes them as operands (pf_k_router_parts): 1 KB an
 // instruction, no conversion.  A row of x is fetched in 32-column pieces, whole 128-byte lines (lane = 8 * row + 16-byte piece),
 // passes through LDS of the wave's own (row pitch 144 bytes; no barrier) because a product step wants columns 8 h .. 8 h + 7 of row i
 // from lane (i, h), and is split there, a step ahead of its products.
 //
-// Bound by what the L2 hands out: 2048 tokens of width 2560 against 512 experts are 420 MB of operands in 41 us traced.  On the FP32
+// Bound by what the L2 hands out: 2048 tokens of width 2560 against 512 experts are 420 MB of operands in 42 us traced.  On the FP32
 // instruction, whose products alone take 34, it was 75; with both factors split in the kernel 53, bound by the vector instructions.
 // 1024 tokens of width 2048: 25.4 us (FP32 38); tiles of 64 x 32 instead of 32 x 64 27.1, two pieces ahead no faster.  Error
-// against 64 bits (2-norm; 2047, 1025, 600, 460 tokens): 3.2, 3.5, 2.5, 3.4e-7, on FP32 3.8, 4.1, 2.9, 3.9e-7.
+// against 64 bits, 2-norm (2047 tokens of width 2560, 1025, 600 of 2048) and largest of the magnitudes' sum: 2.8, 2.5, 2.5e-7 and 5.5, 5.1,
+// 5.1e-8, on FP32 3.3, 2.9, 2.9e-7 and 6.4, 5.9, 5.9e-8.  With h cut off (|m| to 2^-7, 2^-22 of a product left out) the largest were 6.9, 7.7,
+// 7.7e-8 at the same time; m l and l m as well bring nothing (the same errors to four digits) for 6 us of 2048 tokens' 43.
 typedef float float4v __attribute__((ext_vector_type(4)));
+typedef short short2v __attribute__((ext_vector_type(2)));
+typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 struct RouterParts { uint4v part[3]; };
@@ -308,10 +313,15 @@ __device__ __forceinline__ RouterParts router_parts(float4v a, float4v b) {
     RouterParts r;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const uint32_t u = __float_as_uint(x[2 * i]), v = __float_as_uint(x[2 * i + 1]);
-        const float u1 = x[2 * i] - __uint_as_float(u & 0xffff0000u), v1 = x[2 * i + 1] - __uint_as_float(v & 0xffff0000u);
+        // no infinity: as signed halves the positive values end at the largest, as unsigned ones the negative values
+        const short2v most = {0x7f7f, 0x7f7f};
+        const ushort2v least = {0xff7f, 0xff7f};
+        uint32_t upper = router_round2(x[2 * i], x[2 * i + 1]);
+        upper = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(short2v, upper), most));
+        upper = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(ushort2v, upper), least));
+        const float u1 = x[2 * i] - __uint_as_float(upper << 16), v1 = x[2 * i + 1] - __uint_as_float(upper & 0xffff0000u);
         const uint32_t middle = router_round2(u1, v1);
-        r.part[0][i] = __builtin_amdgcn_perm(v, u, 0x07060302u);
+        r.part[0][i] = upper;
         r.part[1][i] = middle;
         r.part[2][i] = router_round2(u1 - __uint_as_float(middle << 16), v1 - __uint_as_float(middle & 0xffff0000u));
     }
@@ -417,7 +427,7 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
 #pragma unroll
         for (int m = 0; m < 6 * TR * TC; m++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                               // a product
-            __builtin_amdgcn_sched_group_barrier(0x002, (46 * TR + 6 * TR * TC - 1) / (6 * TR * TC), 0);   // vector instructions
+            __builtin_amdgcn_sched_group_barrier(0x002, (54 * TR + 6 * TR * TC - 1) / (6 * TR * TC), 0);   // vector instructions
         }
         __builtin_amdgcn_sched_barrier(0);
     };

@@ -72,3 +72,45 @@ def test_odd_number_of_expert_tiles(product, oracle, e, tokens):
         layer.force_grouped()
         _, y, ids, w = layer.forward(few[row])
         assert_parity(y, ids, w, *want, label=f"e={e} T={tokens}")
+
+
+def test_products_of_two_values(product):
+    """Logits of one product each: what the parts that are not multiplied leave out.  Bound: with |m| <= 2^-8 and |l| <= 2^-17 of a value
+    m l + l m + l l is at most 2^-24 (1 + 2^-10) of the product, the last sum is off by at most 2^-23, the five before it, of at most 2^-7
+    of the product, together by less than 2^-27: 2^-24 + 2^-23 + 2^-26 covers them."""
+    hidden, e, tokens = 256, 64, 96
+    cfg = abi.moe_config(hidden, e, 4, 256, 256)
+    weights, x = make_layer_inputs(cfg, abi.GGUF_Q4_K, tokens, seed=11)
+    gen = np.random.default_rng(11)
+
+    def values(n):   # any bits; just under a step of the upper eight; just under half of one
+        any_bits = gen.integers(0x3f800000, 0x40000000, n)
+        step = 0x3f800000 + (gen.integers(0, 8, n) << 16) + 0xff80 + gen.integers(0, 128, n)
+        half = 0x3f800000 + (gen.integers(0, 8, n) << 16) + 0x7f80 + gen.integers(0, 128, n)
+        bits = np.choose(np.arange(n) % 3, [any_bits, step, half]).astype(np.uint32)
+        bits[0], bits[1] = 0x3f80ffff, 0x3f80ff80
+        return bits.view(np.float32) * gen.choice([-1.0, 1.0], n).astype(np.float32)
+
+    router = weights.raw[0].view(np.float32).reshape(e, hidden)
+    x[:] = 0.0
+    x[:, 37] = values(tokens) * np.exp2(gen.integers(-60, 61, tokens)).astype(np.float32)
+    x[2:6, 37] = np.array([0x7f7fffff, 0xff7fffff, 0x7f7f8000, 0x7f7f7fff], np.uint32).view(np.float32)   # on either side of rounding to infinity
+    router[:, 37] = values(e) * np.exp2(gen.integers(-12, -2, e)).astype(np.float32)
+    want, hip = x[:, 37:38].astype(np.float64) * router[:, 37].astype(np.float64), product.hip
+    with pf.MoeLayer(product, cfg, weights, tokens) as layer:
+        layer.force_grouped()
+        moe, work = layer.device_handles()
+        d_x, d_y = hip.to_device(x), hip.to_device(np.zeros_like(x))
+        try:
+            print("router products of two values", flush=True)
+            hip.work_limit_kernels(work, 1)
+            hip.check(hip.moe_forward_device(moe, work, d_x, hidden, d_y, hidden, tokens, None), "forward")
+            hip.check(hip.synchronize(), "wait")
+            got = hip.from_device(hip.work_logits(work), (tokens, e), np.float32)
+        finally:
+            hip.work_limit_kernels(work, 0)
+            hip.free(d_x)
+            hip.free(d_y)
+    error = np.abs(got / want - 1.0)
+    print(f"largest error {error.max() * 2.0 ** 23:.3f} times 2^-23", flush=True)
+    assert error.max() <= 2.0 ** -24 + 2.0 ** -23 + 2.0 ** -26
