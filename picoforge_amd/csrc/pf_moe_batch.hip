@@ -366,18 +366,20 @@ struct BatchItem {
     int token0;           // shared expert: the first row's token
     size_t e;             // where the expert's weights are: its id, or its pool slot
 };
-// Number q of a launch.  The shared expert's rows, the list's last items, come first and a chunk of eight a number: `shared` numbers.  (As
-// row tiles, four chunks one after the other, at the list's end they were a launch's end: 101 tokens of the q2 profile 283 us a forward, first
-// 248; for a layer of few experts they were as long as all else.)  False: no such item.
-__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t q, uint32_t shared, BatchItem &it) {
+// Number q of a launch.  The shared expert's rows, the list's last items, are a chunk of eight a number: `shared` numbers.  They come
+// first, unless `last` is set: then the routed tiles do, the longest at the head of the list (batch_shared_last).  (As row tiles, four chunks
+// one after the other, at the list's end they were a launch's end: 101 tokens of the q2 profile 283 us a forward, first 248; for a layer
+// of few experts they were as long as all else.)  False: no such item.
+__device__ __forceinline__ bool batch_item(const PfKernelArgs &a, uint32_t q, uint32_t shared, bool last, BatchItem &it) {
     const uint32_t count = a.tiles[0], routed = count - (shared + 3) / 4;
-    const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[q < shared ? routed + q / 4 : q - shared];   // {expert, first row, rows, first row within the expert}
     if (q >= shared + routed) return false;
-    const int chunk = q < shared ? BATCH_ROWS * (int)(q % 4) : 0;
+    const uint32_t own = last ? q - routed : q;   // its number among the shared expert's, if it is one
+    it.shared = last ? q >= routed : q < shared;
+    const uint4 entry = reinterpret_cast<const uint4 *>(a.items)[it.shared ? routed + own / 4 : last ? q : q - shared];   // {expert, first row, rows, first row within the expert}
+    const int chunk = it.shared ? BATCH_ROWS * (int)(own % 4) : 0;
     const int expert = (int)entry.x;
-    it.shared = expert == a.experts;
     it.first = (int)entry.y + chunk;
-    it.rows = q < shared ? min(BATCH_ROWS, (int)entry.z - chunk) : (int)entry.z;
+    it.rows = it.shared ? min(BATCH_ROWS, (int)entry.z - chunk) : (int)entry.z;
     it.token0 = (int)entry.w + chunk;
     it.e = it.shared ? 0 : (size_t)expert;
     if (a.slots && !it.shared) {   // expert streaming: the rows of an expert share its pool slot
@@ -492,12 +494,12 @@ template <int PLANES> __device__ __forceinline__ void batch_image_group(uint32_t
 #define BATCH_WAVES 4
 // float_rows: the routed experts' activation rows leave the kernel as FP32 (they become digit rows for pf_k_mx_down), else as images.
 template <int FMT, int FMTS, bool ROWS, int PLANES>
-__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a, uint32_t shared_items, int float_rows) {
+__global__ void __launch_bounds__(64 * BATCH_WAVES) __attribute__((amdgpu_waves_per_eu(FMT == PF_IQ2_XXS ? 4 : 3))) pf_k_batch_gate_up(PfKernelArgs a, uint32_t shared_items, int shared_last, int float_rows) {
     __shared__ float partial[BATCH_WAVES][2][4][64];
     __shared__ BatchFactor factors[BATCH_WAVES][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
     BatchItem it;
-    if (!batch_item(a, blockIdx.y, shared_items, it)) return;
+    if (!batch_item(a, blockIdx.y, shared_items, shared_last != 0, it)) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int tile = blockIdx.x, I = it.shared ? a.shared_inter : a.inter;
     if (32 * tile >= I) return;
@@ -561,13 +563,13 @@ __device__ __forceinline__ void batch_stage_rows(uint32_t *stage, const PfKernel
 // blockIdx.x: 128 output rows, a 32-row tile a wave; blockIdx.y: row tile of the expert.  Bound by the products' chain of a wave
 // (with the weights in a cache 90 us of 104 for Q2_K, 101 tokens).
 template <int FMT, int FMTS, bool ROWS, int PLANES>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, uint32_t shared_items) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) pf_k_batch_down(PfKernelArgs a, uint32_t shared_items, int shared_last) {
     constexpr bool STAGED = FMT == PF_Q2_K && !ROWS;
     __shared__ BatchFactor factors[4][64];
     __shared__ __align__(16) uint32_t tables[batch_tables<FMT>() ? BATCH_TABLE_BYTES / 4 : 4];
     __shared__ __align__(16) uint32_t staged[STAGED ? 4 : 1][STAGED ? 2048 : 4];
     BatchItem it;
-    if (!batch_item(a, blockIdx.y, shared_items, it)) return;
+    if (!batch_item(a, blockIdx.y, shared_items, shared_last != 0, it)) return;
     if (batch_tables<FMT>()) batch_stage_tables(tables, a);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), H = a.hidden;
     const int tile = 4 * blockIdx.x + wave;
@@ -707,6 +709,13 @@ void pf_launch_batch_router(const PfKernelArgs &a, int tokens, int planes, bool 
 }
 
 // ---- dispatch --------------------------------------------------------------------------------------
+// Where the shared expert's chunks come in the launches.  A routed tile is up to four chunks one after the other: with more than about three
+// chunks an expert on average the routed tiles are the long items and start first, else the shared expert's, whose rows are all there
+// are and, in a profile, the wider format.  Forwards, shared first : last, us: 350 tokens of 8 experts, two slots, 2048 x 512, Q4_K 93.8 : 80.3, the
+// q2 profile 113.3 : 90.2, 250 tokens of 16 experts, four slots, 94.4 : 85.5, of 32 96.2 : 88.9; 64 tokens of 64 experts, eight slots 63.5 : 65.5, 40
+// of 8, 1024 x 256, 34.3 : 37.8, 130 of 128, eight, 46.5 : 48.7.  Of 504 batches of 8 to 512 experts none is more than 2.5 % slower than in the
+// other order from this line on, and 6 % before it (32 experts beside a shared expert twice as wide).
+static bool batch_shared_last(int tokens, int experts, int top_k) { return (size_t)tokens * top_k >= (size_t)24 * experts; }
 template <int FG, int FD, int FS, bool ROWS, int PLANES>
 static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned routed_cap, hipStream_t stream, int last) {
     const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
@@ -715,21 +724,22 @@ static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned rout
     // shared expert's down projection.  24 tokens 77 -> 39 + 5 + 12, 300 tokens 229 -> 98 + 9 + 23.
     const bool scaled = FD == PF_MXFP4 && PLANES == 3 && a.wm && pf_batch_down_scaled(tokens, a.experts, a.top_k, a.hidden, a.inter, a.shared_inter);
     const unsigned shared = (unsigned)(tokens + BATCH_ROWS - 1) / BATCH_ROWS;
-    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, shared + routed_cap), dim3(64 * BATCH_WAVES), 0, stream, a, shared, scaled ? 1 : 0);
+    const int last_shared = batch_shared_last(tokens, a.experts, a.top_k) ? 1 : 0;
+    hipLaunchKernelGGL((pf_k_batch_gate_up<FG, FS, ROWS, PLANES>), dim3(widest / 32, shared + routed_cap), dim3(64 * BATCH_WAVES), 0, stream, a, shared, last_shared, scaled ? 1 : 0);
     if (last < 4) return;
     const dim3 grid((a.hidden + 127) / 128, shared + routed_cap);
     if (scaled) {
         pf_launch_rows_to_digits(a.act, a.inter, (size_t)tokens * a.top_k, reinterpret_cast<uint32_t *>(a.act16), a.act_scale, a.error_word, stream);
         pf_launch_mx_down(a, tokens, routed_cap, stream);
-        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, shared), dim3(256), 0, stream, a, shared);
+        hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), dim3(grid.x, shared), dim3(256), 0, stream, a, shared, 0);   // the shared expert's numbers alone
         return;
     }
     // down rows: as gate and up where the layer has one format; Q2_K by whole tiles where they fit a wave's LDS, MXFP4 in tile order
     // where the layer keeps that
     constexpr bool either = FD == PF_Q2_K || (FD == PF_MXFP4 && PLANES == 3);
     const bool lines = FD == PF_Q2_K ? 32 * a.row_bytes[3] <= BATCH_STAGE_BYTES : a.wm != nullptr;
-    if (either && lines) hipLaunchKernelGGL((pf_k_batch_down<FD, FS, either ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, shared);
-    else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, shared);
+    if (either && lines) hipLaunchKernelGGL((pf_k_batch_down<FD, FS, either ? false : FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, shared, last_shared);
+    else hipLaunchKernelGGL((pf_k_batch_down<FD, FS, FD != FG || ROWS, PLANES>), grid, dim3(256), 0, stream, a, shared, last_shared);
 }
 
 template <int FG, int FD, int FS>

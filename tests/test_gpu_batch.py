@@ -169,3 +169,19 @@ def test_experts_of_every_row_count(product, oracle, h, i, s, physical, fmt):
         _, y, ids, w = layer.forward(x)
         assert_parity(y, ids, w, *want, label=f"{fmt}")
         np.testing.assert_array_equal(y, layer.forward(x)[1], err_msg="not deterministic")
+
+
+@pytest.mark.parametrize("h,i,s,physical,fmt", [
+    (512, 256, 512, None, abi.GGUF_Q4_K), (512, 256, 256, None, abi.GGUF_IQ2_XXS), (512, 384, 256, 512, "q2"), (512, 256, 256, None, "q4"), (512, 384, 512, None, "q4")])
+def test_shared_rows_behind_the_routed_ones(product, oracle, h, i, s, physical, fmt):
+    """Few experts of many rows, whose launches take the shared expert's chunks last (from 96 tokens on), on both sides of that line."""
+    print(f"case shared rows last, {fmt} h={h} i={i} s={s}", flush=True)
+    cfg = abi.moe_config(h, 8, 2, i, s, down_physical=physical)
+    weights, x = make_layer_inputs(cfg, fmt, 131, seed=h + i + s)
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, len(x)) as layer:
+        for tokens in (95, 96, 131):
+            assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == 3
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
+        np.testing.assert_array_equal(y, layer.forward(x[:tokens])[1], err_msg="not deterministic")
