@@ -55,6 +55,32 @@ PF_HD uint32_t pf_item_numbers(int slabs, int shift, uint32_t routed, uint32_t s
     return ((routed + deal - 1) / deal * deal + (shared + PF_XCDS - 1) / PF_XCDS * PF_XCDS) * (uint32_t)slabs;   // (no XCD has more)
 }
 
+// Pairs up to which a batch of a layer of one format (with its tile-ordered copies) runs the decode kernels, which read an expert once a
+// pair, and from which on the kernels for a few rows per expert, which read it once for the batch.  The line goes by the work of a pair,
+// hidden x inter: the few-row kernels' launches take at least 30 to 40 us, which short products do not earn back by 32 tokens.
+// Where the two take the same time (pairs; 16 to 32 tokens swept; E (top-k) = 16 (4), 32 (6), 64, 128, 256 (8), 512 (6, 10); > beyond
+// them, < before them):
+//   Q4_K     2048 x 512  120, 110, 128, 136, 140, 190, 170       2560 x 512, 2048 x 768  < but 512 (6): 110, 170
+//            2048 x 256  >, >, 162, 162, 192, >, 210             1024 x 512  >, >, 150, 160, >, >, 280     768 x 768  32 (6) on: 140, 150, 175, >, 280
+//            1024 x 256, 512 x 512, 512 x 256  > (0.64 to 0.9 of the few-row kernels' time up to there)
+//   IQ2_XXS  2048 x 512  70, < from there on                     inter from 512 on, hidden from 512 on  < but 1024 x 512: 64, <
+//            2048 x 256  >, 140, 145, 145, 150, 138, 180         1024 x 256  >, >, 155, 165, 200, >, 230   512 x 256  >, >, 170, 170, 200, >, 260
+// us, decode kernels : few rows: 24 tokens of 64 experts, Q4_K, 2048 x 512 67 : 53, of 128 of 1024 x 256 33 : 42; 20 tokens of 512, ten slots,
+// IQ2_XXS, 2048 x 512 87 : 73, of 512 x 256 36 : 41.  Neither side is nearer to 64 bits on the wide layers (2-norm, 24 tokens of 64 experts of
+// 2048 x 512: Q4_K 3.08 : 3.09 and 3.29 : 3.22e-7, IQ2_XXS 2.68 : 2.70 and 2.73 : 2.70e-7), on narrow ones the decode kernels by up to 4 %.
+// IQ2_XXS layers between the classes keep a line at 165 pairs, up to 1.3 times too late where inter is 512.
+PF_HD size_t pf_decode_pairs(bool q4k, size_t experts, size_t hidden, size_t inter) {
+    const size_t work = hidden * inter, whole = (size_t)1 << 20;
+    if (q4k) {
+        if (work >= whole) return (110 + experts / 4) * whole / work;
+        const size_t many = 150 + experts / 5, few = experts < 232 ? 232 - experts : 0;
+        return work >= whole / 2 ? (many > few ? many : few) : 200 + experts / 2;
+    }
+    if (work >= whole) return 70;
+    if (work >= whole / 2 || inter >= 512) return 165;
+    return experts < 150 ? 160 + experts / 2 : 235;
+}
+
 // Which MXFP4 down projections of a layer that keeps them in tile order run on the block-scaled product.  It saves work for every weight
 // and row, and costs launches of its own (the rows' conversion 3 to 5 us; in the few-row kernels the shared expert's part as well).
 //

@@ -5,6 +5,7 @@
 #include "pf_host_rows.h"
 #include "pf_piece_order.h"
 #include "pf_router_addr.h"
+#include "pf_item_order.h"
 #include "../../include/pf_iq2_codes.h"
 #include <stdio.h>
 #include <stdlib.h>
@@ -913,23 +914,16 @@ struct HcTarget {   // residual streams to inject into instead of writing y
 // The lines follow the batch's pairs P and the layer's experts E, not its tokens alone: with fewer experts the same tokens are more rows
 // an expert.  Up to 64 experts the second is a number of pairs, from there it pays for every expert met; a rule on tokens that fits
 // 512 experts (32 / 240 for Q4_K, 32 / 320, 10 / 400, 16 / 400) is 1.42 times slower than the better side with 64.
-// The first line, in layers of one format, lies where the two sides take the same time from 128 (Q4_K) and 129 (IQ2_XXS) experts on.  Swept
-// over E (top-k) = 16 (4, 8), 32 (6, 10), 48 (8), 64 (4, 8), 128 (4, 8), 256 (8), 512 (6, 10), 8 to 32 tokens, uniform and Zipf popularity, they
-// cross at
-//   Q4_K     112, 128, 102, 108, 96, 96, 136, 116, 136, 188, 190, 245 pairs
-//   IQ2_XXS   64,  90,  66,  90, 80, 64,  90,  68, 112, 128,  96, 120 pairs, 16 tokens and fewer
-// (512 experts, top-10, us: 24 tokens Q4_K 99 : 100, 32 tokens 121 : 115; 16 tokens IQ2_XXS 78 : 74, 32 tokens 123 : 98).  With fewer
-// experts the line is still where earlier kernels crossed, and batches up to it are slower than they need be: Q4_K 28 tokens of 64
-// experts 86 : 62, IQ2_XXS 28 tokens of 128 experts 103 : 69.  Neither side is nearer to 64 bits (2-norm, 24 tokens, decode kernels : few rows:
-// Q4_K 3.15 : 3.13e-7 and 3.13 : 3.07e-7, IQ2_XXS 2.62 : 2.65e-7 and 2.80 : 2.78e-7).
-// The profiles' first line and the second line were drawn on earlier kernels too.  Over the same layers, 5 to 420 tokens, the present
-// kernels cross at
-//   pairs -> few rows      q2 from 32 to 64 pairs on, up to 1.30 beyond the crossing (8 tokens, 64 experts); q4 not up to 16 tokens,
-//                          but at 64 experts, 16
-//   few rows -> grouped    one format 112, 168, 136 to 192, 80 to 224, 136 to 2000, 280 to 3200 pairs; q2 112, 168, 400, 1000, 2560, 4000; q4
-//                          160, 240, 512, 512, 400, 280
-// so a batch just under the second line is 1.02 to 1.27 times slower than on the grouped product (125 tokens, 64 experts, Zipf 1.27;
-// 400 tokens of the q4 profile, 512 experts 1.21).  These lines stay: the side that they keep is the one nearer to the result in 64
+// The first line of a layer of one format is pf_decode_pairs (pf_item_order.h).
+// The profiles' first line and the second line were drawn on earlier kernels.  The present ones cross, over E (top-k) = 16 (4), 32 (6), 64,
+// 128, 256 (8), 512 (10), at
+//   pairs -> few rows      2560 x 640: q2 30, 40 to 50 from 64 experts on, 1.35 beyond the crossing (10 tokens), q4 40, 96 at 64, 128
+//                          at 128 experts, 512 not up to 16 tokens; 2048 x 512: q2 beyond 40, 62 at 64, 68 at 128, 65 at 512 experts; q4 only
+//                          at 64, 104
+//   few rows -> grouped    Q4_K, 2048 x 512, 190, 600, 750, 1200, 2000, 1550 pairs, IQ2_XXS 180, 590, 740, 1250, 1700, 1500; q2, 2560 x 640, 150, 340,
+//                          580, 960, 1650, 1600; q4 250, 470, 680, 850, 1280, 1600
+// so a batch just under the second line is 1.05 to 1.25 times slower than on the grouped product, of 16 experts up to 1.5 times (160
+// tokens of the q2 profile).  These lines stay: the side that they keep is the one nearer to the result in 64
 // bits (60 tokens, 24 experts, decode kernels / few rows / grouped product: Q4_K 3.2 / 3.1 / 6.7e-7, IQ2_XXS 2.6 / 2.6 / 4.0e-7, q2
 // 2.7 / 3.0 / 4.8e-7, q4 2.7 / 2.8 / 4.4e-7).
 struct BatchRange { size_t pair_to, batch_to; };
@@ -942,7 +936,7 @@ static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
     auto within = [](size_t low, size_t v, size_t high) { return v < low ? low : v > high ? high : v; };
     size_t pair_to = PF_DECODE_MAX_TOKENS;   // no tile-ordered copies: the segment kernels take four tokens
     if (combination && throughout)
-        pair_to = within(PF_TILE_DECODE_MAX_TOKENS, (q4k ? (E < 128 ? 200 + E / 2 : 150 + E / 5) : (E <= 128 ? 160 + E / 2 : 165)) / K, PF_PAIR_MAX_TOKENS);
+        pair_to = within(PF_TILE_DECODE_MAX_TOKENS, pf_decode_pairs(q4k, E, moe->desc.hidden, moe->desc.inter) / K, PF_PAIR_MAX_TOKENS);
     else if (combination) pair_to = q4k ? PF_TILE_DECODE_MAX_TOKENS : 10;
     size_t most;
     if (throughout && (q4k || combination)) most = within(1000, 16 * E, 1400 + 9 * E / 2);

@@ -185,3 +185,22 @@ def test_shared_rows_behind_the_routed_ones(product, oracle, h, i, s, physical, 
             _, y, ids, w = layer.forward(x[:tokens])
             assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
         np.testing.assert_array_equal(y, layer.forward(x[:tokens])[1], err_msg="not deterministic")
+
+
+# (hidden, inner width, experts, top-k, format, last batch of the decode kernels): the three classes of widths
+WIDTH_LINES = [(2048, 512, 16, 4, abi.GGUF_Q4_K, 28), (2048, 512, 64, 8, abi.GGUF_Q4_K, 16), (1024, 512, 64, 8, abi.GGUF_Q4_K, 21),
+               (1024, 256, 128, 8, abi.GGUF_Q4_K, 32), (2048, 512, 24, 4, abi.GGUF_IQ2_XXS, 17), (512, 512, 130, 8, abi.GGUF_IQ2_XXS, 20),
+               (1024, 256, 200, 10, abi.GGUF_IQ2_XXS, 23)]
+
+
+@pytest.mark.parametrize("h,i,e,k,fmt,pair_to", WIDTH_LINES)
+def test_first_line_goes_by_the_work_of_a_pair(product, oracle, h, i, e, k, fmt, pair_to):
+    print(f"case first line {fmt} h={h} i={i} e={e} k={k}", flush=True)
+    cfg = abi.moe_config(h, e, k, i, i)
+    weights, x = make_layer_inputs(cfg, fmt, 33, seed=h + e)
+    want = forward_with(oracle, cfg, weights, x)
+    with pf.MoeLayer(product, cfg, weights, 33) as layer:
+        for tokens, family in ((pair_to, 1), (pair_to + 1, 3)):
+            assert product.hip.moe_kernel_family(*layer.device_handles(), tokens) == family, tokens
+            _, y, ids, w = layer.forward(x[:tokens])
+            assert_parity(y, ids, w, want[0][:tokens], want[1][:tokens], want[2][:tokens], label=f"{fmt} T={tokens}")
