@@ -20,3 +20,9 @@ def test_rows_through_the_ring_by_several_callers(tmp_path, sanitizer):
     print(run.stdout, run.stderr)
     assert run.returncode == 0, run.stderr
     assert run.stdout.startswith("0 faults")
+
+
+def test_page_locked_memory_of_a_ring(tmp_path):
+    """A workspace of more than 64 tokens holds 4 MB of it."""
+    source = f'#include "{ROOT}/picoforge_amd/csrc/pf_host_rows.h"\nstatic_assert(PF_RING_SLOTS * PF_RING_BYTES == (size_t)4 << 20, "the ring");\n'
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-x", "c++", "-"], input=source, text=True, check=True)
