@@ -14,9 +14,9 @@
 //   order       by p descending, then id ascending.  The reference orders by fl(p / sum) with the same
 //               tie rule.  Two p four ulps or more apart give quotients that round to different values,
 //               equal p stay equal, and closer p can only tie, which goes to the lower id: no change
-//               when the larger p has the lower id already.  Two neighbours among the k + 1 first that
-//               are fewer than four ulps apart, not equal, with the larger p on the higher id need the
-//               sum itself: then, or with more than 64 candidates, or with probabilities near the
+//               when the larger p has the lower id already.  Two neighbours among the k + 1 first, or
+//               as near to the last chosen, that are fewer than four ulps apart, not equal, with the larger p on the
+//               higher id need the sum itself (pf_fix_doubtful): then, or with more than 64 candidates, or with probabilities near the
 //               subnormals, the workgroup routes the token the long way (all logits serially, 64 experts
 //               a pass through the same chains, then pf_route_exact_wave).
 //
@@ -80,6 +80,21 @@ __device__ __forceinline__ float pf_serial_chunk(float sum, const float *p, int 
         sum = sum + v.w;
     }
     return sum;
+}
+
+// Whether the candidates' p = exp(z - max) leave their order open: one a lane, by p descending, then id ascending, `count` of them.
+// The reference orders by fl(p / sum): two p that are four ulps or more apart give quotients more than one ulp apart, which round to
+// different values; closer p may tie after the division, and a tie goes to the lower id: that changes nothing when the larger p has the
+// lower id already.  So the doubt is a pair of neighbours fewer than four ulps apart, not equal, whose larger p has the higher id: among
+// the first k + 1, and beyond them as far as a p is fewer than four ulps below the last chosen one (of seven equal p the six lowest
+// ids are chosen, and the eighth expert, an ulp lower, may still tie with them and come before the sixth).  And nothing may be near
+// the subnormals.
+__device__ __forceinline__ bool pf_fix_doubtful(float p, uint32_t id, int picks, int count, int lane) {
+    const float next = __shfl_down(p, 1), last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), picks - 1));
+    const uint32_t next_id = (uint32_t)__shfl_down((int)id, 1);
+    const bool paired = lane + 1 < count && (lane < picks || __float_as_uint(last) - __float_as_uint(next) < 4u);
+    const bool near = p != next && __float_as_uint(p) - __float_as_uint(next) < 4u;
+    return __any((paired && near && id > next_id) || (lane < picks && !(p > 1e-30f)) || (lane < picks && paired && !(next > 1e-30f)));
 }
 
 // LDS the workgroup needs: the candidates' ids (64 words), four words of hand-over, the token's row (H floats), then
@@ -214,17 +229,7 @@ __device__ __forceinline__ int pf_route_fix_block(const float *router, const flo
             const int to = active ? rank : lane;   // a permutation of the lanes
             const uint32_t sid = (uint32_t)__builtin_amdgcn_ds_permute(to * 4, (int)id);
             const float sp = __int_as_float(__builtin_amdgcn_ds_permute(to * 4, __float_as_int(pc)));
-            // Neighbours among the first k + 1.  The reference orders by fl(p / sum): two p that are four ulps or more
-            // apart give quotients more than one ulp apart, which round to different values; closer p may tie after the
-            // division, and a tie goes to the lower id: that changes nothing when the larger p has the lower id already.
-            // So the doubt is a pair fewer than four ulps apart, not equal, whose larger p has the higher id; and
-            // nothing may be near the subnormals.
-            const float next = __shfl_down(sp, 1);
-            const uint32_t next_id = (uint32_t)__shfl_down((int)sid, 1);
-            const bool paired = lane < picks && lane + 1 < count;
-            const bool near = sp != next && __float_as_uint(sp) - __float_as_uint(next) < 4u;
-            const bool doubtful = (paired && near && sid > next_id) || (lane < picks && !(sp > 1e-30f)) || (paired && !(next > 1e-30f));
-            long_way = __any(doubtful);
+            long_way = pf_fix_doubtful(sp, sid, picks, count, lane);
             if (!long_way) {
                 const float chosen = pf_wave_sum(lane < picks ? sp : 0.0f);
                 float weight;

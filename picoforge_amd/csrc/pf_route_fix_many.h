@@ -117,17 +117,7 @@ __device__ __forceinline__ bool pf_fix_finish(int count, uint32_t candidate, flo
     const int to = active ? rank : lane;   // a permutation of the lanes
     const uint32_t sid = (uint32_t)__builtin_amdgcn_ds_permute(to * 4, (int)id);
     const float sp = __int_as_float(__builtin_amdgcn_ds_permute(to * 4, __float_as_int(pc)));
-    // Neighbours among the first k + 1.  The reference orders by fl(p / sum): two p that are four ulps or more
-    // apart give quotients more than one ulp apart, which round to different values; closer p may tie after the
-    // division, and a tie goes to the lower id: that changes nothing when the larger p has the lower id already.
-    // So the doubt is a pair fewer than four ulps apart, not equal, whose larger p has the higher id; and
-    // nothing may be near the subnormals.
-    const float next = __shfl_down(sp, 1);
-    const uint32_t next_id = (uint32_t)__shfl_down((int)sid, 1);
-    const bool paired = lane < picks && lane + 1 < count;
-    const bool near = sp != next && __float_as_uint(sp) - __float_as_uint(next) < 4u;
-    const bool doubtful = (paired && near && sid > next_id) || (lane < picks && !(sp > 1e-30f)) || (paired && !(next > 1e-30f));
-    if (__any(doubtful)) return false;
+    if (pf_fix_doubtful(sp, sid, picks, count, lane)) return false;
     const float chosen = pf_wave_sum(lane < picks ? sp : 0.0f);
     float weight;
     if (norm) {
