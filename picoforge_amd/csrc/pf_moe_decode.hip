@@ -1273,7 +1273,7 @@ static void launch_dec_route_lists(const PfKernelArgs &a, int tokens, size_t lds
 
 #if PF_DECODE_PART == 0
 void pf_launch_dec_route(const PfKernelArgs &a, int tokens, hipStream_t stream) {
-    const size_t lds = pf_route_fix_lds_floats(a.hidden, a.experts) * 4;
+    const size_t lds = pf_fix_token_lds_floats(a.experts) * 4;
     const int all = (a.experts + 63) / 64;
     if (all <= 1) launch_dec_route_lists<1>(a, tokens, lds, stream);
     else if (all <= 2) launch_dec_route_lists<2>(a, tokens, lds, stream);

@@ -48,12 +48,13 @@ struct PfKernelArgs {
     uint32_t pool_slots;
     uint32_t *error_word;
     uint32_t *exact_rows;            // count of tokens re-routed in serial order
-    uint32_t *route_flags;           // tokens to route again in serial order: [0] their number, then the tokens; the kernel
-                                     // before the routing clears [0]
+    uint32_t *route_flags;           // layers whose every token is routed in serial order (pf_route_needs_slabs): [0] the tokens' number,
+                                     // then the tokens (pf_k_flag_all)
     // prefill path
     uint32_t token_cap;              // rows the workspace holds; row token_cap (token_cap * top_k for act16) of an fp16 form is all zero
     uint16_t *x16, *act16, *sact16;  // fp16 forms of x, act (pairs in expert order), shared act: per row the high
-                                     // parts, the low parts, then 8 + 8 group-sum parts per 256 columns
+                                     // parts, the low parts, then 8 + 8 group-sum parts per 256 columns (act16 before a Q2_K
+                                     // projection 16 + 16, before an MXFP4 one the digit rows of pf_mx_rows.h)
     float *x_scale, *act_scale, *sact_scale;   // per row: the power of two the fp16 form was divided by
     const float *w_norm2;            // [experts] squared norm of each router row
     const uint8_t *router_parts;     // router as operands of the chunks' logits (pf_k_router_parts)
@@ -273,7 +274,7 @@ void pf_launch_block_split(const uint8_t *d_gguf, uint8_t *d_payload, uint8_t *d
 // pf_moe_prefill.hip
 bool pf_prefill_supported(const PfHipMoeDesc &d);
 void pf_launch_prefill(const PfKernelArgs &a, int tokens, hipStream_t stream, int stage_limit);
-bool pf_group_fits(const uint32_t *d_ids, int pairs, int experts);   // one workgroup groups them
+bool pf_group_fits(const uint32_t *d_ids, int pairs, int experts);   // pf_k_group_fused, or a chunk's pf_k_pf_group_rows, groups them
 void pf_launch_group(const PfKernelArgs &a, const uint32_t *ids, int tokens, hipStream_t stream);
 void pf_launch_combine(const PfKernelArgs &a, int tokens, hipStream_t stream);
 void pf_launch_q4k_tile(const uint8_t *d_src, uint8_t *d_dst, size_t rows, int blocks_per_row, hipStream_t stream);

@@ -359,7 +359,6 @@ __global__ void __launch_bounds__(64 * PF_ROUTER_WAVES) __attribute__((amdgpu_wa
     __shared__ uint32_t largest[32 * TR];                 // the rows' largest magnitudes, as bits
     const int H = a.hidden, E = a.experts, lane = pf_lane(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t0 = blockIdx.x * 32 * TR, e0 = blockIdx.y * 32 * TC;
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.route_flags[0] = 0;   // the routing's list starts empty
     if (threadIdx.x < 32 * TR) largest[threadIdx.x] = 0;
     const int i = lane & 31, kk = lane >> 5;
     // the waves split the rows' 128-byte lines (hidden is a multiple of 32)

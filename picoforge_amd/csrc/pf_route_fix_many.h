@@ -151,7 +151,8 @@ __device__ __forceinline__ void pf_fix_long_way(const float *router, const float
 }
 
 // One token, called by every wave of a workgroup of PF_FIX_THREADS threads, whose routing knows the smallest and the largest of the k
-// best logits (wave 0).  lds: 68 + 2 PF_FIX_CHUNK_FLOATS + 3 E floats; the rest as pf_route_fix_block.
+// best logits (wave 0).  lds: pf_fix_token_lds_floats; the rest as pf_route_fix_block.
+__host__ __device__ constexpr size_t pf_fix_token_lds_floats(int E) { return 68 + 2 * PF_FIX_CHUNK_FLOATS + 3 * (size_t)E; }
 template <int NPL>
 __device__ __forceinline__ int pf_fix_token(const float *router, const float *x, const float *z_row, const float *ssq_row, float kth, float best_z, int E,
                                             int K, bool norm, int H, float *lds, uint32_t *ids_out, float *w_out, int wave, int lane) {
