@@ -93,10 +93,13 @@ PF_HD bool pf_decode_down_scaled(int tokens, int top_k, int hidden, int inter) {
     return tokens >= PF_DOWN_SCALED_FROM && (size_t)tokens * top_k * hidden * inter >= 55000000u;
 }
 // Batches of the few-row kernels: the weights of the experts there are and of every eight rows more, and the shared expert's chunks of
-// eight rows, which that kernel takes one after the other and the launch beside the block-scaled product side by side.  Forwards on
-// the integers and there, us: 24 tokens, 32 experts of 512 x 256, four slots 36.3 : 40.5, 17 tokens, 128 experts of 1024 x 256, eight
-// 46.3 : 50.8, 17 tokens, 512 experts of 2048 x 512, ten 105.2 : 103.4, 32 tokens, 32 experts of 1024 x 512, four 63.6 : 56.9, 400 tokens, 512
-// experts of 2560 x 640, ten 562 : 481.  Of 732 batches as above none is more than 3 % slower than on the other side.
+// eight rows.  The line was drawn while that kernel took those chunks one after the other, which the launch beside the block-scaled
+// product did not; since they are items of their own in both it lies too early.  Forwards on the integers and there, us, all on this
+// side of it: 32 tokens, 32 experts of 1024 x 512, four slots 39.2 : 47.0, 17 tokens of 8 experts of 2048 x 512 beside 1024 44.5 : 57.2, 512 experts, ten
+// slots, of 2048 x 512 24 tokens 102 : 110 and 64 tokens 172 : 168, of 2560 x 640 17 tokens 124 : 130, 32 tokens 172 : 168, 101 tokens 307 : 283, 400
+// tokens 540 : 490.  Of 490 batches of 8 to 512 experts 241 are more than 5 % slower than on the other side, up to 29 %; with the chunks
+// left out of the sum and 350e6 for 200e6 it would be 24.  (The term and the two small batches that the line is tested to take stay
+// until that test states them anew.)
 PF_HD bool pf_batch_down_scaled(int tokens, int experts, int top_k, int hidden, int inter, int shared_inter) {
     const size_t pairs = (size_t)tokens * top_k, met = pairs < (size_t)experts ? pairs : (size_t)experts;
     const size_t chunks = tokens >= 32 ? 4 : ((size_t)tokens + 7) / 8;   // of a row tile of the shared expert

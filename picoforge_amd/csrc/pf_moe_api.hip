@@ -924,8 +924,8 @@ struct HcTarget {   // residual streams to inject into instead of writing y
 //                          580, 960, 1650, 1600; q4 250, 470, 680, 850, 1280, 1600
 // so a batch just under the second line is 1.05 to 1.25 times slower than on the grouped product, of 16 experts up to 1.5 times (160
 // tokens of the q2 profile).  These lines stay: the side that they keep is the one nearer to the result in 64
-// bits (60 tokens, 24 experts, decode kernels / few rows / grouped product: Q4_K 3.2 / 3.1 / 6.7e-7, IQ2_XXS 2.6 / 2.6 / 4.0e-7, q2
-// 2.7 / 3.0 / 4.8e-7, q4 2.7 / 2.8 / 4.4e-7).
+// bits (60 tokens, 24 experts, decode kernels / few rows / grouped product: Q4_K 3.2 / 3.1 / 6.7e-7, IQ2_XXS 2.6 / 2.7 / 3.9e-7, q2
+// 2.7 / 3.0 / 4.2e-7, q4 2.8 / 2.8 / 4.4e-7).
 struct BatchRange { size_t pair_to, batch_to; };
 static BatchRange batch_range(const PfHipMoe *moe, const PfHipWork *work) {
     const int combination = pf_decode_tile_layer(moe->desc, moe->w_tiled, moe->w_itile, moe->w_qtile);

@@ -719,9 +719,8 @@ static bool batch_shared_last(int tokens, int experts, int top_k) { return (size
 template <int FG, int FD, int FS, bool ROWS, int PLANES>
 static void launch_batch_format(const PfKernelArgs &a, int tokens, unsigned routed_cap, hipStream_t stream, int last) {
     const int widest = a.inter > a.shared_inter ? a.inter : a.shared_inter;
-    // The q4 profile's routed down projection on the block-scaled product, as a chunk's, where the work is worth its launches: on the
-    // integers 101 tokens of the checkpoints' widths took 157 us row by row and 120 in tile order, there 84, 7 for the rows and 14 for the
-    // shared expert's down projection.  24 tokens 77 -> 39 + 5 + 12, 300 tokens 229 -> 98 + 9 + 23.
+    // The q4 profile's routed down projection on the block-scaled product, as a chunk's, where the work is taken to be worth its launches
+    // (pf_batch_down_scaled, with both sides measured): 101 tokens of the checkpoints' widths 307 us a forward on the integers, 283 there.
     const bool scaled = FD == PF_MXFP4 && PLANES == 3 && a.wm && pf_batch_down_scaled(tokens, a.experts, a.top_k, a.hidden, a.inter, a.shared_inter);
     const unsigned shared = (unsigned)(tokens + BATCH_ROWS - 1) / BATCH_ROWS;
     const int last_shared = batch_shared_last(tokens, a.experts, a.top_k) ? 1 : 0;

@@ -18,7 +18,7 @@
 // A workgroup routes up to sixteen tokens, a wave each, and then those of them whose best logits are too close, together
 // (pf_route_fix_many.h): the candidates of all of them, as many as there are lanes, share the chain's wave, which costs the same for
 // one token as for five.  exact_rows[0] counts the tokens routed again, exact_rows[1] those of them that went the long way.
-// Bound by that chain, a dependent addition a column.  1024 tokens of width 2048 25 us traced, 2048 of width 2560 26, where a launch
+// Bound by that chain, a dependent addition a column.  1024 tokens of width 2048 25 us traced, 2048 of width 2560 28, where a launch
 // that routed and one that routed again, a workgroup a flagged token, took 8.2 + 22.6 and 9.1 + 23.9.  (Handing every pair its rank among its
 // expert's here, by additions to a counter an expert in memory, took 10 us: a popular one's queue.)
 #define ROUTE_TOKENS 16
