@@ -66,9 +66,10 @@ PF_HD uint32_t pf_item_numbers(int slabs, int shift, uint32_t routed, uint32_t s
 //   IQ2_XXS  2048 x 512  70, < from there on                     inter from 512 on, hidden from 512 on  < but 1024 x 512: 64, <
 //            2048 x 256  >, 140, 145, 145, 150, 138, 180         1024 x 256  >, >, 155, 165, 200, >, 230   512 x 256  >, >, 170, 170, 200, >, 260
 // us, decode kernels : few rows: 24 tokens of 64 experts, Q4_K, 2048 x 512 67 : 53, of 128 of 1024 x 256 33 : 42; 20 tokens of 512, ten slots,
-// IQ2_XXS, 2048 x 512 87 : 73, of 512 x 256 36 : 41.  Neither side is nearer to 64 bits on the wide layers (2-norm, 24 tokens of 64 experts of
-// 2048 x 512: Q4_K 3.08 : 3.09 and 3.29 : 3.22e-7, IQ2_XXS 2.68 : 2.70 and 2.73 : 2.70e-7), on narrow ones the decode kernels by up to 4 %.
-// IQ2_XXS layers between the classes keep a line at 165 pairs, up to 1.3 times too late where inter is 512.
+// IQ2_XXS, 2048 x 512 87 : 73, of 512 x 256 36 : 41.  Distance to 64 bits (2-norm, mean of eight layers each, decode kernels : few rows): Q4_K
+// 3.14 : 3.14e-7 at 2048 x 512, 3.20 : 3.17 at 2560 x 768, 3.04 : 3.03 at 1024 x 512, 3.11 : 3.12 at 2048 x 256; IQ2_XXS 2.67 : 2.69, 2.72 : 2.71, 2.60 : 2.60
+// and 2.63 : 2.69.  So the wide layers' lines follow the clock alone, and narrower IQ2_XXS layers stay with the decode kernels for
+// longer: with few experts up to 1.4 times too late where inter is 512, 1.3 where it is 256.
 PF_HD size_t pf_decode_pairs(bool q4k, size_t experts, size_t hidden, size_t inter) {
     const size_t work = hidden * inter, whole = (size_t)1 << 20;
     if (q4k) {
@@ -77,8 +78,8 @@ PF_HD size_t pf_decode_pairs(bool q4k, size_t experts, size_t hidden, size_t int
         return work >= whole / 2 ? (many > few ? many : few) : 200 + experts / 2;
     }
     if (work >= whole) return 70;
-    if (work >= whole / 2 || inter >= 512) return 165;
-    return experts < 150 ? 160 + experts / 2 : 235;
+    if (work < whole / 2 && inter < 512) return experts < 150 ? 160 + experts / 2 : 235;
+    return experts <= 128 ? 160 + experts / 2 : experts <= 256 ? 224 - (experts - 128) * 59 / 128 : 165;
 }
 
 // Which MXFP4 down projections of a layer that keeps them in tile order run on the block-scaled product.  It saves work for every weight

@@ -189,7 +189,7 @@ def test_shared_rows_behind_the_routed_ones(product, oracle, h, i, s, physical, 
 
 # (hidden, inner width, experts, top-k, format, last batch of the decode kernels): the three classes of widths
 WIDTH_LINES = [(2048, 512, 16, 4, abi.GGUF_Q4_K, 28), (2048, 512, 64, 8, abi.GGUF_Q4_K, 16), (1024, 512, 64, 8, abi.GGUF_Q4_K, 21),
-               (1024, 256, 128, 8, abi.GGUF_Q4_K, 32), (2048, 512, 24, 4, abi.GGUF_IQ2_XXS, 17), (512, 512, 130, 8, abi.GGUF_IQ2_XXS, 20),
+               (1024, 256, 128, 8, abi.GGUF_Q4_K, 32), (2048, 512, 24, 4, abi.GGUF_IQ2_XXS, 17), (512, 512, 256, 8, abi.GGUF_IQ2_XXS, 20),
                (1024, 256, 200, 10, abi.GGUF_IQ2_XXS, 23)]
 
 
